@@ -290,6 +290,46 @@ void gemm_tile(const at::Tensor& x, const at::Tensor& w, const c10::optional<at:
                      (int)silu_gu, (int)variant, (int)splits, pp, cur_stream()));
 }
 
+void gemm_mid(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& y_opt,
+              const c10::optional<at::Tensor>& bias, const c10::optional<at::Tensor>& partial, int64_t splits, int64_t silu_gu) {
+  CHECK_DEV(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_CONTIG(x); CHECK_CONTIG(w);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && w.size(1) == x.size(1), "gemm_mid: x [M, K], w [N, K]");
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(M >= 1 && N >= 16 && N % 16 == 0 && K % 64 == 0, "gemm_mid: N % 16 == 0, K % 64 == 0");
+  TORCH_CHECK(M < (1LL << 24) && N < (1LL << 30) && K < (1LL << 22), "gemm too large");
+  TORCH_CHECK(splits >= 1 && splits <= 16 && K / 64 >= splits, "gemm_mid: bad split count");
+  TORCH_CHECK(!silu_gu || (N % 128 == 0 && !bias.has_value()), "gemm_mid: a gated epilogue needs N % 128, no bias");
+  bf16_t* yp = nullptr;
+  int64_t ldy = silu_gu ? N / 2 : N;
+  if (y_opt.has_value()) {
+    const at::Tensor& y = *y_opt;
+    CHECK_DEV(y); CHECK_BF16(y);
+    TORCH_CHECK(y.dim() == 2 && y.size(0) == M && y.size(1) == ldy && y.stride(1) == 1 && y.stride(0) % 8 == 0 &&
+                    y.stride(0) >= ldy && reinterpret_cast<uintptr_t>(y.data_ptr()) % 16 == 0,
+                "gemm_mid: y [M, N] (N/2 gated), unit column stride, 16-B aligned rows");
+    TORCH_CHECK(splits == 1 || y.stride(0) == ldy, "gemm_mid: the split-K reduce needs a contiguous y");
+    yp = ptr<bf16_t>(y);
+    ldy = y.stride(0);
+  } else {
+    TORCH_CHECK(splits > 1 && !silu_gu, "y may be omitted only for split-K slabs summed by the consumer");
+  }
+  if (bias.has_value()) {
+    CHECK_DEV(*bias); CHECK_BF16(*bias); CHECK_CONTIG(*bias);
+    TORCH_CHECK(bias->numel() == N && splits == 1 && reinterpret_cast<uintptr_t>(bias->data_ptr()) % 16 == 0,
+                "gemm_mid: bias [N], 16-B aligned, one slice");
+  }
+  float* pp = nullptr;
+  if (splits > 1) {
+    TORCH_CHECK(partial.has_value(), "split-K needs a partial buffer");
+    CHECK_DEV(*partial); CHECK_DT(*partial, at::kFloat); CHECK_CONTIG(*partial);
+    TORCH_CHECK(partial->numel() >= splits * M * N, "partial buffer too small");
+    pp = partial->data_ptr<float>();
+  }
+  const c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+  RC(oamd::gemm_mid(ptr<bf16_t>(x), ptr<bf16_t>(w), yp, optr<bf16_t>(bias), pp, (int)M, (int)N, (int)K, (int)ldy, (int)silu_gu,
+                    (int)splits, cur_stream()));
+}
+
 void gemm_pp(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& y_opt,
              const c10::optional<at::Tensor>& p, int64_t splits, int64_t bm, int64_t silu_gu, bool nt, bool one_seg,
              const c10::optional<at::Tensor>& sk_ws, const c10::optional<at::Tensor>& sk_flags) {
@@ -615,6 +655,8 @@ PYBIND11_MODULE(_C, m) {
         pybind11::arg("p") = pybind11::none(), pybind11::arg("splits") = 1, pybind11::arg("bn") = 64,
         pybind11::arg("bm") = 0, pybind11::arg("silu_gu") = 0, pybind11::arg("w_tiled") = false,
         pybind11::arg("stages") = 3);
+  m.def("gemm_mid", &gemm_mid, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("y"), pybind11::arg("bias") = pybind11::none(),
+        pybind11::arg("partial") = pybind11::none(), pybind11::arg("splits") = 1, pybind11::arg("silu_gu") = 0);
   m.def("gemm_tile", &gemm_tile, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("y"),
         pybind11::arg("bias") = pybind11::none(), pybind11::arg("silu_gu") = 0, pybind11::arg("variant") = 0,
         pybind11::arg("splits") = 1, pybind11::arg("partial") = pybind11::none());

@@ -1,0 +1,276 @@
+// GEMM for a few hundred rows: Y[M, N] = X[M, K] . W[N, K]^T, bf16 in, fp32 accumulate, bf16 out -- the
+// projections of one or a few prompts, and vocabularies of up to 128 rows.
+//
+// What bounds it: not the matrix cores but the CUs a launch keeps busy. The 256 x 256 tiles of gemm_tile make 64
+// workgroups of an 885 x 4096 product, each walking the whole K at 1.3 us per 64 columns. Here a tile is 128 x 256
+// and its K may be cut into S slices (fp32 slabs, summed by the consumer or by a reduce pass), so that
+// M N S / 32768 workgroups come close to one per CU:
+//   885 rows (weights from HBM)   4096 x 14336: 297 -> 103 us, 4096 x 4096: 88 -> 36, 6144 x 4096: 89 -> 56
+//   100 rows                      279 -> 30, 85 -> 16, 85 -> 19
+//   vocabulary 128256 x 8192, 64 rows: 422 -> 373 us (5.6 TB/s of weights)
+// A 128 x 256 step is 0.7 us (0.43 of MFMA at 2.4 GHz): a CU takes in 50 to 75 bytes per ns through LDS-DMA however
+// many stages wait (a fourth stage of a 64-row tile gained nothing). With every CU busy for several rounds it is
+// 0.85 us, 1.2 PFLOP/s against 1.45 of the 256-row tiles, so those keep the large products (ops.mid_plan).
+//
+// Why this shape: four waves, one per SIMD, 64 x 128 outputs each in 128 AGPRs, so a step's fragment reads (96 KiB)
+// stay below its MFMA time; three 48 KiB stages leave two steps in flight behind one barrier per step; each stage is
+// refilled as soon as its k-half 1 is in registers. 128-B rows with the chunk swizzle slot ^ (bit1(row) << 1 |
+// bit3(row) << 2) read without bank conflicts; W fragments take interleaved feature rows, so a lane ends with 8
+// neighbouring features: 16-B stores. A workgroup walks its units (tile, slice) in one continuous LDS-DMA stream:
+// the next unit's first stages load while this one's outputs are stored.
+#include "common.h"
+#include "kernels.h"
+
+namespace oamd {
+
+namespace {
+
+constexpr int kBM = 128, kBN = 256;   // tile rows, columns
+constexpr int kBK = 64;      // K per step: one 128-B line per row
+constexpr int kGroupM = 8;   // row tiles that share a W panel before the next one
+
+enum { kEpiStore = 0, kEpiBias = 1, kEpiGlu = 2, kEpiPartial = 3 };   // partial: fp32 slab [M][N] of a K slice
+
+template <int N>
+__device__ __forceinline__ void vm_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// accumulator tied in AGPRs (the builtin makes hipcc copy accumulators between the files)
+__device__ __forceinline__ void mfma_tied(f32x4& acc, const u16x8& a, const u16x8& b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+
+// act(gate) * up in the numerics of the other fused epilogues: gate, up and act(gate) rounded to bf16
+__device__ __forceinline__ f32x4 glu4(const f32x4& gate, const f32x4& up, const GluAct& act) {
+  f32x4 o;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) o[r] = bf2f(f2bf(glu_gate(bf2f(f2bf(gate[r])), act))) * bf2f(f2bf(up[r]));
+  return o;
+}
+
+__device__ __forceinline__ void add_bias(const bf16_t* b, f32x4& v0, f32x4& v1) {
+  const u16x8 bb = *reinterpret_cast<const u16x8*>(b);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    v0[r] += bf2f(bb[r]);
+    v1[r] += bf2f(bb[4 + r]);
+  }
+}
+
+__device__ __forceinline__ void store8(bf16_t* y, const f32x4& v0, const f32x4& v1) {
+  *reinterpret_cast<uint4*>(y) = make_uint4(pack_bf2(v0[0], v0[1]), pack_bf2(v0[2], v0[3]), pack_bf2(v1[0], v1[1]), pack_bf2(v1[2], v1[3]));
+}
+
+}  // namespace
+
+template <int EPI>
+__global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
+                                                       bf16_t* __restrict__ Y, const bf16_t* __restrict__ bias,
+                                                       float* __restrict__ P, int M, int N, int K, int ldy, int S, GluAct act) {
+  constexpr int AUX = 16;
+  constexpr int MI = kBM / 32;                   // X fragments of a wave = its X pieces per step
+  constexpr int NP = MI + 8;                     // LDS-DMA pieces of a wave per step
+  constexpr int NS = 3;                          // stages: 144 KiB
+  constexpr int kX = kBM * 128, kStage = kX + kBN * 128;
+  __shared__ __attribute__((aligned(1024))) char lds[NS * kStage];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = w >> 1, wn = w & 1;
+  const int mt = (M + kBM - 1) / kBM, nt = (N + kBN - 1) / kBN, tiles = mt * nt;
+  const int units = tiles * S, G = gridDim.x;
+  const int slot = xcd_remap(blockIdx.x, G);
+  const int TK = K / kBK, gsz = kGroupM * nt;
+
+  auto swz = [](int row) { return (((row >> 1) & 1) << 1) | (((row >> 3) & 1) << 2); };
+  const int lrow = lane >> 3, lslot = lane & 7;
+  uint32_t vo[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int row = 8 * (w + 4 * q) + lrow;
+    vo[q] = ((uint32_t)row * (uint32_t)K + (uint32_t)((lslot ^ swz(row)) * 8)) * 2u;
+  }
+  // unit u = K slice u / tiles of tile u % tiles: first row, first column, first step, steps (slices differ by at most one)
+  auto unit = [&](int u, int& m0, int& n0, int& kz, int& t0, int& T) {
+    const int tile = u % tiles;
+    kz = u / tiles;
+    t0 = kz * TK / S;
+    T = (kz + 1) * TK / S - t0;
+    const int first_m = (tile / gsz) * kGroupM, gm = min(mt - first_m, kGroupM);
+    m0 = (first_m + (tile % gsz) % gm) * kBM;
+    n0 = ((tile % gsz) / gm) * kBN;
+  };
+  // the (unit, step) whose pieces go out next; an operand tile is a buffer resource (rows past M / N
+  // read as zeros). Past the block's last unit its last step is loaded again, into free stages.
+  int cu = slot, ck, cT;
+  const bf16_t *cxp, *cwp;
+  int cxn, cwn;
+  auto point = [&](int u) {
+    int m0, n0, kz, t0;
+    unit(u, m0, n0, kz, t0, cT);
+    cxp = X + (int64_t)m0 * K + t0 * kBK;
+    cwp = W + (int64_t)n0 * K + t0 * kBK;
+    cxn = (int)((uint32_t)min(M - m0, kBM) * (uint32_t)K * 2u - (uint32_t)t0 * (kBK * 2));
+    cwn = (int)((uint32_t)min(N - n0, kBN) * (uint32_t)K * 2u - (uint32_t)t0 * (kBK * 2));
+    ck = 0;
+  };
+  auto advance = [&]() {
+    if (++ck < cT) return;
+    if (cu + G < units) point(cu += G);
+    else ck = cT - 1;
+  };
+  auto dma_ = [&](const bf16_t* cp, int cn, int step, int off, int q) {
+    char* dst = lds + off + (w + 4 * q) * 1024;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)cp, (short)0, cn, 0x00020000),
+                                             (__attribute__((address_space(3))) void*)dst, 16, (int)vo[q], step * (kBK * 2), 0, AUX);
+  };
+  // piece p of the cursor's step into stage `off`: W first (it comes from further away)
+  auto dma = [&](int off, int p) {
+    if (p < 8) dma_(cwp, cwn, ck, off + kX, p);
+    else dma_(cxp, cxn, ck, off, p - 8);
+  };
+
+  const int l15 = lane & 15, lq = lane >> 4;
+  const int xs = swz(l15), wr = 8 * (l15 >> 2) + (l15 & 3), ws = swz(wr);
+  const int xb0 = (wm * (kBM / 2) + l15) * 128, wb0 = kX + (wn * 32 + wr) * 128;
+  const int xo[2] = {xb0 + ((lq ^ xs) << 4), xb0 + (((4 + lq) ^ xs) << 4)};
+  const int wo[2] = {wb0 + ((lq ^ ws) << 4), wb0 + (((4 + lq) ^ ws) << 4)};
+  // read f of a k-half: the X fragments, then the W ones (j = f-block * 4 + gate|up half * 2 + jj)
+  auto rd = [&](int off, int h, u16x8 (&xf)[MI], u16x8 (&wf)[8], int f) {
+    if (f < MI) {
+      xf[f] = *reinterpret_cast<const u16x8*>(lds + off + xo[h] + f * 2048);
+    } else if (f < MI + 8) {
+      const int j = f - MI, r = (j >> 2) * 128 + ((j >> 1) & 1) * 64 + (j & 1) * 4;
+      wf[j] = *reinterpret_cast<const u16x8*>(lds + off + wo[h] + r * 128);
+    }
+  };
+
+  f32x4 acc[MI][8];
+  auto clear = [&]() {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        asm volatile("" : "+a"(acc[i][j]));
+      }
+    asm volatile("s_nop 4");
+  };
+  clear();
+
+  point(slot);
+#pragma unroll
+  for (int st = 0; st < NS; ++st) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p) dma(st * kStage, p);
+    advance();
+  }
+  vm_wait<(NS - 1) * NP>();
+  __builtin_amdgcn_s_barrier();
+  u16x8 xa[MI], wa[8], xb[MI], wb[8];
+#pragma unroll
+  for (int f = 0; f < NP; ++f) rd(0, 0, xa, wa, f);
+
+  int off = 0;       // this step's stage
+  int relax = 0;     // steps whose wait may leave a whole tile's stores in flight behind the pieces
+  constexpr int kStores = MI * (EPI == kEpiGlu ? 2 : EPI == kEpiPartial ? 8 : 4);
+  for (int u = slot; u < units; u += G) {
+    int m0, n0, kz, t0, T;
+    unit(u, m0, n0, kz, t0, T);
+    for (int t = 0; t < T; ++t) {
+      const int nxt = off + kStage == NS * kStage ? 0 : off + kStage;
+      // k-half 0; the reads of k-half 1 ride on its first MFMAs
+#pragma unroll
+      for (int v = 0; v < 8 * MI; ++v) {
+        mfma_tied(acc[v % MI][v / MI], wa[v / MI], xa[v % MI]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (v < NP) rd(off, 1, xb, wb, v);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // k-half 1: after its first quarter every wave has read this stage and the next step has landed;
+      // then the step NS ahead goes into this stage and the next step's first reads ride along
+#pragma unroll
+      for (int v = 0; v < 8 * MI; ++v) {
+        if (v == 2 * MI) {
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          if (relax > 0) {
+            vm_wait<(NS - 2) * NP + kStores>();
+            --relax;
+          } else {
+            vm_wait<(NS - 2) * NP>();
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          __builtin_amdgcn_s_barrier();
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        mfma_tied(acc[v % MI][v / MI], wb[v / MI], xb[v % MI]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (v >= 2 * MI) {
+          const int q = v - 2 * MI;
+          if (q & 1) dma(off, q >> 1);   // 24 slots: 12 reads, 12 pieces
+          else rd(nxt, 0, xa, wa, q >> 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      advance();
+      off = nxt;
+    }
+
+    asm volatile("s_nop 7\n s_nop 7\n s_nop 7" ::: "memory");
+    // a lane holds features 8 lq .. + 7 of each 32-feature block (fragments jj = 0, 1) of token l15
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const int tok = m0 + wm * (kBM / 2) + i * 16 + l15;
+#pragma unroll
+      for (int f = 0; f < 2; ++f) {
+        if constexpr (EPI == kEpiGlu) {
+          f32x4 o[2];
+#pragma unroll
+          for (int jj = 0; jj < 2; ++jj) o[jj] = glu4(acc[i][f * 4 + jj], acc[i][f * 4 + 2 + jj], act);
+          const int col = (n0 >> 1) + f * 64 + wn * 32 + 8 * lq;
+          if (tok < M && 2 * col < N) store8(Y + (int64_t)tok * ldy + col, o[0], o[1]);
+        } else {
+#pragma unroll
+          for (int ty = 0; ty < 2; ++ty) {
+            f32x4 v0 = acc[i][f * 4 + ty * 2], v1 = acc[i][f * 4 + ty * 2 + 1];
+            const int col = n0 + f * 128 + ty * 64 + wn * 32 + 8 * lq;
+            if (tok >= M || col >= N) continue;
+            if constexpr (EPI == kEpiPartial) {
+              float* pr = P + ((int64_t)kz * M + tok) * N + col;
+              *reinterpret_cast<f32x4*>(pr) = v0;
+              *reinterpret_cast<f32x4*>(pr + 4) = v1;
+            } else {
+              if constexpr (EPI == kEpiBias) add_bias(bias + col, v0, v1);
+              store8(Y + (int64_t)tok * ldy + col, v0, v1);
+            }
+          }
+        }
+      }
+    }
+    // a whole tile issued kStores stores: the next waits count past them
+    relax = m0 + kBM <= M && n0 + kBN <= N ? NS - 1 : 0;
+    clear();
+  }
+  vm_wait<0>();   // the trailing re-loads land before the workgroup's LDS is released
+}
+
+int gemm_mid(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, float* P, int M, int N, int K, int ldy, int glu,
+             int S, hipStream_t stream) {
+  if (M < 1 || N < 16 || N % 16 || K % kBK || S < 1 || S > 16 || K / kBK < S) return -1;
+  if (glu && (N % 128 || bias)) return -2;
+  if (S > 1 && (P == nullptr || bias)) return -3;
+  if (Y == nullptr ? (S == 1 || glu) : (ldy % 8 || reinterpret_cast<uintptr_t>(Y) % 16)) return -4;
+  if (S > 1 && Y != nullptr && ldy != (glu ? N / 2 : N)) return -5;
+  const int64_t units = (int64_t)((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN) * S;
+  if (units > (1LL << 30)) return -6;
+  const int grid = (int)min((int64_t)device_cus(), units);
+  if (S > 1) gemm_mid_kernel<kEpiPartial><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, GluAct{});
+  else if (glu) gemm_mid_kernel<kEpiGlu><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, glu_act(glu));
+  else if (bias) gemm_mid_kernel<kEpiBias><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, GluAct{});
+  else gemm_mid_kernel<kEpiStore><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, GluAct{});
+  OAMD_LAUNCH_CHECK();
+  if (S == 1 || Y == nullptr) return 0;
+  return glu ? splitk_silu(P, Y, M, N, S, glu, stream) : splitk_reduce(P, Y, (int64_t)M * N, S, stream);
+}
+
+}  // namespace oamd

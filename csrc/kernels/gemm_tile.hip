@@ -931,7 +931,7 @@ static void launch_p5(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t*
 }
 
 // compute units of the current device (persistent grids), cached per device
-static int device_cus() {
+int device_cus() {
   static int cus[16] = {0};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) dev = 0;

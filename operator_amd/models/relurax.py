@@ -205,7 +205,8 @@ class ReluraxModel(PaddedModel):
 
     def _window_mixer(self, i: int, lw: ReluraxLayer, h, edges, fb: ForwardBatch, kv: PagedKVCache, ws):
         a, L, cache = self.cfg.layer_specs[i].mixer, self.shapes[i], kv.layer(i)
-        q, k, v, gate = dec.conv_heads(ops.linear(h, lw.win, defer_reduce=True), fb.positions, L, self.dtype, lw.conv, lw.qnorm,
+        # a prefill reads every row once per tap: whole rows, not slabs
+        q, k, v, gate = dec.conv_heads(ops.linear(h, lw.win, defer_reduce=not fb.is_prefill), fb.positions, L, self.dtype, lw.conv, lw.qnorm,
                                        lw.knorm, cache, kv.state[i], fb.slots, edges)
         if fb.is_prefill:
             o = self._prefill(i, q, k, v, gate, fb, L, a.window)

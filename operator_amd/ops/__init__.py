@@ -6,6 +6,7 @@ reference implementations in :mod:`operator_amd.ops.reference`.
 """
 from __future__ import annotations
 
+import functools
 import json
 import os
 
@@ -384,6 +385,16 @@ def skinny_plan(M: int, N: int, K: int) -> int | None:
     return S
 
 
+def _mid_beats_skinny(M: int, N: int, K: int, defer: bool) -> bool:
+    """gemm_skinny streams the weights once per call but pays for every row (a 128256 x 4096 vocabulary: 199 us at
+    1 row, 242 at 8, 440 at 32; 4 % of the one-row time per row at every measured shape); gemm_mid's 128-row
+    tile costs the same at any of them (217 us). A few rows of a projection stay: too little work to split."""
+    if M <= (4 if N >= LM_HEAD_MIN_N else 16):
+        return False
+    S = mid_plan(M, N, K, defer)
+    return S is not None and _mid_cost(M, N, K, S, defer) < (3 + 2e-6 * N * K / 5.4) * (1 + 0.04 * M)
+
+
 # Every GPU GEMM of the model runs on the hand-written gfx950 kernels: prefill projections (M > 256
 # rows) on gemm_tile's persistent p5 schedule (csrc/kernels/gemm_tile.hip), decode buckets on
 # gemm_pp / gemm_tn / gemm_skinny, the lm_head on gemm_tile, fp8 on gemm_fp8. hipBLASLt is reached
@@ -424,14 +435,72 @@ def tile_out_ok(out: torch.Tensor | None) -> bool:
                            and out.data_ptr() % 8 == 0 and out.dtype == torch.bfloat16)
 
 
+# Costs, in us, of the two bf16 tile kernels on one MI355X with weights that stream from HBM (measured on
+# 48 to 6144 rows of 2048 to 28672 x 2048 to 14336 weights): a step is one 64-column piece of K on every
+# busy CU, dearer with the whole chip busy (clock, L2) and where no two workgroups share a weight panel.
+CUS = 256
+
+
+def _tile_cost(M: int, N: int, K: int) -> float:
+    """gemm_tile: 256 x 256 tiles over the whole K, one workgroup per CU."""
+    units = -(-M // 256) * -(-N // 256)
+    return max(3 + -(-units // CUS) * (K // 64) * (1.25 + 0.2 * min(1.0, units / CUS)), 2e-6 * N * K / 4.6)
+
+
+def _mid_cost(M: int, N: int, K: int, S: int, defer: bool) -> float:
+    """gemm_mid: 128 x 256 tiles, K in S slices whose slabs are written, then read by a reduce pass or (``defer``) by
+    the consumer."""
+    mt = -(-M // 128)
+    units = mt * -(-N // 256) * S
+    rounds = -(-units // CUS)
+    step = 0.7 + 0.15 * min(1.0, units / CUS) + (0.12 if mt == 1 else 0.0)
+    t = 4 + rounds * -(-(K // 64) // S) * step + 3 * (rounds - 1)   # a tile's stores between rounds
+    if S > 1:
+        t += S * M * N * 4e-6 * (1 / 4 + 1 / 5) + (0 if defer else 6)
+    return max(t, 2e-6 * N * K / 4.9)
+
+
+@functools.lru_cache(maxsize=4096)
+def mid_plan(M: int, N: int, K: int, defer: bool, slices: bool = True) -> int | None:
+    """K slices for gemm_mid (1: none), or None where the 256-row tiles are cheaper. One prompt of a few hundred
+    tokens has fewer 256-row tiles than the GPU has CUs: smaller tiles and K slices fill it (885 rows: 4096 x 14336
+    103 us against 297, 6144 x 4096 56 against 89); once every CU has a 256-row tile, that tile's fewer operand
+    bytes per product win (4096 rows of 4096 x 14336: 325 us against 371).
+
+    Above 256 rows the plan is the next multiple of 512's: a prefill graph pads its batch to such a size, and a
+    prompt's numbers are the same padded or not. Past 4096 rows the graphs' sizes are coarser and little is left
+    to gain."""
+    if M > 256:
+        M = -(-M // 512) * 512
+    if M < 1 or M > 4096 or K < 128 or (M > 128 and N >= LM_HEAD_MIN_N):   # 256 rows of a vocabulary: 282 us against 253
+        return None
+    tiles = -(-M // 128) * -(-N // 256)
+    most = min(16, K // 128, 2 * CUS // tiles) if slices else 1
+    cost, S = min((_mid_cost(M, N, K, s, defer), s) for s in range(1, max(1, most) + 1))
+    return S if cost < _tile_cost(M, N, K) else None
+
+
 def linear_tile(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None,
-                bias: torch.Tensor | None = None, glu: int = 0) -> torch.Tensor:
-    """Prefill / lm_head GEMM on the compute-bound gfx950 tile kernel (256 x 256 tiles,
-    LDS-DMA ping-pong pipeline; fused bias or gated (``glu``: SILU / GELU_TANH) epilogue)."""
-    M = x.shape[0]
+                bias: torch.Tensor | None = None, glu: int = 0, defer_reduce: bool = False):
+    """Prefill / lm_head GEMM on the compute-bound gfx950 tile kernels (fused bias or gated (``glu``: SILU /
+    GELU_TANH) epilogue): 128 x 256 tiles with K slices for few rows (``mid_plan``), else 256 x 256 tiles (LDS-DMA
+    ping-pong pipeline). ``defer_reduce``: K slices come back as fp32 slabs (:class:`SplitK`)."""
+    M, K = x.shape
     N = w.shape[0]
+    defer = defer_reduce and out is None and bias is None and not glu
+    S = None
+    if (out is None or (out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0)) and (
+            bias is None or (bias.is_contiguous() and bias.data_ptr() % 16 == 0)):   # gemm_mid's 16-B accesses
+        S = mid_plan(M, N, K, defer, bias is None and (out is None or out.is_contiguous()))
+    part = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if S is not None and S > 1 else None
+    if part is not None and defer:
+        kernels().gemm_mid(x, w, None, None, part, S)
+        return SplitK(part, S, M, N)
     y = out if out is not None else torch.empty(M, N // 2 if glu else N, dtype=x.dtype, device=x.device)
-    kernels().gemm_tile(x, w, y, bias, glu)
+    if S is not None:
+        kernels().gemm_mid(x, w, y, bias, part, S, glu)
+    else:
+        kernels().gemm_tile(x, w, y, bias, glu)
     return y
 
 
@@ -474,6 +543,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, sp
     if (x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous() and M <= SKINNY_MAX_M
             and bm is None and bn is None):
         S = splits or skinny_plan(M, N, K)
+        if S is not None and splits is None and out is None and tile_ok(x, w) and _mid_beats_skinny(M, N, K, defer_reduce):
+            return linear_tile(x, w, defer_reduce=defer_reduce)
         if S is not None:
             if S > 1 and (partial is None or partial.numel() < S * M * N):
                 partial = torch.empty(S * M * N, dtype=torch.float32, device=x.device)
@@ -489,7 +560,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, sp
             plan = (row_tile(M), 64, 1)  # explicit request (tests / tuning)
     if plan is None:
         if tile_ok(x, w) and tile_out_ok(out):
-            return linear_tile(x, w, out)
+            return linear_tile(x, w, out, defer_reduce=defer_reduce)
         return _blas(x, w, out, None)
     bm, bn, S = bm or plan[0], bn or plan[1], splits or plan[2]
     ns = stages or (plan[3] if len(plan) > 3 else 3)

@@ -1,0 +1,71 @@
+"""gemm_mid (128 x 256 tiles, K slices): tails, every epilogue, slices by the reduce pass and by the consumer, several
+rounds of tiles per workgroup, against fp64; and the plan that chooses it."""
+import pytest
+import torch
+
+from operator_amd import ops
+from operator_amd.ops import reference as ref
+
+DEV = "cuda"
+
+
+def _rand(*shape, scale=1.0):
+    return (torch.randn(*shape, device=DEV) * scale).to(torch.bfloat16)
+
+
+def _check(y, r, mag, K, extra=0.0):
+    """bf16 rounding of the result (2^-8 of it) plus fp32 accumulation (K 2^-24 of the sum of magnitudes)."""
+    assert ((y.double() - r).abs() <= (2.0 ** -8 + extra) * r.abs() + K * 2.0 ** -24 * mag + 1e-30).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,S", [
+    (1, 16, 64, 1), (127, 272, 128, 2), (128, 256, 192, 3), (129, 528, 1024, 5), (300, 4096, 2048, 16), (885, 4096, 1088, 2),
+    (700, 16384, 128, 1), (700, 16400, 192, 1), (2300, 8192, 64, 1), (130, 48000, 128, 2)])
+def test_gemm_mid(M, N, K, S):
+    torch.manual_seed(M + N + K)
+    x, w, b = _rand(M, K), _rand(N, K, scale=0.05), _rand(N, scale=0.5)
+    r, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    nan = lambda *s, dt=torch.float32: torch.full(s, float("nan"), dtype=dt, device=DEV)  # noqa: E731
+    y = nan(M, N, dt=torch.bfloat16)
+    ops.kernels().gemm_mid(x, w, y, None, nan(S, M, N), S)
+    _check(y, r, mag, K)
+    if S > 1:
+        slabs = nan(S, M, N)
+        ops.kernels().gemm_mid(x, w, None, None, slabs, S)
+        assert ((slabs.double().sum(0) - r).abs() <= K * 2.0 ** -24 * mag).all()
+        return
+    ops.kernels().gemm_mid(x, w, y, b)
+    _check(y, r + b.double(), mag + b.double().abs(), K)
+    wide = nan(M, N + 64, dt=torch.bfloat16)
+    ops.kernels().gemm_mid(x, w, wide[:, 32:32 + N])
+    _check(wide[:, 32:32 + N], r, mag, K)
+    assert wide[:, :32].isnan().all() and wide[:, 32 + N:].isnan().all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", [ops.SILU, ops.GELU_TANH])
+@pytest.mark.parametrize("M,inter,K,S", [(33, 128, 128, 2), (200, 8192, 192, 1), (520, 8256, 256, 1)])
+def test_gemm_mid_gated(M, inter, K, S, act):
+    torch.manual_seed(M + K)
+    x, g, u = _rand(M, K), _rand(inter, K, scale=0.05), _rand(inter, K, scale=0.05)
+    y = torch.full((M, inter), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.kernels().gemm_mid(x, ops.interleave_gate_up(g, u), y, None, torch.empty(S, M, 2 * inter, device=DEV), S, act)
+    gate, up = ((x.double() @ w.double().t()).to(torch.bfloat16) for w in (g, u))
+    r = ref.silu_mul(torch.cat([gate, up], 1), None, act == ops.GELU_TANH).double()
+    # each of gate, act(gate) and up may round the other way (2^-8; the activation's slope is below 1.2),
+    # and a gate near 0 carries its absolute error
+    assert ((y.double() - r).abs() <= 5 * 2.0 ** -8 * r.abs() + 2.0 ** -8 * 1.2 * up.double().abs() * gate.double().abs() + 1e-6).all()
+
+
+def test_mid_plan_is_launchable():
+    """Every plan is one gemm_mid takes, padded batches keep their plan, large products keep the 256-row tiles."""
+    for N, K in ((16, 128), (272, 192), (4096, 4096), (4096, 14336), (28672, 4096), (128256, 4096), (151936, 2048)):
+        for defer in (False, True):
+            for M in (1, 2, 31, 33, 127, 128, 129, 257, 885, 2047, 4096, 9999, 28000):
+                S = ops.mid_plan(M, N, K, defer)
+                assert S is None or 1 <= S <= min(16, K // 64)
+                assert ops.mid_plan(M, N, K, defer, False) in (None, 1)
+            assert ops.mid_plan(322, N, K, defer) == ops.mid_plan(512, N, K, defer)
+    assert ops.mid_plan(28000, 4096, 14336, True) is None
+    assert ops.mid_plan(885, 4096, 14336, True) == 2
