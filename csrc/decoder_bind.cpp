@@ -231,23 +231,22 @@ void attn_gd_prefill(const at::Tensor& q, const at::Tensor& k, const at::Tensor&
     need(*seq_pfx, at::kInt, seqs, "seq_pfx");
   }
   const c10::hip::HIPGuardMasqueradingAsCUDA g(q.device());
+  TORCH_CHECK(work_seq.has_value() && work_q0.has_value(), "attn_gd_prefill: work list");
+  need(*work_seq, at::kInt, work_seq->numel(), "work_seq");
+  need(*work_q0, at::kInt, work_seq->numel(), "work_q0");
   if (f32) {
     oamd::AttnF32 a{};
     a.q = p<float>(q); a.k = p<float>(k); a.v = p<float>(v); a.o = p<float>(o);
     a.o_ld = (int)o.size(1);
-    a.cu_seqlens = p<int>(cu);
-    a.num_seqs = (int)seqs;
+    a.cu_seqlens = p<int>(cu); a.work_seq = p<int>(*work_seq); a.work_q0 = p<int>(*work_q0);
     a.Hkv = (int)Hkv; a.dkp = (int)dkp; a.dvp = (int)dvp;
     a.k_ld = dkp; a.v_ld = dvp;
     a.window = win; a.gate = op<float>(gate);
     a.scale = (float)scale;
     a.pk = op<float>(pk); a.pv = op<float>(pv); a.seq_pfx = op<int>(seq_pfx);
-    RC(oamd::attn_f32(a, (int)T, (int)Hq, false, cur_stream()));
+    RC(oamd::attn_f32_prefill(a, (int)work_seq->numel(), (int)Hq, cur_stream()));
     return;
   }
-  TORCH_CHECK(work_seq.has_value() && work_q0.has_value(), "attn_gd_prefill: work list");
-  need(*work_seq, at::kInt, work_seq->numel(), "work_seq");
-  need(*work_q0, at::kInt, work_seq->numel(), "work_q0");
   oamd::AttnPrefill a{};
   a.q = p<bf16_t>(q); a.k = p<bf16_t>(k); a.v = p<bf16_t>(v); a.o = p<bf16_t>(o);
   a.o_ld = (int)o.size(1);
@@ -282,6 +281,11 @@ void attn_gd_decode(const at::Tensor& q, const at::Tensor& k_cache, const at::Te
                   Hq % Hkv == 0 && o.size(1) >= Hq * dvp && P >= 16 && (P & (P - 1)) == 0 && num_splits >= 1,
               "attn_gd_decode: shapes");
   if (gate.has_value()) need(*gate, at::kFloat, B * Hq, "gate");
+  if (num_splits > 1) {
+    TORCH_CHECK(o_part.has_value() && ml_part.has_value(), "attn_gd_decode: workspace");
+    need(*o_part, at::kFloat, B * Hq * num_splits * dvp, "o_part", true);
+    need(*ml_part, at::kFloat, B * Hq * num_splits * 2, "ml_part", true);
+  }
   const int win = window_of(window);
   const c10::hip::HIPGuardMasqueradingAsCUDA g(q.device());
   if (f32) {
@@ -294,7 +298,7 @@ void attn_gd_decode(const at::Tensor& q, const at::Tensor& k_cache, const at::Te
     a.k_ld = dkp; a.v_ld = dvp;
     a.window = win; a.gate = op<float>(gate);
     a.scale = (float)scale;
-    RC(oamd::attn_f32(a, (int)B, (int)Hq, true, cur_stream()));
+    RC(oamd::attn_f32_decode(a, (int)B, (int)Hq, (int)num_splits, op<float>(o_part), op<float>(ml_part), cur_stream()));
     return;
   }
   oamd::AttnDecode a{};
@@ -303,9 +307,6 @@ void attn_gd_decode(const at::Tensor& q, const at::Tensor& k_cache, const at::Te
   a.out = p<bf16_t>(o);
   a.o_ld = (int)o.size(1);
   if (num_splits > 1) {
-    TORCH_CHECK(o_part.has_value() && ml_part.has_value(), "attn_gd_decode: workspace");
-    need(*o_part, at::kFloat, B * Hq * num_splits * dvp, "o_part", true);
-    need(*ml_part, at::kFloat, B * Hq * num_splits * 2, "ml_part", true);
     a.o_part = p<float>(*o_part); a.ml_part = p<float>(*ml_part);
   }
   a.Hkv = (int)Hkv; a.G = (int)(Hq / Hkv); a.dkp = (int)dkp; a.dvp = (int)dvp;
@@ -335,6 +336,11 @@ void attn_latent_decode(const at::Tensor& q, const at::Tensor& cache, const at::
   need(o, dt, B * H * rp, "o");
   TORCH_CHECK(P >= 16 && (P & (P - 1)) == 0 && num_splits >= 1 && rp >= 16 && rp % 16 == 0 && rp <= ck, "attn_latent_decode: shapes");
   if (gate.has_value()) need(*gate, at::kFloat, B * H, "gate");
+  if (num_splits > 1) {
+    TORCH_CHECK(o_part.has_value() && ml_part.has_value(), "attn_latent_decode: workspace");
+    need(*o_part, at::kFloat, B * H * num_splits * rp, "o_part", true);
+    need(*ml_part, at::kFloat, B * H * num_splits * 2, "ml_part", true);
+  }
   const c10::hip::HIPGuardMasqueradingAsCUDA g(q.device());
   if (f32) {
     oamd::AttnF32 a{};
@@ -345,7 +351,7 @@ void attn_latent_decode(const at::Tensor& q, const at::Tensor& cache, const at::
     a.page_size = (int)P; a.max_pages = (int)bt.size(1);
     a.scale = (float)scale;
     a.window = oamd::kNoWindow; a.gate = op<float>(gate);
-    RC(oamd::attn_f32(a, (int)B, (int)H, true, cur_stream()));
+    RC(oamd::attn_f32_decode(a, (int)B, (int)H, (int)num_splits, op<float>(o_part), op<float>(ml_part), cur_stream()));
     return;
   }
   oamd::AttnDecode a{};
@@ -354,9 +360,6 @@ void attn_latent_decode(const at::Tensor& q, const at::Tensor& cache, const at::
   a.out = p<bf16_t>(o);
   a.o_ld = (int)(H * rp);
   if (num_splits > 1) {
-    TORCH_CHECK(o_part.has_value() && ml_part.has_value(), "attn_latent_decode: workspace");
-    need(*o_part, at::kFloat, B * H * num_splits * rp, "o_part", true);
-    need(*ml_part, at::kFloat, B * H * num_splits * 2, "ml_part", true);
     a.o_part = p<float>(*o_part); a.ml_part = p<float>(*ml_part);
   }
   a.Hkv = 1; a.G = (int)H; a.dkp = (int)ck; a.dvp = (int)rp;
@@ -563,7 +566,8 @@ void head_gemm(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, int64_t 
   RC(oamd::head_gemm(a, cur_stream()));
 }
 
-void gemm_f32(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, int64_t silu_gu, const OptT& gtab, const OptT& rscale) {
+void gemm_f32(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, int64_t silu_gu, const OptT& gtab, const OptT& rscale,
+              const OptT& partial, int64_t splits) {
   TORCH_CHECK(x.dim() == 2 && y.dim() == 2, "gemm_f32: x [M, K], y [M, N]");
   const int64_t M = x.size(0), K = x.size(1), N = w.size(-2);
   need(x, at::kFloat, M * K, "x");
@@ -578,8 +582,13 @@ void gemm_f32(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, int64_t s
   }
   if (rscale.has_value()) need(*rscale, at::kFloat, M, "rscale");
   const c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
-  RC(oamd::gemm_f32(p<float>(x), p<float>(w), p<float>(y), (int)M, (int)N, (int)K, (int)y.size(1), (int)silu_gu,
-                    op<int>(gtab), op<float>(rscale), cur_stream()));
+  TORCH_CHECK(splits >= 1 && splits <= 8, "gemm_f32: splits");
+  if (splits > 1) {
+    TORCH_CHECK(partial.has_value() && !gtab.has_value() && !rscale.has_value() && N % 4 == 0, "gemm_f32: K slices");
+    need(*partial, at::kFloat, splits * M * N, "partial");
+  }
+  RC(oamd::gemm_f32(p<float>(x), p<float>(w), p<float>(y), op<float>(partial), (int)splits, (int)M, (int)N, (int)K, (int)y.size(1),
+                    (int)silu_gu, op<int>(gtab), op<float>(rscale), cur_stream()));
 }
 
 void moe_route(const at::Tensor& h, const at::Tensor& wr, int64_t E, at::Tensor& ids, at::Tensor& weights,
@@ -725,8 +734,9 @@ void register_decoder_bindings(pybind11::module_& m) {
   m.def("rotate_heads", &rotate_heads, py::arg("q"), py::arg("slabs"), py::arg("splits"), py::arg("d"), py::arg("rot"),
         py::arg("pos"), py::arg("cos"), py::arg("sin"));
   m.def("head_gemm", &head_gemm, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("x0") = 0, py::arg("nx") = 0);
+  m.def("gemm_f32_splits", &oamd::gemm_f32_splits, py::arg("M"), py::arg("N"), py::arg("K"), py::arg("glu"));
   m.def("gemm_f32", &gemm_f32, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("silu_gu") = 0,
-        py::arg("gtab") = no, py::arg("rscale") = no);
+        py::arg("gtab") = no, py::arg("rscale") = no, py::arg("partial") = no, py::arg("splits") = 1);
   m.def("moe_route", &moe_route, py::arg("h"), py::arg("wr"), py::arg("E"), py::arg("ids"), py::arg("weights"),
         py::arg("gate") = no, py::arg("logits") = no);
   m.def("moe_topk", &moe_topk, py::arg("logits"), py::arg("E"), py::arg("ids"), py::arg("weights"), py::arg("gate") = no);

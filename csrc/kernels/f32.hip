@@ -1,221 +1,629 @@
 // True 32-bit forms of the model's products, for models served in fp32 (no reduced-precision
-// matrix mode anywhere): a tiled GEMM (plain, SwiGLU, per-expert row groups) and attention
-// for any head size. Precision first: fp32 FMA on the vector units.
+// matrix mode anywhere): GEMMs (plain, gated, per-expert row groups) on the fp32 matrix instruction and attention
+// for any head size.
 #include "common.h"
 #include "kernels.h"
 
 namespace oamd {
 
-// Y[M, N] = X[M, K] W[N, K]^T, 64 x 64 tiles, 256 threads x 4 x 4 outputs.
-// SILU: W holds gate | up rows interleaved in 64-row blocks; a tile is 64 features, Y [M, N/2]
-// = silu(c g) * (c u) with c the row's scale (rscale, or 1).
+namespace {
+
+// Rows the skinny kernel runs: one 16-row fragment streams W best (1 row of 2048 x 8192: 26 us); with two the
+// repeated rows cost more than K slices of the tile kernel do (33 rows 33 us, 32 rows 55 skinny), unless K is
+// too short to cut (32 rows of 1536 x 768: 9 us against 14).
+inline bool skinny_rows(int M, int K) { return M <= 16 || (M <= 32 && K < 2048); }
+
+constexpr int kStages = 3;   // LDS ring of the tile kernel: two 32-column pieces of K in flight
+
+__device__ __forceinline__ f32x4 mfma4(const f32x4& a, const f32x4& b, f32x4 c) {   // k = 4 (lane / 16) + 0..3 of both
+#pragma unroll
+  for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
+  return c;
+}
+
+__device__ __forceinline__ float glu1(float g, float u, const GluAct& act) {
+  return g / (1.f + expf(-g * __builtin_fmaf(act.c, g * g, act.a))) * u;
+}
+
+// 4 neighbouring outputs of a row, n valid ones
+__device__ __forceinline__ void put4(float* y, const f32x4& v, int n, bool vec) {
+  if (n >= 4 && vec) {
+    *reinterpret_cast<f32x4*>(y) = v;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (e < n) y[e] = v[e];
+  }
+}
+
+}  // namespace
+
+struct GemmF32 {
+  const float *X, *W;
+  float *Y, *P;          // P: slabs [S][M][N] of S > 1 K slices
+  int M, N, K, S;
+  int64_t ldx, ldy, xh, yh;   // row strides; head strides of X and Y (one product per head, W [H][N][K])
+  const int* gtab;
+  const float* rscale;
+  GluAct act;
+  int vec;               // Y takes 16-B stores
+};
+
+// Y[M, N] = X[M, K] W[N, K]^T in fp32 on the fp32 matrix instruction (full 32-bit products and sums), 64 x 64
+// tiles, four waves of 32 x 32 outputs in 16 x 16 blocks.
+// What bounds it: the fp32 MFMA rate, 256 flop per clock and CU (157 TFLOP/s; ordinary FMA reaches half of that without
+// packed fp32, which is off). A 32-column step is 1024 clocks of MFMA against 256 of fragment reads and 128 of LDS-DMA
+// writes, so a plain three-stage ring with two or three workgroups per CU hides the rest. 64 x 64 tiles because products
+// here have few rows (500 rows of 2048 features: 256 tiles) and because routed experts' segments are padded to 64 rows.
+// 1000 rows: 16384 x 2048 gated 905 -> 584 us (115 TFLOP/s), 2048 x 8192 590 -> 313; 18 rows of 2048 x 8192 in eight
+// K slices 1000 -> 33.
+// GLU: W holds gate | up rows interleaved in 64-row blocks; a tile is 64 features, Y [M, N/2]
+// = act(c g) * (c u) with c the row's scale (rscale, or 1).
 // gtab != nullptr: rows are expert segments padded to 64-row tiles; gtab[0] = tile count,
 // gtab[1 + i] = expert of tile i, W [experts][N][K].
-template <bool SILU>
-__global__ void __launch_bounds__(256) gemm_f32_kernel(const float* __restrict__ X, const float* __restrict__ W,
-                                                       float* __restrict__ Y, int M, int N, int K, int ldy,
-                                                       const int* __restrict__ gtab, const float* __restrict__ rscale,
-                                                       GluAct act, int64_t ldx, int64_t xh, int64_t yh) {
-  constexpr int NB = SILU ? 2 : 1;
-  __shared__ float xs[16][64 + 4];
-  __shared__ float ws[NB][16][64 + 4];
-  const int m0 = blockIdx.x * 64, f0 = blockIdx.y * 64;
-  if (gtab) {
-    if ((int)blockIdx.x >= gtab[0]) return;
-    W += (int64_t)gtab[1 + blockIdx.x] * N * K;
+// PART: K slice blockIdx.z of S, raw sums into its slab.
+template <bool GLU, bool PART>
+__global__ void __launch_bounds__(256) gemm_f32_kernel(const GemmF32 a) {
+  constexpr int NB = GLU ? 2 : 1;
+  constexpr int kRows = 64 + 64 * NB, kStage = kRows * 128, GL = kRows / 32;
+  __shared__ __attribute__((aligned(1024))) char lds[kStages * kStage];
+  const int K = a.K;
+  const int lid = xcd_remap(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
+  const int mt = lid % gridDim.x, m0 = mt * 64, f0 = (lid / gridDim.x) * 64;
+  const float *X = a.X, *W = a.W;
+  float* Y = a.Y;
+  if (a.gtab) {
+    if (mt >= a.gtab[0]) return;
+    W += (int64_t)a.gtab[1 + mt] * a.N * a.K;
   }
-  if (blockIdx.z) {   // one product per head
-    X += blockIdx.z * xh;
-    W += (int64_t)blockIdx.z * N * K;
-    Y += blockIdx.z * yh;
+  int kbase = 0, T = (a.K + 31) / 32;
+  if constexpr (PART) {
+    const int t0 = (int)blockIdx.z * T / a.S;
+    T = ((int)blockIdx.z + 1) * T / a.S - t0;
+    kbase = t0 * 32;
+    Y = a.P + (int64_t)blockIdx.z * a.M * a.N;
+  } else if (blockIdx.z) {   // one product per head
+    X += blockIdx.z * a.xh;
+    W += (int64_t)blockIdx.z * a.N * a.K;
+    Y += blockIdx.z * a.yh;
   }
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int lr = tid >> 2, lk = (tid & 3) * 4;   // loader: row, 4 consecutive k
-  float acc[NB][4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    __syncthreads();
-    {
-      f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (m0 + lr < M) v = *reinterpret_cast<const f32x4*>(X + (int64_t)(m0 + lr) * ldx + k0 + lk);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), wm = w >> 1, wn = w & 1;
+
+  // LDS-DMA piece i of this wave: stage rows 8 (w + 4 i) .. +7 (X, then W), lane l -> row + l / 8, 16-B slot l % 8;
+  // the slot holds source chunk slot ^ (row / 2 % 8), which keeps the fragment reads free of bank conflicts.
+  // Rows past M / N repeat the last one, columns past K the row's first (never multiplied).
+  const float* src[GL];
+  int col[GL];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) xs[lk + j][lr] = v[j];
+  for (int i = 0; i < GL; ++i) {
+    const int row = 8 * (w + 4 * i) + (lane >> 3);
+    src[i] = row < 64 ? X + min(m0 + row, a.M - 1) * a.ldx : W + (int64_t)min((GLU ? 2 * f0 : f0) + row - 64, a.N - 1) * a.K;
+    col[i] = 4 * ((lane & 7) ^ ((row >> 1) & 7));
+  }
+  auto issue = [&](int t) {
+    char* base = lds + (t % kStages) * kStage;
+#pragma unroll
+    for (int i = 0; i < GL; ++i) {
+      const int k = kbase + t * 32 + col[i];
+      const float* from = src[i] + (k < K ? k : 0);
+      __builtin_amdgcn_global_load_lds(from, (__attribute__((address_space(3))) void*)(base + (w + 4 * i) * 1024), 16, 0, 0);
     }
+  };
+  const int l15 = lane & 15, g = lane >> 4, sw = (l15 >> 1) & 7;
+  f32x4 acc[NB][2][2] = {};   // [gate | up][feature block][token block]
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const int wr = (SILU ? 2 * f0 + 64 * b : f0) + lr;
-      f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (wr < N) v = *reinterpret_cast<const f32x4*>(W + (int64_t)wr * K + k0 + lk);
+  for (int st = 0; st < kStages - 1; ++st)
+    if (T > st) issue(st);
+  for (int t = 0; t < T; ++t) {
+    if (t + 1 < T) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(GL) : "memory");   // all but the next stage's pieces
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (t + kStages - 1 < T) issue(t + kStages - 1);
+    const char* base = lds + (t % kStages) * kStage;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) ws[b][lk + j][lr] = v[j];
-    }
-    __syncthreads();
+    for (int s = 0; s < 2; ++s) {
+      if (kbase + t * 32 + 16 * s >= a.K) break;
+      const int off = ((4 * s + g) ^ sw) << 4;   // row / 2 % 8 depends on the lane only: blocks are 16 rows
+      f32x4 xf[2], wf[NB][2];
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      float xv[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) xv[i] = xs[k][ty * 4 + i];
+      for (int i = 0; i < 2; ++i) xf[i] = *reinterpret_cast<const f32x4*>(base + (wm * 32 + 16 * i + l15) * 128 + off);
 #pragma unroll
       for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float wv = ws[b][k][tx * 4 + j];
+        for (int j = 0; j < 2; ++j)
+          wf[b][j] = *reinterpret_cast<const f32x4*>(base + (64 + 64 * b + wn * 32 + 16 * j + l15) * 128 + off);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[b][i][j] = __builtin_fmaf(xv[i], wv, acc[b][i][j]);
-        }
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+              acc[b][j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[b][j][e], xf[i][e], acc[b][j][i], 0, 0, 0);
     }
   }
+  // a lane holds features 4 g .. + 3 of each block of token l15
+  const int NO = GLU && !PART ? a.N / 2 : a.N;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty * 4 + i;
-    if (m >= M) continue;
-    const float c = rscale ? rscale[m] : 1.f;
+  for (int i = 0; i < 2; ++i) {
+    const int m = m0 + wm * 32 + 16 * i + l15;
+    if (m >= a.M) continue;
+    const float c = a.rscale ? a.rscale[m] : 1.f;
+    float* yr = Y + m * (PART ? (int64_t)a.N : a.ldy);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = f0 + tx * 4 + j;
-      if (n >= (SILU ? N / 2 : N)) continue;
-      float y = acc[0][i][j];
-      if constexpr (SILU) {
-        const float g = c * y, u = c * acc[NB - 1][i][j];
-        y = g / (1.f + expf(-g * __builtin_fmaf(act.c, g * g, act.a))) * u;
+    for (int j = 0; j < 2; ++j) {
+      const int f = wn * 32 + 16 * j + 4 * g;
+      if constexpr (PART) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const int n = (GLU ? 2 * f0 + 64 * b : f0) + f;
+          put4(yr + n, acc[b][j][i], NO - n, a.N % 4 == 0);
+        }
+      } else {
+        f32x4 v = acc[0][j][i];
+        if constexpr (GLU)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = glu1(c * v[r], c * acc[NB - 1][j][i][r], a.act);
+        put4(yr + f0 + f, v, NO - f0 - f, a.vec);
       }
-      Y[(int64_t)m * ldy + n] = y;
     }
   }
 }
 
-int gemm_f32(const float* X, const float* W, float* Y, int M, int N, int K, int ldy, int glu, const int* gtab,
-             const float* rscale, hipStream_t stream) {
-  if (M == 0) return 0;
-  if (K % 16 || (glu && N % 128)) return -1;
-  const int nf = glu ? N / 2 : N;
-  const dim3 grid((M + 63) / 64, (nf + 63) / 64);
-  if (glu) gemm_f32_kernel<true><<<grid, 256, 0, stream>>>(X, W, Y, M, N, K, ldy, gtab, rscale, glu_act(glu), K, 0, 0);
-  else gemm_f32_kernel<false><<<grid, 256, 0, stream>>>(X, W, Y, M, N, K, ldy, gtab, rscale, GluAct{}, K, 0, 0);
+// Y = sum_s P[s] (GLU: of the interleaved gate | up columns, then act(g) u), 4 outputs per thread.
+template <bool GLU>
+__global__ void __launch_bounds__(256) slabs_f32_kernel(const GemmF32 a) {
+  const int NO = GLU ? a.N / 2 : a.N;
+  const int64_t at = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4, MN = (int64_t)a.M * a.N;
+  const int m = (int)(at / NO), f = (int)(at % NO);
+  if (m >= a.M) return;
+  const float* p = a.P + (int64_t)m * a.N + (GLU ? (f >> 6) * 128 + (f & 63) : f);
+  f32x4 v{}, u{};
+  for (int s = 0; s < a.S; ++s, p += MN) {
+    v += *reinterpret_cast<const f32x4*>(p);
+    if constexpr (GLU) u += *reinterpret_cast<const f32x4*>(p + 64);
+  }
+  if constexpr (GLU)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = glu1(v[r], u[r], a.act);
+  put4(a.Y + m * a.ldy + f, v, 4, a.vec);
+}
+
+// The same product for at most 16 MT rows: small decode batches and the last rows of a prefill.
+// What bounds it: streaming W once from HBM (1 row: 16384 x 2048 gated 37 us, 3.6 TB/s; 32000 x 2048 53 us, 5 TB/s; the
+// 64-row FMA tiles before took 450 and 180). A workgroup takes 16 features (GLU: 16 gate and 16 up rows); its waves
+// take 32-column pieces of K in turn, whole 128-B lines of 16 rows straight into MFMA fragments (two to four pieces
+// requested before the first is used), and their sums meet in LDS. The rows come from L2 in the same layout.
+template <bool GLU, int MT, int NW>
+__global__ void __launch_bounds__(64 * NW) gemm_f32_skinny_kernel(const GemmF32 a) {
+  constexpr int NB = GLU ? 2 : 1;
+  __shared__ f32x4 red[NW][NB * MT][64];
+  const int f0 = blockIdx.x * 16, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int l15 = lane & 15, g = lane >> 4;
+  const float* X = a.X + blockIdx.z * a.xh;
+  const float* W = a.W + (int64_t)blockIdx.z * a.N * a.K;
+  const float *xr[MT], *wr[NB];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) xr[i] = X + min(16 * i + l15, a.M - 1) * a.ldx + 4 * g;
+#pragma unroll
+  for (int b = 0; b < NB; ++b) wr[b] = W + (int64_t)min(GLU ? (f0 >> 6) * 128 + 64 * b + (f0 & 63) + l15 : f0 + l15, a.N - 1) * a.K + 4 * g;
+  f32x4 acc[NB][MT] = {};
+  constexpr int U = MT * NB <= 2 ? 4 : 2;   // pieces requested before the first is used
+  const f32x4 zero{};
+  for (int c0 = w * U; c0 * 32 < a.K; c0 += NW * U) {
+    f32x4 wf[U][NB][2], xf[U][MT][2];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int k = (c0 + u) * 32 + 16 * s;
+        const bool in = k < a.K;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) wf[u][b][s] = in ? *reinterpret_cast<const f32x4*>(wr[b] + k) : zero;
+#pragma unroll
+        for (int i = 0; i < MT; ++i) xf[u][i][s] = in ? *reinterpret_cast<const f32x4*>(xr[i] + k) : zero;
+      }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int i = 0; i < MT; ++i) acc[b][i] = mfma4(wf[u][b][s], xf[u][i][s], acc[b][i]);
+  }
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) red[w][b * MT + i][lane] = acc[b][i];
+  __syncthreads();
+  const int NO = GLU ? a.N / 2 : a.N;
+  for (int i = w; i < MT; i += NW) {
+    const int m = 16 * i + l15;
+    f32x4 v{}, u{};
+#pragma unroll
+    for (int x = 0; x < NW; ++x) {
+      v += red[x][i][lane];
+      if constexpr (GLU) u += red[x][MT + i][lane];
+    }
+    if (m >= a.M) continue;
+    const float c = a.rscale ? a.rscale[m] : 1.f;
+    if constexpr (GLU)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = glu1(c * v[r], c * u[r], a.act);
+    put4(a.Y + blockIdx.z * a.yh + m * a.ldy + f0 + 4 * g, v, NO - f0 - 4 * g, a.vec);
+  }
+}
+
+// K slices of the tile kernel: two workgroups per CU where the tiles alone give fewer, slices of 256 columns at least
+int gemm_f32_splits(int M, int N, int K, int glu) {
+  if (skinny_rows(M, K) || N % 4) return 1;
+  const int64_t tiles = (int64_t)((M + 63) / 64) * (((glu ? N / 2 : N) + 63) / 64);
+  int S = 1;
+  while (tiles * S < 512 && S < 8 && K / (2 * S) >= 256) S *= 2;
+  return S;
+}
+
+template <bool GLU, int NW>
+static void launch_skinny(const GemmF32& a, dim3 grid, hipStream_t stream) {
+  if (a.M <= 16) gemm_f32_skinny_kernel<GLU, 1, NW><<<grid, 64 * NW, 0, stream>>>(a);
+  else gemm_f32_skinny_kernel<GLU, 2, NW><<<grid, 64 * NW, 0, stream>>>(a);
+}
+
+static int run_f32(GemmF32 a, bool glu, int H, hipStream_t stream) {
+  const int nf = glu ? a.N / 2 : a.N;
+  a.vec = a.ldy % 4 == 0 && a.yh % 4 == 0 && reinterpret_cast<uintptr_t>(a.Y) % 16 == 0;
+  if (skinny_rows(a.M, a.K) && !a.gtab) {
+    const dim3 grid((nf + 15) / 16, 1, H);
+    // enough waves to keep the loads of one CU in flight, and work for each of them
+    if (glu) launch_skinny<true, 8>(a, grid, stream);
+    else if (a.K >= 1024) launch_skinny<false, 8>(a, grid, stream);
+    else launch_skinny<false, 4>(a, grid, stream);
+  } else {
+    const dim3 grid((a.M + 63) / 64, (nf + 63) / 64, a.S > 1 ? a.S : H);
+    if (grid.y > 65535) return -1;
+    if (a.S > 1 && glu) gemm_f32_kernel<true, true><<<grid, 256, 0, stream>>>(a);
+    else if (a.S > 1) gemm_f32_kernel<false, true><<<grid, 256, 0, stream>>>(a);
+    else if (glu) gemm_f32_kernel<true, false><<<grid, 256, 0, stream>>>(a);
+    else gemm_f32_kernel<false, false><<<grid, 256, 0, stream>>>(a);
+    if (a.S > 1) {
+      const int blocks = (int)(((int64_t)a.M * nf / 4 + 255) / 256);
+      if (glu) slabs_f32_kernel<true><<<blocks, 256, 0, stream>>>(a);
+      else slabs_f32_kernel<false><<<blocks, 256, 0, stream>>>(a);
+    }
+  }
   OAMD_LAUNCH_CHECK();
   return 0;
+}
+
+int gemm_f32(const float* X, const float* W, float* Y, float* P, int S, int M, int N, int K, int ldy, int glu, const int* gtab,
+             const float* rscale, hipStream_t stream) {
+  if (M == 0) return 0;
+  if (K % 16 || (glu && N % 128) || S < 1 || S > 8) return -1;
+  if (S > 1 && (P == nullptr || gtab || rscale || N % 4 || skinny_rows(M, K))) return -2;
+  return run_f32({X, W, Y, P, M, N, K, S, K, ldy, 0, 0, gtab, rscale, glu ? glu_act(glu) : GluAct{}, 0}, glu != 0, 1, stream);
 }
 
 int head_gemm_f32(const float* X, const float* W, float* Y, int M, int N, int K, int H, int64_t ldx, int64_t xh,
                   int64_t ldy, int64_t yh, hipStream_t stream) {
   if (M == 0) return 0;
   if (K % 16 || ldx % 4 || xh % 4 || H < 1 || H > 65535) return -1;
-  const dim3 grid((M + 63) / 64, (N + 63) / 64, H);
-  gemm_f32_kernel<false><<<grid, 256, 0, stream>>>(X, W, Y, M, N, K, (int)ldy, nullptr, nullptr, GluAct{}, ldx, xh, yh);
+  return run_f32({X, W, Y, nullptr, M, N, K, 1, ldx, ldy, xh, yh, nullptr, nullptr, GluAct{}, 0}, false, H, stream);
+}
+
+// Attention on the fp32 matrix instruction: S^T = K Q^T, so a lane holds scores of one query (l15) and the
+// accumulator of the scores is already the operand of O^T += V^T P^T: no round trip for the weights, and the
+// running maximum, sum and rescale stay on the query's lanes.
+namespace {
+
+struct RowStat { float m = -1e30f, l = 0.f; };
+
+// Scores st[kb][r] of keys j0 + 16 kb + 4 g + r -> softmax weights against the running maximum; the factor
+// of what was accumulated. Keys outside [lo, n) get weight 0.
+template <int NB>
+__device__ __forceinline__ float soften(f32x4 (&st)[NB], int j0, int g, int lo, int n, float scale, RowStat& q) {
+  float top = -INFINITY;
+#pragma unroll
+  for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int j = j0 + 16 * kb + 4 * g + r;
+      st[kb][r] = j >= lo && j < n ? st[kb][r] * scale : -INFINITY;
+      top = fmaxf(top, st[kb][r]);
+    }
+  top = fmaxf(top, __shfl_xor(top, 16, kWave));
+  top = fmaxf(top, __shfl_xor(top, 32, kWave));
+  const float mn = fmaxf(q.m, top), alpha = expf(q.m - mn);
+  float sum = 0.f;
+#pragma unroll
+  for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      st[kb][r] = expf(st[kb][r] - mn);
+      sum += st[kb][r];
+    }
+  q.m = mn;
+  q.l = q.l * alpha + sum;   // this lane's keys; the query's four lanes meet at the end
+  return alpha;
+}
+
+__device__ __forceinline__ float lanes_sum(float v) {
+  v += __shfl_xor(v, 16, kWave);
+  return v + __shfl_xor(v, 32, kWave);
+}
+
+}  // namespace
+
+// Prefill: a workgroup is 64 query rows of one sequence and head, a wave 16 of them; 32-key tiles of K and V
+// are shared through LDS (rows padded by 16 B) and the next tile's loads are in flight while one is used.
+// What bounds it: the fp32 MFMA rate of the workgroups with the longest rows (2 x 500 rows of 16 heads of 128: 866 us
+// with a row per workgroup on FMA, 72 here; 2018 rows 3956 -> 243).
+// D: instantiated size >= both head sizes.
+template <int D>
+__global__ void __launch_bounds__(256) attn_f32_prefill_kernel(const AttnF32 a) {
+  constexpr int BK = 32, LD = D + 4, NC = D / 32;   // NC: 16-B chunks of a row per loading thread
+  __shared__ __attribute__((aligned(16))) float ks[BK * LD], vs[BK * LD];
+  const int seq = a.work_seq[blockIdx.x];
+  if (seq < 0) return;   // padding item of a graph-captured prefill (fixed grid)
+  const int s0 = a.cu_seqlens[seq], slen = a.cu_seqlens[seq + 1] - s0;
+  const int q0 = a.work_q0[blockIdx.x] + 64 * blockIdx.z;
+  if (q0 >= slen) return;
+  const int Hq = gridDim.y, hq = blockIdx.y, kvh = hq / (Hq / a.Hkv);
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, l15 = lane & 15, g = lane >> 4;
+  const int pl = a.seq_pfx ? a.seq_pfx[seq] : 0;
+  const int qrow = q0 + 16 * w + l15;
+  const int n = qrow < slen ? pl + qrow + 1 : 0, lo = max(0, pl + qrow + 1 - a.window);   // keys [lo, n) of this lane's query
+  const int kend = pl + min(slen, q0 + 64), kbeg = max(0, pl + q0 + 1 - a.window) & ~(BK - 1);
+
+  const f32x4 zero{};
+  f32x4 qf[D / 16];
+#pragma unroll
+  for (int c = 0; c < D / 16; ++c)
+    qf[c] = n > 0 && 16 * c + 4 * g < a.dkp ? *reinterpret_cast<const f32x4*>(a.q + ((int64_t)(s0 + qrow) * Hq + hq) * a.dkp + 16 * c + 4 * g) : zero;
+  // loader: thread -> row tid / 8 of the tile, chunks tid % 8 + 8 i
+  const int lr = tid >> 3, lc = tid & 7;
+  f32x4 kn[NC], vn[NC];
+  auto load = [&](int j0) {
+    const int j = j0 + lr;
+    const bool in = j < kend, pre = j < pl;
+    const int64_t r = pre ? j : s0 + j - pl;
+    const float* kp = (pre ? a.pk : a.k) + (r * a.Hkv + kvh) * a.dkp;
+    const float* vp = (pre ? a.pv : a.v) + (r * a.Hkv + kvh) * a.dvp;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int c = 4 * (lc + 8 * i);
+      kn[i] = in && c < a.dkp ? *reinterpret_cast<const f32x4*>(kp + c) : zero;
+      vn[i] = in && c < a.dvp ? *reinterpret_cast<const f32x4*>(vp + c) : zero;
+    }
+  };
+  f32x4 acc[D / 16] = {};   // dims 16 b + 4 g + r of query l15
+  RowStat st;
+  load(kbeg);
+  for (int j0 = kbeg; j0 < kend; j0 += BK) {
+    __syncthreads();
+    bool odd = false;   // a value that must not meet the weight 0 of a query that does not see its key
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      *reinterpret_cast<f32x4*>(ks + lr * LD + 4 * (lc + 8 * i)) = kn[i];
+      *reinterpret_cast<f32x4*>(vs + lr * LD + 4 * (lc + 8 * i)) = vn[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) odd |= !(fabsf(vn[i][e]) <= 3.4028234e38f);
+    }
+    odd = __syncthreads_or(odd);
+    if (j0 + BK < kend) load(j0 + BK);
+    if (j0 >= pl + q0 + 16 * w + 16) continue;   // past every query of this wave
+    f32x4 s[2] = {};
+#pragma unroll
+    for (int c = 0; c < D / 16; ++c) {
+      if (16 * c >= a.dkp) break;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) s[kb] = mfma4(*reinterpret_cast<const f32x4*>(ks + (16 * kb + l15) * LD + 16 * c + 4 * g), qf[c], s[kb]);
+    }
+    const float alpha = soften<2>(s, j0, g, lo, n, a.scale, st);
+    if (odd) {   // infinities or NaN among the values: key by key, for the queries that see it
+#pragma unroll
+      for (int b = 0; b < D / 16; ++b) acc[b] *= alpha;
+#pragma unroll
+      for (int i = 0; i < BK; ++i) {
+        const float p = __shfl(s[i >> 4][i & 3], (i >> 2 & 3) * 16 + l15, kWave);
+        if (j0 + i < lo || j0 + i >= n) continue;
+#pragma unroll
+        for (int b = 0; b < D / 16; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[b][r] = __builtin_fmaf(p, vs[i * LD + 16 * b + 4 * g + r], acc[b][r]);
+      }
+      continue;
+    }
+#pragma unroll
+    for (int b = 0; b < D / 16; ++b) {
+      if (16 * b >= a.dvp) break;
+      acc[b] *= alpha;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(vs[(16 * kb + 4 * g + e) * LD + 16 * b + l15], s[kb][e], acc[b], 0, 0, 0);
+    }
+  }
+  const float l = lanes_sum(st.l);
+  if (n <= 0) return;
+  const float c = (a.gate ? a.gate[(int64_t)(s0 + qrow) * Hq + hq] : 1.f);
+  float* out = a.o + (int64_t)(s0 + qrow) * a.o_ld + hq * a.dvp + 4 * g;
+#pragma unroll
+  for (int b = 0; b < D / 16; ++b) {
+    if (16 * b >= a.dvp) break;
+    f32x4 v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = a.gate ? acc[b][r] / l * c : acc[b][r] / l;
+    *reinterpret_cast<f32x4*>(out + 16 * b) = v;
+  }
+}
+
+int attn_f32_prefill(const AttnF32& a, int items, int Hq, hipStream_t stream) {
+  if (items == 0) return 0;
+  const int top = a.dkp > a.dvp ? a.dkp : a.dvp;
+  if (a.dkp % 16 || a.dvp % 16 || a.o_ld % 4 || top > 256 || Hq % a.Hkv || a.window < 1) return -1;
+  const dim3 grid(items, Hq, 2);   // items are 128 query rows
+  if (top <= 64) attn_f32_prefill_kernel<64><<<grid, 256, 0, stream>>>(a);
+  else if (top <= 128) attn_f32_prefill_kernel<128><<<grid, 256, 0, stream>>>(a);
+  else attn_f32_prefill_kernel<256><<<grid, 256, 0, stream>>>(a);
   OAMD_LAUNCH_CHECK();
   return 0;
 }
 
-// Attention of one query row and head per workgroup; each of the 4 waves takes every fourth
-// 64-key block (a key per lane), then owns NE output dims lane, lane + 64, ...
-// PAGED: row b's keys come from the paged cache (token rows); else from packed k / v rows of
-// the sequence holding the row, after the shared-prefix rows.
-template <bool PAGED, int NE>
-__global__ void __launch_bounds__(256) attn_f32_kernel(const AttnF32 a) {
-  __shared__ float qs[64 * NE];
-  __shared__ float ps[4][64];
-  __shared__ float red[4][64 * NE];
-  __shared__ float mls[4][2];
-  const int t = blockIdx.x, hq = blockIdx.y, kvh = hq / (gridDim.y / a.Hkv);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  float* out = a.o + (int64_t)t * a.o_ld + hq * a.dvp;
-  int n = 0, pl = 0;
-  int64_t base = 0;
-  if constexpr (PAGED) {
-    n = min(a.seq_lens[t], a.max_pages * a.page_size);
-    if (n <= 0) {
-      for (int d = tid; d < a.dvp; d += 256) out[d] = 0.f;
-      return;
-    }
-  } else {
-    int s = 0;
-    while (s < a.num_seqs && a.cu_seqlens[s + 1] <= t) ++s;
-    if (s >= a.num_seqs) return;   // padding row of a graph-captured prefill
-    base = a.cu_seqlens[s];
-    pl = a.seq_pfx ? a.seq_pfx[s] : 0;
-    n = pl + t - (int)base + 1;
-  }
-  for (int d = tid; d < a.dkp; d += 256) qs[d] = a.q[((int64_t)t * gridDim.y + hq) * a.dkp + d];
+// Decode: a workgroup takes one sequence, up to 16 query heads of one key / value head (`chunks` of them) and one of
+// `splits` pieces of its context; its eight waves take 16-key tiles in turn, K and V straight from the pages into
+// fragments (a tile is in one page, one row read serves all heads), and meet in LDS. One piece writes the
+// result, several leave (sums, m, l) to attn_f32_combine. What bounds it: the latency of a wave's tiles, so the loads
+// of a tile go out in large groups, with small heads its values before the scores are computed. 18 sequences of 1282
+// tokens: 16 heads on one latent row of 288 454 -> 37 us, 4 heads of 128 on a key head, window 512, 202 -> 27 (with a
+// workgroup per query head and a key per lane before).
+// NB: 16-dim blocks of the value size.
+template <int NB>
+__global__ void __launch_bounds__(512) attn_f32_decode_kernel(const AttnF32 a, int Hq, int chunks, int splits, float* part, float* ml) {
+  constexpr int NW = 8, RB = 4;                // waves, value blocks merged at a time
+  constexpr bool kEarly = NB <= 8;             // a tile's values fit in registers beside the sums
+  constexpr int KC = NB <= 8 ? 8 : 20;         // 16-column pieces of the keys requested at a time
+  __shared__ f32x4 red[NW][RB][64];
+  __shared__ float mls[NW][2][16];
+  __shared__ __attribute__((aligned(16))) float qs[16 * (640 + 4)];
+  const int t = blockIdx.x, kvh = blockIdx.y / chunks, G = Hq / a.Hkv, sp = blockIdx.z;
+  const int h0 = kvh * G + (blockIdx.y % chunks) * 16, heads = min(16, (kvh + 1) * G - h0);
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, l15 = lane & 15, g = lane >> 4;
+  const int n = min(a.seq_lens[t], a.max_pages * a.page_size), lo = max(0, n - a.window);
+  const int first = lo >> 4, tiles = n > 0 ? ((n + 15) >> 4) - first : 0;
+  const int ta = first + (int)((int64_t)tiles * sp / splits), tb = first + (int)((int64_t)tiles * (sp + 1) / splits);
+  const int ldq = a.dkp + 4;
+  for (int i = tid * 4; i < heads * a.dkp; i += 64 * NW * 4)
+    *reinterpret_cast<f32x4*>(qs + i / a.dkp * ldq + i % a.dkp) = *reinterpret_cast<const f32x4*>(a.q + ((int64_t)t * Hq + h0) * a.dkp + i);
   __syncthreads();
-  // row index (in units of one head's row) of key j
-  auto key = [&](int j, const float*& kp, const float*& vp) {
-    if constexpr (PAGED) {
-      const int64_t r = ((int64_t)a.block_tables[(int64_t)t * a.max_pages + j / a.page_size] * a.Hkv + kvh) * a.page_size + j % a.page_size;
-      kp = a.k + r * a.k_ld;
-      vp = a.v + r * a.v_ld;
-    } else {
-      const int64_t r = j < pl ? j : base + j - pl;
-      kp = (j < pl ? a.pk : a.k) + (r * a.Hkv + kvh) * a.dkp;
-      vp = (j < pl ? a.pv : a.v) + (r * a.Hkv + kvh) * a.dvp;
-    }
-  };
-  float m = -1e30f, l = 0.f;
-  float acc[NE] = {};
-  const int lo = max(0, n - a.window);   // first key in the window
-  for (int j0 = lo + w * 64; j0 < n; j0 += 256) {
-    const int j = j0 + lane;
-    float s = -INFINITY;
-    if (j < n) {
-      const float *kp, *vp;
-      key(j, kp, vp);
-      float d0 = 0.f;
-      for (int d = 0; d < a.dkp; d += 4) {
-        const f32x4 kv = *reinterpret_cast<const f32x4*>(kp + d);
+  const float* qp = qs + min(l15, heads - 1) * ldq + 4 * g;
+  f32x4 acc[NB] = {};
+  RowStat st;
+  for (int tl = ta + w; tl < tb; tl += NW) {
+    const int j0 = tl * 16;
+    const int64_t row = ((int64_t)a.block_tables[(int64_t)t * a.max_pages + j0 / a.page_size] * a.Hkv + kvh) * a.page_size + j0 % a.page_size;
+    const float* kp = a.k + (row + l15) * a.k_ld + 4 * g;
+    const float* vp = a.v + (row + 4 * g) * a.v_ld + l15;
+    float vf[8][4];
+    if constexpr (kEarly)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) d0 = __builtin_fmaf(qs[d + e], kv[e], d0);
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) vf[b][e] = vp[e * a.v_ld + (16 * b < a.dvp ? 16 * b : 0)];
+    __builtin_amdgcn_sched_barrier(0);   // ... here, not where they are used
+    f32x4 s[1] = {};
+    for (int c0 = 0; c0 < a.dkp; c0 += 16 * KC) {
+      f32x4 kf[KC];
+#pragma unroll
+      for (int c = 0; c < KC; ++c) kf[c] = *reinterpret_cast<const f32x4*>(kp + (c0 + 16 * c < a.dkp ? c0 + 16 * c : 0));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int c = 0; c < KC; ++c)
+        if (c0 + 16 * c < a.dkp) s[0] = mfma4(kf[c], *reinterpret_cast<const f32x4*>(qp + c0 + 16 * c), s[0]);
+    }
+    const float alpha = soften<1>(s, j0, g, lo, n, a.scale, st);
+    constexpr int VB = kEarly ? NB : 8;   // value blocks requested at a time
+#pragma unroll
+    for (int b0 = 0; b0 < NB; b0 += VB) {
+      if constexpr (!kEarly) {
+#pragma unroll
+        for (int b = 0; b < VB; ++b)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) vf[b][e] = vp[e * a.v_ld + (16 * (b0 + b) < a.dvp ? 16 * (b0 + b) : 0)];
+        __builtin_amdgcn_sched_barrier(0);
       }
-      s = d0 * a.scale;
-    }
-    const float mn = fmaxf(m, wave_max(s));
-    const float alpha = expf(m - mn);
-    const float p = expf(s - mn);
-    m = mn;
-    l = l * alpha + wave_sum(p);
-    ps[w][lane] = p;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-    for (int e = 0; e < NE; ++e) acc[e] *= alpha;
-    const int cnt = min(64, n - j0);
-    for (int i = 0; i < cnt; ++i) {
-      const float *kp, *vp;
-      key(j0 + i, kp, vp);
+      for (int b = 0; b < VB; ++b) {
+        if (16 * (b0 + b) >= a.dvp) continue;
+        acc[b0 + b] *= alpha;
 #pragma unroll
-      for (int e = 0; e < NE; ++e)
-        if (lane + 64 * e < a.dvp) acc[e] = __builtin_fmaf(ps[w][i], vp[lane + 64 * e], acc[e]);
+        for (int e = 0; e < 4; ++e) {
+          const int j = j0 + 4 * g + e;
+          const float v = j >= lo && j < n ? vf[b][e] : 0.f;   // rows outside may hold anything
+          acc[b0 + b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, s[0][e], acc[b0 + b], 0, 0, 0);
+        }
+      }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-#pragma unroll
-  for (int e = 0; e < NE; ++e) red[w][lane + 64 * e] = acc[e];
-  if (lane == 0) {
-    mls[w][0] = m;
-    mls[w][1] = l;
+  const float l = lanes_sum(st.l);
+  if (g == 0) {
+    mls[w][0][l15] = st.m;
+    mls[w][1][l15] = l;
   }
   __syncthreads();
-  const float M = fmaxf(fmaxf(mls[0][0], mls[1][0]), fmaxf(mls[2][0], mls[3][0]));
-  for (int d = tid; d < a.dvp; d += 256) {
-    float o = 0.f, L = 0.f;
+  float M = -1e30f, L = 0.f, f[NW];
 #pragma unroll
-    for (int ww = 0; ww < 4; ++ww) {
-      const float f = expf(mls[ww][0] - M);
-      o += f * red[ww][d];
-      L += f * mls[ww][1];
+  for (int x = 0; x < NW; ++x) M = fmaxf(M, mls[x][0][l15]);
+#pragma unroll
+  for (int x = 0; x < NW; ++x) {
+    f[x] = expf(mls[x][0][l15] - M);
+    L += f[x] * mls[x][1][l15];
+  }
+  const int64_t hq = (int64_t)t * Hq + h0 + l15;
+  const bool mine = l15 < heads;
+  if (splits > 1 && w == 0 && g == 0 && mine) {
+    ml[(hq * splits + sp) * 2] = M;
+    ml[(hq * splits + sp) * 2 + 1] = L;
+  }
+#pragma unroll
+  for (int b0 = 0; b0 < NB; b0 += RB) {
+    if (16 * b0 >= a.dvp) continue;
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < RB && b0 + b < NB; ++b) red[w][b][lane] = acc[b0 + b];
+    __syncthreads();
+    const int b = b0 + w;   // wave w < RB finishes block b0 + w
+    if (w < RB && b < NB && 16 * b < a.dvp && mine) {
+      f32x4 o{};
+#pragma unroll
+      for (int x = 0; x < NW; ++x) o += f[x] * red[x][w][lane];
+      if (splits > 1) {
+        *reinterpret_cast<f32x4*>(part + (hq * splits + sp) * a.dvp + 16 * b + 4 * g) = o;
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = n <= 0 ? 0.f : a.gate ? o[r] / L * a.gate[hq] : o[r] / L;
+        *reinterpret_cast<f32x4*>(a.o + (int64_t)t * a.o_ld + (h0 + l15) * a.dvp + 16 * b + 4 * g) = o;
+      }
     }
-    out[d] = a.gate ? o / L * a.gate[(int64_t)t * gridDim.y + hq] : o / L;
   }
 }
 
-int attn_f32(const AttnF32& a, int rows, int Hq, bool paged, hipStream_t stream) {
+// One workgroup per sequence and head: the pieces' sums against their common maximum.
+__global__ void __launch_bounds__(64) attn_f32_combine_kernel(const AttnF32 a, int Hq, int splits, const float* part, const float* ml) {
+  const int64_t hq = (int64_t)blockIdx.x * Hq + blockIdx.y;
+  float* out = a.o + (int64_t)blockIdx.x * a.o_ld + blockIdx.y * a.dvp;
+  const bool any = a.seq_lens[blockIdx.x] > 0;
+  float M = -1e30f, L = 0.f;
+  for (int s = 0; s < splits; ++s) M = fmaxf(M, ml[(hq * splits + s) * 2]);
+  for (int s = 0; s < splits; ++s) L += expf(ml[(hq * splits + s) * 2] - M) * ml[(hq * splits + s) * 2 + 1];
+  for (int d = 4 * threadIdx.x; d < a.dvp; d += 256) {
+    f32x4 o{};
+    for (int s = 0; s < splits; ++s) o += expf(ml[(hq * splits + s) * 2] - M) * *reinterpret_cast<const f32x4*>(part + (hq * splits + s) * a.dvp + d);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = !any ? 0.f : a.gate ? o[r] / L * a.gate[hq] : o[r] / L;
+    *reinterpret_cast<f32x4*>(out + d) = o;
+  }
+}
+
+int attn_f32_decode(const AttnF32& a, int rows, int Hq, int splits, float* part, float* ml, hipStream_t stream) {
   if (rows == 0) return 0;
-  const int top = a.dkp > a.dvp ? a.dkp : a.dvp;
-  if (a.dkp % 4 || top > (paged ? 640 : 256) || Hq % a.Hkv || a.window < 1) return -1;
-  if (paged && top > 256) attn_f32_kernel<true, 10><<<dim3(rows, Hq), 256, 0, stream>>>(a);
-  else if (paged) attn_f32_kernel<true, 4><<<dim3(rows, Hq), 256, 0, stream>>>(a);
-  else attn_f32_kernel<false, 4><<<dim3(rows, Hq), 256, 0, stream>>>(a);
+  if (a.dkp % 16 || a.dvp % 16 || a.o_ld % 4 || a.dkp > 640 || a.dvp > 640 || Hq % a.Hkv || a.window < 1 || a.page_size % 16) return -1;
+  if (splits < 1 || splits > 256 || (splits > 1 && (part == nullptr || ml == nullptr))) return -2;
+  const int chunks = (Hq / a.Hkv + 15) / 16;
+  const dim3 grid(rows, a.Hkv * chunks, splits);
+  if (a.dvp <= 128) attn_f32_decode_kernel<8><<<grid, 512, 0, stream>>>(a, Hq, chunks, splits, part, ml);
+  else if (a.dvp <= 256) attn_f32_decode_kernel<16><<<grid, 512, 0, stream>>>(a, Hq, chunks, splits, part, ml);
+  else attn_f32_decode_kernel<40><<<grid, 512, 0, stream>>>(a, Hq, chunks, splits, part, ml);
   OAMD_LAUNCH_CHECK();
+  if (splits > 1) {
+    attn_f32_combine_kernel<<<dim3(rows, Hq), 64, 0, stream>>>(a, Hq, splits, part, ml);
+    OAMD_LAUNCH_CHECK();
+  }
   return 0;
 }
 

@@ -314,8 +314,10 @@ struct HeadGemm {
 int head_gemm(const HeadGemm& a, hipStream_t stream);
 
 // fp32 forms (f32.hip)
-int gemm_f32(const float* X, const float* W, float* Y, int M, int N, int K, int ldy, int glu, const int* gtab,
+// S > 1 (where gemm_f32_splits, the count that fills the GPU, gives more; no gtab / rscale): K slices through P [S][M][N].
+int gemm_f32(const float* X, const float* W, float* Y, float* P, int S, int M, int N, int K, int ldy, int glu, const int* gtab,
              const float* rscale, hipStream_t stream);
+int gemm_f32_splits(int M, int N, int K, int glu);
 // One product per head: as HeadGemm, without the extra columns.
 int head_gemm_f32(const float* X, const float* W, float* Y, int M, int N, int K, int H, int64_t ldx, int64_t xh,
                   int64_t ldy, int64_t yh, hipStream_t stream);
@@ -323,8 +325,7 @@ struct AttnF32 {
   const float *q, *k, *v;       // k / v: packed rows, or the paged cache (token rows)
   float* o;
   int o_ld;
-  const int *cu_seqlens;        // packed: [num_seqs + 1]
-  int num_seqs;
+  const int *cu_seqlens, *work_seq, *work_q0;   // packed: [num_seqs + 1], items of 128 query rows as in AttnPrefill
   const int *block_tables, *seq_lens;   // paged
   int Hkv, dkp, dvp, page_size, max_pages;
   int64_t k_ld, v_ld;           // elements between the rows of one head's keys / values in k, v
@@ -334,7 +335,9 @@ struct AttnF32 {
   int window;                   // as in AttnPrefill
   const float* gate;            // [rows][Hq] or nullptr
 };
-int attn_f32(const AttnF32& a, int rows, int Hq, bool paged, hipStream_t stream);
+int attn_f32_prefill(const AttnF32& a, int items, int Hq, hipStream_t stream);
+// splits > 1: pieces of every context through part [rows][Hq][splits][dvp] and ml [rows][Hq][splits][2]
+int attn_f32_decode(const AttnF32& a, int rows, int Hq, int splits, float* part, float* ml, hipStream_t stream);
 
 // Routed experts (moe.hip)
 // Router: logits of E experts (rows 0..E-1 of wr) and, with `gate`, one more row E, in fp32;

@@ -511,10 +511,14 @@ def f32_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def linear_f32(x: torch.Tensor, w: torch.Tensor, glu: int = 0) -> torch.Tensor:
-    """True 32-bit x @ w^T (fp32 FMA), optionally with the gated epilogue (SILU / GELU_TANH) over a 64-row
+    """x @ w^T in full 32-bit products and sums, optionally with the gated epilogue (SILU / GELU_TANH) over a 64-row
     interleaved gate|up weight."""
-    y = torch.empty(x.shape[0], w.shape[0] // 2 if glu else w.shape[0], dtype=x.dtype, device=x.device)
-    kernels().gemm_f32(x, w, y, glu)
+    M, K = x.shape
+    N = w.shape[0]
+    y = torch.empty(M, N // 2 if glu else N, dtype=x.dtype, device=x.device)
+    S = kernels().gemm_f32_splits(M, N, K, glu)
+    part = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if S > 1 else None
+    kernels().gemm_f32(x, w, y, glu, partial=part, splits=S)
     return y
 
 

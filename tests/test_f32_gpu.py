@@ -1,0 +1,126 @@
+"""fp32 kernels on the fp32 matrix instruction (csrc/kernels/f32.hip) against fp64, at the borders of their rules and tiles."""
+import pytest
+import torch
+
+from operator_amd import ops
+from operator_amd.ops import decoder as dec
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _close(y, r, mag, K):
+    """fp32 accumulation of K products: K 2^-24 of the sum of their magnitudes."""
+    assert ((y.double() - r).abs() <= (K + 8) * 2.0 ** -24 * mag + 1e-30).all()
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 20, 16), (16, 64, 48), (17, 100, 2032), (17, 100, 2048), (32, 1000, 80), (33, 1000, 80), (64, 130, 512), (65, 68, 528),
+    (130, 50, 16), (200, 2048, 1040), (257, 64, 4112)])
+def test_gemm_f32_rules(M, N, K):
+    torch.manual_seed(M + N + K)
+    x, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV)
+    mag = x.double().abs() @ w.double().abs().t()
+    _close(ops.linear_f32(x, w), x.double() @ w.double().t(), mag, K)
+    gate, up = torch.randn(64, K, device=DEV) * K ** -0.5, torch.randn(64, K, device=DEV) * K ** -0.5
+    y = ops.linear_f32(x, ops.interleave_gate_up(gate, up), ops.SILU).double()
+    a, b = x.double() @ gate.double().t(), x.double() @ up.double().t()
+    ma, mb = (x.double().abs() @ t.double().abs().t() for t in (gate, up))
+    # silu's slope is below 1.1; expf and the quotient are within a few ulp
+    err = (K + 8) * 2.0 ** -24 * (1.1 * ma * b.abs() + mb * a.abs()) + 2.0 ** -21 * (a * torch.sigmoid(a) * b).abs()
+    assert ((y - a * torch.sigmoid(a) * b).abs() <= err + 1e-30).all()
+
+
+@pytest.mark.parametrize("M", [1, 33, 70])
+def test_head_gemm_f32(M):
+    torch.manual_seed(M)
+    x, w = torch.randn(M, 3, 88, device=DEV), torch.randn(3, 48, 80, device=DEV)
+    y = torch.full((M, 3, 64), float("nan"), device=DEV)
+    ops.kernels().head_gemm(x, w, y)
+    r = torch.einsum("mhk,hnk->mhn", x[..., :80].double(), w.double())
+    _close(y[..., :48], r, torch.einsum("mhk,hnk->mhn", x[..., :80].double().abs(), w.double().abs()), 80)
+    assert y[..., 48:].isnan().all()
+
+
+def _attend(q, k, v, scale, window=0):
+    n, T = k.shape[0], q.shape[0]
+    s = torch.einsum("thd,jhd->htj", q.double(), k.double()) * scale
+    i, j = torch.arange(n - T, n, device=DEV)[:, None], torch.arange(n, device=DEV)[None]
+    hidden = (j > i) | ((i - j >= window) if window else False)
+    return torch.einsum("htj,jhd->thd", torch.softmax(s.masked_fill(hidden, float("-inf")), -1), v.double())
+
+
+@pytest.mark.parametrize("lens", [[1], [31, 32, 33], [64, 65, 200]])
+@pytest.mark.parametrize("D,Dv,window", [(48, 32, 0), (128, 96, 40), (240, 256, 0)])
+def test_prefill_attention_keeps_odd_values_to_their_queries(lens, D, Dv, window):
+    """An infinity among the values of a token reaches the queries that see it and no other."""
+    torch.manual_seed(len(lens) + D)
+    H, G, T = 4, 2, sum(lens)
+    L = dec.HeadLayout(H, G, D, Dv)
+    q, k, v = (torch.randn(T, h, d, device=DEV) for h, d in ((H, D), (G, D), (G, Dv)))
+    for odd in (False, True):
+        bad = [sum(lens[:i]) + n - 1 - n // 3 for i, n in enumerate(lens)]
+        if odd:
+            v[bad, 0, 5] = float("inf")
+        o = dec.attn_gd_prefill(q, k, v, lens, L, D ** -0.5, window=window).view(T, -1)[:, :H * Dv].view(T, H, Dv)
+        a = 0
+        for n, at in zip(lens, bad):
+            clean = v[a:a + n].clone()
+            clean[clean.isinf()] = 0.0
+            r = _attend(q[a:a + n], k[a:a + n].repeat_interleave(H // G, 1), clean.repeat_interleave(H // G, 1), D ** -0.5, window)
+            got = o[a:a + n]
+            rows = torch.arange(a, a + n, device=DEV)
+            sees = (rows >= at) & ((rows - at < window) if window else True)
+            mask = torch.zeros_like(got, dtype=torch.bool)
+            if odd:
+                mask[:, :H // G, 5] = sees[:, None]
+                assert (got[mask] == float("inf")).all()
+            torch.testing.assert_close(got[~mask].double(), r[~mask], atol=2e-5, rtol=2e-5)
+            a += n
+
+
+@pytest.mark.parametrize("H,G,D,Dv,splits,window", [(40, 2, 64, 64, 1, 0), (4, 4, 128, 160, 3, 0), (16, 1, 256, 256, 4, 0), (6, 2, 48, 32, 2, 50)])
+def test_decode_attention_pieces(H, G, D, Dv, splits, window):
+    torch.manual_seed(H + D)
+    P, ctx = 16, [1, 0, 15, 16, 17, 130, 500]
+    L, B = dec.HeadLayout(H, G, D, Dv), len(ctx)
+    pages = [-(-n // P) for n in ctx]
+    perm = torch.randperm(sum(pages) + 1).int()
+    kc, vc = (torch.full((len(perm), G, P, d), float("nan"), device=DEV) for d in (D, Dv))   # what no token wrote stays out
+    bt = torch.zeros(B, max(pages), dtype=torch.int32)
+    q, seqs, at = torch.randn(B, H, D, device=DEV), [], 0
+    for b, n in enumerate(ctx):
+        bt[b, :pages[b]] = perm[at:at + pages[b]]
+        at += pages[b]
+        k, v = torch.randn(n, G, D, device=DEV), torch.randn(n, G, Dv, device=DEV)
+        for t in range(n):
+            kc[bt[b, t // P], :, t % P], vc[bt[b, t // P], :, t % P] = k[t], v[t]
+        seqs.append((k, v))
+    gate = torch.rand(B, H, device=DEV)
+    o = dec.attn_gd_decode(q, (kc, vc), bt.to(DEV), torch.tensor(ctx, dtype=torch.int32, device=DEV), L, D ** -0.5, splits, window=window,
+                           gate=gate)[:, :H * Dv].view(B, H, Dv)
+    for b, (k, v) in enumerate(seqs):
+        if ctx[b] == 0:
+            assert (o[b] == 0).all()
+            continue
+        r = _attend(q[b:b + 1], k.repeat_interleave(H // G, 1), v.repeat_interleave(H // G, 1), D ** -0.5, window)[0]
+        torch.testing.assert_close(o[b].double(), r * gate[b].double()[:, None], atol=2e-5, rtol=2e-5)
+
+
+@pytest.mark.parametrize("rank,splits", [(256, 2), (544, 1), (608, 3)])
+def test_latent_decode_f32_wide_rows(rank, splits):
+    torch.manual_seed(rank)
+    P, ctx, H, rot = 16, [3, 40, 200], 18, 32
+    L = dec.LatentLayout(H, 64, rot, 64, 128, rank)
+    B, pages = len(ctx), 1 + max(-(-n // P) for n in ctx)
+    cache = torch.full((B * pages, 1, P, L.ck), float("nan"), device=DEV)
+    bt = torch.arange(B * pages, dtype=torch.int32).view(B, pages)
+    rows = [torch.randn(n, L.ck, device=DEV) for n in ctx]
+    for b, r in enumerate(rows):
+        r[:, L.rp + rot:] = 0
+        cache[b * pages:(b + 1) * pages].view(-1, L.ck)[:ctx[b]] = r
+    q = torch.randn(B, H, L.ck, device=DEV)
+    o = dec.attn_latent_decode(q, cache, bt.to(DEV), torch.tensor(ctx, dtype=torch.int32, device=DEV), L, 0.05, splits)
+    for b, r in enumerate(rows):
+        p = torch.softmax(q[b].double() @ r.double().t() * 0.05, -1)
+        torch.testing.assert_close(o[b].double(), p @ r.double()[:, :L.rp], atol=2e-5, rtol=2e-5)
