@@ -151,6 +151,16 @@ void decode_advance(const at::Tensor& tok, at::Tensor& ids, at::Tensor& hist, at
                           ptr<int>(ctx), ptr<int64_t>(step), (int)B, (int)hist.size(1), cur_stream()));
 }
 
+void scatter_rows_f32(const at::Tensor& x, const at::Tensor& dst, at::Tensor& out) {
+  CHECK_DEV(x); CHECK_DEV(dst); CHECK_DEV(out); CHECK_DT(dst, at::kInt); CHECK_CONTIG(dst); CHECK_DT(out, at::kFloat); CHECK_CONTIG(out);
+  TORCH_CHECK(x.dim() == 2 && out.dim() == 2 && x.size(1) == out.size(1) && x.stride(1) == 1 && dst.numel() == x.size(0) &&
+                  (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kFloat),
+              "scatter_rows_f32: x [rows, cols] bf16 or fp32, dst [rows], out [n, cols]");
+  const c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+  RC(oamd::scatter_rows_f32(x.data_ptr(), x.scalar_type() == at::kBFloat16, x.stride(0), ptr<int>(dst), out.data_ptr<float>(),
+                            (int)x.size(0), (int)out.size(0), (int)out.size(1), cur_stream()));
+}
+
 static bool kv_is_fp8(const at::Tensor& t) {
   return t.scalar_type() == at::kFloat8_e4m3fn || t.scalar_type() == at::kByte;
 }
@@ -645,6 +655,7 @@ PYBIND11_MODULE(_C, m) {
         pybind11::arg("bias") = pybind11::none());
   m.def("decode_slots", &decode_slots);
   m.def("decode_advance", &decode_advance);
+  m.def("scatter_rows_f32", &scatter_rows_f32, pybind11::arg("x"), pybind11::arg("dst"), pybind11::arg("out"));
   m.def("quantize_fp8", &quantize_fp8);
   m.def("silu_quantize_fp8", &silu_quantize_fp8, pybind11::arg("gu"), pybind11::arg("q"), pybind11::arg("sx"),
         pybind11::arg("slabs") = pybind11::none(), pybind11::arg("splits") = 1);

@@ -19,6 +19,9 @@ int silu_mul(const bf16_t* gu, bf16_t* out, int64_t rows, int inter, int block, 
 // then the state advance after sampling (B <= 1024 rows, one workgroup each).
 int decode_slots(const int* bt, const int64_t* pos, const int* ctx, int64_t* slots, int64_t* spos, int B,
                  int max_pages, int page_size, hipStream_t stream);
+// out[dst[r]] [cols] = fp32 of row r of x (bf16 or fp32, row stride ld); rows whose dst is outside [0, n_out) are dropped
+int scatter_rows_f32(const void* x, bool bf16, int64_t ld, const int* dst, float* out, int rows, int n_out, int cols,
+                     hipStream_t stream);
 int decode_advance(const int64_t* tok, int64_t* ids, int64_t* hist, int64_t* pos, int* ctx, int64_t* step, int B,
                    int ms, hipStream_t stream);
 int embedding(const int64_t* ids, const bf16_t* table, bf16_t* out, int tokens, int hidden,
