@@ -14,6 +14,7 @@
 // Replaces the reference's external log-parser (J/service/LogParserClient.java:36-55);
 // the pattern schema and scoring are our design.
 #include <pybind11/pybind11.h>
+#include <pybind11/numpy.h>
 #include <pybind11/stl.h>
 
 #include <algorithm>
@@ -349,6 +350,90 @@ struct PatSpec {
   std::vector<int> window;
 };
 
+// A pattern set's scoring tables, kept between batches; score() is the host form of the scorer.
+class Scorer {
+ public:
+  Scorer(const std::vector<int64_t>& primary, std::vector<double> conf, std::vector<int64_t> sev,
+         std::vector<std::vector<int64_t>> sec, std::vector<std::vector<double>> w, std::vector<std::vector<int64_t>> win,
+         int64_t num_matchers)
+      : conf_(std::move(conf)), sev_(std::move(sev)), sec_(std::move(sec)), w_(std::move(w)), win_(std::move(win)), primary_of_(num_matchers) {
+    const size_t P = primary.size();
+    if (conf_.size() != P || sev_.size() != P || sec_.size() != P || w_.size() != P || win_.size() != P)
+      throw std::invalid_argument("pattern tables differ in length");
+    for (size_t p = 0; p < P; ++p) {
+      if (primary[p] < 0 || primary[p] >= num_matchers) throw std::out_of_range("pattern primary");
+      if (w_[p].size() != sec_[p].size() || win_[p].size() != sec_[p].size()) throw std::invalid_argument("secondary tables differ in length");
+      primary_of_[primary[p]].push_back(static_cast<int>(p));
+    }
+  }
+
+  // hits [n, 3] = (doc, matcher, line) -> per doc its events (pattern, line, score), best first
+  py::list score(py::array_t<int64_t, py::array::c_style | py::array::forcecast> hits, int64_t num_docs) const {
+    if (hits.ndim() != 2 || hits.shape(1) != 3) throw std::invalid_argument("hits [n, 3]");
+    const int64_t* h = hits.data();
+    std::vector<std::vector<std::pair<int64_t, int64_t>>> by_doc(num_docs);  // (matcher, line)
+    for (py::ssize_t i = 0; i < hits.shape(0); ++i, h += 3) {
+      if (h[0] < 0 || h[0] >= num_docs) throw std::out_of_range("hit doc");
+      by_doc[h[0]].emplace_back(h[1], h[2]);
+    }
+    py::list result;
+    std::vector<Ev> evs;
+    for (auto& v : by_doc) {
+      std::sort(v.begin(), v.end());
+      v.erase(std::unique(v.begin(), v.end()), v.end());
+      evs.clear();
+      for (const auto& hit : v) {
+        if (hit.first < 0 || hit.first >= (int64_t)primary_of_.size()) continue;
+        for (int p : primary_of_[hit.first]) {
+          double bonus = 0.0, wsum = 0.0;
+          for (size_t j = 0; j < sec_[p].size(); ++j) {
+            const double w = w_[p][j];
+            wsum += w;
+            const int64_t dist = nearest(v, sec_[p][j], hit.second);
+            if (dist >= 0 && dist <= win_[p][j]) bonus += w * (1.0 - double(dist) / double(win_[p][j] + 1));
+          }
+          evs.push_back({conf_[p] * (1.0 + bonus) / (1.0 + wsum), static_cast<int>(sev_[p]), hit.second, p});
+        }
+      }
+      std::sort(evs.begin(), evs.end(), [](const Ev& a, const Ev& b) {
+        if (a.score != b.score) return a.score > b.score;
+        if (a.sev != b.sev) return a.sev > b.sev;
+        if (a.line != b.line) return a.line < b.line;
+        return a.pat < b.pat;
+      });
+      py::list dl(evs.size());
+      for (size_t i = 0; i < evs.size(); ++i) dl[i] = py::make_tuple(evs[i].pat, evs[i].line, evs[i].score);
+      result.append(std::move(dl));
+    }
+    return result;
+  }
+
+ private:
+  struct Ev { double score; int sev; int64_t line; int pat; };
+
+  // distance of the nearest line of matcher m among a doc's sorted hits, or -1
+  static int64_t nearest(const std::vector<std::pair<int64_t, int64_t>>& v, int64_t m, int64_t line) {
+    auto lo = std::lower_bound(v.begin(), v.end(), std::make_pair(m, line));
+    int64_t best = -1;
+    if (lo != v.end() && lo->first == m) best = lo->second - line;
+    if (lo != v.begin()) {
+      auto pr = std::prev(lo);
+      if (pr->first == m) {
+        const int64_t dd = line - pr->second;
+        if (best < 0 || dd < best) best = dd;
+      }
+    }
+    return best;
+  }
+
+  std::vector<double> conf_;
+  std::vector<int64_t> sev_;
+  std::vector<std::vector<int64_t>> sec_;
+  std::vector<std::vector<double>> w_;
+  std::vector<std::vector<int64_t>> win_;
+  std::vector<std::vector<int>> primary_of_;
+};
+
 py::list score_events(const std::vector<int64_t>& hit_doc, const std::vector<int64_t>& hit_matcher,
                       const std::vector<int64_t>& hit_line, int64_t num_docs, const std::vector<int64_t>& pat_primary,
                       const std::vector<double>& pat_conf, const std::vector<int64_t>& pat_sev,
@@ -356,63 +441,14 @@ py::list score_events(const std::vector<int64_t>& hit_doc, const std::vector<int
                       const std::vector<std::vector<int64_t>>& pat_win, int64_t num_matchers) {
   const size_t n = hit_doc.size();
   if (hit_matcher.size() != n || hit_line.size() != n) throw std::invalid_argument("hit arrays differ in length");
-  const size_t P = pat_primary.size();
-  // (doc, matcher) -> sorted lines
-  std::vector<std::vector<std::pair<int64_t, int64_t>>> by_doc(num_docs);  // (matcher, line)
+  py::array_t<int64_t> hits({(py::ssize_t)n, (py::ssize_t)3});
+  int64_t* h = hits.mutable_data();
   for (size_t i = 0; i < n; ++i) {
-    if (hit_doc[i] < 0 || hit_doc[i] >= num_docs) throw std::out_of_range("hit doc");
-    by_doc[hit_doc[i]].emplace_back(hit_matcher[i], hit_line[i]);
+    h[3 * i] = hit_doc[i];
+    h[3 * i + 1] = hit_matcher[i];
+    h[3 * i + 2] = hit_line[i];
   }
-  std::vector<std::vector<int>> primary_of(num_matchers);
-  for (size_t p = 0; p < P; ++p) {
-    if (pat_primary[p] < 0 || pat_primary[p] >= num_matchers) throw std::out_of_range("pattern primary");
-    primary_of[pat_primary[p]].push_back(static_cast<int>(p));
-  }
-  py::list result;
-  for (int64_t d = 0; d < num_docs; ++d) {
-    auto& v = by_doc[d];
-    std::sort(v.begin(), v.end());
-    v.erase(std::unique(v.begin(), v.end()), v.end());
-    struct Ev { double score; int sev; int64_t line; int pat; };
-    std::vector<Ev> evs;
-    auto nearest = [&](int64_t m, int64_t line) -> int64_t {
-      auto lo = std::lower_bound(v.begin(), v.end(), std::make_pair(m, line));
-      int64_t best = -1;
-      if (lo != v.end() && lo->first == m) best = lo->second - line;
-      if (lo != v.begin()) {
-        auto pr = std::prev(lo);
-        if (pr->first == m) {
-          const int64_t dd = line - pr->second;
-          if (best < 0 || dd < best) best = dd;
-        }
-      }
-      return best;
-    };
-    for (const auto& h : v) {
-      if (h.first >= num_matchers) continue;
-      for (int p : primary_of[h.first]) {
-        double bonus = 0.0, wsum = 0.0;
-        for (size_t j = 0; j < pat_sec[p].size(); ++j) {
-          const double w = pat_w[p][j];
-          wsum += w;
-          const int64_t dist = nearest(pat_sec[p][j], h.second);
-          if (dist >= 0 && dist <= pat_win[p][j]) bonus += w * (1.0 - double(dist) / double(pat_win[p][j] + 1));
-        }
-        const double score = pat_conf[p] * (1.0 + bonus) / (1.0 + wsum);
-        evs.push_back({score, static_cast<int>(pat_sev[p]), h.second, p});
-      }
-    }
-    std::sort(evs.begin(), evs.end(), [](const Ev& a, const Ev& b) {
-      if (a.score != b.score) return a.score > b.score;
-      if (a.sev != b.sev) return a.sev > b.sev;
-      if (a.line != b.line) return a.line < b.line;
-      return a.pat < b.pat;
-    });
-    py::list dl;
-    for (const auto& e : evs) dl.append(py::make_tuple(e.pat, e.line, e.score));
-    result.append(dl);
-  }
-  return result;
+  return Scorer(pat_primary, pat_conf, pat_sev, pat_sec, pat_w, pat_win, num_matchers).score(hits, num_docs);
 }
 
 }  // namespace
@@ -429,6 +465,12 @@ PYBIND11_MODULE(_patterns, m) {
   m.def("pack_docs", &pack_docs, py::arg("docs"), py::arg("first_seg"), py::arg("seg_bytes"), py::arg("dst"),
         py::arg("threads") = 8);
   m.def("score_events", &score_events);
+  py::class_<Scorer>(m, "Scorer")
+      .def(py::init<const std::vector<int64_t>&, std::vector<double>, std::vector<int64_t>, std::vector<std::vector<int64_t>>,
+                    std::vector<std::vector<double>>, std::vector<std::vector<int64_t>>, int64_t>(),
+           py::arg("primary"), py::arg("conf"), py::arg("severity"), py::arg("secondary"), py::arg("weights"), py::arg("windows"),
+           py::arg("num_matchers"))
+      .def("score", &Scorer::score, py::arg("hits"), py::arg("num_docs"));
   m.attr("MAX_FACTOR_LEN") = kMaxFactorLen;
   m.attr("MAX_STATES") = kMaxStates;
   register_verify(m);

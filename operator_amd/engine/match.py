@@ -164,7 +164,12 @@ class MatchEngine:
     """Compile a PatternSet once, then analyze batches of logs on one device."""
 
     SCAN_LANES = 256 * 1024   # ac_scan v2 streams on MI355X (256 CUs x 1024 threads)
-    PACK_CHUNK = 64 << 20     # host pack / H2D pipelining granule (bytes; profiles/scan_config2_e2e.jsonl)
+    HOST_SCORE_HITS = 2048
+    # context windows of a few logs' events are read from the logs on the host (3 events: 1 us against 39 for the round
+    # trip; 192: 71 against 86; 768: 323 against 307); larger batches leave the host to the next batch's packing
+    HOST_CONTEXT_DOCS = 8
+    HEAD_MATCHES = 2048       # match records read back with the count (a 64-log batch has some hundred)
+    PACK_CHUNK = 32 << 20     # host pack / H2D pipelining granule (84 MB: 2.5 ms; 64 MB 2.9, 8 MB 2.8 to 3.8)
 
     def __init__(self, patterns: PatternSet | CompiledPatterns, device: str | torch.device = "cuda",
                  seg_bytes: int = 1024, max_events: int = 50, significance: float = 0.5,
@@ -187,6 +192,10 @@ class MatchEngine:
         self.use_native_scorer = use_native_scorer
         # score + rank events on the GPU (score.hip) when scanning there
         self.gpu_scorer = (self.device.type == "cuda") if gpu_scorer is None else gpu_scorer
+        # ... unless it is asked for, batches of few hits stay on the host: the round trip to the GPU takes 65 us
+        # for 3 hits (5 here) and 195 for 195 (130); past some thousand the sorts are the GPU's
+        self._gpu_score_from = 0 if gpu_scorer else self.HOST_SCORE_HITS
+        self._scorer = None
         self._score_tables = None
         self.stats = ScanStats()
         # scan -> line index -> fixup -> per-doc newlines -> D2H as ONE captured hipGraph per
@@ -200,11 +209,10 @@ class MatchEngine:
         self._text: torch.Tensor | None = None
         self._seg_nl: torch.Tensor | None = None
         self._nl_excl: torch.Tensor | None = None
-        self._lp_state: torch.Tensor | None = None
-        self._doc_nl: torch.Tensor | None = None
-        self._doc_nl_h: torch.Tensor | None = None
+        self._meta: torch.Tensor | None = None
+        self._meta_h: torch.Tensor | None = None
+        self._head_h: torch.Tensor | None = None
         self._matches: torch.Tensor | None = None
-        self._count: torch.Tensor | None = None
         self._doc_newlines: tuple[list[bytes], list[int]] | None = None   # (docs, newlines) of the last GPU scan
         # matcher -> list of (pattern) where it is primary, for quick checks
         self._nm = self.cp.num_matchers
@@ -348,10 +356,18 @@ class MatchEngine:
         while seg > 64 and approx // seg < self.SCAN_LANES:
             seg //= 2
         self.last_seg = seg
-        total, first = P.plan_docs([len(d) for d in docs], seg)
-        n_segs = total // seg
-        pinned = self._ensure("_pinned" + sfx, total, torch.uint8, pinned=True)
-        text = self._ensure("_text" + sfx, total, torch.uint8)
+        lens = [len(d) for d in docs]
+        total, first = P.plan_docs(lens, seg)
+        n_segs, nd = total // seg, len(docs)
+        # behind the text, in the same upload: first segment per doc (and the end), byte offset, length
+        lay = 8 * (3 * nd + 1)
+        pinned = self._ensure("_pinned" + sfx, total + lay, torch.uint8, pinned=True)
+        text = self._ensure("_text" + sfx, total + lay, torch.uint8)
+        layout = pinned[total:total + lay].numpy().view(np.int64)
+        layout[:nd + 1] = first
+        np.multiply(layout[:nd], seg, out=layout[nd + 1:2 * nd + 1])
+        layout[2 * nd + 1:] = lens
+        first_t, base_t, lens_t = text[total:total + lay].view(torch.int64).split([nd + 1, nd, nd])
         # pack and upload in doc-aligned chunks of >= PACK_CHUNK bytes: the host packs
         # chunk k+1 (native threads) while chunk k's DMA runs, so a large batch pays
         # max(pack, H2D) rather than the sum (1.2 GB)
@@ -362,37 +378,46 @@ class MatchEngine:
             while b < len(docs) and (first[b] - first[a]) * seg < self.PACK_CHUNK:
                 b += 1
             lo, hi = first[a] * seg, first[b] * seg
-            threads = max(1, min(self.pack_threads, (hi - lo) >> 23))   # ~8 MB per packing thread
+            threads = max(1, min(self.pack_threads, (hi - lo) >> 20))   # ~1 MB per packing thread (4.6 MB: 177 us on one, 93 on four)
             P.pack_docs(docs[a:b], [f - first[a] for f in first[a:b + 1]], seg, ptr + lo, threads)
             if self.profile_bytes > 0 and not self._profiled:
                 self._profile_states(pinned[:min(total, self.profile_bytes, hi)].numpy().tobytes())
+            if b == nd:
+                hi += lay
             text[lo:hi].copy_(pinned[lo:hi], non_blocking=True)
             a = b
         C = kernels()
         seg_nl = self._ensure("_seg_nl" + sfx, 2 * n_segs, torch.int32)   # totals, then split-segment heads
-        first_t = torch.tensor(first, dtype=torch.int64).to(self.device, non_blocking=True)
         # N3 on the GPU: exclusive newline prefix per segment (decoupled look-back scan),
         # match records -> (doc, factor, line, offset), newlines per doc
         excl = self._ensure("_nl_excl" + sfx, n_segs + 1, torch.int64)
-        lp_state = self._ensure("_lp_state" + sfx, C.line_prefix_state_words(n_segs), torch.int64)
-        doc_nl = self._ensure("_doc_nl" + sfx, len(docs), torch.int64)
-        doc_nl_h = self._ensure("_doc_nl_h" + sfx, len(docs), torch.int64, pinned=True)
+        # what the host reads stands together, and comes back with the first match records in one wait:
+        # newlines per doc, the match count, line_prefix's state (its second word: a look-back timed out)
+        at = (nd + 2) // 2 * 2   # the state is 16-B aligned
+        words = at + C.line_prefix_state_words(n_segs)
+        meta = self._ensure("_meta" + sfx, words, torch.int64)
+        meta_h = self._ensure("_meta_h" + sfx, at + 2, torch.int64, pinned=True)
+        doc_nl, count, lp_state = meta[:nd], meta[at - 1:at].view(torch.int32)[:1], meta[at:words]
+        head_h = self._ensure("_head_h" + sfx, 4 * self.HEAD_MATCHES, torch.int32, pinned=True)
         while True:
             matches = getattr(self, "_matches" + sfx, None)
             if matches is None or matches.shape[0] < self.match_cap:
                 matches = torch.empty(self.match_cap, 4, dtype=torch.int32, device=self.device)
                 setattr(self, "_matches" + sfx, matches)
-            count = getattr(self, "_count" + sfx, None)
-            if count is None:
-                count = torch.zeros(1, dtype=torch.int32, device=self.device)
-                setattr(self, "_count" + sfx, count)
+            head = min(self.HEAD_MATCHES, matches.shape[0])
             count.zero_()
             C.ac_scan(text[:total], seg, self.cls_map, self.table, self.log2c, self.hot_states, self.out_off,
                       self.out_ids, matches, count, seg_nl, self.grid_blocks, self.hot_table, self.chain)
             C.line_prefix(seg_nl[:n_segs], excl, lp_state)
             C.scan_fixup(matches, count, excl[:n_segs], first_t, seg, seg_nl[n_segs:2 * n_segs])
-            cnt = int(count.item())
-            if int(lp_state[1].item()) != 0:
+            # newlines per doc from the per-segment counts the scan already produced (the
+            # host would otherwise re-read every byte for AnalysisResult.metadata.totalLines)
+            C.doc_lines(excl, first_t, doc_nl)
+            meta_h[:at + 2].copy_(meta[:at + 2], non_blocking=True)
+            head_h[:4 * head].copy_(matches[:head].view(-1), non_blocking=True)
+            torch.cuda.current_stream(self.device).synchronize()
+            cnt = int(meta_h[at - 1:at].view(torch.int32)[0])
+            if int(meta_h[at + 1]) != 0:
                 # a line_prefix look-back hit its spin bound: the line numbers of this launch
                 # are wrong, so the batch is recomputed on the host path instead
                 log.warning("line_prefix look-back timed out; rescanning %d docs on the CPU path", len(docs))
@@ -401,14 +426,10 @@ class MatchEngine:
             if cnt <= matches.shape[0]:
                 break
             self.match_cap = int(cnt * 1.25) + 1024  # overflow: grow and rescan (rare)
-        # newlines per doc from the per-segment counts the scan already produced (the
-        # host would otherwise re-read every byte for AnalysisResult.metadata.totalLines)
-        C.doc_lines(excl, first_t, doc_nl)
-        doc_nl_h[:len(docs)].copy_(doc_nl[:len(docs)], non_blocking=True)
         self.stats.raw_matches += cnt
-        self.stats.bytes_scanned += sum(len(d) for d in docs)
-        hits = matches[:cnt].cpu().numpy().astype(np.int64) if cnt else np.zeros((0, 4), np.int64)
-        return hits, (docs, first_t, seg, text), (docs, doc_nl_h[:len(docs)].tolist())
+        self.stats.bytes_scanned += sum(lens)
+        hits = head_h[:4 * cnt].view(-1, 4) if cnt <= head else matches[:cnt].cpu()
+        return hits.numpy().astype(np.int64), (docs, base_t, lens_t, text), (docs, meta_h[:nd].tolist())
 
     def _contexts_gpu(self, docs: list[bytes], q_doc: list[int], q_off: list[int], q_k: list[int],
                       resident: tuple | None = None, stream=None):
@@ -420,19 +441,17 @@ class MatchEngine:
         r = self._resident if resident is None else resident
         if r is None or r[0] is not docs or not q_doc:
             return None
-        _, first_t, seg, text = r
+        _, base, lens, text = r
         n = len(q_doc)
         # every input is made on the scan stream, where the kernel runs: the engine thread's
         # stream (the LLM's decode graphs, tens of ms deep) would let the kernel read the
         # query / length / base buffers before their copies land (a memory fault in the
         # flagship pipeline)
         with (torch.cuda.stream(stream) if stream is not None else self._on_stream()):
-            q = torch.tensor(np.stack([np.asarray(q_doc, np.int64), np.asarray(q_off, np.int64),
-                                       np.asarray(q_k, np.int64)], 1)).to(self.device, non_blocking=True)
-            lens = torch.tensor([len(d) for d in docs], dtype=torch.int64).to(self.device, non_blocking=True)
-            base = first_t[:-1] * seg
+            q = torch.empty(n, 3, dtype=torch.int64, pin_memory=True)
+            q.numpy().T[:] = q_doc, q_off, q_k
             out = torch.empty(n, 4, dtype=torch.int64, device=self.device)
-            kernels().context_spans(text, base, lens, q, out)
+            kernels().context_spans(text, base, lens, q.to(self.device, non_blocking=True), out)
             spans = out.cpu().numpy()
         return patterns().contexts_from_spans(docs, q_doc, spans)
 
@@ -528,7 +547,7 @@ class MatchEngine:
                 sec_w=t([s_.weight for p in pats for s_ in p.secondary] or [0.0], torch.float64),
                 sec_win=t([s_.window for p in pats for s_ in p.secondary] or [0]),
                 conf=t([p.primary.confidence for p in pats], torch.float64),
-                severity=t([p.severity_rank for p in pats]))
+                severity=t([p.severity_rank for p in pats]), severity_h=[p.severity_rank for p in pats])
         return self._score_tables
 
     def _events_gpu(self, hits: np.ndarray, n_docs: int) -> list[list[oracle.Event]]:
@@ -546,18 +565,23 @@ class MatchEngine:
         ev_ptr[1:] = np.cumsum(per_hit)
         ev_doc_ptr = ev_ptr[doc_ptr]
         E = int(ev_ptr[-1])
-        i32 = lambda a: torch.as_tensor(a, dtype=torch.int32).to(dev, non_blocking=True)  # noqa: E731
-        keys = torch.as_tensor((mat << 32) | line, dtype=torch.long).to(dev, non_blocking=True)
-        ev_score = torch.empty(max(E, 1), dtype=torch.float64, device=dev)[:E]
-        ev_pat = torch.empty(E, dtype=torch.int32, device=dev)
-        ev_line = torch.empty(E, dtype=torch.int32, device=dev)
-        order = torch.empty(E, dtype=torch.int32, device=dev)
+        # one upload (keys, then the int32 index arrays) and one read-back (scores, then the int32 columns)
+        parts = (doc, doc_ptr, ev_ptr, ev_doc_ptr)
+        buf = torch.empty(8 * n + 4 * sum(map(len, parts)), dtype=torch.uint8, pin_memory=True)
+        host = buf.numpy()
+        np.bitwise_or(mat << 32, line, out=host[:8 * n].view(np.int64))
+        np.concatenate(parts, out=host[8 * n:].view(np.int32), casting="same_kind")
+        buf = buf.to(dev, non_blocking=True)
+        keys, ints = buf[:8 * n].view(torch.int64), buf[8 * n:].view(torch.int32).split([len(x) for x in parts])
+        res = torch.empty(20 * E, dtype=torch.uint8, device=dev)
+        ev_score, (ev_pat, ev_line, order) = res[:8 * E].view(torch.float64), res[8 * E:].view(torch.int32).split([E] * 3)
         summary = torch.empty(3 * max(n_docs, 1), dtype=torch.int32, device=dev)
-        kernels().score_events(keys, i32(doc), i32(doc_ptr), T["prim_ptr"], T["prim_pat"], i32(ev_ptr),
-                               i32(ev_doc_ptr), T["sec_ptr"], T["sec_matcher"], T["sec_w"], T["sec_win"], T["conf"],
-                               T["severity"], float(self.significance), ev_score, ev_pat, ev_line, order, summary)
-        sc, pt, ln, od = (x.cpu().numpy() for x in (ev_score, ev_pat, ev_line, order))
-        sev = T["severity"].cpu().numpy()
+        kernels().score_events(keys, ints[0], ints[1], T["prim_ptr"], T["prim_pat"], ints[2], ints[3], T["sec_ptr"], T["sec_matcher"],
+                               T["sec_w"], T["sec_win"], T["conf"], T["severity"], float(self.significance), ev_score, ev_pat, ev_line,
+                               order, summary)
+        res = res.cpu().numpy()
+        sc, (pt, ln, od) = res[:8 * E].view(np.float64), res[8 * E:].view(np.int32).reshape(3, E)
+        sev = T["severity_h"]
         out = []
         for d in range(n_docs):
             a, b = int(ev_doc_ptr[d]), int(ev_doc_ptr[d + 1])
@@ -574,19 +598,19 @@ class MatchEngine:
 
     def _events_from_hits(self, docs: list[bytes], hits: np.ndarray, stream=None) -> list[list[oracle.Event]]:
         cp = self.cp
-        if self.gpu_scorer and self.device.type == "cuda":
+        if self.gpu_scorer and self.device.type == "cuda" and len(hits) > self._gpu_score_from:
             with (torch.cuda.stream(stream) if stream is not None else self._on_stream()):
                 return self._events_gpu(hits, len(docs))
         if self.use_native_scorer:
-            from operator_amd.ops import patterns
+            if self._scorer is None:   # the pattern tables, once per engine
+                from operator_amd.ops import patterns
 
-            pats = cp.patset.patterns
-            res = patterns().score_events(
-                hits[:, 0].tolist(), hits[:, 1].tolist(), hits[:, 2].tolist(), len(docs),
-                cp.pattern_primary, [p.primary.confidence for p in pats], [p.severity_rank for p in pats],
-                cp.pattern_secondary, [[s.weight for s in p.secondary] for p in pats],
-                [[s.window for s in p.secondary] for p in pats], cp.num_matchers)
-            evs = [[oracle.Event(int(p), int(l), float(s)) for (p, l, s) in d] for d in res]
+                pats = cp.patset.patterns
+                self._scorer = patterns().Scorer(
+                    cp.pattern_primary, [p.primary.confidence for p in pats], [p.severity_rank for p in pats],
+                    cp.pattern_secondary, [[s.weight for s in p.secondary] for p in pats],
+                    [[s.window for s in p.secondary] for p in pats], cp.num_matchers)
+            evs = [[oracle.Event(*e) for e in d] for d in self._scorer.score(hits, len(docs))]
         else:
             per: list[set] = [set() for _ in docs]
             for d_, m_, l_ in hits.tolist():
@@ -747,7 +771,7 @@ class MatchEngine:
             q_doc.extend([di] * len(o_))
             q_off.extend(o_)
             q_k.extend(k_)
-        ctxs = self._contexts_gpu(docs, q_doc, q_off, q_k, resident, stream) if q_doc else None
+        ctxs = self._contexts_gpu(docs, q_doc, q_off, q_k, resident, stream) if q_doc and len(docs) > self.HOST_CONTEXT_DOCS else None
         if ctxs is None:
             ctxs = patterns().contexts(docs, q_doc, q_off, q_k) if q_doc else []
         starts = [0]
