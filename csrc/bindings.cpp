@@ -593,7 +593,7 @@ void attn_prefill(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
 
 void sample(const at::Tensor& logits, const at::Tensor& temperature, const at::Tensor& seeds,
             const at::Tensor& positions, at::Tensor& out, int64_t col_offset,
-            const c10::optional<at::Tensor>& out_val) {
+            const c10::optional<at::Tensor>& out_val, const c10::optional<at::Tensor>& part) {
   CHECK_DEV(logits);
   TORCH_CHECK(logits.dim() == 2 && logits.stride(1) == 1, "logits must be [rows, vocab] row-major");
   TORCH_CHECK(logits.scalar_type() == at::kFloat || logits.scalar_type() == at::kBFloat16, "logits dtype");
@@ -605,10 +605,14 @@ void sample(const at::Tensor& logits, const at::Tensor& temperature, const at::T
     CHECK_DT(*out_val, at::kFloat);
     TORCH_CHECK(out_val->numel() == rows, "out_val shape");
   }
+  if (part.has_value()) {
+    CHECK_DEV(*part); CHECK_DT(*part, at::kFloat); CHECK_CONTIG(*part);
+    TORCH_CHECK(part->numel() >= 2 * rows * oamd::sample_parts((int)rows, (int)logits.size(1)), "sampler workspace too small");
+  }
   const c10::hip::HIPGuardMasqueradingAsCUDA g(logits.device());
   RC(oamd::sample_tokens(logits.data_ptr(), logits.scalar_type() == at::kBFloat16, logits.stride(0), (int)rows,
                          (int)logits.size(1), ptr<float>(temperature), ptr<int64_t>(seeds), ptr<int64_t>(positions),
-                         ptr<int64_t>(out), col_offset, optr<float>(out_val), cur_stream()));
+                         ptr<int64_t>(out), col_offset, optr<float>(out_val), optr<float>(part), cur_stream()));
 }
 
 }  // namespace
@@ -685,7 +689,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("attn_prefill_block_q", &oamd::attn_prefill_block_q);
   m.def("sample", &sample, pybind11::arg("logits"), pybind11::arg("temperature"), pybind11::arg("seeds"),
         pybind11::arg("positions"), pybind11::arg("out"), pybind11::arg("col_offset") = 0,
-        pybind11::arg("out_val") = pybind11::none());
+        pybind11::arg("out_val") = pybind11::none(), pybind11::arg("part") = pybind11::none());
+  m.def("sample_parts", &oamd::sample_parts, pybind11::arg("rows"), pybind11::arg("vocab"));
   m.def("graph_launch", &graph_launch, pybind11::arg("graph_exec"), pybind11::arg("count"), pybind11::arg("stream"));
   register_decoder_bindings(m);
   m.attr("ARCH") = "gfx950";

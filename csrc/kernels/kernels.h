@@ -129,7 +129,8 @@ int attn_prefill(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16_t* o, c
                  const bf16_t* pk = nullptr, const bf16_t* pv = nullptr, const int* seq_pfx = nullptr);
 int sample_tokens(const void* logits, bool logits_bf16, int64_t stride, int rows, int vocab,
                   const float* temperature, const int64_t* seeds, const int64_t* positions,
-                  int64_t* out_tokens, int64_t col_offset, float* out_val, hipStream_t stream);
+                  int64_t* out_tokens, int64_t col_offset, float* out_val, float* part, hipStream_t stream);
+int sample_parts(int rows, int vocab);   // part: 2 x rows x sample_parts floats, or nullptr (one workgroup per row)
 
 // One-shot all-reduce over peer-mapped fine-grained buffers (allreduce.hip).
 size_t car_buffer_bytes(size_t cap_bytes, int world);

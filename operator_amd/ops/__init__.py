@@ -778,7 +778,10 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, seeds: torch.Tensor,
             return out
         return tok
     o = out if out is not None else torch.empty(logits.shape[0], dtype=torch.long, device=logits.device)
-    kernels().sample(logits, temperature, seeds, positions, o, col_offset, out_val)
+    rows = logits.shape[0]
+    parts = kernels().sample_parts(rows, logits.shape[1])   # workgroups per row, merged by a second kernel
+    part = torch.empty(2 * rows * parts, dtype=torch.float32, device=logits.device) if parts > 1 else None
+    kernels().sample(logits, temperature, seeds, positions, o, col_offset, out_val, part)
     return o
 
 
