@@ -19,7 +19,7 @@ from ._native import kernels, native_available, patterns
 __all__ = [
     "rmsnorm", "silu_mul", "embedding", "rope_kv", "attn_prefill", "attn_decode", "attn_decode_rope", "sample",
     "kernels", "patterns", "native_available", "reference", "prefill_work_list", "prefill_block_q", "prefill_variant", "decode_splits",
-    "decode_workspace", "linear", "gemm_splits", "gemm_plan", "gate_up_silu", "interleave_gate_up",
+    "decode_workspace", "linear", "gemm_plan", "gate_up_silu", "interleave_gate_up",
     "quantize_fp8", "silu_quantize_fp8", "linear_fp8", "fp8_plan", "SplitK", "linear_tile", "tile_ok", "BLAS_CALLS",
     "linear_f32", "decoder",
 ]
@@ -100,14 +100,31 @@ def interleave_gate_up(g: torch.Tensor, u: torch.Tensor, block: int = GU_BLOCK) 
         2 * inter, H).contiguous()
 
 
-def _gu_splits(M: int, N: int, K: int) -> int:
-    """K slices of a narrow gate|up decode GEMM: one block per 128-column tile leaves most CUs
+def _gu_splits(M: int, N: int, K: int, bm: int = 0) -> int:
+    """K slices of a narrow gate|up decode GEMM: one block per tile leaves most CUs
     idle below 96 tiles, and the extra SwiGLU pass over the slabs is worth it."""
-    tiles = N // 128 * (M // row_tile(M))
+    tiles = N // 128 * (M // (bm or row_tile(M)))
     S = 1
     while tiles * S < 96 and S < 8 and K // 64 >= 4 * S:
         S *= 2
     return S
+
+
+def gate_up_plan(M: int, N: int):
+    """Kernel of a gate|up decode bucket of 64 to 256 rows without a measured entry: row tile of gemm_decode, "pp256" /
+    "pp128" (gemm_pp) or None (gemm_mid). A workgroup takes in about 45 bytes per ns of both operands, so the
+    smallest tile that still leaves one workgroup per CU wins (256 rows of 16384 x 2048: two 128-row tiles 28 us,
+    one of 256 38; 128 rows of it: 64-row tiles 22 us, 128 25), then the one whose workgroups come in one round
+    (128 rows of 57344 x 8192: gemm_mid's 224 units 179 us, gemm_pp 217). 256 rows stay on gemm_pp: gemm_mid's W
+    tile goes to two CUs (28672 x 4096 by itself 70 us against 78, but 12 us behind within a decode step)."""
+    tiles = N // 128
+    if M == 64:
+        return 64
+    if M == 128:
+        return 64 if 2 * tiles <= CUS else "pp128" if tiles <= CUS else None
+    if M == 256:
+        return 128 if 2 * tiles <= CUS else "pp256"
+    return 64 if M // 64 * tiles <= CUS else None
 
 
 def gate_up_silu(x: torch.Tensor, wgu: torch.Tensor, block: int | None, act: int = SILU) -> torch.Tensor:
@@ -127,20 +144,22 @@ def gate_up_silu(x: torch.Tensor, wgu: torch.Tensor, block: int | None, act: int
     if (x.is_cuda and block == 64 and x.dtype == torch.bfloat16 and M % 64 == 0 and M <= 256 and N % 128 == 0
             and K % 64 == 0 and x.is_contiguous() and wgu.is_contiguous()):
         t = _gemm_table_get().get(("silu", M, N, K))
-        if isinstance(t, str) and t.startswith("pp"):   # ping-pong kernel, nt weight loads (bm 128 / 256)
+        bm = gate_up_plan(M, N) if t is None else t if isinstance(t, str) else t[0]
+        if t is None and bm is None:
+            return linear_tile(x, wgu, glu=act)
+        if isinstance(bm, str) and bm.startswith("pp"):   # ping-pong kernel, nt weight loads (bm 128 / 256)
             y = torch.empty(M, N // 2, dtype=x.dtype, device=x.device)
-            bm = int(t[2:])
+            bm = int(bm[2:])
             ws, fl = _pp_sk_workspace(x.device, N // 128) if (bm == 256 and PP_STREAM_K) else (None, None)
             kernels().gemm_pp(x, wgu, y, None, 1, bm, act, True, False, ws, fl)
             return y
-        if t is None and (S := _gu_splits(M, N, K)) > 1:   # too few column tiles to fill the GPU: split K
+        if t is None and (S := _gu_splits(M, N, K, bm)) > 1:   # too few column tiles to fill the GPU: split K
             y = torch.empty(M, N // 2, dtype=x.dtype, device=x.device)
             slabs = torch.empty(S * M * N, dtype=torch.float32, device=x.device)
-            kernels().gemm_decode(x, wgu, None, slabs, S, 128, row_tile(M), False, False, 3)
+            kernels().gemm_decode(x, wgu, None, slabs, S, 128, bm, False, False, 3)
             kernels().splitk_silu(slabs, y, S, act)
             return y
         if t != "blas":
-            bm = t[0] if t else row_tile(M)
             ns = t[1] if t and len(t) > 1 else 3
             y = torch.empty(M, N // 2, dtype=x.dtype, device=x.device)
             kernels().gemm_decode(x, wgu, y, None, 1, 128, bm, act, False, ns)
@@ -339,22 +358,9 @@ def _measured_blas(M: int, N: int, K: int) -> bool:
     return t.get(("skinny", M, N, K) if M <= SKINNY_MAX_M else (M, N, K)) == "blas"
 
 
-def gemm_splits(M: int, N: int, K: int) -> int:
-    """Heuristic split-K ways for gemm_decode (shapes not in the tuned table): the
-    smallest S | 8 whose (N/64) x S blocks reach one block per CU (256)."""
-    tiles = N // 64
-    best = 1
-    for S in (1, 2, 4, 8):
-        if K % (64 * S):
-            break
-        best = S
-        if tiles * S >= 256:
-            return S
-    return best
-
-
-def gemm_plan(M: int, N: int, K: int):
-    """(bm, bn, splits) for the gfx950 gemm_decode kernel, or None for hipBLASLt."""
+def gemm_plan(M: int, N: int, K: int, defer: bool = True):
+    """(bm, bn, splits, stages) for the gfx950 gemm_decode kernel, or None for the tile kernels (or hipBLASLt).
+    ``defer``: the consumer sums the K slices."""
     if M % 64 or N % 64 or K % 64 or M > 256:
         return None
     t = _gemm_table_get().get((M, N, K))
@@ -364,7 +370,35 @@ def gemm_plan(M: int, N: int, K: int):
         return tuple(t)   # (bm, bn, S[, stages]) for gemm_decode
     if N >= LM_HEAD_MIN_N:
         return _vocab_plan(M, N, K)
-    return (row_tile(M), 64, gemm_splits(M, N, K))
+    return _decode_tiles(M, N, K, defer)
+
+
+def _slab_us(S: int, M: int, N: int, defer: bool) -> float:
+    """Writing and reading S fp32 slabs, and the reduce pass where the consumer does not sum them."""
+    return 0.0 if S == 1 else S * M * N * 1.8e-6 + (0 if defer else 6)
+
+
+@functools.lru_cache(maxsize=4096)
+def _decode_tiles(M: int, N: int, K: int, defer: bool):
+    """Tile, K slices and stages of a decode bucket's projection. A CU takes in 40 to 47 bytes per ns through LDS-DMA
+    whatever the tile, so a workgroup's time is its K steps times its (rows + columns) of 128 bytes, and the best
+    plan has the fewest such bytes at one workgroup per CU: 64 rows of 5120 x 14336 in 64 x 128 tiles and 5
+    slices 29 us (64 x 64 tiles, 4 slices: 42), 256 rows of 3584 x 3584 in 128 x 128 tiles 14 (256 x 64: 19), 64
+    rows of 2048 x 2048 in 64 x 64 tiles 4.6. None: gemm_mid, whose loop is a little faster but starts later (256
+    rows of 8192 x 8192: 42 us against 46 and the former 61)."""
+    best = None
+    for bm in (64, 128, 256):
+        for bn in (64, 128):
+            if M % bm or N % bn:
+                continue
+            tiles = M // bm * (N // bn)
+            for S in range(1, max(1, min(16, K // 128, CUS // tiles)) + 1):
+                t = 4 + -(-tiles * S // CUS) * -(-(K // 64) // S) * (bm + bn) * 128 / 45e3 + _slab_us(S, M, N, defer)
+                cost = (max(t, 2e-6 * N * K / 5.8), t)
+                if best is None or cost < best[0]:
+                    best = cost, (bm, bn, S, 4 if bm + bn <= 320 else 3)
+    S = mid_plan(M, N, K, defer)
+    return None if S is not None and _mid_cost(M, N, K, S, defer) < best[0][0] else best[1]
 
 
 def _vocab_plan(M: int, N: int, K: int):
@@ -465,11 +499,9 @@ def _mid_cost(M: int, N: int, K: int, S: int, defer: bool) -> float:
     mt = -(-M // 128)
     units = mt * -(-N // 256) * S
     rounds = -(-units // CUS)
-    step = 0.7 + 0.15 * min(1.0, units / CUS) + (0.12 if mt == 1 else 0.0)
-    t = 4 + rounds * -(-(K // 64) // S) * step + 3 * (rounds - 1)   # a tile's stores between rounds
-    if S > 1:
-        t += S * M * N * 4e-6 * (1 / 4 + 1 / 5) + (0 if defer else 6)
-    return max(t, 2e-6 * N * K / 4.9)
+    step = 0.7 + (0.15 if M > 256 else 0.3) * min(1.0, units / CUS)   # few rows: the weights come from HBM
+    t = (4 if M > 256 else 6) + rounds * -(-(K // 64) // S) * step + 3 * (rounds - 1)   # a tile's stores between rounds
+    return max(t + _slab_us(S, M, N, defer), 2e-6 * N * K / 4.9)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -571,7 +603,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, sp
             kernels().gemm_skinny(x, w, y, partial if S > 1 else None, S, False)
             return y
     if x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous():
-        plan = gemm_plan(M, N, K)
+        plan = gemm_plan(M, N, K, defer_reduce and out is None)
         if plan is None and (splits or bn or bm) and M % 64 == 0 and M <= 256 and N % 64 == 0 and K % 64 == 0:
             plan = (row_tile(M), 64, 1)  # explicit request (tests / tuning)
     if plan is None:
