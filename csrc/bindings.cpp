@@ -472,6 +472,35 @@ void gemm_fp8(const at::Tensor& x8, const at::Tensor& w8, const at::Tensor& sx, 
                     (int)bm, cur_stream()));
 }
 
+// y omitted: the consumer sums the fp32 slabs
+void gemm_fp8_tile(const at::Tensor& x8, const at::Tensor& w8, const at::Tensor& sx, const at::Tensor& sw,
+                   const c10::optional<at::Tensor>& y, const c10::optional<at::Tensor>& p, int64_t splits) {
+  CHECK_DEV(x8); CHECK_CONTIG(x8); CHECK_CONTIG(w8); CHECK_CONTIG(sx); CHECK_CONTIG(sw); CHECK_DT(sx, at::kFloat); CHECK_DT(sw, at::kFloat);
+  for (auto* t : {&x8, &w8})
+    TORCH_CHECK(t->scalar_type() == at::kByte || t->scalar_type() == at::kFloat8_e4m3fn, "fp8 operands");
+  TORCH_CHECK(x8.dim() == 2 && w8.dim() == 2, "x8 [M,K], w8 [N,K]");
+  const int64_t M = x8.size(0), K = x8.size(1), N = w8.size(0);
+  TORCH_CHECK(w8.size(1) == K && sx.numel() == M && sw.numel() == N, "gemm_fp8_tile shapes");
+  TORCH_CHECK(N >= 16 && N % 16 == 0 && K % 128 == 0 && N < (1LL << 31) && M < (1LL << 31) && K < (1LL << 23),
+              "gemm_fp8_tile: N % 16 == 0, K % 128 == 0");
+  TORCH_CHECK(splits >= 1 && splits <= 16 && K / 128 / splits >= 3, "gemm_fp8_tile: slices of at least 3 x 128");
+  if (y.has_value()) {
+    CHECK_BF16(*y); CHECK_CONTIG(*y);
+    TORCH_CHECK(y->dim() == 2 && y->size(0) == M && y->size(1) == N && reinterpret_cast<uintptr_t>(y->data_ptr()) % 16 == 0, "gemm_fp8_tile: y [M, N], 16-B aligned");
+  } else {
+    TORCH_CHECK(splits > 1, "y may be omitted only for slabs summed by the consumer");
+  }
+  float* pp = nullptr;
+  if (splits > 1) {
+    TORCH_CHECK(p.has_value() && p->scalar_type() == at::kFloat && p->is_contiguous() && p->numel() >= splits * M * N,
+                "split-K needs an fp32 partial buffer");
+    pp = p->data_ptr<float>();
+  }
+  const c10::hip::HIPGuardMasqueradingAsCUDA g(x8.device());
+  RC(oamd::gemm_fp8_tile(static_cast<const uint8_t*>(x8.data_ptr()), static_cast<const uint8_t*>(w8.data_ptr()), ptr<float>(sx),
+                         ptr<float>(sw), optr<bf16_t>(y), pp, (int)M, (int)N, (int)K, (int)splits, cur_stream()));
+}
+
 void attn_decode(const at::Tensor& q, const at::Tensor& k_cache, const at::Tensor& v_cache,
                  const at::Tensor& block_tables, const at::Tensor& seq_lens, at::Tensor& out,
                  at::Tensor& o_part, at::Tensor& ml_part, int64_t num_splits, double scale, int64_t variant,
@@ -663,6 +692,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("quantize_fp8", &quantize_fp8);
   m.def("silu_quantize_fp8", &silu_quantize_fp8, pybind11::arg("gu"), pybind11::arg("q"), pybind11::arg("sx"),
         pybind11::arg("slabs") = pybind11::none(), pybind11::arg("splits") = 1);
+  m.def("gemm_fp8_tile", &gemm_fp8_tile, pybind11::arg("x8"), pybind11::arg("w8"), pybind11::arg("sx"), pybind11::arg("sw"),
+        pybind11::arg("y"), pybind11::arg("p") = pybind11::none(), pybind11::arg("splits") = 1);
   m.def("gemm_fp8", &gemm_fp8, pybind11::arg("x8"), pybind11::arg("w8"), pybind11::arg("sx"), pybind11::arg("sw"),
         pybind11::arg("y"), pybind11::arg("p") = pybind11::none(), pybind11::arg("splits") = 1,
         pybind11::arg("bn") = 64, pybind11::arg("bm") = 64, pybind11::arg("reduce") = true);

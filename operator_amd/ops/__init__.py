@@ -370,7 +370,7 @@ def gemm_plan(M: int, N: int, K: int, defer: bool = True):
         return tuple(t)   # (bm, bn, S[, stages]) for gemm_decode
     if N >= LM_HEAD_MIN_N:
         return _vocab_plan(M, N, K)
-    return _decode_tiles(M, N, K, defer)
+    return _decode_plan(M, N, K, defer)
 
 
 def _slab_us(S: int, M: int, N: int, defer: bool) -> float:
@@ -380,12 +380,11 @@ def _slab_us(S: int, M: int, N: int, defer: bool) -> float:
 
 @functools.lru_cache(maxsize=4096)
 def _decode_tiles(M: int, N: int, K: int, defer: bool):
-    """Tile, K slices and stages of a decode bucket's projection. A CU takes in 40 to 47 bytes per ns through LDS-DMA
+    """(estimate in us, (rows, columns, K slices, stages)) of a decode bucket's projection on gemm_decode. A CU takes in 40 to 47 bytes per ns through LDS-DMA
     whatever the tile, so a workgroup's time is its K steps times its (rows + columns) of 128 bytes, and the best
     plan has the fewest such bytes at one workgroup per CU: 64 rows of 5120 x 14336 in 64 x 128 tiles and 5
     slices 29 us (64 x 64 tiles, 4 slices: 42), 256 rows of 3584 x 3584 in 128 x 128 tiles 14 (256 x 64: 19), 64
-    rows of 2048 x 2048 in 64 x 64 tiles 4.6. None: gemm_mid, whose loop is a little faster but starts later (256
-    rows of 8192 x 8192: 42 us against 46 and the former 61)."""
+    rows of 2048 x 2048 in 64 x 64 tiles 4.6."""
     best = None
     for bm in (64, 128, 256):
         for bn in (64, 128):
@@ -397,8 +396,15 @@ def _decode_tiles(M: int, N: int, K: int, defer: bool):
                 cost = (max(t, 2e-6 * N * K / 5.8), t)
                 if best is None or cost < best[0]:
                     best = cost, (bm, bn, S, 4 if bm + bn <= 320 else 3)
+    return best[0][0], best[1]
+
+
+def _decode_plan(M: int, N: int, K: int, defer: bool):
+    """_decode_tiles' plan, or None for gemm_mid, whose loop is a little faster but starts later (256 rows of
+    8192 x 8192: 42 us against 46 and, in 256 x 64 tiles, 61)."""
+    cost, plan = _decode_tiles(M, N, K, defer)
     S = mid_plan(M, N, K, defer)
-    return None if S is not None and _mid_cost(M, N, K, S, defer) < best[0][0] else best[1]
+    return None if S is not None and _mid_cost(M, N, K, S, defer) < cost else plan
 
 
 def _vocab_plan(M: int, N: int, K: int):
@@ -673,22 +679,58 @@ def _fp8_overrides() -> dict:
 _FP8_OVERRIDES = _fp8_overrides()
 
 
-def fp8_plan(M: int, N: int, K: int) -> tuple[int, int, int]:
-    """(bm, bn, splits) for gemm_fp8: row tile by M, 128-column tiles for wide N, and
-    split-K until the blocks reach one per CU (K permitting)."""
-    if (N, K) in _FP8_OVERRIDES:
-        return _FP8_OVERRIDES[(N, K)]
+def _fp8_slices(M: int, N: int, K: int) -> tuple[int, int, int]:
+    """(rows, columns, K slices) of an fp8 projection: a power of two of slices until blocks of (64, 128 or 256) rows and
+    64 columns (128 of wide N) reach one per CU. Both kernels keep to the slices, whatever the tile: they fix the order
+    of a sum, and rows whose rounding to e4m3fn turns on its last bit come out visibly different further on."""
     bm = 64 if M <= 64 else 128 if M <= 128 else 256
     bn = 128 if N % 128 == 0 and N // 128 >= 192 else 64
-    mt = -(-M // bm)
     S = 1
     for s in (1, 2, 4, 8):
         if K % (128 * s):
             break
         S = s
-        if (N // bn) * s * mt >= 256:
+        if (N // bn) * s * -(-M // bm) >= CUS:
             break
     return bm, bn, S
+
+
+# us of a 128-K step of gemm_fp8's tiles, every CU busy (8192 x 28672, 57344 x 8192)
+_FP8_STEP = {(64, 64): 0.40, (64, 128): 0.56, (128, 64): 0.51, (128, 128): 0.80, (256, 64): 0.71, (256, 128): 1.16}
+
+
+@functools.lru_cache(maxsize=4096)
+def _fp8_tiles(M: int, N: int, K: int):
+    """(estimate in us, (bm, bn, S)) of gemm_fp8: the tile with the shortest rounds (128 rows of 10240 x 8192 in 128 x 128
+    tiles: one round of 160 workgroups 30 us, two of 128 x 64 35). Up to 64 rows two or three workgroups share a CU and
+    the narrow tile stays (1 row: 20.5 against 21.3)."""
+    bm, bn, S = _fp8_slices(M, N, K)
+    steps = -(-(K // 128) // S)
+    best = None
+    for (r, c), step in _FP8_STEP.items():
+        if N % c == 0 and (M > 64 or (r, c) == (bm, bn)):
+            t = 4 + -(-(-(-M // r) * (N // c) * S) // CUS) * steps * step
+            best = min(best or (t, (r, c, S)), (t, (r, c, S)))
+    return best or (float("inf"), (bm, bn, S))
+
+
+def fp8_plan(M: int, N: int, K: int) -> tuple[int, int, int]:
+    """(bm, bn, splits) for gemm_fp8."""
+    return _FP8_OVERRIDES.get((N, K)) or _fp8_tiles(M, N, K)[1]
+
+
+def fp8_tile_plan(M: int, N: int, K: int) -> int | None:
+    """The slices where gemm_fp8_tile's 128 x 256 tiles are faster than gemm_fp8's, else None: 512 rows of
+    57344 x 8192 306 -> 229 us, 4096 rows of 8192 x 8192 384 -> 208 (2.6 PFLOP/s), 256 rows of 10240 x 8192 57 -> 36; but
+    512 rows of 8192 x 28672 in one slice 187, against 158, and up to 64 rows the weights' stream is all there is
+    (57344 x 8192: 104, against 90)."""
+    S = _fp8_slices(M, N, K)[2]
+    if M <= 64 or N % 64 or K // 128 // S < 3 or (N, K) in _FP8_OVERRIDES:
+        return None
+    units = -(-M // 128) * -(-N // 256) * S
+    step = 0.7 + (0.15 if M > 256 else 0.3) * min(1.0, units / CUS)
+    cost = 6 + -(-units // CUS) * -(-(K // 128) // S) * step
+    return S if cost < _fp8_tiles(M, N, K)[0] else None
 
 
 def linear_fp8(x: torch.Tensor | tuple[torch.Tensor, torch.Tensor], w8: torch.Tensor, sw: torch.Tensor,
@@ -704,10 +746,17 @@ def linear_fp8(x: torch.Tensor | tuple[torch.Tensor, torch.Tensor], w8: torch.Te
     if not q.is_cuda:
         y = (q.float() * sx[:, None]) @ (w8.float() * sw[:, None]).t()
         return out.copy_(y) if out is not None else y.to(torch.bfloat16 if isinstance(x, tuple) else x.dtype)
+    defer = defer_reduce and out is None
+    if plan is None and M and (out is None or (out.is_contiguous() and out.data_ptr() % 16 == 0)) and (
+            S := fp8_tile_plan(M, N, K)) is not None and (q.data_ptr() | w8.data_ptr()) % 16 == 0:
+        part = torch.empty(S * M * N, dtype=torch.float32, device=q.device) if S > 1 else None
+        y = None if defer and S > 1 else out if out is not None else torch.empty(M, N, dtype=torch.bfloat16, device=q.device)
+        kernels().gemm_fp8_tile(q, w8, sx, sw, y, part, S)
+        return SplitK(part, S, M, N) if y is None else y
     bm, bn, S = plan or fp8_plan(M, N, K)
     y = out if out is not None else torch.empty(M, N, dtype=torch.bfloat16, device=q.device)
     part = torch.empty(S * M * N, dtype=torch.float32, device=q.device) if S > 1 else None
-    if defer_reduce and S > 1 and out is None:
+    if defer and S > 1:
         kernels().gemm_fp8(q, w8, sx, sw, y, part, S, bn, bm, False)
         return SplitK(part, S, M, N)
     kernels().gemm_fp8(q, w8, sx, sw, y, part, S, bn, bm)
