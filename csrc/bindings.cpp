@@ -62,6 +62,36 @@ void rmsnorm(const at::Tensor& x, const c10::optional<at::Tensor>& residual, con
                    cur_stream()));
 }
 
+// rmsnorm with the row quantized to e4m3fn: x bf16 rows, or fp32 slabs [splits, rows, hidden] in `partial`
+void rmsnorm_fp8(const c10::optional<at::Tensor>& x, const c10::optional<at::Tensor>& residual, const at::Tensor& w, at::Tensor& q,
+                 at::Tensor& sx, double eps, const c10::optional<at::Tensor>& partial, int64_t splits) {
+  CHECK_DEV(q); CHECK_CONTIG(q); CHECK_CONTIG(sx); CHECK_DT(sx, at::kFloat); CHECK_BF16(w); CHECK_CONTIG(w);
+  TORCH_CHECK(q.dim() == 2 && (q.scalar_type() == at::kByte || q.scalar_type() == at::kFloat8_e4m3fn), "q must be [rows, hidden] uint8 / e4m3fn");
+  const int64_t rows = q.size(0), hidden = q.size(1);
+  TORCH_CHECK(hidden % 8 == 0 && hidden <= 256 * 8 * 8, "hidden must be a multiple of 8 and <= 16384");
+  TORCH_CHECK(w.numel() == hidden && sx.numel() == rows, "rmsnorm_fp8 shape mismatch");
+  TORCH_CHECK(x.has_value() != partial.has_value(), "rmsnorm_fp8: rows or slabs");
+  const float* xp = nullptr;
+  int64_t xstride = 0, rstride = 0;
+  if (partial.has_value()) {
+    CHECK_DT(*partial, at::kFloat); CHECK_CONTIG(*partial);
+    TORCH_CHECK(splits >= 1 && partial->numel() >= splits * rows * hidden, "rmsnorm_fp8: partial slabs too small");
+    xp = partial->data_ptr<float>();
+  } else {
+    CHECK_BF16(*x); ROWMAJOR_VEC(*x);
+    TORCH_CHECK(x->size(0) == rows && x->size(1) == hidden, "rmsnorm_fp8 shape mismatch");
+    xstride = x->stride(0);
+  }
+  if (residual.has_value()) {
+    CHECK_BF16(*residual); ROWMAJOR_VEC(*residual);
+    TORCH_CHECK(residual->size(0) == rows && residual->size(1) == hidden, "residual shape mismatch");
+    rstride = residual->stride(0);
+  }
+  const c10::hip::HIPGuardMasqueradingAsCUDA g(q.device());
+  RC(oamd::rmsnorm_fp8(optr<bf16_t>(x), optr<bf16_t>(residual), ptr<bf16_t>(w), static_cast<uint8_t*>(q.data_ptr()), ptr<float>(sx),
+                       (int)rows, (int)hidden, xstride, rstride, (float)eps, xp, (int)splits, cur_stream()));
+}
+
 // gemm_xr (csrc/kernels/gemm_xr.hip): the 256-row decode GEMM with register-streamed activations.
 // xt: the activations [256, K] in the tiled layout (rmsnorm(tiled_out=True) / tile_rows / the SwiGLU
 // epilogue with epi 3); epi 0 = fp32 split-K slabs into p, 1 = bf16 y [256, N], 2 = SwiGLU y [256, N/2],
@@ -431,7 +461,7 @@ void silu_quantize_fp8(const at::Tensor& gu, at::Tensor& q, at::Tensor& sx, cons
   TORCH_CHECK(gu.dim() == 2 && gu.stride(1) == 1, "gu must be [M, 2I] row-major");
   TORCH_CHECK(q.scalar_type() == at::kByte || q.scalar_type() == at::kFloat8_e4m3fn, "q must be uint8 / e4m3fn");
   const int64_t M = gu.size(0), I = gu.size(1) / 2;
-  TORCH_CHECK(gu.size(1) % 128 == 0 && I <= 16384, "silu_quantize_fp8: 2I % 128 == 0, I <= 16384");
+  TORCH_CHECK(gu.size(1) % 128 == 0 && I <= 32768, "silu_quantize_fp8: 2I % 128 == 0, I <= 32768");
   TORCH_CHECK(q.numel() == M * I && sx.numel() == M, "silu_quantize_fp8 shapes");
   const float* pp = nullptr;
   if (slabs.has_value()) {
@@ -692,6 +722,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("quantize_fp8", &quantize_fp8);
   m.def("silu_quantize_fp8", &silu_quantize_fp8, pybind11::arg("gu"), pybind11::arg("q"), pybind11::arg("sx"),
         pybind11::arg("slabs") = pybind11::none(), pybind11::arg("splits") = 1);
+  m.def("rmsnorm_fp8", &rmsnorm_fp8, pybind11::arg("x"), pybind11::arg("residual"), pybind11::arg("w"), pybind11::arg("q"),
+        pybind11::arg("sx"), pybind11::arg("eps"), pybind11::arg("partial") = pybind11::none(), pybind11::arg("splits") = 1);
   m.def("gemm_fp8_tile", &gemm_fp8_tile, pybind11::arg("x8"), pybind11::arg("w8"), pybind11::arg("sx"), pybind11::arg("sw"),
         pybind11::arg("y"), pybind11::arg("p") = pybind11::none(), pybind11::arg("splits") = 1);
   m.def("gemm_fp8", &gemm_fp8, pybind11::arg("x8"), pybind11::arg("w8"), pybind11::arg("sx"), pybind11::arg("sw"),

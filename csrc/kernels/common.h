@@ -72,6 +72,16 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// e4m3fn of v[0..7] * inv.
+__device__ __forceinline__ uint2 pack_fp8x8(const float (&v)[8], float inv) {
+  int lo = 0, hi = 0;
+  lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[0] * inv, v[1] * inv, lo, false);
+  lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[2] * inv, v[3] * inv, lo, true);
+  hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[4] * inv, v[5] * inv, hi, false);
+  hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[6] * inv, v[7] * inv, hi, true);
+  return make_uint2(static_cast<uint32_t>(lo), static_cast<uint32_t>(hi));
+}
+
 // Sum within aligned groups of `width` lanes (width power of two <= 64).
 template <int WIDTH>
 __device__ __forceinline__ float group_sum(float v) {

@@ -142,10 +142,11 @@ __global__ void __launch_bounds__(f8::kWaves * 64, 1)
 }
 
 // Per-row dynamic quantization: sx[m] = max|x[m, :]| / 448, q = e4m3fn(x / sx).
-// One 256-thread block per row. Rows of up to 256 x 8 x MAXV elements are loaded ONCE
+// One block of NT threads per row. Rows of up to NT x 8 x MAXV elements are loaded ONCE
 // into registers (all loads in flight together), reduced, then quantized from the
 // registers: a decode row is latency-bound, and the former two streaming passes with
 // a dependent load per step cost 12.6 us for a 64 x 8192 block (profiles/tp8_sim_*).
+// Rows past 8192 take 1024 threads, up to 32768 (64 rows of 28672 SwiGLU features: silu_mul + quantize 14 us -> 9).
 // SILU: the input is the 64-feature-interleaved gate|up projection [M, 2K] and the
 // row quantized is bf16(bf16(silu(bf16 g)) * bf16 u) — the SwiGLU and the down
 // projection's input quantization in one kernel.
@@ -153,11 +154,11 @@ __global__ void __launch_bounds__(f8::kWaves * 64, 1)
 // they are summed in slab order and bf16-rounded first (== splitk_reduce_fp32 then SILU).
 // SC (SILU with slabs): compile-time slab count, so every slab load of an element is issued
 // before the first add (0: runtime S, one slab per loop trip).
-template <int MAXV, bool SILU, int SC = 0>
-__global__ void __launch_bounds__(256) quantize_rows_reg_kernel(const bf16_t* __restrict__ x, uint8_t* __restrict__ q,
+template <int MAXV, bool SILU, int SC = 0, int NT = 256>
+__global__ void __launch_bounds__(NT) quantize_rows_reg_kernel(const bf16_t* __restrict__ x, uint8_t* __restrict__ q,
                                                                 float* __restrict__ sx, int K, int64_t ld,
                                                                 const float* __restrict__ P, int S) {
-  __shared__ float red[4];
+  __shared__ float red[NT / 64];
   const int64_t m = blockIdx.x;
   const bf16_t* xr = x + m * ld;
   const int nv = K >> 3;
@@ -165,7 +166,7 @@ __global__ void __launch_bounds__(256) quantize_rows_reg_kernel(const bf16_t* __
   float amax = 0.f;
 #pragma unroll
   for (int i = 0; i < MAXV; ++i) {
-    const int vi = threadIdx.x + i * 256;
+    const int vi = threadIdx.x + i * NT;
     if (vi < nv) {
       if constexpr (SILU) {
         const int c = (vi >> 3) * 128 + (vi & 7) * 8;   // 64-feature blocks: gate then up
@@ -193,6 +194,7 @@ __global__ void __launch_bounds__(256) quantize_rows_reg_kernel(const bf16_t* __
               u1 += sl[s - 1][3];
             }
           } else if constexpr (SC == 0) {
+#pragma unroll 4
             for (int s = 1; s < S; ++s) {
               const float* ps = pr + s * MN;
               g0 += *reinterpret_cast<const f32x4*>(ps);
@@ -229,22 +231,16 @@ __global__ void __launch_bounds__(256) quantize_rows_reg_kernel(const bf16_t* __
   amax = wave_max(amax);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
   __syncthreads();
-  amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+#pragma unroll
+  for (int i = 0; i < NT / 64; ++i) amax = fmaxf(amax, red[i]);
   const float s = amax > 0.f ? amax / 448.f : 1.f;
   const float inv = 1.f / s;
   if (threadIdx.x == 0) sx[m] = s;
   uint8_t* qr = q + m * (int64_t)K;
 #pragma unroll
   for (int i = 0; i < MAXV; ++i) {
-    const int vi = threadIdx.x + i * 256;
-    if (vi < nv) {
-      int lo = 0, hi = 0;
-      lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[i][0] * inv, v[i][1] * inv, lo, false);
-      lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[i][2] * inv, v[i][3] * inv, lo, true);
-      hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[i][4] * inv, v[i][5] * inv, hi, false);
-      hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[i][6] * inv, v[i][7] * inv, hi, true);
-      *reinterpret_cast<uint2*>(qr + vi * 8) = make_uint2(static_cast<uint32_t>(lo), static_cast<uint32_t>(hi));
-    }
+    const int vi = threadIdx.x + i * NT;
+    if (vi < nv) *reinterpret_cast<uint2*>(qr + vi * 8) = pack_fp8x8(v[i], inv);
   }
 }
 
@@ -300,17 +296,18 @@ int silu_quantize_fp8(const bf16_t* gu, const float* P, int S, uint8_t* q, float
   if (inter % 64 != 0 || (gu == nullptr) == (P == nullptr) || S < 1) return -1;
   const int nv = inter / 8;
   const int sc = P == nullptr ? 1 : S;
-#define OAMD_SQ(MV)                                                                                       \
-  switch (sc) {                                                                                           \
-    case 1: quantize_rows_reg_kernel<MV, true, 1><<<M, 256, 0, stream>>>(gu, q, sx, inter, ld, P, S); break; \
-    case 2: quantize_rows_reg_kernel<MV, true, 2><<<M, 256, 0, stream>>>(gu, q, sx, inter, ld, P, S); break; \
-    case 4: quantize_rows_reg_kernel<MV, true, 4><<<M, 256, 0, stream>>>(gu, q, sx, inter, ld, P, S); break; \
-    case 8: quantize_rows_reg_kernel<MV, true, 8><<<M, 256, 0, stream>>>(gu, q, sx, inter, ld, P, S); break; \
-    default: quantize_rows_reg_kernel<MV, true, 0><<<M, 256, 0, stream>>>(gu, q, sx, inter, ld, P, S); break; \
+#define OAMD_SQ(MV, NT)                                                                                         \
+  switch (sc) {                                                                                                 \
+    case 1: quantize_rows_reg_kernel<MV, true, 1, NT><<<M, NT, 0, stream>>>(gu, q, sx, inter, ld, P, S); break; \
+    case 2: quantize_rows_reg_kernel<MV, true, 2, NT><<<M, NT, 0, stream>>>(gu, q, sx, inter, ld, P, S); break; \
+    case 4: quantize_rows_reg_kernel<MV, true, 4, NT><<<M, NT, 0, stream>>>(gu, q, sx, inter, ld, P, S); break; \
+    case 8: quantize_rows_reg_kernel<MV, true, 8, NT><<<M, NT, 0, stream>>>(gu, q, sx, inter, ld, P, S); break; \
+    default: quantize_rows_reg_kernel<MV, true, 0, NT><<<M, NT, 0, stream>>>(gu, q, sx, inter, ld, P, S); break; \
   }
-  if (nv <= 256 * 2) { OAMD_SQ(2) }
-  else if (nv <= 256 * 4) { OAMD_SQ(4) }
-  else if (nv <= 256 * 8) { OAMD_SQ(8) }
+  if (nv <= 256 * 2) { OAMD_SQ(2, 256) }
+  else if (nv <= 256 * 4) { OAMD_SQ(4, 256) }
+  else if (nv <= 1024 * 2) { OAMD_SQ(2, 1024) }
+  else if (nv <= 1024 * 4) { OAMD_SQ(4, 1024) }
   else return -2;
 #undef OAMD_SQ
   OAMD_LAUNCH_CHECK();

@@ -13,6 +13,9 @@ typedef uint16_t bf16_t;
 int rmsnorm(const bf16_t* x, bf16_t* residual, const bf16_t* w, bf16_t* y, int rows, int hidden,
             int64_t x_stride, int64_t r_stride, int64_t y_stride, float eps, const float* xp, int S,
             hipStream_t stream);
+// The same row as e4m3fn q with scale sx, == quantize_fp8_rows(rmsnorm(...)).
+int rmsnorm_fp8(const bf16_t* x, bf16_t* residual, const bf16_t* w, uint8_t* q, float* sx, int rows, int hidden, int64_t x_stride,
+                int64_t r_stride, float eps, const float* xp, int S, hipStream_t stream);
 int silu_mul(const bf16_t* gu, bf16_t* out, int64_t rows, int inter, int block, int64_t in_stride,
              int64_t out_stride, int glu, hipStream_t stream);   // glu: Glu of common.h
 // Decode-step bookkeeping (norm_act.hip): cache slots + sampler positions of the step's tokens,

@@ -17,12 +17,14 @@ namespace oamd {
 // SC = compile-time slab count (0: runtime S) so the S slab loads of a vector are
 // all issued before the first add (a runtime-trip-count loop waits for each load
 // in turn: S dependent L2/HBM round trips per vector).
-template <int NT, int MAXV, int SC>
+// Q8: the row goes out as e4m3fn with its scale amax / 448 instead of bf16, as quantize_fp8_rows makes them of the bf16
+// row: an fp8 projection's input needs no second pass (64 rows of 8192 from 2 slabs: 7.4 + 4.6 us -> 8.0).
+template <int NT, int MAXV, int SC, bool Q8 = false>
 __global__ void __launch_bounds__(NT) rmsnorm_kernel(
     const bf16_t* __restrict__ x, bf16_t* __restrict__ residual,
     const bf16_t* __restrict__ w, bf16_t* __restrict__ y, int hidden,
     int64_t x_stride, int64_t r_stride, int64_t y_stride, float eps,
-    const float* __restrict__ xp, int S_rt, int64_t slab) {
+    const float* __restrict__ xp, int S_rt, int64_t slab, uint8_t* __restrict__ q = nullptr, float* __restrict__ sx = nullptr) {
   const int S = SC > 0 ? SC : S_rt;
   __shared__ float scratch[NT / 64];
   const int row = blockIdx.x;
@@ -52,6 +54,7 @@ __global__ void __launch_bounds__(NT) rmsnorm_kernel(
             hi += ph[sp - 1];
           }
         } else {
+#pragma unroll 4
           for (int sp = 1; sp < S; ++sp) {
             lo += *reinterpret_cast<const f32x4*>(pr + sp * slab);
             hi += *reinterpret_cast<const f32x4*>(pr + sp * slab + 4);
@@ -94,6 +97,34 @@ __global__ void __launch_bounds__(NT) rmsnorm_kernel(
   }
   const float tot = block_sum<NT>(ss, scratch);
   const float rs = rsqrtf(tot / static_cast<float>(hidden) + eps);
+  if constexpr (Q8) {
+    float amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < MAXV; ++i) {
+      if (threadIdx.x + i * NT < nvec) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          v[i][j] = bf2f(f2bf(bf2f(f2bf(v[i][j] * rs)) * bf2f(wpre[i][j])));
+          amax = fmaxf(amax, fabsf(v[i][j]));
+        }
+      }
+    }
+    amax = wave_max(amax);
+    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = amax;   // block_sum ended in a barrier
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NT / 64; ++i) amax = fmaxf(amax, scratch[i]);
+    const float s = amax > 0.f ? amax / 448.f : 1.f;
+    const float inv = 1.f / s;
+    if (threadIdx.x == 0) sx[row] = s;
+    uint2* qr = reinterpret_cast<uint2*>(q + (int64_t)row * hidden);
+#pragma unroll
+    for (int i = 0; i < MAXV; ++i) {
+      const int vi = threadIdx.x + i * NT;
+      if (vi < nvec) qr[vi] = pack_fp8x8(v[i], inv);
+    }
+    return;
+  }
   // y_stride < 0: y is written in the fragment-major tiled layout that gemm_xr reads its
   // activations from (common.h xr_tiled_off; one block per row, rows % 16 == 0)
   const bool tiled = y_stride < 0;
@@ -118,46 +149,53 @@ __global__ void __launch_bounds__(NT) rmsnorm_kernel(
   }
 }
 
-int rmsnorm(const bf16_t* x, bf16_t* residual, const bf16_t* w, bf16_t* y,
-            int rows, int hidden, int64_t x_stride, int64_t r_stride,
-            int64_t y_stride, float eps, const float* xp, int S, hipStream_t stream) {
-  if (rows == 0) return 0;
+template <bool Q8>
+static void rmsnorm_launch(const bf16_t* x, bf16_t* residual, const bf16_t* w, bf16_t* y, int rows, int hidden, int64_t x_stride,
+                           int64_t r_stride, int64_t y_stride, float eps, const float* xp, int S, uint8_t* q, float* sx,
+                           hipStream_t stream) {
   constexpr int NT = 256;
   const int nvec = hidden / 8;
   const int64_t slab = (int64_t)rows * hidden;
   const int sc = xp == nullptr ? 1 : S;
+#define OAMD_RMS(NTH, MV, SCC) \
+  rmsnorm_kernel<NTH, MV, SCC, Q8><<<rows, NTH, 0, stream>>>(x, residual, w, y, hidden, x_stride, r_stride, y_stride, eps, xp, S, slab, q, sx)
+#define OAMD_RMS_S(NTH, MV)                  \
+  switch (sc) {                              \
+    case 1: OAMD_RMS(NTH, MV, 1); break;     \
+    case 2: OAMD_RMS(NTH, MV, 2); break;     \
+    case 4: OAMD_RMS(NTH, MV, 4); break;     \
+    case 8: OAMD_RMS(NTH, MV, 8); break;     \
+    default: OAMD_RMS(NTH, MV, 0); break;    \
+  }
   // split-K slab sums of rows up to 4096 wide: 512 threads, one vector each, so a row's
   // slab loads all leave in one round (OAMD_RMS_WIDE=0: 256 threads x 2 vectors)
   static const bool wide = [] { const char* e = getenv("OAMD_RMS_WIDE"); return !(e && e[0] == '0'); }();
   if (wide && xp != nullptr && sc > 1 && nvec > NT && nvec <= 2 * NT) {
-    switch (sc) {
-      case 2: rmsnorm_kernel<2 * NT, 1, 2><<<rows, 2 * NT, 0, stream>>>(x, residual, w, y, hidden, x_stride, r_stride, y_stride, eps, xp, S, slab); break;
-      case 4: rmsnorm_kernel<2 * NT, 1, 4><<<rows, 2 * NT, 0, stream>>>(x, residual, w, y, hidden, x_stride, r_stride, y_stride, eps, xp, S, slab); break;
-      case 8: rmsnorm_kernel<2 * NT, 1, 8><<<rows, 2 * NT, 0, stream>>>(x, residual, w, y, hidden, x_stride, r_stride, y_stride, eps, xp, S, slab); break;
-      default: rmsnorm_kernel<2 * NT, 1, 0><<<rows, 2 * NT, 0, stream>>>(x, residual, w, y, hidden, x_stride, r_stride, y_stride, eps, xp, S, slab); break;
-    }
-    OAMD_LAUNCH_CHECK();
-    return 0;
-  }
-#define OAMD_RMS(MV, SCC) \
-  rmsnorm_kernel<NT, MV, SCC><<<rows, NT, 0, stream>>>(x, residual, w, y, hidden, x_stride, r_stride, y_stride, eps, xp, S, slab)
-#define OAMD_RMS_S(MV)                  \
-  switch (sc) {                         \
-    case 1: OAMD_RMS(MV, 1); break;     \
-    case 2: OAMD_RMS(MV, 2); break;     \
-    case 4: OAMD_RMS(MV, 4); break;     \
-    case 8: OAMD_RMS(MV, 8); break;     \
-    default: OAMD_RMS(MV, 0); break;    \
-  }
-  if (nvec <= NT * 2) {
-    OAMD_RMS_S(2)
+    OAMD_RMS_S(2 * NT, 1)
+  } else if (nvec <= NT * 2) {
+    OAMD_RMS_S(NT, 2)
   } else if (nvec <= NT * 4) {
-    OAMD_RMS_S(4)
+    OAMD_RMS_S(NT, 4)
   } else {
-    OAMD_RMS_S(8)
+    OAMD_RMS_S(NT, 8)
   }
 #undef OAMD_RMS_S
 #undef OAMD_RMS
+}
+
+int rmsnorm(const bf16_t* x, bf16_t* residual, const bf16_t* w, bf16_t* y,
+            int rows, int hidden, int64_t x_stride, int64_t r_stride,
+            int64_t y_stride, float eps, const float* xp, int S, hipStream_t stream) {
+  if (rows == 0) return 0;
+  rmsnorm_launch<false>(x, residual, w, y, rows, hidden, x_stride, r_stride, y_stride, eps, xp, S, nullptr, nullptr, stream);
+  OAMD_LAUNCH_CHECK();
+  return 0;
+}
+
+int rmsnorm_fp8(const bf16_t* x, bf16_t* residual, const bf16_t* w, uint8_t* q, float* sx, int rows, int hidden, int64_t x_stride,
+                int64_t r_stride, float eps, const float* xp, int S, hipStream_t stream) {
+  if (rows == 0) return 0;
+  rmsnorm_launch<true>(x, residual, w, nullptr, rows, hidden, x_stride, r_stride, 0, eps, xp, S, q, sx, stream);
   OAMD_LAUNCH_CHECK();
   return 0;
 }

@@ -221,9 +221,9 @@ class LlamaModel(DecoderModel):
         """Run all layers; returns logits [n_out, vocab_local] for fb.logits_index rows."""
         c = self.cfg
         h = ops.embedding(fb.input_ids, self.embed)          # residual stream [T, H]
-        x = ops.rmsnorm(h, self.layers[0].attn_norm, c.rms_eps)
         T = h.shape[0]
         q8 = self.fp8 and h.is_cuda   # block epilogues emit e4m3fn rows for the next fp8 GEMM
+        x = (ops.rmsnorm_fp8 if q8 else ops.rmsnorm)(h, self.layers[0].attn_norm, c.rms_eps)
         ws = None
         if not fb.is_prefill and h.is_cuda:  # split-KV partials, shared by every layer
             ws = ops.decode_workspace(T, self.hq, fb.num_splits, h.device)

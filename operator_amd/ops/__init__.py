@@ -20,7 +20,7 @@ __all__ = [
     "rmsnorm", "silu_mul", "embedding", "rope_kv", "attn_prefill", "attn_decode", "attn_decode_rope", "sample",
     "kernels", "patterns", "native_available", "reference", "prefill_work_list", "prefill_block_q", "prefill_variant", "decode_splits",
     "decode_workspace", "linear", "gemm_plan", "gate_up_silu", "interleave_gate_up",
-    "quantize_fp8", "silu_quantize_fp8", "linear_fp8", "fp8_plan", "SplitK", "linear_tile", "tile_ok", "BLAS_CALLS",
+    "quantize_fp8", "rmsnorm_fp8", "silu_quantize_fp8", "linear_fp8", "fp8_plan", "SplitK", "linear_tile", "tile_ok", "BLAS_CALLS",
     "linear_f32", "decoder",
 ]
 
@@ -70,6 +70,17 @@ def rmsnorm(x, w: torch.Tensor, eps: float, residual: torch.Tensor | None = None
     y = out if out is not None else torch.empty_like(x)
     kernels().rmsnorm(x, residual, w, y, eps)
     return y
+
+
+def rmsnorm_fp8(x, w: torch.Tensor, eps: float, residual: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
+    """quantize_fp8(rmsnorm(x, ...)) — on the GPU one kernel, the input of an fp8 projection."""
+    slabs = isinstance(x, SplitK)
+    if not slabs and not x.is_cuda:
+        return quantize_fp8(rmsnorm(x, w, eps, residual=residual))
+    q = torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=x.device)
+    sx = torch.empty(x.shape[0], dtype=torch.float32, device=x.device)
+    kernels().rmsnorm_fp8(None if slabs else x, residual, w, q, sx, eps, *((x.p, x.S) if slabs else ()))
+    return q, sx
 
 
 # activation of a gated feed-forward (common.h Glu): act(gate) * up
@@ -651,7 +662,7 @@ def silu_quantize_fp8(gu, block: int | None = GU_BLOCK) -> tuple[torch.Tensor, t
     the gate|up GEMM's split-K slabs (:class:`SplitK`), summed inside the kernel."""
     M, N2 = gu.shape
     inter = N2 // 2
-    if gu.is_cuda and block == GU_BLOCK and inter <= 16384 and N2 % 128 == 0:
+    if gu.is_cuda and block == GU_BLOCK and inter <= 32768 and N2 % 128 == 0:
         q = torch.empty(M, inter, dtype=torch.float8_e4m3fn, device=gu.device)
         sx = torch.empty(M, dtype=torch.float32, device=gu.device)
         if isinstance(gu, SplitK):

@@ -148,8 +148,7 @@ class Group:
             if isinstance(t, ops.SplitK):
                 t = t.materialize()
             self.all_reduce_(t)
-        y = ops.rmsnorm(t, w, eps, residual=residual)
-        return ops.quantize_fp8(y) if quant else y
+        return (ops.rmsnorm_fp8 if quant else ops.rmsnorm)(t, w, eps, residual=residual)
 
     def all_gather(self, t: torch.Tensor, dim: int = 0) -> torch.Tensor:
         if self.world == 1:
@@ -212,8 +211,7 @@ class SimulatedTPGroup(Group):
         if self.car is not None and self.car.fits_rows(t) and residual.is_contiguous():
             COLLECTIVES.add("all_reduce_rmsnorm", "oneshot-sim", 2 * t.shape[0] * t.shape[1])
             return self.car.all_reduce_rmsnorm_(t, residual, w, eps, quant=quant)
-        y = ops.rmsnorm(t, w, eps, residual=residual)
-        return ops.quantize_fp8(y) if quant else y
+        return (ops.rmsnorm_fp8 if quant else ops.rmsnorm)(t, w, eps, residual=residual)
 
     def all_gather(self, t: torch.Tensor, dim: int = 0) -> torch.Tensor:
         return torch.cat([t] * self.world, dim=dim)
