@@ -355,8 +355,7 @@ void gemm_mid(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::
   }
   if (bias.has_value()) {
     CHECK_DEV(*bias); CHECK_BF16(*bias); CHECK_CONTIG(*bias);
-    TORCH_CHECK(bias->numel() == N && splits == 1 && reinterpret_cast<uintptr_t>(bias->data_ptr()) % 16 == 0,
-                "gemm_mid: bias [N], 16-B aligned, one slice");
+    TORCH_CHECK(bias->numel() == N && reinterpret_cast<uintptr_t>(bias->data_ptr()) % 16 == 0, "gemm_mid: bias [N], 16-B aligned");
   }
   float* pp = nullptr;
   if (splits > 1) {

@@ -8,6 +8,7 @@
 //   885 rows (weights from HBM)   4096 x 14336: 297 -> 103 us, 4096 x 4096: 88 -> 36, 6144 x 4096: 89 -> 56
 //   100 rows                      279 -> 30, 85 -> 16, 85 -> 19
 //   vocabulary 128256 x 8192, 64 rows: 422 -> 373 us (5.6 TB/s of weights)
+// The first slice carries a bias (4608 x 3584, 100 rows: 56 us in one slice, 21 in 7; 300 rows 54, 29 in 3).
 // A 128 x 256 step is 0.7 us (0.43 of MFMA at 2.4 GHz): a CU takes in 50 to 75 bytes per ns through LDS-DMA however
 // many stages wait (a fourth stage of a 64-row tile gained nothing). With every CU busy for several rounds it is
 // 0.85 us, 1.2 PFLOP/s against 1.45 of the 256-row tiles, so those keep the large products (ops.mid_plan).
@@ -236,6 +237,7 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
             const int col = n0 + f * 128 + ty * 64 + wn * 32 + 8 * lq;
             if (tok >= M || col >= N) continue;
             if constexpr (EPI == kEpiPartial) {
+              if (bias != nullptr && kz == 0) add_bias(bias + col, v0, v1);
               float* pr = P + ((int64_t)kz * M + tok) * N + col;
               *reinterpret_cast<f32x4*>(pr) = v0;
               *reinterpret_cast<f32x4*>(pr + 4) = v1;
@@ -258,7 +260,7 @@ int gemm_mid(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, fl
              int S, hipStream_t stream) {
   if (M < 1 || N < 16 || N % 16 || K % kBK || S < 1 || S > 16 || K / kBK < S) return -1;
   if (glu && (N % 128 || bias)) return -2;
-  if (S > 1 && (P == nullptr || bias)) return -3;
+  if (S > 1 && P == nullptr) return -3;
   if (Y == nullptr ? (S == 1 || glu) : (ldy % 8 || reinterpret_cast<uintptr_t>(Y) % 16)) return -4;
   if (S > 1 && Y != nullptr && ldy != (glu ? N / 2 : N)) return -5;
   const int64_t units = (int64_t)((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN) * S;

@@ -231,10 +231,10 @@ class LlamaModel(DecoderModel):
             kc, vc = kv.layer(i)
             # a split-K decode QKV projection hands its fp32 slabs to rope_kv, which sums
             # them per element (no separate reduce kernel) and adds a Qwen2 bias before
-            # rounding; a prefill bias rides the tile GEMM's epilogue
+            # rounding; a prefill bias rides the tile GEMM's epilogue or its first slab
             bias = lw.bqkv
             if bias is not None and fb.is_prefill and lw.sqkv is None:
-                qkv, bias = ops.linear(x, lw.wqkv, bias=bias), None
+                qkv, bias = ops.linear(x, lw.wqkv, bias=bias, defer_reduce=self.tp.world == 1), None
             else:
                 qkv = self._lin(x, lw.wqkv, lw.sqkv, defer=True)
             if fb.is_prefill:

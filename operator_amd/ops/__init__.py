@@ -548,14 +548,14 @@ def linear_tile(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = Non
     ping-pong pipeline). ``defer_reduce``: K slices come back as fp32 slabs (:class:`SplitK`)."""
     M, K = x.shape
     N = w.shape[0]
-    defer = defer_reduce and out is None and bias is None and not glu
+    defer = defer_reduce and out is None and not glu
     S = None
     if (out is None or (out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0)) and (
             bias is None or (bias.is_contiguous() and bias.data_ptr() % 16 == 0)):   # gemm_mid's 16-B accesses
-        S = mid_plan(M, N, K, defer, bias is None and (out is None or out.is_contiguous()))
+        S = mid_plan(M, N, K, defer, out is None or out.is_contiguous())
     part = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if S is not None and S > 1 else None
     if part is not None and defer:
-        kernels().gemm_mid(x, w, None, None, part, S)
+        kernels().gemm_mid(x, w, None, bias, part, S)
         return SplitK(part, S, M, N)
     y = out if out is not None else torch.empty(M, N // 2 if glu else N, dtype=x.dtype, device=x.device)
     if S is not None:
@@ -599,7 +599,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, sp
         return linear_f32(x, w)
     if bias is not None:
         if tile_ok(x, w) and tile_out_ok(out):
-            return linear_tile(x, w, out, bias)
+            return linear_tile(x, w, out, bias, defer_reduce=defer_reduce)
         return _blas(x, w, out, bias)
     if x.is_cuda and bm is None and bn is None and splits is None and _measured_blas(M, N, K):
         return _blas(x, w, out, None)

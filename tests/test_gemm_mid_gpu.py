@@ -58,6 +58,22 @@ def test_gemm_mid_gated(M, inter, K, S, act):
     assert ((y.double() - r).abs() <= 5 * 2.0 ** -8 * r.abs() + 2.0 ** -8 * 1.2 * up.double().abs() * gate.double().abs() + 1e-6).all()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,S", [(1, 16, 128, 2), (130, 272, 448, 3), (300, 4608, 3584, 2)])
+def test_bias_is_in_the_first_slab(M, N, K, S):
+    torch.manual_seed(M + N)
+    x, w, b = _rand(M, K), _rand(N, K, scale=0.05), _rand(N, scale=0.5)
+    r = x.double() @ w.double().t() + b.double()
+    mag = x.double().abs() @ w.double().abs().t() + b.double().abs()
+    y, slabs = torch.empty(M, N, dtype=torch.bfloat16, device=DEV), torch.full((S, M, N), float("nan"), device=DEV)
+    ops.kernels().gemm_mid(x, w, y, b, slabs, S)
+    _check(y, r, mag, K)
+    for y in (ops.linear(x, w, bias=b), ops.linear(x, w, bias=b, defer_reduce=True)):
+        if isinstance(y, ops.SplitK):
+            y = y.p[:y.S * M * N].view(y.S, M, N).sum(0)
+        _check(y, r, mag, K)
+
+
 def test_mid_plan_is_launchable():
     """Every plan is one gemm_mid takes, padded batches keep their plan, large products keep the 256-row tiles."""
     for N, K in ((16, 128), (272, 192), (4096, 4096), (4096, 14336), (28672, 4096), (128256, 4096), (151936, 2048)):
