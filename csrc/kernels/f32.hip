@@ -36,6 +36,15 @@ __device__ __forceinline__ void put4(float* y, const f32x4& v, int n, bool vec) 
   }
 }
 
+// 4 neighbouring values of a row, n valid ones, the others 0
+__device__ __forceinline__ f32x4 get4(const float* x, int n) {
+  f32x4 v{};
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (e < n) v[e] = x[e];
+  return v;
+}
+
 }  // namespace
 
 struct GemmF32 {
@@ -362,8 +371,9 @@ __device__ __forceinline__ float lanes_sum(float v) {
 // are shared through LDS (rows padded by 16 B) and the next tile's loads are in flight while one is used.
 // What bounds it: the fp32 MFMA rate of the workgroups with the longest rows (2 x 500 rows of 16 heads of 128: 866 us
 // with a row per workgroup on FMA, 72 here; 2018 rows 3956 -> 243).
-// D: instantiated size >= both head sizes.
-template <int D>
+// D: instantiated size >= both head sizes. ODD: value heads that are no multiple of 16 columns, or output rows that take no
+// 16-B stores (key heads are multiples of 4 in either form).
+template <int D, bool ODD>
 __global__ void __launch_bounds__(256) attn_f32_prefill_kernel(const AttnF32 a) {
   constexpr int BK = 32, LD = D + 4, NC = D / 32;   // NC: 16-B chunks of a row per loading thread
   __shared__ __attribute__((aligned(16))) float ks[BK * LD], vs[BK * LD];
@@ -397,7 +407,8 @@ __global__ void __launch_bounds__(256) attn_f32_prefill_kernel(const AttnF32 a) 
     for (int i = 0; i < NC; ++i) {
       const int c = 4 * (lc + 8 * i);
       kn[i] = in && c < a.dkp ? *reinterpret_cast<const f32x4*>(kp + c) : zero;
-      vn[i] = in && c < a.dvp ? *reinterpret_cast<const f32x4*>(vp + c) : zero;
+      if constexpr (ODD) vn[i] = in ? get4(vp + c, a.dvp - c) : zero;
+      else vn[i] = in && c < a.dvp ? *reinterpret_cast<const f32x4*>(vp + c) : zero;
     }
   };
   f32x4 acc[D / 16] = {};   // dims 16 b + 4 g + r of query l15
@@ -459,18 +470,28 @@ __global__ void __launch_bounds__(256) attn_f32_prefill_kernel(const AttnF32 a) 
     f32x4 v;
 #pragma unroll
     for (int r = 0; r < 4; ++r) v[r] = a.gate ? acc[b][r] / l * c : acc[b][r] / l;
-    *reinterpret_cast<f32x4*>(out + 16 * b) = v;
+    if constexpr (ODD) put4(out + 16 * b, v, a.dvp - 16 * b - 4 * g, false);
+    else *reinterpret_cast<f32x4*>(out + 16 * b) = v;
   }
 }
 
 int attn_f32_prefill(const AttnF32& a, int items, int Hq, hipStream_t stream) {
   if (items == 0) return 0;
   const int top = a.dkp > a.dvp ? a.dkp : a.dvp;
-  if (a.dkp % 16 || a.dvp % 16 || a.o_ld % 4 || top > 256 || Hq % a.Hkv || a.window < 1) return -1;
+  if (a.dkp < 4 || a.dkp % 4 || a.dvp < 1 || top > 256 || Hq % a.Hkv || a.window < 1) return -1;
   const dim3 grid(items, Hq, 2);   // items are 128 query rows
-  if (top <= 64) attn_f32_prefill_kernel<64><<<grid, 256, 0, stream>>>(a);
-  else if (top <= 128) attn_f32_prefill_kernel<128><<<grid, 256, 0, stream>>>(a);
-  else attn_f32_prefill_kernel<256><<<grid, 256, 0, stream>>>(a);
+  const bool odd = a.dvp % 16 || a.o_ld % 4;
+#define OAMD_PF(D)                                                              \
+  if (odd) attn_f32_prefill_kernel<D, true><<<grid, 256, 0, stream>>>(a);       \
+  else attn_f32_prefill_kernel<D, false><<<grid, 256, 0, stream>>>(a)
+  if (top <= 64) {
+    OAMD_PF(64);
+  } else if (top <= 128) {
+    OAMD_PF(128);
+  } else {
+    OAMD_PF(256);
+  }
+#undef OAMD_PF
   OAMD_LAUNCH_CHECK();
   return 0;
 }
@@ -482,8 +503,9 @@ int attn_f32_prefill(const AttnF32& a, int items, int Hq, hipStream_t stream) {
 // of a tile go out in large groups, with small heads its values before the scores are computed. 18 sequences of 1282
 // tokens: 16 heads on one latent row of 288 454 -> 37 us, 4 heads of 128 on a key head, window 512, 202 -> 27 (with a
 // workgroup per query head and a key per lane before).
-// NB: 16-dim blocks of the value size.
-template <int NB>
+// NB: 16-dim blocks of the value size. ODD: heads that are no multiple of 16 columns (keys: of 4), or output rows that take
+// no 16-B stores.
+template <int NB, bool ODD>
 __global__ void __launch_bounds__(512) attn_f32_decode_kernel(const AttnF32 a, int Hq, int chunks, int splits, float* part, float* ml) {
   constexpr int NW = 8, RB = 4;                // waves, value blocks merged at a time
   constexpr bool kEarly = NB <= 8;             // a tile's values fit in registers beside the sums
@@ -509,22 +531,35 @@ __global__ void __launch_bounds__(512) attn_f32_decode_kernel(const AttnF32 a, i
     const int64_t row = ((int64_t)a.block_tables[(int64_t)t * a.max_pages + j0 / a.page_size] * a.Hkv + kvh) * a.page_size + j0 % a.page_size;
     const float* kp = a.k + (row + l15) * a.k_ld + 4 * g;
     const float* vp = a.v + (row + 4 * g) * a.v_ld + l15;
+    // column of value block b: past the head its first block again, its last column in the lanes past that (not stored)
+    auto vcol = [&](int b) {
+      if constexpr (ODD)
+        if (16 * b < a.dvp) return 16 * b + min(l15, a.dvp - 1 - 16 * b) - l15;
+      return 16 * b < a.dvp ? 16 * b : ODD ? min(l15, a.dvp - 1) - l15 : 0;
+    };
     float vf[8][4];
     if constexpr (kEarly)
 #pragma unroll
       for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) vf[b][e] = vp[e * a.v_ld + (16 * b < a.dvp ? 16 * b : 0)];
+        for (int e = 0; e < 4; ++e) vf[b][e] = vp[e * a.v_ld + vcol(b)];
     __builtin_amdgcn_sched_barrier(0);   // ... here, not where they are used
     f32x4 s[1] = {};
-    for (int c0 = 0; c0 < a.dkp; c0 += 16 * KC) {
+    const int dk = ODD ? a.dkp & ~15 : a.dkp;
+    for (int c0 = 0; c0 < dk; c0 += 16 * KC) {
       f32x4 kf[KC];
 #pragma unroll
-      for (int c = 0; c < KC; ++c) kf[c] = *reinterpret_cast<const f32x4*>(kp + (c0 + 16 * c < a.dkp ? c0 + 16 * c : 0));
+      for (int c = 0; c < KC; ++c) kf[c] = *reinterpret_cast<const f32x4*>(kp + (c0 + 16 * c < dk ? c0 + 16 * c : 0));
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int c = 0; c < KC; ++c)
-        if (c0 + 16 * c < a.dkp) s[0] = mfma4(kf[c], *reinterpret_cast<const f32x4*>(qp + c0 + 16 * c), s[0]);
+        if (c0 + 16 * c < dk) s[0] = mfma4(kf[c], *reinterpret_cast<const f32x4*>(qp + c0 + 16 * c), s[0]);
+    }
+    if constexpr (ODD) {   // the last columns of a key
+      const f32x4 zero{};
+      const bool in = dk + 4 * g < a.dkp;
+      const f32x4 kt = in ? *reinterpret_cast<const f32x4*>(kp + dk) : zero, qt = in ? *reinterpret_cast<const f32x4*>(qp + dk) : zero;
+      s[0] = mfma4(kt, qt, s[0]);
     }
     const float alpha = soften<1>(s, j0, g, lo, n, a.scale, st);
     constexpr int VB = kEarly ? NB : 8;   // value blocks requested at a time
@@ -534,7 +569,7 @@ __global__ void __launch_bounds__(512) attn_f32_decode_kernel(const AttnF32 a, i
 #pragma unroll
         for (int b = 0; b < VB; ++b)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) vf[b][e] = vp[e * a.v_ld + (16 * (b0 + b) < a.dvp ? 16 * (b0 + b) : 0)];
+          for (int e = 0; e < 4; ++e) vf[b][e] = vp[e * a.v_ld + vcol(b0 + b)];
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
@@ -582,18 +617,18 @@ __global__ void __launch_bounds__(512) attn_f32_decode_kernel(const AttnF32 a, i
       f32x4 o{};
 #pragma unroll
       for (int x = 0; x < NW; ++x) o += f[x] * red[x][w][lane];
-      if (splits > 1) {
-        *reinterpret_cast<f32x4*>(part + (hq * splits + sp) * a.dvp + 16 * b + 4 * g) = o;
-      } else {
+      float* out = splits > 1 ? part + (hq * splits + sp) * a.dvp : a.o + (int64_t)t * a.o_ld + (h0 + l15) * a.dvp;
+      if (splits == 1)
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[r] = n <= 0 ? 0.f : a.gate ? o[r] / L * a.gate[hq] : o[r] / L;
-        *reinterpret_cast<f32x4*>(a.o + (int64_t)t * a.o_ld + (h0 + l15) * a.dvp + 16 * b + 4 * g) = o;
-      }
+      if constexpr (ODD) put4(out + 16 * b + 4 * g, o, a.dvp - 16 * b - 4 * g, false);
+      else *reinterpret_cast<f32x4*>(out + 16 * b + 4 * g) = o;
     }
   }
 }
 
 // One workgroup per sequence and head: the pieces' sums against their common maximum.
+template <bool ODD>
 __global__ void __launch_bounds__(64) attn_f32_combine_kernel(const AttnF32 a, int Hq, int splits, const float* part, const float* ml) {
   const int64_t hq = (int64_t)blockIdx.x * Hq + blockIdx.y;
   float* out = a.o + (int64_t)blockIdx.x * a.o_ld + blockIdx.y * a.dvp;
@@ -603,25 +638,39 @@ __global__ void __launch_bounds__(64) attn_f32_combine_kernel(const AttnF32 a, i
   for (int s = 0; s < splits; ++s) L += expf(ml[(hq * splits + s) * 2] - M) * ml[(hq * splits + s) * 2 + 1];
   for (int d = 4 * threadIdx.x; d < a.dvp; d += 256) {
     f32x4 o{};
-    for (int s = 0; s < splits; ++s) o += expf(ml[(hq * splits + s) * 2] - M) * *reinterpret_cast<const f32x4*>(part + (hq * splits + s) * a.dvp + d);
+    for (int s = 0; s < splits; ++s) {
+      const float* p = part + (hq * splits + s) * a.dvp + d;
+      o += expf(ml[(hq * splits + s) * 2] - M) * (ODD ? get4(p, a.dvp - d) : *reinterpret_cast<const f32x4*>(p));
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) o[r] = !any ? 0.f : a.gate ? o[r] / L * a.gate[hq] : o[r] / L;
-    *reinterpret_cast<f32x4*>(out + d) = o;
+    if constexpr (ODD) put4(out + d, o, a.dvp - d, false);
+    else *reinterpret_cast<f32x4*>(out + d) = o;
   }
 }
 
 int attn_f32_decode(const AttnF32& a, int rows, int Hq, int splits, float* part, float* ml, hipStream_t stream) {
   if (rows == 0) return 0;
-  if (a.dkp % 16 || a.dvp % 16 || a.o_ld % 4 || a.dkp > 640 || a.dvp > 640 || Hq % a.Hkv || a.window < 1 || a.page_size % 16) return -1;
+  if (a.dkp < 4 || a.dkp % 4 || a.dvp < 1 || a.dkp > 640 || a.dvp > 640 || Hq % a.Hkv || a.window < 1 || a.page_size % 16) return -1;
   if (splits < 1 || splits > 256 || (splits > 1 && (part == nullptr || ml == nullptr))) return -2;
   const int chunks = (Hq / a.Hkv + 15) / 16;
   const dim3 grid(rows, a.Hkv * chunks, splits);
-  if (a.dvp <= 128) attn_f32_decode_kernel<8><<<grid, 512, 0, stream>>>(a, Hq, chunks, splits, part, ml);
-  else if (a.dvp <= 256) attn_f32_decode_kernel<16><<<grid, 512, 0, stream>>>(a, Hq, chunks, splits, part, ml);
-  else attn_f32_decode_kernel<40><<<grid, 512, 0, stream>>>(a, Hq, chunks, splits, part, ml);
+  const bool odd = a.dkp % 16 || a.dvp % 16 || a.o_ld % 4;
+#define OAMD_DEC(NB)                                                                                        \
+  if (odd) attn_f32_decode_kernel<NB, true><<<grid, 512, 0, stream>>>(a, Hq, chunks, splits, part, ml);     \
+  else attn_f32_decode_kernel<NB, false><<<grid, 512, 0, stream>>>(a, Hq, chunks, splits, part, ml)
+  if (a.dvp <= 128) {
+    OAMD_DEC(8);
+  } else if (a.dvp <= 256) {
+    OAMD_DEC(16);
+  } else {
+    OAMD_DEC(40);
+  }
+#undef OAMD_DEC
   OAMD_LAUNCH_CHECK();
   if (splits > 1) {
-    attn_f32_combine_kernel<<<dim3(rows, Hq), 64, 0, stream>>>(a, Hq, splits, part, ml);
+    if (odd) attn_f32_combine_kernel<true><<<dim3(rows, Hq), 64, 0, stream>>>(a, Hq, splits, part, ml);
+    else attn_f32_combine_kernel<false><<<dim3(rows, Hq), 64, 0, stream>>>(a, Hq, splits, part, ml);
     OAMD_LAUNCH_CHECK();
   }
   return 0;

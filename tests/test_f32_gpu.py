@@ -107,6 +107,48 @@ def test_decode_attention_pieces(H, G, D, Dv, splits, window):
         torch.testing.assert_close(o[b].double(), r * gate[b].double()[:, None], atol=2e-5, rtol=2e-5)
 
 
+@pytest.mark.parametrize("D,Dv", [(4, 1), (20, 18), (36, 100), (132, 130), (256, 255), (20, 96), (64, 17)])
+def test_prefill_attention_unpadded_heads(D, Dv):
+    """Key heads of any multiple of 4 columns, value heads of any number; columns past the heads stay as they are."""
+    torch.manual_seed(D + Dv)
+    H, G, lens = 4, 2, [1, 70, 131]
+    T = sum(lens)
+    L = dec.HeadLayout(H, G, D, Dv)
+    q, k, v = (torch.randn(T, h, d, device=DEV) for h, d in ((H, D), (G, D), (G, Dv)))
+    o = dec.attn_gd_prefill(q, k, v, lens, L, D ** -0.5, window=50)
+    a = 0
+    for n in lens:
+        r = _attend(q[a:a + n], k[a:a + n].repeat_interleave(H // G, 1), v[a:a + n].repeat_interleave(H // G, 1), D ** -0.5, 50)
+        torch.testing.assert_close(o[a:a + n, :H * Dv].view(n, H, Dv).double(), r, atol=2e-5, rtol=2e-5)
+        a += n
+    assert (o[:, H * L.pads[1]:] == 0).all()
+
+
+@pytest.mark.parametrize("D,Dv", [(4, 1), (20, 18), (36, 100), (132, 130), (640, 639), (20, 320), (64, 17)])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_decode_attention_unpadded_heads(D, Dv, splits):
+    torch.manual_seed(D + Dv)
+    P, ctx, H, G = 16, [1, 0, 17, 200], 6, 2
+    L, B, pages = dec.HeadLayout(H, G, D, Dv), len(ctx), 13
+    kc, vc = (torch.full((B * pages, G, P, d), float("nan"), device=DEV) for d in (D, Dv))
+    bt = torch.arange(B * pages, dtype=torch.int32).flip(0).view(B, pages).contiguous()   # the last page is read to its end
+    q = torch.randn(B, H, D, device=DEV)
+    seqs = []
+    for b, n in enumerate(ctx):
+        k, v = torch.randn(n, G, D, device=DEV), torch.randn(n, G, Dv, device=DEV)
+        for t in range(n):
+            kc[bt[b, t // P], :, t % P], vc[bt[b, t // P], :, t % P] = k[t], v[t]
+        seqs.append((k, v))
+    o = dec.attn_gd_decode(q, (kc, vc), bt.to(DEV), torch.tensor(ctx, dtype=torch.int32, device=DEV), L, D ** -0.5, splits)
+    for b, (k, v) in enumerate(seqs):
+        got = o[b, :H * Dv].view(H, Dv)
+        if ctx[b] == 0:
+            assert (got == 0).all()
+            continue
+        r = _attend(q[b:b + 1], k.repeat_interleave(H // G, 1), v.repeat_interleave(H // G, 1), D ** -0.5)[0]
+        torch.testing.assert_close(got.double(), r, atol=2e-5, rtol=2e-5)
+
+
 @pytest.mark.parametrize("rank,splits", [(256, 2), (544, 1), (608, 3)])
 def test_latent_decode_f32_wide_rows(rank, splits):
     torch.manual_seed(rank)
