@@ -462,6 +462,7 @@ class LLMEngine:
         self.use_graphs = use_graphs and self.device.type == "cuda"
         self.multi_step = max(1, multi_step)
         self._active: _BucketState | None = None   # bucket whose device state matches self.running
+        self._given_work: tuple | None = None   # (stream, event | None) behind the last given-token call's GPU work
         self.waiting: deque[GenRequest] = deque()
         self.running: list[GenRequest] = []
         # the batch between _admit (pages allocated, off `waiting`) and its append to
@@ -695,6 +696,7 @@ class LLMEngine:
         ``splits`` defaults to every split count a bucket can use up to max_context."""
         if not self.use_graphs:
             return
+        self._after_given()
         bs = sorted(buckets or self.buckets, reverse=True)
         for bp in bs:
             for ns in (splits or self.split_options(bp)):
@@ -706,6 +708,7 @@ class LLMEngine:
 
     # ------------------------------------------------------------------ scheduling
     def step(self) -> list[GenRequest]:
+        self._after_given()
         self.stats.steps += 1
         if self._inflight is not None and (self._admittable() or not self.running):
             self._consume(self._inflight)   # composition is about to change: drain first
@@ -941,20 +944,41 @@ class LLMEngine:
         if need > 0:
             r.pages = r.pages + self.kv.allocator.alloc(need)
 
+    def _after_given(self) -> None:
+        """Order the current stream behind the last given-token call, which returns before its GPU work is done: bucket
+        states, graph outputs and cache pages are the engine's, whichever stream a call comes from."""
+        if self._given_work is not None:
+            last, done = self._given_work
+            cur = torch.cuda.current_stream(self.device)
+            if cur != last:
+                cur.wait_event(done) if done is not None else cur.wait_stream(last)
+
+    def _given_queued(self) -> None:
+        if self.device.type == "cuda":
+            cur = torch.cuda.current_stream(self.device)
+            # torch's own streams outlive the engine: the event is made when another stream needs it (one per step costs 4 us
+            # of a 676 us decode step); a stream of the caller's may be gone by then (its id is its handle)
+            own = cur.stream_id != cur.cuda_stream or cur.cuda_stream == 0
+            self._given_work = (cur, None if own else cur.record_event())
+
     def given_start(self, prompts: list[list[int]], want: list[list[int]]) -> tuple[list[GenRequest], torch.Tensor | None]:
         """Prefill new sequences as one batch: (requests, logits [wanted, vocab] of the places
         ``want`` of each prompt, in order)."""
+        self._after_given()
         reqs = [GenRequest(list(p), max_tokens=0) for p in prompts]
         for r in reqs:
             self._reserve(r)
         p = self._pack_prefill(reqs)
         rows = [int(p["cu"][i]) + j for i, w in enumerate(want) for j in w]
         logits = self._eager_prefill(p, rows or [0])
+        self._given_queued()
         self.stats.prefill_tokens += len(p["ids"])
         return reqs, logits if rows else None
 
     def given_next(self, reqs: list[GenRequest], tokens: list[int]) -> torch.Tensor:
-        """One decode step of ``reqs`` with the given next tokens: logits [len(reqs), vocab]."""
+        """One decode step of ``reqs`` with the given next tokens: logits [len(reqs), vocab], queued on the current
+        stream (the call does not wait for them)."""
+        self._after_given()
         out = torch.empty(len(reqs), self.model.cfg.vocab_size, dtype=torch.float32, device=self.device)
         for r, t in zip(reqs, tokens):
             r.output.append(int(t))
@@ -973,6 +997,7 @@ class LLMEngine:
             else:
                 out[part] = g.logits[:n].float()
             self.stats.decode_tokens += len(rows)
+        self._given_queued()
         self._active = None
         return out
 
