@@ -6,9 +6,9 @@
 // and its K may be cut into S slices (fp32 slabs, summed by the consumer or by a reduce pass), so that
 // M N S / 32768 workgroups come close to one per CU:
 //   885 rows (weights from HBM)   4096 x 14336: 297 -> 103 us, 4096 x 4096: 88 -> 36, 6144 x 4096: 89 -> 56
-//   100 rows                      279 -> 30, 85 -> 16, 85 -> 19
+//   100 rows, the norm included   285 -> 58, 90 -> 25, 91 -> 38 (in the slices of 512 rows, see ops.mid_plan)
 //   vocabulary 128256 x 8192, 64 rows: 422 -> 373 us (5.6 TB/s of weights)
-// The first slice carries a bias (4608 x 3584, 100 rows: 56 us in one slice, 21 in 7; 300 rows 54, 29 in 3).
+// The first slice carries a bias (4608 x 3584, 300 rows: 54 us in one slice, 29 in 3).
 // A 128 x 256 step is 0.7 us (0.43 of MFMA at 2.4 GHz): a CU takes in 50 to 75 bytes per ns through LDS-DMA however
 // many stages wait (a fourth stage of a 64-row tile gained nothing). With every CU busy for several rounds it is
 // 0.85 us, 1.2 PFLOP/s against 1.45 of the 256-row tiles, so those keep the large products (ops.mid_plan).

@@ -528,15 +528,19 @@ def mid_plan(M: int, N: int, K: int, defer: bool, slices: bool = True) -> int | 
     103 us against 297, 6144 x 4096 56 against 89); once every CU has a 256-row tile, that tile's fewer operand
     bytes per product win (4096 rows of 4096 x 14336: 325 us against 371).
 
-    Above 256 rows the plan is the next multiple of 512's: a prefill graph pads its batch to such a size, and a
-    prompt's numbers are the same padded or not. Past 4096 rows the graphs' sizes are coarser and little is left
-    to gain."""
-    if M > 256:
+    Rows that are no decode bucket's (above 256, or above 32 and no multiple of 64) are a prompt's and take the plan of
+    the next multiple of 512: a prefill graph pads its batch to such a size, and a prompt's numbers are the same padded or
+    not (100 rows of 4096 x 14336 with the norm behind them: 58 us in the four slices of 512 rows, 36 in fourteen, 285 on
+    the 256-row tiles). From LM_HEAD_MIN_N features on, where 512 rows run on the 256-row tiles, they are not sliced. Past
+    4096 rows the graphs' sizes are coarser and little is left to gain. Prompts of up to 32, and of 64, 128, 192 or 256
+    rows run on a decode kernel when they are not padded."""
+    prompt = M > SKINNY_MAX_M and M % 64 != 0
+    if M > 256 or (prompt and N < LM_HEAD_MIN_N):
         M = -(-M // 512) * 512
     if M < 1 or M > 4096 or K < 128 or (M > 128 and N >= LM_HEAD_MIN_N):   # 256 rows of a vocabulary: 282 us against 253
         return None
     tiles = -(-M // 128) * -(-N // 256)
-    most = min(16, K // 128, 2 * CUS // tiles) if slices else 1
+    most = 1 if not slices or (prompt and N >= LM_HEAD_MIN_N) else min(16, K // 128, 2 * CUS // tiles)
     cost, S = min((_mid_cost(M, N, K, s, defer), s) for s in range(1, max(1, most) + 1))
     return S if cost < _tile_cost(M, N, K) else None
 

@@ -83,5 +83,10 @@ def test_mid_plan_is_launchable():
                 assert S is None or 1 <= S <= min(16, K // 64)
                 assert ops.mid_plan(M, N, K, defer, False) in (None, 1)
             assert ops.mid_plan(322, N, K, defer) == ops.mid_plan(512, N, K, defer)
+            for M in (33, 63, 65, 100, 127, 129, 200, 255):   # no decode bucket: a prompt, in its graph one of 512 rows
+                if N < ops.LM_HEAD_MIN_N:
+                    assert ops.mid_plan(M, N, K, defer) == ops.mid_plan(512, N, K, defer)
+                else:   # the 512-row plan is the 256-row tiles over the whole K: no slices
+                    assert ops.mid_plan(M, N, K, defer) in (None, 1) and ops.mid_plan(512, N, K, defer) is None
     assert ops.mid_plan(28000, 4096, 14336, True) is None
     assert ops.mid_plan(885, 4096, 14336, True) == 2

@@ -265,6 +265,24 @@ def test_graph_prefill_equals_eager_prefill():
     assert torch.equal(caches[0], caches[1])
 
 
+@pytest.mark.parametrize("name", ["tiny-gqa4", "tiny-qwen"])
+@pytest.mark.parametrize("lens", [[40], [33, 60], [100, 99], [255], [130, 170], [700]])
+def test_prompt_rows_are_the_same_in_a_graph(name, lens):
+    """Prompts that are no decode bucket's size (33 to 255 tokens, or more) write the same keys and values, bit for bit,
+    eagerly and padded to their graph's 512 or 1024 rows: the K slices of a projection do not change with the padding."""
+    cfg = get_config(name)
+    m = LlamaModel(cfg, device="cuda").init_random(seed=7)
+    caches = []
+    for pg in (False, True):
+        kv = PagedKVCache(cfg.layers, 64, cfg.kv_heads, 128, 16, device="cuda")
+        eng = LLMEngine(m, kv, max_batch=4, max_prefill_tokens=1024, max_context=1024, prefill_graphs=pg, prefix_sharing=False)
+        reqs = [GenRequest(list(range(3 + i, 3 + i + n)), max_tokens=1, ignore_eos=True) for i, n in enumerate(lens)]
+        eng.generate(reqs)
+        assert eng.stats.prefill_graph_replays == pg
+        caches.append(torch.stack([t.float() for i in range(cfg.layers) for t in kv.layer(i)]).cpu())
+    assert torch.equal(caches[0], caches[1])
+
+
 @pytest.mark.parametrize("B", [3, 64])
 def test_qwen_decode_step_matches_cpu_reference(B):
     """Qwen2-shaped decode (q/k/v bias, GQA group 7): one paged decode step after a
