@@ -192,7 +192,7 @@ class MatchEngine:
         self.use_native_scorer = use_native_scorer
         # score + rank events on the GPU (score.hip) when scanning there
         self.gpu_scorer = (self.device.type == "cuda") if gpu_scorer is None else gpu_scorer
-        # ... unless it is asked for, batches of few hits stay on the host: the round trip to the GPU takes 65 us
+        # ... unless it is asked for, batches of few hits go to the native scorer: the round trip to the GPU takes 65 us
         # for 3 hits (5 here) and 195 for 195 (130); past some thousand the sorts are the GPU's
         self._gpu_score_from = 0 if gpu_scorer else self.HOST_SCORE_HITS
         self._scorer = None
@@ -598,7 +598,8 @@ class MatchEngine:
 
     def _events_from_hits(self, docs: list[bytes], hits: np.ndarray, stream=None) -> list[list[oracle.Event]]:
         cp = self.cp
-        if self.gpu_scorer and self.device.type == "cuda" and len(hits) > self._gpu_score_from:
+        few = self.use_native_scorer and len(hits) <= self._gpu_score_from
+        if self.gpu_scorer and self.device.type == "cuda" and not few:
             with (torch.cuda.stream(stream) if stream is not None else self._on_stream()):
                 return self._events_gpu(hits, len(docs))
         if self.use_native_scorer:

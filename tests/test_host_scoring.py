@@ -3,6 +3,7 @@ import random
 
 import numpy as np
 import pytest
+import torch
 
 from operator_amd.engine.match import MatchEngine
 from operator_amd.patterns import oracle
@@ -27,6 +28,20 @@ def test_kept_scorer_matches_oracle(docs, n):
             assert [e.score for e in evs[d]] == pytest.approx([e.score for e in want], abs=1e-12)
 
 
+@pytest.mark.parametrize("native,gpu_scorer,n,on_gpu", [
+    (True, None, 0, False), (True, None, MatchEngine.HOST_SCORE_HITS, False), (True, None, MatchEngine.HOST_SCORE_HITS + 1, True),
+    (False, None, 1, True), (True, True, 1, True), (False, True, 1, True), (True, False, 9999, False), (False, False, 9, False)])
+def test_where_a_gpu_engine_scores(monkeypatch, native, gpu_scorer, n, on_gpu):
+    """Few hits go to the native scorer; without it, or where the GPU scorer is asked for, they are the GPU's."""
+    eng = MatchEngine(compile_patterns(synthetic_library(20, seed=2)), device="cpu", use_native_scorer=native, gpu_scorer=gpu_scorer)
+    if gpu_scorer is None:
+        eng.gpu_scorer = True   # what an engine on the GPU sets
+    monkeypatch.setattr(eng, "device", torch.device("cuda"))
+    monkeypatch.setattr(eng, "_events_gpu", lambda hits, docs: "gpu")
+    hits = np.stack([np.zeros(n, np.int64), np.zeros(n, np.int64), np.arange(n)], 1)
+    assert (eng._events_from_hits([b""], hits) == "gpu") == on_gpu
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("docs", [1, 7])
 def test_host_and_gpu_forms_agree(docs):
@@ -36,3 +51,14 @@ def test_host_and_gpu_forms_agree(docs):
     gpu.HOST_CONTEXT_DOCS = 0
     for a, b in zip(host.analyze(logs), gpu.analyze(logs)):
         assert a.summary == b.summary and a.events == b.events
+
+
+@pytest.mark.gpu
+def test_gpu_scorer_alone():
+    """Without the native scorer the GPU scores every batch, one without hits among them."""
+    cp = compile_patterns(synthetic_library(100, seed=0))
+    logs = LogFactory(100, seed=4, pool_lines=256).batch(3, 9000)[0]
+    alone, host = MatchEngine(cp, device="cuda", use_native_scorer=False), MatchEngine(cp, device="cpu")
+    for docs in ([b"zzz\n", b""], logs):
+        for a, b in zip(alone.analyze(docs), host.analyze(docs)):
+            assert a.summary == b.summary and a.events == b.events
