@@ -556,7 +556,7 @@ def linear_tile(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = Non
     S = None
     if (out is None or (out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0)) and (
             bias is None or (bias.is_contiguous() and bias.data_ptr() % 16 == 0)):   # gemm_mid's 16-B accesses
-        S = mid_plan(M, N, K, defer, out is None or out.is_contiguous())
+        S = mid_plan(M, N, K, defer, out is None or out.stride(0) == out.shape[1])   # the reduce pass has no row stride
     part = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if S is not None and S > 1 else None
     if part is not None and defer:
         kernels().gemm_mid(x, w, None, bias, part, S)

@@ -90,3 +90,34 @@ def test_mid_plan_is_launchable():
                     assert ops.mid_plan(M, N, K, defer) in (None, 1) and ops.mid_plan(512, N, K, defer) is None
     assert ops.mid_plan(28000, 4096, 14336, True) is None
     assert ops.mid_plan(885, 4096, 14336, True) == 2
+
+
+@pytest.mark.parametrize("M,N,K,wide", [(1, 4096, 4096, 8192), (1, 272, 1024, 288), (1, 4096, 4096, 4096), (40, 4096, 4096, 8192)])
+def test_rows_of_a_wider_output_are_not_sliced(monkeypatch, M, N, K, wide):
+    """The reduce pass of K slices writes its rows back to back: one row out of a wider buffer is contiguous for torch,
+    but its row stride is the buffer's, which the kernel takes in one slice only."""
+    seen = []
+
+    class Kernels:
+        def gemm_mid(self, x, w, y, bias, part, S, glu=0):
+            seen.append((S, y.stride(0)))
+
+        def gemm_tile(self, x, w, y, bias, glu):
+            seen.append((1, y.stride(0)))
+
+    monkeypatch.setattr(ops, "kernels", Kernels)
+    x, w, b = (torch.zeros(s, dtype=torch.bfloat16) for s in ((M, K), (N, K), (N,)))
+    out = torch.zeros(M, wide, dtype=torch.bfloat16)[:, :N]
+    ops.linear_tile(x, w, out, b)
+    assert seen[0][1] == wide and (seen[0][0] == 1 or wide == N)
+    assert (seen[0][0] > 1) == (wide == N)
+
+
+@pytest.mark.gpu
+def test_one_row_into_a_wider_output():
+    torch.manual_seed(1)
+    x, w, b = _rand(1, 4096), _rand(4096, 4096, scale=0.05), _rand(4096)
+    buf = torch.full((3, 8192), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.linear(x, w, out=buf[:1, :4096], bias=b)
+    _check(buf[:1, :4096], x.double() @ w.double().t() + b.double(), x.double().abs() @ w.double().abs().t() + b.double().abs(), 4096)
+    assert buf[0, 4096:].isnan().all() and buf[1:].isnan().all()
