@@ -451,8 +451,9 @@ def skinny_plan(M: int, N: int, K: int) -> int | None:
 def _mid_beats_skinny(M: int, N: int, K: int, defer: bool) -> bool:
     """gemm_skinny streams the weights once per call but pays for every row (a 128256 x 4096 vocabulary: 199 us at
     1 row, 242 at 8, 440 at 32; 4 % of the one-row time per row at every measured shape); gemm_mid's 128-row
-    tile costs the same at any of them (217 us). A few rows of a projection stay: too little work to split."""
-    if M <= (4 if N >= LM_HEAD_MIN_N else 16):
+    tile costs the same at any of them (217 us). A few rows of a projection stay: too little work to split. So do shapes
+    with a measured entry (32 rows of 4096 x 4096: 15.5 us against 17.6 in slices)."""
+    if M <= (4 if N >= LM_HEAD_MIN_N else 16) or ("skinny", M, N, K) in _gemm_table_get():
         return False
     S = mid_plan(M, N, K, defer)
     return S is not None and _mid_cost(M, N, K, S, defer) < (3 + 2e-6 * N * K / 5.4) * (1 + 0.04 * M)

@@ -121,3 +121,9 @@ def test_one_row_into_a_wider_output():
     ops.linear(x, w, out=buf[:1, :4096], bias=b)
     _check(buf[:1, :4096], x.double() @ w.double().t() + b.double(), x.double().abs() @ w.double().abs().t() + b.double().abs(), 4096)
     assert buf[0, 4096:].isnan().all() and buf[1:].isnan().all()
+
+
+def test_a_measured_entry_of_few_rows_wins(monkeypatch):
+    assert ops._mid_beats_skinny(32, 4096, 14336, True)
+    monkeypatch.setitem(ops._gemm_table_get(), ("skinny", 32, 4096, 14336), 8)
+    assert not ops._mid_beats_skinny(32, 4096, 14336, True) and ops.skinny_plan(32, 4096, 14336) == 8
