@@ -613,7 +613,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, sp
     if (x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous() and M <= SKINNY_MAX_M
             and bm is None and bn is None):
         S = splits or skinny_plan(M, N, K)
-        if S is not None and splits is None and out is None and tile_ok(x, w) and _mid_beats_skinny(M, N, K, defer_reduce):
+        if (S is not None and splits is None and out is None and tile_ok(x, w) and (x.data_ptr() | w.data_ptr()) % 16 == 0
+                and _mid_beats_skinny(M, N, K, defer_reduce)):
             return linear_tile(x, w, defer_reduce=defer_reduce)
         if S is not None:
             if S > 1 and (partial is None or partial.numel() < S * M * N):

@@ -127,3 +127,21 @@ def test_a_measured_entry_of_few_rows_wins(monkeypatch):
     assert ops._mid_beats_skinny(32, 4096, 14336, True)
     monkeypatch.setitem(ops._gemm_table_get(), ("skinny", 32, 4096, 14336), 8)
     assert not ops._mid_beats_skinny(32, 4096, 14336, True) and ops.skinny_plan(32, 4096, 14336) == 8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dx,dw,kernel", [(0, 0, "gemm_mid"), (1, 0, "gemm_skinny"), (0, 4, "gemm_skinny"), (8, 8, "gemm_mid")])
+def test_few_rows_off_their_alignment_stay_on_plain_loads(monkeypatch, dx, dw, kernel):
+    """gemm_mid stages 16-B pieces by LDS-DMA; gemm_skinny's loads take operands at any address. Nothing is launched."""
+    M, N, K = 24, 4096, 14336
+    seen = []
+
+    class Kernels:
+        def __getattr__(self, name):
+            return lambda *a: seen.append(name)
+
+    monkeypatch.setattr(ops, "kernels", Kernels)
+    x, w = (torch.empty(n * K + 8, dtype=torch.bfloat16, device=DEV)[d:d + n * K].view(n, K) for n, d in ((M, dx), (N, dw)))
+    for defer in (False, True):
+        ops.linear(x, w, defer_reduce=defer)
+    assert seen == [kernel] * 2
