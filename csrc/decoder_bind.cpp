@@ -38,6 +38,8 @@ template <typename T>
 T* p(const at::Tensor& t) { return reinterpret_cast<T*>(t.data_ptr()); }
 template <typename T>
 T* op(const OptT& t) { return t.has_value() ? reinterpret_cast<T*>(t->data_ptr()) : nullptr; }
+// an operand of 16-B LDS-DMA pieces: copied where it starts elsewhere
+at::Tensor on16(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 ? t.clone() : t; }
 void* vp(const OptT& t) { return t.has_value() ? t->data_ptr() : nullptr; }
 
 bool elem_f32(const at::Tensor& t, const char* what) {
@@ -555,7 +557,9 @@ void head_gemm(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, int64_t 
                   nx <= yd - N, "head_gemm: sizes");
   const c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
   if (f32) {
-    RC(oamd::head_gemm_f32(p<float>(x), p<float>(w), p<float>(y), (int)M, (int)N, (int)K, (int)H, H * xd, xd, ldy, yd, cur_stream()));
+    const bool tiles = oamd::f32_tiles((int)M, (int)K, false);
+    const at::Tensor xa = tiles ? on16(x) : x, wa = tiles ? on16(w) : w;
+    RC(oamd::head_gemm_f32(p<float>(xa), p<float>(wa), p<float>(y), (int)M, (int)N, (int)K, (int)H, H * xd, xd, ldy, yd, cur_stream()));
     return;
   }
   oamd::HeadGemm a{};
@@ -587,7 +591,9 @@ void gemm_f32(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, int64_t s
     TORCH_CHECK(partial.has_value() && !gtab.has_value() && !rscale.has_value() && N % 4 == 0, "gemm_f32: K slices");
     need(*partial, at::kFloat, splits * M * N, "partial");
   }
-  RC(oamd::gemm_f32(p<float>(x), p<float>(w), p<float>(y), op<float>(partial), (int)splits, (int)M, (int)N, (int)K, (int)y.size(1),
+  const bool tiles = oamd::f32_tiles((int)M, (int)K, gtab.has_value());
+  const at::Tensor xa = tiles ? on16(x) : x, wa = tiles ? on16(w) : w;
+  RC(oamd::gemm_f32(p<float>(xa), p<float>(wa), p<float>(y), op<float>(partial), (int)splits, (int)M, (int)N, (int)K, (int)y.size(1),
                     (int)silu_gu, op<int>(gtab), op<float>(rscale), cur_stream()));
 }
 

@@ -268,6 +268,8 @@ __global__ void __launch_bounds__(64 * NW) gemm_f32_skinny_kernel(const GemmF32 
   }
 }
 
+bool f32_tiles(int M, int K, bool grouped) { return grouped || !skinny_rows(M, K); }
+
 // K slices of the tile kernel: two workgroups per CU where the tiles alone give fewer, slices of 256 columns at least
 int gemm_f32_splits(int M, int N, int K, int glu) {
   if (skinny_rows(M, K) || N % 4) return 1;
@@ -286,7 +288,7 @@ static void launch_skinny(const GemmF32& a, dim3 grid, hipStream_t stream) {
 static int run_f32(GemmF32 a, bool glu, int H, hipStream_t stream) {
   const int nf = glu ? a.N / 2 : a.N;
   a.vec = a.ldy % 4 == 0 && a.yh % 4 == 0 && reinterpret_cast<uintptr_t>(a.Y) % 16 == 0;
-  if (skinny_rows(a.M, a.K) && !a.gtab) {
+  if (!f32_tiles(a.M, a.K, a.gtab != nullptr)) {
     const dim3 grid((nf + 15) / 16, 1, H);
     // enough waves to keep the loads of one CU in flight, and work for each of them
     if (glu) launch_skinny<true, 8>(a, grid, stream);

@@ -329,6 +329,7 @@ int head_gemm(const HeadGemm& a, hipStream_t stream);
 int gemm_f32(const float* X, const float* W, float* Y, float* P, int S, int M, int N, int K, int ldy, int glu, const int* gtab,
              const float* rscale, hipStream_t stream);
 int gemm_f32_splits(int M, int N, int K, int glu);
+bool f32_tiles(int M, int K, bool grouped);   // these run on the tile kernel, whose operands are 16-B aligned
 // One product per head: as HeadGemm, without the extra columns.
 int head_gemm_f32(const float* X, const float* W, float* Y, int M, int N, int K, int H, int64_t ldx, int64_t xh,
                   int64_t ldy, int64_t yh, hipStream_t stream);

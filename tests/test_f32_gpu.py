@@ -42,6 +42,27 @@ def test_head_gemm_f32(M):
     assert y[..., 48:].isnan().all()
 
 
+@pytest.mark.parametrize("M", [3, 33, 200])
+@pytest.mark.parametrize("dx,dw", [(1, 0), (0, 2), (3, 3)])
+def test_operands_off_their_alignment(M, dx, dw):
+    """The tile kernel stages 16-B pieces; operands that start elsewhere give the same numbers."""
+    torch.manual_seed(M + dx)
+
+    def at(t, d):
+        return torch.cat([torch.full((d,), float("nan"), device=DEV), t.flatten()])[d:].view(t.shape)
+
+    x, w = torch.randn(M, 528, device=DEV), torch.randn(128, 528, device=DEV)
+    xo, wo = at(x, dx), at(w, dw)
+    assert (xo.data_ptr() % 16 == 0) == (dx == 0) and (wo.data_ptr() % 16 == 0) == (dw == 0)
+    for glu in (0, ops.SILU):
+        assert torch.equal(ops.linear_f32(xo, wo, glu), ops.linear_f32(x, w, glu))
+    x, w = torch.randn(M, 2, 48, device=DEV), torch.randn(2, 32, 48, device=DEV)
+    y, yo = (torch.empty(M, 2, 32, device=DEV) for _ in range(2))
+    ops.kernels().head_gemm(x, w, y)
+    ops.kernels().head_gemm(at(x, dx), at(w, dw), yo)
+    assert torch.equal(y, yo)
+
+
 def _attend(q, k, v, scale, window=0):
     n, T = k.shape[0], q.shape[0]
     s = torch.einsum("thd,jhd->htj", q.double(), k.double()) * scale
