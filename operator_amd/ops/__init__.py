@@ -449,14 +449,33 @@ def skinny_plan(M: int, N: int, K: int) -> int | None:
 
 
 def _mid_beats_skinny(M: int, N: int, K: int, defer: bool) -> bool:
-    """gemm_skinny streams the weights once per call but pays for every row (a 128256 x 4096 vocabulary: 199 us at
-    1 row, 242 at 8, 440 at 32; 4 % of the one-row time per row at every measured shape); gemm_mid's 128-row
+    """gemm_skinny streams the weights once per call but pays for every row (a 128256 x 4096 vocabulary: 186 us at
+    1 row, 238 at 8, 428 at 32; 4 % of the one-row time per row at every measured shape); gemm_mid's 128-row
     tile costs the same at any of them (217 us). A few rows of a projection stay: too little work to split. So do shapes
-    with a measured entry (32 rows of 4096 x 4096: 15.5 us against 17.6 in slices)."""
+    with a measured entry (32 rows of 4096 x 4096: 15.5 us against 17.6 in slices).
+
+    Few rows stream the weights at 5.3 to 5.8 TB/s, rows of 2048 or 4096 columns (a power of two: neighbouring rows
+    share memory channels) at 4.1 to 4.8: vocabularies of 32768 x 4096, 5 rows 55 us against 66, of 128256 x 3072 176
+    against 135. A consumer that sums up to 16 slabs of a few rows waits for them in turn, 2 us (5): 24 rows of
+    2560 x 2048 with the norm behind them 11.5 us against 13.8, 17 of 4096 x 4096 16.1 against 17.9."""
     if M <= (4 if N >= LM_HEAD_MIN_N else 16) or ("skinny", M, N, K) in _gemm_table_get():
         return False
+    return _mid_few_rows(M, N, K, defer)
+
+
+@functools.lru_cache(maxsize=4096)
+def _mid_few_rows(M: int, N: int, K: int, defer: bool) -> bool:
+    """The estimates of _mid_beats_skinny."""
     S = mid_plan(M, N, K, defer)
-    return S is not None and _mid_cost(M, N, K, S, defer) < (3 + 2e-6 * N * K / 5.4) * (1 + 0.04 * M)
+    if S is None:
+        return False
+    shared = K & (K - 1) == 0 and K <= 4096
+    mid = _mid_cost(M, N, K, S, defer)
+    if N >= LM_HEAD_MIN_N:
+        mid = max(mid, 6 + 2e-6 * N * K / (4.2 if shared else 5.2))
+    elif defer and S > 1:
+        mid += 5 if shared else 2
+    return mid < (3 + 2e-6 * N * K / 5.4) * (1 + 0.04 * M)
 
 
 # Every GPU GEMM of the model runs on the hand-written gfx950 kernels: prefill projections (M > 256
@@ -613,8 +632,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, sp
     if (x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous() and M <= SKINNY_MAX_M
             and bm is None and bn is None):
         S = splits or skinny_plan(M, N, K)
-        if (S is not None and splits is None and out is None and tile_ok(x, w) and (x.data_ptr() | w.data_ptr()) % 16 == 0
-                and _mid_beats_skinny(M, N, K, defer_reduce)):
+        if (S is not None and splits is None and out is None and _mid_beats_skinny(M, N, K, defer_reduce) and tile_ok(x, w)
+                and (x.data_ptr() | w.data_ptr()) % 16 == 0):
             return linear_tile(x, w, defer_reduce=defer_reduce)
         if S is not None:
             if S > 1 and (partial is None or partial.numel() < S * M * N):

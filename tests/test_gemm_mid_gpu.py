@@ -145,3 +145,14 @@ def test_few_rows_off_their_alignment_stay_on_plain_loads(monkeypatch, dx, dw, k
     for defer in (False, True):
         ops.linear(x, w, defer_reduce=defer)
     assert seen == [kernel] * 2
+
+
+def test_few_rows_leave_gemm_skinny_where_it_was_measured_slower():
+    """Both sides were timed at these shapes (rows, N, K, deferred): none of the first is faster in gemm_mid."""
+    for M, N, K, defer in ((17, 3072, 3072, True), (24, 2560, 2048, True), (32, 2048, 2048, True), (17, 4096, 4096, True),
+                           (17, 2048, 8192, True), (5, 32768, 4096, False), (8, 32768, 4096, False), (6, 151936, 2048, False),
+                           (5, 64128, 4096, False), (5, 128256, 2048, False)):
+        assert not ops._mid_beats_skinny(M, N, K, defer), (M, N, K, defer)
+    for M, N, K, defer in ((17, 4096, 14336, True), (24, 3584, 3584, True), (32, 6144, 4096, False), (5, 128256, 3072, False),
+                           (6, 128256, 8192, False), (5, 152064, 3584, False), (8, 128256, 4096, False), (16, 32768, 4096, False)):
+        assert ops._mid_beats_skinny(M, N, K, defer), (M, N, K, defer)
