@@ -26,6 +26,7 @@ everything else is a hand-written HIP kernel too (operator_amd.ops).
 """
 from __future__ import annotations
 
+import functools
 import math
 import os
 from dataclasses import dataclass
@@ -129,12 +130,12 @@ class LlamaModel(DecoderModel):
             setattr(lw, {"wqkv": "sqkv", "wo": "so", "wgu": "sgu", "wd": "sd"}[name], sc)
         return lw
 
-    def _lin(self, x: torch.Tensor, w: torch.Tensor, sc: torch.Tensor | None, defer: bool = False):
-        """Projection; ``defer`` lets a split-K decode GEMM hand its fp32 slabs to the
-        following rmsnorm (only when no TP all-reduce sits in between)."""
+    def _lin(self, x: torch.Tensor, w: torch.Tensor, sc: torch.Tensor | None, defer: bool = False, prompt: bool = False):
+        """Projection; ``defer`` lets a split-K GEMM hand its fp32 slabs to the following
+        rmsnorm (only when no TP all-reduce sits in between), ``prompt``: as for ``ops.linear``."""
         if sc is not None:   # every fp8 consumer (rope_kv, the AR + norm, SwiGLU) sums slabs
             return ops.linear_fp8(x, w, sc, defer_reduce=defer)
-        return ops.linear(x, w, defer_reduce=defer and self.tp.world == 1)
+        return ops.linear(x, w, defer_reduce=defer and self.tp.world == 1, prompt=prompt)
 
     def _shard_layer(self, wq, wk, wv, wo, wg, wu, wd, an, mn, bias=None) -> LayerWeights:
         """One layer's weights, sharded for this TP rank; ``bias`` = (bq, bk, bv) or None."""
@@ -224,6 +225,7 @@ class LlamaModel(DecoderModel):
         T = h.shape[0]
         q8 = self.fp8 and h.is_cuda   # block epilogues emit e4m3fn rows for the next fp8 GEMM
         x = (ops.rmsnorm_fp8 if q8 else ops.rmsnorm)(h, self.layers[0].attn_norm, c.rms_eps)
+        lin = functools.partial(self._lin, prompt=True) if fb.is_prefill else self._lin
         ws = None
         if not fb.is_prefill and h.is_cuda:  # split-KV partials, shared by every layer
             ws = ops.decode_workspace(T, self.hq, fb.num_splits, h.device)
@@ -234,9 +236,9 @@ class LlamaModel(DecoderModel):
             # rounding; a prefill bias rides the tile GEMM's epilogue or its first slab
             bias = lw.bqkv
             if bias is not None and fb.is_prefill and lw.sqkv is None:
-                qkv, bias = ops.linear(x, lw.wqkv, bias=bias, defer_reduce=self.tp.world == 1), None
+                qkv, bias = ops.linear(x, lw.wqkv, bias=bias, defer_reduce=self.tp.world == 1, prompt=True), None
             else:
-                qkv = self._lin(x, lw.wqkv, lw.sqkv, defer=True)
+                qkv = lin(x, lw.wqkv, lw.sqkv, defer=True)
             if fb.is_prefill:
                 q, k, v = ops.rope_kv(qkv, fb.positions, self.cos, self.sin, self.hq, self.hkv, kc, vc, fb.slots,
                                       want_kv=True, bias=bias, k_scale=kv.k_scale, v_scale=kv.v_scale)
@@ -251,15 +253,15 @@ class LlamaModel(DecoderModel):
                 o = ops.attn_decode_rope(qkv, fb.positions, self.cos, self.sin, self.hq, kc, vc, fb.slots,
                                          fb.block_tables, fb.context_lens, self.scale, fb.num_splits, workspace=ws,
                                          bias=bias, k_scale=kv.k_scale, v_scale=kv.v_scale, quant=q8)
-            a = self._lin(o if isinstance(o, tuple) else o.view(T, self.hq * c.head_dim), lw.wo, lw.so, defer=True)
+            a = lin(o if isinstance(o, tuple) else o.view(T, self.hq * c.head_dim), lw.wo, lw.so, defer=True)
             x = self.tp.all_reduce_rmsnorm(a, lw.mlp_norm, c.rms_eps, residual=h, quant=q8)   # fused under TP
             if lw.sgu is None:
-                m = ops.gate_up_silu(x, lw.wgu, self.gu_block)
+                m = ops.gate_up_silu(x, lw.wgu, self.gu_block, prompt=fb.is_prefill)
             elif q8:   # SwiGLU (+ the split-K sum) fused into the down GEMM's input quantization
                 m = ops.silu_quantize_fp8(ops.linear_fp8(x, lw.wgu, lw.sgu, defer_reduce=True), self.gu_block)
             else:
                 m = ops.silu_mul(ops.linear_fp8(x, lw.wgu, lw.sgu), block=self.gu_block)
-            d = self._lin(m, lw.wd, lw.sd, defer=True)
+            d = lin(m, lw.wd, lw.sd, defer=True)
             last = i + 1 == len(self.layers)
             nw = self.final_norm if last else self.layers[i + 1].attn_norm
             x = self.tp.all_reduce_rmsnorm(d, nw, c.rms_eps, residual=h, quant=q8 and not last)

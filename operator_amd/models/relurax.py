@@ -188,8 +188,9 @@ class ReluraxModel(PaddedModel):
             after = None if i + 1 == len(self.layers) else (one, self.layers[i + 1].norm1)
             if lw.norm2 is not None:
                 h = self._step(x, dec.SublayerOut(y=y), self.hc, (one, lw.norm2), fb, lw.norm1b)
-                m = ops.gate_up_silu(h, lw.wgu, self.gu_block, ops.GELU_TANH)
-                h = self._step(x, dec.SublayerOut(y=ops.linear(m, lw.wd, defer_reduce=True)), self.hc, after, fb, lw.norm2b)
+                m = ops.gate_up_silu(h, lw.wgu, self.gu_block, ops.GELU_TANH, fb.is_prefill)
+                y = ops.linear(m, lw.wd, defer_reduce=True, prompt=fb.is_prefill)
+                h = self._step(x, dec.SublayerOut(y=y), self.hc, after, fb, lw.norm2b)
             else:
                 h = self._step(x, dec.SublayerOut(y=y), self.hc, after, fb, lw.norm1b)
             if fb.residual_sink is not None:
@@ -206,32 +207,33 @@ class ReluraxModel(PaddedModel):
     def _window_mixer(self, i: int, lw: ReluraxLayer, h, edges, fb: ForwardBatch, kv: PagedKVCache, ws):
         a, L, cache = self.cfg.layer_specs[i].mixer, self.shapes[i], kv.layer(i)
         # a prefill reads every row once per tap: whole rows, not slabs
-        q, k, v, gate = dec.conv_heads(ops.linear(h, lw.win, defer_reduce=not fb.is_prefill), fb.positions, L, self.dtype, lw.conv, lw.qnorm,
-                                       lw.knorm, cache, kv.state[i], fb.slots, edges)
+        y = ops.linear(h, lw.win, defer_reduce=not fb.is_prefill, prompt=fb.is_prefill)
+        q, k, v, gate = dec.conv_heads(y, fb.positions, L, self.dtype, lw.conv, lw.qnorm, lw.knorm, cache, kv.state[i], fb.slots, edges)
         if fb.is_prefill:
             o = self._prefill(i, q, k, v, gate, fb, L, a.window)
         else:
             # the step's split count is chosen for whole contexts; a window needs no more than its own
             splits = min(fb.num_splits, ops.decode_splits(a.window or self.cfg.max_position, h.shape[0], L.kv_heads, self.split_tokens))
             o = dec.attn_gd_decode(q, cache, fb.block_tables, fb.context_lens, L, a.scale, splits, ws, a.window, gate)
-        return ops.linear(o, lw.wo, defer_reduce=True)
+        return ops.linear(o, lw.wo, defer_reduce=True, prompt=fb.is_prefill)
 
     def _latent_mixer(self, i: int, lw: ReluraxLayer, h, rows: dict, fb: ForwardBatch, kv: PagedKVCache, ws):
         a, L = self.cfg.layer_specs[i].mixer, self.shapes[i]
         src = i if L.own else a.kv_from
         cache = kv.layer(src)[0]
-        cq, gate, row = dec.latent_rows(ops.linear(h, lw.win, defer_reduce=True), fb.positions, self.rot[i], L, self.dtype, lw.qnorm,
-                                        lw.knorm, cache if L.own else None, fb.slots)
-        q = dec.rotate_heads(ops.linear(cq, lw.wuq, defer_reduce=True), fb.positions, self.rot[i], L, self.dtype)
+        y = ops.linear(h, lw.win, defer_reduce=True, prompt=fb.is_prefill)
+        cq, gate, row = dec.latent_rows(y, fb.positions, self.rot[i], L, self.dtype, lw.qnorm, lw.knorm, cache if L.own else None, fb.slots)
+        y = ops.linear(cq, lw.wuq, defer_reduce=True, prompt=fb.is_prefill)
+        q = dec.rotate_heads(y, fb.positions, self.rot[i], L, self.dtype)
         if fb.is_prefill:
             if L.own:
                 rows[i] = row
             T, (dk, dv) = cq.shape[0], L.pads
-            k = ops.linear(rows[src], lw.wk).view(T, L.heads, dk)
-            v = ops.linear(rows[src], lw.wv).view(T, L.heads, dv)
+            k = ops.linear(rows[src], lw.wk, prompt=True).view(T, L.heads, dk)
+            v = ops.linear(rows[src], lw.wv, prompt=True).view(T, L.heads, dv)
             o = self._prefill(i, q, k, v, gate, fb, L)
         else:
             o = dec.attn_latent_decode(dec.to_latent(q, lw.wabs, L), cache, fb.block_tables, fb.context_lens, L, a.scale,
                                        fb.num_splits, ws, gate)
             o = dec.from_latent(o, lw.wuv, L)
-        return ops.linear(o, lw.wo, defer_reduce=True)
+        return ops.linear(o, lw.wo, defer_reduce=True, prompt=fb.is_prefill)

@@ -170,7 +170,7 @@ class SufolixModel(PaddedModel):
             hc = dec.Stream(lw.in1, lw.mix1, lw.out1)
             if lw.norm2 is not None:
                 h = self._step(x, dec.SublayerOut(y=y), hc, (lw.in2, lw.norm2), fb)
-                y = self._feed_forward(lw, c.layer_specs[i].mlp, h)
+                y = self._feed_forward(lw, c.layer_specs[i].mlp, h, fb.is_prefill)
                 hc = dec.Stream(lw.in2, lw.mix2, lw.out2)
             else:
                 y = dec.SublayerOut(y=y)
@@ -183,7 +183,7 @@ class SufolixModel(PaddedModel):
         """(o-projection output, the first mixing layer's values)."""
         a, L = self.cfg.layer_specs[i].mixer, self.heads[i]
         cache = kv.layer(i)
-        qkv = ops.linear(h, lw.wqkv, defer_reduce=True)
+        qkv = ops.linear(h, lw.wqkv, defer_reduce=True, prompt=fb.is_prefill)
         mixed = v_first if lw.lam is not None else None
         q, k, v = dec.qkv_heads(qkv, fb.positions, self.rot[i], L, self.dtype, bias=lw.bqkv, cache=cache, slots=fb.slots,
                                 want_k=fb.is_prefill, want_v=fb.is_prefill or i == self.first_mix, v_first=mixed, lam=lw.lam)
@@ -196,14 +196,15 @@ class SufolixModel(PaddedModel):
             o = dec.attn_gd_prefill(q, k, v, fb.seq_lens, L, a.scale, work=fb.prefill_work, prefix=pre)
         else:
             o = dec.attn_gd_decode(q, cache, fb.block_tables, fb.context_lens, L, a.scale, fb.num_splits, ws)
-        return ops.linear(o, lw.wo, defer_reduce=True), v_first
+        return ops.linear(o, lw.wo, defer_reduce=True, prompt=fb.is_prefill), v_first
 
-    def _feed_forward(self, lw: SufolixLayer, m, h) -> dec.SublayerOut:
+    def _feed_forward(self, lw: SufolixLayer, m, h, prompt: bool) -> dec.SublayerOut:
         if not m.experts:
-            return dec.SublayerOut(y=ops.linear(ops.gate_up_silu(h, lw.wgu, self.gu_block), lw.wd, defer_reduce=True))
+            return dec.SublayerOut(y=ops.linear(ops.gate_up_silu(h, lw.wgu, self.gu_block, prompt=prompt), lw.wd, defer_reduce=True,
+                                                prompt=prompt))
         ids, wt, gate = dec.route(h, lw.wr, m.experts, m.top, bool(m.shared_ff))
         e, epos = dec.experts(h, ids, wt, lw.wgu, lw.wd)
         y = None
         if m.shared_ff:
-            y = ops.linear(ops.gate_up_silu(h, lw.sgu, self.gu_block), lw.sd, defer_reduce=True)
+            y = ops.linear(ops.gate_up_silu(h, lw.sgu, self.gu_block, prompt=prompt), lw.sd, defer_reduce=True, prompt=prompt)
         return dec.SublayerOut(y=y, gate=gate, e=e, epos=epos, top=m.top)

@@ -138,14 +138,14 @@ def gate_up_plan(M: int, N: int):
     return 64 if M // 64 * tiles <= CUS else None
 
 
-def gate_up_silu(x: torch.Tensor, wgu: torch.Tensor, block: int | None, act: int = SILU) -> torch.Tensor:
+def gate_up_silu(x: torch.Tensor, wgu: torch.Tensor, block: int | None, act: int = SILU, prompt: bool = False) -> torch.Tensor:
     """act(x Wg^T) * (x Wu^T) from the interleaved gate|up weight (``act``: SILU or GELU_TANH). Decode
     buckets run one fused gfx950 kernel (GEMM + gated epilogue, no [M, 2I] intermediate);
-    other shapes run the GEMM then the silu_mul kernel."""
+    other shapes run the GEMM then the silu_mul kernel. ``prompt``: as for ``linear``."""
     M, K = x.shape
     N = wgu.shape[0]
     if x.is_cuda and block == 64 and f32_ok(x, wgu):
-        return linear_f32(x, wgu, glu=act)
+        return linear_f32(x, wgu, glu=act, prompt=prompt)
     if (x.is_cuda and block == 64 and x.dtype == torch.bfloat16 and M <= SKINNY_MAX_M and N % 128 == 0
             and K % 128 == 0 and x.is_contiguous() and wgu.is_contiguous()
             and skinny_plan(M, N, K) is not None and _gemm_table_get().get(("silu", M, N, K)) != "blas"):
@@ -157,7 +157,7 @@ def gate_up_silu(x: torch.Tensor, wgu: torch.Tensor, block: int | None, act: int
         t = _gemm_table_get().get(("silu", M, N, K))
         bm = gate_up_plan(M, N) if t is None else t if isinstance(t, str) else t[0]
         if t is None and bm is None:
-            return linear_tile(x, wgu, glu=act)
+            return linear_tile(x, wgu, glu=act, prompt=prompt)
         if isinstance(bm, str) and bm.startswith("pp"):   # ping-pong kernel, nt weight loads (bm 128 / 256)
             y = torch.empty(M, N // 2, dtype=x.dtype, device=x.device)
             bm = int(bm[2:])
@@ -176,8 +176,8 @@ def gate_up_silu(x: torch.Tensor, wgu: torch.Tensor, block: int | None, act: int
             kernels().gemm_decode(x, wgu, y, None, 1, 128, bm, act, False, ns)
             return y
     if block == 64 and tile_ok(x, wgu) and N % 128 == 0:
-        return linear_tile(x, wgu, glu=act)   # prefill: gating fused into the tile epilogue
-    return silu_mul(linear(x, wgu), block=block, act=act)
+        return linear_tile(x, wgu, glu=act, prompt=prompt)   # prefill: gating fused into the tile epilogue
+    return silu_mul(linear(x, wgu, prompt=prompt), block=block, act=act)
 
 
 # Stream-K form of the 256-row gate|up+SwiGLU decode GEMM (csrc/kernels/gemm_pp.hip SK): one block per
@@ -542,19 +542,18 @@ def _mid_cost(M: int, N: int, K: int, S: int, defer: bool) -> float:
 
 
 @functools.lru_cache(maxsize=4096)
-def mid_plan(M: int, N: int, K: int, defer: bool, slices: bool = True) -> int | None:
+def mid_plan(M: int, N: int, K: int, defer: bool, slices: bool = True, prompt: bool = False) -> int | None:
     """K slices for gemm_mid (1: none), or None where the 256-row tiles are cheaper. One prompt of a few hundred
     tokens has fewer 256-row tiles than the GPU has CUs: smaller tiles and K slices fill it (885 rows: 4096 x 14336
     103 us against 297, 6144 x 4096 56 against 89); once every CU has a 256-row tile, that tile's fewer operand
     bytes per product win (4096 rows of 4096 x 14336: 325 us against 371).
 
-    Rows that are no decode bucket's (above 256, or above 32 and no multiple of 64) are a prompt's and take the plan of
-    the next multiple of 512: a prefill graph pads its batch to such a size, and a prompt's numbers are the same padded or
-    not (100 rows of 4096 x 14336 with the norm behind them: 58 us in the four slices of 512 rows, 36 in fourteen, 285 on
-    the 256-row tiles). From LM_HEAD_MIN_N features on, where 512 rows run on the 256-row tiles, they are not sliced. Past
+    Above 256 rows, and from 33 rows of a ``prompt`` on, the plan is the next multiple of 512's: a prefill graph pads its
+    batch to such a size, and a prompt's numbers are the same padded or not (100 rows of 4096 x 14336 with the norm behind them: 58 us in the four slices of 512 rows, 36 in fourteen, 285 on
+    the 256-row tiles). From LM_HEAD_MIN_N features on, where 512 rows run on the 256-row tiles, a prompt is not sliced. Past
     4096 rows the graphs' sizes are coarser and little is left to gain. Prompts of up to 32, and of 64, 128, 192 or 256
     rows run on a decode kernel when they are not padded."""
-    prompt = M > SKINNY_MAX_M and M % 64 != 0
+    prompt = prompt and M > SKINNY_MAX_M
     if M > 256 or (prompt and N < LM_HEAD_MIN_N):
         M = -(-M // 512) * 512
     if M < 1 or M > 4096 or K < 128 or (M > 128 and N >= LM_HEAD_MIN_N):   # 256 rows of a vocabulary: 282 us against 253
@@ -566,17 +565,18 @@ def mid_plan(M: int, N: int, K: int, defer: bool, slices: bool = True) -> int | 
 
 
 def linear_tile(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None,
-                bias: torch.Tensor | None = None, glu: int = 0, defer_reduce: bool = False):
+                bias: torch.Tensor | None = None, glu: int = 0, defer_reduce: bool = False, prompt: bool = False):
     """Prefill / lm_head GEMM on the compute-bound gfx950 tile kernels (fused bias or gated (``glu``: SILU /
     GELU_TANH) epilogue): 128 x 256 tiles with K slices for few rows (``mid_plan``), else 256 x 256 tiles (LDS-DMA
-    ping-pong pipeline). ``defer_reduce``: K slices come back as fp32 slabs (:class:`SplitK`)."""
+    ping-pong pipeline). ``defer_reduce``: K slices come back as fp32 slabs (:class:`SplitK`);
+    ``prompt``: rows a prefill graph may pad."""
     M, K = x.shape
     N = w.shape[0]
     defer = defer_reduce and out is None and not glu
     S = None
     if (out is None or (out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0)) and (
             bias is None or (bias.is_contiguous() and bias.data_ptr() % 16 == 0)):   # gemm_mid's 16-B accesses
-        S = mid_plan(M, N, K, defer, out is None or out.stride(0) == out.shape[1])   # the reduce pass has no row stride
+        S = mid_plan(M, N, K, defer, out is None or out.stride(0) == out.shape[1], prompt)   # the reduce pass has no row stride
     part = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if S is not None and S > 1 else None
     if part is not None and defer:
         kernels().gemm_mid(x, w, None, bias, part, S)
@@ -595,13 +595,19 @@ def f32_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
             and w.is_contiguous() and x.shape[1] % 16 == 0)
 
 
-def linear_f32(x: torch.Tensor, w: torch.Tensor, glu: int = 0) -> torch.Tensor:
+def f32_plan_rows(M: int, prompt: bool) -> int:
+    """Rows whose K slices an fp32 product takes: a prompt's are those of its padded prefill graph (see mid_plan), so its
+    numbers are the same padded or not; up to 32 rows run on the few-row kernel."""
+    return -(-M // 512) * 512 if prompt and M > SKINNY_MAX_M else M
+
+
+def linear_f32(x: torch.Tensor, w: torch.Tensor, glu: int = 0, prompt: bool = False) -> torch.Tensor:
     """x @ w^T in full 32-bit products and sums, optionally with the gated epilogue (SILU / GELU_TANH) over a 64-row
-    interleaved gate|up weight."""
+    interleaved gate|up weight. ``prompt``: as for ``linear``."""
     M, K = x.shape
     N = w.shape[0]
     y = torch.empty(M, N // 2 if glu else N, dtype=x.dtype, device=x.device)
-    S = kernels().gemm_f32_splits(M, N, K, glu)
+    S = kernels().gemm_f32_splits(f32_plan_rows(M, prompt), N, K, glu)
     part = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if S > 1 else None
     kernels().gemm_f32(x, w, y, glu, partial=part, splits=S)
     return y
@@ -609,21 +615,22 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, glu: int = 0) -> torch.Tensor:
 
 def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, splits: int | None = None,
            partial: torch.Tensor | None = None, bn: int | None = None, bm: int | None = None,
-           defer_reduce: bool = False, stages: int | None = None, bias: torch.Tensor | None = None):
+           defer_reduce: bool = False, stages: int | None = None, bias: torch.Tensor | None = None, prompt: bool = False):
     """y = x @ w^T (+ bias) in bf16 on the gfx950 kernels: M <= 32 decode buckets on the
     weight-streaming gemm_skinny, M in {64, 128, 256} on the LDS-staged split-K
     gemm_decode (tuned tables), everything else (prefill, the lm_head, biased
     projections) on the 256x256-tile gemm_tile (persistent p5 past 256 rows). hipBLASLt only
     for shapes none of them takes (K % 64 != 0, N % 16 != 0, non-bf16), for decode shapes the
-    tuned table measured it fastest on, or under OAMD_PREFILL_BLAS=1 (A/B); CPU tensors on torch."""
+    tuned table measured it fastest on, or under OAMD_PREFILL_BLAS=1 (A/B); CPU tensors on torch.
+    ``prompt``: rows of prompts, which a prefill graph pads (mid_plan)."""
     M, K = x.shape
     N = w.shape[0]
     plan = None
     if x.is_cuda and bias is None and out is None and f32_ok(x, w):
-        return linear_f32(x, w)
+        return linear_f32(x, w, prompt=prompt)
     if bias is not None:
         if tile_ok(x, w) and tile_out_ok(out):
-            return linear_tile(x, w, out, bias, defer_reduce=defer_reduce)
+            return linear_tile(x, w, out, bias, defer_reduce=defer_reduce, prompt=prompt)
         return _blas(x, w, out, bias)
     if x.is_cuda and bm is None and bn is None and splits is None and _measured_blas(M, N, K):
         return _blas(x, w, out, None)
@@ -650,7 +657,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, sp
             plan = (row_tile(M), 64, 1)  # explicit request (tests / tuning)
     if plan is None:
         if tile_ok(x, w) and tile_out_ok(out):
-            return linear_tile(x, w, out, defer_reduce=defer_reduce)
+            return linear_tile(x, w, out, defer_reduce=defer_reduce, prompt=prompt)
         return _blas(x, w, out, None)
     bm, bn, S = bm or plan[0], bn or plan[1], splits or plan[2]
     ns = stages or (plan[3] if len(plan) > 3 else 3)

@@ -83,13 +83,21 @@ def test_mid_plan_is_launchable():
                 assert S is None or 1 <= S <= min(16, K // 64)
                 assert ops.mid_plan(M, N, K, defer, False) in (None, 1)
             assert ops.mid_plan(322, N, K, defer) == ops.mid_plan(512, N, K, defer)
-            for M in (33, 63, 65, 100, 127, 129, 200, 255):   # no decode bucket: a prompt, in its graph one of 512 rows
+            for M in (33, 64, 65, 100, 127, 129, 200, 255):   # a prompt, in its graph one of 512 rows
                 if N < ops.LM_HEAD_MIN_N:
-                    assert ops.mid_plan(M, N, K, defer) == ops.mid_plan(512, N, K, defer)
+                    assert ops.mid_plan(M, N, K, defer, prompt=True) == ops.mid_plan(512, N, K, defer)
                 else:   # the 512-row plan is the 256-row tiles over the whole K: no slices
-                    assert ops.mid_plan(M, N, K, defer) in (None, 1) and ops.mid_plan(512, N, K, defer) is None
+                    assert ops.mid_plan(M, N, K, defer, prompt=True) in (None, 1) and ops.mid_plan(512, N, K, defer) is None
     assert ops.mid_plan(28000, 4096, 14336, True) is None
     assert ops.mid_plan(885, 4096, 14336, True) == 2
+    # a decode batch of the same rows is not padded: slices that fill the GPU
+    assert ops.mid_plan(100, 4096, 14336, True) == 14 > ops.mid_plan(100, 4096, 14336, True, prompt=True) == 4
+
+
+def test_fp32_prompts_take_their_graphs_slices():
+    for M in (33, 100, 255, 256, 500, 512):
+        assert ops.f32_plan_rows(M, True) == 512 and ops.f32_plan_rows(M, False) == M
+    assert ops.f32_plan_rows(513, True) == 1024 and ops.f32_plan_rows(32, True) == 32
 
 
 @pytest.mark.parametrize("M,N,K,wide", [(1, 4096, 4096, 8192), (1, 272, 1024, 288), (1, 4096, 4096, 4096), (40, 4096, 4096, 8192)])

@@ -7,6 +7,7 @@ from operator_amd.engine.llm import GenRequest, LLMEngine
 from operator_amd.models.config import get_config
 from operator_amd.models.kv_cache import PagedKVCache
 from operator_amd.models.llama import ForwardBatch, LlamaModel
+from operator_amd.models.registry import build_model
 
 pytestmark = pytest.mark.gpu
 
@@ -265,22 +266,25 @@ def test_graph_prefill_equals_eager_prefill():
     assert torch.equal(caches[0], caches[1])
 
 
-@pytest.mark.parametrize("name", ["tiny-gqa4", "tiny-qwen"])
+@pytest.mark.parametrize("name,dtype", [("tiny-gqa4", "bfloat16"), ("tiny-qwen", "bfloat16"), ("tiny-sufolix", "bfloat16"),
+                                        ("tiny-relurax", "bfloat16"), ("tiny-sufolix", "float32"), ("tiny-relurax", "float32")])
 @pytest.mark.parametrize("lens", [[40], [33, 60], [100, 99], [255], [130, 170], [700]])
-def test_prompt_rows_are_the_same_in_a_graph(name, lens):
+def test_prompt_rows_are_the_same_in_a_graph(name, dtype, lens):
     """Prompts that are no decode bucket's size (33 to 255 tokens, or more) write the same keys and values, bit for bit,
     eagerly and padded to their graph's 512 or 1024 rows: the K slices of a projection do not change with the padding."""
-    cfg = get_config(name)
-    m = LlamaModel(cfg, device="cuda").init_random(seed=7)
+    m = build_model(get_config(name), device="cuda", dtype=getattr(torch, dtype)).init_random(7)
     caches = []
     for pg in (False, True):
-        kv = PagedKVCache(cfg.layers, 64, cfg.kv_heads, 128, 16, device="cuda")
+        kv = PagedKVCache.for_model(m, 64, 16)
+        for t in (*kv.k, *kv.v):
+            t.zero_()
         eng = LLMEngine(m, kv, max_batch=4, max_prefill_tokens=1024, max_context=1024, prefill_graphs=pg, prefix_sharing=False)
-        reqs = [GenRequest(list(range(3 + i, 3 + i + n)), max_tokens=1, ignore_eos=True) for i, n in enumerate(lens)]
+        reqs = [GenRequest([3 + (i + j) % 900 for j in range(n)], max_tokens=1, ignore_eos=True) for i, n in enumerate(lens)]
         eng.generate(reqs)
         assert eng.stats.prefill_graph_replays == pg
-        caches.append(torch.stack([t.float() for i in range(cfg.layers) for t in kv.layer(i)]).cpu())
-    assert torch.equal(caches[0], caches[1])
+        caches.append([t.float().cpu() for t in (*kv.k, *kv.v)])
+    for a, b in zip(*caches):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("B", [3, 64])
