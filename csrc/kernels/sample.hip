@@ -138,10 +138,12 @@ __global__ void __launch_bounds__(256) sample_merge_kernel(const float2* __restr
   }
 }
 
-// Workgroups per row: up to eight per CU in all, 2048 columns each at least. From 256 rows on one per row fills the
-// GPU (128256 columns, 256 rows: 33 us against 36; 128 rows 31 against 24).
+// Workgroups per row: up to eight per CU in all, 2048 columns each at least, where they gain more than the merge kernel
+// costs (captured, one workgroup against several): 16384 columns 1 row 6.7 us against 5.7, 64 rows 7.3 and 6.6 (12288: 6.1 and
+// 6.6); 32000 columns 128 rows 13.7 and 11.0 (20480: 7.9 and 8.2); 100000 columns 192 rows 25.0 and 22.2 (65536: 18.2 and 21.6).
+// More rows fill the GPU with one each (128256 columns, 240 rows: 31.7 and 34.5).
 int sample_parts(int rows, int vocab) {
-  if (rows >= 256) return 1;
+  if (rows > 224 || vocab < (rows <= 64 ? 16384 : rows <= 160 ? 28672 : 98304)) return 1;
   return max(1, min(min(32, 2048 / max(rows, 1)), vocab / 2048));
 }
 
