@@ -358,11 +358,11 @@ class Scorer {
          int64_t num_matchers)
       : conf_(std::move(conf)), sev_(std::move(sev)), sec_(std::move(sec)), w_(std::move(w)), win_(std::move(win)), primary_of_(num_matchers) {
     const size_t P = primary.size();
-    if (conf_.size() != P || sev_.size() != P || sec_.size() != P || w_.size() != P || win_.size() != P)
-      throw std::invalid_argument("pattern tables differ in length");
+    if (conf_.size() < P || sev_.size() < P || sec_.size() < P || w_.size() < P || win_.size() < P)
+      throw std::invalid_argument("pattern tables shorter than the patterns");
     for (size_t p = 0; p < P; ++p) {
       if (primary[p] < 0 || primary[p] >= num_matchers) throw std::out_of_range("pattern primary");
-      if (w_[p].size() != sec_[p].size() || win_[p].size() != sec_[p].size()) throw std::invalid_argument("secondary tables differ in length");
+      if (w_[p].size() < sec_[p].size() || win_[p].size() < sec_[p].size()) throw std::invalid_argument("secondary tables too short");
       primary_of_[primary[p]].push_back(static_cast<int>(p));
     }
   }

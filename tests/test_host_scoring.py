@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from operator_amd.engine.match import MatchEngine
+from operator_amd.ops import patterns
 from operator_amd.patterns import oracle
 from operator_amd.patterns.compiler import compile_patterns
 from operator_amd.patterns.synth import LogFactory, synthetic_library
@@ -26,6 +27,21 @@ def test_kept_scorer_matches_oracle(docs, n):
             want = oracle.score_doc(eng.cp, {(int(m), int(l)) for i, m, l in hits if i == d})
             assert [(e.pattern, e.line) for e in evs[d]] == [(e.pattern, e.line) for e in want]
             assert [e.score for e in evs[d]] == pytest.approx([e.score for e in want], abs=1e-12)
+
+
+def test_score_events_takes_longer_tables():
+    """The tables' extra entries are not read; missing ones are refused, not read past the end."""
+    P = patterns()
+    hits, m = ([0, 0, 0], [0, 1, 1], [4, 6, 9]), 2
+    exact = ([0], [0.5], [3], [[1]], [[2.0]], [[10]])
+    longer = ([0], [0.5, 9.0], [3, 1], [[1], [0]], [[2.0, 7.0], []], [[10, 1], [5]])
+    want = P.score_events(*hits, 1, *exact, m)
+    assert len(want[0]) == 1 and P.score_events(*hits, 1, *longer, m) == want
+    for i in range(1, 6):
+        short = list(exact)
+        short[i] = [] if i < 4 else [[]]
+        with pytest.raises(ValueError):
+            P.score_events(*hits, 1, *short, m)
 
 
 @pytest.mark.parametrize("native,gpu_scorer,n,on_gpu", [
