@@ -701,7 +701,7 @@ def silu_quantize_fp8(gu, block: int | None = GU_BLOCK) -> tuple[torch.Tensor, t
             kernels().silu_quantize_fp8(torch.empty(M, N2, dtype=torch.bfloat16, device=gu.device), q, sx,
                                         gu.p, gu.S)
             return q, sx
-        if gu.stride(1) == 1:
+        if gu.stride(1) == 1 and (inter <= 16384 or gu.stride(0) % 8 == 0):   # long rows: as silu_mul takes them
             kernels().silu_quantize_fp8(gu, q, sx)
             return q, sx
     if isinstance(gu, SplitK):

@@ -45,3 +45,14 @@ def test_swiglu_of_long_rows(inter, S):
     # one e4m3fn ulp where the two kernels' silu differ in the last bit of its bf16 rounding
     got, want = q.float(), q0.float()
     assert ((got - want).abs() <= want.abs().clamp(min=2 ** -6) * 2 ** -3 + 1e-12).all() and (got == want).float().mean() > 0.99
+
+
+def test_long_rows_need_silu_muls_row_stride():
+    """Rows past 16384 features come in 16-B aligned strides, as they did when silu_mul read them; shorter ones in any."""
+    x = torch.randn(3, 2 * 16448 + 4, device="cuda").bfloat16()
+    with pytest.raises(RuntimeError, match="16-B aligned rows"):
+        ops.silu_quantize_fp8(x[:, :2 * 16448], block=64)
+    y = x[:, :2 * 8192]
+    q, s = ops.silu_quantize_fp8(y, block=64)
+    q0, s0 = ops.silu_quantize_fp8(y.contiguous(), block=64)
+    assert torch.equal(q.view(torch.uint8), q0.view(torch.uint8)) and torch.equal(s, s0)
