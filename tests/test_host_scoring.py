@@ -78,3 +78,24 @@ def test_gpu_scorer_alone():
     for docs in ([b"zzz\n", b""], logs):
         for a, b in zip(alone.analyze(docs), host.analyze(docs)):
             assert a.summary == b.summary and a.events == b.events
+
+
+@pytest.mark.gpu
+def test_default_engine_on_both_sides_of_the_host_threshold(monkeypatch):
+    """The same logs' events with as many hits as the host takes, and with one more."""
+    cp = compile_patterns(synthetic_library(100, seed=0))
+    eng, host = MatchEngine(cp, device="cuda"), MatchEngine(cp, device="cpu")
+    scored = []
+    monkeypatch.setattr(eng, "_events_gpu", lambda hits, docs, f=eng._events_gpu: scored.append(len(hits)) or f(hits, docs))
+    rng, n = random.Random(3), MatchEngine.HOST_SCORE_HITS
+    for extra in (0, 1):
+        rows = set()
+        while len(rows) < n + extra:
+            rows.add((rng.randrange(7), rng.randrange(cp.num_matchers), rng.randrange(400)))
+        hits = np.asarray(sorted(rows), dtype=np.int64)
+        got, want = (e._events_from_hits([b""] * 7, hits) for e in (eng, host))
+        for a, b in zip(got, want):
+            # an fp64 score is a dozen roundings of 2^-53 each, fused on the GPU; scores that differ so little may swap places
+            assert sorted((e.pattern, e.line) for e in a) == sorted((e.pattern, e.line) for e in b)
+            assert [e.score for e in a] == pytest.approx([e.score for e in b], rel=1e-14)
+    assert scored == [n + 1]

@@ -233,13 +233,30 @@ def test_context_spans_equal_host_contexts():
         assert a["metadata"]["totalLines"] == b["metadata"]["totalLines"]
 
 
-def test_context_windows_while_default_stream_is_busy():
+def _gpu_forms(eng: MatchEngine, monkeypatch) -> list:
+    """Scoring and context windows of ``eng`` on the GPU whatever the batch; the calls are listed."""
+    calls = []
+    monkeypatch.setattr(eng, "HOST_CONTEXT_DOCS", 0)
+    for name in ("_events_gpu", "_contexts_gpu"):
+        def spy(*a, _f=getattr(eng, name), _n=name, **k):
+            r = _f(*a, **k)
+            assert r is not None
+            calls.append(_n)
+            return r
+        monkeypatch.setattr(eng, name, spy)
+    return calls
+
+
+@pytest.mark.parametrize("gpu_scorer", [None, True])
+def test_context_windows_while_default_stream_is_busy(gpu_scorer, monkeypatch):
     """The flagship runs the LLM's decode graphs on the default stream while the match
     engine scans on its own: the GPU context windows (lazy analyze) must not read their
-    query / length buffers before those land (they are made on the scan stream)."""
+    query / length buffers before those land (they are made on the scan stream). With the GPU
+    scorer asked for, neither must its kernels."""
     ps = synthetic_library(200, seed=3)
     bdocs = LogFactory(n_patterns=200, seed=9).batch(48, 8 * 1024, n_failures=3, seed=5)[0]
-    eng = MatchEngine(ps, device="cuda", seg_bytes=1024, profile_bytes=0)
+    eng = MatchEngine(ps, device="cuda", seg_bytes=1024, profile_bytes=0, gpu_scorer=gpu_scorer)
+    calls = _gpu_forms(eng, monkeypatch)
     host = [r.to_obj() for r in MatchEngine(ps, device="cpu").analyze(bdocs)]
     for _ in range(3):
         torch.cuda._sleep(300_000_000)   # the default stream stays busy for ~0.1 s
@@ -247,6 +264,7 @@ def test_context_windows_while_default_stream_is_busy():
         for i, b in enumerate(host):
             a = got[i].to_obj()
             assert [e["context"] for e in a["events"]] == [e["context"] for e in b["events"]]
+    assert calls == (["_events_gpu", "_contexts_gpu"] if gpu_scorer else ["_contexts_gpu"]) * 3
     torch.cuda.synchronize()
 
 
@@ -276,19 +294,23 @@ def test_noisy_log_every_line_matches_equals_cpu_scan():
     assert _rows(gpu) == _rows(cpu)
 
 
+@pytest.mark.parametrize("gpu_forms", [False, True])
 @pytest.mark.parametrize("lazy", [False, True])
-def test_pipelined_analyze_equals_one_batch(lazy):
+def test_pipelined_analyze_equals_one_batch(lazy, gpu_forms, monkeypatch):
     """A large batch is analysed in sub-batches (MatchEngine._analyze_pipelined: the next
     sub-batch's pack + H2D + scan on a worker thread in the other buffer set, while the
     host verifies, scores and builds the previous one): every result equals the
     one-batch analyze and the host path, and three back-to-back calls reuse both
-    buffer sets."""
+    buffer sets. ``gpu_forms``: every sub-batch is scored and its context windows are read
+    on the GPU, on a second stream beside the next sub-batch's scan (by default sub-batches of
+    few documents and hits do both on the host)."""
     ps = synthetic_library(300, seed=4)
     docs = LogFactory(n_patterns=300, seed=11).batch(61, 24 * 1024, n_failures=3, seed=3)[0]
     docs[7] = b""                      # an empty doc inside a sub-batch
     one = MatchEngine(ps, device="cuda", seg_bytes=1024, profile_bytes=0)
     one.PIPE_SUB_BYTES = 0
-    pipe = MatchEngine(ps, device="cuda", seg_bytes=1024, profile_bytes=0)
+    pipe = MatchEngine(ps, device="cuda", seg_bytes=1024, profile_bytes=0, gpu_scorer=gpu_forms or None)
+    calls = _gpu_forms(pipe, monkeypatch) if gpu_forms else None
     pipe.PIPE_MIN_BYTES = 1
     pipe.PIPE_SUB_BYTES = 200 * 1024   # ~7 sub-batches
     subs = pipe._sub_batches(docs)
@@ -314,4 +336,8 @@ def test_pipelined_analyze_equals_one_batch(lazy):
         assert len(got) == len(docs)
         assert [strip(got[i].to_obj()) for i in range(len(docs))] == want
         assert pipe.last_timing["subs"] == len(subs)
+        if gpu_forms:
+            some = sum(any(w["events"] for w in want[lo:hi]) for lo, hi in subs)
+            assert some >= 5 and calls == ["_events_gpu", "_contexts_gpu"] * some
+            calls.clear()
     torch.cuda.synchronize()
