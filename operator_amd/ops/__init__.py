@@ -19,7 +19,7 @@ from ._native import kernels, native_available, patterns
 __all__ = [
     "rmsnorm", "silu_mul", "embedding", "rope_kv", "attn_prefill", "attn_decode", "attn_decode_rope", "sample",
     "kernels", "patterns", "native_available", "reference", "prefill_work_list", "prefill_block_q", "prefill_variant", "decode_splits",
-    "decode_workspace", "linear", "gemm_plan", "gate_up_silu", "interleave_gate_up",
+    "decode_workspace", "linear", "gemm_splits", "gemm_plan", "gate_up_silu", "interleave_gate_up",
     "quantize_fp8", "rmsnorm_fp8", "silu_quantize_fp8", "linear_fp8", "fp8_plan", "SplitK", "linear_tile", "tile_ok", "BLAS_CALLS",
     "linear_f32", "decoder",
 ]
@@ -367,6 +367,19 @@ def _measured_blas(M: int, N: int, K: int) -> bool:
         return False
     t = _gemm_table_get()
     return t.get(("skinny", M, N, K) if M <= SKINNY_MAX_M else (M, N, K)) == "blas"
+
+
+def gemm_splits(M: int, N: int, K: int) -> int:
+    """K slices (1, 2, 4 or 8) that bring gemm_decode's 64-column tiles to one block per CU, for callers that pass
+    ``linear`` their own ``splits``; its own plans are gemm_plan's."""
+    best = 1
+    for S in (1, 2, 4, 8):
+        if K % (64 * S):
+            break
+        best = S
+        if N // 64 * S >= CUS:
+            break
+    return best
 
 
 def gemm_plan(M: int, N: int, K: int, defer: bool = True):

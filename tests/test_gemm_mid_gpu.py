@@ -164,3 +164,9 @@ def test_few_rows_leave_gemm_skinny_where_it_was_measured_slower():
     for M, N, K, defer in ((17, 4096, 14336, True), (24, 3584, 3584, True), (32, 6144, 4096, False), (5, 128256, 3072, False),
                            (6, 128256, 8192, False), (5, 152064, 3584, False), (8, 128256, 4096, False), (16, 32768, 4096, False)):
         assert ops._mid_beats_skinny(M, N, K, defer), (M, N, K, defer)
+
+
+def test_gemm_splits_is_still_there():
+    from operator_amd.ops import gemm_splits
+
+    assert [gemm_splits(64, n, k) for n, k in ((4096, 14336), (4096, 192), (16384, 4096), (8192, 4096), (64, 8192))] == [4, 1, 1, 2, 8]
