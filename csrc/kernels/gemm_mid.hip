@@ -5,7 +5,8 @@
 // workgroups of an 885 x 4096 product, each walking the whole K at 1.3 us per 64 columns. Here a tile is 128 x 256
 // and its K may be cut into S slices (fp32 slabs, summed by the consumer or by a reduce pass), so that
 // M N S / 32768 workgroups come close to one per CU:
-//   885 rows (weights from HBM)   4096 x 14336: 297 -> 103 us, 4096 x 4096: 88 -> 36, 6144 x 4096: 89 -> 56
+//   885 rows (weights from HBM)   4096 x 14336: 297 -> 103 us, 4096 x 4096: 88 -> 36, 6144 x 4096: 89 -> 56 (within a prefill the
+//                                 first two take 155 together, the last 62)
 //   100 rows, the norm included   285 -> 58, 90 -> 25, 91 -> 38 (in the slices of 512 rows, see ops.mid_plan)
 //   vocabulary 128256 x 8192, 64 rows: 422 -> 373 us (5.6 TB/s of weights)
 // The first slice carries a bias (4608 x 3584, 300 rows: 54 us in one slice, 29 in 3).

@@ -317,7 +317,7 @@ int decode_advance(const int64_t* tok, int64_t* ids, int64_t* hist, int64_t* pos
 }
 
 // out[dst[r]] = fp32 of row r: a decode step's logits, in the caller's order. Bound by memory: one 2-byte read and
-// one 4-byte write per element (256 x 128256: 41 us against 125 for a conversion pass and an indexed copy).
+// one 4-byte write per element (256 x 128256: 32 us within a decode step, 6.2 TB/s, against 125 for a conversion pass and an indexed copy).
 template <typename T>
 __global__ void __launch_bounds__(256) scatter_rows_f32_kernel(const T* __restrict__ x, int64_t ld, const int* __restrict__ dst,
                                                                float* __restrict__ out, int n_out, int cols, bool vec) {

@@ -198,9 +198,6 @@ class MatchEngine:
         self._scorer = None
         self._score_tables = None
         self.stats = ScanStats()
-        # scan -> line index -> fixup -> per-doc newlines -> D2H as ONE captured hipGraph per
-        # (segment size, segment-count bucket, doc-count bucket): one launch and one sync
-        # per batch instead of ~10 launches and 3 syncs
         # the scan's text and doc layout stay on the GPU until the next scan: the context
         # windows of the reported events are located there (line_index.hip context_spans)
         self._resident: tuple | None = None

@@ -36,8 +36,9 @@ DECODE_ATTN_VARIANT = int(os.environ.get("OAMD_DECODE_ATTN_VARIANT", "0"))
 
 
 class SplitK:
-    """A decode GEMM's output left as S fp32 split-K slabs [S, M, N]; the consumer
-    (rmsnorm) sums them, so the GEMM's separate reduction pass disappears."""
+    """A product left as S fp32 split-K slabs [S, M, N], of a decode batch or of prompts of up to 4096 rows (a bias is in
+    the first slab); the consumer (a norm, rope_kv, a head or stream kernel, the fp8 SwiGLU) sums them, so the GEMM's
+    separate reduction pass disappears. ``linear(defer_reduce=True)`` returns one where it cuts K, else a tensor."""
 
     __slots__ = ("p", "S", "shape", "device", "dtype", "is_cuda")
 
@@ -363,7 +364,7 @@ LM_HEAD_MIN_N = 32768
 def _measured_blas(M: int, N: int, K: int) -> bool:
     """The tuned table measured hipBLASLt fastest for this decode-bucket shape (small-M
     GEMMs that neither the decode kernels nor the 256-row tile kernel win)."""
-    if N >= LM_HEAD_MIN_N:   # vocab projections always run on gemm_tile (weight-streaming bound there)
+    if N >= LM_HEAD_MIN_N:   # vocabulary projections never do (gemm_skinny, gemm_mid, gemm_decode or gemm_tile)
         return False
     t = _gemm_table_get()
     return t.get(("skinny", M, N, K) if M <= SKINNY_MAX_M else (M, N, K)) == "blas"
@@ -435,7 +436,9 @@ def _vocab_plan(M: int, N: int, K: int):
     """Decode-bucket vocabulary projection: one row tile of all rows against 128-column tiles, so that the weights
     are read once (256 rows of 32768 x 4096: 73 us, 102 on 64 columns; 128 rows 59 and 62). A 128256-row
     vocabulary at 256 rows is the tile kernel's (253 us against 289), one of 8192 columns too (64 rows 373 against
-    389, 256 rows 449 against 617); rows that are not one tile would read the weights again."""
+    389, 256 rows 449 against 617); rows that are not one tile would read the weights again. Both lines lie between sizes
+    that were timed: 32000 to 152064 rows of 2048 to 8192 columns, 64 to 256 rows, none of them slower than on 64 columns
+    (152064 x 3584: 64 rows 192 us against 223, 256 rows 306 against 430; profiles/plans_before_after.txt)."""
     if row_tile(M) != M or K >= 8192 or (M == 256 and N >= 2 * LM_HEAD_MIN_N) or N % 128:
         return None
     return (M, 128, 1, 3)
@@ -491,9 +494,10 @@ def _mid_few_rows(M: int, N: int, K: int, defer: bool) -> bool:
     return mid < (3 + 2e-6 * N * K / 5.4) * (1 + 0.04 * M)
 
 
-# Every GPU GEMM of the model runs on the hand-written gfx950 kernels: prefill projections (M > 256
-# rows) on gemm_tile's persistent p5 schedule (csrc/kernels/gemm_tile.hip), decode buckets on
-# gemm_pp / gemm_tn / gemm_skinny, the lm_head on gemm_tile, fp8 on gemm_fp8. hipBLASLt is reached
+# Every GPU GEMM of the model runs on the hand-written gfx950 kernels: prompts on gemm_mid up to some 4096 rows
+# (mid_plan) and on gemm_tile's persistent p5 schedule (csrc/kernels/gemm_tile.hip) beyond, decode buckets on
+# gemm_pp / gemm_tn / gemm_mid / gemm_skinny, the lm_head on whichever of them its rows call for (_mid_beats_skinny,
+# _vocab_plan, mid_plan), fp8 on gemm_fp8 and, past 64 rows, gemm_fp8_tile, fp32 on gemm_f32. hipBLASLt is reached
 # only by shapes none of them takes (K % 64 != 0, N % 16 != 0, non-bf16), counted in BLAS_CALLS.
 # OAMD_PREFILL_BLAS=1 routes the plain prefill projections (QKV, O, down) to hipBLASLt instead, for
 # A/B runs against the vendor library (profiles/gemm_tile_p5_vs_hipblaslt_r6.jsonl).
@@ -533,7 +537,8 @@ def tile_out_ok(out: torch.Tensor | None) -> bool:
 
 # Costs, in us, of the two bf16 tile kernels on one MI355X with weights that stream from HBM (measured on
 # 48 to 6144 rows of 2048 to 28672 x 2048 to 14336 weights): a step is one 64-column piece of K on every
-# busy CU, dearer with the whole chip busy (clock, L2) and where no two workgroups share a weight panel.
+# busy CU, dearer with the whole chip busy (clock, L2) and where no two workgroups share a weight panel. The plans are for
+# the whole card's CUs; on a part of one the kernels' grids adapt, and the plans cost speed only.
 CUS = 256
 
 
@@ -629,10 +634,12 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, glu: int = 0, prompt: bool = Fa
 def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, splits: int | None = None,
            partial: torch.Tensor | None = None, bn: int | None = None, bm: int | None = None,
            defer_reduce: bool = False, stages: int | None = None, bias: torch.Tensor | None = None, prompt: bool = False):
-    """y = x @ w^T (+ bias) in bf16 on the gfx950 kernels: M <= 32 decode buckets on the
-    weight-streaming gemm_skinny, M in {64, 128, 256} on the LDS-staged split-K
-    gemm_decode (tuned tables), everything else (prefill, the lm_head, biased
-    projections) on the 256x256-tile gemm_tile (persistent p5 past 256 rows). hipBLASLt only
+    """y = x @ w^T (+ bias) in bf16 on the gfx950 kernels: up to 32 rows on the weight-streaming gemm_skinny, or on
+    gemm_mid where the rows cost more than its tile (_mid_beats_skinny); 64, 128, 192 and 256 rows on the LDS-staged
+    split-K gemm_decode (the measured table, else _decode_tiles; vocabularies _vocab_plan) or where it is estimated
+    faster gemm_mid; everything else (prompts, the lm_head of many of them, biased projections) on gemm_mid's 128 x 256
+    tiles with K slices (mid_plan) or gemm_tile's 256 x 256 tiles (persistent p5 past 256 rows). ``defer_reduce``: K
+    slices come back as fp32 slabs (:class:`SplitK`). fp32 operands: linear_f32. hipBLASLt only
     for shapes none of them takes (K % 64 != 0, N % 16 != 0, non-bf16), for decode shapes the
     tuned table measured it fastest on, or under OAMD_PREFILL_BLAS=1 (A/B); CPU tensors on torch.
     ``prompt``: rows of prompts, which a prefill graph pads (mid_plan)."""
@@ -751,7 +758,8 @@ def _fp8_slices(M: int, N: int, K: int) -> tuple[int, int, int]:
     return bm, bn, S
 
 
-# us of a 128-K step of gemm_fp8's tiles, every CU busy (8192 x 28672, 57344 x 8192)
+# us of a 128-K step of gemm_fp8's tiles, every CU busy (8192 x 28672, 57344 x 8192; the plans they give were timed on eight
+# shapes of 4096 to 57344 features, 1 to 4000 rows: none slower than the former fixed tile, profiles/plans_before_after.txt)
 _FP8_STEP = {(64, 64): 0.40, (64, 128): 0.56, (128, 64): 0.51, (128, 128): 0.80, (256, 64): 0.71, (256, 128): 1.16}
 
 
