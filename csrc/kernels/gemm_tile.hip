@@ -538,11 +538,15 @@ __global__ void __launch_bounds__(256) gemm_tile256_h4_kernel(const bf16_t* __re
 //     tile's epilogue stores go out (no per-tile prologue fill, no workgroup relaunch);
 //   * two barriers and one counted vmcnt per K-step (the h4 loop had three and two):
 //       segment A: k-half 0 (64 MFMAs); the 16 fragment reads of k-half 1 ride on its first
-//         16 MFMAs; after 40 MFMAs lgkmcnt(0) + barrier (every wave is done with this buffer)
-//         and the 8 W pieces of step g + 2 go into it between the last 24;
-//       segment B: k-half 1 (64 MFMAs); the 8 X pieces of step g + 2 ride on its first 40;
-//         then vmcnt(16) + barrier (step g + 1 landed for every wave) and its k-half-0
-//         fragment reads ride on the last 24 MFMAs;
+//         16 MFMAs; after 40 MFMAs lgkmcnt(0) + barrier (every wave is done with this buffer);
+//       segment B: k-half 1 (64 MFMAs); after 40 of them step g + 1 has landed for every wave (counted
+//         vmcnt + barrier) and its k-half-0 fragment reads ride on the last 24;
+//     the 16 pieces of step g + 2 are spread over the MFMAs behind the first barrier, up to the next step's
+//     first rows: a CU's address unit takes about 20 clocks per KiB piece and a wave whose piece has to wait
+//     issues no MFMA meanwhile. Four waves with 16 pieces within 64 MFMAs (1024 clocks) asked for 1280; on
+//     104 (kWin 144: a later one left the last pieces too little time to land, 136 to 152 were equal)
+//     they fit. 28208 rows of 4096 x 14336: 2266 -> 2195 us (1.51 PFLOP/s), 2048 rows of 6144 x 4096 92 -> 82, 8192 rows
+//     of 4096 x 4096 193 -> 187, 28672 x 4096 with W three deep 4755 -> 4720;
 //   * 16-B output stores: the two W fragments of a 32-feature block take interleaved feature
 //     rows (fragment jj, row m -> feature 8 (m / 4) + 4 jj + m % 4), so the lane holding
 //     accumulator rows 4q .. 4q+3 of both has features 8q .. 8q+7 -- one dwordx4 store per
@@ -555,12 +559,10 @@ __global__ void __launch_bounds__(256) gemm_tile256_h4_kernel(const bf16_t* __re
 // DEEP: which operand streams through THREE LDS buffers (its pieces issued 3 K-steps ahead, two steps
 // of flight) -- 0: neither (2 + 2 buffers, 128 KiB), 1: X (narrow N: the X panels come from HBM,
 // W stays in the Infinity Cache), 2: W (wide N: the W panels come from HBM); 160 KiB of LDS.
-// OPT (A/B arms): bit 0 = s_setprio 1 over the MFMA streams; bit 1 = MFMA groups over W fragments
-// (srcA fixed for 8 MFMAs, as hipBLASLt's MT256x256x64 loop issues them)
 // GRP: routed experts. X's rows are expert segments padded to 256-row tiles (moe_sort): gtab[0] =
 // row tiles, gtab[1 + i] = expert of row tile i, W [experts][N][K]; rscale[row] multiplies both
 // SwiGLU operands (an expert reads its token scaled by the router weight).
-template <int EPI, int DEEP = 0, int OPT = 0, bool GRP = false>
+template <int EPI, int DEEP = 0, bool GRP = false>
 __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __restrict__ X,
                                                               const bf16_t* __restrict__ W, bf16_t* __restrict__ Y,
                                                               const bf16_t* __restrict__ bias, int M, int N, int K,
@@ -569,6 +571,7 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
                                                               const float* __restrict__ rscale = nullptr, GluAct act = {}) {
   constexpr int AUX = 16;
   constexpr int kHalf = 32768;   // one operand of a K-step: 256 rows x 128 B
+  constexpr int kWin = DEEP ? 128 : 144;   // a step's pieces go out between its MFMA 40 and this one (past 127: of the next step)
   __shared__ __attribute__((aligned(1024))) char lds[DEEP ? 5 * kHalf : 4 * kHalf];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -681,68 +684,52 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
     for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[i][j]));
   asm volatile("s_nop 4");
   u16x8 xa[8], wa[8], xb[8], wb[8];
-  constexpr bool kCols = (OPT & 2) != 0;
-  // one MFMA row: 8 MFMAs sharing fragment `u` of the per-row set (X fragment i = u, or with
-  // kCols W fragment j = u), op(v) after MFMA v
+  // one MFMA row: 8 MFMAs sharing X fragment u, op(v) after MFMA v
   auto row = [&](const u16x8 (&xf)[8], const u16x8 (&wf)[8], int u, auto op) {
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
-      if constexpr (kCols) mfma_tied(acc[v][u], wf[u], xf[v]);
-      else mfma_tied(acc[u][v], wf[v], xf[u]);
+      mfma_tied(acc[u][v], wf[v], xf[u]);
       __builtin_amdgcn_sched_barrier(0);
       op(v);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // fragment reads in row order: the set every row needs (W, or X with kCols) first
-  auto rd_all = [&](int ox, int ow, int h, u16x8 (&xf)[8], u16x8 (&wf)[8], int v) {
-    if constexpr (kCols) rdx(ox, h, xf, v);
-    else rdw(ow, h, wf, v);
-  };
-  auto rd_row = [&](int ox, int ow, int h, u16x8 (&xf)[8], u16x8 (&wf)[8], int u) {
-    if constexpr (kCols) rdw(ow, h, wf, u);
-    else rdx(ox, h, xf, u);
-  };
-  auto none = [](int) {};
-
-  // prologue. DEEP == 0: steps 0 and 1 of both operands (W, X per step). DEEP != 0: shallow 0,
-  // deep 0, shallow 1, deep 1, deep 2 -- the order the loop keeps (shallow g+2, deep g+3 per step),
-  // so "step g+1 landed" is always "all but the 16 / 24 youngest pieces"
-  if constexpr (DEEP == 0) {
-#pragma unroll
-    for (int st = 0; st < 2; ++st) {
-#pragma unroll
-      for (int q = 0; q < 8; ++q) dma(cw, woff(st, 0), q);
-#pragma unroll
-      for (int q = 0; q < 8; ++q) dma(cx, xoff(st, 0), q);
+  // what goes out z MFMAs behind the barrier that frees the buffers at ox, ow: piece p of 16, if its turn is z.
+  // DEEP == 0: W, then X of step g + 2; DEEP != 0: the shallow operand of step g + 2, the deep one of step g + 3
+  auto piece = [&](int z, int ox, int ow) {
+    constexpr int n = kWin - 40;
+    const int p = (z * 16 + n - 1) / n;
+    if (p >= 16 || p * n / 16 != z) return;
+    if ((DEEP == 2) == (p < 8)) dma(cx, ox, p & 7);
+    else dma(cw, ow, p & 7);
+    if (p == 15) {
       advance(cx, true);
       advance(cw, false);
     }
-    vm_wait<16>();
-  } else {
-    Cur& cs = DEEP == 1 ? cw : cx;   // shallow operand
-    Cur& cd = DEEP == 1 ? cx : cw;   // deep operand
-    auto soff = [&](int st) { return DEEP == 1 ? woff(st & 1, st % 3) : xoff(st & 1, st % 3); };
-    auto doff = [&](int st) { return DEEP == 1 ? xoff(st & 1, st % 3) : woff(st & 1, st % 3); };
+  };
+  constexpr auto kPieces = [](int z) { return (z * 16 + kWin - 41) / (kWin - 40) < 16 ? (z * 16 + kWin - 41) / (kWin - 40) : 16; };   // gone out before z
+
+  // prologue: the pieces in the loop's order. The deep operand's step 0, the pieces of a step -2, then as many of
+  // step -1's as a step sends before its end; the rest ride on step 0
+  if constexpr (DEEP != 0) {
+    Cur& cd = DEEP == 1 ? cx : cw;
 #pragma unroll
-    for (int st = 0; st < 2; ++st) {
-#pragma unroll
-      for (int q = 0; q < 8; ++q) dma(cs, soff(st), q);
-      advance(cs, DEEP == 2);
-#pragma unroll
-      for (int q = 0; q < 8; ++q) dma(cd, doff(st), q);
-      advance(cd, DEEP == 1);
-    }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) dma(cd, doff(2), q);
+    for (int q = 0; q < 8; ++q) dma(cd, DEEP == 1 ? xoff(0, 0) : woff(0, 0), q);
     advance(cd, DEEP == 1);
-    vm_wait<24>();
   }
+  constexpr int kAhead = DEEP ? 1 : 0;   // steps the deep operand is ahead
+#pragma unroll
+  for (int z = 0; z < kWin - 40; ++z)
+    piece(z, DEEP == 1 ? xoff(1, 1) : xoff(0, 0), DEEP == 2 ? woff(1, 1) : woff(0, 0));
+  int pox = DEEP == 1 ? xoff(0, 2) : xoff(1, 1), pow = DEEP == 2 ? woff(0, 2) : woff(1, 1);   // buffers of the pieces still to come
+#pragma unroll
+  for (int z = 0; z < 88; ++z) piece(z, pox, pow);
+  vm_wait<kPieces(88) + 8 * kAhead>();   // step 0
   seg_barrier();
 #pragma unroll
-  for (int v = 0; v < 8; ++v) rd_all(xoff(0, 0), woff(0, 0), 0, xa, wa, v);
+  for (int v = 0; v < 8; ++v) rdw(woff(0, 0), 0, wa, v);
 #pragma unroll
-  for (int u = 0; u < 8; ++u) rd_row(xoff(0, 0), woff(0, 0), 0, xa, wa, u);
+  for (int u = 0; u < 8; ++u) rdx(xoff(0, 0), 0, xa, u);
 
   int g = 0, p3 = 0;   // flattened step counter (buffer parity) and g % 3
   int m0 = 0, n0 = 0;
@@ -752,69 +739,53 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
       const int ox = xoff(p2, p3), ow = woff(p2, p3);          // this step's buffers
       const int nox = xoff(n2, n3), now_ = woff(n2, n3);       // step g + 1's
       // ---- segment A: k-half 0 from A; k-half 1 reads (row 0, row 1); this step's buffers released
-      if constexpr (OPT & 1) __builtin_amdgcn_s_setprio(1);
-      asm volatile("s_waitcnt lgkmcnt(7)" ::: "memory");   // the 8 shared + row 0's fragment
+      asm volatile("s_waitcnt lgkmcnt(7)" ::: "memory");   // the W fragments + row 0's
       __builtin_amdgcn_sched_barrier(0);
-      row(xa, wa, 0, [&](int v) { rd_all(ox, ow, 1, xb, wb, v); });
+      row(xa, wa, 0, [&](int v) {
+        rdw(ow, 1, wb, v);
+        piece(88 + v, pox, pow);
+      });
       asm volatile("s_waitcnt lgkmcnt(14)" ::: "memory");  // + row 1's
       __builtin_amdgcn_sched_barrier(0);
-      row(xa, wa, 1, [&](int v) { rd_row(ox, ow, 1, xb, wb, v); });
+      row(xa, wa, 1, [&](int v) {
+        rdx(ox, 1, xb, v);
+        piece(96 + v, pox, pow);
+      });
       asm volatile("s_waitcnt lgkmcnt(15)" ::: "memory");  // every k-half-0 read of the step
       __builtin_amdgcn_sched_barrier(0);
-      row(xa, wa, 2, none);
-      row(xa, wa, 3, none);
-      row(xa, wa, 4, none);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      if constexpr (OPT & 1) __builtin_amdgcn_s_setprio(0);
-      seg_barrier();   // every wave is done reading this step's buffers
-      if constexpr (OPT & 1) __builtin_amdgcn_s_setprio(1);
-      // DEEP == 0: W of step g+2 here, X of step g+2 in segment B (both into this step's buffers);
-      // DEEP != 0: the shallow operand of step g+2 here, the deep one of step g+3 in segment B
 #pragma unroll
-      for (int i = 5; i < 8; ++i)
-        row(xa, wa, i, [&](int j) {
-          const int m = (i - 5) * 8 + j;
-          if (m % 3 == 0) {
-            if constexpr (DEEP == 1) dma(cw, ow, m / 3);
-            else if constexpr (DEEP == 2) dma(cx, ox, m / 3);
-            else dma(cw, ow, m / 3);
-          }
-        });
+      for (int i = 2; i < 5; ++i) row(xa, wa, i, [](int) {});
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      seg_barrier();   // every wave is done reading this step's buffers
+#pragma unroll
+      for (int i = 5; i < 8; ++i) row(xa, wa, i, [&](int v) { piece((i - 5) * 8 + v, ox, ow); });
       // ---- segment B: k-half 1 from B; then step g + 1 lands
 #pragma unroll
-      for (int i = 0; i < 5; ++i)
-        row(xb, wb, i, [&](int j) {
-          const int m = i * 8 + j;
-          if (m % 5 == 0) {
-            if constexpr (DEEP == 1) dma(cx, ox, m / 5);
-            else if constexpr (DEEP == 2) dma(cw, ow, m / 5);
-            else dma(cx, ox, m / 5);
-          }
-        });
-      advance(cx, true);
-      advance(cw, false);
-      if constexpr (DEEP == 0) vm_wait<16>();   // this wave's pieces of step g + 1
-      else vm_wait<24>();
-      if constexpr (OPT & 1) __builtin_amdgcn_s_setprio(0);
+      for (int i = 0; i < 5; ++i) row(xb, wb, i, [&](int v) { piece(24 + i * 8 + v, ox, ow); });
+      vm_wait<kPieces(64) + 8 * kAhead>();   // this wave's pieces of step g + 1
       seg_barrier();   // ... every wave's
-      if constexpr (OPT & 1) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
       for (int i = 5; i < 8; ++i)
-        row(xb, wb, i, [&](int j) {
-          const int m = (i - 5) * 8 + j;   // 16 reads on 24 MFMAs: the shared 8, then the per-row 8
+        row(xb, wb, i, [&](int v) {
+          const int m = (i - 5) * 8 + v;   // 16 reads on 24 MFMAs: W's 8, then X's
           if (m % 3 != 2) {
-            const int k = m - m / 3;
-            if (k < 8) rd_all(nox, now_, 0, xa, wa, k);
-            else rd_row(nox, now_, 0, xa, wa, k - 8);
+            const int f = m - m / 3;
+            if (f < 8) rdw(now_, 0, wa, f);
+            else rdx(nox, 0, xa, f - 8);
           }
+          piece(64 + m, ox, ow);
         });
+      pox = ox;
+      pow = ow;
       p3 = n3;
     }
-    if constexpr (OPT & 1) __builtin_amdgcn_s_setprio(0);
 
     // ---- epilogue of the tile (the next tile's step 0 is in registers / flight); lane holds
     // features 8 lq .. 8 lq + 7 of each 32-feature block (fragments jj = 0, 1) of token l15
     asm volatile("s_nop 7\n s_nop 7\n s_nop 7" ::: "memory");
+    int le;   // the lane once more: kept over the K loop it would be spilled, and its reload waits for every piece in flight
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n v_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(le));
+    const int l15 = le & 15, lq = le >> 4;
     f32x4 bv[2][2][2];   // bias of this lane's features per (f, type, jj): independent of the token block
     if constexpr (EPI == kEpiBias) {
 #pragma unroll
@@ -950,9 +921,9 @@ int moe_gemm_tile(const bf16_t* X, const bf16_t* W, bf16_t* Y, int max_rows, int
   if (silu_gu && (N % 128 != 0 || rscale == nullptr)) return -2;
   const int grid = min((max_rows / kT) * ((N + kT - 1) / kT), device_cus());
   if (silu_gu)
-    gemm_tile256_p5_kernel<kEpiSilu, 0, 0, true><<<grid, 256, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, N / 2, 4, gtab, rscale);
+    gemm_tile256_p5_kernel<kEpiSilu, 0, true><<<grid, 256, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, N / 2, 4, gtab, rscale);
   else
-    gemm_tile256_p5_kernel<kEpiStore, 0, 0, true><<<grid, 256, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, N, 4, gtab, rscale);
+    gemm_tile256_p5_kernel<kEpiStore, 0, true><<<grid, 256, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, N, 4, gtab, rscale);
   OAMD_LAUNCH_CHECK();
   return 0;
 }
