@@ -572,7 +572,10 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
   constexpr int AUX = 16;
   constexpr int kHalf = 32768;   // one operand of a K-step: 256 rows x 128 B
   constexpr int kWin = DEEP ? 128 : 144;   // a step's pieces go out between its MFMA 40 and this one (past 127: of the next step)
-  __shared__ __attribute__((aligned(1024))) char lds[DEEP ? 5 * kHalf : 4 * kHalf];
+  constexpr bool kScale = GRP && EPI == kEpiSilu;
+  constexpr int kRs = DEEP ? 5 * kHalf : 4 * kHalf;   // kScale: behind the buffers the scales of each wave's 128 rows
+  static_assert(!kScale || DEEP == 0, "no room for the scales");
+  __shared__ __attribute__((aligned(1024))) char lds[kRs + (kScale ? 4 * 512 : 0)];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = w >> 1, wn = w & 1;
@@ -734,6 +737,14 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
   int g = 0, p3 = 0;   // flattened step counter (buffer parity) and g % 3
   int m0 = 0, n0 = 0;
   for (int r = 0; tile_rc(r, m0, n0); ++r) {
+    if constexpr (kScale) {
+      // landed by the first step's count; read in the epilogue as plain loads they would wait for every piece in
+      // flight, eight times a tile (M is whole tiles)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        __builtin_amdgcn_global_load_lds(rscale + m0 + wm * 128 + h * 64 + lane,
+                                         (__attribute__((address_space(3))) void*)(lds + kRs + w * 512 + h * 256), 4, 0, 0);
+    }
     for (int t = 0; t < T; ++t, ++g) {
       const int p2 = g & 1, n2 = p2 ^ 1, n3 = p3 == 2 ? 0 : p3 + 1;
       const int ox = xoff(p2, p3), ow = woff(p2, p3);          // this step's buffers
@@ -810,7 +821,7 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
       const int tok = m0 + wm * 128 + i * 16 + l15;
       bf16_t* yrow = Y + (int64_t)tok * ldy;
       float rsc = 1.f;
-      if constexpr (GRP && EPI == kEpiSilu) rsc = rscale[min(tok, M - 1)];
+      if constexpr (kScale) rsc = *reinterpret_cast<const float*>(lds + kRs + w * 512 + (i * 16 + l15) * 4);
 #pragma unroll
       for (int f = 0; f < 2; ++f) {
         if constexpr (EPI == kEpiSilu) {
@@ -818,7 +829,7 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
 #pragma unroll
           for (int jj = 0; jj < 2; ++jj) {
             f32x4 gt = acc[i][f * 4 + jj], up = acc[i][f * 4 + 2 + jj];
-            if constexpr (GRP) {
+            if constexpr (kScale) {
               gt *= rsc;
               up *= rsc;
             }
