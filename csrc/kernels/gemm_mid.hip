@@ -2,24 +2,25 @@
 // projections of one or a few prompts, and vocabularies of up to 128 rows.
 //
 // What bounds it: not the matrix cores but the CUs a launch keeps busy. The 256 x 256 tiles of gemm_tile make 64
-// workgroups of an 885 x 4096 product, each walking the whole K at 1.3 us per 64 columns. Here a tile is 128 x 256
-// and its K may be cut into S slices (fp32 slabs, summed by the consumer or by a reduce pass), so that
-// M N S / 32768 workgroups come close to one per CU:
-//   885 rows (weights from HBM)   4096 x 14336: 297 -> 103 us, 4096 x 4096: 88 -> 36, 6144 x 4096: 89 -> 56 (within a prefill the
-//                                 first two take 155 together, the last 62)
-//   100 rows, the norm included   285 -> 58, 90 -> 25, 91 -> 38 (in the slices of 512 rows, see ops.mid_plan)
-//   vocabulary 128256 x 8192, 64 rows: 422 -> 373 us (5.6 TB/s of weights)
-// The first slice carries a bias (4608 x 3584, 300 rows: 54 us in one slice, 29 in 3).
-// A 128 x 256 step is 0.7 us (0.43 of MFMA at 2.4 GHz): a CU takes in 50 to 75 bytes per ns through LDS-DMA however
-// many stages wait (a fourth stage of a 64-row tile gained nothing). With every CU busy for several rounds it is
-// 0.85 us, 1.2 PFLOP/s against 1.45 of the 256-row tiles, so those keep the large products (ops.mid_plan).
+// workgroups of an 885 x 4096 product, each walking the whole K at 1.2 us per 64 columns. Here a tile is 96, 128 or 160 rows
+// (ops.tile_rows) by 256 columns and its K may be cut into S slices (fp32 slabs, summed by the consumer or by a reduce pass),
+// so that the workgroups come close to one per CU or to whole rounds of them:
+//   885 rows (weights from HBM)   6144 x 4096, 96-row tiles: 49 us (128-row tiles 55); 4096 x 4096 in 2 slices 35; 4096 x 14336 in 2
+//                                 101 (297 on the 256-row tiles)
+//   300 rows                      28672 x 4096, 160-row tiles: 68 us (128 rows 110, 256 rows 95)
+//   1500 rows                     6144 x 4096, 160-row tiles: 62 us (128 rows 93, 256 rows 90)
+//   vocabulary 128256 x 8192, 64 rows: 373 us (5.6 TB/s of weights; the 256-row tiles 422)
+// The first slice carries a bias (4608 x 3584, 300 rows: 54 us in one slice, 22 in 3).
+// A 128 x 256 step takes 0.63 us alone, 0.79 with every CU busy (clock). Its MFMAs are 0.47, its LDS-DMA pieces by themselves 0.45 (a CU's
+// address unit takes about 20 clocks per KiB piece), its fragment reads 0.23. A wave whose piece has to wait issues no MFMA, so
+// the pieces are spread over the whole step: within the 24 MFMAs behind the barrier, as before, 885 rows of 6144 x 4096 took 60 us
+// and not 55, of 4096 x 4096 38 and not 35. A 64-row tile's step is no shorter than a 96-row one's (0.61, 0.65: the weight pieces).
 //
-// Why this shape: four waves, one per SIMD, 64 x 128 outputs each in 128 AGPRs, so a step's fragment reads (96 KiB)
-// stay below its MFMA time; three 48 KiB stages leave two steps in flight behind one barrier per step; each stage is
-// refilled as soon as its k-half 1 is in registers. 128-B rows with the chunk swizzle slot ^ (bit1(row) << 1 |
-// bit3(row) << 2) read without bank conflicts; W fragments take interleaved feature rows, so a lane ends with 8
-// neighbouring features: 16-B stores. A workgroup walks its units (tile, slice) in one continuous LDS-DMA stream:
-// the next unit's first stages load while this one's outputs are stored.
+// Why this shape: four waves, one per SIMD, 16 MI x 128 outputs each in AGPRs, so a step's fragment reads stay below its
+// MFMA time; three stages (44, 48 or 52 KiB) leave one to two steps in flight behind one barrier per step. 128-B rows with the
+// chunk swizzle slot ^ (bit1(row) << 1 | bit3(row) << 2) read without bank conflicts; W fragments take interleaved feature
+// rows, so a lane ends with 8 neighbouring features: 16-B stores. A workgroup walks its units (tile, slice) in one
+// continuous LDS-DMA stream: the next unit's first stages load while this one's outputs are stored.
 #include "common.h"
 #include "kernels.h"
 
@@ -27,9 +28,8 @@ namespace oamd {
 
 namespace {
 
-constexpr int kBM = 128, kBN = 256;   // tile rows, columns
+constexpr int kBN = 256;     // tile columns
 constexpr int kBK = 64;      // K per step: one 128-B line per row
-constexpr int kGroupM = 8;   // row tiles that share a W panel before the next one
 
 enum { kEpiStore = 0, kEpiBias = 1, kEpiGlu = 2, kEpiPartial = 3 };   // partial: fp32 slab [M][N] of a K slice
 
@@ -66,14 +66,16 @@ __device__ __forceinline__ void store8(bf16_t* y, const f32x4& v0, const f32x4& 
 
 }  // namespace
 
-template <int EPI>
+// MI: 32-row blocks of a tile
+template <int MI, int EPI>
 __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                        bf16_t* __restrict__ Y, const bf16_t* __restrict__ bias,
                                                        float* __restrict__ P, int M, int N, int K, int ldy, int S, GluAct act) {
   constexpr int AUX = 16;
-  constexpr int MI = kBM / 32;                   // X fragments of a wave = its X pieces per step
+  constexpr int kBM = 32 * MI;                   // a wave has MI X fragments and as many X pieces per step
   constexpr int NP = MI + 8;                     // LDS-DMA pieces of a wave per step
   constexpr int NS = 3;                          // stages: 144 KiB
+  constexpr int kGroupM = 32 / MI;               // row tiles that share a W panel before the next one
   constexpr int kX = kBM * 128, kStage = kX + kBN * 128;
   __shared__ __attribute__((aligned(1024))) char lds[NS * kStage];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -126,10 +128,10 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
     __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)cp, (short)0, cn, 0x00020000),
                                              (__attribute__((address_space(3))) void*)dst, 16, (int)vo[q], step * (kBK * 2), 0, AUX);
   };
-  // piece p of the cursor's step into stage `off`: W first (it comes from further away)
+  // piece p of the cursor's step into stage `off`
   auto dma = [&](int off, int p) {
-    if (p < 8) dma_(cwp, cwn, ck, off + kX, p);
-    else dma_(cxp, cxn, ck, off, p - 8);
+    if (p < MI) dma_(cxp, cxn, ck, off, p);
+    else dma_(cwp, cwn, ck, off + kX, p - MI);
   };
 
   const int l15 = lane & 15, lq = lane >> 4;
@@ -160,21 +162,34 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
   };
   clear();
 
+  // A barrier inside every step (after kBar of k-half 1's kH MFMAs) says that the step's stage has been read and the
+  // next one has landed. The NP pieces of the step NS ahead go into that stage, spread over the 2 kH MFMAs up to
+  // the next barrier: piece p with MFMA number p * 2 kH / NP behind it.
+  constexpr int kH = 8 * MI, kBar = 2 * MI, kTail = kH - kBar;
+  auto piece = [&](int z, int o) {
+    const int p = (z * NP + 2 * kH - 1) / (2 * kH);
+    if (p < NP && p * 2 * kH / NP == z) {
+      dma(o, p);
+      if (p == NP - 1) advance();
+    }
+  };
   point(slot);
 #pragma unroll
-  for (int st = 0; st < NS; ++st) {
+  for (int st = 0; st < NS - 1; ++st) {
 #pragma unroll
     for (int p = 0; p < NP; ++p) dma(st * kStage, p);
     advance();
   }
-  vm_wait<(NS - 1) * NP>();
+#pragma unroll
+  for (int z = 0; z < kTail; ++z) piece(z, (NS - 1) * kStage);   // of the last stage, what k-half 1 of a step before would issue
+  vm_wait<NP>();
   __builtin_amdgcn_s_barrier();
   u16x8 xa[MI], wa[8], xb[MI], wb[8];
 #pragma unroll
   for (int f = 0; f < NP; ++f) rd(0, 0, xa, wa, f);
 
-  int off = 0;       // this step's stage
-  int relax = 0;     // steps whose wait may leave a whole tile's stores in flight behind the pieces
+  int off = 0, prev = (NS - 1) * kStage;   // this step's stage, the one before
+  bool relax = false;   // the next wait may leave a whole tile's stores in flight behind the pieces
   constexpr int kStores = MI * (EPI == kEpiGlu ? 2 : EPI == kEpiPartial ? 8 : 4);
   for (int u = slot; u < units; u += G) {
     int m0, n0, kz, t0, T;
@@ -183,23 +198,23 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
       const int nxt = off + kStage == NS * kStage ? 0 : off + kStage;
       // k-half 0; the reads of k-half 1 ride on its first MFMAs
 #pragma unroll
-      for (int v = 0; v < 8 * MI; ++v) {
+      for (int v = 0; v < kH; ++v) {
         mfma_tied(acc[v % MI][v / MI], wa[v / MI], xa[v % MI]);
         __builtin_amdgcn_sched_barrier(0);
         if (v < NP) rd(off, 1, xb, wb, v);
+        piece(kTail + v, prev);
         __builtin_amdgcn_sched_barrier(0);
       }
-      // k-half 1: after its first quarter every wave has read this stage and the next step has landed;
-      // then the step NS ahead goes into this stage and the next step's first reads ride along
+      // k-half 1; behind the barrier the next step's first reads ride along
 #pragma unroll
-      for (int v = 0; v < 8 * MI; ++v) {
-        if (v == 2 * MI) {
+      for (int v = 0; v < kH; ++v) {
+        if (v == kBar) {
           asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-          if (relax > 0) {
-            vm_wait<(NS - 2) * NP + kStores>();
-            --relax;
+          if (relax) {
+            vm_wait<NP + kStores>();
+            relax = false;
           } else {
-            vm_wait<(NS - 2) * NP>();
+            vm_wait<NP>();
           }
           __builtin_amdgcn_sched_barrier(0);
           __builtin_amdgcn_s_barrier();
@@ -207,14 +222,16 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
         }
         mfma_tied(acc[v % MI][v / MI], wb[v / MI], xb[v % MI]);
         __builtin_amdgcn_sched_barrier(0);
-        if (v >= 2 * MI) {
-          const int q = v - 2 * MI;
-          if (q & 1) dma(off, q >> 1);   // 24 slots: 12 reads, 12 pieces
-          else rd(nxt, 0, xa, wa, q >> 1);
+        if (v < kBar) {
+          piece(kTail + kH + v, prev);
+        } else {
+          const int z = v - kBar, f = (z * NP + kTail - 1) / kTail;
+          if (f < NP && f * kTail / NP == z) rd(nxt, 0, xa, wa, f);
+          piece(z, off);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
-      advance();
+      prev = off;
       off = nxt;
     }
 
@@ -251,26 +268,35 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
       }
     }
     // a whole tile issued kStores stores: the next waits count past them
-    relax = m0 + kBM <= M && n0 + kBN <= N ? NS - 1 : 0;
+    relax = m0 + kBM <= M && n0 + kBN <= N;
     clear();
   }
   vm_wait<0>();   // the trailing re-loads land before the workgroup's LDS is released
 }
 
+template <int MI>
+static void launch_mid(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, float* P, int M, int N, int K, int ldy,
+                       int glu, int S, int grid, hipStream_t stream) {
+  if (S > 1) gemm_mid_kernel<MI, kEpiPartial><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, GluAct{});
+  else if (glu) gemm_mid_kernel<MI, kEpiGlu><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, glu_act(glu));
+  else if (bias) gemm_mid_kernel<MI, kEpiBias><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, GluAct{});
+  else gemm_mid_kernel<MI, kEpiStore><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, GluAct{});
+}
+
 int gemm_mid(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, float* P, int M, int N, int K, int ldy, int glu,
-             int S, hipStream_t stream) {
+             int S, int rows, hipStream_t stream) {
   if (M < 1 || N < 16 || N % 16 || K % kBK || S < 1 || S > 16 || K / kBK < S) return -1;
   if (glu && (N % 128 || bias)) return -2;
   if (S > 1 && P == nullptr) return -3;
   if (Y == nullptr ? (S == 1 || glu) : (ldy % 8 || reinterpret_cast<uintptr_t>(Y) % 16)) return -4;
   if (S > 1 && Y != nullptr && ldy != (glu ? N / 2 : N)) return -5;
-  const int64_t units = (int64_t)((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN) * S;
+  if (rows != 96 && rows != 128 && rows != 160) return -7;
+  const int64_t units = (int64_t)((M + rows - 1) / rows) * ((N + kBN - 1) / kBN) * S;
   if (units > (1LL << 30)) return -6;
   const int grid = (int)min((int64_t)device_cus(), units);
-  if (S > 1) gemm_mid_kernel<kEpiPartial><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, GluAct{});
-  else if (glu) gemm_mid_kernel<kEpiGlu><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, glu_act(glu));
-  else if (bias) gemm_mid_kernel<kEpiBias><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, GluAct{});
-  else gemm_mid_kernel<kEpiStore><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, GluAct{});
+  if (rows == 96) launch_mid<3>(X, W, Y, bias, P, M, N, K, ldy, glu, S, grid, stream);
+  else if (rows == 128) launch_mid<4>(X, W, Y, bias, P, M, N, K, ldy, glu, S, grid, stream);
+  else launch_mid<5>(X, W, Y, bias, P, M, N, K, ldy, glu, S, grid, stream);
   OAMD_LAUNCH_CHECK();
   if (S == 1 || Y == nullptr) return 0;
   return glu ? splitk_silu(P, Y, M, N, S, glu, stream) : splitk_reduce(P, Y, (int64_t)M * N, S, stream);

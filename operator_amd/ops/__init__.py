@@ -582,26 +582,55 @@ def mid_plan(M: int, N: int, K: int, defer: bool, slices: bool = True, prompt: b
     return S if cost < _tile_cost(M, N, K) else None
 
 
+# us of a 64-column piece of K on a CU, and what it takes more with every CU busy (power, L2): gemm_mid's tiles of 96, 128
+# and 160 rows, gemm_tile's of 256 (fitted to those products)
+_ROW_STEP = {96: (0.53, 0.16), 128: (0.58, 0.20), 160: (0.70, 0.20), 256: (1.00, 0.38)}
+
+
+def _rows_us(rows: int, M: int, N: int, K: int, S: int) -> float:
+    units = -(-M // rows) * -(-N // 256) * S
+    full, last = divmod(units, CUS)
+    one, busy = _ROW_STEP[rows]
+    rounds = full * (one + busy) + (one + busy * last / CUS if last else 0)
+    return -(-(K // 64) // S) * rounds + 5 + 3 * (units - 1) // CUS   # a tile's stores between rounds
+
+
+@functools.lru_cache(maxsize=4096)
+def tile_rows(M: int, N: int, K: int, S: int = 1) -> int:
+    """Rows of the tiles (256 columns wide) of a prompt's product in S slices of K: 96, 128 or 160 (gemm_mid) or, in one
+    slice, 256 (gemm_tile). All sum a K slice in the same order, so the bits are the same and the rows are free: those whose
+    rounds of one workgroup per CU take least. Fewer rows fill the CUs (885 rows of 6144 x 4096: 168 tiles of
+    128 rows 55 us, 240 of 96 49), more rows save a round (300 rows of 28672 x 4096: 336 tiles of 128 rows 110 us, 224 of 160 68,
+    224 of 256 95; 1500 rows of 6144 x 4096: 93, 62 and 90) and per product take in fewer bytes (4096 rows of 4096 x
+    14336: 362, 421 and 317). Over 159 products of 16 shapes, 129 to 8000 rows, the estimate's choices take 0.1 % more than
+    the best ones and 5 % less than 128 or 256 rows by the slices' plan alone. Up to 128 rows are one tile."""
+    if M <= 128:
+        return 128
+    return min((_rows_us(r, M, N, K, S), r) for r in ((96, 128, 160) if S > 1 else _ROW_STEP))[1]
+
+
 def linear_tile(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None,
                 bias: torch.Tensor | None = None, glu: int = 0, defer_reduce: bool = False, prompt: bool = False):
     """Prefill / lm_head GEMM on the compute-bound gfx950 tile kernels (fused bias or gated (``glu``: SILU /
-    GELU_TANH) epilogue): 128 x 256 tiles with K slices for few rows (``mid_plan``), else 256 x 256 tiles (LDS-DMA
-    ping-pong pipeline). ``defer_reduce``: K slices come back as fp32 slabs (:class:`SplitK`);
-    ``prompt``: rows a prefill graph may pad."""
+    GELU_TANH) epilogue): tiles of 96 to 256 rows (``tile_rows``), for few rows with K slices (``mid_plan``).
+    ``defer_reduce``: K slices come back as fp32 slabs (:class:`SplitK`); ``prompt``: rows a prefill graph may pad."""
     M, K = x.shape
     N = w.shape[0]
     defer = defer_reduce and out is None and not glu
-    S = None
+    S, rows = None, 256
     if (out is None or (out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0)) and (
             bias is None or (bias.is_contiguous() and bias.data_ptr() % 16 == 0)):   # gemm_mid's 16-B accesses
         S = mid_plan(M, N, K, defer, out is None or out.stride(0) == out.shape[1], prompt)   # the reduce pass has no row stride
+        if S is not None or (N < LM_HEAD_MIN_N and K >= 128):
+            rows = tile_rows(M, N, K, S or 1)
     part = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if S is not None and S > 1 else None
+    opt = {} if rows == 128 else {"rows": rows}
     if part is not None and defer:
-        kernels().gemm_mid(x, w, None, bias, part, S)
+        kernels().gemm_mid(x, w, None, bias, part, S, **opt)
         return SplitK(part, S, M, N)
     y = out if out is not None else torch.empty(M, N // 2 if glu else N, dtype=x.dtype, device=x.device)
-    if S is not None:
-        kernels().gemm_mid(x, w, y, bias, part, S, glu)
+    if rows < 256:
+        kernels().gemm_mid(x, w, y, bias, part, S or 1, glu, **opt)
     else:
         kernels().gemm_tile(x, w, y, bias, glu)
     return y
