@@ -409,13 +409,13 @@ __global__ void __launch_bounds__(256, (NT == 1 && G <= 4) ? 3 : 2)
       }
     }
     load_k(r, nc, tile_lds);
-    const float alpha = exp2f(m_run - m_new);
+    const float alpha = exp2_weight(m_run - m_new);
     float psum = 0.f;
 #pragma unroll
     for (int i = 0; i < NT; ++i)
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
-        const float p = exp2f(sc[i][rr] - m_new);
+        const float p = exp2_weight(sc[i][rr] - m_new);
         psum += p;
         if (l15 < G) pwv[(16 * i + 4 * lg + rr) * GP + l15] = p;
       }
@@ -471,7 +471,7 @@ __global__ void __launch_bounds__(256, (NT == 1 && G <= 4) ? 3 : 2)
     float M = m_run;   // lane (head l15, group lg)
     M = fmaxf(M, __shfl_xor(M, 16, kWave));
     M = fmaxf(M, __shfl_xor(M, 32, kWave));
-    const float f = exp2f(m_run - M);
+    const float f = exp2_weight(m_run - M);
     float L = l_run * f;
     L += __shfl_xor(L, 16, kWave);
     L += __shfl_xor(L, 32, kWave);
@@ -518,7 +518,7 @@ __global__ void __launch_bounds__(256, (NT == 1 && G <= 4) ? 3 : 2)
     float o = 0.f, L = 0.f;
 #pragma unroll
     for (int ww = 0; ww < 4; ++ww) {
-      const float f = exp2f(mls[ww][h][0] - M);
+      const float f = exp2_weight(mls[ww][h][0] - M);
       o += f * red[ww][h][d];
       L += f * mls[ww][h][1];
     }
@@ -553,7 +553,7 @@ __global__ void attn_decode_combine_kernel(const float* __restrict__ o_part, con
   for (int s = 0; s < ns; ++s) M = fmaxf(M, ml[2 * s]);
   float L = 0.f, o = 0.f;
   for (int s = 0; s < ns; ++s) {
-    const float wgt = exp2f(ml[2 * s] - M);
+    const float wgt = exp2_weight(ml[2 * s] - M);
     L += wgt * ml[2 * s + 1];
     o += wgt * o_part[((int64_t)bh * num_splits + s) * D + d];
   }
@@ -599,7 +599,7 @@ __global__ void __launch_bounds__(1024) attn_decode_combine_q8_kernel(
       for (int sp = 0; sp < ns; ++sp) M = fmaxf(M, wst[tid * ns + sp]);
       float L = 0.f;
       for (int sp = 0; sp < ns; ++sp) {
-        const float wgt = exp2f(wst[tid * ns + sp] - M);
+        const float wgt = exp2_weight(wst[tid * ns + sp] - M);
         L += wgt * lst[tid * ns + sp];
         wst[tid * ns + sp] = wgt;
       }

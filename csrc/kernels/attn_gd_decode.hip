@@ -130,7 +130,7 @@ __global__ void __launch_bounds__(256, (NK + NV <= 8) ? 2 : 1) attn_gd_decode_ke
     mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
     mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
     if (__any(mx > m_run)) {
-      const float alpha = exp2f(m_run - mx);
+      const float alpha = exp2_weight(m_run - mx);
       l_run *= alpha;
 #pragma unroll
       for (int m = 0; m < 2 * NV; ++m) acc[m] *= alpha;
@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(256, (NK + NV <= 8) ? 2 : 1) attn_gd_decode_ke
       f32x4 p;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        p[j] = exp2f(sc[i][j] - m_run);
+        p[j] = exp2_weight(sc[i][j] - m_run);
         l_run += p[j];
       }
       const s16x4 pb = __builtin_bit_cast(s16x4, __builtin_convertvector(p, bf16x4));
@@ -192,7 +192,7 @@ __global__ void __launch_bounds__(256, (NK + NV <= 8) ? 2 : 1) attn_gd_decode_ke
     float o = 0.f, L = 0.f;
 #pragma unroll
     for (int ww = 0; ww < 4; ++ww) {
-      const float f = exp2f(mls[ww][h][0] - M);
+      const float f = exp2_weight(mls[ww][h][0] - M);
       o += f * red[ww][h][d];
       L += f * mls[ww][h][1];
     }
@@ -224,12 +224,12 @@ __global__ void __launch_bounds__(256) attn_gd_combine_kernel(const AttnDecode a
   float M = -INFINITY;
   for (int s = 0; s < ns; ++s) M = fmaxf(M, ml[2 * s]);
   float L = 0.f;
-  for (int s = 0; s < ns; ++s) L += exp2f(ml[2 * s] - M) * ml[2 * s + 1];
+  for (int s = 0; s < ns; ++s) L += exp2_weight(ml[2 * s] - M) * ml[2 * s + 1];
   float inv = L > 0.f ? 1.f / L : 0.f;
   if (a.gate) inv *= a.gate[bh];
   for (int d = threadIdx.x; d < a.dvp; d += blockDim.x) {
     float o = 0.f;
-    for (int s = 0; s < ns; ++s) o += exp2f(ml[2 * s] - M) * a.o_part[(bh * a.num_splits + s) * a.dvp + d];
+    for (int s = 0; s < ns; ++s) o += exp2_weight(ml[2 * s] - M) * a.o_part[(bh * a.num_splits + s) * a.dvp + d];
     a.out[b * (int64_t)a.o_ld + hq * a.dvp + d] = f2bf(o * inv);
   }
 }

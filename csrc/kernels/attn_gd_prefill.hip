@@ -69,6 +69,12 @@ __global__ void __launch_bounds__(256, (DK + DV <= 320) ? 2 : 1) attn_gd_prefill
     qb[s] = (wave_used && qrow < slen && 16 * s + 8 * h < a.dkp)
                 ? *reinterpret_cast<const u16x8*>(a.q + ((int64_t)(s0 + qrow) * Hq + hq) * a.dkp + 16 * s + 8 * h)
                 : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  float scale = a.scale_log2;   // positive from here on, see attn_prefill.hip
+  if (scale <= 0.f) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qb[s] = scale < 0.f ? qb[s] ^ (uint16_t)0x8000 : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    scale = scale < 0.f ? -scale : 1.f;
+  }
   f32x16 oacc[DB];
 #pragma unroll
   for (int dd = 0; dd < DB; ++dd)
@@ -162,25 +168,27 @@ __global__ void __launch_bounds__(256, (DK + DV <= 320) ? 2 : 1) attn_gd_prefill
     const int wlo = qrow - a.window - (ptile ? kt * BK - pl : kb);   // tile keys up to here are out of the row's window
     const bool mask = (ptile ? (pend < BK) : ((kb + BK > rbase + 1) || (kb + BK > slen))) ||
                       rbase + 31 - a.window >= (ptile ? kt * BK - pl : kb);
-    float mx = -INFINITY;
+    if (mask) {   // the tile's first key past those the row sees, the last one before them
+      const int end = (ptile ? pend : min(qrow + 1, slen) - kb) - 4 * h, out = wlo - 4 * h;
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int j = 32 * b + (i & 3) + 8 * (i >> 2);
+          if (j >= end || j <= out) sacc[b][i] = -INFINITY;
+        }
+    }
+    float mx = sacc[0][0];
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        float sv = sacc[b][i] * a.scale_log2;
-        if (mask) {
-          const int j = 32 * b + (i & 3) + 8 * (i >> 2) + 4 * h;
-          if ((ptile ? (j >= pend) : (kb + j > qrow || kb + j >= slen)) || j <= wlo) sv = -INFINITY;
-        }
-        sacc[b][i] = sv;
-        mx = fmaxf(mx, sv);
-      }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[b][i]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave)) * scale;
     float mnew = fmaxf(mrow, mx);
     const bool rescale = mrow == -INFINITY || mnew > mrow + 8.f;
     if (!rescale) mnew = mrow;
     const float msafe = (mnew == -INFINITY) ? 0.f : mnew;
-    const float alpha = rescale ? exp2f(mrow - msafe) : 1.f;
+    const float alpha = rescale ? exp2_weight(mrow - msafe) : 1.f;
     mrow = mnew;
     float rs = 0.f;
     u16x8 pb[2][2];
@@ -191,13 +199,13 @@ __global__ void __launch_bounds__(256, (DK + DV <= 320) ? 2 : 1) attn_gd_prefill
         f32x8 p;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          p[j] = exp2f(sacc[b][8 * s + j] - msafe);
+          p[j] = exp2_weight(weight_arg(sacc[b][8 * s + j], scale, msafe));
           rs += p[j];
         }
         pb[b][s] = __builtin_bit_cast(u16x8, __builtin_convertvector(p, bf16x8));
       }
     lpart = lpart * alpha + rs;
-    if (rescale) {
+    if (__any(rescale)) {
 #pragma unroll
       for (int dd = 0; dd < DB; ++dd)
 #pragma unroll

@@ -128,7 +128,7 @@ __global__ void __launch_bounds__(256 * HG, HG == 1 && NK < 16 ? 2 : 1) attn_lat
 #pragma unroll
     for (int ww = 0; ww < 4; ++ww) mx = fmaxf(mx, stat[hg][ww][l15]);
     if (__any(mx > m_run)) {
-      const float alpha = exp2f(m_run - mx);
+      const float alpha = exp2_weight(m_run - mx);
       l_run *= alpha;
 #pragma unroll
       for (int m = 0; m < NB; ++m) acc[m] *= alpha;
@@ -137,7 +137,7 @@ __global__ void __launch_bounds__(256 * HG, HG == 1 && NK < 16 ? 2 : 1) attn_lat
     f32x4 p;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      p[i] = exp2f(sc[i] - m_run);
+      p[i] = exp2_weight(sc[i] - m_run);
       l_run += p[i];
     }
     ps[hg][w][lane] = __builtin_bit_cast(s16x4, __builtin_convertvector(p, bf16x4));

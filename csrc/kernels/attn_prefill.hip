@@ -386,19 +386,16 @@ __global__ void __launch_bounds__(512) attn_prefill_gqa_kernel(
 //                 bounce for P); V^T comes from the row-major V tile with
 //                 ds_read_b64_tr_b16 (hardware transpose)
 // A 32-row wave reads each staged K/V byte from LDS once per 32 rows instead of
-// once per 16 (v2), halving LDS read traffic per MFMA, and both tiles are staged
-// with plain 16-B row writes (v2 scattered V with 2-B transposing writes).
+// once per 16 (v2), halving LDS read traffic per MFMA.
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 
-// K tile image: rows padded to 272 B (kRowK), chunk ch of row r at 272 r + 16 ch -> the
-// ds_read_b128 of 16 consecutive rows at one chunk hits 16 distinct bank groups, and a
-// lane's reads of one tile are its row base plus compile-time offsets (no per-read
-// address arithmetic, unlike an XOR swizzle).
-constexpr int kRowK = 272;
-__device__ __forceinline__ int k_img(int r, int ch) { return kRowK * r + 16 * ch; }
-// V tile image (§5.5 T10 image (b)): conflict-free for the 32x32x16 transposed reads.
-__device__ __forceinline__ int v_img(int r, int ch) { return 256 * r + 16 * (ch ^ (((r & 3) << 2) | ((r >> 2) & 3))); }
+// Tile images: rows of 256 B, chunk ch of row r in a slot that depends on the row, as the LDS-DMA's source order.
+// K: the ds_read_b128 of 16 consecutive rows at one chunk hits 16 distinct slots.
+__device__ __forceinline__ int k_img(int r, int ch) { return 256 * r + 16 * (ch ^ (r & 15)); }
+__device__ __forceinline__ int v_swz(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
+// V: conflict-free for the 32x32x16 transposed reads.
+__device__ __forceinline__ int v_img(int r, int ch) { return 256 * r + 16 * (ch ^ v_swz(r)); }
 
 __device__ __forceinline__ s16x4 ds_read_tr16(const char* p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p));
@@ -409,17 +406,23 @@ __device__ __forceinline__ s16x4 ds_read_tr16(const char* p) {
 // share) followed by its own slen keys; its query rows are its own tokens, at positions
 // seq_pfx[seq] + row. Prefix keys are visible to every row; a last, partial prefix tile is
 // masked past the prefix length.
-// Schedule: the next tile's K/V loads are issued after this tile's S MFMAs (they are in
-// flight during softmax + P.V instead of holding registers across the S MFMAs), and the
-// rescale is deferred — a row keeps its running max until a tile raises it by more than 8
-// (log2 units, so P <= 256 in fp32 / bf16), skipping the O / l rescale otherwise. Measured
-// against the plain schedule on MI355X (profiles/prefill_attn_v3_schedule_variants.jsonl):
-// 16x1024 0.290 vs 0.326 ms, 4x4096 0.857 vs 0.963 ms; the late loads alone, and two LDS
-// tile buffers with one barrier per tile (with or without the deferred rescale), were
-// slower than this pair and were removed.
+// Schedule: two LDS buffers of a K and a V tile; the next tile's LDS-DMA goes out when this one's work begins, one barrier per
+// tile. The rescale is deferred: a row keeps its running max until a tile raises it by more than 8 (log2 units, so
+// P <= 256 in fp32 / bf16), skipping the O / l rescale otherwise.
+// What bounds it: the instructions of a wave. Per 64-key tile 32 MFMAs (1024 clocks), 48 LDS reads and, per lane, 32 scores; with
+// the library's exp2f (range checks around v_exp_f32), a scale, a select and a subtraction per score and K/V staged through registers
+// behind two barriers a tile took 2.9 us alone on a CU. The bare v_exp_f32 (arguments are at most 8, and what underflows
+// is zero), the maximum over unscaled scores, masks in tiles that need them only: 2.0; LDS-DMA: 1.6. 885 tokens, 32 / 8 heads:
+// 44.6 -> 25.8 us, 32 prompts of about 885: 430 -> 335 (600 TFLOP/s), 4 x 2048: 267 -> 175. Neither more tiles in flight nor fragments
+// read ahead gained, nor keys split over two groups of waves (23 us, but 440 for the 32 prompts).
 // NW: waves per workgroup. 8 (one work item = 8 waves of (head, 32-row block)) holds a CU
-// alone at 239 VGPRs (2 waves per SIMD), so every barrier of its K/V tile loop idles the
+// alone at over 200 VGPRs (2 waves per SIMD), so every barrier of its K/V tile loop idles the
 // CU; NW = 4 (G <= 4) halves the work item and puts two workgroups on each CU.
+template <int N>
+__device__ __forceinline__ void vm_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
 template <int G, int NW = 8>
 __global__ void __launch_bounds__(NW * 64, 2) attn_prefill_mfma32_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
@@ -427,10 +430,10 @@ __global__ void __launch_bounds__(NW * 64, 2) attn_prefill_mfma32_kernel(
     const int* __restrict__ work_q0, int Hq, int Hkv, float scale_log2, const bf16_t* __restrict__ pk,
     const bf16_t* __restrict__ pv, const int* __restrict__ seq_pfx) {
   constexpr int D = 128, BK = 64, RG = NW / G, BQ = 32 * RG;
-  constexpr int NT = NW * 64, NC = BK * 16 / NT;   // threads; 16-B K (and V) chunks each stages per tile
+  constexpr int kTile = BK * 256;   // bytes of a K or V tile
+  constexpr int NP = 16 / NW;       // 1 KiB pieces (4 rows) of each a wave stages per tile
   static_assert(RG >= 1, "a workgroup needs a row block per head");
-  __shared__ __attribute__((aligned(16))) char Ks[BK * kRowK];
-  __shared__ __attribute__((aligned(16))) char Vs[BK * 256];
+  __shared__ __attribute__((aligned(1024))) char lds[2 * 2 * kTile];   // two buffers of a K and a V tile
 
   const int wi = blockIdx.x, kvh = blockIdx.y;
   const int seq = work_seq[wi];
@@ -438,7 +441,8 @@ __global__ void __launch_bounds__(NW * 64, 2) attn_prefill_mfma32_kernel(
   const int s0 = cu_seqlens[seq];
   const int slen = cu_seqlens[seq + 1] - s0;
   const int q0 = work_q0[wi];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r32 = lane & 31, h = lane >> 5;
   const int hq = kvh * G + (w % G);
   const int rbase = q0 + 32 * (w / G);  // this wave's first query row
@@ -453,6 +457,13 @@ __global__ void __launch_bounds__(NW * 64, 2) attn_prefill_mfma32_kernel(
   for (int s = 0; s < 8; ++s)
     qb[s] = qrow < slen ? *reinterpret_cast<const u16x8*>(q + ((int64_t)(s0 + qrow) * Hq + hq) * D + 16 * s + 8 * h)
                         : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  // the largest score is the scale times the largest product only for a positive scale: a negative one goes into q's signs
+  // (exact), of a zero one the products are zero
+  if (scale_log2 <= 0.f) {
+#pragma unroll
+    for (int s = 0; s < 8; ++s) qb[s] = scale_log2 < 0.f ? qb[s] ^ (uint16_t)0x8000 : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    scale_log2 = scale_log2 < 0.f ? -scale_log2 : 1.f;
+  }
   f32x16 oacc[4];
 #pragma unroll
   for (int dd = 0; dd < 4; ++dd)
@@ -467,130 +478,130 @@ __global__ void __launch_bounds__(NW * 64, 2) attn_prefill_mfma32_kernel(
   const bool active = wave_used && rbase < slen;
   const int wend = min(slen, rbase + 32);  // own keys this wave can see: < wend
 
+  // staging: piece p = rows 4p .. 4p+3 of the tile, lane -> row lane / 16, LDS chunk lane % 16, source chunk swizzled
+  const int rb = Hkv * D * 2;   // bytes from row to row
+  uint32_t vk[NP], vv[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int row = 4 * (w + NW * i) + (lane >> 4), ch = lane & 15;
+    vk[i] = (uint32_t)(row * rb + ((ch ^ (row & 15)) << 4));
+    vv[i] = (uint32_t)(row * rb + ((ch ^ v_swz(row)) << 4));
+  }
+  auto stage = [&](int kt, int buf) {   // key tile kt: a prefix tile (kt < npt) or own tile kt - npt
+    const bf16_t *kp, *vp;
+    int rows;
+    if (kt < npt) {
+      const int64_t off = ((int64_t)kt * BK * Hkv + kvh) * D;
+      kp = pk + off; vp = pv + off; rows = pl - kt * BK;
+    } else {
+      const int64_t off = ((int64_t)(s0 + (kt - npt) * BK) * Hkv + kvh) * D;
+      kp = k + off; vp = v + off; rows = slen - (kt - npt) * BK;
+    }
+    const int n = (min(rows, BK) - 1) * rb + 256;   // rows past the end read as zeros
+    char* dst = lds + buf * 2 * kTile;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)kp, (short)0, n, 0x00020000),
+                                               (__attribute__((address_space(3))) void*)(dst + (w + NW * i) * 1024), 16, (int)vk[i], 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)vp, (short)0, n, 0x00020000),
+                                               (__attribute__((address_space(3))) void*)(dst + kTile + (w + NW * i) * 1024), 16, (int)vv[i], 0, 0, 0);
+    }
+  };
+
   // transposed-read addressing: 16-lane group g reads rows r0 + q (q = i >> 2) at
   // columns d0 + 4p .. +3 (p = i & 3), d0 = 32 dd + 16 (g & 1); lane i gets column d0 + i
   const int gi = lane & 15, g = lane >> 4;
   const int trq = gi >> 2, trp = gi & 3;
 
-  u16x8 kr[NC], vr[NC];
-  auto load_tile = [&](int kt) {   // key tile kt: a prefix tile (kt < npt) or own tile kt - npt
-#pragma unroll
-    for (int r = 0; r < NC; ++r) {
-      const int c = tid + r * NT;
-      const int key = c >> 4, ch = c & 15;
-      kr[r] = vr[r] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-      if (kt < npt) {
-        if (kt * BK + key < pl) {
-          const int64_t off = ((int64_t)(kt * BK + key) * Hkv + kvh) * D + ch * 8;
-          kr[r] = *reinterpret_cast<const u16x8*>(pk + off);
-          vr[r] = *reinterpret_cast<const u16x8*>(pv + off);
-        }
-      } else if ((kt - npt) * BK + key < slen) {
-        const int64_t off = ((int64_t)(s0 + (kt - npt) * BK + key) * Hkv + kvh) * D + ch * 8;
-        kr[r] = *reinterpret_cast<const u16x8*>(k + off);
-        vr[r] = *reinterpret_cast<const u16x8*>(v + off);
-      }
-    }
-  };
-  auto store_tile = [&]() {
-#pragma unroll
-    for (int r = 0; r < NC; ++r) {
-      const int c = tid + r * NT;
-      const int key = c >> 4, ch = c & 15;
-      *reinterpret_cast<u16x8*>(Ks + k_img(key, ch)) = kr[r];
-      *reinterpret_cast<u16x8*>(Vs + v_img(key, ch)) = vr[r];
-    }
-  };
-
-  load_tile(0);
-  for (int kt = 0; kt < ntiles; ++kt) {
+  stage(0, 0);
+  vm_wait<0>();
+  __syncthreads();
+  for (int kt = 0, buf = 0; kt < ntiles; ++kt, buf ^= 1) {
+    if (kt + 1 < ntiles) stage(kt + 1, buf ^ 1);
     const int kb = (kt - npt) * BK;   // own-key coordinates (negative: a prefix tile)
-    const char* Kc = Ks;
-    const char* Vc = Vs;
-    __syncthreads();  // previous tile fully consumed
-    store_tile();
+    const char* Kc = lds + buf * 2 * kTile;
+    const char* Vc = Kc + kTile;
+    if (active && kb < wend) {   // wave-uniform
+      // ---- S^T = K Q^T (two 32-key blocks) ----
+      f32x16 sacc[2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sacc[b][i] = 0.f;
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          const u16x8 ka = *reinterpret_cast<const u16x8*>(Kc + k_img(32 * b + r32, 2 * s + h));
+          sacc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(ka), as_bf8(qb[s]), sacc[b], 0, 0, 0);
+        }
+      // ---- online softmax: register i of block b is key kb + 32b + (i&3) + 8(i>>2) + 4h ----
+      const bool ptile = kb < 0;
+      const int pend = pl - kt * BK;   // prefix tile: its keys below pend are prefix keys
+      const bool mask = ptile ? (pend < BK) : ((kb + BK > rbase + 1) || (kb + BK > slen));
+      if (mask) {
+        // the tile's first key this lane's row does not see
+        const int lim = (ptile ? pend : min(qrow + 1, slen) - kb) - 4 * h;
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            if (32 * b + (i & 3) + 8 * (i >> 2) >= lim) sacc[b][i] = -INFINITY;
+      }
+      float mx = sacc[0][0];
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[b][i]);
+      mx = fmaxf(mx, __shfl_xor(mx, 32, kWave)) * scale_log2;
+      float mnew = fmaxf(mrow, mx);
+      const bool rescale = mrow == -INFINITY || mnew > mrow + 8.f;   // deferred rescale
+      if (!rescale) mnew = mrow;
+      const float msafe = (mnew == -INFINITY) ? 0.f : mnew;
+      const float alpha = rescale ? exp2_weight(mrow - msafe) : 1.f;
+      mrow = mnew;
+      float rs = 0.f;
+      u16x8 pb[2][2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          f32x8 p;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            p[j] = exp2_weight(weight_arg(sacc[b][8 * s + j], scale_log2, msafe));
+            rs += p[j];
+          }
+          pb[b][s] = __builtin_bit_cast(u16x8, __builtin_convertvector(p, bf16x8_t));
+        }
+      lpart = lpart * alpha + rs;
+      if (__any(rescale)) {
+#pragma unroll
+        for (int dd = 0; dd < 4; ++dd)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) oacc[dd][i] *= alpha;
+      }
+
+      // ---- O^T += V^T P^T: B element j of half h is key 32b + 16s + 8(j>>2) + 4h + (j&3) ----
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const int r0 = 32 * b + 16 * s + 4 * h + trq;
+#pragma unroll
+          for (int dd = 0; dd < 4; ++dd) {
+            const int d = 32 * dd + 16 * (g & 1) + 4 * trp;
+            const s16x4 lo = ds_read_tr16(Vc + v_img(r0, d >> 3) + 8 * ((d >> 2) & 1));
+            const s16x4 hi = ds_read_tr16(Vc + v_img(r0 + 8, d >> 3) + 8 * ((d >> 2) & 1));
+            const s16x8 va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+            oacc[dd] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, va),
+                                                              as_bf8(pb[b][s]), oacc[dd], 0, 0, 0);
+          }
+        }
+  
+    }
+    vm_wait<0>();
     __syncthreads();
-    if (!active || kb >= wend) {   // wave-uniform: no visible key for this wave
-      if (kt + 1 < ntiles) load_tile(kt + 1);
-      continue;
-    }
-
-    // ---- S^T = K Q^T (two 32-key blocks) ----
-    f32x16 sacc[2];
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) sacc[b][i] = 0.f;
-      const int key = 32 * b + r32;
-#pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        const u16x8 ka = *reinterpret_cast<const u16x8*>(Kc + k_img(key, 2 * s + h));
-        sacc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(ka), as_bf8(qb[s]), sacc[b], 0, 0, 0);
-      }
-    }
-    if (kt + 1 < ntiles) load_tile(kt + 1);   // in flight during softmax + P.V
-    // ---- online softmax: register i of block b is key kb + 32b + (i&3) + 8(i>>2) + 4h ----
-    const bool ptile = kb < 0;
-    const int pend = pl - kt * BK;   // prefix tile: its keys below pend are prefix keys
-    const bool mask = ptile ? (pend < BK) : ((kb + BK > rbase + 1) || (kb + BK > slen));
-    float mx = -INFINITY;
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        float sv = sacc[b][i] * scale_log2;
-        if (mask) {
-          const int j = 32 * b + (i & 3) + 8 * (i >> 2) + 4 * h;   // key within the tile
-          if (ptile ? (j >= pend) : (kb + j > qrow || kb + j >= slen)) sv = -INFINITY;
-        }
-        sacc[b][i] = sv;
-        mx = fmaxf(mx, sv);
-      }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-    float mnew = fmaxf(mrow, mx);
-    const bool rescale = mrow == -INFINITY || mnew > mrow + 8.f;   // deferred rescale
-    if (!rescale) mnew = mrow;
-    const float msafe = (mnew == -INFINITY) ? 0.f : mnew;
-    const float alpha = rescale ? exp2f(mrow - msafe) : 1.f;
-    mrow = mnew;
-    float rs = 0.f;
-    u16x8 pb[2][2];
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        f32x8 p;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          p[j] = exp2f(sacc[b][8 * s + j] - msafe);
-          rs += p[j];
-        }
-        pb[b][s] = __builtin_bit_cast(u16x8, __builtin_convertvector(p, bf16x8_t));
-      }
-    lpart = lpart * alpha + rs;
-    if (rescale) {
-#pragma unroll
-      for (int dd = 0; dd < 4; ++dd)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) oacc[dd][i] *= alpha;
-    }
-
-    // ---- O^T += V^T P^T: B element j of half h is key 32b + 16s + 8(j>>2) + 4h + (j&3) ----
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int r0 = 32 * b + 16 * s + 4 * h + trq;
-#pragma unroll
-        for (int dd = 0; dd < 4; ++dd) {
-          const int d = 32 * dd + 16 * (g & 1) + 4 * trp;
-          const s16x4 lo = ds_read_tr16(Vc + v_img(r0, d >> 3) + 8 * ((d >> 2) & 1));
-          const s16x4 hi = ds_read_tr16(Vc + v_img(r0 + 8, d >> 3) + 8 * ((d >> 2) & 1));
-          const s16x8 va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-          oacc[dd] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, va),
-                                                            as_bf8(pb[b][s]), oacc[dd], 0, 0, 0);
-        }
-      }
   }
   if (!active) return;
   const float lsum = lpart + __shfl_xor(lpart, 32, kWave);

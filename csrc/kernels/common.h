@@ -60,6 +60,18 @@ __device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) {
   return static_cast<uint32_t>(f2bf(lo)) | (static_cast<uint32_t>(f2bf(hi)) << 16);
 }
 
+// 2^x of softmax weights: the bare v_exp_f32. exp2f brackets it with a range check, a select and a scaling that keep
+// results below 2^-126, which are zero weights here.
+__device__ __forceinline__ float exp2_weight(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// A weight's argument from the raw score: scaled and rounded, then the row's maximum (a scaled score itself) subtracted. Not
+// contracted, so the largest score's own argument is exactly 0.
+__device__ __forceinline__ float weight_arg(float score, float scale, float top) {
+#pragma clang fp contract(off)
+  const float x = score * scale;
+  return x - top;
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
