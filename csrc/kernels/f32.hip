@@ -62,10 +62,12 @@ struct GemmF32 {
 // tiles, four waves of 32 x 32 outputs in 16 x 16 blocks.
 // What bounds it: the fp32 MFMA rate, 256 flop per clock and CU (157 TFLOP/s; ordinary FMA reaches half of that without
 // packed fp32, which is off). A 32-column step is 1024 clocks of MFMA against 256 of fragment reads and 128 of LDS-DMA
-// writes, so a plain three-stage ring with two or three workgroups per CU hides the rest. 64 x 64 tiles because products
+// writes; with two or three workgroups per CU, reads, requests and products one after the other left the MFMAs a third of
+// the time (962 rows of 16384 x 2048 gated 632 us). So a step's second fragments are read under its first products, the next step's
+// first under its second ones, and the LDS-DMA pieces go out between them: 560 us (123 TFLOP/s with the padding rows, what a large product
+// reaches), 12 products of 2048 features 146 -> 131 on average. 64 x 64 tiles because products
 // here have few rows (500 rows of 2048 features: 256 tiles) and because routed experts' segments are padded to 64 rows.
-// 1000 rows: 16384 x 2048 gated 905 -> 584 us (115 TFLOP/s), 2048 x 8192 590 -> 313; 18 rows of 2048 x 8192 in eight
-// K slices 1000 -> 33.
+// 18 rows of 2048 x 8192 in eight K slices 33 us.
 // GLU: W holds gate | up rows interleaved in 64-row blocks; a tile is 64 features, Y [M, N/2]
 // = act(c g) * (c u) with c the row's scale (rscale, or 1).
 // gtab != nullptr: rows are expert segments padded to 64-row tiles; gtab[0] = tile count,
@@ -110,50 +112,81 @@ __global__ void __launch_bounds__(256) gemm_f32_kernel(const GemmF32 a) {
     src[i] = row < 64 ? X + min(m0 + row, a.M - 1) * a.ldx : W + (int64_t)min((GLU ? 2 * f0 : f0) + row - 64, a.N - 1) * a.K;
     col[i] = 4 * ((lane & 7) ^ ((row >> 1) & 7));
   }
-  auto issue = [&](int t) {
-    char* base = lds + (t % kStages) * kStage;
-#pragma unroll
-    for (int i = 0; i < GL; ++i) {
-      const int k = kbase + t * 32 + col[i];
-      const float* from = src[i] + (k < K ? k : 0);
-      __builtin_amdgcn_global_load_lds(from, (__attribute__((address_space(3))) void*)(base + (w + 4 * i) * 1024), 16, 0, 0);
-    }
+  auto issue = [&](int t, int off, int i) {
+    const int k = kbase + t * 32 + col[i];
+    const float* from = src[i] + (k < K ? k : 0);
+    __builtin_amdgcn_global_load_lds(from, (__attribute__((address_space(3))) void*)(lds + off + (w + 4 * i) * 1024), 16, 0, 0);
   };
-  const int l15 = lane & 15, g = lane >> 4, sw = (l15 >> 1) & 7;
+  const int l15 = lane & 15, g = lane >> 4, sw = (l15 >> 1) & 7;   // row / 2 % 8 depends on the lane only: blocks are 16 rows
+  const int xo = (wm * 32 + l15) * 128, wo = (64 + wn * 32 + l15) * 128;
+  constexpr int NF = 2 + 2 * NB;   // fragments of a 16-column half: two token blocks, then the features'
+  auto rd = [&](int off, int s, f32x4 (&f)[NF], int i) {
+    const int at = off + (((4 * s + g) ^ sw) << 4);
+    f[i] = *reinterpret_cast<const f32x4*>(lds + at + (i < 2 ? xo + i * 2048 : wo + ((i - 2) >> 1) * 8192 + (i & 1) * 2048));
+  };
+  // A barrier inside every step (after kBar of the second half's kH MFMAs) says that its stage has been read and the next one
+  // has landed: the next step's first fragments are read behind it, and the pieces of the step kStages ahead go into the stage,
+  // spread over the 2 kH MFMAs up to the next barrier.
+  constexpr int kH = 16 * NB, kBar = kH / 4, kTail = kH - kBar;
   f32x4 acc[NB][2][2] = {};   // [gate | up][feature block][token block]
+  auto mul = [&](const f32x4 (&f)[NF], int v) {
+    const int e = v / (4 * NB), b = v / 4 % NB, j = v / 2 % 2, i = v % 2;
+    acc[b][j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[2 + 2 * b + j][e], f[i][e], acc[b][j][i], 0, 0, 0);
+  };
+  auto piece = [&](int z, int t, int off) {
+    const int i = (z * GL + 2 * kH - 1) / (2 * kH);
+    if (i < GL && i * 2 * kH / GL == z && t < T) issue(t, off, i);
+  };
 #pragma unroll
-  for (int st = 0; st < kStages - 1; ++st)
-    if (T > st) issue(st);
+  for (int st = 0; st < kStages; ++st)
+    if (T > st)
+#pragma unroll
+      for (int i = 0; i < GL; ++i) issue(st, st * kStage, i);
+  if (T > 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * GL) : "memory");
+  else if (T > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(GL) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  f32x4 fa[NF], fb[NF];
+#pragma unroll
+  for (int i = 0; i < NF; ++i) rd(0, 0, fa, i);
+  int off = 0, prev = -1;   // this step's stage; the one of the step before, whose refill goes on
   for (int t = 0; t < T; ++t) {
-    if (t + 1 < T) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(GL) : "memory");   // all but the next stage's pieces
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (t + kStages - 1 < T) issue(t + kStages - 1);
-    const char* base = lds + (t % kStages) * kStage;
+    const int nxt = off + kStage == kStages * kStage ? 0 : off + kStage;
+    const int fill = prev < 0 ? T : t + kStages - 1;   // the step that goes into `prev`
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      if (kbase + t * 32 + 16 * s >= a.K) break;
-      const int off = ((4 * s + g) ^ sw) << 4;   // row / 2 % 8 depends on the lane only: blocks are 16 rows
-      f32x4 xf[2], wf[NB][2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) xf[i] = *reinterpret_cast<const f32x4*>(base + (wm * 32 + 16 * i + l15) * 128 + off);
-#pragma unroll
-      for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          wf[b][j] = *reinterpret_cast<const f32x4*>(base + (64 + 64 * b + wn * 32 + 16 * j + l15) * 128 + off);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-              acc[b][j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[b][j][e], xf[i][e], acc[b][j][i], 0, 0, 0);
+    for (int v = 0; v < kH; ++v) {
+      mul(fa, v);
+      __builtin_amdgcn_sched_barrier(0);
+      if (v < NF) rd(off, 1, fb, v);
+      piece(kTail + v, fill, prev);
+      __builtin_amdgcn_sched_barrier(0);
     }
+    const bool two = kbase + t * 32 + 16 < K;   // K % 32 == 16: the last step has one half
+#pragma unroll
+    for (int v = 0; v < kBar; ++v) {
+      if (two) mul(fb, v);
+      __builtin_amdgcn_sched_barrier(0);
+      piece(kTail + kH + v, fill, prev);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (t + 2 < T) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(GL) : "memory");   // all but the pieces of the step after the next
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (two) {
+#pragma unroll
+      for (int v = kBar; v < kH; ++v) {
+        mul(fb, v);
+        __builtin_amdgcn_sched_barrier(0);
+        if (v - kBar < NF) rd(nxt, 0, fa, v - kBar);
+        piece(v - kBar, t + kStages, off);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    prev = off;
+    off = nxt;
   }
   // a lane holds features 4 g .. + 3 of each block of token l15
   const int NO = GLU && !PART ? a.N / 2 : a.N;
