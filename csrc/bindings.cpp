@@ -755,6 +755,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("sample", &sample, pybind11::arg("logits"), pybind11::arg("temperature"), pybind11::arg("seeds"),
         pybind11::arg("positions"), pybind11::arg("out"), pybind11::arg("col_offset") = 0,
         pybind11::arg("out_val") = pybind11::none(), pybind11::arg("part") = pybind11::none());
+  m.attr("NO_SAMPLE_BITS") = oamd::kNoSampleBits;
   m.def("sample_parts", &oamd::sample_parts, pybind11::arg("rows"), pybind11::arg("vocab"));
   m.def("graph_launch", &graph_launch, pybind11::arg("graph_exec"), pybind11::arg("count"), pybind11::arg("stream"));
   register_decoder_bindings(m);

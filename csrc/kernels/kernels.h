@@ -134,6 +134,7 @@ int attn_prefill(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16_t* o, c
                  const int* work_seq, const int* work_q0, int num_work, int Hq, int Hkv, int head_dim,
                  float scale, int variant, hipStream_t stream,
                  const bf16_t* pk = nullptr, const bf16_t* pv = nullptr, const int* seq_pfx = nullptr);
+constexpr uint32_t kNoSampleBits = 0x7fc5a5a5u;   // temperature of a row that is not sampled: a quiet NaN that nothing computes
 int sample_tokens(const void* logits, bool logits_bf16, int64_t stride, int rows, int vocab,
                   const float* temperature, const int64_t* seeds, const int64_t* positions,
                   int64_t* out_tokens, int64_t col_offset, float* out_val, float* part, hipStream_t stream);

@@ -190,7 +190,7 @@ class _BucketState:
 
     def load(self, reqs: list[GenRequest], max_pages: int, dst: list[int] | None = None) -> None:
         """Write the per-row state of ``reqs`` (rows beyond are padding; ``dst``: the row of the caller's logits each
-        takes, see given_next). Built in numpy
+        takes, see given_next; their tokens are not sampled). Built in numpy
         (one pass over the rows, no per-element tensor indexing: ~0.3 ms instead of
         ~10 ms for 256 rows at every batch-composition change) and copied in once."""
         n = len(reqs)
@@ -198,15 +198,17 @@ class _BucketState:
         v = {k: t.numpy() for k, t in self._views(host).items()}
         ids, pos, ctx, bt, temp, seeds = v["ids"], v["pos"], v["ctx"], v["bt"], v["temp"], v["seeds"]
         assert bt.shape[1] == max_pages
+        temp.view(np.uint32)[:] = ops.NO_SAMPLE_BITS   # padding rows, and given tokens
         if n:
             lens = np.fromiter((r.length for r in reqs), dtype=np.int64, count=n)
             ids[:n] = np.fromiter((r.output[-1] for r in reqs), dtype=np.int64, count=n)
             pos[:n] = lens - 1
             ctx[:n] = lens
-            temp[:n] = np.fromiter((r.temperature for r in reqs), dtype=np.float32, count=n)
-            seeds[:n] = np.fromiter((r.seed for r in reqs), dtype=np.int64, count=n)
             if dst is not None:
                 v["dst"][:n] = dst
+            else:
+                temp[:n] = np.fromiter((r.temperature for r in reqs), dtype=np.float32, count=n)
+                seeds[:n] = np.fromiter((r.seed for r in reqs), dtype=np.int64, count=n)
             for i, r in enumerate(reqs):
                 bt[i, :len(r.pages)] = r.pages
         nb = self._buf.is_cuda

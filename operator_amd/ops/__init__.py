@@ -948,6 +948,11 @@ def attn_decode_rope(qkv, pos: torch.Tensor, cos: torch.Tensor, sin: torch.Tenso
     return (q8, sx) if quant else o
 
 
+# temperature bits of a row whose token nobody reads: it gets token 0, its logits are not read (csrc/kernels/sample.hip;
+# the CPU reference samples it like any NaN, greedily)
+NO_SAMPLE_BITS = 0x7FC5A5A5
+
+
 def sample(logits: torch.Tensor, temperature: torch.Tensor, seeds: torch.Tensor, positions: torch.Tensor,
            out: torch.Tensor | None = None, col_offset: int = 0, out_val: torch.Tensor | None = None) -> torch.Tensor:
     """Temperature / Gumbel-max sampling (greedy rows where temperature <= 0).
