@@ -850,14 +850,31 @@ class LLMEngine:
     def _to_device(self, x, dt=torch.long) -> torch.Tensor:
         return torch.as_tensor(np.asarray(x)).to(dtype=dt).to(self.device, non_blocking=True)
 
+    def _upload(self, *parts) -> list[torch.Tensor]:
+        """Arrays of int64, then of int32, on the device in one copy (a copy each costs the GPU 5 us)."""
+        parts = [np.asarray(x, dtype=dt) for x, dt in parts]
+        gpu = self.device.type == "cuda"
+        host = torch.empty(sum(x.nbytes for x in parts), dtype=torch.uint8, pin_memory=gpu)
+        view, off, out = host.numpy(), 0, []
+        for x in parts:
+            view[off:off + x.nbytes].view(x.dtype)[:] = x
+            off += x.nbytes
+        buf, off = host.to(self.device, non_blocking=True), 0
+        for x in parts:
+            out.append(buf[off:off + x.nbytes].view(torch.int64 if x.dtype == np.int64 else torch.int32))
+            off += x.nbytes
+        return out
+
     def _eager_prefill(self, p: dict, last) -> torch.Tensor:
         """Logits of rows ``last`` of a packed prefill batch, computed without a graph."""
-        t = self._to_device
-        work = (t(p["cu"], torch.int32), t(p["ws"], torch.int32), t(p["wq"], torch.int32), p["var"]) \
-            if self.device.type == "cuda" else None
-        pre = (self._pk, self._pv, t(p["skip"], torch.int32), p["skip"]) if any(p["skip"]) else None
-        fb = ForwardBatch(t(p["ids"]), t(p["pos"]), t(p["slots"]), True, t(last), seq_lens=p["lens"], prefill_work=work,
-                          prefix=pre, prev_pages=None if pre is None else t(p["prev"], torch.int32))
+        i64, i32 = np.int64, np.int32
+        ids, pos, slots, last, cu, ws, wq, skip, prev = self._upload(
+            (p["ids"], i64), (p["pos"], i64), (p["slots"], i64), (last, i64), (p["cu"], i32), (p["ws"], i32), (p["wq"], i32),
+            (p["skip"], i32), (p["prev"], i32))
+        work = (cu, ws, wq, p["var"]) if self.device.type == "cuda" else None
+        pre = (self._pk, self._pv, skip, p["skip"]) if any(p["skip"]) else None
+        fb = ForwardBatch(ids, pos, slots, True, last, seq_lens=p["lens"], prefill_work=work,
+                          prefix=pre, prev_pages=None if pre is None else prev)
         return self.model.forward(fb, self.kv)
 
     def _prefill_impl(self, batch: list[GenRequest]) -> _PendingPrefill:
