@@ -505,7 +505,7 @@ void gemm_fp8(const at::Tensor& x8, const at::Tensor& w8, const at::Tensor& sx, 
 
 // y omitted: the consumer sums the fp32 slabs
 void gemm_fp8_tile(const at::Tensor& x8, const at::Tensor& w8, const at::Tensor& sx, const at::Tensor& sw,
-                   const c10::optional<at::Tensor>& y, const c10::optional<at::Tensor>& p, int64_t splits) {
+                   const c10::optional<at::Tensor>& y, const c10::optional<at::Tensor>& p, int64_t splits, int64_t rows) {
   CHECK_DEV(x8); CHECK_CONTIG(x8); CHECK_CONTIG(w8); CHECK_CONTIG(sx); CHECK_CONTIG(sw); CHECK_DT(sx, at::kFloat); CHECK_DT(sw, at::kFloat);
   for (auto* t : {&x8, &w8})
     TORCH_CHECK(t->scalar_type() == at::kByte || t->scalar_type() == at::kFloat8_e4m3fn, "fp8 operands");
@@ -515,6 +515,7 @@ void gemm_fp8_tile(const at::Tensor& x8, const at::Tensor& w8, const at::Tensor&
   TORCH_CHECK(N >= 16 && N % 16 == 0 && K % 128 == 0 && N < (1LL << 31) && M < (1LL << 31) && K < (1LL << 23),
               "gemm_fp8_tile: N % 16 == 0, K % 128 == 0");
   TORCH_CHECK(splits >= 1 && splits <= 16 && K / 128 / splits >= 3, "gemm_fp8_tile: slices of at least 3 x 128");
+  TORCH_CHECK(rows == 96 || rows == 128 || rows == 160, "gemm_fp8_tile: tiles of 96, 128 or 160 rows");
   if (y.has_value()) {
     CHECK_BF16(*y); CHECK_CONTIG(*y);
     TORCH_CHECK(y->dim() == 2 && y->size(0) == M && y->size(1) == N && reinterpret_cast<uintptr_t>(y->data_ptr()) % 16 == 0, "gemm_fp8_tile: y [M, N], 16-B aligned");
@@ -529,7 +530,7 @@ void gemm_fp8_tile(const at::Tensor& x8, const at::Tensor& w8, const at::Tensor&
   }
   const c10::hip::HIPGuardMasqueradingAsCUDA g(x8.device());
   RC(oamd::gemm_fp8_tile(static_cast<const uint8_t*>(x8.data_ptr()), static_cast<const uint8_t*>(w8.data_ptr()), ptr<float>(sx),
-                         ptr<float>(sw), optr<bf16_t>(y), pp, (int)M, (int)N, (int)K, (int)splits, cur_stream()));
+                         ptr<float>(sw), optr<bf16_t>(y), pp, (int)M, (int)N, (int)K, (int)splits, (int)rows, cur_stream()));
 }
 
 void attn_decode(const at::Tensor& q, const at::Tensor& k_cache, const at::Tensor& v_cache,
@@ -726,7 +727,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("rmsnorm_fp8", &rmsnorm_fp8, pybind11::arg("x"), pybind11::arg("residual"), pybind11::arg("w"), pybind11::arg("q"),
         pybind11::arg("sx"), pybind11::arg("eps"), pybind11::arg("partial") = pybind11::none(), pybind11::arg("splits") = 1);
   m.def("gemm_fp8_tile", &gemm_fp8_tile, pybind11::arg("x8"), pybind11::arg("w8"), pybind11::arg("sx"), pybind11::arg("sw"),
-        pybind11::arg("y"), pybind11::arg("p") = pybind11::none(), pybind11::arg("splits") = 1);
+        pybind11::arg("y"), pybind11::arg("p") = pybind11::none(), pybind11::arg("splits") = 1, pybind11::arg("rows") = 128);
   m.def("gemm_fp8", &gemm_fp8, pybind11::arg("x8"), pybind11::arg("w8"), pybind11::arg("sx"), pybind11::arg("sw"),
         pybind11::arg("y"), pybind11::arg("p") = pybind11::none(), pybind11::arg("splits") = 1,
         pybind11::arg("bn") = 64, pybind11::arg("bm") = 64, pybind11::arg("reduce") = true);

@@ -1,13 +1,13 @@
 // FP8 (e4m3fn) GEMM for prompts: Y[M, N] = (X8[M, K] . W8[N, K]^T) * sx[m] * sw[n], fp32 accumulate, bf16 out.
 //
-// What bounds it: the bytes a CU takes in (0.85 to 0.9 us per 48 KiB step, 0.43 of it MFMA), where gemm_fp8 waits for a
-// stage, reads its fragments and runs its MFMAs one after the other. This is gemm_mid's continuous pipeline (128 x 256
-// tiles, four waves of 64 x 128 outputs in AGPRs, three 48 KiB stages filled by LDS-DMA, units (tile, K slice) walked
+// What bounds it: what a CU takes in (a 128-row step's 48 pieces of 1 KiB are 960 clocks of its address unit, its MFMAs 1024) and
+// the rounds of tiles on the CUs. This is gemm_mid's continuous pipeline (tiles of 96, 128 or 160 rows by 256 columns,
+// ops.fp8_tile_rows, four waves of 16 MI x 128 outputs in AGPRs, three stages filled by LDS-DMA, units (tile, K slice) walked
 // by persistent workgroups) with 128 of K per 128-B line. The f8f6f4 MFMA of unit block scales takes a whole line of 16
 // rows, so a step's fragments are read one step ahead, each W fragment into the registers of the one just used, while
-// the 32 MFMAs of this step run, and the stage that was read goes back to the LDS-DMA at once.
-//   57344 x 8192: 512 rows 306 -> 229 us, 16384 rows 9.07 -> 6.44 ms (2.4 PFLOP/s)
-//   8192 x 28672: 1024 rows 319 -> 196 us, 4096 rows 1230 -> 784; 8192 x 8192: 4096 rows 384 -> 208 (2.6 PFLOP/s)
+// the MFMAs of this step run, and the stage that was read goes back to the LDS-DMA, its pieces spread over the step.
+//   57344 x 8192: 512 rows 306 -> 218 us (gemm_fp8 before), 8640 rows 4.78 -> 3.28 ms (2.5 PFLOP/s; 128-row tiles 3.37)
+//   8192 x 28672: 1200 rows 440 -> 215 us (128-row tiles 354); 8192 x 8192: 700 rows 69 -> 48 (57), 4096 rows 287 -> 203
 // Fragments, steps and slices are gemm_fp8's, so the sums are the same bits.
 // The row and column scales of a unit come through LDS-DMA too, behind its first steps: a plain load would make the
 // epilogue wait for the stages in flight.
@@ -21,9 +21,8 @@ namespace {
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-constexpr int kBM = 128, kBN = 256;   // tile rows, columns
+constexpr int kBN = 256;              // tile columns
 constexpr int kBK = 128;              // K (bytes) per step: one 128-B line per row
-constexpr int kGroupM = 8;            // row tiles that share a W panel before the next one
 constexpr int kMinSteps = 3;          // steps of a unit: its scales have landed when it ends
 
 template <int N>
@@ -39,16 +38,18 @@ __device__ __forceinline__ void mfma_tied(f32x4& acc, const v8i& a, const v8i& b
 
 }  // namespace
 
-template <bool PARTIAL>
+// MI: 32-row blocks of a tile
+template <int MI, bool PARTIAL>
 __global__ void __launch_bounds__(256) gemm_fp8_tile_kernel(const uint8_t* __restrict__ X, const uint8_t* __restrict__ W,
                                                             const float* __restrict__ sx, const float* __restrict__ sw,
                                                             bf16_t* __restrict__ Y, float* __restrict__ P, int M, int N, int K, int S) {
   constexpr int AUX = 16;
-  constexpr int MI = kBM / 32;       // X fragments of a wave = its X pieces per step
+  constexpr int kBM = 32 * MI;       // a wave has MI X fragments and as many X pieces per step
   constexpr int NP = MI + 8;         // LDS-DMA pieces of a wave per step
-  constexpr int NS = 3;              // stages: 144 KiB
+  constexpr int NS = 3;              // stages
+  constexpr int kGroupM = 32 / MI;   // row tiles that share a W panel before the next one
   constexpr int kX = kBM * kBK, kStage = kX + kBN * kBK;
-  constexpr int kScales = NS * kStage, kScaleBytes = (kBM + kBN) * 4;   // sw, then sx; two sets
+  constexpr int kScales = NS * kStage, kScaleBytes = (kBN + 256) * 4;   // sw, then sx; two sets
   __shared__ __attribute__((aligned(1024))) char lds[kScales + 2 * kScaleBytes];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -108,7 +109,7 @@ __global__ void __launch_bounds__(256) gemm_fp8_tile_kernel(const uint8_t* __res
     if (p < 8) dma_(cwp, cwn, vw[p], ck, off + kX, p);
     else dma_(cxp, cxn, vx[p - 8], ck, off, p - 8);
   };
-  // 64 column scales per wave and 64 row scales (the upper waves' copies are the lower ones' again): 2 pieces
+  // 64 column scales per wave and 64 row scales (past the tile's: zeros): 2 pieces
   auto scales = [&](int m0, int n0, int set) {
     char* dst = lds + kScales + set * kScaleBytes;
     const float *swp = sw + n0, *sxp = sx + m0;
@@ -116,8 +117,8 @@ __global__ void __launch_bounds__(256) gemm_fp8_tile_kernel(const uint8_t* __res
     __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)swp, (short)0, swn, 0x00020000),
                                              (__attribute__((address_space(3))) void*)(dst + w * 256), 4, (w * 64 + lane) * 4, 0, 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)sxp, (short)0, sxn, 0x00020000),
-                                             (__attribute__((address_space(3))) void*)(dst + kBN * 4 + wn * 256), 4,
-                                             (wn * 64 + lane) * 4, 0, 0, 0);
+                                             (__attribute__((address_space(3))) void*)(dst + kBN * 4 + w * 256), 4,
+                                             (w * 64 + lane) * 4, 0, 0, 0);
   };
 
   const int l15 = lane & 15, lq = lane >> 4;
@@ -195,8 +196,9 @@ __global__ void __launch_bounds__(256) gemm_fp8_tile_kernel(const uint8_t* __res
           mfma_tied(acc[i][j], wf[j], xf[i]);
           __builtin_amdgcn_sched_barrier(0);
           if (v % 8 == 1) xn[v / 8] = xfrag(nxt, v / 8);
-          else if (i == 3) wf[j] = wfrag(nxt, j);
-          else if (v >= 2 && (v & 1) == 0 && v < 2 + 2 * NP) dma(off, (v - 2) >> 1);
+          if (i == MI - 1) wf[j] = wfrag(nxt, j);
+          const int p = (v * NP + 8 * MI - 1) / (8 * MI);   // a piece every 8 MI / NP MFMAs
+          if (p < NP && p * 8 * MI / NP == v) dma(off, p);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -242,17 +244,26 @@ __global__ void __launch_bounds__(256) gemm_fp8_tile_kernel(const uint8_t* __res
   vm_wait<0>();   // the trailing re-loads land before the workgroup's LDS is released
 }
 
+template <int MI>
+static void launch_fp8(const uint8_t* X, const uint8_t* W, const float* sx, const float* sw, bf16_t* Y, float* P, int M, int N, int K,
+                       int S, int grid, hipStream_t stream) {
+  if (S > 1) gemm_fp8_tile_kernel<MI, true><<<grid, 256, 0, stream>>>(X, W, sx, sw, Y, P, M, N, K, S);
+  else gemm_fp8_tile_kernel<MI, false><<<grid, 256, 0, stream>>>(X, W, sx, sw, Y, P, M, N, K, S);
+}
+
 int gemm_fp8_tile(const uint8_t* X, const uint8_t* W, const float* sx, const float* sw, bf16_t* Y, float* P, int M, int N, int K,
-                  int S, hipStream_t stream) {
+                  int S, int rows, hipStream_t stream) {
   if (M <= 0) return 0;
   if (N < 16 || N % 16 || K % kBK || S < 1 || S > 16 || K / kBK / S < kMinSteps) return -1;
   if (reinterpret_cast<uintptr_t>(X) % 16 || reinterpret_cast<uintptr_t>(W) % 16) return -2;
   if (S > 1 ? P == nullptr : Y == nullptr) return -3;
-  const int64_t units = (int64_t)((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN) * S;
+  if (rows != 96 && rows != 128 && rows != 160) return -5;
+  const int64_t units = (int64_t)((M + rows - 1) / rows) * ((N + kBN - 1) / kBN) * S;
   if (units > (1LL << 30) || (int64_t)K * kBN >= (1LL << 31)) return -4;
   const int grid = (int)min((int64_t)device_cus(), units);
-  if (S > 1) gemm_fp8_tile_kernel<true><<<grid, 256, 0, stream>>>(X, W, sx, sw, Y, P, M, N, K, S);
-  else gemm_fp8_tile_kernel<false><<<grid, 256, 0, stream>>>(X, W, sx, sw, Y, P, M, N, K, S);
+  if (rows == 96) launch_fp8<3>(X, W, sx, sw, Y, P, M, N, K, S, grid, stream);
+  else if (rows == 128) launch_fp8<4>(X, W, sx, sw, Y, P, M, N, K, S, grid, stream);
+  else launch_fp8<5>(X, W, sx, sw, Y, P, M, N, K, S, grid, stream);
   OAMD_LAUNCH_CHECK();
   return S > 1 && Y != nullptr ? splitk_reduce(P, Y, (int64_t)M * N, S, stream) : 0;
 }

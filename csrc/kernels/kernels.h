@@ -79,10 +79,10 @@ int gemm_skinny(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, in
 // FP8 e4m3fn W8A8: Y = (X8 . W8^T) * sx[m] * sw[n]; any M (BM-row tiles), S | 8 split-K.
 int gemm_fp8(const uint8_t* X, const uint8_t* W, const float* sx, const float* sw, bf16_t* Y, float* P, int M,
              int N, int K, int S, int BN, int BM, hipStream_t stream);
-// The same product for prompts on 128 x 256 tiles (gemm_fp8_tile.hip): N % 16 == 0, K % 128 == 0, at least 3 steps of
+// The same product for prompts on tiles of `rows` (96, 128 or 160) x 256 (gemm_fp8_tile.hip): N % 16 == 0, K % 128 == 0, at least 3 steps of
 // 128 in each of S <= 16 slices; fp32 slabs P[S][M][N], then one reduce pass unless Y == nullptr.
 int gemm_fp8_tile(const uint8_t* X, const uint8_t* W, const float* sx, const float* sw, bf16_t* Y, float* P, int M, int N, int K,
-                  int S, hipStream_t stream);
+                  int S, int rows, hipStream_t stream);
 // Per-row dynamic quantization to e4m3fn: sx[m] = max|x[m]| / 448.
 int quantize_fp8_rows(const bf16_t* x, uint8_t* q, float* sx, int M, int K, int64_t ld, hipStream_t stream);
 // Fused SwiGLU + per-row e4m3fn quantization of the 64-feature-interleaved gate|up rows [M, 2 inter]

@@ -812,18 +812,34 @@ def fp8_plan(M: int, N: int, K: int) -> tuple[int, int, int]:
     return _FP8_OVERRIDES.get((N, K)) or _fp8_tiles(M, N, K)[1]
 
 
+# us of a 128-column step of gemm_fp8_tile's tiles of 96, 128 and 160 rows, and what it takes more with every CU busy
+_FP8_ROW_STEP = {96: (0.63, 0.06), 128: (0.66, 0.11), 160: (0.68, 0.25)}
+
+
+@functools.lru_cache(maxsize=4096)
+def fp8_tile_rows(M: int, N: int, K: int, S: int) -> tuple[float, int]:
+    """(estimate in us, rows of the tiles, 256 columns wide) of gemm_fp8_tile: those whose rounds of one workgroup per CU
+    take least, as tile_rows (700 rows of 8192 x 8192: 192 tiles of 128 rows 57 us, 256 of 96 48; 1200 rows of 8192 x 28672: 320
+    tiles of 128 rows 354 us, 256 of 160 215)."""
+    best = None
+    for rows, (one, busy) in _FP8_ROW_STEP.items():
+        units = -(-M // rows) * -(-N // 256) * S
+        full, last = divmod(units, CUS)
+        rounds = full * (one + busy) + (one + busy * last / CUS if last else 0)
+        cost = -(-(K // 128) // S) * rounds + 8 + 3 * (units - 1) // CUS
+        best = min(best or (cost, rows), (cost, rows))
+    return best
+
+
 def fp8_tile_plan(M: int, N: int, K: int) -> int | None:
-    """The slices where gemm_fp8_tile's 128 x 256 tiles are faster than gemm_fp8's, else None: 512 rows of
-    57344 x 8192 306 -> 229 us, 4096 rows of 8192 x 8192 384 -> 208 (2.6 PFLOP/s), 256 rows of 10240 x 8192 57 -> 36; but
-    512 rows of 8192 x 28672 in one slice 187, against 158, and up to 64 rows the weights' stream is all there is
+    """The slices where gemm_fp8_tile is faster than gemm_fp8, whose bits it gives, else None: 512 rows of
+    57344 x 8192 306 -> 218 us, 4096 rows of 8192 x 8192 384 -> 203 (2.7 PFLOP/s), 256 rows of 10240 x 8192 57 -> 33; but
+    512 rows of 8192 x 28672 in one slice 164, against 157, and up to 64 rows the weights' stream is all there is
     (57344 x 8192: 104, against 90)."""
     S = _fp8_slices(M, N, K)[2]
     if M <= 64 or N % 64 or K // 128 // S < 3 or (N, K) in _FP8_OVERRIDES:
         return None
-    units = -(-M // 128) * -(-N // 256) * S
-    step = 0.7 + (0.15 if M > 256 else 0.3) * min(1.0, units / CUS)
-    cost = 6 + -(-units // CUS) * -(-(K // 128) // S) * step
-    return S if cost < _fp8_tiles(M, N, K)[0] else None
+    return S if fp8_tile_rows(M, N, K, S)[0] < _fp8_tiles(M, N, K)[0] else None
 
 
 def linear_fp8(x: torch.Tensor | tuple[torch.Tensor, torch.Tensor], w8: torch.Tensor, sw: torch.Tensor,
@@ -844,7 +860,7 @@ def linear_fp8(x: torch.Tensor | tuple[torch.Tensor, torch.Tensor], w8: torch.Te
             S := fp8_tile_plan(M, N, K)) is not None and (q.data_ptr() | w8.data_ptr()) % 16 == 0:
         part = torch.empty(S * M * N, dtype=torch.float32, device=q.device) if S > 1 else None
         y = None if defer and S > 1 else out if out is not None else torch.empty(M, N, dtype=torch.bfloat16, device=q.device)
-        kernels().gemm_fp8_tile(q, w8, sx, sw, y, part, S)
+        kernels().gemm_fp8_tile(q, w8, sx, sw, y, part, S, rows=fp8_tile_rows(M, N, K, S)[1])
         return SplitK(part, S, M, N) if y is None else y
     bm, bn, S = plan or fp8_plan(M, N, K)
     y = out if out is not None else torch.empty(M, N, dtype=torch.bfloat16, device=q.device)
