@@ -180,14 +180,16 @@ __global__ void __launch_bounds__(256) context_spans_kernel(const uint8_t* __res
 
 int64_t line_prefix_state_words(int64_t n) { return 2 + (n + kLpTile - 1) / kLpTile; }
 
-int line_prefix(const uint32_t* cnt, int64_t n, int64_t* excl, uint64_t* state, hipStream_t stream) {
+int line_prefix(const uint32_t* cnt, int64_t n, int64_t* excl, uint64_t* state, hipStream_t stream, bool zeroed) {
   if (n < 1) return -1;
   const int64_t tiles = (n + kLpTile - 1) / kLpTile;
   if (tiles >= (1ll << 31)) return -2;
   // zero the counter + granules (a multiple of 16 B from the allocation's start)
   const int64_t words = (line_prefix_state_words(n) + 1) & ~1ll;
-  const hipError_t e = hipMemsetAsync(state, 0, words * 8, stream);
-  if (e != hipSuccess) return (int)e;
+  if (!zeroed) {
+    const hipError_t e = hipMemsetAsync(state, 0, words * 8, stream);
+    if (e != hipSuccess) return (int)e;
+  }
   line_prefix_kernel<<<(unsigned)tiles, kLpThreads, 0, stream>>>(cnt, n, excl, state);
   OAMD_LAUNCH_CHECK();
   return 0;

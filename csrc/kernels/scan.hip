@@ -576,7 +576,7 @@ static int num_cus() {
 int ac_scan(const uint8_t* text, int64_t n_segs, int seg_bytes, const uint8_t* cls_map, const uint16_t* table,
             int num_states, int log2_classes, int hot_states, const uint32_t* out_off, const uint32_t* out_ids,
             MatchRec* matches, uint32_t* match_count, uint32_t match_cap, uint32_t* seg_nl, int grid_blocks,
-            const uint16_t* hot_table, const uint8_t* chain, hipStream_t stream) {
+            const uint16_t* hot_table, const uint8_t* chain, hipStream_t stream, bool zeroed) {
   if (n_segs == 0) return 0;
   if (!scan_v1_requested()) {
     if (hot_table == nullptr || chain == nullptr) return -8;
@@ -626,7 +626,7 @@ int ac_scan(const uint8_t* text, int64_t n_segs, int seg_bytes, const uint8_t* c
     int shift = 0;
     while ((1 << shift) < seg_bytes) ++shift;
     // seg_nl holds [n_segs] totals (atomically accumulated) then [n_segs] split-segment heads
-    if (hipMemsetAsync(seg_nl, 0, sizeof(uint32_t) * 2 * n_segs, stream) != hipSuccess) return -5;
+    if (!zeroed && hipMemsetAsync(seg_nl, 0, sizeof(uint32_t) * 2 * n_segs, stream) != hipSuccess) return -5;
     uint32_t* seg_head = seg_nl + n_segs;
     const uint8_t* txt = text;
     const uint16_t* tgp = table;
@@ -668,8 +668,17 @@ int ac_scan(const uint8_t* text, int64_t n_segs, int seg_bytes, const uint8_t* c
 // doc_first_seg[num_docs + 1] = first segment of each doc (last = total).
 __global__ void scan_fixup_kernel(MatchRec* __restrict__ m, const uint32_t* __restrict__ count, uint32_t cap,
                                   const int64_t* __restrict__ nl_excl, const int64_t* __restrict__ doc_first_seg,
-                                  int num_docs, int seg_bytes, const uint32_t* __restrict__ seg_head) {
+                                  int num_docs, int seg_bytes, const uint32_t* __restrict__ seg_head,
+                                  const uint64_t* __restrict__ lp_state, int64_t* __restrict__ report) {
   const uint32_t n = min(*count, cap);
+  if (report != nullptr) {
+    for (int d = blockIdx.x * blockDim.x + threadIdx.x; d < num_docs; d += gridDim.x * blockDim.x)
+      report[d] = nl_excl[doc_first_seg[d + 1]] - nl_excl[doc_first_seg[d]];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      report[num_docs] = *count;
+      report[num_docs + 1] = (int64_t)lp_state[1];
+    }
+  }
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     MatchRec r = m[i];
     const int64_t g = r.x;
@@ -693,10 +702,10 @@ __global__ void scan_fixup_kernel(MatchRec* __restrict__ m, const uint32_t* __re
 
 int scan_fixup(MatchRec* matches, const uint32_t* match_count, uint32_t match_cap, const int64_t* seg_nl_excl,
                const int64_t* doc_first_seg, int num_docs, int seg_bytes, const uint32_t* seg_head,
-               hipStream_t stream) {
+               hipStream_t stream, const uint64_t* lp_state, int64_t* report) {
   if (num_docs == 0 || match_cap == 0) return 0;
   scan_fixup_kernel<<<256, 256, 0, stream>>>(matches, match_count, match_cap, seg_nl_excl, doc_first_seg, num_docs,
-                                            seg_bytes, seg_head);
+                                            seg_bytes, seg_head, lp_state, report);
   OAMD_LAUNCH_CHECK();
   return 0;
 }

@@ -104,6 +104,87 @@ void doc_lines(const at::Tensor& excl, const at::Tensor& first, at::Tensor& doc_
   TORCH_CHECK(rc == 0, "doc_lines launch failed rc=", rc);
 }
 
+// Sizes of a scan's device buffers: bytes of `work` (line_prefix state, match count, newline counts: cleared by one fill;
+// then their prefix), and bytes in front of the first record of `recs`.
+int64_t scan_clear_bytes(int64_t n_segs) { return 8 * ((oamd::line_prefix_state_words(n_segs) + 1) & ~1ll) + 16 + 8 * n_segs; }
+int64_t scan_work_bytes(int64_t n_segs) { return scan_clear_bytes(n_segs) + 8 * (n_segs + 1); }
+int64_t scan_report_bytes(int64_t num_docs) { return (8 * (num_docs + 2) + 15) & ~15ll; }
+
+// Bytes [lo, hi) of the packed text to the GPU, on the current stream.
+void scan_upload(const at::Tensor& text, const at::Tensor& pinned, int64_t lo, int64_t hi) {
+  TORCH_CHECK(text.is_cuda() && !pinned.is_cuda() && text.scalar_type() == at::kByte && pinned.scalar_type() == at::kByte &&
+                  text.is_contiguous() && pinned.is_contiguous(), "scan_upload: contiguous byte buffers, device and host");
+  TORCH_CHECK(lo >= 0 && lo <= hi && hi <= text.numel() && hi <= pinned.numel(), "scan_upload: range");
+  if (lo == hi) return;
+  const c10::hip::HIPGuardMasqueradingAsCUDA g(text.device());
+  const hipError_t e = hipMemcpyAsync(text.data_ptr<uint8_t>() + lo, pinned.data_ptr<uint8_t>() + lo, hi - lo, hipMemcpyHostToDevice,
+                                      c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream());
+  TORCH_CHECK(e == hipSuccess, "scan_upload failed: ", hipGetErrorString(e));
+}
+
+// A whole scan of the uploaded text on the current stream, and its report and first `head` records back in `host`: one
+// fill, the scan, the newline prefix, the records with the line counts, one read-back, one wait. Launches and host
+// calls bound a small scan: as five calls with three fills and two read-backs the analysis of a 64 KiB log took 186 us, as this 113. text: the packed logs, then the layout (first segment
+// per document and the end) at `total`. Returns (matches, line_prefix's error word).
+std::pair<int64_t, int64_t> scan_batch(const at::Tensor& text, int64_t total, int64_t seg_bytes, int64_t num_docs, const at::Tensor& cls_map,
+                                       const at::Tensor& table, int64_t log2_classes, int64_t hot_states, const at::Tensor& out_off,
+                                       const at::Tensor& out_ids, const at::Tensor& hot_table, const at::Tensor& chain,
+                                       int64_t grid_blocks, at::Tensor& work, at::Tensor& recs, int64_t cap, at::Tensor& host, int64_t head) {
+  CHECK_T(text, at::kByte); CHECK_T(cls_map, at::kByte); CHECK_T(table, at::kShort); CHECK_T(out_off, at::kInt); CHECK_T(out_ids, at::kInt);
+  CHECK_T(hot_table, at::kShort); CHECK_T(chain, at::kByte); CHECK_T(work, at::kByte); CHECK_T(recs, at::kByte);
+  TORCH_CHECK(!host.is_cuda() && host.is_contiguous() && host.scalar_type() == at::kByte, "scan_batch: host bytes");
+  TORCH_CHECK(hot_table.numel() == oamd::kScanHotStates * oamd::kScanHotStride, "hot_table must be [256 bytes x 258] (MatchEngine builds it)");
+  TORCH_CHECK(seg_bytes >= 64 && (seg_bytes & (seg_bytes - 1)) == 0, "seg_bytes must be a power of two >= 64");
+  TORCH_CHECK(total >= seg_bytes && total % seg_bytes == 0 && num_docs >= 1, "text must be padded to a multiple of seg_bytes");
+  TORCH_CHECK(text.numel() >= total + 8 * (num_docs + 1), "scan_batch: the layout stands behind the text");
+  TORCH_CHECK(cls_map.numel() == 256, "class map must have 256 entries");
+  const int64_t C = int64_t(1) << log2_classes;
+  TORCH_CHECK(table.dim() == 2 && table.size(1) == C, "table must be [states, 2^log2_classes]");
+  const int64_t S = table.size(0);
+  TORCH_CHECK(S >= 1 && S <= 32768, "DFA must have 1..32768 states");
+  TORCH_CHECK(chain.numel() >= (S + 15) / 16 * 16 + 16, "chain must have round_up(states, 16) + 16 bytes (dfa_chain)");
+  for (const void* a : {chain.data_ptr(), work.data_ptr(), recs.data_ptr(), text.data_ptr()})
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(a) % 16 == 0, "scan_batch: buffers must be 16-byte aligned");
+  TORCH_CHECK(out_off.numel() == S + 1, "out_off must have states+1 entries");
+  TORCH_CHECK(hot_states >= 1 && hot_states <= S && hot_states <= oamd::max_hot_states((int)log2_classes), "hot_states out of range");
+  TORCH_CHECK(((hot_states * C) % 8) == 0, "hot table must be a multiple of 16 bytes");
+  const int64_t n_segs = total / seg_bytes, front = scan_report_bytes(num_docs);
+  TORCH_CHECK(n_segs < (int64_t(1) << 32), "too many segments");
+  TORCH_CHECK(cap >= 1 && cap < (int64_t(1) << 32) && recs.numel() >= front + 16 * cap && work.numel() >= scan_work_bytes(n_segs), "scan_batch: buffers");
+  TORCH_CHECK(head >= 0 && head <= cap && host.numel() >= front + 16 * head, "scan_batch: host buffer");
+  const c10::hip::HIPGuardMasqueradingAsCUDA g(text.device());
+  hipStream_t st = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
+  uint8_t* w = work.data_ptr<uint8_t>();
+  const int64_t clear = scan_clear_bytes(n_segs);
+  uint64_t* state = reinterpret_cast<uint64_t*>(w);
+  uint32_t* seg_nl = reinterpret_cast<uint32_t*>(w + clear - 8 * n_segs);
+  uint32_t* count = reinterpret_cast<uint32_t*>(w + clear - 8 * n_segs - 16);
+  int64_t* excl = reinterpret_cast<int64_t*>(w + clear);
+  const int64_t* first = reinterpret_cast<const int64_t*>(text.data_ptr<uint8_t>() + total);
+  oamd::MatchRec* m = reinterpret_cast<oamd::MatchRec*>(recs.data_ptr<uint8_t>() + front);
+  int64_t* report = reinterpret_cast<int64_t*>(recs.data_ptr<uint8_t>());
+  int rc = (int)hipMemsetAsync(w, 0, clear, st);
+  TORCH_CHECK(rc == 0, "scan_batch: fill failed rc=", rc);
+  rc = oamd::ac_scan(text.data_ptr<uint8_t>(), n_segs, (int)seg_bytes, cls_map.data_ptr<uint8_t>(), reinterpret_cast<const uint16_t*>(table.data_ptr()),
+                     (int)S, (int)log2_classes, (int)hot_states, reinterpret_cast<const uint32_t*>(out_off.data_ptr()),
+                     reinterpret_cast<const uint32_t*>(out_ids.data_ptr()), m, count, (uint32_t)cap, seg_nl, (int)grid_blocks,
+                     reinterpret_cast<const uint16_t*>(hot_table.data_ptr()), chain.data_ptr<uint8_t>(), st, true);
+  TORCH_CHECK(rc == 0, "ac_scan launch failed rc=", rc);
+  rc = oamd::line_prefix(seg_nl, n_segs, excl, state, st, true);
+  TORCH_CHECK(rc == 0, "line_prefix launch failed rc=", rc);
+  rc = oamd::scan_fixup(m, count, (uint32_t)cap, excl, first, (int)num_docs, (int)seg_bytes, seg_nl + n_segs, st, state, report);
+  TORCH_CHECK(rc == 0, "scan_fixup launch failed rc=", rc);
+  uint8_t* h = host.data_ptr<uint8_t>();
+  hipError_t e = hipMemcpyAsync(h, recs.data_ptr<uint8_t>(), front + 16 * head, hipMemcpyDeviceToHost, st);
+  if (e == hipSuccess) {
+    pybind11::gil_scoped_release nogil;
+    e = hipStreamSynchronize(st);
+  }
+  TORCH_CHECK(e == hipSuccess, "scan_batch failed: ", hipGetErrorString(e));
+  const int64_t* r = reinterpret_cast<const int64_t*>(h);
+  return {r[num_docs], r[num_docs + 1]};
+}
+
 void context_spans(const at::Tensor& text, const at::Tensor& doc_base, const at::Tensor& doc_len,
                    const at::Tensor& q, at::Tensor& out) {
   CHECK_T(text, at::kByte);
@@ -164,6 +245,10 @@ PYBIND11_MODULE(_S, m) {
   m.def("context_spans", &context_spans);
   m.def("line_prefix_state_words", [](int64_t n) { return (oamd::line_prefix_state_words(n) + 1) & ~1ll; });
   m.def("ac_scan", &ac_scan);
+  m.def("scan_work_bytes", &scan_work_bytes);
+  m.def("scan_report_bytes", &scan_report_bytes);
+  m.def("scan_upload", &scan_upload);
+  m.def("scan_batch", &scan_batch);
   m.def("score_events", &score_events);
   m.def("scan_fixup", &scan_fixup);
   m.def("max_hot_states", [](int64_t log2c) { return oamd::max_hot_states((int)log2c); });

@@ -7,7 +7,7 @@ GPU path (one call per batch of failures):
   H2D   : one contiguous async copy
   device: ac_scan (DFA walk, LDS hot states) -> per-segment newline counts
           -> line_prefix (decoupled look-back exclusive prefix) -> scan_fixup
-          (doc, factor, line, offset) -> doc_lines (newlines per doc)
+          (doc, factor, line, offset; newlines per doc), launched by one call
   D2H   : the (small) match list
   host  : factor -> matcher expansion, regex verification of candidate lines
           only, native event scoring (or the score_reduce kernel)
@@ -204,12 +204,9 @@ class MatchEngine:
         self._lock = threading.Lock()
         self._pinned: torch.Tensor | None = None
         self._text: torch.Tensor | None = None
-        self._seg_nl: torch.Tensor | None = None
-        self._nl_excl: torch.Tensor | None = None
-        self._meta: torch.Tensor | None = None
-        self._meta_h: torch.Tensor | None = None
+        self._work: torch.Tensor | None = None
         self._head_h: torch.Tensor | None = None
-        self._matches: torch.Tensor | None = None
+        self._recs: torch.Tensor | None = None
         self._doc_newlines: tuple[list[bytes], list[int]] | None = None   # (docs, newlines) of the last GPU scan
         # matcher -> list of (pattern) where it is primary, for quick checks
         self._nm = self.cp.num_matchers
@@ -344,7 +341,7 @@ class MatchEngine:
         from operator_amd.ops import kernels, patterns
         sfx = "" if slot == 0 else f"_s{slot}"
 
-        P = patterns()
+        P, C = patterns(), kernels()
         seg = self.seg_bytes
         # ac_scan v2 cuts the text into (CUs x 1024) equal streams of >= seg bytes: a
         # small batch (a 256-failure flagship wave is 16 MB) gets smaller segments so
@@ -381,52 +378,34 @@ class MatchEngine:
                 self._profile_states(pinned[:min(total, self.profile_bytes, hi)].numpy().tobytes())
             if b == nd:
                 hi += lay
-            text[lo:hi].copy_(pinned[lo:hi], non_blocking=True)
+            C.scan_upload(text, pinned, lo, hi)
             a = b
-        C = kernels()
-        seg_nl = self._ensure("_seg_nl" + sfx, 2 * n_segs, torch.int32)   # totals, then split-segment heads
-        # N3 on the GPU: exclusive newline prefix per segment (decoupled look-back scan),
-        # match records -> (doc, factor, line, offset), newlines per doc
-        excl = self._ensure("_nl_excl" + sfx, n_segs + 1, torch.int64)
-        # what the host reads stands together, and comes back with the first match records in one wait:
-        # newlines per doc, the match count, line_prefix's state (its second word: a look-back timed out)
-        at = (nd + 2) // 2 * 2   # the state is 16-B aligned
-        words = at + C.line_prefix_state_words(n_segs)
-        meta = self._ensure("_meta" + sfx, words, torch.int64)
-        meta_h = self._ensure("_meta_h" + sfx, at + 2, torch.int64, pinned=True)
-        doc_nl, count, lp_state = meta[:nd], meta[at - 1:at].view(torch.int32)[:1], meta[at:words]
-        head_h = self._ensure("_head_h" + sfx, 4 * self.HEAD_MATCHES, torch.int32, pinned=True)
+        work = self._ensure("_work" + sfx, C.scan_work_bytes(n_segs), torch.uint8)
+        # newlines per doc, the match count and an error word stand in front of the match records, and come back with the
+        # first of those in one wait
+        front = C.scan_report_bytes(nd)
         while True:
-            matches = getattr(self, "_matches" + sfx, None)
-            if matches is None or matches.shape[0] < self.match_cap:
-                matches = torch.empty(self.match_cap, 4, dtype=torch.int32, device=self.device)
-                setattr(self, "_matches" + sfx, matches)
-            head = min(self.HEAD_MATCHES, matches.shape[0])
-            count.zero_()
-            C.ac_scan(text[:total], seg, self.cls_map, self.table, self.log2c, self.hot_states, self.out_off,
-                      self.out_ids, matches, count, seg_nl, self.grid_blocks, self.hot_table, self.chain)
-            C.line_prefix(seg_nl[:n_segs], excl, lp_state)
-            C.scan_fixup(matches, count, excl[:n_segs], first_t, seg, seg_nl[n_segs:2 * n_segs])
-            # newlines per doc from the per-segment counts the scan already produced (the
-            # host would otherwise re-read every byte for AnalysisResult.metadata.totalLines)
-            C.doc_lines(excl, first_t, doc_nl)
-            meta_h[:at + 2].copy_(meta[:at + 2], non_blocking=True)
-            head_h[:4 * head].copy_(matches[:head].view(-1), non_blocking=True)
-            torch.cuda.current_stream(self.device).synchronize()
-            cnt = int(meta_h[at - 1:at].view(torch.int32)[0])
-            if int(meta_h[at + 1]) != 0:
+            recs = self._ensure("_recs" + sfx, front + 16 * self.match_cap, torch.uint8)
+            cap = (recs.numel() - front) // 16
+            head = min(self.HEAD_MATCHES, cap)
+            host = self._ensure("_head_h" + sfx, front + 16 * head, torch.uint8, pinned=True)
+            cnt, err = C.scan_batch(text, total, seg, nd, self.cls_map, self.table, self.log2c, self.hot_states, self.out_off,
+                                    self.out_ids, self.hot_table, self.chain, self.grid_blocks, work, recs, cap, host, head)
+            if err:
                 # a line_prefix look-back hit its spin bound: the line numbers of this launch
                 # are wrong, so the batch is recomputed on the host path instead
-                log.warning("line_prefix look-back timed out; rescanning %d docs on the CPU path", len(docs))
+                log.warning("line_prefix look-back timed out; rescanning %d docs on the CPU path", nd)
                 self.stats.gpu_fallbacks += 1
                 return self.scan_cpu(docs), None, None
-            if cnt <= matches.shape[0]:
+            if cnt <= cap:
                 break
             self.match_cap = int(cnt * 1.25) + 1024  # overflow: grow and rescan (rare)
         self.stats.raw_matches += cnt
         self.stats.bytes_scanned += sum(lens)
-        hits = head_h[:4 * cnt].view(-1, 4) if cnt <= head else matches[:cnt].cpu()
-        return hits.numpy().astype(np.int64), (docs, base_t, lens_t, text), (docs, meta_h[:nd].tolist())
+        read = host.numpy()
+        newlines = read[:8 * nd].view(np.int64).tolist()
+        hits = read[front:front + 16 * cnt] if cnt <= head else recs[front:front + 16 * cnt].cpu().numpy()
+        return hits.view(np.int32).reshape(-1, 4).astype(np.int64), (docs, base_t, lens_t, text), (docs, newlines)
 
     def _contexts_gpu(self, docs: list[bytes], q_doc: list[int], q_off: list[int], q_k: list[int],
                       resident: tuple | None = None, stream=None):

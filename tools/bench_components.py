@@ -62,14 +62,15 @@ def bench_scan(n_docs, doc_kb, n_patterns):
     from operator_amd.ops import kernels
     C = kernels()
     seg = eng.last_seg
-    n_segs = eng._text.numel() // seg
     tot_pad = sum(((len(d) + 1 + seg - 1) // seg) * seg for d in docs)
+    matches = torch.empty(eng.match_cap, 4, dtype=torch.int32, device="cuda")
+    count, seg_nl = (torch.empty(n, dtype=torch.int32, device="cuda") for n in (1, 2 * (tot_pad // seg)))
     ev0, ev1 = torch.cuda.Event(True), torch.cuda.Event(True)
     ev0.record()
     for _ in range(5):
-        eng._count.zero_()
+        count.zero_()
         C.ac_scan(eng._text[:tot_pad], seg, eng.cls_map, eng.table, eng.log2c, eng.hot_states, eng.out_off,
-                  eng.out_ids, eng._matches, eng._count, eng._seg_nl, 0, eng.hot_table, eng.chain)
+                  eng.out_ids, matches, count, seg_nl, 0, eng.hot_table, eng.chain)
     ev1.record()
     torch.cuda.synchronize()
     ms = ev0.elapsed_time(ev1) / 5

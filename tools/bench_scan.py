@@ -30,18 +30,20 @@ def kernel_ms(eng, docs, iters):
     tot_pad = sum(((len(d) + 1 + seg - 1) // seg) * seg for d in docs)
     ev0, ev1 = torch.cuda.Event(True), torch.cuda.Event(True)
     with torch.cuda.stream(eng._stream):
+        matches = torch.empty(eng.match_cap, 4, dtype=torch.int32, device="cuda")
+        count, seg_nl = (torch.empty(n, dtype=torch.int32, device="cuda") for n in (1, 2 * (tot_pad // seg)))
         for _ in range(2):
-            eng._count.zero_()
+            count.zero_()
             C.ac_scan(eng._text[:tot_pad], seg, eng.cls_map, eng.table, eng.log2c, eng.hot_states, eng.out_off,
-                      eng.out_ids, eng._matches, eng._count, eng._seg_nl, eng.grid_blocks, eng.hot_table, eng.chain)
+                      eng.out_ids, matches, count, seg_nl, eng.grid_blocks, eng.hot_table, eng.chain)
         ev0.record()
         for _ in range(iters):
-            eng._count.zero_()
+            count.zero_()
             C.ac_scan(eng._text[:tot_pad], seg, eng.cls_map, eng.table, eng.log2c, eng.hot_states, eng.out_off,
-                      eng.out_ids, eng._matches, eng._count, eng._seg_nl, eng.grid_blocks, eng.hot_table, eng.chain)
+                      eng.out_ids, matches, count, seg_nl, eng.grid_blocks, eng.hot_table, eng.chain)
         ev1.record()
     torch.cuda.synchronize()
-    return ev0.elapsed_time(ev1) / iters, tot_pad, int(eng._count.item())
+    return ev0.elapsed_time(ev1) / iters, tot_pad, int(count.item()), matches
 
 
 def main():
@@ -67,15 +69,15 @@ def main():
         eng = MatchEngine(ps, device="cuda", seg_bytes=a.seg, profile_bytes=(1 << 20) if arm == "profiled" else 0)
         raw = eng.scan_gpu(docs)
         torch.cuda.synchronize()
-        ms, tot_pad, cnt = kernel_ms(eng, docs, a.iters)
+        ms, tot_pad, cnt, matches = kernel_ms(eng, docs, a.iters)
         key = sorted(map(tuple, raw.tolist()))
         same = None if ref is None else (key == ref)
         ref = ref or key
         probe_stats = None
         if os.environ.get("OAMD_SCAN_PROBE") in ("4", "5", "6", "7"):
             # per-wave {cycles, slow cycles, slow entries, cold wave-steps} (csrc/kernels/scan.hip)
-            cap = eng._matches.shape[0]
-            w = eng._matches[cap // 2: cap // 2 + 196608].cpu().view(torch.int32).numpy().view("uint32").reshape(-1, 12)
+            cap = matches.shape[0]
+            w = matches[cap // 2: cap // 2 + 196608].cpu().view(torch.int32).numpy().view("uint32").reshape(-1, 12)
             w = w[w[:, 0] > 0].astype("float64")
             probe_stats = {"waves": int(w.shape[0]), "cycles_mean": round(float(w[:, 0].mean())),
                            "cycles_max": round(float(w[:, 0].max())), "slow_cycles_mean": round(float(w[:, 1].mean())),
