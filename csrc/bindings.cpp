@@ -289,7 +289,7 @@ void gemm_decode(const at::Tensor& x, const at::Tensor& w, const c10::optional<a
 
 void gemm_tile(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& y_opt,
                const c10::optional<at::Tensor>& bias, int64_t silu_gu, int64_t variant, int64_t splits,
-               const c10::optional<at::Tensor>& partial) {
+               const c10::optional<at::Tensor>& partial, int64_t rows) {
   CHECK_DEV(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_CONTIG(x); CHECK_CONTIG(w);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2, "x [M,K], w [N,K]");
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
@@ -327,7 +327,7 @@ void gemm_tile(const at::Tensor& x, const at::Tensor& w, const c10::optional<at:
   TORCH_CHECK(M * K < (1LL << 40) && N * K < (1LL << 40) && M < (1LL << 31) && N < (1LL << 31), "gemm too large");
   const c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
   RC(oamd::gemm_tile(ptr<bf16_t>(x), ptr<bf16_t>(w), yp, optr<bf16_t>(bias), (int)M, (int)N, (int)K, (int)ldy,
-                     (int)silu_gu, (int)variant, (int)splits, pp, cur_stream()));
+                     (int)silu_gu, (int)variant, (int)splits, pp, (int)rows, cur_stream()));
 }
 
 void gemm_mid(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& y_opt,
@@ -740,7 +740,7 @@ PYBIND11_MODULE(_C, m) {
         pybind11::arg("rows") = 128);
   m.def("gemm_tile", &gemm_tile, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("y"),
         pybind11::arg("bias") = pybind11::none(), pybind11::arg("silu_gu") = 0, pybind11::arg("variant") = 0,
-        pybind11::arg("splits") = 1, pybind11::arg("partial") = pybind11::none());
+        pybind11::arg("splits") = 1, pybind11::arg("partial") = pybind11::none(), pybind11::arg("rows") = 256);
   m.def("gemm_pp", &gemm_pp, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("y"),
         pybind11::arg("p") = pybind11::none(), pybind11::arg("splits") = 1, pybind11::arg("bm") = 256,
         pybind11::arg("silu_gu") = 0, pybind11::arg("nt") = true, pybind11::arg("one_seg") = false,

@@ -562,7 +562,9 @@ __global__ void __launch_bounds__(256) gemm_tile256_h4_kernel(const bf16_t* __re
 // GRP: routed experts. X's rows are expert segments padded to 256-row tiles (moe_sort): gtab[0] =
 // row tiles, gtab[1 + i] = expert of row tile i, W [experts][N][K]; rscale[row] multiplies both
 // SwiGLU operands (an expert reads its token scaled by the router weight).
-template <int EPI, int DEEP = 0, bool GRP = false>
+// MI: 32-row blocks of a tile (8: 256 rows). 192- and 224-row tiles are for prompts whose last round of 256-row tiles
+// is nearly empty (ops.tile_rows); a step's barriers, piece window and waits scale with its 16 MI MFMAs.
+template <int EPI, int DEEP = 0, bool GRP = false, int MI = 8>
 __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __restrict__ X,
                                                               const bf16_t* __restrict__ W, bf16_t* __restrict__ Y,
                                                               const bf16_t* __restrict__ bias, int M, int N, int K,
@@ -570,22 +572,30 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
                                                               const int* __restrict__ gtab = nullptr,
                                                               const float* __restrict__ rscale = nullptr, GluAct act = {}) {
   constexpr int AUX = 16;
-  constexpr int kHalf = 32768;   // one operand of a K-step: 256 rows x 128 B
-  constexpr int kWin = DEEP ? 128 : 144;   // a step's pieces go out between its MFMA 40 and this one (past 127: of the next step)
+  constexpr int kBM = 32 * MI;
+  constexpr int kHalf = 32768;   // W of a K-step: 256 rows x 128 B
+  constexpr int kXB = kBM * 128;   // X of it
+  constexpr int kH = 8 * MI;       // MFMAs of a k-half
+  constexpr int kB = MI - 3;       // rows of MFMAs in front of a half's barrier; the other three take the next reads
+  constexpr int kTail = kH - 8 * kB;
+  constexpr int kFree = 8 * kB;    // the MFMA of a step behind which its buffers are free
+  constexpr int NP = MI + 8;       // LDS-DMA pieces of a wave per step
+  constexpr int kWin = 2 * kH + (DEEP ? 0 : 16);   // they go out between MFMA kFree and this one (past 2 kH: of the next step)
   constexpr bool kScale = GRP && EPI == kEpiSilu;
-  constexpr int kRs = DEEP ? 5 * kHalf : 4 * kHalf;   // kScale: behind the buffers the scales of each wave's 128 rows
+  constexpr int kRs = 2 * (kXB + kHalf) + (DEEP == 1 ? kXB : DEEP == 2 ? kHalf : 0);   // kScale: behind the buffers the scales of each wave's 128 rows
   static_assert(!kScale || DEEP == 0, "no room for the scales");
+  static_assert(!GRP || MI == 8, "an expert's rows are whole tiles");
   __shared__ __attribute__((aligned(1024))) char lds[kRs + (kScale ? 4 * 512 : 0)];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = w >> 1, wn = w & 1;
-  int mt = (M + kT - 1) / kT;
+  int mt = (M + kBM - 1) / kBM;
   if constexpr (GRP) mt = min(mt, gtab[0]);   // tiles the router really filled
   const int nt = (N + kT - 1) / kT;
   const int ntiles = mt * nt;
   const int G = gridDim.x;
   auto wbase = [&](int m) -> const bf16_t* {   // the weight of row tile m0 / 256's expert
-    if constexpr (GRP) return W + (int64_t)gtab[1 + m / kT] * N * K;
+    if constexpr (GRP) return W + (int64_t)gtab[1 + m / kBM] * N * K;
     else return W;
   };
   const int slot = xcd_remap(blockIdx.x, G);
@@ -597,24 +607,24 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
     if (lid >= ntiles) return false;
     const int first_m = (lid / gsz) * group_m;
     const int gm = min(mt - first_m, group_m);
-    m0 = (first_m + (lid % gsz) % gm) * kT;
+    m0 = (first_m + (lid % gsz) % gm) * kBM;
     n0 = ((lid % gsz) / gm) * kT;
     return true;
   };
   // LDS byte offsets of an operand's buffer for K-step (parity p2 = g & 1, p3 = g % 3)
   auto xoff = [&](int p2, int p3) -> int {
-    if constexpr (DEEP == 0) return p2 * 2 * kHalf;
-    else if constexpr (DEEP == 1) return 2 * kHalf + p3 * kHalf;
-    else return p2 * kHalf;
+    if constexpr (DEEP == 0) return p2 * (kXB + kHalf);
+    else if constexpr (DEEP == 1) return 2 * kHalf + p3 * kXB;
+    else return p2 * kXB;
   };
   auto woff = [&](int p2, int p3) -> int {
-    if constexpr (DEEP == 0) return p2 * 2 * kHalf + kHalf;
-    else if constexpr (DEEP == 2) return 2 * kHalf + p3 * kHalf;
+    if constexpr (DEEP == 0) return p2 * (kXB + kHalf) + kXB;
+    else if constexpr (DEEP == 2) return 2 * kXB + p3 * kHalf;
     else return p2 * kHalf;
   };
   auto swz = [](int row) { return (((row >> 1) & 1) << 1) | (((row >> 3) & 1) << 2); };
 
-  // DMA piece q (0..7) of an operand for wave w = tile rows 8 (w + 4q) .. +7; lane l -> row + l/8,
+  // DMA piece q (0..7; X: 0..MI - 1) of an operand for wave w = tile rows 8 (w + 4q) .. +7; lane l -> row + l/8,
   // LDS slot l % 8, source chunk slot ^ swz(row). Same offsets for X and W (both K wide).
   const int lrow = lane >> 3, lslot = lane & 7;
   uint32_t vo[8];
@@ -633,7 +643,7 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
     int m0 = 0, n0 = 0;
     if (!tile_rc(0, m0, n0)) return;   // grid <= tiles: taken only when GRP has fewer tiles than the bound
     cx.p = X + (int64_t)m0 * K;
-    cx.n = (int)((uint32_t)min(M - m0, kT) * (uint32_t)K * 2u);
+    cx.n = (int)((uint32_t)min(M - m0, kBM) * (uint32_t)K * 2u);
     cw.p = wbase(m0) + (int64_t)n0 * K;
     cw.n = (int)((uint32_t)min(N - n0, kT) * (uint32_t)K * 2u);
   }
@@ -645,7 +655,7 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
         c.kt = 0;
         const int row0 = isx ? m0n : n0n;
         c.p = (isx ? X : wbase(m0n)) + (int64_t)row0 * K;
-        c.n = (int)((uint32_t)min((isx ? M : N) - row0, kT) * (uint32_t)K * 2u);
+        c.n = (int)((uint32_t)min((isx ? M : N) - row0, isx ? kBM : kT) * (uint32_t)K * 2u);
       } else {
         c.kt = T - 1;   // past the block's last tile: harmless re-loads of its last step
       }
@@ -661,14 +671,14 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
   };
   auto dma = [&](const Cur& c, int off, int q) { dma_(c.p, c.n, c.kt, off, q); };
 
-  // fragments: X fragment i = tile rows wm*128 + 16 i + l15; W fragment j (f = j / 4, type =
+  // fragments: X fragment i = tile rows wm*kBM/2 + 16 i + l15; W fragment j (f = j / 4, type =
   // (j / 2) % 2, jj = j % 2) = rows f*128 + type*64 + wn*32 + 8 (l15 / 4) + 4 jj + l15 % 4; k-half h
   // reads chunk 4h + lane/16 of the row at its swizzled slot (swz depends on the lane only)
   const int l15 = lane & 15, lq = lane >> 4;
   const int xs = swz(l15), wr = 8 * (l15 >> 2) + (l15 & 3), ws = swz(wr);
-  const int xo0 = (wm * 128 + l15) * 128 + ((lq ^ xs) << 4), xo1 = (wm * 128 + l15) * 128 + (((4 + lq) ^ xs) << 4);
+  const int xrow = (wm * (kBM / 2) + l15) * 128, xo0 = xrow + ((lq ^ xs) << 4), xo1 = xrow + (((4 + lq) ^ xs) << 4);
   const int wo0 = (wn * 32 + wr) * 128 + ((lq ^ ws) << 4), wo1 = (wn * 32 + wr) * 128 + (((4 + lq) ^ ws) << 4);
-  auto rdx = [&](int off, int h, u16x8 (&xf)[8], int i) {
+  auto rdx = [&](int off, int h, u16x8 (&xf)[MI], int i) {
     xf[i] = *reinterpret_cast<const u16x8*>(lds + off + (h ? xo1 : xo0) + i * 2048);
   };
   auto rdw = [&](int off, int h, u16x8 (&wf)[8], int j) {
@@ -676,19 +686,19 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
     wf[j] = *reinterpret_cast<const u16x8*>(lds + off + (h ? wo1 : wo0) + r * 128);
   };
 
-  f32x4 acc[8][8];
+  f32x4 acc[MI][8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[i][j]));
   asm volatile("s_nop 4");
-  u16x8 xa[8], wa[8], xb[8], wb[8];
+  u16x8 xa[MI], wa[8], xb[MI], wb[8];
   // one MFMA row: 8 MFMAs sharing X fragment u, op(v) after MFMA v
-  auto row = [&](const u16x8 (&xf)[8], const u16x8 (&wf)[8], int u, auto op) {
+  auto row = [&](const u16x8 (&xf)[MI], const u16x8 (&wf)[8], int u, auto op) {
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
       mfma_tied(acc[u][v], wf[v], xf[u]);
@@ -697,42 +707,42 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // what goes out z MFMAs behind the barrier that frees the buffers at ox, ow: piece p of 16, if its turn is z.
+  // what goes out z MFMAs behind the barrier that frees the buffers at ox, ow: piece p of NP, if its turn is z.
   // DEEP == 0: W, then X of step g + 2; DEEP != 0: the shallow operand of step g + 2, the deep one of step g + 3
   auto piece = [&](int z, int ox, int ow) {
-    constexpr int n = kWin - 40;
-    const int p = (z * 16 + n - 1) / n;
-    if (p >= 16 || p * n / 16 != z) return;
-    if ((DEEP == 2) == (p < 8)) dma(cx, ox, p & 7);
-    else dma(cw, ow, p & 7);
-    if (p == 15) {
+    constexpr int n = kWin - kFree, first = DEEP == 2 ? MI : 8;   // DEEP == 2: X goes first, else W
+    const int p = (z * NP + n - 1) / n;
+    if (p >= NP || p * n / NP != z) return;
+    if ((DEEP == 2) == (p < first)) dma(cx, ox, p < first ? p : p - first);
+    else dma(cw, ow, p < first ? p : p - first);
+    if (p == NP - 1) {
       advance(cx, true);
       advance(cw, false);
     }
   };
-  constexpr auto kPieces = [](int z) { return (z * 16 + kWin - 41) / (kWin - 40) < 16 ? (z * 16 + kWin - 41) / (kWin - 40) : 16; };   // gone out before z
+  constexpr auto kPieces = [](int z) { return (z * NP + kWin - kFree - 1) / (kWin - kFree) < NP ? (z * NP + kWin - kFree - 1) / (kWin - kFree) : NP; };   // gone out before z
 
   // prologue: the pieces in the loop's order. The deep operand's step 0, the pieces of a step -2, then as many of
   // step -1's as a step sends before its end; the rest ride on step 0
   if constexpr (DEEP != 0) {
     Cur& cd = DEEP == 1 ? cx : cw;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) dma(cd, DEEP == 1 ? xoff(0, 0) : woff(0, 0), q);
+    for (int q = 0; q < (DEEP == 1 ? MI : 8); ++q) dma(cd, DEEP == 1 ? xoff(0, 0) : woff(0, 0), q);
     advance(cd, DEEP == 1);
   }
-  constexpr int kAhead = DEEP ? 1 : 0;   // steps the deep operand is ahead
+  constexpr int kAhead = DEEP == 0 ? 0 : DEEP == 1 ? MI : 8;   // pieces of the step more that the deep operand is ahead
 #pragma unroll
-  for (int z = 0; z < kWin - 40; ++z)
+  for (int z = 0; z < kWin - kFree; ++z)
     piece(z, DEEP == 1 ? xoff(1, 1) : xoff(0, 0), DEEP == 2 ? woff(1, 1) : woff(0, 0));
   int pox = DEEP == 1 ? xoff(0, 2) : xoff(1, 1), pow = DEEP == 2 ? woff(0, 2) : woff(1, 1);   // buffers of the pieces still to come
 #pragma unroll
-  for (int z = 0; z < 88; ++z) piece(z, pox, pow);
-  vm_wait<kPieces(88) + 8 * kAhead>();   // step 0
+  for (int z = 0; z < 2 * kH - kFree; ++z) piece(z, pox, pow);
+  vm_wait<kPieces(2 * kH - kFree) + kAhead>();   // step 0
   seg_barrier();
 #pragma unroll
   for (int v = 0; v < 8; ++v) rdw(woff(0, 0), 0, wa, v);
 #pragma unroll
-  for (int u = 0; u < 8; ++u) rdx(xoff(0, 0), 0, xa, u);
+  for (int u = 0; u < MI; ++u) rdx(xoff(0, 0), 0, xa, u);
 
   int g = 0, p3 = 0;   // flattened step counter (buffer parity) and g % 3
   int m0 = 0, n0 = 0;
@@ -750,41 +760,41 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
       const int ox = xoff(p2, p3), ow = woff(p2, p3);          // this step's buffers
       const int nox = xoff(n2, n3), now_ = woff(n2, n3);       // step g + 1's
       // ---- segment A: k-half 0 from A; k-half 1 reads (row 0, row 1); this step's buffers released
-      asm volatile("s_waitcnt lgkmcnt(7)" ::: "memory");   // the W fragments + row 0's
+      asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(MI - 1) : "memory");   // the W fragments + row 0's
       __builtin_amdgcn_sched_barrier(0);
       row(xa, wa, 0, [&](int v) {
         rdw(ow, 1, wb, v);
-        piece(88 + v, pox, pow);
+        piece(2 * kH - kFree + v, pox, pow);
       });
-      asm volatile("s_waitcnt lgkmcnt(14)" ::: "memory");  // + row 1's
+      asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(MI + 6) : "memory");  // + row 1's
       __builtin_amdgcn_sched_barrier(0);
       row(xa, wa, 1, [&](int v) {
-        rdx(ox, 1, xb, v);
-        piece(96 + v, pox, pow);
+        if (v < MI) rdx(ox, 1, xb, v);
+        piece(2 * kH - kFree + 8 + v, pox, pow);
       });
-      asm volatile("s_waitcnt lgkmcnt(15)" ::: "memory");  // every k-half-0 read of the step
+      asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(MI + 8 < 15 ? MI + 8 : 15) : "memory");  // every k-half-0 read of the step
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 2; i < 5; ++i) row(xa, wa, i, [](int) {});
+      for (int i = 2; i < kB; ++i) row(xa, wa, i, [](int) {});
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       seg_barrier();   // every wave is done reading this step's buffers
 #pragma unroll
-      for (int i = 5; i < 8; ++i) row(xa, wa, i, [&](int v) { piece((i - 5) * 8 + v, ox, ow); });
+      for (int i = kB; i < MI; ++i) row(xa, wa, i, [&](int v) { piece((i - kB) * 8 + v, ox, ow); });
       // ---- segment B: k-half 1 from B; then step g + 1 lands
 #pragma unroll
-      for (int i = 0; i < 5; ++i) row(xb, wb, i, [&](int v) { piece(24 + i * 8 + v, ox, ow); });
-      vm_wait<kPieces(64) + 8 * kAhead>();   // this wave's pieces of step g + 1
+      for (int i = 0; i < kB; ++i) row(xb, wb, i, [&](int v) { piece(kH - kFree + i * 8 + v, ox, ow); });
+      vm_wait<kPieces(kH) + kAhead>();   // this wave's pieces of step g + 1
       seg_barrier();   // ... every wave's
 #pragma unroll
-      for (int i = 5; i < 8; ++i)
+      for (int i = kB; i < MI; ++i)
         row(xb, wb, i, [&](int v) {
-          const int m = (i - 5) * 8 + v;   // 16 reads on 24 MFMAs: W's 8, then X's
-          if (m % 3 != 2) {
-            const int f = m - m / 3;
+          const int m = (i - kB) * 8 + v;   // NP reads on kTail MFMAs: W's 8, then X's
+          const int f = (m * NP + kTail - 1) / kTail;
+          if (f < NP && f * kTail / NP == m) {
             if (f < 8) rdw(now_, 0, wa, f);
             else rdx(nox, 0, xa, f - 8);
           }
-          piece(64 + m, ox, ow);
+          piece(kH + m, ox, ow);
         });
       pox = ox;
       pow = ow;
@@ -817,8 +827,8 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
             make_uint4(pack_bf2(v0[0], v0[1]), pack_bf2(v0[2], v0[3]), pack_bf2(v1[0], v1[1]), pack_bf2(v1[2], v1[3]));
     };
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int tok = m0 + wm * 128 + i * 16 + l15;
+    for (int i = 0; i < MI; ++i) {
+      const int tok = m0 + wm * (kBM / 2) + i * 16 + l15;
       bf16_t* yrow = Y + (int64_t)tok * ldy;
       float rsc = 1.f;
       if constexpr (kScale) rsc = *reinterpret_cast<const float*>(lds + kRs + w * 512 + (i * 16 + l15) * 4);
@@ -858,7 +868,7 @@ __global__ void __launch_bounds__(256) gemm_tile256_p5_kernel(const bf16_t* __re
       }
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -904,12 +914,12 @@ int splitk_silu(const float* P, bf16_t* Y, int M, int N, int S, int glu, hipStre
   return 0;
 }
 
-template <int DEEP>
+template <int DEEP, int MI = 8>
 static void launch_p5(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, int M, int N, int K, int ldy,
                       int glu, int grid, hipStream_t stream, int gm = kGroupM) {
-  if (glu) gemm_tile256_p5_kernel<kEpiSilu, DEEP><<<grid, 256, 0, stream>>>(X, W, Y, bias, M, N, K, ldy, gm, nullptr, nullptr, glu_act(glu));
-  else if (bias) gemm_tile256_p5_kernel<kEpiBias, DEEP><<<grid, 256, 0, stream>>>(X, W, Y, bias, M, N, K, ldy, gm);
-  else gemm_tile256_p5_kernel<kEpiStore, DEEP><<<grid, 256, 0, stream>>>(X, W, Y, bias, M, N, K, ldy, gm);
+  if (glu) gemm_tile256_p5_kernel<kEpiSilu, DEEP, false, MI><<<grid, 256, 0, stream>>>(X, W, Y, bias, M, N, K, ldy, gm, nullptr, nullptr, glu_act(glu));
+  else if (bias) gemm_tile256_p5_kernel<kEpiBias, DEEP, false, MI><<<grid, 256, 0, stream>>>(X, W, Y, bias, M, N, K, ldy, gm);
+  else gemm_tile256_p5_kernel<kEpiStore, DEEP, false, MI><<<grid, 256, 0, stream>>>(X, W, Y, bias, M, N, K, ldy, gm);
 }
 
 // compute units of the current device (persistent grids), cached per device
@@ -940,12 +950,24 @@ int moe_gemm_tile(const bf16_t* X, const bf16_t* W, bf16_t* Y, int max_rows, int
 }
 
 int gemm_tile(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, int M, int N, int K, int ldy,
-              int glu, int variant, int S, float* P, hipStream_t stream) {
+              int glu, int variant, int S, float* P, int rows, hipStream_t stream) {
   if (M < 1 || N < 16 || N % 16 != 0 || K < kBK || K % kBK != 0) return -1;
   if (glu && (N % 128 != 0 || bias != nullptr)) return -2;
   if (Y != nullptr && ldy < (glu ? N / 2 : N)) return -3;
   if (S < 1 || S > 64 || K % (kBK * S) != 0 || (S > 1 && (P == nullptr || bias != nullptr))) return -5;
   if (Y == nullptr && (S == 1 || glu)) return -6;
+  if (rows != kT) {   // p5 alone has them
+    if ((rows != 192 && rows != 224) || S != 1 || variant != 0 || K < 2 * kBK || ldy % 8 || reinterpret_cast<uintptr_t>(Y) % 16) return -8;
+    const int64_t units = (int64_t)((M + rows - 1) / rows) * ((N + kT - 1) / kT);
+    if (units > (1LL << 30)) return -9;
+    const int grid = (int)min(units, (int64_t)device_cus());
+    if (rows == 192 && N >= 16384) launch_p5<2, 6>(X, W, Y, bias, M, N, K, ldy, glu, grid, stream, 4);
+    else if (rows == 192) launch_p5<0, 6>(X, W, Y, bias, M, N, K, ldy, glu, grid, stream, 4);
+    else if (N >= 16384) launch_p5<2, 7>(X, W, Y, bias, M, N, K, ldy, glu, grid, stream, 4);
+    else launch_p5<0, 7>(X, W, Y, bias, M, N, K, ldy, glu, grid, stream, 4);
+    OAMD_LAUNCH_CHECK();
+    return 0;
+  }
   const int nwg = ((M + kT - 1) / kT) * ((N + kT - 1) / kT);
   if (S > 1) {   // fp32 slabs, then (unless the consumer sums them) one reduce pass
     gemm_tile256_kernel<kEpiPartial><<<dim3(nwg, S), 512, 0, stream>>>(X, W, Y, bias, M, N, K, ldy, P);
@@ -962,11 +984,12 @@ int gemm_tile(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, i
   }
   const bool off32 = (int64_t)M * K * 2 < (1LL << 32) && (int64_t)N * K * 2 < (1LL << 32);
   const bool st16 = ldy % 8 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0;   // p5's 16-B stores
-  // persistent p5 (variant 5; the default past 256 rows): one workgroup per CU; wide N (>= 16384:
+  // persistent p5 (variant 5; the default where its 16-B stores reach): one workgroup per CU (220 rows of 6144 x 4096 77 us,
+  // on the h4 schedule 92; 256 rows of 128256 x 4096 278 and 291); wide N (>= 16384:
   // gate|up, the W panels stream from HBM) gives W a third LDS buffer -- a 2-step prefetch
   // (M = 32k, N = 28672: 5786 -> 5366 us; at N = 4096 / 6144 the 2-buffer form is faster,
   // profiles/gemm_tile_p5_vs_hipblaslt_r6.jsonl)
-  if ((variant == 5 || (variant == 0 && M > kT)) && K >= 2 * kBK && st16) {
+  if ((variant == 5 || variant == 0) && K >= 2 * kBK && st16) {
     const int grid = min(nwg, device_cus());
     // GROUP_M 4 for the narrow projections (M = 32k, N = 6144: 1106 vs 1145 us at GROUP_M 8; N = 4096
     // equal; 16 / 32 slower: profiles/gemm_tile_p5_vs_hipblaslt_r6.jsonl)

@@ -45,7 +45,7 @@ int gemm_decode(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, in
 // S > 1: S-way split-K into fp32 slabs P[S][M][N], then reduced into Y (SwiGLU applied when glu);
 // Y == nullptr leaves the slabs to the consumer (rmsnorm / rope_kv sum them).
 int gemm_tile(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, int M, int N, int K, int ldy,
-              int glu, int variant, int S, float* P, hipStream_t stream);
+              int glu, int variant, int S, float* P, int rows, hipStream_t stream);   // rows: 256, or 192 / 224 (one slice, 16-B aligned Y, ldy % 8 == 0)
 int device_cus();   // compute units of the current device (persistent grids)
 // The same product for few rows on tiles of `rows` (96, 128 or 160) x 256 (gemm_mid.hip), Y 16-B aligned, ldy % 8 == 0, K cut into S <= 16
 // slices: fp32 slabs P[S][M][N], then one reduce pass (ldy = the row's length) unless Y == nullptr. A bias is in the first slab.

@@ -583,8 +583,8 @@ def mid_plan(M: int, N: int, K: int, defer: bool, slices: bool = True, prompt: b
 
 
 # us of a 64-column piece of K on a CU, and what it takes more with every CU busy (power, L2): gemm_mid's tiles of 96, 128
-# and 160 rows, gemm_tile's of 256 (fitted to those products)
-_ROW_STEP = {96: (0.53, 0.16), 128: (0.58, 0.20), 160: (0.70, 0.20), 256: (1.00, 0.38)}
+# and 160 rows, gemm_tile's of 192, 224 and 256 (fitted to those products)
+_ROW_STEP = {96: (0.68, 0.02), 128: (0.70, 0.14), 160: (0.68, 0.32), 192: (0.78, 0.40), 224: (0.90, 0.44), 256: (1.03, 0.48)}
 
 
 def _rows_us(rows: int, M: int, N: int, K: int, S: int) -> float:
@@ -598,12 +598,13 @@ def _rows_us(rows: int, M: int, N: int, K: int, S: int) -> float:
 @functools.lru_cache(maxsize=4096)
 def tile_rows(M: int, N: int, K: int, S: int = 1) -> int:
     """Rows of the tiles (256 columns wide) of a prompt's product in S slices of K: 96, 128 or 160 (gemm_mid) or, in one
-    slice, 256 (gemm_tile). All sum a K slice in the same order, so the bits are the same and the rows are free: those whose
+    slice, 192, 224 or 256 (gemm_tile). All sum a K slice in the same order, so the bits are the same and the rows are free: those whose
     rounds of one workgroup per CU take least. Fewer rows fill the CUs (885 rows of 6144 x 4096: 168 tiles of
     128 rows 55 us, 240 of 96 49), more rows save a round (300 rows of 28672 x 4096: 336 tiles of 128 rows 110 us, 224 of 160 68,
-    224 of 256 95; 1500 rows of 6144 x 4096: 93, 62 and 90) and per product take in fewer bytes (4096 rows of 4096 x
-    14336: 362, 421 and 317). Over 159 products of 16 shapes, 129 to 8000 rows, the estimate's choices take 0.1 % more than
-    the best ones and 5 % less than 128 or 256 rows by the slices' plan alone. Up to 128 rows are one tile."""
+    224 of 256 95; 1500 rows of 6144 x 4096: 93, 62 and 90; 885 rows of 28672 x 4096: 196 us on 160 rows, 182 on 224, 199 on 256;
+    380 rows of it 120 on 128, 82 on 192, 106 on 256) and per product take in fewer bytes (4096 rows of 4096 x
+    14336: 362, 421 and 317). Over 140 products of 7 shapes, 180 to 8000 rows, the estimate's choices take 0.2 % more than
+    the best ones, 2.1 % without the 192 and 224 rows. Up to 128 rows are one tile."""
     if M <= 128:
         return 128
     return min((_rows_us(r, M, N, K, S), r) for r in ((96, 128, 160) if S > 1 else _ROW_STEP))[1]
@@ -621,7 +622,7 @@ def linear_tile(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = Non
     if (out is None or (out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0)) and (
             bias is None or (bias.is_contiguous() and bias.data_ptr() % 16 == 0)):   # gemm_mid's 16-B accesses
         S = mid_plan(M, N, K, defer, out is None or out.stride(0) == out.shape[1], prompt)   # the reduce pass has no row stride
-        if S is not None or (N < LM_HEAD_MIN_N and K >= 128):
+        if K >= 128:
             rows = tile_rows(M, N, K, S or 1)
     part = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if S is not None and S > 1 else None
     opt = {} if rows == 128 else {"rows": rows}
@@ -629,10 +630,10 @@ def linear_tile(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = Non
         kernels().gemm_mid(x, w, None, bias, part, S, **opt)
         return SplitK(part, S, M, N)
     y = out if out is not None else torch.empty(M, N // 2 if glu else N, dtype=x.dtype, device=x.device)
-    if rows < 256:
+    if rows < 192:
         kernels().gemm_mid(x, w, y, bias, part, S or 1, glu, **opt)
     else:
-        kernels().gemm_tile(x, w, y, bias, glu)
+        kernels().gemm_tile(x, w, y, bias, glu, rows=rows)
     return y
 
 

@@ -1,4 +1,4 @@
-"""Tiles of 96, 128, 160 (gemm_mid) and 256 rows (gemm_tile) sum in the same order, so a plan may take whichever is fastest: the same
+"""Tiles of 96, 128, 160 (gemm_mid), 192, 224 and 256 rows (gemm_tile) sum in the same order, so a plan may take whichever is fastest: the same
 bits for every epilogue, at edges of tiles and remainders; and the rule that chooses the rows."""
 import pytest
 import torch
@@ -15,7 +15,7 @@ def _rand(*shape, scale=1.0):
 # one row; a row less and more than a tile of each kind; several rounds of workgroups with a nearly empty last one; the
 # shortest K the 256-row tiles take on their persistent schedule, odd numbers of steps
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(1, 128, 128), (95, 272, 192), (97, 256, 320), (161, 1024, 128), (300, 384, 1024), (321, 4224, 192),
+@pytest.mark.parametrize("M,N,K", [(1, 128, 128), (95, 272, 192), (97, 256, 320), (161, 1024, 128), (193, 528, 192), (225, 384, 320), (300, 384, 1024), (321, 4224, 192),
                                    (885, 6144, 256), (2600, 16384, 128)])
 def test_every_tile_gives_the_same_bits(M, N, K):
     torch.manual_seed(M + N + K)
@@ -32,6 +32,14 @@ def test_every_tile_gives_the_same_bits(M, N, K):
             for rows in (96, 128, 160):
                 C.gemm_mid(x, w, y := new(N // 2), None, None, 1, act, rows=rows)
                 assert torch.equal(y, want), (rows, act)
+    for rows in (192, 224):
+        C.gemm_tile(x, w, want := new(), b, 0, 5)
+        C.gemm_tile(x, w, y := new(), b, rows=rows)
+        assert torch.equal(y, want), rows
+        if N % 128 == 0:
+            C.gemm_tile(x, w, want := new(N // 2), None, ops.SILU, 5)
+            C.gemm_tile(x, w, y := new(N // 2), None, ops.SILU, rows=rows)
+            assert torch.equal(y, want), rows
     S = min(3, K // 64)
     slabs = [torch.full((S, M, N), float("nan"), device=DEV) for _ in range(3)]
     for p, rows in zip(slabs, (96, 128, 160)):
@@ -46,6 +54,6 @@ def test_rows_that_the_kernels_have():
     for N, K in ((16, 128), (272, 192), (4096, 4096), (28672, 4096), (3584, 18944)):
         for M in (1, 128, 129, 300, 885, 4096, 30000):
             assert ops.tile_rows(M, N, K, 2) in (96, 128, 160)
-            assert ops.tile_rows(M, N, K) in (96, 128, 160, 256)
+            assert ops.tile_rows(M, N, K) in (96, 128, 160, 192, 224, 256)
     assert ops.tile_rows(100, 6144, 4096) == 128
     assert [ops.tile_rows(885, 6144, 4096), ops.tile_rows(300, 28672, 4096), ops.tile_rows(28000, 4096, 14336)] == [96, 160, 256]
