@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -26,9 +27,13 @@
 #include <map>
 #include <stdexcept>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <unordered_map>
 #include <vector>
+#if defined(__SSE2__)
+#include <emmintrin.h>
+#endif
 
 namespace py = pybind11;
 
@@ -298,37 +303,110 @@ py::tuple plan_docs(const std::vector<size_t>& lens, int64_t seg) {
   return py::make_tuple(first.back() * seg, first);
 }
 
-// Copy docs into dst (uintptr, >= total bytes) per the plan, zero-filling padding. Multi-threaded.
-void pack_docs(const std::vector<py::bytes>& docs, const std::vector<int64_t>& first, int64_t seg, uintptr_t dst,
-               int threads) {
-  if (first.size() != docs.size() + 1) throw std::invalid_argument("plan/doc count mismatch");
-  std::vector<std::pair<const char*, size_t>> views(docs.size());
-  for (size_t i = 0; i < docs.size(); ++i) {
-    char* p = nullptr;
-    Py_ssize_t n = 0;
-    PyBytes_AsStringAndSize(docs[i].ptr(), &p, &n);
-    views[i] = {p, static_cast<size_t>(n)};
-    if (static_cast<int64_t>(n) + 1 > (first[i + 1] - first[i]) * seg) throw std::invalid_argument("plan too small");
-  }
-  char* out = reinterpret_cast<char*>(dst);
-  auto work = [&](size_t lo, size_t hi) {
-    for (size_t i = lo; i < hi; ++i) {
+// n bytes past the caches (dst 16-B aligned): a buffer that only the GPU reads next, without the read that an ordinary
+// store makes of the line it replaces.
+inline void copy_past_cache(char* d, const char* s, size_t n) {
+#if defined(__SSE2__)
+  for (; n >= 64; n -= 64, d += 64, s += 64)
+    for (int i = 0; i < 64; i += 16)
+      _mm_stream_si128(reinterpret_cast<__m128i*>(d + i), _mm_loadu_si128(reinterpret_cast<const __m128i*>(s + i)));
+  _mm_sfence();   // before the piece counts as done
+#endif
+  std::memcpy(d, s, n);
+}
+
+// Copies docs into dst (uintptr, >= total bytes) per the plan, zero-filling padding, on `threads` threads, the waiting one
+// among them: wait(n) returns once the first n docs are in place, so a caller uploads them while the rest is copied.
+// Pieces of at most kPackPiece bytes are taken in order, so a batch of one long log is split too. dst stays valid
+// until close() (or the destructor), which ends the copying.
+class PackJob {
+ public:
+  PackJob(std::vector<py::bytes> docs, const std::vector<int64_t>& first, int64_t seg, uintptr_t dst, int threads)
+      : docs_(std::move(docs)) {
+    if (first.size() != docs_.size() + 1) throw std::invalid_argument("plan/doc count mismatch");
+    char* out = reinterpret_cast<char*>(dst);
+    size_t total = 0;
+    ends_.reserve(docs_.size() + 1);
+    ends_.push_back(0);
+    for (size_t i = 0; i < docs_.size(); ++i) {
+      char* p = nullptr;
+      Py_ssize_t n = 0;
+      if (PyBytes_AsStringAndSize(docs_[i].ptr(), &p, &n) != 0) throw py::error_already_set();
+      const int64_t cap = (first[i + 1] - first[i]) * seg;
+      if (static_cast<int64_t>(n) + 1 > cap) throw std::invalid_argument("plan too small");
       char* d = out + first[i] * seg;
-      const size_t cap = static_cast<size_t>((first[i + 1] - first[i]) * seg);
-      std::memcpy(d, views[i].first, views[i].second);
-      std::memset(d + views[i].second, 0, cap - views[i].second);
+      for (int64_t o = 0; o < cap; o += kPackPiece) {
+        const int64_t len = std::min(kPackPiece, cap - o), text = std::max<int64_t>(0, std::min<int64_t>(len, n - o));
+        pieces_.push_back({d + o, p + (text ? o : 0), static_cast<size_t>(text), static_cast<size_t>(len - text)});
+      }
+      ends_.push_back(pieces_.size());
+      total += static_cast<size_t>(cap);
     }
-  };
-  py::gil_scoped_release nogil;
-  threads = std::max(1, std::min<int>(threads, static_cast<int>(docs.size())));
-  if (threads == 1) { work(0, docs.size()); return; }
-  std::vector<std::thread> pool;
-  const size_t per = (docs.size() + threads - 1) / threads;
-  for (int t = 0; t < threads; ++t) {
-    const size_t lo = t * per, hi = std::min(docs.size(), lo + per);
-    if (lo < hi) pool.emplace_back(work, lo, hi);
+    past_cache_ = total >= kPastCache && dst % 16 == 0 && seg % 16 == 0;
+    done_ = std::vector<std::atomic<uint8_t>>(pieces_.size());
+    const int more = std::min<int>(threads, static_cast<int>(pieces_.size())) - 1;
+    try {
+      for (int t = 0; t < more; ++t) pool_.emplace_back([this] { while (step()) {} });
+    } catch (const std::system_error&) {   // no more threads to be had: those there are, and the waiting one
+    }
   }
-  for (auto& th : pool) th.join();
+  ~PackJob() { close(); }
+
+  void wait(int64_t n) {
+    if (n < 0 || n >= static_cast<int64_t>(ends_.size())) throw std::out_of_range("PackJob.wait: docs");
+    py::gil_scoped_release nogil;
+    for (const size_t end = ends_[n]; ready_ < end;) {
+      if (done_[ready_].load(std::memory_order_acquire)) ++ready_;
+      else if (closed_) throw std::runtime_error("PackJob.wait: closed");
+      else if (!step()) std::this_thread::yield();   // every piece is taken: some are still being copied
+    }
+  }
+
+  void close() {
+    closed_ = true;
+    next_.store(pieces_.size());
+    if (pool_.empty()) return;
+    py::gil_scoped_release nogil;
+    for (auto& th : pool_) th.join();
+    pool_.clear();
+  }
+
+ private:
+  struct Piece {
+    char* dst;
+    const char* src;
+    size_t text, zeros;
+  };
+  static constexpr int64_t kPackPiece = 256 << 10;
+  // 84 MB in place on the GPU: 1.9 ms past the caches, 2.1 to 2.3 through them; 4.6 MB the same either way
+  static constexpr size_t kPastCache = 8 << 20;
+
+  bool step() {
+    size_t i = next_.load(std::memory_order_relaxed);
+    do {
+      if (i >= pieces_.size()) return false;
+    } while (!next_.compare_exchange_weak(i, i + 1));
+    const Piece& p = pieces_[i];
+    if (past_cache_) copy_past_cache(p.dst, p.src, p.text);
+    else std::memcpy(p.dst, p.src, p.text);
+    std::memset(p.dst + p.text, 0, p.zeros);
+    done_[i].store(1, std::memory_order_release);
+    return true;
+  }
+
+  std::vector<py::bytes> docs_;
+  std::vector<Piece> pieces_;
+  std::vector<size_t> ends_;   // pieces in front of doc i
+  std::vector<std::atomic<uint8_t>> done_;
+  std::atomic<size_t> next_{0};
+  size_t ready_ = 0;           // pieces known to be in place
+  bool past_cache_ = false, closed_ = false;
+  std::vector<std::thread> pool_;
+};
+
+void pack_docs(std::vector<py::bytes> docs, const std::vector<int64_t>& first, int64_t seg, uintptr_t dst, int threads) {
+  const int64_t n = static_cast<int64_t>(docs.size());
+  PackJob(std::move(docs), first, seg, dst, threads).wait(n);
 }
 
 // ---------------------------------------------------------------------------
@@ -464,6 +542,11 @@ PYBIND11_MODULE(_patterns, m) {
   m.def("plan_docs", &plan_docs, py::arg("lens"), py::arg("seg_bytes"));
   m.def("pack_docs", &pack_docs, py::arg("docs"), py::arg("first_seg"), py::arg("seg_bytes"), py::arg("dst"),
         py::arg("threads") = 8);
+  py::class_<PackJob>(m, "PackJob")
+      .def(py::init<std::vector<py::bytes>, const std::vector<int64_t>&, int64_t, uintptr_t, int>(), py::arg("docs"),
+           py::arg("first_seg"), py::arg("seg_bytes"), py::arg("dst"), py::arg("threads") = 8)
+      .def("wait", &PackJob::wait, py::arg("docs"))
+      .def("close", &PackJob::close);
   m.def("score_events", &score_events);
   py::class_<Scorer>(m, "Scorer")
       .def(py::init<const std::vector<int64_t>&, std::vector<double>, std::vector<int64_t>, std::vector<std::vector<int64_t>>,

@@ -21,6 +21,7 @@ CPU path: the same post-processing fed by the pure-Python oracle.
 """
 from __future__ import annotations
 
+import bisect
 import contextlib
 import gc
 import logging
@@ -169,7 +170,7 @@ class MatchEngine:
     # trip; 192: 71 against 86; 768: 323 against 307); larger batches leave the host to the next batch's packing
     HOST_CONTEXT_DOCS = 8
     HEAD_MATCHES = 2048       # match records read back with the count (a 64-log batch has some hundred)
-    PACK_CHUNK = 32 << 20     # host pack / H2D pipelining granule (84 MB: 2.5 ms; 64 MB 2.9, 8 MB 2.8 to 3.8)
+    PACK_CHUNK = 16 << 20     # bytes of an upload while the host packs on (84 MB: 1.9 ms; 4 MB 2.0, 1 MB 2.5)
 
     def __init__(self, patterns: PatternSet | CompiledPatterns, device: str | torch.device = "cuda",
                  seg_bytes: int = 1024, max_events: int = 50, significance: float = 0.5,
@@ -362,24 +363,24 @@ class MatchEngine:
         np.multiply(layout[:nd], seg, out=layout[nd + 1:2 * nd + 1])
         layout[2 * nd + 1:] = lens
         first_t, base_t, lens_t = text[total:total + lay].view(torch.int64).split([nd + 1, nd, nd])
-        # pack and upload in doc-aligned chunks of >= PACK_CHUNK bytes: the host packs
-        # chunk k+1 (native threads) while chunk k's DMA runs, so a large batch pays
-        # max(pack, H2D) rather than the sum (1.2 GB)
-        ptr = pinned.data_ptr()
-        a = 0
-        while a < len(docs):
-            b = a + 1
-            while b < len(docs) and (first[b] - first[a]) * seg < self.PACK_CHUNK:
-                b += 1
-            lo, hi = first[a] * seg, first[b] * seg
-            threads = max(1, min(self.pack_threads, (hi - lo) >> 20))   # ~1 MB per packing thread (4.6 MB: 177 us on one, 93 on four)
-            P.pack_docs(docs[a:b], [f - first[a] for f in first[a:b + 1]], seg, ptr + lo, threads)
-            if self.profile_bytes > 0 and not self._profiled:
-                self._profile_states(pinned[:min(total, self.profile_bytes, hi)].numpy().tobytes())
-            if b == nd:
-                hi += lay
-            C.scan_upload(text, pinned, lo, hi)
-            a = b
+        # native threads pack the whole batch in order, and each doc-aligned chunk of >= PACK_CHUNK bytes is uploaded as soon
+        # as it is in place, so a large batch pays max(pack, H2D) rather than the sum (a batch of 1.2 GB)
+        threads = max(1, min(self.pack_threads, total >> 20))   # ~1 MB per packing thread (4.6 MB: 177 us on one, 93 on four)
+        job = P.PackJob(docs, first, seg, pinned.data_ptr(), threads)
+        try:
+            a = 0
+            while a < nd:
+                b = min(nd, max(a + 1, bisect.bisect_left(first, first[a] + -(-self.PACK_CHUNK // seg), a + 1)))
+                lo, hi = first[a] * seg, first[b] * seg
+                job.wait(b)
+                if self.profile_bytes > 0 and not self._profiled:
+                    self._profile_states(pinned[:min(total, self.profile_bytes, hi)].numpy().tobytes())
+                if b == nd:
+                    hi += lay
+                C.scan_upload(text, pinned, lo, hi)
+                a = b
+        finally:
+            job.close()   # nothing writes into the buffer any more
         work = self._ensure("_work" + sfx, C.scan_work_bytes(n_segs), torch.uint8)
         # newlines per doc, the match count and an error word stand in front of the match records, and come back with the
         # first of those in one wait
