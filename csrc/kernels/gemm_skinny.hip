@@ -5,7 +5,7 @@
 // decode step): the kernel's only job is to keep enough W bytes in flight to
 // run HBM at full rate. Structure (cdna_hip_programming.md §5, row "GEMV /
 // M <= 16 decode weights": straight to VGPRs, deep unroll, no LDS round trip):
-//   * a block owns a 16-row tile of W (two for the fused SwiGLU: the gate rows
+//   * a block owns one, two or four 16-row tiles of W (skinny_tiles; for the fused SwiGLU gate rows
 //     and the matching up rows 64 rows later) and its 4 waves split K;
 //   * each wave streams its K range in 32-deep steps: lane l loads 16 B of W
 //     row (l & 15) at k = 8 (l >> 4) -- exactly the A-fragment of
@@ -29,28 +29,31 @@ typedef __bf16 bf16x8s_t __attribute__((ext_vector_type(8)));
 namespace sk {
 constexpr int kWaves = 4;
 constexpr int kThreads = kWaves * 64;
-constexpr int kU = 8;  // k-steps (32 deep) in flight per wave
 enum { kStore = 0, kPartial = 1, kSilu = 2 };
 }  // namespace sk
 
-// NT = W tiles per block (2 for SwiGLU: gate + up), MT = 16-column X tiles (M <= 16 * MT).
-template <int NT, int MT, int EPI>
+// NT: 16-row W tiles of a block (for SwiGLU in pairs of gate and up rows), MT: 16-column X tiles (M <= 16 * MT), U: k-steps in
+// flight per wave.
+template <int NT, int MT, int EPI, int U>
 __global__ void __launch_bounds__(sk::kThreads) gemm_skinny_kernel(const bf16_t* __restrict__ X,
                                                                  const bf16_t* __restrict__ W,
                                                                  bf16_t* __restrict__ Y, float* __restrict__ P,
                                                                  int M, int N, int K, int S, GluAct act = {}) {
+  constexpr int NO = EPI == sk::kSilu ? NT / 2 : NT;   // output tiles
   __shared__ float red[sk::kWaves][NT * MT][64 * 4];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = tid >> 6;
   const int r = lane & 15, kq = lane >> 4;
-  // W rows of this block's tile(s)
+  // W rows of this block's tiles; SwiGLU: 16-row slices of the gate half of a 128-row group, then of its up half
   int rows[NT];
-  if constexpr (EPI == sk::kSilu) {
-    const int g = blockIdx.x >> 2, sub = blockIdx.x & 3;  // 128-row gate|up group, 16-row slice
-    rows[0] = g * 128 + sub * 16;
-    rows[NT - 1] = g * 128 + 64 + sub * 16;
-  } else {
-    rows[0] = blockIdx.x * 16;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    if constexpr (EPI == sk::kSilu) {
+      const int sub = blockIdx.x * NO + t % NO;
+      rows[t] = (sub >> 2) * 128 + (t / NO) * 64 + (sub & 3) * 16;
+    } else {
+      rows[t] = (blockIdx.x * NT + t) * 16;
+    }
   }
   const int kz = blockIdx.y;
   const int Kb = K / S;             // this block's K range
@@ -77,17 +80,17 @@ __global__ void __launch_bounds__(sk::kThreads) gemm_skinny_kernel(const bf16_t*
 
   const u16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
   int s = 0;
-  for (; s + sk::kU <= steps; s += sk::kU) {
-    u16x8 a[sk::kU][NT], b[sk::kU][MT];
+  for (; s + U <= steps; s += U) {
+    u16x8 a[U][NT], b[U][MT];
 #pragma unroll
-    for (int u = 0; u < sk::kU; ++u) {
+    for (int u = 0; u < U; ++u) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) a[u][t] = __builtin_nontemporal_load(wp[t] + (s + u) * 4);
 #pragma unroll
       for (int j = 0; j < MT; ++j) b[u][j] = xv[j] ? xp[j][(s + u) * 4] : zero;
     }
 #pragma unroll
-    for (int u = 0; u < sk::kU; ++u)
+    for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -96,7 +99,7 @@ __global__ void __launch_bounds__(sk::kThreads) gemm_skinny_kernel(const bf16_t*
                                                               __builtin_bit_cast(bf16x8s_t, b[u][j]), acc[t][j], 0, 0,
                                                               0);
   }
-  for (; s < steps; ++s) {  // remainder (< kU steps)
+  for (; s < steps; ++s) {  // remainder (< U steps)
     u16x8 a[NT], b[MT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) a[t] = __builtin_nontemporal_load(wp[t] + s * 4);
@@ -118,31 +121,66 @@ __global__ void __launch_bounds__(sk::kThreads) gemm_skinny_kernel(const bf16_t*
 #pragma unroll
       for (int i = 0; i < 4; ++i) red[w][t * MT + j][i * 64 + lane] = acc[t][j][i];
   __syncthreads();
-  // thread -> (tile pair j, element e): 64 lanes x 4 regs per tile
-  for (int e = tid; e < MT * 256; e += sk::kThreads) {
-    const int j = e >> 8, i = (e >> 6) & 3, l = e & 63;
+  // thread -> (output tile, X tile j, element e): 64 lanes x 4 regs per tile
+  for (int e = tid; e < NO * MT * 256; e += sk::kThreads) {
+    const int t = e / (MT * 256), j = (e >> 8) % MT, i = (e >> 6) & 3, l = e & 63;
     const int m = j * 16 + (l & 15);
     const int rr = 4 * (l >> 4) + i;  // row within the 16-row tile
-    float v[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      v[t] = 0.f;
-#pragma unroll
-      for (int ww = 0; ww < sk::kWaves; ++ww) v[t] += red[ww][t * MT + j][i * 64 + l];
-    }
     if (m >= M) continue;
+    auto sum = [&](int tile) {
+      float v = 0.f;
+#pragma unroll
+      for (int ww = 0; ww < sk::kWaves; ++ww) v += red[ww][tile * MT + j][i * 64 + l];
+      return v;
+    };
     if constexpr (EPI == sk::kSilu) {
-      const float g = bf2f(f2bf(v[0]));
-      const float u = bf2f(f2bf(v[NT - 1]));
+      const float g = bf2f(f2bf(sum(t)));
+      const float u = bf2f(f2bf(sum(NO + t)));
       const float sg = bf2f(f2bf(glu_gate(g, act)));
-      const int f = (blockIdx.x >> 2) * 64 + (blockIdx.x & 3) * 16 + rr;
+      const int f = (blockIdx.x * NO + t) * 16 + rr;
       Y[(int64_t)m * (N / 2) + f] = f2bf(sg * u);
     } else if constexpr (EPI == sk::kPartial) {
-      P[((int64_t)kz * M + m) * N + rows[0] + rr] = v[0];
+      P[((int64_t)kz * M + m) * N + (blockIdx.x * NT + t) * 16 + rr] = sum(t);
     } else {
-      Y[(int64_t)m * N + rows[0] + rr] = f2bf(v[0]);
+      Y[(int64_t)m * N + (blockIdx.x * NT + t) * 16 + rr] = f2bf(sum(t));
     }
   }
+}
+
+template <int NT, int U>
+static void launch_skinny(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, int N, int K, int S, int glu,
+                          hipStream_t stream) {
+  const dim3 grid(N / (16 * NT), S);
+  if (glu) {
+    if constexpr (NT > 1) {
+      if (M <= 16) gemm_skinny_kernel<NT, 1, sk::kSilu, U><<<grid, sk::kThreads, 0, stream>>>(X, W, Y, P, M, N, K, 1, glu_act(glu));
+      else gemm_skinny_kernel<NT, 2, sk::kSilu, U><<<grid, sk::kThreads, 0, stream>>>(X, W, Y, P, M, N, K, 1, glu_act(glu));
+    }
+  } else if (S > 1) {
+    if (M <= 16) gemm_skinny_kernel<NT, 1, sk::kPartial, U><<<grid, sk::kThreads, 0, stream>>>(X, W, Y, P, M, N, K, S);
+    else gemm_skinny_kernel<NT, 2, sk::kPartial, U><<<grid, sk::kThreads, 0, stream>>>(X, W, Y, P, M, N, K, S);
+  } else {
+    if (M <= 16) gemm_skinny_kernel<NT, 1, sk::kStore, U><<<grid, sk::kThreads, 0, stream>>>(X, W, Y, P, M, N, K, 1);
+    else gemm_skinny_kernel<NT, 2, sk::kStore, U><<<grid, sk::kThreads, 0, stream>>>(X, W, Y, P, M, N, K, 1);
+  }
+}
+
+// 16-row W tiles of a workgroup. It reads the X rows of its K range once for all of them, and a CU takes in X and W at the same rate:
+// 32 rows of 128256 x 4096 429 us on one tile, 345 on two, 304 on four; 16 rows of 4096 x 14336 in 2 slices 38 on one, 30 on two
+// (256 workgroups), 48 on four (128: half the CUs idle). So the tiles whose rounds of one workgroup per CU take in the fewest rows;
+// more tiles stream a little worse (one row of the vocabulary 196 on one, 203 and 252). Over 189 products of 12 shapes, 1 to 32 rows, the choices take
+// 1 % more than the best ones and 7 % less than one tile. The sums' order is the same on any.
+constexpr int kCus = 256;
+static int skinny_tiles(int M, int N, int Kb, int S, int glu) {
+  int best = 0;
+  double least = 0;
+  for (int nt = glu ? 2 : 1; nt <= 4; nt *= 2) {
+    if (N % (16 * nt)) break;
+    const int rounds = (N / (16 * nt) * S + kCus - 1) / kCus;
+    const double cost = rounds * ((16.0 * nt * (nt == 4 ? 1.15 : 1.0) + 0.8 * M) * Kb + (nt == 2 && !glu ? 3300 : 0));
+    if (best == 0 || cost < least) best = nt, least = cost;
+  }
+  return best;
 }
 
 int gemm_skinny(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, int N, int K, int S, int glu,
@@ -152,21 +190,14 @@ int gemm_skinny(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, in
   if (glu && (S != 1 || N % 128 != 0)) return -3;
   if (N % 16 != 0) return -4;
   if (S > 1 && P == nullptr) return -5;
-  const int MT = M <= 16 ? 1 : 2;
-  if (glu) {
-    const dim3 grid(N / 32, 1);  // one block per (16 gate rows, 16 up rows)
-    if (MT == 1) gemm_skinny_kernel<2, 1, sk::kSilu><<<grid, sk::kThreads, 0, stream>>>(X, W, Y, P, M, N, K, 1, glu_act(glu));
-    else gemm_skinny_kernel<2, 2, sk::kSilu><<<grid, sk::kThreads, 0, stream>>>(X, W, Y, P, M, N, K, 1, glu_act(glu));
-  } else {
-    const dim3 grid(N / 16, S);
-    if (S > 1) {
-      if (MT == 1) gemm_skinny_kernel<1, 1, sk::kPartial><<<grid, sk::kThreads, 0, stream>>>(X, W, Y, P, M, N, K, S);
-      else gemm_skinny_kernel<1, 2, sk::kPartial><<<grid, sk::kThreads, 0, stream>>>(X, W, Y, P, M, N, K, S);
-    } else {
-      if (MT == 1) gemm_skinny_kernel<1, 1, sk::kStore><<<grid, sk::kThreads, 0, stream>>>(X, W, Y, P, M, N, K, 1);
-      else gemm_skinny_kernel<1, 2, sk::kStore><<<grid, sk::kThreads, 0, stream>>>(X, W, Y, P, M, N, K, 1);
-    }
-  }
+  const int nt = skinny_tiles(M, N, K / S, S, glu), steps = K / S / (sk::kWaves * 32), rounds = (N / (16 * nt) * S + kCus - 1) / kCus;
+  // k-steps in flight: long streams of many rounds take more (128256 x 4096, one row: 16 steps 191 us, 8 196; 8 rows on two tiles: 8 steps
+  // 222, 4 226), but never a remainder, whose steps wait one by one
+  if (nt == 4) launch_skinny<4, 2>(X, W, Y, P, M, N, K, S, glu, stream);
+  else if (nt == 2 && steps % 8 == 0 && (glu || rounds >= 4)) launch_skinny<2, 8>(X, W, Y, P, M, N, K, S, glu, stream);
+  else if (nt == 2) launch_skinny<2, 4>(X, W, Y, P, M, N, K, S, glu, stream);
+  else if (steps % 16 == 0 && rounds >= 4) launch_skinny<1, 16>(X, W, Y, P, M, N, K, S, glu, stream);
+  else launch_skinny<1, 8>(X, W, Y, P, M, N, K, S, glu, stream);
   OAMD_LAUNCH_CHECK();
   if (S > 1 && Y != nullptr) {  // Y == nullptr: the consumer sums the slabs
     const int64_t MN = (int64_t)M * N;

@@ -465,10 +465,11 @@ def skinny_plan(M: int, N: int, K: int) -> int | None:
 
 
 def _mid_beats_skinny(M: int, N: int, K: int, defer: bool) -> bool:
-    """gemm_skinny streams the weights once per call but pays for every row (a 128256 x 4096 vocabulary: 186 us at
-    1 row, 238 at 8, 428 at 32; 4 % of the one-row time per row at every measured shape); gemm_mid's 128-row
-    tile costs the same at any of them (217 us). A few rows of a projection stay: too little work to split. So do shapes
-    with a measured entry (32 rows of 4096 x 4096: 15.5 us against 17.6 in slices).
+    """gemm_skinny streams the weights once per call but pays for every row (a 128256 x 4096 vocabulary: 191 us at
+    1 row, 222 at 8, 300 at 32; 4096 x 14336 26, 27 and 38: 2 % of the one-row time per row, 4 where its tiles do not come in
+    whole rounds, which is what the estimate takes); gemm_mid's 128-row tile costs the same at any of them (217 us; 25).
+    A few rows of a projection stay: the consumer of up to 16 slabs waits longer than is gained (16 rows of 4096 x 14336: 30
+    against 25 before the slabs are read). So do shapes with a measured entry.
 
     Few rows stream the weights at 5.3 to 5.8 TB/s, rows of 2048 or 4096 columns (a power of two: neighbouring rows
     share memory channels) at 4.1 to 4.8: vocabularies of 32768 x 4096, 5 rows 55 us against 66, of 128256 x 3072 176
