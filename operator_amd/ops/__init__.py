@@ -123,17 +123,17 @@ def _gu_splits(M: int, N: int, K: int, bm: int = 0) -> int:
 
 
 def gate_up_plan(M: int, N: int):
-    """Kernel of a gate|up decode bucket of 64 to 256 rows without a measured entry: row tile of gemm_decode, "pp256" /
-    "pp128" (gemm_pp) or None (gemm_mid). A workgroup takes in about 45 bytes per ns of both operands, so the
+    """Kernel of a gate|up decode bucket of 64 to 256 rows without a measured entry: row tile of gemm_decode, "pp256"
+    (gemm_pp) or None (gemm_mid). A workgroup takes in about 45 bytes per ns of both operands, so the
     smallest tile that still leaves one workgroup per CU wins (256 rows of 16384 x 2048: two 128-row tiles 28 us,
-    one of 256 38; 128 rows of it: 64-row tiles 22 us, 128 25), then the one whose workgroups come in one round
-    (128 rows of 57344 x 8192: gemm_mid's 224 units 179 us, gemm_pp 217). 256 rows stay on gemm_pp: gemm_mid's W
+    one of 256 38; 128 rows of it: 64-row tiles 22 us, 128 25; of 28672 x 4096 128-row tiles 58, gemm_pp's 61), then the one whose
+    workgroups come in one round (128 rows of 57344 x 8192: gemm_mid's 224 units 179 us, gemm_pp 217). 256 rows stay on gemm_pp: gemm_mid's W
     tile goes to two CUs (28672 x 4096 by itself 70 us against 78, but 12 us behind within a decode step)."""
     tiles = N // 128
     if M == 64:
         return 64
     if M == 128:
-        return 64 if 2 * tiles <= CUS else "pp128" if tiles <= CUS else None
+        return 64 if 2 * tiles <= CUS else 128 if tiles <= CUS else None
     if M == 256:
         return 128 if 2 * tiles <= CUS else "pp256"
     return 64 if M // 64 * tiles <= CUS else None
@@ -172,7 +172,8 @@ def gate_up_silu(x: torch.Tensor, wgu: torch.Tensor, block: int | None, act: int
             kernels().splitk_silu(slabs, y, S, act)
             return y
         if t != "blas":
-            ns = t[1] if t and len(t) > 1 else 3
+            # one workgroup of 64-row tiles per CU: a fourth stage (64 rows of 28672 x 4096: 52 us on three, 49), two keep theirs in LDS on three
+            ns = t[1] if t and len(t) > 1 else 4 if bm == 64 and M // 64 * (N // 128) <= CUS else 3
             y = torch.empty(M, N // 2, dtype=x.dtype, device=x.device)
             kernels().gemm_decode(x, wgu, y, None, 1, 128, bm, act, False, ns)
             return y
