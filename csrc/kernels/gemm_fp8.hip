@@ -10,7 +10,7 @@
 //   bf16 16x16x32 form at 2x its cycles — twice the bf16 MFMA rate — and half
 //   the bytes per weight, which is what decode (weight-streaming) needs.
 // * Same pipeline as gemm.hip: LDS-DMA (global_load_lds_dwordx4) of full
-//   128-B lines (= 128 K-elements per row) into a 3-deep ring, counted vmcnt,
+//   128-B lines (= 128 K-elements per row) into a ring of NS stages, counted vmcnt,
 //   raw s_barrier, split-K slabs for narrow N, M tiles of BM rows. Rows past M
 //   are clamped duplicates on load and skipped on store, so any M works.
 // * Fragment read = 32 K-bytes per lane (two ds_read_b128 of chunks 2g, 2g+1).
@@ -28,17 +28,22 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 namespace f8 {
 
 constexpr int kBK = 128;  // K elements (bytes) per stage: one 128-B line per row
-constexpr int kStages = 3;
 constexpr int kWaves = 8;
+constexpr int kCus = 256;
 
-template <int BM, int BN>
+// NS stages, all but one in flight. A workgroup that has its CU to itself streams at what it keeps in flight (64 x 64 tiles on
+// three stages: 32 KiB per microsecond of latency, 31 B per ns), so narrow products of one workgroup per CU and long slices
+// take a ring of 128 or 144 KiB: 64 rows of 8192 x 28672 58 -> 50 us, 1 row 54 -> 41, 64 rows of 4096 x 14336 16 -> 15, 128 rows of
+// 8192 x 28672 62 -> 60. Slices of eight steps lose by it (64 rows of 4096 x 4096 7.8 -> 8.4 us), and so do two workgroups per CU on
+// five stages (10240 x 8192 26.0 -> 26.7) and wider tiles on more than three.
+template <int BM, int BN, int NS>
 struct Cfg {
   static constexpr int WM = 4, WN = kWaves / WM;
   static constexpr int FM = BM / WM / 16, FN = BN / WN / 16;
   static constexpr int ROWS = BM + BN;
   static constexpr int STAGE_BYTES = ROWS * kBK;
   static constexpr int GL = ROWS / 8 / kWaves;
-  static constexpr int LDS_BYTES = kStages * STAGE_BYTES;
+  static constexpr int LDS_BYTES = NS * STAGE_BYTES;
   static_assert(ROWS % (8 * kWaves) == 0, "stage rows must split evenly over the waves");
 };
 
@@ -51,14 +56,25 @@ __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// `later` of at most N stages of GL pieces may still be in flight
+template <int GL, int N>
+__device__ __forceinline__ void wait_stages(int later) {
+  if constexpr (N == 0) {
+    wait_vmcnt<0>();
+  } else {
+    if (later >= N) wait_vmcnt<GL * N>();
+    else wait_stages<GL, N - 1>(later);
+  }
+}
+
 }  // namespace f8
 
-template <int BM, int BN, bool PARTIAL>
+template <int BM, int BN, bool PARTIAL, int NS>
 __global__ void __launch_bounds__(f8::kWaves * 64, 1)
     gemm_fp8_kernel(const uint8_t* __restrict__ X, const uint8_t* __restrict__ W, const float* __restrict__ sx,
                     const float* __restrict__ sw, bf16_t* __restrict__ Y, float* __restrict__ P, int M, int N, int K,
                     int S, int wnt) {
-  using C = f8::Cfg<BM, BN>;
+  using C = f8::Cfg<BM, BN, NS>;
   __shared__ __attribute__((aligned(1024))) char lds[C::LDS_BYTES];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -112,16 +128,17 @@ __global__ void __launch_bounds__(f8::kWaves * 64, 1)
         acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[i], b[j], acc[i][j], 0, 0, 0, 127, 0, 127);
   };
 
-  issue(0, 0);
-  if (T > 1) issue(1, 1);
+  for (int t = 0; t < min(NS - 1, T); ++t) issue(t, t);
+  int buf = 0, free_ = NS - 1;   // this step's stage; the one of the step before it
   for (int t = 0; t < T; ++t) {
-    if (t + 1 < T) f8::wait_vmcnt<C::GL>();
-    else f8::wait_vmcnt<0>();
+    f8::wait_stages<C::GL, NS - 2>(T - 1 - t);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (t + 2 < T) issue(t + 2, (t + 2) % f8::kStages);
-    compute(t % f8::kStages);
+    if (t + NS - 1 < T) issue(t + NS - 1, free_);
+    compute(buf);
+    free_ = buf;
+    buf = buf + 1 == NS ? 0 : buf + 1;
   }
 
 #pragma unroll
@@ -334,18 +351,24 @@ int gemm_fp8(const uint8_t* X, const uint8_t* W, const float* sx, const float* s
   if (S > 1 && P == nullptr) return -4;
   const dim3 grid((N / BN) * S, (M + BM - 1) / BM);
   static const int wnt = [] { const char* e = getenv("OAMD_FP8_WNT"); return e && e[0] == '0' ? 0 : 1; }();
-#define OAMD_G8(BMM, BNN)                                                                                     \
-  if (S > 1)                                                                                                  \
-    gemm_fp8_kernel<BMM, BNN, true><<<grid, f8::kWaves * 64, 0, stream>>>(X, W, sx, sw, Y, P, M, N, K, S, wnt); \
-  else gemm_fp8_kernel<BMM, BNN, false><<<grid, f8::kWaves * 64, 0, stream>>>(X, W, sx, sw, Y, P, M, N, K, S, wnt)
-#define OAMD_G8M(BMM) \
-  if (BN == 64) { OAMD_G8(BMM, 64); } else { OAMD_G8(BMM, 128); }
-  switch (BM) {
-    case 64: OAMD_G8M(64); break;
-    case 128: OAMD_G8M(128); break;
-    default: OAMD_G8M(256); break;
+  const bool deep = (int64_t)grid.x * grid.y <= f8::kCus && K / f8::kBK / S >= 24;
+#define OAMD_G8(BMM, BNN, NS)                                                                                       \
+  if (S > 1)                                                                                                        \
+    gemm_fp8_kernel<BMM, BNN, true, NS><<<grid, f8::kWaves * 64, 0, stream>>>(X, W, sx, sw, Y, P, M, N, K, S, wnt); \
+  else gemm_fp8_kernel<BMM, BNN, false, NS><<<grid, f8::kWaves * 64, 0, stream>>>(X, W, sx, sw, Y, P, M, N, K, S, wnt)
+  if (BM == 64 && BN == 64) {
+    if (deep) { OAMD_G8(64, 64, 8); } else { OAMD_G8(64, 64, 3); }
+  } else if (BM == 64) {
+    OAMD_G8(64, 128, 3);
+  } else if (BM == 128 && BN == 64) {
+    if (deep) { OAMD_G8(128, 64, 6); } else { OAMD_G8(128, 64, 3); }
+  } else if (BM == 128) {
+    OAMD_G8(128, 128, 3);
+  } else if (BN == 64) {
+    OAMD_G8(256, 64, 3);
+  } else {
+    OAMD_G8(256, 128, 3);
   }
-#undef OAMD_G8M
 #undef OAMD_G8
   OAMD_LAUNCH_CHECK();
   if (S > 1 && Y != nullptr) {   // Y == nullptr: the consumer sums the slabs
