@@ -403,22 +403,32 @@ __device__ __forceinline__ float lanes_sum(float v) {
 }  // namespace
 
 // Prefill: a workgroup is 64 query rows of one sequence and head, a wave 16 of them; 32-key tiles of K and V
-// are shared through LDS (rows padded by 16 B) and the next tile's loads are in flight while one is used.
-// What bounds it: the fp32 MFMA rate of the workgroups with the longest rows (2 x 500 rows of 16 heads of 128: 866 us
-// with a row per workgroup on FMA, 72 here; 2018 rows 3956 -> 243).
+// are shared through LDS (rows padded by 16 B) and the next tile's loads are in flight while one is used. Two groups of four waves
+// take tiles in turn, each with sums of its own, which meet in LDS at the end: a short prompt has one workgroup per CU, whose softmax
+// would leave the matrix cores idle, and whose longest rows bound the launch.
+// What bounds it: the workgroups with the longest rows, whose 32-key tile is 1.7 us of fp32 MFMAs and about as much of softmax, staging and
+// barriers. With one group 2 x 500 rows of 16 heads of 128 took 75 us, with two 60; 200 rows 34 -> 28, 1000 rows of 8 heads of 256
+// 279 -> 204, 2018 rows of 16 heads 404 -> 402; 32 x 64 rows, where the second group has nothing to do half of the time, 24 -> 28. One group for those
+// would make a prompt's rounding depend on what it is packed with. The products run over all D columns (zeros past the heads):
+// a way out per 16 columns kept each block's reads behind the block before.
 // D: instantiated size >= both head sizes. ODD: value heads that are no multiple of 16 columns, or output rows that take no
 // 16-B stores (key heads are multiples of 4 in either form).
 template <int D, bool ODD>
-__global__ void __launch_bounds__(256) attn_f32_prefill_kernel(const AttnF32 a) {
+__global__ void __launch_bounds__(512) attn_f32_prefill_kernel(const AttnF32 a) {
   constexpr int BK = 32, LD = D + 4, NC = D / 32;   // NC: 16-B chunks of a row per loading thread
-  __shared__ __attribute__((aligned(16))) float ks[BK * LD], vs[BK * LD];
+  constexpr int kTile = 2 * BK * LD;   // a group's K and V
+  constexpr int kSums = 4 * (D / 16) + 2;   // a lane's
+  static_assert(256 * kSums <= 2 * kTile, "the second group's sums take the tiles' place");
+  __shared__ __attribute__((aligned(16))) float lds[2 * kTile];
   const int seq = a.work_seq[blockIdx.x];
   if (seq < 0) return;   // padding item of a graph-captured prefill (fixed grid)
   const int s0 = a.cu_seqlens[seq], slen = a.cu_seqlens[seq + 1] - s0;
   const int q0 = a.work_q0[blockIdx.x] + 64 * blockIdx.z;
   if (q0 >= slen) return;
   const int Hq = gridDim.y, hq = blockIdx.y, kvh = hq / (Hq / a.Hkv);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, l15 = lane & 15, g = lane >> 4;
+  const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const int tid = threadIdx.x & 255, lane = tid & 63, w = tid >> 6, l15 = lane & 15, g = lane >> 4;
+  float *ks = lds + grp * kTile, *vs = ks + BK * LD;
   const int pl = a.seq_pfx ? a.seq_pfx[seq] : 0;
   const int qrow = q0 + 16 * w + l15;
   const int n = qrow < slen ? pl + qrow + 1 : 0, lo = max(0, pl + qrow + 1 - a.window);   // keys [lo, n) of this lane's query
@@ -448,8 +458,9 @@ __global__ void __launch_bounds__(256) attn_f32_prefill_kernel(const AttnF32 a) 
   };
   f32x4 acc[D / 16] = {};   // dims 16 b + 4 g + r of query l15
   RowStat st;
-  load(kbeg);
-  for (int j0 = kbeg; j0 < kend; j0 += BK) {
+  load(kbeg + BK * grp);
+  for (int jj = kbeg; jj < kend; jj += 2 * BK) {
+    const int j0 = jj + BK * grp;
     __syncthreads();
     bool odd = false;   // a value that must not meet the weight 0 of a query that does not see its key
 #pragma unroll
@@ -460,15 +471,30 @@ __global__ void __launch_bounds__(256) attn_f32_prefill_kernel(const AttnF32 a) 
       for (int e = 0; e < 4; ++e) odd |= !(fabsf(vn[i][e]) <= 3.4028234e38f);
     }
     odd = __syncthreads_or(odd);
-    if (j0 + BK < kend) load(j0 + BK);
-    if (j0 >= pl + q0 + 16 * w + 16) continue;   // past every query of this wave
-    f32x4 s[2] = {};
+    if (jj + 2 * BK < kend) load(j0 + 2 * BK);
+    if (j0 >= min(kend, pl + q0 + 16 * w + 16)) continue;   // past every query of this wave
+    f32x4 s[2] = {}, kf[2][2];
+    auto keys = [&](int c) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) kf[c & 1][kb] = *reinterpret_cast<const f32x4*>(ks + (16 * kb + l15) * LD + 16 * c + 4 * g);
+    };
+    keys(0);
 #pragma unroll
     for (int c = 0; c < D / 16; ++c) {
-      if (16 * c >= a.dkp) break;
+      if (c + 1 < D / 16) keys(c + 1);
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) s[kb] = mfma4(*reinterpret_cast<const f32x4*>(ks + (16 * kb + l15) * LD + 16 * c + 4 * g), qf[c], s[kb]);
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) s[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c & 1][kb][e], qf[c][e], s[kb], 0, 0, 0);
     }
+    float vf[2][2][8];   // two blocks' values, and the next two's
+    auto values = [&](int b) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) vf[(b >> 1) & 1][h][e] = vs[(16 * (e >> 2) + 4 * g + (e & 3)) * LD + 16 * (b + h) + l15];
+    };
+    values(0);
     const float alpha = soften<2>(s, j0, g, lo, n, a.scale, st);
     if (odd) {   // infinities or NaN among the values: key by key, for the queries that see it
 #pragma unroll
@@ -485,16 +511,32 @@ __global__ void __launch_bounds__(256) attn_f32_prefill_kernel(const AttnF32 a) 
       continue;
     }
 #pragma unroll
-    for (int b = 0; b < D / 16; ++b) {
-      if (16 * b >= a.dvp) break;
+    for (int b = 0; b < D / 16; b += 2) {
+      if (b + 2 < D / 16) values(b + 2);
       acc[b] *= alpha;
+      acc[b + 1] *= alpha;
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+      for (int e = 0; e < 8; ++e)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(vs[(16 * kb + 4 * g + e) * LD + 16 * b + l15], s[kb][e], acc[b], 0, 0, 0);
+        for (int h = 0; h < 2; ++h)
+          acc[b + h] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[(b >> 1) & 1][h][e], s[e >> 2][e & 3], acc[b + h], 0, 0, 0);
     }
   }
+  __syncthreads();   // the tiles are free
+  f32x4* sums = reinterpret_cast<f32x4*>(lds) + tid;   // [block][thread], behind them m and l
+  float* mine = lds + 1024 * (D / 16) + tid;
+  if (grp == 1) {
+#pragma unroll
+    for (int b = 0; b < D / 16; ++b) sums[256 * b] = acc[b];
+    mine[0] = st.m;
+    mine[256] = st.l;
+  }
+  __syncthreads();
+  if (grp == 1) return;
+  const float m1 = mine[0], mn = fmaxf(st.m, m1), a0 = expf(st.m - mn), a1 = expf(m1 - mn);
+  st.l = st.l * a0 + mine[256] * a1;
+#pragma unroll
+  for (int b = 0; b < D / 16; ++b) acc[b] = acc[b] * a0 + sums[256 * b] * a1;
   const float l = lanes_sum(st.l);
   if (n <= 0) return;
   const float c = (a.gate ? a.gate[(int64_t)(s0 + qrow) * Hq + hq] : 1.f);
@@ -517,8 +559,8 @@ int attn_f32_prefill(const AttnF32& a, int items, int Hq, hipStream_t stream) {
   const dim3 grid(items, Hq, 2);   // items are 128 query rows
   const bool odd = a.dvp % 16 || a.o_ld % 4;
 #define OAMD_PF(D)                                                              \
-  if (odd) attn_f32_prefill_kernel<D, true><<<grid, 256, 0, stream>>>(a);       \
-  else attn_f32_prefill_kernel<D, false><<<grid, 256, 0, stream>>>(a)
+  if (odd) attn_f32_prefill_kernel<D, true><<<grid, 512, 0, stream>>>(a);       \
+  else attn_f32_prefill_kernel<D, false><<<grid, 512, 0, stream>>>(a)
   if (top <= 64) {
     OAMD_PF(64);
   } else if (top <= 128) {
