@@ -2,8 +2,12 @@
 // [c (rp) | rotated part | 0 .. ck), its score is the product with the whole row and its value is c.
 //
 // Workgroup = (sequence, split, 16 HG query heads), 4 HG waves, 64-token tiles. A tile is loaded once,
-// held in registers while the previous one is worked on, and stored to LDS, from which both
-// products read:
+// held in registers while the one before it is worked on (up to 16 heads: the two before it; with 32 that gains nothing), and stored
+// to LDS, from which both products read. A tile's rows are loaded by eight threads each, with one page lookup and one address per row:
+// chunks dealt out over the whole tile cost a division, a lookup and an address each, and registers that some sizes spilled.
+// 48 sequences of 3600 rows, combine included: 16 heads on 320 columns 48 -> 39 us, on 384 117 -> 49, 32 heads on 576 75 -> 72
+// (2.8 TB/s: a tile's phases, one after the other behind four barriers, are what bounds it).
+//
 //   S = K Q^T     v_mfma_f32_16x16x32_bf16, A = rows (tokens x dims), B = q (one head per column);
 //                 wave w of a head group takes tokens 16 w .. 16 w + 15
 //   O^T += V^T P  the same instruction, A = the same rows through the transposing LDS read, B = P, which
@@ -33,8 +37,9 @@ __device__ __forceinline__ int latent_split(int len, int num_splits) {
 
 // NK: 32-dim steps of a row (even), ck = 32 NK; HG: groups of 16 heads
 template <int NK, int HG>
-__global__ void __launch_bounds__(256 * HG, HG == 1 && NK < 16 ? 2 : 1) attn_latent_decode_kernel(const AttnDecode a, int rp, int B) {
-  constexpr int CK = 32 * NK, RK = 2 * CK + 16, NC = CK / 8, NT = 256 * HG, NL = NK / HG, NB = NK / 2;
+__global__ void __launch_bounds__(256 * HG, HG == 1 && NK < 12 ? 2 : 1) attn_latent_decode_kernel(const AttnDecode a, int rp, int B) {
+  constexpr int CK = 32 * NK, RK = 2 * CK + 16, NT = 256 * HG, NL = NK / HG, NB = NK / 2;
+  constexpr int kAhead = HG == 1 ? 2 : 1;   // tiles in registers
   __shared__ int pg[kMaxPages];
   __shared__ __attribute__((aligned(16))) char tile[kRound * RK];
   __shared__ __attribute__((aligned(16))) s16x4 ps[HG][4][64];
@@ -74,22 +79,29 @@ __global__ void __launch_bounds__(256 * HG, HG == 1 && NK < 16 ? 2 : 1) attn_lat
                      : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
   __syncthreads();
 
-  u16x8 kr[NL];
-  auto load = [&](int ti) {
+  // a thread's rows of a tile are row0 and, of 16 heads, row0 + 32, its 16-B chunks of a row ch0 + 8 j: one page lookup and one
+  // address per row, the rest are offsets
+  constexpr int NR = 2 / HG, NJ = NL / NR;
+  const int row0 = tid >> 3, ch0 = tid & 7;
+  u16x8 even[NL], odd[NL];   // the next two tiles (kAhead == 1: the next)
+  auto load = [&](u16x8 (&kr)[NL], int ti) {
 #pragma unroll
-    for (int i = 0; i < NL; ++i) {
-      const int c = NT * i + tid, row = c / NC, ch = c % NC;
-      const int t = min(start + kRound * ti + row, end - 1);   // past the end: a row that exists, zeroed below
-      kr[i] = *reinterpret_cast<const u16x8*>(
-          a.k_cache + ((int64_t)pg[(t >> a.log2_page) - page0] * a.page_size + (t & (a.page_size - 1))) * CK + 8 * ch);
+    for (int h = 0; h < NR; ++h) {
+      const int t = min(start + kRound * ti + row0 + 32 * h, end - 1);   // past the end: a row that exists, zeroed below
+      const u16x8* p = reinterpret_cast<const u16x8*>(
+          a.k_cache + ((int64_t)pg[(t >> a.log2_page) - page0] * a.page_size + (t & (a.page_size - 1))) * CK) + ch0;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) kr[h * NJ + j] = p[8 * j];
     }
   };
-  auto store = [&](int ti) {
+  auto store = [&](const u16x8 (&kr)[NL], int ti) {
     const int left = end - (start + kRound * ti);   // rows that exist
 #pragma unroll
-    for (int i = 0; i < NL; ++i) {
-      const int c = NT * i + tid, row = c / NC, ch = c % NC;
-      *reinterpret_cast<u16x8*>(tile + RK * row + 16 * ch) = row < left ? kr[i] : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    for (int h = 0; h < NR; ++h) {
+      const bool in = row0 + 32 * h < left;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        *reinterpret_cast<u16x8*>(tile + RK * (row0 + 32 * h) + 16 * ch0 + 128 * j) = in ? kr[h * NJ + j] : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
     }
   };
 
@@ -99,12 +111,11 @@ __global__ void __launch_bounds__(256 * HG, HG == 1 && NK < 16 ? 2 : 1) attn_lat
   for (int m = 0; m < NB; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int nb = rp >> 4;
 
-  load(0);
-  for (int ti = 0; ti < ntile; ++ti) {
+  auto work = [&](u16x8 (&kr)[NL], int ti) {
     __syncthreads();   // every wave is done with the previous tile
-    store(ti);
+    store(kr, ti);
     __syncthreads();
-    if (ti + 1 < ntile) load(ti + 1);
+    if (ti + kAhead < ntile) load(kr, ti + kAhead);
     f32x4 d0 = f32x4{0.f, 0.f, 0.f, 0.f}, d1 = d0;
     const char* krow = tile + RK * (16 * w + l15) + 16 * lg;
 #pragma unroll
@@ -156,6 +167,12 @@ __global__ void __launch_bounds__(256 * HG, HG == 1 && NK < 16 ? 2 : 1) attn_lat
           acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, va), __builtin_bit_cast(bf16x8, pb), acc[m], 0, 0, 0);
         }
     }
+  };
+  load(even, 0);
+  if (kAhead == 2 && ntile > 1) load(odd, 1);
+  for (int ti = 0; ti < ntile; ti += kAhead) {
+    work(even, ti);
+    if (kAhead == 2 && ti + 1 < ntile) work(odd, ti + 1);
   }
   l_run += __shfl_xor(l_run, 16, kWave);
   l_run += __shfl_xor(l_run, 32, kWave);
