@@ -637,8 +637,11 @@ void moe_sort(const at::Tensor& ids, const at::Tensor& weights, int64_t E, int64
   TORCH_CHECK(bm > 0 && rows % bm == 0, "moe_sort: rows");
   need(gtab, at::kInt, 1 + rows / bm, "gtab", true);
   const c10::hip::HIPGuardMasqueradingAsCUDA g(ids.device());
+  TORCH_CHECK(slots < (int64_t(1) << 30) && E >= 0 && E < (1 << 20), "moe_sort: sizes");
+  const int64_t words = oamd::moe_sort_words((int)slots, (int)E);
+  const at::Tensor ws = at::empty({words}, ids.options());
   RC(oamd::moe_sort(p<int>(ids), p<float>(weights), (int)slots, (int)ids.size(1), (int)E, (int)bm, (int)rows,
-                    p<int>(pos), p<int>(src), p<float>(rscale), p<int>(gtab), cur_stream()));
+                    p<int>(pos), p<int>(src), p<float>(rscale), p<int>(gtab), words ? p<int>(ws) : nullptr, cur_stream()));
 }
 
 void moe_gather(const at::Tensor& h, const at::Tensor& src, const at::Tensor& gtab, int64_t bm, at::Tensor& xp) {

@@ -361,8 +361,9 @@ int moe_topk(const float* logits, int ld, int T, int E, int top, int* ids, float
              hipStream_t stream);
 // Expert-sorted row order, every expert's segment padded to bm rows: pos[slot] = row, src[row] =
 // token (-1: padding), rscale[row], gtab = {tiles, expert of tile i ...}; slots = T * top.
+int64_t moe_sort_words(int slots, int E);   // of ws
 int moe_sort(const int* ids, const float* weights, int slots, int top, int E, int bm, int max_rows, int* pos, int* src,
-             float* rscale, int* gtab, hipStream_t stream);
+             float* rscale, int* gtab, int* ws, hipStream_t stream);
 // xp[row] = h[src[row]] (zeros for padding) for the rows of gtab's tiles; row_bytes % 16 == 0
 int moe_gather(const void* h, const int* src, const int* gtab, int bm, int max_rows, void* xp, int row_bytes,
                hipStream_t stream);
