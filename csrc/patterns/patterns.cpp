@@ -27,7 +27,6 @@
 #include <map>
 #include <stdexcept>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <unordered_map>
 #include <vector>
@@ -345,9 +344,10 @@ class PackJob {
     past_cache_ = total >= kPastCache && dst % 16 == 0 && seg % 16 == 0;
     done_ = std::vector<std::atomic<uint8_t>>(pieces_.size());
     const int more = std::min<int>(threads, static_cast<int>(pieces_.size())) - 1;
+    if (more > 0) pool_.reserve(more);
     try {
       for (int t = 0; t < more; ++t) pool_.emplace_back([this] { while (step()) {} });
-    } catch (const std::system_error&) {   // no more threads to be had: those there are, and the waiting one
+    } catch (const std::exception&) {   // no more threads to be had: those there are, and the waiting one
     }
   }
   ~PackJob() { close(); }

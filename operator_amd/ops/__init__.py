@@ -624,7 +624,7 @@ def linear_tile(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = Non
     if (out is None or (out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0)) and (
             bias is None or (bias.is_contiguous() and bias.data_ptr() % 16 == 0)):   # gemm_mid's 16-B accesses
         S = mid_plan(M, N, K, defer, out is None or out.stride(0) == out.shape[1], prompt)   # the reduce pass has no row stride
-        if K >= 128:
+        if 128 <= K < 1 << 22 and M < 1 << 24 and N < 1 << 30:   # gemm_mid's
             rows = tile_rows(M, N, K, S or 1)
     part = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if S is not None and S > 1 else None
     opt = {} if rows == 128 else {"rows": rows}
@@ -670,7 +670,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, sp
     gemm_mid where the rows cost more than its tile (_mid_beats_skinny); 64, 128, 192 and 256 rows on the LDS-staged
     split-K gemm_decode (the measured table, else _decode_tiles; vocabularies _vocab_plan) or where it is estimated
     faster gemm_mid; everything else (prompts, the lm_head of many of them, biased projections) on gemm_mid's 128 x 256
-    tiles with K slices (mid_plan) or gemm_tile's 256 x 256 tiles (persistent p5 past 256 rows). ``defer_reduce``: K
+    tiles with K slices (mid_plan) or gemm_tile's tiles of 192 to 256 rows (the persistent p5 schedule). ``defer_reduce``: K
     slices come back as fp32 slabs (:class:`SplitK`). fp32 operands: linear_f32. hipBLASLt only
     for shapes none of them takes (K % 64 != 0, N % 16 != 0, non-bf16), for decode shapes the
     tuned table measured it fastest on, or under OAMD_PREFILL_BLAS=1 (A/B); CPU tensors on torch.
