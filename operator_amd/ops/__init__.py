@@ -799,8 +799,11 @@ _FP8_STEP = {(64, 64): 0.40, (64, 128): 0.56, (128, 64): 0.51, (128, 128): 0.80,
 def _fp8_tiles(M: int, N: int, K: int):
     """(estimate in us, (bm, bn, S)) of gemm_fp8: the tile with the shortest rounds (128 rows of 10240 x 8192 in 128 x 128
     tiles: one round of 160 workgroups 30 us, two of 128 x 64 35). Up to 64 rows two or three workgroups share a CU and
-    the narrow tile stays (1 row: 20.5 against 21.3)."""
+    the narrow tile stays (1 row: 20.5 against 21.3), of wide N too where the CU with the most of them takes in no more (16 rows of
+    40960 x 8192: 640 workgroups 71 us, 320 of 128 columns 82; of 57344 x 8192 896 99, 448 92)."""
     bm, bn, S = _fp8_slices(M, N, K)
+    if M <= 64 and bn == 128 and -(-(N // 64) * S // CUS) * (64 + 64) <= -(-(N // 128) * S // CUS) * (64 + 128):
+        bn = 64
     steps = -(-(K // 128) // S)
     best = None
     for (r, c), step in _FP8_STEP.items():

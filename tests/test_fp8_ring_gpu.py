@@ -28,3 +28,9 @@ def test_rings_give_the_same_bits(M, N, K, S):
     mag = (q.double().abs() * sx[:, None]) @ (w.double().abs() * sw[:, None]).t()
     # one bf16 rounding, fp32 sums of K products and the two scales
     assert ((got[64, 64].double() - exact).abs() <= 2.0 ** -8 * exact.abs() + (K + 2 + S) * 2.0 ** -24 * mag).all()
+
+
+def test_columns_of_few_rows():
+    """Up to 64 rows: the narrow tile unless more of them end on one CU; the slices stay."""
+    for n, k, cols in ((40960, 8192, 64), (37888, 3584, 64), (57344, 8192, 128), (28672, 4096, 128), (10240, 8192, 64)):
+        assert all(ops.fp8_plan(m, n, k) == (64, cols, ops._fp8_slices(m, n, k)[2]) for m in (1, 64))
