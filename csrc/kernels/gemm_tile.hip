@@ -989,7 +989,8 @@ int gemm_tile(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, i
   // gate|up, the W panels stream from HBM) gives W a third LDS buffer -- a 2-step prefetch
   // (M = 32k, N = 28672: 5786 -> 5366 us; at N = 4096 / 6144 the 2-buffer form is faster,
   // profiles/gemm_tile_p5_vs_hipblaslt_r6.jsonl)
-  if ((variant == 5 || variant == 0) && K >= 2 * kBK && st16) {
+  const bool one16 = M > kT || bias == nullptr || reinterpret_cast<uintptr_t>(bias) % 16 == 0;   // one row tile of an unaligned bias: h4's narrower loads
+  if ((variant == 5 || (variant == 0 && one16)) && K >= 2 * kBK && st16) {
     const int grid = min(nwg, device_cus());
     // GROUP_M 4 for the narrow projections (M = 32k, N = 6144: 1106 vs 1145 us at GROUP_M 8; N = 4096
     // equal; 16 / 32 slower: profiles/gemm_tile_p5_vs_hipblaslt_r6.jsonl)

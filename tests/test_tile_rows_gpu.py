@@ -50,6 +50,19 @@ def test_every_tile_gives_the_same_bits(M, N, K):
     assert ((slabs[0].double().sum(0) - r).abs() <= K * 2.0 ** -24 * mag).all()   # fp32 sums of K terms
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 200, 256, 257])
+def test_operands_off_their_alignment(M):
+    """Biases and outputs off 16 bytes run on the kernels with narrower accesses: the same bits."""
+    torch.manual_seed(M)
+    x, w, b = _rand(M, 256), _rand(512, 256, scale=0.05), _rand(512)
+    want = ops.linear_tile(x, w, bias=b)
+    off = torch.cat([b[:1], b])[1:]
+    wide = torch.zeros(M, 524, dtype=torch.bfloat16, device=DEV)
+    assert off.data_ptr() % 16 and torch.equal(ops.linear_tile(x, w, bias=off), want)
+    assert torch.equal(ops.linear_tile(x, w, wide[:, 4:516], bias=b), want) and not wide[:, :4].any() and not wide[:, 516:].any()
+
+
 def test_rows_that_the_kernels_have():
     for N, K in ((16, 128), (272, 192), (4096, 4096), (28672, 4096), (3584, 18944)):
         for M in (1, 128, 129, 300, 885, 4096, 30000):
