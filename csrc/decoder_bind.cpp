@@ -246,7 +246,7 @@ void attn_gd_prefill(const at::Tensor& q, const at::Tensor& k, const at::Tensor&
     a.window = win; a.gate = op<float>(gate);
     a.scale = (float)scale;
     a.pk = op<float>(pk); a.pv = op<float>(pv); a.seq_pfx = op<int>(seq_pfx);
-    RC(oamd::attn_f32_prefill(a, (int)work_seq->numel(), (int)Hq, cur_stream()));
+    RC(oamd::attn_f32_prefill(a, T, (int)work_seq->numel(), (int)Hq, cur_stream()));
     return;
   }
   oamd::AttnPrefill a{};

@@ -403,36 +403,40 @@ __device__ __forceinline__ float lanes_sum(float v) {
 }  // namespace
 
 // Prefill: a workgroup is 64 query rows of one sequence and head, a wave 16 of them; 32-key tiles of K and V
-// are shared through LDS (rows padded by 16 B) and the next tile's loads are in flight while one is used. Two groups of four waves
-// take tiles in turn, each with sums of its own, which meet in LDS at the end: a short prompt has one workgroup per CU, whose softmax
-// would leave the matrix cores idle, and whose longest rows bound the launch.
-// What bounds it: the workgroups with the longest rows, whose 32-key tile is 1.7 us of fp32 MFMAs and about as much of softmax, staging and
-// barriers. With one group 2 x 500 rows of 16 heads of 128 took 75 us, with two 60; 200 rows 34 -> 28, 1000 rows of 8 heads of 256
-// 279 -> 204, 2018 rows of 16 heads 404 -> 402; 32 x 64 rows, where the second group has nothing to do half of the time, 24 -> 28. One group for those
-// would make a prompt's rounding depend on what it is packed with. The products run over all D columns (zeros past the heads):
-// a way out per 16 columns kept each block's reads behind the block before.
+// are shared through LDS (rows padded by 16 B) and the next tile's loads are in flight while one is used.
+// NG: the even tiles and the odd ones have sums of their own, which meet at the end. Two groups of four waves (NG == 2) take them side
+// by side: with few workgroups on the chip one group's softmax would leave the matrix cores idle, and the longest rows bound the
+// launch. One group (NG == 1) takes the even tiles, then the odd ones: half the LDS, and nobody waits where there is but one tile. Same
+// sums, same bits, so the launch chooses (f32_prefill_groups) and a prompt's numbers do not depend on what it is packed with.
+// What bounds it: with few workgroups those with the longest rows, whose 32-key tile is 1.7 us of fp32 MFMAs and about as much of softmax,
+// staging and barriers; with many, the MFMA rate. One group and two: 2 x 500 rows of 16 heads of 128 72 and 59 us, 1000 rows of 8 heads of 256
+// 250 and 206, 128 x 64 rows of 16 heads of 128 75 and 98, 64 x 16 rows 22 and 33.
+// LESS: heads that end before D's last blocks, behind a way out per block: 2000 rows of 32 heads of 192 and 128 columns 1520 us without one, 1140 with it.
+// Where no block is left out it would keep reads from crossing it.
 // D: instantiated size >= both head sizes. ODD: value heads that are no multiple of 16 columns, or output rows that take no
 // 16-B stores (key heads are multiples of 4 in either form).
-template <int D, bool ODD>
-__global__ void __launch_bounds__(512) attn_f32_prefill_kernel(const AttnF32 a) {
+template <int D, bool ODD, bool LESS, int NG>
+__global__ void __launch_bounds__(256 * NG, NG == 1 && D == 64 ? 4 : 1) attn_f32_prefill_kernel(const AttnF32 a) {
   constexpr int BK = 32, LD = D + 4, NC = D / 32;   // NC: 16-B chunks of a row per loading thread
   constexpr int kTile = 2 * BK * LD;   // a group's K and V
   constexpr int kSums = 4 * (D / 16) + 2;   // a lane's
-  static_assert(256 * kSums <= 2 * kTile, "the second group's sums take the tiles' place");
-  __shared__ __attribute__((aligned(16))) float lds[2 * kTile];
+  static_assert(NG == 1 || 256 * kSums <= 2 * kTile, "the second group's sums take the tiles' place");
+  __shared__ __attribute__((aligned(16))) float lds[NG * kTile];
+  __shared__ int odds[4 * NG];   // of every wave: its values of the tile are not all finite
   const int seq = a.work_seq[blockIdx.x];
   if (seq < 0) return;   // padding item of a graph-captured prefill (fixed grid)
   const int s0 = a.cu_seqlens[seq], slen = a.cu_seqlens[seq + 1] - s0;
   const int q0 = a.work_q0[blockIdx.x] + 64 * blockIdx.z;
   if (q0 >= slen) return;
   const int Hq = gridDim.y, hq = blockIdx.y, kvh = hq / (Hq / a.Hkv);
-  const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const int grp = NG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
   const int tid = threadIdx.x & 255, lane = tid & 63, w = tid >> 6, l15 = lane & 15, g = lane >> 4;
   float *ks = lds + grp * kTile, *vs = ks + BK * LD;
   const int pl = a.seq_pfx ? a.seq_pfx[seq] : 0;
   const int qrow = q0 + 16 * w + l15;
   const int n = qrow < slen ? pl + qrow + 1 : 0, lo = max(0, pl + qrow + 1 - a.window);   // keys [lo, n) of this lane's query
   const int kend = pl + min(slen, q0 + 64), kbeg = max(0, pl + q0 + 1 - a.window) & ~(BK - 1);
+  float* out = a.o + (int64_t)(s0 + qrow) * a.o_ld + hq * a.dvp + 4 * g;   // of rows that exist: n > 0
 
   const f32x4 zero{};
   f32x4 qf[D / 16];
@@ -457,10 +461,14 @@ __global__ void __launch_bounds__(512) attn_f32_prefill_kernel(const AttnF32 a) 
     }
   };
   f32x4 acc[D / 16] = {};   // dims 16 b + 4 g + r of query l15
-  RowStat st;
-  load(kbeg + BK * grp);
-  for (int jj = kbeg; jj < kend; jj += 2 * BK) {
-    const int j0 = jj + BK * grp;
+  f32x4 acc0[D / 16];
+  RowStat st, st0;          // acc0, st0 (NG == 1): of the even tiles
+  // steps of the group: a tile of its own each (NG == 2, the second group's last may be past the end), or the even tiles, then the odd ones
+  const int tiles = (kend - kbeg + BK - 1) / BK, evens = (tiles + 1) >> 1, steps = NG == 1 ? tiles : evens;
+  auto key0 = [&](int t) { return kbeg + BK * (NG == 2 ? 2 * t + grp : t < evens ? 2 * t : 2 * (t - evens) + 1); };
+  load(key0(0));
+  for (int t = 0; t < steps; ++t) {
+    const int j0 = key0(t);
     __syncthreads();
     bool odd = false;   // a value that must not meet the weight 0 of a query that does not see its key
 #pragma unroll
@@ -470,9 +478,22 @@ __global__ void __launch_bounds__(512) attn_f32_prefill_kernel(const AttnF32 a) 
 #pragma unroll
       for (int e = 0; e < 4; ++e) odd |= !(fabsf(vn[i][e]) <= 3.4028234e38f);
     }
-    odd = __syncthreads_or(odd);
-    if (jj + 2 * BK < kend) load(j0 + 2 * BK);
+    odd = __any(odd);
+    if (lane == 0) odds[4 * grp + w] = odd;
+    __syncthreads();
+    odd = odds[4 * grp] | odds[4 * grp + 1] | odds[4 * grp + 2] | odds[4 * grp + 3];   // of the group's tile alone
+    if (t + 1 < steps) load(key0(t + 1));
+    if (NG == 1 && t == evens) {   // the odd tiles begin
+#pragma unroll
+      for (int b = 0; b < D / 16; ++b) {
+        acc0[b] = acc[b];
+        acc[b] = zero;
+      }
+      st0 = st;
+      st = RowStat{};
+    }
     if (j0 >= min(kend, pl + q0 + 16 * w + 16)) continue;   // past every query of this wave
+    // the reads of a block go out under the block before, and behind the last block of a smaller head is the way out
     f32x4 s[2] = {}, kf[2][2];
     auto keys = [&](int c) {
 #pragma unroll
@@ -486,6 +507,7 @@ __global__ void __launch_bounds__(512) attn_f32_prefill_kernel(const AttnF32 a) 
       for (int e = 0; e < 4; ++e)
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) s[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c & 1][kb][e], qf[c][e], s[kb], 0, 0, 0);
+      if (LESS && 16 * (c + 1) >= a.dkp) break;
     }
     float vf[2][2][8];   // two blocks' values, and the next two's
     auto values = [&](int b) {
@@ -520,27 +542,51 @@ __global__ void __launch_bounds__(512) attn_f32_prefill_kernel(const AttnF32 a) 
 #pragma unroll
         for (int h = 0; h < 2; ++h)
           acc[b + h] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[(b >> 1) & 1][h][e], s[e >> 2][e & 3], acc[b + h], 0, 0, 0);
+      if (LESS && 16 * (b + 2) >= a.dvp) break;
     }
   }
-  __syncthreads();   // the tiles are free
-  f32x4* sums = reinterpret_cast<f32x4*>(lds) + tid;   // [block][thread], behind them m and l
-  float* mine = lds + 1024 * (D / 16) + tid;
-  if (grp == 1) {
+  // the even tiles' sums f and m0, l0; the odd ones' e and m1, l1
+  auto meet = [](float& f, float a0, float e, float a1) { f = __builtin_fmaf(e, a1, f * a0); };
+  if constexpr (NG == 2) {
+    __syncthreads();   // the tiles are free
+    f32x4* sums = reinterpret_cast<f32x4*>(lds) + tid;   // [block][thread], behind them m and l
+    float* mine = lds + 1024 * (D / 16) + tid;
+    if (grp == 1) {
 #pragma unroll
-    for (int b = 0; b < D / 16; ++b) sums[256 * b] = acc[b];
-    mine[0] = st.m;
-    mine[256] = st.l;
+      for (int b = 0; b < D / 16; ++b) sums[256 * b] = acc[b];
+      mine[0] = st.m;
+      mine[256] = st.l;
+    }
+    __syncthreads();
+    if (grp == 1) return;
+    const float m1 = mine[0], mn = fmaxf(st.m, m1), a0 = expf(st.m - mn), a1 = expf(m1 - mn);
+    meet(st.l, a0, mine[256], a1);
+#pragma unroll
+    for (int b = 0; b < D / 16; ++b) {
+      const f32x4 e = sums[256 * b];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float f = acc[b][r];
+        meet(f, a0, e[r], a1);
+        acc[b][r] = f;
+      }
+    }
+  } else if (tiles > 1) {
+    const float mn = fmaxf(st0.m, st.m), a0 = expf(st0.m - mn), a1 = expf(st.m - mn);
+    meet(st0.l, a0, st.l, a1);
+    st.l = st0.l;
+#pragma unroll
+    for (int b = 0; b < D / 16; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float f = acc0[b][r];
+        meet(f, a0, acc[b][r], a1);
+        acc[b][r] = f;
+      }
   }
-  __syncthreads();
-  if (grp == 1) return;
-  const float m1 = mine[0], mn = fmaxf(st.m, m1), a0 = expf(st.m - mn), a1 = expf(m1 - mn);
-  st.l = st.l * a0 + mine[256] * a1;
-#pragma unroll
-  for (int b = 0; b < D / 16; ++b) acc[b] = acc[b] * a0 + sums[256 * b] * a1;
   const float l = lanes_sum(st.l);
   if (n <= 0) return;
   const float c = (a.gate ? a.gate[(int64_t)(s0 + qrow) * Hq + hq] : 1.f);
-  float* out = a.o + (int64_t)(s0 + qrow) * a.o_ld + hq * a.dvp + 4 * g;
 #pragma unroll
   for (int b = 0; b < D / 16; ++b) {
     if (16 * b >= a.dvp) break;
@@ -552,15 +598,35 @@ __global__ void __launch_bounds__(512) attn_f32_prefill_kernel(const AttnF32 a) 
   }
 }
 
-int attn_f32_prefill(const AttnF32& a, int items, int Hq, hipStream_t stream) {
+// Two groups pay until their workgroups, twice as large, come in more than a round or two of the CUs, and not where most query rows have a single
+// tile of keys (two, of the largest heads, which have a workgroup per CU either way). `blocks` is about the number of workgroups that have rows. Over 26
+// packings of 4 to 8192 rows and ten head layouts the choices take 0.3 % more than the better form; nowhere more than 7 %.
+static int f32_prefill_groups(int D, int64_t rows, int items, int Hq) {
+  const int64_t blocks = (items + rows / 128) * Hq;
+  return rows > (int64_t)items * (D == 256 ? 64 : 32) && blocks <= (D == 64 ? 600 : D == 128 ? 400 : 2000) ? 2 : 1;
+}
+
+template <int D, bool ODD>
+static void launch_f32_prefill(const AttnF32& a, int64_t rows, const dim3& grid, hipStream_t stream) {
+  const bool less = a.dkp <= D - 16 || a.dvp <= D - 32;   // loops that may end before D
+  if (f32_prefill_groups(D, rows, grid.x, grid.y) == 1) {
+    if (less) attn_f32_prefill_kernel<D, ODD, true, 1><<<grid, 256, 0, stream>>>(a);
+    else attn_f32_prefill_kernel<D, ODD, false, 1><<<grid, 256, 0, stream>>>(a);
+  } else {
+    if (less) attn_f32_prefill_kernel<D, ODD, true, 2><<<grid, 512, 0, stream>>>(a);
+    else attn_f32_prefill_kernel<D, ODD, false, 2><<<grid, 512, 0, stream>>>(a);
+  }
+}
+
+int attn_f32_prefill(const AttnF32& a, int64_t rows, int items, int Hq, hipStream_t stream) {
   if (items == 0) return 0;
   const int top = a.dkp > a.dvp ? a.dkp : a.dvp;
   if (a.dkp < 4 || a.dkp % 4 || a.dvp < 1 || top > 256 || Hq % a.Hkv || a.window < 1) return -1;
   const dim3 grid(items, Hq, 2);   // items are 128 query rows
   const bool odd = a.dvp % 16 || a.o_ld % 4;
-#define OAMD_PF(D)                                                              \
-  if (odd) attn_f32_prefill_kernel<D, true><<<grid, 512, 0, stream>>>(a);       \
-  else attn_f32_prefill_kernel<D, false><<<grid, 512, 0, stream>>>(a)
+#define OAMD_PF(D)                                                   \
+  if (odd) launch_f32_prefill<D, true>(a, rows, grid, stream);       \
+  else launch_f32_prefill<D, false>(a, rows, grid, stream)
   if (top <= 64) {
     OAMD_PF(64);
   } else if (top <= 128) {

@@ -348,7 +348,7 @@ struct AttnF32 {
   int window;                   // as in AttnPrefill
   const float* gate;            // [rows][Hq] or nullptr
 };
-int attn_f32_prefill(const AttnF32& a, int items, int Hq, hipStream_t stream);
+int attn_f32_prefill(const AttnF32& a, int64_t rows, int items, int Hq, hipStream_t stream);   // rows: of q
 // splits > 1: pieces of every context through part [rows][Hq][splits][dvp] and ml [rows][Hq][splits][2]
 int attn_f32_decode(const AttnF32& a, int rows, int Hq, int splits, float* part, float* ml, hipStream_t stream);
 
