@@ -1,4 +1,4 @@
-"""Routed slots in expert segments: one workgroup for few, a workgroup per 1024 slots for many."""
+"""Routed slots in expert segments: one workgroup for few, a workgroup per 1024 slots for many (the line grows with the experts)."""
 import pytest
 import torch
 
@@ -12,7 +12,8 @@ DEV = "cuda"
 # workgroup's share
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,top,E,bm,skew", [(1, 2, 8, 64, 0), (1024, 2, 8, 256, 0), (1025, 2, 8, 256, 0), (2049, 1, 3, 128, 1), (7950, 2, 8, 256, 0),
-                                             (3000, 2, 8, 256, 2), (700, 4, 512, 64, 0), (4097, 8, 512, 64, 0)])
+                                             (3000, 2, 8, 256, 2), (700, 4, 512, 64, 0), (4097, 8, 512, 64, 0), (1589, 2, 8, 64, 0), (1590, 2, 8, 64, 0),
+                                             (2741, 1, 3, 128, 1), (1400, 8, 512, 64, 0)])
 def test_segments(T, top, E, bm, skew):
     torch.manual_seed(T + E)
     score = torch.randn(T, E, device=DEV)
