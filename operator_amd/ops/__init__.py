@@ -790,27 +790,34 @@ def _fp8_slices(M: int, N: int, K: int) -> tuple[int, int, int]:
     return bm, bn, S
 
 
-# us of a 128-K step of gemm_fp8's tiles, every CU busy (8192 x 28672, 57344 x 8192; the plans they give were timed on eight
-# shapes of 4096 to 57344 features, 1 to 4000 rows: none slower than the former fixed tile, profiles/plans_before_after.txt)
-_FP8_STEP = {(64, 64): 0.40, (64, 128): 0.56, (128, 64): 0.51, (128, 128): 0.80, (256, 64): 0.71, (256, 128): 1.16}
+# Estimates of the two fp8 kernels by tile (rows, columns): us to start and to store, us of a 128-column step on a CU and what it takes more
+# with every CU busy, us between rounds, us per million fp32 slab elements. gemm_fp8_tile has the tiles of 256 columns. Fitted to 299 products of
+# 20 shapes, 65 to 4100 rows, weights from HBM: the choices take 0.7 % more than the best ones
+_FP8_US = {(64, 64): (3.8, 0.04, 0.30, 0.4, 0.19), (128, 64): (4.9, 0.12, 0.34, 1.1, 0.30), (128, 128): (8.4, 0.48, 0.16, 5.6, 0.20),
+           (256, 64): (8.5, 0.45, 0.21, 5.7, 0.26), (256, 128): (13.1, 0.73, 0.26, 10.0, 0.19),
+           (96, 256): (6.4, 0.66, 0.03, 2.0, 0.52), (128, 256): (7.4, 0.75, 0.06, 3.5, 0.54), (160, 256): (8.6, 0.79, 0.15, 4.6, 0.55)}
+
+
+def _fp8_us(rows: int, cols: int, M: int, N: int, K: int, S: int) -> float:
+    start, one, busy, between, slabs = _FP8_US[rows, cols]
+    units = -(-M // rows) * -(-N // cols) * S
+    full, last = divmod(units, CUS)
+    rounds = full * (one + busy) + (one + busy * last / CUS if last else 0)
+    return start + -(-(K // 128) // S) * rounds + between * ((units - 1) // CUS) + (slabs * S * M * N * 1e-6 if S > 1 else 0)
 
 
 @functools.lru_cache(maxsize=4096)
 def _fp8_tiles(M: int, N: int, K: int):
-    """(estimate in us, (bm, bn, S)) of gemm_fp8: the tile with the shortest rounds (128 rows of 10240 x 8192 in 128 x 128
+    """(estimate in us, (bm, bn, S)) of gemm_fp8: the fastest tile (128 rows of 10240 x 8192 in 128 x 128
     tiles: one round of 160 workgroups 30 us, two of 128 x 64 35). Up to 64 rows two or three workgroups share a CU and
     the narrow tile stays (1 row: 20.5 against 21.3), of wide N too where the CU with the most of them takes in no more (16 rows of
     40960 x 8192: 640 workgroups 71 us, 320 of 128 columns 82; of 57344 x 8192 896 99, 448 92)."""
     bm, bn, S = _fp8_slices(M, N, K)
-    if M <= 64 and bn == 128 and -(-(N // 64) * S // CUS) * (64 + 64) <= -(-(N // 128) * S // CUS) * (64 + 128):
-        bn = 64
-    steps = -(-(K // 128) // S)
-    best = None
-    for (r, c), step in _FP8_STEP.items():
-        if N % c == 0 and (M > 64 or (r, c) == (bm, bn)):
-            t = 4 + -(-(-(-M // r) * (N // c) * S) // CUS) * steps * step
-            best = min(best or (t, (r, c, S)), (t, (r, c, S)))
-    return best or (float("inf"), (bm, bn, S))
+    if M <= 64:
+        if bn == 128 and -(-(N // 64) * S // CUS) * (64 + 64) <= -(-(N // 128) * S // CUS) * (64 + 128):
+            bn = 64
+        return 0.0, (bm, bn, S)
+    return min(((_fp8_us(r, c, M, N, K, S), (r, c, S)) for r, c in _FP8_US if c < 256 and N % c == 0), default=(float("inf"), (bm, bn, S)))
 
 
 def fp8_plan(M: int, N: int, K: int) -> tuple[int, int, int]:
@@ -818,29 +825,18 @@ def fp8_plan(M: int, N: int, K: int) -> tuple[int, int, int]:
     return _FP8_OVERRIDES.get((N, K)) or _fp8_tiles(M, N, K)[1]
 
 
-# us of a 128-column step of gemm_fp8_tile's tiles of 96, 128 and 160 rows, and what it takes more with every CU busy
-_FP8_ROW_STEP = {96: (0.63, 0.06), 128: (0.66, 0.11), 160: (0.68, 0.25)}
-
-
 @functools.lru_cache(maxsize=4096)
 def fp8_tile_rows(M: int, N: int, K: int, S: int) -> tuple[float, int]:
     """(estimate in us, rows of the tiles, 256 columns wide) of gemm_fp8_tile: those whose rounds of one workgroup per CU
     take least, as tile_rows (700 rows of 8192 x 8192: 192 tiles of 128 rows 57 us, 256 of 96 48; 1200 rows of 8192 x 28672: 320
     tiles of 128 rows 354 us, 256 of 160 215)."""
-    best = None
-    for rows, (one, busy) in _FP8_ROW_STEP.items():
-        units = -(-M // rows) * -(-N // 256) * S
-        full, last = divmod(units, CUS)
-        rounds = full * (one + busy) + (one + busy * last / CUS if last else 0)
-        cost = -(-(K // 128) // S) * rounds + 8 + 3 * (units - 1) // CUS
-        best = min(best or (cost, rows), (cost, rows))
-    return best
+    return min((_fp8_us(rows, 256, M, N, K, S), rows) for rows in (96, 128, 160))
 
 
 def fp8_tile_plan(M: int, N: int, K: int) -> int | None:
     """The slices where gemm_fp8_tile is faster than gemm_fp8, whose bits it gives, else None: 512 rows of
-    57344 x 8192 306 -> 218 us, 4096 rows of 8192 x 8192 384 -> 203 (2.7 PFLOP/s), 256 rows of 10240 x 8192 57 -> 33; but
-    512 rows of 8192 x 28672 in one slice 164, against 157, and up to 64 rows the weights' stream is all there is
+    57344 x 8192 306 -> 218 us, 4096 rows of 8192 x 8192 384 -> 203 (2.7 PFLOP/s), 256 rows of 10240 x 8192 57 -> 33, 700 rows of 3072 x 2048
+    21.9 -> 13.7; but 128 rows of 4096 x 4096 in 4 slices 13.3, against 10.6, and up to 64 rows the weights' stream is all there is
     (57344 x 8192: 104, against 90)."""
     S = _fp8_slices(M, N, K)[2]
     if M <= 64 or N % 64 or K // 128 // S < 3 or (N, K) in _FP8_OVERRIDES:
