@@ -836,7 +836,7 @@ def fp8_tile_rows(M: int, N: int, K: int, S: int) -> tuple[float, int]:
 def fp8_tile_plan(M: int, N: int, K: int) -> int | None:
     """The slices where gemm_fp8_tile is faster than gemm_fp8, whose bits it gives, else None: 512 rows of
     57344 x 8192 306 -> 218 us, 4096 rows of 8192 x 8192 384 -> 203 (2.7 PFLOP/s), 256 rows of 10240 x 8192 57 -> 33, 700 rows of 3072 x 2048
-    21.9 -> 13.7; but 128 rows of 4096 x 4096 in 4 slices 13.3, against 10.6, and up to 64 rows the weights' stream is all there is
+    16 -> 14; but 128 rows of 4096 x 4096 in 4 slices 13.3, against 10.6, and up to 64 rows the weights' stream is all there is
     (57344 x 8192: 104, against 90)."""
     S = _fp8_slices(M, N, K)[2]
     if M <= 64 or N % 64 or K // 128 // S < 3 or (N, K) in _FP8_OVERRIDES:
