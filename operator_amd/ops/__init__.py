@@ -612,6 +612,15 @@ def tile_rows(M: int, N: int, K: int, S: int = 1) -> int:
     return min((_rows_us(r, M, N, K, S), r) for r in ((96, 128, 160) if S > 1 else _ROW_STEP))[1]
 
 
+def loose_tiles(M: int, N: int, K: int) -> bool:
+    """One row tile of a vocabulary whose rows are a power of two apart: gemm_tile's schedule of a workgroup per tile (h4), whose workgroups
+    drift apart. In the persistent one all CUs walk their weight rows in step, and rows 8 or 16 KiB apart share memory channels:
+    128256 x 4096 253 us against 290 at 256 rows, 258 and 272 at 192, 258 and 259 at 129; 128256 x 8192 485 and 506 at 256, but 471 and
+    450 at 192. Rows of 3072 or 3584 columns (152064 x 3584: 319 and 304) and vocabularies of one round (32768 x 4096: 106 and 95) are not
+    slowed. The bits are the same."""
+    return (128 if K == 4096 else 208) < M <= 256 and N > 256 * CUS and K >= 4096 and K & (K - 1) == 0
+
+
 def linear_tile(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None,
                 bias: torch.Tensor | None = None, glu: int = 0, defer_reduce: bool = False, prompt: bool = False):
     """Prefill / lm_head GEMM on the compute-bound gfx950 tile kernels (fused bias or gated (``glu``: SILU /
@@ -625,7 +634,7 @@ def linear_tile(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = Non
             bias is None or (bias.is_contiguous() and bias.data_ptr() % 16 == 0)):   # gemm_mid's 16-B accesses
         S = mid_plan(M, N, K, defer, out is None or out.stride(0) == out.shape[1], prompt)   # the reduce pass has no row stride
         if 128 <= K < 1 << 22 and M < 1 << 24 and N < 1 << 30:   # gemm_mid's
-            rows = tile_rows(M, N, K, S or 1)
+            rows = 256 if not glu and loose_tiles(M, N, K) else tile_rows(M, N, K, S or 1)
     part = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if S is not None and S > 1 else None
     opt = {} if rows == 128 else {"rows": rows}
     if part is not None and defer:
@@ -635,7 +644,7 @@ def linear_tile(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = Non
     if rows < 192:
         kernels().gemm_mid(x, w, y, bias, part, S or 1, glu, **opt)
     else:
-        kernels().gemm_tile(x, w, y, bias, glu, rows=rows)
+        kernels().gemm_tile(x, w, y, bias, glu, 1 if not glu and loose_tiles(M, N, K) else 0, rows=rows)
     return y
 
 

@@ -76,3 +76,20 @@ def test_one_round_has_no_stores_between_rounds():
     """Tiles that come in one round of workgroups cost their steps alone: the smaller ones win (257 rows of 3072 x 2048 in 3 slices:
     13.7 us on 96 rows, 18.4 on 160; 385 rows of 768 x 4096 in 8 12.1 and 15.8)."""
     assert all(ops.tile_rows(*a) == 96 for a in ((257, 3072, 2048, 3), (300, 2048, 2048, 4), (385, 768, 4096, 8), (160, 3584, 4096, 4), (129, 3584, 4096, 4)))
+
+
+# the smallest vocabulary of more than a round of 256-column tiles; rows at the edges of the rule
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,Ms", [(4096, (129, 256)), (8192, (208, 209))])
+def test_wide_vocabularies_give_the_same_bits_on_either_schedule(K, Ms):
+    torch.manual_seed(K)
+    w, x = _rand(65552, K, scale=0.05), _rand(256, K)
+    for M in Ms:
+        ops.kernels().gemm_tile(x[:M], w, want := torch.full((M, 65552), float("nan"), dtype=torch.bfloat16, device=DEV), None, 0, 5)
+        assert torch.equal(ops.linear_tile(x[:M], w), want)
+
+
+def test_schedule_of_wide_vocabularies():
+    assert all(ops.loose_tiles(M, 128256, 4096) for M in (129, 192, 256)) and ops.loose_tiles(256, 128256, 8192)
+    assert not any(ops.loose_tiles(*a) for a in ((128, 128256, 4096), (257, 128256, 4096), (192, 128256, 8192), (256, 152064, 3584),
+                                                 (256, 32768, 4096), (256, 151936, 2048)))
