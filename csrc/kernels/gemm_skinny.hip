@@ -168,8 +168,10 @@ static void launch_skinny(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P,
 // 16-row W tiles of a workgroup. It reads the X rows of its K range once for all of them, and a CU takes in X and W at the same rate:
 // 32 rows of 128256 x 4096 429 us on one tile, 345 on two, 304 on four; 16 rows of 4096 x 14336 in 2 slices 38 on one, 30 on two
 // (256 workgroups), 48 on four (128: half the CUs idle). So the tiles whose rounds of one workgroup per CU take in the fewest rows;
-// more tiles stream a little worse (one row of the vocabulary 196 on one, 203 and 252). Over 189 products of 12 shapes, 1 to 32 rows, the choices take
-// 1 % more than the best ones and 7 % less than one tile. The sums' order is the same on any.
+// more tiles stream a little worse (one row of the vocabulary 196 on one, 203 and 252), which two tiles are charged as the bytes of 3300 / Kb more rows
+// a round. Of up to 12 X rows and W rows 16 KiB apart or a larger power of two, whose tiles fall on the same memory channels, each tile more is charged
+// a tenth: one row of 128256 x 8192 400 on one, 438 on two, of 8192 x 8192 31 and 34. Over 477 products of 27 shapes, 1 to 32 rows, the choices take
+// 1 % more than the best ones and 8 % less than one tile. The sums' order is the same on any.
 constexpr int kCus = 256;
 static int skinny_tiles(int M, int N, int Kb, int S, int glu) {
   int best = 0;
@@ -177,7 +179,8 @@ static int skinny_tiles(int M, int N, int Kb, int S, int glu) {
   for (int nt = glu ? 2 : 1; nt <= 4; nt *= 2) {
     if (N % (16 * nt)) break;
     const int rounds = (N / (16 * nt) * S + kCus - 1) / kCus;
-    const double cost = rounds * ((16.0 * nt * (nt == 4 ? 1.15 : 1.0) + 0.8 * M) * Kb + (nt == 2 && !glu ? 3300 : 0));
+    const double far = M <= 12 && Kb >= 8192 && (Kb & (Kb - 1)) == 0 ? 1.0 + 0.1 * (nt - 1) : 1.0;
+    const double cost = rounds * ((16.0 * nt * far * (nt == 4 ? 1.15 : 1.0) + 0.8 * M) * Kb + (nt == 2 && !glu ? 3300 : 0));
     if (best == 0 || cost < least) best = nt, least = cost;
   }
   return best;
@@ -192,7 +195,7 @@ int gemm_skinny(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, in
   if (S > 1 && P == nullptr) return -5;
   const int nt = skinny_tiles(M, N, K / S, S, glu), steps = K / S / (sk::kWaves * 32), rounds = (N / (16 * nt) * S + kCus - 1) / kCus;
   // k-steps in flight: long streams of many rounds take more (128256 x 4096, one row: 16 steps 191 us, 8 196; 8 rows on two tiles: 8 steps
-  // 222, 4 226), but never a remainder, whose steps wait one by one
+  // 222, 4 226), but not where it leaves a remainder, whose steps wait one by one
   if (nt == 4) launch_skinny<4, 2>(X, W, Y, P, M, N, K, S, glu, stream);
   else if (nt == 2 && steps % 8 == 0 && (glu || rounds >= 4)) launch_skinny<2, 8>(X, W, Y, P, M, N, K, S, glu, stream);
   else if (nt == 2) launch_skinny<2, 4>(X, W, Y, P, M, N, K, S, glu, stream);

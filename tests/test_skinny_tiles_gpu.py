@@ -11,7 +11,7 @@ DEV = "cuda"
 # features: one tile, an odd number of tiles (only one fits), two and four per workgroup, several rounds; K steps of a wave: one, a
 # remainder, groups of 8 and 16; rows at the edges of the two X tiles
 @pytest.mark.parametrize("N,K,S", [(16, 128, 1), (48, 1152, 1), (8224, 384, 1), (4096, 1024, 2), (4096, 2304, 2), (8192, 2048, 4), (70016, 2048, 1),
-                                   (131072, 256, 1)])
+                                   (131072, 256, 1), (8192, 8192, 1)])   # the last: W rows 16 KiB apart, up to 12 X rows on fewer tiles
 @pytest.mark.parametrize("M", [1, 5, 16, 17, 32])
 def test_rows_are_the_same_beside_others(M, N, K, S):
     torch.manual_seed(N + K + M)
