@@ -956,8 +956,9 @@ int gemm_tile(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, i
   if (Y != nullptr && ldy < (glu ? N / 2 : N)) return -3;
   if (S < 1 || S > 64 || K % (kBK * S) != 0 || (S > 1 && (P == nullptr || bias != nullptr))) return -5;
   if (Y == nullptr && (S == 1 || glu)) return -6;
+  const bool p5_k = K >= 2 * kBK && K < (1 << 23);   // two steps; an operand's tile, 512 K bytes, within its buffer bound's 32 bits
   if (rows != kT) {   // p5 alone has them
-    if ((rows != 192 && rows != 224) || S != 1 || variant != 0 || K < 2 * kBK || ldy % 8 || reinterpret_cast<uintptr_t>(Y) % 16) return -8;
+    if ((rows != 192 && rows != 224) || S != 1 || variant != 0 || !p5_k || ldy % 8 || reinterpret_cast<uintptr_t>(Y) % 16) return -8;
     const int64_t units = (int64_t)((M + rows - 1) / rows) * ((N + kT - 1) / kT);
     if (units > (1LL << 30)) return -9;
     const int grid = (int)min(units, (int64_t)device_cus());
@@ -990,13 +991,13 @@ int gemm_tile(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, i
   // (M = 32k, N = 28672: 5786 -> 5366 us; at N = 4096 / 6144 the 2-buffer form is faster,
   // profiles/gemm_tile_p5_vs_hipblaslt_r6.jsonl)
   const bool one16 = M > kT || bias == nullptr || reinterpret_cast<uintptr_t>(bias) % 16 == 0;   // one row tile of an unaligned bias: h4's narrower loads
-  if ((variant == 5 || (variant == 0 && one16)) && K >= 2 * kBK && st16) {
+  if ((variant == 5 || (variant == 0 && one16)) && p5_k && st16) {
     const int grid = min(nwg, device_cus());
     // GROUP_M 4 for the narrow projections (M = 32k, N = 6144: 1106 vs 1145 us at GROUP_M 8; N = 4096
     // equal; 16 / 32 slower: profiles/gemm_tile_p5_vs_hipblaslt_r6.jsonl)
     if (N >= 16384) launch_p5<2>(X, W, Y, bias, M, N, K, ldy, glu, grid, stream, 4);   // GROUP_M 4: -1.1 / -1.4 % at M = 12k / 32k
     else launch_p5<0>(X, W, Y, bias, M, N, K, ldy, glu, grid, stream, 4);
-  } else if (variant >= 6 && variant <= 14 && K >= 2 * kBK && st16) {   // p5 A/B arms (timing, same numerics)
+  } else if (variant >= 6 && variant <= 14 && p5_k && st16) {   // p5 A/B arms (timing, same numerics)
     const int grid = min(nwg, device_cus());
     if (variant == 6) launch_p5<0>(X, W, Y, bias, M, N, K, ldy, glu, grid, stream, 4);         // GROUP_M 4
     else if (variant == 7) launch_p5<0>(X, W, Y, bias, M, N, K, ldy, glu, grid, stream, 16);   // GROUP_M 16

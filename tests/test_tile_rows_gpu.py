@@ -93,3 +93,26 @@ def test_schedule_of_wide_vocabularies():
     assert all(ops.loose_tiles(M, 128256, 4096) for M in (129, 192, 256)) and ops.loose_tiles(256, 128256, 8192)
     assert not any(ops.loose_tiles(*a) for a in ((128, 128256, 4096), (257, 128256, 4096), (192, 128256, 8192), (256, 152064, 3584),
                                                  (256, 32768, 4096), (256, 151936, 2048)))
+
+
+@pytest.mark.gpu
+def test_rows_longer_than_a_buffer_bound():
+    """256 weight rows of 2^23 columns are 4 GiB, past the 32 bits of the persistent schedule's buffer bounds: such products run on the
+    kernel with 64-bit addresses. Small whole numbers: every sum is exact in fp32, whatever its order."""
+    if torch.cuda.get_device_properties(0).total_memory < 32 << 30:
+        pytest.skip("needs 20 GB")
+    K, M, N, step = 1 << 23, 3, 256, 1 << 19
+    torch.manual_seed(0)
+    w, x = torch.empty(N, K, dtype=torch.bfloat16, device=DEV), torch.empty(M, K, dtype=torch.bfloat16, device=DEV)
+    want = torch.zeros(M, N, device=DEV)
+    for k in range(0, K, step):
+        w[:, k:k + step] = torch.randint(-1, 2, (N, step), device=DEV, dtype=torch.int8)
+        x[:, k:k + step] = torch.randint(-1, 2, (M, step), device=DEV, dtype=torch.int8)
+        want += x[:, k:k + step].float() @ w[:, k:k + step].float().t()
+    assert want.abs().max() < 1 << 24
+    y = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    ops.kernels().gemm_tile(x, w, y)
+    assert torch.equal(y, want.bfloat16())
+    assert torch.equal(ops.linear_tile(x, w), y)
+    with pytest.raises(RuntimeError):
+        ops.kernels().gemm_tile(x, w, y, rows=192)
