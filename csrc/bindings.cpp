@@ -326,7 +326,10 @@ void gemm_tile(const at::Tensor& x, const at::Tensor& w, const c10::optional<at:
   }
   TORCH_CHECK(M * K < (1LL << 40) && N * K < (1LL << 40) && M < (1LL << 31) && N < (1LL << 31), "gemm too large");
   const c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
-  RC(oamd::gemm_tile(ptr<bf16_t>(x), ptr<bf16_t>(w), yp, optr<bf16_t>(bias), (int)M, (int)N, (int)K, (int)ldy,
+  // the epilogues read a bias 8 or 16 bytes at a time: one off 16 bytes comes as a copy
+  c10::optional<at::Tensor> b16 = bias;
+  if (bias.has_value() && reinterpret_cast<uintptr_t>(bias->data_ptr()) % 16) b16 = bias->clone();
+  RC(oamd::gemm_tile(ptr<bf16_t>(x), ptr<bf16_t>(w), yp, optr<bf16_t>(b16), (int)M, (int)N, (int)K, (int)ldy,
                      (int)silu_gu, (int)variant, (int)splits, pp, (int)rows, cur_stream()));
 }
 

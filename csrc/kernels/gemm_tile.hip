@@ -956,6 +956,7 @@ int gemm_tile(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, i
   if (Y != nullptr && ldy < (glu ? N / 2 : N)) return -3;
   if (S < 1 || S > 64 || K % (kBK * S) != 0 || (S > 1 && (P == nullptr || bias != nullptr))) return -5;
   if (Y == nullptr && (S == 1 || glu)) return -6;
+  if (reinterpret_cast<uintptr_t>(bias) % 16) return -10;   // read 8 or 16 bytes at a time
   const bool p5_k = K >= 2 * kBK && K < (1 << 23);   // two steps; an operand's tile, 512 K bytes, within its buffer bound's 32 bits
   if (rows != kT) {   // p5 alone has them
     if ((rows != 192 && rows != 224) || S != 1 || variant != 0 || !p5_k || ldy % 8 || reinterpret_cast<uintptr_t>(Y) % 16) return -8;
@@ -990,8 +991,7 @@ int gemm_tile(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, i
   // gate|up, the W panels stream from HBM) gives W a third LDS buffer -- a 2-step prefetch
   // (M = 32k, N = 28672: 5786 -> 5366 us; at N = 4096 / 6144 the 2-buffer form is faster,
   // profiles/gemm_tile_p5_vs_hipblaslt_r6.jsonl)
-  const bool one16 = M > kT || bias == nullptr || reinterpret_cast<uintptr_t>(bias) % 16 == 0;   // one row tile of an unaligned bias: h4's narrower loads
-  if ((variant == 5 || (variant == 0 && one16)) && p5_k && st16) {
+  if ((variant == 5 || variant == 0) && p5_k && st16) {
     const int grid = min(nwg, device_cus());
     // GROUP_M 4 for the narrow projections (M = 32k, N = 6144: 1106 vs 1145 us at GROUP_M 8; N = 4096
     // equal; 16 / 32 slower: profiles/gemm_tile_p5_vs_hipblaslt_r6.jsonl)

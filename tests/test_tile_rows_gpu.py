@@ -53,7 +53,7 @@ def test_every_tile_gives_the_same_bits(M, N, K):
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 200, 256, 257])
 def test_operands_off_their_alignment(M):
-    """Biases and outputs off 16 bytes run on the kernels with narrower accesses: the same bits."""
+    """Biases off 16 bytes come as a copy, outputs run on the kernels with narrower stores: the same bits."""
     torch.manual_seed(M)
     x, w, b = _rand(M, 256), _rand(512, 256, scale=0.05), _rand(512)
     want = ops.linear_tile(x, w, bias=b)
@@ -61,6 +61,24 @@ def test_operands_off_their_alignment(M):
     wide = torch.zeros(M, 524, dtype=torch.bfloat16, device=DEV)
     assert off.data_ptr() % 16 and torch.equal(ops.linear_tile(x, w, bias=off), want)
     assert torch.equal(ops.linear_tile(x, w, wide[:, 4:516], bias=b), want) and not wide[:, :4].any() and not wide[:, 516:].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,rows", [(1, 256), (256, 256), (257, 256), (200, 192), (300, 224)])
+def test_bias_off_its_alignment_is_copied(M, rows):
+    """The epilogues load a bias 16 (8) bytes at a time: one off that alignment is read from an aligned copy, whatever the tile."""
+    torch.manual_seed(M)
+    C, x, w, b = ops.kernels(), _rand(M, 256), _rand(512, 256, scale=0.05), _rand(512)
+    y, want = (torch.empty(M, 512, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    made = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]  # noqa: E731
+    n = made()
+    C.gemm_tile(x, w, want, b, rows=rows)
+    assert made() == n
+    for shift in (1, 4):   # 2 and 8 bytes
+        off = torch.cat([b[:shift], b])[shift:]
+        n = made()
+        C.gemm_tile(x, w, y.zero_(), off, rows=rows)
+        assert made() == n + 1 and torch.equal(y, want)
 
 
 def test_rows_that_the_kernels_have():
