@@ -636,6 +636,12 @@ void attn_prefill(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
   TORCH_CHECK(q.size(0) == k.size(0) && q.size(2) == 128 && k.size(2) == 128, "T / head_dim mismatch");
   TORCH_CHECK(q.size(1) % k.size(1) == 0, "Hq % Hkv");
   TORCH_CHECK(work_seq.numel() == work_q0.numel(), "work list shape");
+  const c10::hip::HIPGuardMasqueradingAsCUDA g(q.device());
+  // variants 3 and 4 bring keys and values to LDS 16 bytes at a time: ones off 16 bytes come as a copy
+  const bool dma = variant == 3 || variant == 4;
+  const auto on16 = [&](const at::Tensor& t) { return dma && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 ? t.clone() : t; };
+  const at::Tensor k16 = on16(k), v16 = on16(v);
+  at::Tensor pk16, pv16;
   const bf16_t *pkp = nullptr, *pvp = nullptr;
   const int* pfx = nullptr;
   if (seq_pfx.has_value()) {
@@ -645,12 +651,13 @@ void attn_prefill(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                 "pk / pv [prefix, Hkv, 128]");
     CHECK_DEV(*seq_pfx); CHECK_DT(*seq_pfx, at::kInt); CHECK_CONTIG(*seq_pfx);
     TORCH_CHECK(seq_pfx->numel() >= cu_seqlens.numel() - 1, "seq_pfx: one prefix length per sequence");
-    pkp = ptr<bf16_t>(*pk);
-    pvp = ptr<bf16_t>(*pv);
+    pk16 = on16(*pk);
+    pv16 = on16(*pv);
+    pkp = ptr<bf16_t>(pk16);
+    pvp = ptr<bf16_t>(pv16);
     pfx = ptr<int>(*seq_pfx);
   }
-  const c10::hip::HIPGuardMasqueradingAsCUDA g(q.device());
-  RC(oamd::attn_prefill(ptr<bf16_t>(q), ptr<bf16_t>(k), ptr<bf16_t>(v), ptr<bf16_t>(o), ptr<int>(cu_seqlens),
+  RC(oamd::attn_prefill(ptr<bf16_t>(q), ptr<bf16_t>(k16), ptr<bf16_t>(v16), ptr<bf16_t>(o), ptr<int>(cu_seqlens),
                         ptr<int>(work_seq), ptr<int>(work_q0), (int)work_seq.numel(), (int)q.size(1),
                         (int)k.size(1), 128, (float)scale, (int)variant, cur_stream(), pkp, pvp, pfx));
 }

@@ -58,3 +58,53 @@ def test_windows_and_scales(scale, window):
     q, k, v = (torch.randn(T, h, d, device=DEV).bfloat16() for h, d in ((Hq, dk), (Hkv, dk), (Hkv, dv)))
     o = dec.attn_gd_prefill(q, k, v, LENS, L, scale, window=window)
     _close(o.view(T, Hq, dv), _exact(q, k, v, LENS, scale, window or 1 << 30), v)
+
+
+def _off(t, shift):
+    """t's rows ``shift`` elements past a 16-byte alignment."""
+    b = torch.empty(t.numel() + shift, dtype=t.dtype, device=DEV)[shift:].view(t.shape)
+    return b.copy_(t)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hkv", [(4, 2), (7, 1)])
+@pytest.mark.parametrize("shift", [1, 2, 4])
+def test_keys_off_their_alignment(Hq, Hkv, shift):
+    """Keys and values off 16 bytes, own and of a prefix, come as a copy: the same bits."""
+    torch.manual_seed(shift)
+    lens, P = [70, 33, 130], 100
+    T = sum(lens)
+    q, k, v = (torch.randn(T, h, 128, device=DEV).bfloat16() for h in (Hq, Hkv, Hkv))
+    pk, pv = (torch.randn(P, Hkv, 128, device=DEV).bfloat16() for _ in range(2))
+    var = ops.prefill_variant(Hq, Hkv)
+    ws, wq = ops.prefill_work_list(lens, ops.prefill_block_q(Hq, Hkv, var))
+    work = tuple(torch.tensor(t, dtype=torch.int32, device=DEV) for t in ([0, 70, 103, 233], ws, wq)) + (var,)
+    sp = torch.full((3,), P, dtype=torch.int32, device=DEV)
+    assert _off(k, shift).data_ptr() % 16 == 2 * shift
+    for pre, pre_off in ((None, None), ((pk, pv, sp, [P] * 3), (_off(pk, shift), _off(pv, shift), sp, [P] * 3))):
+        want = ops.attn_prefill(q, k, v, lens, 0.09, work=work, prefix=pre)
+        assert torch.equal(ops.attn_prefill(q, _off(k, shift), _off(v, shift), lens, 0.09, work=work, prefix=pre_off), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hkv", [(4, 2), (8, 1)])
+@pytest.mark.parametrize("P", [1, 63, 65, 100])
+def test_prefix_ends_inside_a_tile(Hq, Hkv, P):
+    """What stands behind the last row of a prefix is NaN, and so is what stands behind the own rows: neither is ever multiplied."""
+    torch.manual_seed(P)
+    lens = [1, 40, 65]
+    T, nan = sum(lens), float("nan")
+    q = torch.randn(T, Hq, 128, device=DEV).bfloat16()
+    pk, pv, k, v = (torch.full((n + 64, Hkv, 128), nan, dtype=torch.bfloat16, device=DEV) for n in (P, P, T, T))
+    for t, n in ((pk, P), (pv, P), (k, T), (v, T)):
+        t[:n] = torch.randn(n, Hkv, 128, device=DEV).bfloat16()
+    var = ops.prefill_variant(Hq, Hkv)
+    ws, wq = ops.prefill_work_list(lens, ops.prefill_block_q(Hq, Hkv, var))
+    work = tuple(torch.tensor(t, dtype=torch.int32, device=DEV) for t in ([0, 1, 41, 106], ws, wq)) + (var,)
+    sp = torch.full((3,), P, dtype=torch.int32, device=DEV)
+    o, a = ops.attn_prefill(q, k[:T], v[:T], lens, 128 ** -0.5, work=work, prefix=(pk, pv, sp, [P] * 3)), 0
+    for n in lens:
+        kk, vv = torch.cat([pk[:P], k[a:a + n]]), torch.cat([pv[:P], v[a:a + n]])
+        qq = torch.cat([torch.zeros(P, Hq, 128, dtype=q.dtype, device=DEV), q[a:a + n]])   # rows of their own for the prefix, not looked at
+        _close(o[a:a + n], _exact(qq, kk, vv, [P + n], 128 ** -0.5)[P:], vv)
+        a += n
