@@ -339,6 +339,14 @@ class MatchEngine:
         pipelined analyze). Returns (hits, resident, newlines): the text and layout the
         scan leaves on the GPU for the context windows, and (docs, newlines per doc);
         both None when the batch fell back to the host scan."""
+        try:
+            return self._scan_slot(docs, slot)
+        except BaseException:
+            # an upload may still be reading the pinned buffer, which the next scan writes into or replaces
+            torch.cuda.current_stream(self.device).synchronize()
+            raise
+
+    def _scan_slot(self, docs: list[bytes], slot: int):
         from operator_amd.ops import kernels, patterns
         sfx = "" if slot == 0 else f"_s{slot}"
 
@@ -362,7 +370,7 @@ class MatchEngine:
         layout[:nd + 1] = first
         np.multiply(layout[:nd], seg, out=layout[nd + 1:2 * nd + 1])
         layout[2 * nd + 1:] = lens
-        first_t, base_t, lens_t = text[total:total + lay].view(torch.int64).split([nd + 1, nd, nd])
+        base_t, lens_t = text[total + 8 * (nd + 1):total + lay].view(torch.int64).split([nd, nd])
         # native threads pack the whole batch in order, and each doc-aligned chunk of >= PACK_CHUNK bytes is uploaded as soon
         # as it is in place, so a large batch pays max(pack, H2D) rather than the sum (a batch of 1.2 GB)
         threads = max(1, min(self.pack_threads, total >> 20))   # ~1 MB per packing thread (4.6 MB: 177 us on one, 93 on four)

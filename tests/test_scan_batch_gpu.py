@@ -1,7 +1,9 @@
 """One-call scan: the report in front of the records, at the edges of the read-back and of the match buffer."""
 import numpy as np
 import pytest
+import torch
 
+from operator_amd import ops
 from operator_amd.engine.match import MatchEngine
 from operator_amd.patterns.schema import PatternSet
 
@@ -21,3 +23,23 @@ def test_scan_report_edges(nd, cap, monkeypatch):
         assert len(hits) == n and sorted(map(tuple, hits.tolist())) == sorted(map(tuple, want.tolist()))
         assert eng._doc_newlines[1] == [d.count(b"\n") for d in docs]
         assert hits.dtype == np.int64
+
+
+def test_nothing_reads_the_buffer_after_an_error(monkeypatch):
+    """An error behind the uploads: none of them still reads the pinned buffer when it reaches the caller, and the next scan is right."""
+    eng = MatchEngine(PatternSet.from_dicts([{"id": "a", "primary_pattern": {"literal": "refused"}}]), device="cuda", seg_bytes=256)
+    docs = [b"refused\n" + b"x" * (1 << 20)] * 256   # 5 ms of upload
+    want = eng.scan_gpu(docs)                          # buffers of the size are there
+    idle = []
+
+    def fail(*a):
+        idle.append(torch.cuda.current_stream().query())   # the uploads are under way
+        raise RuntimeError("no memory")
+
+    with monkeypatch.context() as m:
+        m.setattr(ops.kernels(), "scan_batch", fail)
+        with pytest.raises(RuntimeError, match="no memory"):
+            eng._scan_gpu(docs)
+        idle.append(torch.cuda.current_stream().query())
+    assert idle == [False, True]
+    assert np.array_equal(np.sort(eng.scan_gpu(docs), axis=0), np.sort(want, axis=0)) and len(want) == 256
