@@ -74,7 +74,7 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
   constexpr int AUX = 16;
   constexpr int kBM = 32 * MI;                   // a wave has MI X fragments and as many X pieces per step
   constexpr int NP = MI + 8;                     // LDS-DMA pieces of a wave per step
-  constexpr int NS = 3;                          // stages: 144 KiB
+  constexpr int NS = 3;                          // stages: 132, 144 or 156 KiB
   constexpr int kGroupM = 32 / MI;               // row tiles that share a W panel before the next one
   constexpr int kX = kBM * 128, kStage = kX + kBN * 128;
   __shared__ __attribute__((aligned(1024))) char lds[NS * kStage];

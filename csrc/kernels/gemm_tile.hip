@@ -1,9 +1,8 @@
 // Compute-bound GEMM for prefill projections and the lm_head:
 //   Y[M, N] = X[M, K] . W[N, K]^T     bf16 in, fp32 accumulate, bf16 out
-// (SURVEY.md §2.4 N7 "prefill is compute-bound tiles (256² 8-phase template)";
-// replaces the external LLM behind J/service/AIInterfaceRestClient.java:37-39).
+// (replaces the external LLM behind J/service/AIInterfaceRestClient.java:37-39).
 //
-// Two schedules of one 256 x 256 output tile per workgroup, BK = 64, both operands staged
+// Three schedules of 256 x 256 output tiles (p5 also of 192 or 224 rows), BK = 64, both operands staged
 // global -> LDS by LDS-DMA into two 64 KiB buffers (128-B rows; the st_16x32-style XOR
 // swizzle slot = chunk ^ ((row >> 1) & 7) applied to the global SOURCE chunk and to the read
 // address, rule 21: conflict-free ds_read_b128), v_mfma_f32_16x16x32_bf16 with operands
@@ -12,16 +11,20 @@
 // the gate|up weight is interleaved in 64-row blocks. XCD-aware, grouped tile order (T1
 // bijective remap, then GROUP_M m-tiles per n-tile) so the 32 tiles an XCD runs at once
 // share X/W panels in L2.
-//   * h4 (default, gemm_tile256_h4_kernel below): 4 waves, one per SIMD, 128 x 128 outputs
+//   * p5 (the default, gemm_tile256_p5_kernel): a persistent workgroup per CU, 4 waves, one LDS-DMA
+//     stream across its tiles, two barriers per K-tile (details at the kernel);
+//   * h4 (gemm_tile256_h4_kernel; vocabularies of one row tile, ops.loose_tiles, outputs off 16 bytes
+//     and K = 64): a workgroup per tile, 4 waves, one per SIMD, 128 x 128 outputs
 //     each in 256 tied AGPRs; four 32-MFMA phases per K-tile with the next tile's DMA and
-//     fragment reads between the MFMAs and 3 barriers (details at the kernel);
-//   * ping-pong (gemm_tile256_kernel, variants 2 / 3 and the split-K slabs): 8 waves, two
+//     fragment reads between the MFMAs and 3 barriers;
+//   * ping-pong (gemm_tile256_kernel, variants 2 / 3, the split-K slabs and operands past the others' 32-bit
+//     offsets): 8 waves, two
 //     per SIMD; every tile split into four 16 KiB regions (X rows 0-127, W rows 0-127, W rows
 //     128-255, X rows 128-255) loaded, waited for and recycled one at a time; the K-tile in
 //     four (or two, PH2) phases, one per (X half, W half) quadrant; waves 4-7 run one
 //     barrier segment behind waves 0-3 so on every SIMD one wave issues its LDS reads + DMA
 //     while the other runs its MFMA cluster (s_setprio 1 around it, T5).
-// Round 4 measured and deleted three other 4-wave schedules (a 4-stage BK = 32 ring with
+// Three other 4-wave schedules were measured and deleted (a 4-stage BK = 32 ring with
 // LDS-DMA or register staging, a BK = 64 region ring): 16 x 64-B DMA pieces cost twice the
 // memory requests of 8 x 128-B ones and register-staged loads cost as much as LDS-DMA
 // (profiles/gemm_tile_pmc_l2_r4.txt, gemm_tile_variants_r4*.jsonl).
@@ -300,7 +303,7 @@ __device__ __forceinline__ void mfma_tied(f32x4& acc, const u16x8& a, const u16x
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
 
-// Variant 1, the default ("h4": two buffers, four phases): four waves (one per SIMD, 128 x 128 outputs
+// Variant 1 ("h4": two buffers, four phases): four waves (one per SIMD, 128 x 128 outputs
 // each, 256 tied AGPR accumulators), BK = 64 tiles in two 64 KiB LDS buffers filled by
 // LDS-DMA pieces of 8 rows x 128 B (buffer_load ... lds: per-lane 32-bit row offsets fixed
 // for the kernel, the K step in soffset) — half the memory requests of 16 x 64-B pieces
@@ -526,7 +529,7 @@ __global__ void __launch_bounds__(256) gemm_tile256_h4_kernel(const bf16_t* __re
   }
 }
 
-// Variant 5, the persistent "p5" schedule (round 6): the h4 tile (4 waves, 128 x 128 outputs
+// Variants 0 and 5, the persistent "p5" schedule: the h4 tile (4 waves, 128 x 128 outputs
 // per wave in 256 tied AGPRs, BK = 64, two 64 KiB LDS buffers filled by 8-row x 128-B LDS-DMA
 // pieces with a source-side chunk swizzle), but
 //   * ONE workgroup per CU (grid = min(tiles, CUs)) walking its tiles in rounds: in round r
@@ -555,7 +558,7 @@ __global__ void __launch_bounds__(256) gemm_tile256_h4_kernel(const bf16_t* __re
 //     kernel (K sweep, profiles/gemm_tile_p5_vs_hipblaslt_r6.jsonl). The chunk swizzle
 //     slot ^ (bit1(row) << 1 | bit3(row) << 2) keeps both fragment-read patterns conflict-free;
 //   * per-tile buffer resources (base = the tile's first row, num_records = its rows x K x 2):
-//     rows past M / N read as zeros, no clamps, no 32-bit limit on the operand size.
+//     rows past M / N read as zeros, no clamps, no 32-bit limit on the operand size (on a tile: K < 2^23).
 // DEEP: which operand streams through THREE LDS buffers (its pieces issued 3 K-steps ahead, two steps
 // of flight) -- 0: neither (2 + 2 buffers, 128 KiB), 1: X (narrow N: the X panels come from HBM,
 // W stays in the Infinity Cache), 2: W (wide N: the W panels come from HBM); 160 KiB of LDS.
@@ -987,7 +990,7 @@ int gemm_tile(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, i
   const bool off32 = (int64_t)M * K * 2 < (1LL << 32) && (int64_t)N * K * 2 < (1LL << 32);
   const bool st16 = ldy % 8 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0;   // p5's 16-B stores
   // persistent p5 (variant 5; the default where its 16-B stores reach): one workgroup per CU (220 rows of 6144 x 4096 77 us,
-  // on the h4 schedule 92; 256 rows of 128256 x 4096 278 and 291); wide N (>= 16384:
+  // on the h4 schedule 92; 256 rows of 152064 x 3584 304 and 319; ops.loose_tiles has the exception); wide N (>= 16384:
   // gate|up, the W panels stream from HBM) gives W a third LDS buffer -- a 2-step prefetch
   // (M = 32k, N = 28672: 5786 -> 5366 us; at N = 4096 / 6144 the 2-buffer form is faster,
   // profiles/gemm_tile_p5_vs_hipblaslt_r6.jsonl)
@@ -1017,7 +1020,7 @@ int gemm_tile(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, i
     else if (bias) gemm_tile256_h4_kernel<kEpiBias, 16, true><<<nwg, 256, 0, stream>>>(X, W, Y, bias, M, N, K, ldy);
     else gemm_tile256_h4_kernel<kEpiStore, 16, true><<<nwg, 256, 0, stream>>>(X, W, Y, bias, M, N, K, ldy);
   } else if (variant == 2 || (variant == 0 && M > 256)) {
-    // 8-wave ping-pong, two barrier segments per K-tile (the round-3 default; 2-8 % behind
+    // 8-wave ping-pong, two barrier segments per K-tile (2-8 % behind
     // variant 1 on the prefill shapes, profiles/gemm_tile_h4_vs_ph2_m32k.jsonl); also the
     // fallback for operands past 32-bit offsets
     if (glu) gemm_tile256_kernel<kEpiSilu, true><<<nwg, 512, 0, stream>>>(X, W, Y, bias, M, N, K, ldy, nullptr, glu_act(glu));

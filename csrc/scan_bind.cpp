@@ -59,25 +59,6 @@ void ac_scan(const at::Tensor& text, int64_t seg_bytes, const at::Tensor& cls_ma
   TORCH_CHECK(rc == 0, "ac_scan launch failed rc=", rc);
 }
 
-void scan_fixup(at::Tensor& matches, const at::Tensor& match_count, const at::Tensor& seg_nl_excl,
-                const at::Tensor& doc_first_seg, int64_t seg_bytes, const at::Tensor& seg_head) {
-  CHECK_T(matches, at::kInt);
-  CHECK_T(match_count, at::kInt);
-  CHECK_T(seg_nl_excl, at::kLong);
-  CHECK_T(doc_first_seg, at::kLong);
-  TORCH_CHECK(matches.dim() == 2 && matches.size(1) == 4, "matches must be [cap, 4]");
-  TORCH_CHECK(doc_first_seg.numel() >= 2, "doc_first_seg must have num_docs+1 >= 2 entries");
-  CHECK_T(seg_head, at::kInt);
-  TORCH_CHECK(seg_head.numel() >= seg_nl_excl.numel(), "seg_head needs one entry per segment");
-  const c10::hip::HIPGuardMasqueradingAsCUDA g(matches.device());
-  const int rc = oamd::scan_fixup(reinterpret_cast<oamd::MatchRec*>(matches.data_ptr()),
-                                  reinterpret_cast<const uint32_t*>(match_count.data_ptr()), (uint32_t)matches.size(0),
-                                  seg_nl_excl.data_ptr<int64_t>(), doc_first_seg.data_ptr<int64_t>(),
-                                  (int)doc_first_seg.numel() - 1, (int)seg_bytes,
-                                  reinterpret_cast<const uint32_t*>(seg_head.data_ptr()), c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream());
-  TORCH_CHECK(rc == 0, "scan_fixup launch failed rc=", rc);
-}
-
 void line_prefix(const at::Tensor& cnt, at::Tensor& excl, at::Tensor& state) {
   CHECK_T(cnt, at::kInt);
   CHECK_T(excl, at::kLong);
@@ -250,7 +231,6 @@ PYBIND11_MODULE(_S, m) {
   m.def("scan_upload", &scan_upload);
   m.def("scan_batch", &scan_batch);
   m.def("score_events", &score_events);
-  m.def("scan_fixup", &scan_fixup);
   m.def("max_hot_states", [](int64_t log2c) { return oamd::max_hot_states((int)log2c); });
   m.attr("SCAN_HOT_STRIDE") = oamd::kScanHotStride;
   register_comm_bindings(m);

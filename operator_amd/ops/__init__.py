@@ -496,8 +496,8 @@ def _mid_few_rows(M: int, N: int, K: int, defer: bool) -> bool:
     return mid < (3 + 2e-6 * N * K / 5.4) * (1 + 0.04 * M)
 
 
-# Every GPU GEMM of the model runs on the hand-written gfx950 kernels: prompts on gemm_mid up to some 4096 rows
-# (mid_plan) and on gemm_tile's persistent p5 schedule (csrc/kernels/gemm_tile.hip) beyond, decode buckets on
+# Every GPU GEMM of the model runs on the hand-written gfx950 kernels: prompts on gemm_mid or gemm_tile (csrc/kernels/gemm_tile.hip),
+# whichever has the tile rows that fit (tile_rows), in K slices (mid_plan) on gemm_mid, decode buckets on
 # gemm_pp / gemm_tn / gemm_mid / gemm_skinny, the lm_head on whichever of them its rows call for (_mid_beats_skinny,
 # _vocab_plan, mid_plan), fp8 on gemm_fp8 and, past 64 rows, gemm_fp8_tile, fp32 on gemm_f32. hipBLASLt is reached
 # only by shapes none of them takes (K % 64 != 0, N % 16 != 0, non-bf16), counted in BLAS_CALLS.
@@ -678,8 +678,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, sp
     """y = x @ w^T (+ bias) in bf16 on the gfx950 kernels: up to 32 rows on the weight-streaming gemm_skinny, or on
     gemm_mid where the rows cost more than its tile (_mid_beats_skinny); 64, 128, 192 and 256 rows on the LDS-staged
     split-K gemm_decode (the measured table, else _decode_tiles; vocabularies _vocab_plan) or where it is estimated
-    faster gemm_mid; everything else (prompts, the lm_head of many of them, biased projections) on gemm_mid's 128 x 256
-    tiles with K slices (mid_plan) or gemm_tile's tiles of 192 to 256 rows (the persistent p5 schedule). ``defer_reduce``: K
+    faster gemm_mid; everything else (prompts, the lm_head of many of them, biased projections) on gemm_mid's tiles of 96 to 160 rows,
+    with K slices where mid_plan has them, or gemm_tile's of 192 to 256 (tile_rows). ``defer_reduce``: K
     slices come back as fp32 slabs (:class:`SplitK`). fp32 operands: linear_f32. hipBLASLt only
     for shapes none of them takes (K % 64 != 0, N % 16 != 0, non-bf16), for decode shapes the
     tuned table measured it fastest on, or under OAMD_PREFILL_BLAS=1 (A/B); CPU tensors on torch.
