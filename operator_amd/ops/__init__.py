@@ -615,7 +615,7 @@ def tile_rows(M: int, N: int, K: int, S: int = 1) -> int:
 def loose_tiles(M: int, N: int, K: int) -> bool:
     """One row tile of a vocabulary whose rows are a power of two apart: gemm_tile's schedule of a workgroup per tile (h4), whose workgroups
     drift apart. In the persistent one all CUs walk their weight rows in step, and rows 8 or 16 KiB apart share memory channels:
-    128256 x 4096 253 us against 290 at 256 rows, 258 and 272 at 192, 258 and 259 at 129; 128256 x 8192 485 and 506 at 256, but 471 and
+    128256 x 4096 253 us against 290 at 256 rows (285 and 293 within a decode step), 258 and 272 at 192, 258 and 259 at 129; 128256 x 8192 485 and 506 at 256, but 471 and
     450 at 192. Rows of 3072 or 3584 columns (152064 x 3584: 319 and 304) and vocabularies of one round (32768 x 4096: 106 and 95) are not
     slowed. The bits are the same."""
     return (128 if K == 4096 else 208) < M <= 256 and N > 256 * CUS and K >= 4096 and K & (K - 1) == 0
