@@ -1,4 +1,4 @@
-// One-shot and two-shot all-reduce over peer-mapped HBM (SURVEY.md §2.4 X1, §5.8).
+// One-shot and two-shot all-reduce over peer-mapped HBM.
 //
 // Tensor-parallel decode all-reduces are small (M x hidden x 2 B: 16 KB per
 // token at 70B) and latency-bound; a ring all-reduce over xGMI takes 2 (n - 1)
@@ -337,8 +337,8 @@ __global__ void __launch_bounds__(car::kThreads) allreduce_kernel(const uint4* _
 // Fused TP block epilogue: h = h + bf16(sum over ranks of in); y = RMSNorm(h) * w.
 // Row-partitioned (block b owns rows [r0, r1)), so after the all-reduce each block
 // holds whole rows and normalises them in place: the all-reduce's output never
-// round-trips through HBM before the norm, and one launch replaces two (SURVEY.md
-// §7.4 item 6: the fusion that makes TP=8 pay). TWO: the block's rows go through the
+// round-trips through HBM before the norm, and one launch replaces two
+// (the fusion that makes TP=8 pay). TWO: the block's rows go through the
 // two-shot protocol (reduce-scatter of pieces, all-gather of their sums) instead of
 // one-shot; the sums are bit-identical.
 // Numerics are those of all-reduce + rmsnorm_kernel: the sum is rounded to bf16,

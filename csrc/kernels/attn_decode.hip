@@ -1,4 +1,4 @@
-// Paged decode attention, GQA, streaming split-KV (SURVEY.md §2.4 N12).
+// Paged decode attention, GQA, streaming split-KV.
 //
 // One query token per sequence. Workgroup = (sequence, split, kv-head); the
 // G = Hq/Hkv query heads sharing the kv-head are processed together so every

@@ -1,5 +1,5 @@
 // Causal flash attention for prefill, variable-length packed sequences, GQA,
-// on MFMA (SURVEY.md §2.4 N11). Four variants share the work-list contract
+// on MFMA. Four variants share the work-list contract
 // (attn_prefill_block_q): v1 per-query-head (below), v2 GQA-grouped 16-row waves
 // with a software-pipelined K/V tile, v3 GQA-grouped swapped-operand 32x32 MFMA
 // waves (S^T = K Q^T, P stays in registers as the next MFMA's B operand) in 8-wave

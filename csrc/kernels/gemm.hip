@@ -1,5 +1,5 @@
 // Decode-shape GEMM: Y[M, N] = X[M, K] . W[N, K]^T, bf16 in, fp32 accumulate
-// (SURVEY.md §2.4 N7 — the explanation model's projections at decode batch).
+// (the explanation model's projections at decode batch).
 //
 // At decode the activations are small (M = bucket size, 64..256 rows) and the
 // weights are streamed once per step, so the kernel is designed around the

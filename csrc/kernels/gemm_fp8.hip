@@ -1,5 +1,5 @@
-// FP8 (OCP e4m3fn) W8A8 GEMM for the large explanation models (SURVEY.md §2.4
-// N8; BASELINE config 5, Llama-3-70B): Y[M, N] = (X8[M, K] . W8[N, K]^T) *
+// FP8 (OCP e4m3fn) W8A8 GEMM for the large explanation models
+// (Llama-3-70B): Y[M, N] = (X8[M, K] . W8[N, K]^T) *
 // sx[m] * sw[n], bf16 out, fp32 accumulate.
 //
 // * Weights are quantized once per output channel (sw[n] = amax / 448) and

@@ -1,10 +1,9 @@
 // Decode-bucket GEMM on the ping-pong schedule of gemm_tile.hip:
 //   Y[M, N] = X[M, K] . W[N, K]^T, M <= 256 (decode batch), bf16 in, fp32 accumulate
-// (SURVEY.md §2.4 N7 "Decode uses skinny-M split-K with nt weight streaming";
-// replaces the external LLM behind J/service/AIInterfaceRestClient.java:37-39).
+// (replaces the external LLM behind J/service/AIInterfaceRestClient.java:37-39).
 //
-// Round 2's gemm_decode waits for a stage, barriers all 8 waves and then reads
-// fragments and runs MFMAs in lock-step, once per k-step: rocprofv3 put 38 % of
+// gemm_decode's first form waited for a stage, barriered all 8 waves and then read
+// fragments and ran MFMAs in lock-step, once per k-step: rocprofv3 put 38 % of
 // its wave-cycles in s_waitcnt (profiles/gemm_decode_m256_stalls_pmc.txt). Here:
 //   * tile = BM (128 x XH) tokens x 128 features, 8 waves in two groups running
 //     one barrier segment apart (waves 4-7 behind): on every SIMD one wave reads

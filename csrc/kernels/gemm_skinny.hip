@@ -1,10 +1,10 @@
 // Skinny-M GEMM for small decode buckets: Y[M, N] = X[M, K] . W[N, K]^T with
-// M <= 32 ("decode uses skinny-M ... with weight streaming").
+// M <= 32.
 //
 // At M = 1..32 the step is a pure weight stream (16 GB of bf16 weights per 8B
 // decode step): the kernel's only job is to keep enough W bytes in flight to
-// run HBM at full rate. Structure (cdna_hip_programming.md §5, row "GEMV /
-// M <= 16 decode weights": straight to VGPRs, deep unroll, no LDS round trip):
+// run HBM at full rate. Structure (weights straight
+// to VGPRs, deep unroll, no LDS round trip):
 //   * a block owns one, two or four 16-row tiles of W (skinny_tiles; for the fused SwiGLU gate rows
 //     and the matching up rows 64 rows later) and its 4 waves split K;
 //   * each wave streams its K range in 32-deep steps: lane l loads 16 B of W

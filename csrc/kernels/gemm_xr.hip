@@ -1,10 +1,10 @@
 // Decode GEMM for the 256-row bucket with the activations streamed through REGISTERS
 // ("xr"): Y[256, N] = X[256, K] . W[N, K]^T, bf16 in, fp32 accumulate
-// (SURVEY.md §2.4 N7 decode GEMMs; replaces the external LLM behind
+// (replaces the external LLM behind
 // J/service/AIInterfaceRestClient.java:37-39).
 //
 // Why: at M = 256 the decode GEMMs are bound by what one CU can keep in flight, not by the
-// MFMA (round 5: gemm_pp's gate|up spends 55 of its 71 us loading operands; a CU ingests
+// MFMA (gemm_pp's gate|up spends 55 of its 71 us loading operands; a CU ingests
 // ~ its bytes in flight / ~2.1 us, profiles/decode_gemm_ingest_gate_up.jsonl). Every
 // workgroup of a column tile needs ALL 256 activation rows, so X is 2/3 of what a CU
 // ingests, and with both operands staged through LDS the 160 KiB of LDS caps what is in
@@ -123,7 +123,7 @@ __global__ void __launch_bounds__(256) gemm_xr_kernel(const bf16_t* __restrict__
 
   // Issue order (what every vmcnt below counts): prologue X(0), W(0), X(1), W(1), X(2), W(2),
   // W(3) .. W(NS-1) -- the first step's operands first, so its wait is not behind the whole
-  // weight prefill (in-order vmcnt: the round-6 first cut issued W(0..7) first and its first
+  // weight prefill (in-order vmcnt: a first cut issued W(0..7) first and its first
   // MFMA waited for 128 KiB per CU); then in the middle of step s: X(s + PX) into ring slot
   // (s + PX) % R (last read by step s - 1) and W(s + NS) into LDS buffer s % NS (released by
   // the barrier just passed), each only if < T.

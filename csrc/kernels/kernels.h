@@ -140,7 +140,7 @@ int sample_tokens(const void* logits, bool logits_bf16, int64_t stride, int rows
                   int64_t* out_tokens, int64_t col_offset, float* out_val, float* part, hipStream_t stream);
 int sample_parts(int rows, int vocab);   // part: 2 x rows x sample_parts floats, or nullptr (one workgroup per row)
 
-// One-shot all-reduce over peer-mapped fine-grained buffers (allreduce.hip, SURVEY.md X1).
+// One-shot all-reduce over peer-mapped fine-grained buffers (allreduce.hip).
 size_t car_buffer_bytes(size_t cap_bytes, int world);
 int car_alloc(size_t cap_bytes, int world, void** base, void* handle_out /* 64 B hipIpcMemHandle_t */);
 int car_open(const void* handle, void** ptr);

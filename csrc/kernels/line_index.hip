@@ -1,4 +1,4 @@
-// Line index and context windows of the pattern scan (SURVEY.md §2.4 N3; replaces the
+// Line index and context windows of the pattern scan (replaces the
 // log-parser's line splitting behind J/service/LogParserRestClient.java:37-39):
 //
 //  * line_prefix: exclusive prefix of the per-segment newline counts ac_scan produced

@@ -1,7 +1,7 @@
 // RMSNorm (+ fused residual add), SiLU-and-mul, embedding gather.
 //
 // These are the memory-bound elementwise/normalisation ops of the explanation
-// model (SURVEY.md §2.4 N9, N13, N15). All bf16 traffic is 16 B per lane.
+// model. All bf16 traffic is 16 B per lane.
 #include "common.h"
 #include "kernels.h"
 

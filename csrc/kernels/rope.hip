@@ -1,4 +1,4 @@
-// Fused RoPE + paged KV-cache write (SURVEY.md §2.4 N10).
+// Fused RoPE + paged KV-cache write.
 //
 // Input is the packed output of the fused QKV projection, one row per token:
 //   qkv[t] = [ q(Hq*D) | k(Hkv*D) | v(Hkv*D) ]  (bf16)

@@ -1,4 +1,4 @@
-// Token sampler (SURVEY.md §2.4 N14): temperature + Gumbel-max over the
+// Token sampler: temperature + Gumbel-max over the
 // vocabulary (or one tensor-parallel vocab shard: col_offset + out_val let the
 // caller take the max over shards, Gumbel-max being decomposable), greedy when temperature <= 0. Several workgroups
 // per row, each on a run of columns, then a merge (few rows leave CUs idle: 1 row of 128256 28 us on one

@@ -1,4 +1,4 @@
-// Launchers for the multi-pattern log scan (SURVEY.md §2.4 N2/N3).
+// Launchers for the multi-pattern log scan.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

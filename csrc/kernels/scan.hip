@@ -1,5 +1,5 @@
 // Multi-pattern log scan: Aho-Corasick DFA walk over a batch of pod logs
-// (SURVEY.md §2.4 N2 ac_scan + N3 line index), replacing the reference's
+// and the line index of its matches, replacing the reference's
 // external log-parser service (J/service/LogParserRestClient.java:37-39).
 //
 // Data layout (built by the host packer, csrc/patterns/patterns.cpp):

@@ -1,4 +1,4 @@
-// Pattern-event scoring on the GPU (SURVEY.md §2.4 N5 "score_reduce").
+// Pattern-event scoring on the GPU.
 //
 // Input: verified matcher hits sorted by (doc, matcher, line), unique, with a
 // CSR doc index; the pattern table as CSR arrays. Two kernels:

@@ -1,18 +1,18 @@
 // Host-side pattern data plane (operator_amd._patterns), CPU only.
 //
-//  * compile_dfa   (SURVEY.md §2.4 N1): literal factors -> Aho-Corasick trie ->
+//  * compile_dfa: literal factors -> Aho-Corasick trie ->
 //    complete DFA over case-folded byte equivalence classes, states numbered
 //    breadth-first (shallow = hot = first rows, staged in LDS by ac_scan),
 //    uint16 table with an "has outputs" flag bit, CSR output lists.
 //  * pack_docs: lays a batch of pod logs out for ac_scan (NUL-padded to a
 //    multiple of the segment size) and memcpys them into a (pinned) staging
 //    buffer with a thread pool, so H2D is one contiguous copy.
-//  * score_events (SURVEY.md §2.4 N5 host path): turns verified factor hits
+//  * score_events: turns verified factor hits
 //    into scored events per doc (proximity search of secondary matchers), the
 //    same algorithm as operator_amd/patterns/oracle.py.
 //
 // Replaces the reference's external log-parser (J/service/LogParserClient.java:36-55);
-// the pattern schema and scoring are our design (SURVEY.md §2.2).
+// the pattern schema and scoring are our design.
 #include <pybind11/pybind11.h>
 #include <pybind11/numpy.h>
 #include <pybind11/stl.h>

@@ -1,7 +1,6 @@
 // Native verification of regex candidate lines and context-window extraction
-// (SURVEY.md §2.4 N3 "line_index + context windows" and N4 "verify": "Confirms
-// regex candidates flagged by N1 on the matched line only ... bit-exact with the
-// Python regex oracle"). Replaces the log-parser's matching semantics behind
+// (regex candidates flagged by the literal scan are confirmed on the matched line only,
+// bit-exact with the Python regex oracle). Replaces the log-parser's matching semantics behind
 // J/service/LogParserRestClient.java:37-39.
 //
 // * RegexProg: a Pike VM (Thompson NFA simulation) over a bytecode the Python side

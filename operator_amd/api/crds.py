@@ -8,9 +8,9 @@ tests/test_crds.py checks the equivalence against the reference files when
 they are present.
 
 Deployment shape (ours): the operator and its GPU engines are ONE pod per
-node-GPU group (no separate log-parser / ai-interface services, SURVEY.md §2.3),
+node-GPU group (no separate log-parser / ai-interface services),
 requesting ``amd.com/gpu``. RBAC adds ``apps`` get/list for the owner lookup of
-Events (the reference's ClusterRole lacks it: SURVEY.md Q9).
+Events (the reference's ClusterRole lacks it).
 """
 from __future__ import annotations
 

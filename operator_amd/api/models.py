@@ -2,7 +2,7 @@
 
 The reference takes these classes from its external ``common-lib``
 (pom.xml:83-87, not vendored); they are reconstructed here from every call
-site (SURVEY.md §2.2) and from the CRD schemas
+site and from the CRD schemas
 (src/main/kubernetes/{podmortem,patternlibrary,aiprovider}-crd.yaml).
 Field names are the Kubernetes/JSON camelCase names; Python attribute names
 are snake_case. Unknown fields are preserved (``extra="allow"``) so a

@@ -88,7 +88,7 @@ def cmd_explain(args) -> int:
 
 
 def _build_pool(s, patterns):
-    """One engine process per GPU (SURVEY.md §5.8): the controller stays a CPU process."""
+    """One engine process per GPU: the controller stays a CPU process."""
     from operator_amd.engine.pool import EnginePool, PoolExplainService, PoolMatchService
 
     if s.engine.device == "cpu":

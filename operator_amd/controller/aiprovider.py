@@ -1,4 +1,4 @@
-"""AIProvider reconciler — an extension (SURVEY.md §8 Q14): the reference has no
+"""AIProvider reconciler — an extension: the reference has no
 controller for AIProvider, so its status (phase Pending/Ready/Failed,
 message, lastValidated, observedGeneration; K/aiprovider-crd.yaml:64-77) is
 never written. Here the provider is validated against the on-node engine:

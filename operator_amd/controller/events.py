@@ -5,7 +5,7 @@ reasons, types, message formats and size caps are identical; every Event goes
 to the failed pod and to the Podmortem CR, and to the owning Deployment when
 the pod -> ReplicaSet -> Deployment owner chain resolves.
 
-Deliberate fixes (SURVEY.md §8 Q9): owner resolution runs on the worker pool
+Deliberate fixes: owner resolution runs on the worker pool
 instead of the caller's thread and a 403/404 there is swallowed (the
 reference's RBAC grants no ``apps`` access: K/operator-rbac.yaml:6-17; our
 generated ClusterRole adds get on replicasets/deployments).

@@ -1,4 +1,4 @@
-"""Pod-failure detection and de-duplication (SURVEY.md §5.3).
+"""Pod-failure detection and de-duplication.
 
 Reference semantics: a pod has failed iff any ``containerStatuses[].state.terminated``
 has ``exitCode != 0`` (J/service/PodFailureWatcher.java:147-159); the dedupe
@@ -136,7 +136,7 @@ class FailureDeduper:
 
 def matches_monitor(pod: dict, monitor: dict) -> bool:
     """Podmortem selects pod? matchLabels AND matchExpressions; a selector with neither
-    matches NOTHING (J/service/PodFailureWatcher.java:247-265; SURVEY.md Q2)."""
+    matches NOTHING (J/service/PodFailureWatcher.java:247-265)."""
     from operator_amd.kube.resources import match_selector, selector_is_empty
 
     spec: dict[str, Any] = (monitor or {}).get("spec") or {}

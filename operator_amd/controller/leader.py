@@ -1,7 +1,7 @@
 """Lease-based leader election (coordination.k8s.io/v1).
 
-The reference runs a single replica with no lease (SURVEY.md §5.3 "Elastic
-recovery / leader election: none"; K/operator-deployment.yaml:11). Here
+The reference runs a single replica with no lease
+(K/operator-deployment.yaml:11). Here
 several operator replicas may run: only the Lease holder starts the watcher
 and the reconcilers, and a standby takes over when the holder stops renewing
 (crash, partition) — so pod-failure handling survives the loss of a node.

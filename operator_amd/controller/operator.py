@@ -1,5 +1,4 @@
-"""Operator assembly: the process that replaces the reference's Quarkus app
-(SURVEY.md §3.1 "init").
+"""Operator assembly: the process that replaces the reference's Quarkus app.
 
     kube client (HTTPS or FakeKube)
       -> Podmortem cache (informer) + PodFailureWatcher      (hot path)

@@ -8,7 +8,7 @@
   an exception -> phase Failed "Failed to reconcile: <msg>" (:97-101);
 * refresh interval grammar: ``Ns | Nm | Nh | Nd | NhMm`` (case-insensitive,
   trimmed), anything else -> 1 hour (:282-306);
-* fixes (SURVEY.md Q7/Q8): credentials are read from the PatternLibrary's own
+* fixes: credentials are read from the PatternLibrary's own
   namespace (falling back to ``podmortem-system``), the ``token`` key (or
   ``username`` + ``password``) is base64-DECODED; ``syncedRepositories`` is
   populated {name, lastCommit, syncTime, status, error}.

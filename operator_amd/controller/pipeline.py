@@ -1,5 +1,5 @@
 """The per-failure analysis pipeline, shared by the pod watcher and the
-Podmortem reconciler (Q3 "fix": one code path, one dedupe).
+Podmortem reconciler (one code path, one dedupe).
 
     emitFailureDetected -> collect(log, core events) -> match -> [AI] -> store -> status -> Events
 

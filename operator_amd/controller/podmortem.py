@@ -2,7 +2,7 @@
 
 On every reconcile: list pods in ANY namespace that match spec.podSelector
 (full LabelSelector), route each failed one through the SAME dedupe +
-pipeline as the watcher (SURVEY.md Q3 fix: the reference re-analysed every
+pipeline as the watcher (a fix: the reference re-analysed every
 failed pod on every reconcile and never stored results), then set status
 phase Ready / "Monitoring pods for failures" (:88), or Error /
 "Failed to reconcile: <msg>" (:92-96). ``observedGeneration`` is now set.

@@ -10,7 +10,7 @@ Mirrors J/service/AnalysisStorageService.java:
   retried on 409 up to 5 times with 100 ms doubling backoff (:75-76, :179-187);
   403 on the pod gives up immediately (:188-193).
 
-Race fix (SURVEY.md §5.2 R1/R3): all status writes for one Podmortem go through
+Race fix: all status writes for one Podmortem go through
 one ``StatusWriter`` lock, and the phase/message update is a merge patch of
 just those two fields on a fresh object, so it can never clobber
 ``recentFailures`` (the reference patches the whole status from a stale list).

@@ -1,5 +1,5 @@
 """Real-time pod failure watcher (J/service/PodFailureWatcher.java, the
-reference's hot path; SURVEY.md §3.2).
+reference's hot path).
 
 * one watch on all namespaces, or one per namespace listed in
   ``podmortem.watch.namespaces`` (comma separated, trimmed, empties dropped:

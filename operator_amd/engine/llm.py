@@ -1,5 +1,5 @@
 """LLM generation engine: continuous batching over a paged KV cache with
-hipGraph-captured decode steps (SURVEY.md §2.4 N16, §7.2 step 4-5).
+hipGraph-captured decode steps.
 
 * Admission reserves the pages a request can ever need (prompt + max_tokens),
   so a running request is never preempted; with 288 GB of HBM per GPU the
@@ -120,7 +120,7 @@ def _prefill_bucket_sizes(max_tokens: int) -> list[int]:
     bucket). A batch cut at bucket T (LLMEngine._prefill_cap) holds more than T minus
     one request, so it replays a graph padded by at most ~20 %; with power-of-two
     buckets and a 15 % padding rule, the batches cut at 2-4k tokens missed their bucket
-    and ran eagerly (57 of 231 batches in the round-4 20-wave driver-shaped run, each
+    and ran eagerly (57 of 231 batches in a run of 20 waves, each
     ~400 launches under the operator threads' GIL contention)."""
     out, t = set(), 512
     while t < max_tokens:
@@ -175,7 +175,7 @@ class _BucketState:
         # steps replayed since the last load: the device counter (``step``, bumped by every
         # replay; hist column = step % multi_step) mirrored on the host, so a window needs
         # no kernel to reset it (the one-element fill it replaced sat ~1 ms behind the previous
-        # window's token copy on the GPU at every window boundary, round-4 flagship trace)
+        # window's token copy on the GPU at every window boundary)
         self.step_host = 0
         self.slots = torch.zeros(bp, dtype=torch.long, device=dev)   # per step: cache slot of each row's token
         self.spos = torch.zeros(bp, dtype=torch.long, device=dev)    # per step: sampler stream position

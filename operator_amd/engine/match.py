@@ -14,7 +14,7 @@ GPU path (one call per batch of failures):
   device: context_spans: the +-k line window of every reported event, located in
           the text still resident from the scan; the host slices and decodes them
           (csrc/kernels/line_index.hip, verify.cpp contexts_from_spans).
-The scan tail is eager: a captured hipGraph of it (round 3) scanned a bucket-padded
+The scan tail is eager: a captured hipGraph of it scanned a bucket-padded
 length and cost more than the handful of launches it replaced (0.59 vs 0.40 ms per
 64-log batch, profiles/scan_graph_vs_eager.jsonl); it was removed (docs/PARITY.md).
 CPU path: the same post-processing fed by the pure-Python oracle.
@@ -643,7 +643,7 @@ class MatchEngine:
 
     def _sub_batches(self, docs: list[bytes]) -> list[tuple[int, int]] | None:
         """Doc-aligned (lo, hi) sub-batches of about PIPE_SUB_BYTES for a large GPU batch,
-        else None. BASELINE config 2 (1.2 GB) is H2D-bound on the GPU (~24 ms of its
+        else None. A batch of 1.2 GB is H2D-bound on the GPU (~24 ms of its
         ~27 ms scan) and host-bound after it (~60 ms of verification, scoring, context
         windows and result objects): in sub-batches the next one's pack + H2D + scan runs
         while the host finishes the previous one."""
@@ -806,7 +806,7 @@ class MatchEngine:
 
     def _result(self, doc: bytes, ev: list[oracle.Event], ctxs: list, pod, ms: float,
                 newlines: int | None = None, analysis_id: str | None = None) -> AnalysisResult:
-        # the hot host loop of a scan batch (4096 results for BASELINE config 2): per-pattern
+        # the hot host loop of a scan batch (4096 results of 290 KiB logs): per-pattern
         # constants looked up once (_pattern_info), severities counted by rank, and every
         # model built by _mk from a complete field dict (all fields given, so no defaults /
         # factories to merge)

@@ -1,6 +1,6 @@
 """Multi-GPU engine pool: one engine process per GPU behind the CPU controller.
 
-SURVEY.md §5.8 "Process model": the controller (kube watches, reconcilers,
+Process model: the controller (kube watches, reconcilers,
 sinks) is a CPU process; each GPU gets its own engine process holding the
 log-scan DFA and a TP=1 explanation model (P1 / P2: data parallel over
 failures and over explanation requests). The reference's two single-replica
@@ -12,7 +12,7 @@ local pipes instead of HTTP.
   worker holds the full pattern set and model, so any worker can serve any
   failure; batching happens inside the worker (LocalMatchService micro-batches
   scans, the LLM engine continuously batches explanations).
-* Health loop (SURVEY.md §5.3 "GPU-worker health loop"): a worker that exits
+* Health loop : a worker that exits
   (GPU fault, OOM kill) or stops heart-beating is drained — its in-flight
   requests are re-queued to the surviving workers — and respawned up to
   ``max_restarts`` times.

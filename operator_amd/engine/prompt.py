@@ -1,4 +1,4 @@
-"""Prompt rendering for explanation requests (SURVEY.md §2.4 N6).
+"""Prompt rendering for explanation requests.
 
 The reference forwards ``AIProvider.spec.promptTemplate`` untouched to its
 ai-interface service (J/service/AIInterfaceClient.java:82), which owns the

@@ -1,6 +1,6 @@
 """Wire-compatible REST front for the on-node engines.
 
-Serves the two contracts the reference operator calls (SURVEY.md §2.3), so an
+Serves the two contracts the reference operator calls, so an
 unmodified podmortem operator (or any other client) can point its
 ``quarkus.rest-client.{log-parser,ai-interface}.url`` at this process:
 

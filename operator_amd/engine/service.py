@@ -1,5 +1,5 @@
 """Service fronts used by the controller pipeline (the two REST hops of the
-reference, pulled in-process; SURVEY.md §2.3).
+reference, pulled in-process).
 
 * ``LocalMatchService``  — micro-batching front of a MatchEngine: every
   ``analyze()`` call made within ``max_wait_ms`` of another is scanned in ONE
@@ -117,7 +117,7 @@ class LocalMatchService:
 
 
 class StubMatchService:
-    """The stub log-parser of BASELINE config 1 (``services.match=stub``): one fixed
+    """The stub log-parser of plumbing benchmarks (``services.match=stub``): one fixed
     CRITICAL out-of-memory event per pod, no scan — for benchmarking the operator's and
     the engine pool's plumbing on its own."""
 

@@ -1,4 +1,4 @@
-"""Tokenizer for the explanation model (SURVEY.md §2.4 N6).
+"""Tokenizer for the explanation model.
 
 If a HuggingFace ``tokenizer.json`` is available (model directory or
 ``OAMD_TOKENIZER``) it is used as-is. Otherwise — the normal case offline,

@@ -1,5 +1,5 @@
 """Tensor-parallel serving: one LLM engine replica spread over the ranks of a
-TP group (BASELINE config 5 "Llama-3-70B, TP=8 over xGMI").
+TP group (Llama-3-70B, TP=8 over xGMI).
 
 Every rank holds a column/row shard of the model (models/llama.py) and must
 run the SAME engine steps on the SAME requests: each step's forward has 2

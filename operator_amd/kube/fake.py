@@ -1,7 +1,7 @@
 """FakeKube: an in-memory Kubernetes API server for tests and the plumbing
-benchmark (SURVEY.md §4.2 "Controller integration, CPU").
+benchmark.
 
-The reference has no test double at all (SURVEY.md §4.1). FakeKube models the
+The reference has no test double at all. FakeKube models the
 behaviour the controllers depend on:
 
 * namespaced objects with uid / resourceVersion / generation / creationTimestamp;

@@ -1,6 +1,6 @@
 """Resource descriptors, API errors, label/field selectors.
 
-Every kube verb the reference issues (SURVEY.md §3 tables) goes through one
+Every kube verb the reference issues goes through one
 of these descriptors, for both the in-memory FakeKube and the HTTPS client.
 """
 from __future__ import annotations

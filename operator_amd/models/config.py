@@ -9,10 +9,9 @@ architectures share one decoder (pre-norm RMSNorm, RoPE, GQA, SwiGLU):
   mistral  Mistral-7B v0.2/v0.3 (no sliding window in those releases)
   qwen2    Qwen2 / Qwen2.5 (bias on the q/k/v projections, rms eps 1e-6)
 
-BASELINE.json names Llama-3-8B (TP=1) and Llama-3-70B (TP=8) as the configs.
-There are no checkpoints offline, so weights are random-initialised with the
-exact architecture, or loaded from a local HF safetensors directory whose
-``config.json`` then defines the architecture (``config_from_hf``).
+The benchmarks run Llama-3-8B (TP=1) and Llama-3-70B (TP=8). There are no
+checkpoints offline, so weights are random-initialised with the exact
+architecture, or loaded from a local HF safetensors directory whose ``config.json`` then defines the architecture (``config_from_hf``).
 
   sufolix  Sufolix (``config_from_dir``): hyper-connected residual streams, attention layers
            with their own head sizes, per-head q/k norm and value mixing, dense or

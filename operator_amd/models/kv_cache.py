@@ -1,4 +1,4 @@
-"""Paged KV cache (SURVEY.md §2.4 N10/N12, §7.1 runtime/kvcache).
+"""Paged KV cache.
 
 Layout per layer: K and V tensors [pages, Hkv_local, page_size, D] (bf16) —
 a kv-head's tokens of one page are contiguous, which is what the decode

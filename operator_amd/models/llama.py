@@ -2,7 +2,7 @@
 
 This is the on-node replacement for the reference's external LLM hop
 (ai-interface -> provider, J/service/AIInterfaceClient.java:45-59 and
-AIInterfaceRestClient.java:37-39). Per layer (SURVEY.md §2.4 N7-N15):
+AIInterfaceRestClient.java:37-39). Per layer:
 
     x   = rmsnorm(h)                          HIP  (fused residual add)
     qkv = x @ Wqkv^T                          GEMM (fused QKV projection)

@@ -1,8 +1,7 @@
 """Model-weight cache: one rank's ready-to-run shard (TP-sliced, gate|up interleaved,
 fp8-quantized) as a safetensors file, memory-mapped back at start-up.
 
-SURVEY.md §5.4 ("an optional ... model-weight mmap cache"; the engine is otherwise
-stateless across restarts). The reference has no weights (its LLM is external,
+Optional; the engine is otherwise stateless across restarts. The reference has no weights (its LLM is external,
 J/service/AIInterfaceRestClient.java:37-39); here a restarted engine skips the HF
 read + re-shard + re-quantize (or the random init) and maps the shard it had: the
 file is read by the OS's page cache straight into the device tensors

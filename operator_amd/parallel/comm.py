@@ -1,5 +1,5 @@
 """Collective layer over torch.distributed (backend "nccl" == RCCL on ROCm,
-"gloo" for the CPU test tier). SURVEY.md §2.4 X1 / §5.8.
+"gloo" for the CPU test tier).
 
 * ``init_from_env()`` — torchrun-style env:// rendezvous (RANK, WORLD_SIZE,
   LOCAL_RANK, MASTER_ADDR=127.0.0.1), one process per GPU.
@@ -61,8 +61,7 @@ def init_from_env(backend: str | None = None, timeout_s: int = 600) -> DistInfo:
 
 
 class _CollectiveStats:
-    """Process-wide collective counters for the metrics endpoint (SURVEY.md §5.5 "RCCL
-    time"): calls and bytes per (op, impl); wall time only where the host waits on
+    """Process-wide collective counters for the metrics endpoint: calls and bytes per (op, impl); wall time only where the host waits on
     the call (an RCCL / gloo collective issued eagerly: the launch-to-return time as
     seen by the host; calls recorded into a hipGraph are counted at capture only)."""
 

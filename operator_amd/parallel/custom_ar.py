@@ -1,5 +1,5 @@
 """One-shot / two-shot all-reduce over peer-mapped HBM for tensor-parallel decode
-(SURVEY.md §2.4 X1, §5.8; kernel: csrc/kernels/allreduce.hip).
+(kernel: csrc/kernels/allreduce.hip).
 
 RCCL's ring all-reduce over xGMI takes 2(n-1) dependent link hops; a TP decode
 all-reduce is only M x hidden x 2 B (16 KB per token at 70B), so those hops,

@@ -1,4 +1,4 @@
-"""Pattern set -> literal factors -> DFA (host compile step, SURVEY.md §2.4 N1/N4).
+"""Pattern set -> literal factors -> DFA (host compile step).
 
 Every matcher (primary or secondary) is reduced to *factors*: literals, one of
 which must occur (case-folded) on any line the matcher accepts.

@@ -1,6 +1,6 @@
-"""Regex -> Pike-VM bytecode for the native verifier (csrc/patterns/verify.cpp, SURVEY.md
-§2.4 N4: "Confirms regex candidates flagged by N1 on the matched line only ...
-bit-exact with the Python regex oracle").
+"""Regex -> Pike-VM bytecode for the native verifier (csrc/patterns/verify.cpp: it confirms
+regex candidates flagged by the literal scan on the matched line only, bit-exact with the
+Python regex oracle).
 
 A matcher's verification question is ``re.search(line) is not None``. For the regular
 subset below that answer does not depend on backtracking order (greedy vs lazy,

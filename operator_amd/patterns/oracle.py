@@ -1,6 +1,6 @@
 """CPU reference matcher + scorer: the correctness oracle for the GPU scan.
 
-Semantics (our design, SURVEY.md §2.2 "Decision"):
+Semantics (our design):
 * a log is split into lines on ``\\n``; matcher m hits line L iff
   ``re.search(m.regex, line)`` (bytes regex; IGNORECASE = ASCII folding);
 * every primary hit (doc, L) of pattern p is one event with

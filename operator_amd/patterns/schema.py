@@ -1,5 +1,5 @@
 """Pattern-library schema (OUR design — the reference's pattern format and
-scoring live in external repos/services it never vendors: SURVEY.md §2.2,
+scoring live in external repos/services it never vendors:
 README.md:43-47 of the reference).
 
 A pattern library is a YAML file::
@@ -177,7 +177,7 @@ class PatternSet:
     @staticmethod
     def load_dir(root: str | Path, enabled: Iterable[str] | None = None) -> "PatternSet":
         """Load every *.yaml/*.yml under root (sorted). ``enabled`` filters by file stem
-        or library_id (PatternLibrary.spec.enabledLibraries; SURVEY.md Q8 'fix')."""
+        or library_id (PatternLibrary.spec.enabledLibraries)."""
         root = Path(root)
         en = set(enabled) if enabled else None
         pats: list[Pattern] = []

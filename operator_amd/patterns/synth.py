@@ -7,8 +7,8 @@ available. This module generates both deterministically from a seed:
 * ``catalog_library()``  — ~30 hand-written signatures of common container
   failures (OOM, crash loops, connection errors, JVM/Go/Python crashes...).
 * ``synthetic_library(n)`` — the catalog plus generated signatures up to n
-  patterns (literal and regex primaries, shared secondary phrases), sized like
-  BASELINE.json config 2 ("1k patterns").
+  patterns (literal and regex primaries, shared secondary phrases), up to the
+  thousand that the scan benchmarks take.
 * ``LogFactory`` — fast log synthesis: a pool of benign lines is sampled with
   numpy and failure lines (matching primaries, with secondaries nearby) are
   injected; returns the bytes plus the ground-truth injected pattern ids.

@@ -1,4 +1,4 @@
-"""Prometheus metrics (SURVEY.md §5.5 — the reference exposes none): analyses/s,
+"""Prometheus metrics (the reference exposes none): analyses/s,
 stage latency histograms, scan GB/s, tokens/s, per-GPU HBM, collective (RCCL /
 one-shot all-reduce) calls, bytes and time.
 

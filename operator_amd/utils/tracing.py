@@ -1,4 +1,4 @@
-"""ROCTx ranges + per-failure stage timestamps (SURVEY.md §5.1).
+"""ROCTx ranges + per-failure stage timestamps.
 
 ``trace_range("scan")`` pushes/pops a roctx range (visible in
 ``rocprofv3 --marker-trace`` timelines) when ``libroctx64`` is loadable, and is
