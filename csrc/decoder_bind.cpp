@@ -571,7 +571,7 @@ void head_gemm(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, int64_t 
 }
 
 void gemm_f32(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, int64_t silu_gu, const OptT& gtab, const OptT& rscale,
-              const OptT& partial, int64_t splits) {
+              const OptT& partial, int64_t splits, int64_t rows) {
   TORCH_CHECK(x.dim() == 2 && y.dim() == 2, "gemm_f32: x [M, K], y [M, N]");
   const int64_t M = x.size(0), K = x.size(1), N = w.size(-2);
   need(x, at::kFloat, M * K, "x");
@@ -591,10 +591,10 @@ void gemm_f32(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, int64_t s
     TORCH_CHECK(partial.has_value() && !gtab.has_value() && !rscale.has_value() && N % 4 == 0, "gemm_f32: K slices");
     need(*partial, at::kFloat, splits * M * N, "partial");
   }
-  const bool tiles = oamd::f32_tiles((int)M, (int)K, gtab.has_value());
+  const bool tiles = rows || oamd::f32_tiles((int)M, (int)K, gtab.has_value());
   const at::Tensor xa = tiles ? on16(x) : x, wa = tiles ? on16(w) : w;
   RC(oamd::gemm_f32(p<float>(xa), p<float>(wa), p<float>(y), op<float>(partial), (int)splits, (int)M, (int)N, (int)K, (int)y.size(1),
-                    (int)silu_gu, op<int>(gtab), op<float>(rscale), cur_stream()));
+                    (int)silu_gu, op<int>(gtab), op<float>(rscale), (int)rows, cur_stream()));
 }
 
 void moe_route(const at::Tensor& h, const at::Tensor& wr, int64_t E, at::Tensor& ids, at::Tensor& weights,
@@ -745,7 +745,7 @@ void register_decoder_bindings(pybind11::module_& m) {
   m.def("head_gemm", &head_gemm, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("x0") = 0, py::arg("nx") = 0);
   m.def("gemm_f32_splits", &oamd::gemm_f32_splits, py::arg("M"), py::arg("N"), py::arg("K"), py::arg("glu"));
   m.def("gemm_f32", &gemm_f32, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("silu_gu") = 0,
-        py::arg("gtab") = no, py::arg("rscale") = no, py::arg("partial") = no, py::arg("splits") = 1);
+        py::arg("gtab") = no, py::arg("rscale") = no, py::arg("partial") = no, py::arg("splits") = 1, py::arg("rows") = 0);
   m.def("moe_route", &moe_route, py::arg("h"), py::arg("wr"), py::arg("E"), py::arg("ids"), py::arg("weights"),
         py::arg("gate") = no, py::arg("logits") = no);
   m.def("moe_topk", &moe_topk, py::arg("logits"), py::arg("E"), py::arg("ids"), py::arg("weights"), py::arg("gate") = no);

@@ -1,7 +1,8 @@
-// True 32-bit forms of the model's products, for models served in fp32 (no reduced-precision
-// matrix mode anywhere): GEMMs (plain, gated, per-expert row groups) on the fp32 matrix instruction and attention
-// for any head size.
+// 32-bit forms of the model's products, for models served in fp32 (32-bit operands, products and
+// sums): GEMMs (plain, gated, per-expert row groups) on the fp32 matrix instruction and attention
+// for any head size. Larger GEMMs run in gemm_f32_split.hip.
 #include "common.h"
+#include "gemm_f32.h"
 #include "kernels.h"
 
 namespace oamd {
@@ -21,21 +22,6 @@ __device__ __forceinline__ f32x4 mfma4(const f32x4& a, const f32x4& b, f32x4 c) 
   return c;
 }
 
-__device__ __forceinline__ float glu1(float g, float u, const GluAct& act) {
-  return g / (1.f + expf(-g * __builtin_fmaf(act.c, g * g, act.a))) * u;
-}
-
-// 4 neighbouring outputs of a row, n valid ones
-__device__ __forceinline__ void put4(float* y, const f32x4& v, int n, bool vec) {
-  if (n >= 4 && vec) {
-    *reinterpret_cast<f32x4*>(y) = v;
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (e < n) y[e] = v[e];
-  }
-}
-
 // 4 neighbouring values of a row, n valid ones, the others 0
 __device__ __forceinline__ f32x4 get4(const float* x, int n) {
   f32x4 v{};
@@ -46,17 +32,6 @@ __device__ __forceinline__ f32x4 get4(const float* x, int n) {
 }
 
 }  // namespace
-
-struct GemmF32 {
-  const float *X, *W;
-  float *Y, *P;          // P: slabs [S][M][N] of S > 1 K slices
-  int M, N, K, S;
-  int64_t ldx, ldy, xh, yh;   // row strides; head strides of X and Y (one product per head, W [H][N][K])
-  const int* gtab;
-  const float* rscale;
-  GluAct act;
-  int vec;               // Y takes 16-B stores
-};
 
 // Y[M, N] = X[M, K] W[N, K]^T in fp32 on the fp32 matrix instruction (full 32-bit products and sums), 64 x 64
 // tiles, four waves of 32 x 32 outputs in 16 x 16 blocks.
@@ -318,10 +293,12 @@ static void launch_skinny(const GemmF32& a, dim3 grid, hipStream_t stream) {
   else gemm_f32_skinny_kernel<GLU, 2, NW><<<grid, 64 * NW, 0, stream>>>(a);
 }
 
-static int run_f32(GemmF32 a, bool glu, int H, hipStream_t stream) {
+static int run_f32(GemmF32 a, bool glu, int H, int rows, hipStream_t stream) {
   const int nf = glu ? a.N / 2 : a.N;
   a.vec = a.ldy % 4 == 0 && a.yh % 4 == 0 && reinterpret_cast<uintptr_t>(a.Y) % 16 == 0;
-  if (!f32_tiles(a.M, a.K, a.gtab != nullptr)) {
+  if (rows) {
+    if (const int rc = gemm_f32_split(a, glu, rows, stream)) return rc;
+  } else if (!f32_tiles(a.M, a.K, a.gtab != nullptr)) {
     const dim3 grid((nf + 15) / 16, 1, H);
     // enough waves to keep the loads of one CU in flight, and work for each of them
     if (glu) launch_skinny<true, 8>(a, grid, stream);
@@ -334,29 +311,30 @@ static int run_f32(GemmF32 a, bool glu, int H, hipStream_t stream) {
     else if (a.S > 1) gemm_f32_kernel<false, true><<<grid, 256, 0, stream>>>(a);
     else if (glu) gemm_f32_kernel<true, false><<<grid, 256, 0, stream>>>(a);
     else gemm_f32_kernel<false, false><<<grid, 256, 0, stream>>>(a);
-    if (a.S > 1) {
-      const int blocks = (int)(((int64_t)a.M * nf / 4 + 255) / 256);
-      if (glu) slabs_f32_kernel<true><<<blocks, 256, 0, stream>>>(a);
-      else slabs_f32_kernel<false><<<blocks, 256, 0, stream>>>(a);
-    }
+  }
+  if (a.S > 1) {
+    const int blocks = (int)(((int64_t)a.M * nf / 4 + 255) / 256);
+    if (glu) slabs_f32_kernel<true><<<blocks, 256, 0, stream>>>(a);
+    else slabs_f32_kernel<false><<<blocks, 256, 0, stream>>>(a);
   }
   OAMD_LAUNCH_CHECK();
   return 0;
 }
 
 int gemm_f32(const float* X, const float* W, float* Y, float* P, int S, int M, int N, int K, int ldy, int glu, const int* gtab,
-             const float* rscale, hipStream_t stream) {
+             const float* rscale, int rows, hipStream_t stream) {
   if (M == 0) return 0;
+  if (rows && ((rows != 64 && rows != 128 && rows != 256) || gtab || rscale)) return -3;
   if (K % 16 || (glu && N % 128) || S < 1 || S > 8) return -1;
-  if (S > 1 && (P == nullptr || gtab || rscale || N % 4 || skinny_rows(M, K))) return -2;
-  return run_f32({X, W, Y, P, M, N, K, S, K, ldy, 0, 0, gtab, rscale, glu ? glu_act(glu) : GluAct{}, 0}, glu != 0, 1, stream);
+  if (S > 1 && (P == nullptr || gtab || rscale || N % 4 || (!rows && skinny_rows(M, K)))) return -2;
+  return run_f32({X, W, Y, P, M, N, K, S, K, ldy, 0, 0, gtab, rscale, glu ? glu_act(glu) : GluAct{}, 0}, glu != 0, 1, rows, stream);
 }
 
 int head_gemm_f32(const float* X, const float* W, float* Y, int M, int N, int K, int H, int64_t ldx, int64_t xh,
                   int64_t ldy, int64_t yh, hipStream_t stream) {
   if (M == 0) return 0;
   if (K % 16 || ldx % 4 || xh % 4 || H < 1 || H > 65535) return -1;
-  return run_f32({X, W, Y, nullptr, M, N, K, 1, ldx, ldy, xh, yh, nullptr, nullptr, GluAct{}, 0}, false, H, stream);
+  return run_f32({X, W, Y, nullptr, M, N, K, 1, ldx, ldy, xh, yh, nullptr, nullptr, GluAct{}, 0}, false, H, 0, stream);
 }
 
 // Attention on the fp32 matrix instruction: S^T = K Q^T, so a lane holds scores of one query (l15) and the

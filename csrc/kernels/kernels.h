@@ -326,9 +326,10 @@ struct HeadGemm {
 int head_gemm(const HeadGemm& a, hipStream_t stream);
 
 // fp32 forms (f32.hip)
+// rows 0: on the fp32 matrix instruction; 64, 128, 256: gemm_f32_split.hip on tiles of so many (any M, no gtab / rscale).
 // S > 1 (where gemm_f32_splits, the count that fills the GPU, gives more; no gtab / rscale): K slices through P [S][M][N].
 int gemm_f32(const float* X, const float* W, float* Y, float* P, int S, int M, int N, int K, int ldy, int glu, const int* gtab,
-             const float* rscale, hipStream_t stream);
+             const float* rscale, int rows, hipStream_t stream);
 int gemm_f32_splits(int M, int N, int K, int glu);
 bool f32_tiles(int M, int K, bool grouped);   // these run on the tile kernel, whose operands are 16-B aligned
 // One product per head: as HeadGemm, without the extra columns.

@@ -499,7 +499,7 @@ def _mid_few_rows(M: int, N: int, K: int, defer: bool) -> bool:
 # Every GPU GEMM of the model runs on the hand-written gfx950 kernels: prompts on gemm_mid or gemm_tile (csrc/kernels/gemm_tile.hip),
 # whichever has the tile rows that fit (tile_rows), in K slices (mid_plan) on gemm_mid, decode buckets on
 # gemm_pp / gemm_tn / gemm_mid / gemm_skinny, the lm_head on whichever of them its rows call for (_mid_beats_skinny,
-# _vocab_plan, mid_plan), fp8 on gemm_fp8 and, past 64 rows, gemm_fp8_tile, fp32 on gemm_f32. hipBLASLt is reached
+# _vocab_plan, mid_plan), fp8 on gemm_fp8 and, past 64 rows, gemm_fp8_tile, fp32 on gemm_f32 in one of its two forms (f32_split_slices). hipBLASLt is reached
 # only by shapes none of them takes (K % 64 != 0, N % 16 != 0, non-bf16), counted in BLAS_CALLS.
 # OAMD_PREFILL_BLAS=1 routes the plain prefill projections (QKV, O, down) to hipBLASLt instead, for
 # A/B runs against the vendor library (profiles/gemm_tile_p5_vs_hipblaslt_r6.jsonl).
@@ -660,15 +660,67 @@ def f32_plan_rows(M: int, prompt: bool) -> int:
     return -(-M // 512) * 512 if prompt and M > SKINNY_MAX_M else M
 
 
+# us, fitted to 4300 products of 17 to 3000 rows of 16 shapes on one MI355X (rms 5 %). The split kernel's tiles of 64 rows, one and two to a CU, of
+# 128 and of 256: a 32-column step with one CU busy, and what it takes more with all of them (power); then the fp32 instruction's, with one, two
+# and three tiles to a CU.
+_F32_SPLIT = {64: (0.69, 0.14), 128: (0.94, 0.40), 256: (1.76, 0.56)}
+_F32_PAIR = 1.37   # two 64-row tiles
+_F32_PLAIN = (0.66, 1.16, 1.70)
+
+
+def _f32_slabs(M: int, N: int, S: int, glu: int) -> float:
+    return 2.2 + 1.3e-6 * M * N * (S + (0.5 if glu else 1)) if S > 1 else 0.0
+
+
+def _f32_split_us(rows: int, S: int, M: int, N: int, K: int, glu: int) -> float:
+    one, busy = _F32_SPLIT[rows]
+    full, last = divmod(-(-M // rows) * -(-N // 128) * S, 2 * CUS if rows == 64 else CUS)
+    t = full * (_F32_PAIR if rows == 64 else one + busy)
+    if last:
+        t += _F32_PAIR if last > CUS else one + busy * last / CUS
+    t = 6 + -(-K // (32 * S)) * t + 1.1 * (full + (last > 0) - 1)
+    return max(t, 6 + 4e-6 * N * K / 4.5) + _f32_slabs(M, N, S, glu)
+
+
+def _f32_plain_us(M: int, N: int, K: int, glu: int) -> float:
+    S = kernels().gemm_f32_splits(M, N, K, glu)
+    full, last = divmod(-(-(-(-M // 64) * -(-(N // 2 if glu else N) // 64) * S) // CUS), 3)
+    t = 3.2 + -(-K // (32 * S)) * (2 if glu else 1) * (full * _F32_PLAIN[2] + (_F32_PLAIN[last - 1] if last else 0))
+    return max(t, 3.2 + 4e-6 * N * K / 4) + _f32_slabs(M, N, S, glu)
+
+
+@functools.lru_cache(maxsize=4096)
+def f32_split_slices(M: int, N: int, K: int, glu: int) -> int | None:
+    """K slices in which ``M`` rows (f32_plan_rows) run on the split kernel (gemm_f32_split.hip), or None: on the fp32 matrix instruction
+    (f32.hip), up to 32 rows and where the split kernel, whose steps wait for more before the first, is not estimated 10 % faster (512
+    rows of 2048 x 288 9 us against 14, of 2048 x 768 24 and 24, of 2048 x 2048 50 and 37; 2000 rows of 2048 x 288 27 and 20)."""
+    if M <= SKINNY_MAX_M:
+        return None
+    cost, S = min((_f32_split_us(r, s, M, N, K, glu), s) for r in _F32_SPLIT for s in range(1, 9)
+                  if s == 1 or (N % 4 == 0 and K // 32 // s >= 4))
+    return S if cost < 0.9 * _f32_plain_us(M, N, K, glu) else None
+
+
+@functools.lru_cache(maxsize=4096)
+def f32_split_rows(M: int, N: int, K: int, S: int, glu: int) -> int:
+    """Rows of the split kernel's tiles: the sums, and so the bits, are the same for all (the choices take 0.5 % more than the best slices and
+    rows of 318 products)."""
+    return min((_f32_split_us(r, S, M, N, K, glu), r) for r in _F32_SPLIT)[1]
+
+
 def linear_f32(x: torch.Tensor, w: torch.Tensor, glu: int = 0, prompt: bool = False) -> torch.Tensor:
-    """x @ w^T in full 32-bit products and sums, optionally with the gated epilogue (SILU / GELU_TANH) over a 64-row
+    """x @ w^T with 32-bit operands and sums, optionally with the gated epilogue (SILU / GELU_TANH) over a 64-row
     interleaved gate|up weight. ``prompt``: as for ``linear``."""
     M, K = x.shape
     N = w.shape[0]
     y = torch.empty(M, N // 2 if glu else N, dtype=x.dtype, device=x.device)
-    S = kernels().gemm_f32_splits(f32_plan_rows(M, prompt), N, K, glu)
+    plan = f32_plan_rows(M, prompt)
+    S = f32_split_slices(plan, N, K, glu) if M else None
+    rows = 0 if S is None else f32_split_rows(M, N, K, S, glu)
+    if S is None:
+        S = kernels().gemm_f32_splits(plan, N, K, glu)
     part = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if S > 1 else None
-    kernels().gemm_f32(x, w, y, glu, partial=part, splits=S)
+    kernels().gemm_f32(x, w, y, glu, partial=part, splits=S, rows=rows)
     return y
 
 

@@ -187,3 +187,55 @@ def test_latent_decode_f32_wide_rows(rank, splits):
     for b, r in enumerate(rows):
         p = torch.softmax(q[b].double() @ r.double().t() * 0.05, -1)
         torch.testing.assert_close(o[b].double(), p @ r.double()[:, :L.rp], atol=2e-5, rtol=2e-5)
+
+
+@pytest.mark.parametrize("M,N,K,S", [(1, 4, 16, 1), (33, 100, 48, 1), (64, 130, 528, 1), (65, 128, 2032, 3), (129, 260, 1040, 2), (257, 1000, 96, 3),
+                                     (300, 128, 4112, 8), (40, 64, 16, 2)])
+def test_gemm_f32_split(M, N, K, S):
+    """Ragged tiles, a last piece of 16 columns, slices (empty ones too): the bits do not depend on the tile's rows, and the sums are no
+    further from the 64-bit result than the fp32 instruction's."""
+    torch.manual_seed(M + N + K)
+    x, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV)
+    C, r, mag = ops.kernels(), x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+
+    def run(rows, splits, w=w, n=N, glu=0):
+        y = torch.full((M, n), float("nan"), device=DEV)
+        part = torch.full((splits * M * w.shape[0],), float("nan"), device=DEV) if splits > 1 else None
+        C.gemm_f32(x, w, y, glu, partial=part, splits=splits, rows=rows)
+        return y
+
+    for s in {1, S if N % 4 == 0 else 1}:
+        ys = [run(rows, s) for rows in (64, 128, 256)]
+        assert torch.equal(ys[0], ys[1]) and torch.equal(ys[0], ys[2])
+        _close(ys[0], r, mag, K)
+        if K >= 512:
+            assert (ys[0].double() - r).norm() <= 1.02 * (run(0, 1).double() - r).norm()
+    gate, up = torch.randn(128, K, device=DEV) * K ** -0.5, torch.randn(128, K, device=DEV) * K ** -0.5
+    wgu = ops.interleave_gate_up(gate, up)
+    a, b = x.double() @ gate.double().t(), x.double() @ up.double().t()
+    for s in {1, S}:
+        ys = [run(rows, s, wgu, 128, ops.SILU) for rows in (64, 128, 256)]
+        assert torch.equal(ys[0], ys[1]) and torch.equal(ys[0], ys[2])
+        torch.testing.assert_close(ys[0].double(), a * torch.sigmoid(a) * b, atol=2e-5, rtol=2e-5)
+
+
+@pytest.mark.parametrize("rows,S", [(64, 1), (128, 2), (256, 1)])
+def test_gemm_f32_split_keeps_odd_values_and_small_ones(rows, S):
+    """Infinities, NaN and operands whose parts leave bf16's range give what 32-bit products give, in their own rows and columns."""
+    torch.manual_seed(rows)
+    M, N, K = 300, 260, 96
+    x, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV)
+    x[3, 5], x[200, 95], x[77, 0], w[131, 7] = float("inf"), float("-inf"), float("nan"), float("inf")
+    x[150] *= 1e-36           # third parts below bf16's range
+    w[40:45] *= 1e-30
+    x[20, 9], w[200, 3] = 3.4e38, -3.4028234e38   # round to an infinity in bf16
+    x[30] = 0
+    y = torch.empty(M, N, device=DEV)
+    part = torch.empty(S * M * N, device=DEV) if S > 1 else None
+    ops.kernels().gemm_f32(x, w, y, 0, partial=part, splits=S, rows=rows)
+    r = (x.double() @ w.double().t())
+    r32, mag = r.float(), x.double().abs() @ w.double().abs().t()
+    assert torch.equal(y.isnan(), r32.isnan()) and torch.equal(y.isinf() & ~r.isinf(), r32.isinf() & ~r.isinf())
+    assert torch.equal(y[r.isinf()], r32[r.isinf()])
+    fin = r.isfinite() & r32.isfinite()
+    assert ((y[fin].double() - r[fin]).abs() <= (K + 8) * 2.0 ** -24 * mag[fin] + 1e-44).all()
