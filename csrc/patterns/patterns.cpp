@@ -34,6 +34,8 @@
 #include <emmintrin.h>
 #endif
 
+#include "scorer.h"
+
 namespace py = pybind11;
 
 namespace {
@@ -344,11 +346,9 @@ class PackJob {
     past_cache_ = total >= kPastCache && dst % 16 == 0 && seg % 16 == 0;
     done_ = std::vector<std::atomic<uint8_t>>(pieces_.size());
     const int more = std::min<int>(threads, static_cast<int>(pieces_.size())) - 1;
-    if (more > 0) pool_.reserve(more);
-    try {
-      for (int t = 0; t < more; ++t) pool_.emplace_back([this] { while (step()) {} });
-    } catch (const std::exception&) {   // no more threads to be had: those there are, and the waiting one
-    }
+    if (more > 0) pool_.resize(more);
+    start(0);
+    start(1);
   }
   ~PackJob() { close(); }
 
@@ -367,7 +367,8 @@ class PackJob {
     next_.store(pieces_.size());
     if (pool_.empty()) return;
     py::gil_scoped_release nogil;
-    for (auto& th : pool_) th.join();
+    for (auto& th : pool_)   // a thread's own two come behind it
+      if (th.joinable()) th.join();
     pool_.clear();
   }
 
@@ -380,6 +381,20 @@ class PackJob {
   static constexpr int64_t kPackPiece = 256 << 10;
   // 84 MB in place on the GPU: 1.9 ms past the caches, 2.1 to 2.3 through them; 4.6 MB the same either way
   static constexpr size_t kPastCache = 8 << 20;
+
+  // Thread t, which starts 2 t + 2 and 2 t + 3 before it copies: one takes 14 us to start, so fifteen of them one behind the other kept the
+  // first piece waiting for 220 us.
+  void start(size_t t) {
+    if (t >= pool_.size()) return;
+    try {
+      pool_[t] = std::thread([this, t] {
+        start(2 * t + 2);
+        start(2 * t + 3);
+        while (step()) {}
+      });
+    } catch (const std::exception&) {   // no more threads to be had: those there are, and the waiting one
+    }
+  }
 
   bool step() {
     size_t i = next_.load(std::memory_order_relaxed);
@@ -409,109 +424,6 @@ void pack_docs(std::vector<py::bytes> docs, const std::vector<int64_t>& first, i
   PackJob(std::move(docs), first, seg, dst, threads).wait(n);
 }
 
-// ---------------------------------------------------------------------------
-// Event scoring. Inputs are per-hit arrays (doc, matcher, line) of VERIFIED,
-// de-duplicated hits, plus per-pattern matcher tables. Algorithm (our design,
-// mirrored exactly by operator_amd/patterns/oracle.py::score_doc):
-//   for each primary hit (doc d, line L) of pattern p:
-//     bonus = sum_j w_j * (1 - |dL_j| / (W_j + 1))  over secondaries j whose
-//             nearest hit in doc d lies within |dL_j| <= W_j
-//     score = confidence_p * (1 + bonus) / (1 + sum_j w_j)
-// Events are sorted by (score desc, severity desc, doc line asc, pattern asc).
-// ---------------------------------------------------------------------------
-struct PatSpec {
-  int primary;
-  double confidence;
-  int severity;
-  std::vector<int> sec;
-  std::vector<double> weight;
-  std::vector<int> window;
-};
-
-// A pattern set's scoring tables, kept between batches; score() is the host form of the scorer.
-class Scorer {
- public:
-  Scorer(const std::vector<int64_t>& primary, std::vector<double> conf, std::vector<int64_t> sev,
-         std::vector<std::vector<int64_t>> sec, std::vector<std::vector<double>> w, std::vector<std::vector<int64_t>> win,
-         int64_t num_matchers)
-      : conf_(std::move(conf)), sev_(std::move(sev)), sec_(std::move(sec)), w_(std::move(w)), win_(std::move(win)), primary_of_(num_matchers) {
-    const size_t P = primary.size();
-    if (conf_.size() < P || sev_.size() < P || sec_.size() < P || w_.size() < P || win_.size() < P)
-      throw std::invalid_argument("pattern tables shorter than the patterns");
-    for (size_t p = 0; p < P; ++p) {
-      if (primary[p] < 0 || primary[p] >= num_matchers) throw std::out_of_range("pattern primary");
-      if (w_[p].size() < sec_[p].size() || win_[p].size() < sec_[p].size()) throw std::invalid_argument("secondary tables too short");
-      primary_of_[primary[p]].push_back(static_cast<int>(p));
-    }
-  }
-
-  // hits [n, 3] = (doc, matcher, line) -> per doc its events (pattern, line, score), best first
-  py::list score(py::array_t<int64_t, py::array::c_style | py::array::forcecast> hits, int64_t num_docs) const {
-    if (hits.ndim() != 2 || hits.shape(1) != 3) throw std::invalid_argument("hits [n, 3]");
-    const int64_t* h = hits.data();
-    std::vector<std::vector<std::pair<int64_t, int64_t>>> by_doc(num_docs);  // (matcher, line)
-    for (py::ssize_t i = 0; i < hits.shape(0); ++i, h += 3) {
-      if (h[0] < 0 || h[0] >= num_docs) throw std::out_of_range("hit doc");
-      by_doc[h[0]].emplace_back(h[1], h[2]);
-    }
-    py::list result;
-    std::vector<Ev> evs;
-    for (auto& v : by_doc) {
-      std::sort(v.begin(), v.end());
-      v.erase(std::unique(v.begin(), v.end()), v.end());
-      evs.clear();
-      for (const auto& hit : v) {
-        if (hit.first < 0 || hit.first >= (int64_t)primary_of_.size()) continue;
-        for (int p : primary_of_[hit.first]) {
-          double bonus = 0.0, wsum = 0.0;
-          for (size_t j = 0; j < sec_[p].size(); ++j) {
-            const double w = w_[p][j];
-            wsum += w;
-            const int64_t dist = nearest(v, sec_[p][j], hit.second);
-            if (dist >= 0 && dist <= win_[p][j]) bonus += w * (1.0 - double(dist) / double(win_[p][j] + 1));
-          }
-          evs.push_back({conf_[p] * (1.0 + bonus) / (1.0 + wsum), static_cast<int>(sev_[p]), hit.second, p});
-        }
-      }
-      std::sort(evs.begin(), evs.end(), [](const Ev& a, const Ev& b) {
-        if (a.score != b.score) return a.score > b.score;
-        if (a.sev != b.sev) return a.sev > b.sev;
-        if (a.line != b.line) return a.line < b.line;
-        return a.pat < b.pat;
-      });
-      py::list dl(evs.size());
-      for (size_t i = 0; i < evs.size(); ++i) dl[i] = py::make_tuple(evs[i].pat, evs[i].line, evs[i].score);
-      result.append(std::move(dl));
-    }
-    return result;
-  }
-
- private:
-  struct Ev { double score; int sev; int64_t line; int pat; };
-
-  // distance of the nearest line of matcher m among a doc's sorted hits, or -1
-  static int64_t nearest(const std::vector<std::pair<int64_t, int64_t>>& v, int64_t m, int64_t line) {
-    auto lo = std::lower_bound(v.begin(), v.end(), std::make_pair(m, line));
-    int64_t best = -1;
-    if (lo != v.end() && lo->first == m) best = lo->second - line;
-    if (lo != v.begin()) {
-      auto pr = std::prev(lo);
-      if (pr->first == m) {
-        const int64_t dd = line - pr->second;
-        if (best < 0 || dd < best) best = dd;
-      }
-    }
-    return best;
-  }
-
-  std::vector<double> conf_;
-  std::vector<int64_t> sev_;
-  std::vector<std::vector<int64_t>> sec_;
-  std::vector<std::vector<double>> w_;
-  std::vector<std::vector<int64_t>> win_;
-  std::vector<std::vector<int>> primary_of_;
-};
-
 py::list score_events(const std::vector<int64_t>& hit_doc, const std::vector<int64_t>& hit_matcher,
                       const std::vector<int64_t>& hit_line, int64_t num_docs, const std::vector<int64_t>& pat_primary,
                       const std::vector<double>& pat_conf, const std::vector<int64_t>& pat_sev,
@@ -532,6 +444,7 @@ py::list score_events(const std::vector<int64_t>& hit_doc, const std::vector<int
 }  // namespace
 
 void register_verify(py::module_& m);   // verify.cpp (N3 / N4)
+void register_results(py::module_& m);  // results.cpp
 
 PYBIND11_MODULE(_patterns, m) {
   m.doc() = "operator_amd host pattern compiler / packer / scorer";
@@ -557,4 +470,5 @@ PYBIND11_MODULE(_patterns, m) {
   m.attr("MAX_FACTOR_LEN") = kMaxFactorLen;
   m.attr("MAX_STATES") = kMaxStates;
   register_verify(m);
+  register_results(m);
 }

@@ -12,8 +12,9 @@ GPU path (one call per batch of failures):
   host  : factor -> matcher expansion, regex verification of candidate lines
           only, native event scoring (or the score_reduce kernel)
   device: context_spans: the +-k line window of every reported event, located in
-          the text still resident from the scan; the host slices and decodes them
-          (csrc/kernels/line_index.hip, verify.cpp contexts_from_spans).
+          the text still resident from the scan (csrc/kernels/line_index.hip)
+  host  : context lines decoded and result objects built natively
+          (csrc/patterns/results.cpp)
 The scan tail is eager: a captured hipGraph of it scanned a bucket-padded
 length and cost more than the handful of launches it replaced (0.59 vs 0.40 ms per
 64-log batch, profiles/scan_graph_vs_eager.jsonl); it was removed (docs/PARITY.md).
@@ -165,12 +166,15 @@ class MatchEngine:
     """Compile a PatternSet once, then analyze batches of logs on one device."""
 
     SCAN_LANES = 256 * 1024   # ac_scan v2 streams on MI355X (256 CUs x 1024 threads)
-    HOST_SCORE_HITS = 2048
-    # context windows of a few logs' events are read from the logs on the host (3 events: 1 us against 39 for the round
-    # trip; 192: 71 against 86; 768: 323 against 307); larger batches leave the host to the next batch's packing
+    # hits that are scored natively, and whose results are built so: 3077 events of 1024 logs 10.9 ms, 18.4 by way of the GPU's sorts and Python's
+    # results; 12828 of 64 logs 7.7 and 18.3
+    HOST_SCORE_HITS = 1 << 16
+    # context windows of a few logs' events are located on the host (3 events: 1 us against 30 for the round trip to the GPU);
+    # larger batches leave the host to the next batch's packing
     HOST_CONTEXT_DOCS = 8
     HEAD_MATCHES = 2048       # match records read back with the count (a 64-log batch has some hundred)
     PACK_CHUNK = 16 << 20     # bytes of an upload while the host packs on (84 MB: 1.9 ms; 4 MB 2.0, 1 MB 2.5)
+    PACK_FIRST = 2 << 20      # ... of the first one
 
     def __init__(self, patterns: PatternSet | CompiledPatterns, device: str | torch.device = "cuda",
                  seg_bytes: int = 1024, max_events: int = 50, significance: float = 0.5,
@@ -193,10 +197,9 @@ class MatchEngine:
         self.use_native_scorer = use_native_scorer
         # score + rank events on the GPU (score.hip) when scanning there
         self.gpu_scorer = (self.device.type == "cuda") if gpu_scorer is None else gpu_scorer
-        # ... unless it is asked for, batches of few hits go to the native scorer: the round trip to the GPU takes 65 us
-        # for 3 hits (5 here) and 195 for 195 (130); past some thousand the sorts are the GPU's
+        # ... unless it is asked for, only from HOST_SCORE_HITS hits on (the round trip to the GPU takes 65 us for 3 hits, 5 here)
         self._gpu_score_from = 0 if gpu_scorer else self.HOST_SCORE_HITS
-        self._scorer = None
+        self._scorer = self._tables = None
         self._score_tables = None
         self.stats = ScanStats()
         # the scan's text and doc layout stay on the GPU until the next scan: the context
@@ -208,6 +211,8 @@ class MatchEngine:
         self._work: torch.Tensor | None = None
         self._head_h: torch.Tensor | None = None
         self._recs: torch.Tensor | None = None
+        self._query_h: torch.Tensor | None = None
+        self._span_h: torch.Tensor | None = None
         self._doc_newlines: tuple[list[bytes], list[int]] | None = None   # (docs, newlines) of the last GPU scan
         # matcher -> list of (pattern) where it is primary, for quick checks
         self._nm = self.cp.num_matchers
@@ -378,7 +383,8 @@ class MatchEngine:
         try:
             a = 0
             while a < nd:
-                b = min(nd, max(a + 1, bisect.bisect_left(first, first[a] + -(-self.PACK_CHUNK // seg), a + 1)))
+                chunk = self.PACK_CHUNK if a else self.PACK_FIRST
+                b = min(nd, max(a + 1, bisect.bisect_left(first, first[a] + -(-chunk // seg), a + 1)))
                 lo, hi = first[a] * seg, first[b] * seg
                 job.wait(b)
                 if self.profile_bytes > 0 and not self._profiled:
@@ -416,29 +422,23 @@ class MatchEngine:
         hits = read[front:front + 16 * cnt] if cnt <= head else recs[front:front + 16 * cnt].cpu().numpy()
         return hits.view(np.int32).reshape(-1, 4).astype(np.int64), (docs, base_t, lens_t, text), (docs, newlines)
 
-    def _contexts_gpu(self, docs: list[bytes], q_doc: list[int], q_off: list[int], q_k: list[int],
-                      resident: tuple | None = None, stream=None):
-        """Context windows of the reported events located in the text the last GPU scan
-        (or the given ``resident`` one) left on the GPU (None when that scan was not of
-        ``docs``: the host path)."""
-        from operator_amd.ops import kernels, patterns
+    def _contexts_gpu(self, docs: list[bytes], queries: np.ndarray, resident: tuple | None = None, stream=None) -> np.ndarray | None:
+        """(window start, window end, line start, line end) of every query (doc, byte offset, lines), located in the text the last GPU
+        scan (or the given ``resident`` one) left on the GPU; None when that scan was not of ``docs``: the host path."""
+        from operator_amd.ops import kernels
 
         r = self._resident if resident is None else resident
-        if r is None or r[0] is not docs or not q_doc:
+        if r is None or r[0] is not docs or not len(queries):
             return None
         _, base, lens, text = r
-        n = len(q_doc)
-        # every input is made on the scan stream, where the kernel runs: the engine thread's
-        # stream (the LLM's decode graphs, tens of ms deep) would let the kernel read the
-        # query / length / base buffers before their copies land (a memory fault in the
-        # flagship pipeline)
+        n = len(queries)
+        q, out = self._ensure("_query_h", 3 * n, torch.int64, pinned=True), self._ensure("_span_h", 4 * n, torch.int64, pinned=True)
+        q.numpy()[:3 * n] = queries.reshape(-1)
+        # the kernel runs on the scan stream, behind the scan, and reads and writes pinned memory: no copy on a stream that the
+        # LLM's decode graphs keep busy for tens of ms
         with (torch.cuda.stream(stream) if stream is not None else self._on_stream()):
-            q = torch.empty(n, 3, dtype=torch.int64, pin_memory=True)
-            q.numpy().T[:] = q_doc, q_off, q_k
-            out = torch.empty(n, 4, dtype=torch.int64, device=self.device)
-            kernels().context_spans(text, base, lens, q.to(self.device, non_blocking=True), out)
-            spans = out.cpu().numpy()
-        return patterns().contexts_from_spans(docs, q_doc, spans)
+            kernels().context_spans_pinned(text, base, lens, q, out, n)
+        return out.numpy()[:4 * n].reshape(n, 4)
 
     def scan_cpu(self, docs: list[bytes]) -> np.ndarray:
         """Same contract as scan_gpu, computed with Python (used without a GPU)."""
@@ -461,12 +461,20 @@ class MatchEngine:
     # ------------------------------------------------------------------ analysis
     def hits(self, docs: list[bytes]) -> tuple[np.ndarray, dict]:
         """Verified, de-duplicated matcher hits [n, 3] = (doc, matcher, line) + offsets."""
+        return self._split_hits(self._scan_and_verify(docs))
+
+    @staticmethod
+    def _split_hits(rows: np.ndarray) -> tuple[np.ndarray, dict]:
+        return np.ascontiguousarray(rows[:, :3]), dict(zip(map(tuple, rows[:, :3].tolist()), rows[:, 3].tolist()))
+
+    def _scan_and_verify(self, docs: list[bytes]) -> np.ndarray:
         t0 = time.perf_counter()
         raw = self.scan_gpu(docs) if (self.device.type == "cuda" and self.cp.factors) else (
             self.scan_cpu(docs) if self.cp.factors else np.zeros((0, 4), np.int64))
-        return self._hits_from_raw(docs, raw, t0)
+        return self._verified(docs, raw, t0)
 
-    def _hits_from_raw(self, docs: list[bytes], raw: np.ndarray, t0: float) -> tuple[np.ndarray, dict]:
+    def _verified(self, docs: list[bytes], raw: np.ndarray, t0: float) -> np.ndarray:
+        """Hits [n, 4] = (doc, matcher, line, byte offset), each (doc, matcher, line) once, in order."""
         t1 = time.perf_counter()
         from operator_amd.ops import patterns
 
@@ -504,12 +512,10 @@ class MatchEngine:
             keep = np.ones(allh.shape[0], dtype=bool)
             keep[1:] = np.any(allh[1:, :3] != allh[:-1, :3], axis=1)
             allh = allh[keep]
-        offs = dict(zip(map(tuple, allh[:, :3].tolist()), allh[:, 3].tolist()))
-        arr = np.ascontiguousarray(allh[:, :3])
-        self.stats.verified_hits += arr.shape[0]
+        self.stats.verified_hits += allh.shape[0]
         self.stats.scan_ms += (t1 - t0) * 1e3
         self.stats.host_ms += (time.perf_counter() - t1) * 1e3
-        return arr, offs
+        return allh
 
     def _gpu_tables(self):
         """Static pattern tables for score.hip (CSR), uploaded once per pattern set."""
@@ -581,22 +587,27 @@ class MatchEngine:
         hits, offs = self.hits(docs)
         return self._events_from_hits(docs, hits), offs
 
+    def _scores_on_gpu(self, hits: int) -> bool:
+        return self.gpu_scorer and self.device.type == "cuda" and not (self.use_native_scorer and hits <= self._gpu_score_from)
+
+    def _native_scorer(self):
+        if self._scorer is None:   # the pattern tables, once per engine
+            from operator_amd.ops import patterns
+
+            cp, pats = self.cp, self.cp.patset.patterns
+            self._scorer = patterns().Scorer(
+                cp.pattern_primary, [p.primary.confidence for p in pats], [p.severity_rank for p in pats],
+                cp.pattern_secondary, [[s.weight for s in p.secondary] for p in pats],
+                [[s.window for s in p.secondary] for p in pats], cp.num_matchers)
+        return self._scorer
+
     def _events_from_hits(self, docs: list[bytes], hits: np.ndarray, stream=None) -> list[list[oracle.Event]]:
         cp = self.cp
-        few = self.use_native_scorer and len(hits) <= self._gpu_score_from
-        if self.gpu_scorer and self.device.type == "cuda" and not few:
+        if self._scores_on_gpu(len(hits)):
             with (torch.cuda.stream(stream) if stream is not None else self._on_stream()):
                 return self._events_gpu(hits, len(docs))
         if self.use_native_scorer:
-            if self._scorer is None:   # the pattern tables, once per engine
-                from operator_amd.ops import patterns
-
-                pats = cp.patset.patterns
-                self._scorer = patterns().Scorer(
-                    cp.pattern_primary, [p.primary.confidence for p in pats], [p.severity_rank for p in pats],
-                    cp.pattern_secondary, [[s.weight for s in p.secondary] for p in pats],
-                    [[s.window for s in p.secondary] for p in pats], cp.num_matchers)
-            evs = [[oracle.Event(*e) for e in d] for d in self._scorer.score(hits, len(docs))]
+            evs = [[oracle.Event(*e) for e in d] for d in self._native_scorer().score(hits, len(docs))]
         else:
             per: list[set] = [set() for _ in docs]
             for d_, m_, l_ in hits.tolist():
@@ -619,12 +630,12 @@ class MatchEngine:
             if subs is not None:
                 return self._analyze_pipelined(docs, pods, lazy, subs, t0)
             self._doc_newlines = None
-            evs, offs = self.events(docs)
+            score = self._score(docs, self._scan_and_verify(docs))
             t_ev = time.perf_counter()
             nls = self._doc_newlines[1] if self._doc_newlines and self._doc_newlines[0] is docs else None
             self._doc_newlines = None
             self.stats.docs += len(docs)
-            build, n_ctx = self._finish(docs, evs, offs, nls, None, None, pods, 0, t0)
+            build, build_all = self._finish(docs, score, nls, None, None, pods, t0)
             t_ctx = time.perf_counter()
             if lazy:
                 # contexts are done (one batched call); only the result objects are
@@ -632,7 +643,7 @@ class MatchEngine:
                 self.last_timing = {"events_s": t_ev - t0, "contexts_s": t_ctx - t_ev}
                 ms = (t_ctx - t0) * 1e3
                 return LazyResults(lambda di: build(di, ms), len(docs))
-            out = [build(di) for di in range(len(docs))]
+            out = build_all()
             t_end = time.perf_counter()
             self.last_timing = {"events_s": t_ev - t0, "contexts_s": t_ctx - t_ev, "results_s": t_end - t_ctx}
             return out
@@ -699,18 +710,16 @@ class MatchEngine:
                     raise item
                 i, sub, raw, resident, nl, _ = item
                 u0 = time.perf_counter()
-                hits, offs = self._hits_from_raw(sub, raw, u0)
-                evs = self._events_from_hits(sub, hits, self._stream2)
+                score = self._score(sub, self._verified(sub, raw, u0), self._stream2)
                 u1 = time.perf_counter()
                 nls = nl[1] if nl is not None and nl[0] is sub else None
                 lo = subs[i][0]
-                build, _ = self._finish(sub, evs, offs, nls, resident, self._stream2,
-                                        pods[lo:subs[i][1]] if pods else None, lo, t0)
+                build = self._finish(sub, score, nls, resident, self._stream2, pods[lo:subs[i][1]] if pods else None, t0)
                 free.release()   # this buffer set's text is no longer needed
                 u2 = time.perf_counter()
                 t_host += u1 - u0
                 t_ctx_total += u2 - u1
-                builds.append((lo, subs[i][1], build))
+                builds.append((lo, subs[i][1], *build))
         finally:
             stop.set()
             free.release()
@@ -721,7 +730,7 @@ class MatchEngine:
         self.stats.docs += len(docs)
         t_ctx = time.perf_counter()
         owner = [0] * len(docs)
-        for bi, (lo, hi, _) in enumerate(builds):
+        for bi, (lo, hi, *_) in enumerate(builds):
             owner[lo:hi] = [bi] * (hi - lo)
         if lazy:
             ms = (t_ctx - t0) * 1e3
@@ -729,25 +738,51 @@ class MatchEngine:
                                 "pipelined_s": t_ctx - t0}
 
             def get(di: int):
-                lo, _, build = builds[owner[di]]
+                lo, _, build, _ = builds[owner[di]]
                 return build(di - lo, ms)
 
             return LazyResults(get, len(docs))
         out = []
-        for lo, hi, build in builds:
-            out.extend(build(di) for di in range(hi - lo))
+        for _, _, _, build_all in builds:
+            out.extend(build_all())
         t_end = time.perf_counter()
         self.last_timing = {"subs": len(subs), "events_s": t_host, "contexts_s": t_ctx_total,
                             "results_s": t_end - t_ctx, "pipelined_s": t_ctx - t0}
         return out
 
-    def _finish(self, docs: list[bytes], evs: list, offs: dict, nls, resident, stream, pods, doc_base: int,
-                t0: float):
-        """The context windows of every reported event of ``docs`` (one batched call),
-        then a ``build(di, ms=None)`` for result i (``ms`` None: processing time measured
-        at the build). ``offs`` keys use batch-local doc indices."""
+    def _score(self, docs: list[bytes], rows: np.ndarray, stream=None):
+        """The events of verified hits: a native batch (csrc/patterns/results.cpp), which goes on to the results by itself, or, scored
+        on the GPU or in Python, (events per doc, byte offset by (doc, matcher, line))."""
+        if not self.use_native_scorer or self._scores_on_gpu(len(rows)):
+            hits, offs = self._split_hits(rows)
+            return self._events_from_hits(docs, hits, stream), offs
         from operator_amd.ops import patterns
 
+        if self._tables is None:
+            info, pats = self._pattern_info(), self.cp.patset.patterns
+            self._tables = patterns().ResultTables(
+                self._native_scorer(), [p.context_lines for p in pats], [r for r, _, _ in info], [mp for _, mp, _ in info],
+                [rem for _, _, rem in info], SEVERITIES, AnalysisEvent, _EVENT_FIELDS, AnalysisSummary, _SUMMARY_FIELDS,
+                AnalysisResult, _RESULT_FIELDS, self._engine_name())
+        return patterns().ResultBatch(self._tables, docs if type(docs) is list else list(docs), rows, self.max_events, self.significance,
+                                      os.urandom(16 * len(docs)))
+
+    def _finish(self, docs: list[bytes], score, nls, resident, stream, pods, t0: float):
+        """The context windows of every reported event of ``docs`` (one batched call), then ``build(i, ms)`` for result i and
+        ``build_all()``, whose processing times are measured as they are built."""
+        from operator_amd.ops import patterns
+
+        on_gpu = len(docs) > self.HOST_CONTEXT_DOCS
+        if not isinstance(score, tuple):
+            spans = self._contexts_gpu(docs, score.queries(), resident, stream) if on_gpu and len(score) else None
+            score.windows(spans)
+
+            def build(di: int, ms: float) -> AnalysisResult:
+                pod = pods[di] if pods else (None, None)
+                return score.build(di, pod[0], pod[1], -1 if nls is None else nls[di], ms)
+
+            return build, lambda: score.build_all(pods or None, nls, t0)
+        evs, offs = score
         ids = uuid4_strs(len(docs))
         # the +-k context windows of every reported event, extracted natively in one
         # call over the whole batch (N3)
@@ -757,20 +792,22 @@ class MatchEngine:
             q_doc.extend([di] * len(o_))
             q_off.extend(o_)
             q_k.extend(k_)
-        ctxs = self._contexts_gpu(docs, q_doc, q_off, q_k, resident, stream) if q_doc and len(docs) > self.HOST_CONTEXT_DOCS else None
-        if ctxs is None:
-            ctxs = patterns().contexts(docs, q_doc, q_off, q_k) if q_doc else []
+        ctxs = []
+        if q_doc:
+            spans = self._contexts_gpu(docs, np.stack([q_doc, q_off, q_k], 1), resident, stream) if on_gpu else None
+            P = patterns()
+            ctxs = P.contexts(docs, q_doc, q_off, q_k) if spans is None else P.contexts_from_spans(docs, q_doc, spans)
         starts = [0]
         for ev in evs:
             starts.append(starts[-1] + min(len(ev), self.max_events))
 
-        def build(di: int, ms: float | None = None) -> AnalysisResult:
+        def build_one(di: int, ms: float | None = None) -> AnalysisResult:
             return self._result(docs[di], evs[di], ctxs[starts[di]:starts[di + 1]],
                                 pods[di] if pods else (None, None),
                                 (time.perf_counter() - t0) * 1e3 if ms is None else ms,
                                 None if nls is None else nls[di], ids[di])
 
-        return build, len(q_doc)
+        return build_one, lambda: [build_one(di) for di in range(len(docs))]
 
     def _context_queries(self, di: int, doc: bytes, ev: list[oracle.Event], offs: dict) -> tuple[list, list]:
         """(byte offset, context lines) of each reported event of doc ``di``: the offset
@@ -788,6 +825,9 @@ class MatchEngine:
             q_off.append(off)
             q_k.append(pats[e.pattern].context_lines)
         return q_off, q_k
+
+    def _engine_name(self) -> str:
+        return "gpu-ac" if self.device.type == "cuda" else "cpu-oracle"
 
     def _matched(self, pi: int) -> MatchedPattern:
         mp = self._mp_cache.get(pi)
@@ -835,7 +875,7 @@ class MatchEngine:
         return _mk(AnalysisResult, {
             "analysis_id": analysis_id or str(uuid.uuid4()), "pod_name": pod[0], "pod_namespace": pod[1],
             "events": events, "summary": summary,
-            "metadata": {"engine": "gpu-ac" if self.device.type == "cuda" else "cpu-oracle",
+            "metadata": {"engine": self._engine_name(),
                          "patternsChecked": len(info),
                          "totalLines": (doc.count(b"\n") if newlines is None else newlines) + 1,
                          "bytes": len(doc), "processingTimeMs": round(ms, 3)}}, _RESULT_FIELDS)

@@ -99,3 +99,65 @@ def test_default_engine_on_both_sides_of_the_host_threshold(monkeypatch):
             assert sorted((e.pattern, e.line) for e in a) == sorted((e.pattern, e.line) for e in b)
             assert [e.score for e in a] == pytest.approx([e.score for e in b], rel=1e-14)
     assert scored == [n + 1]
+
+
+def _plain(results):
+    """Everything a result holds but its id, its processing time and the object identities."""
+    out = []
+    for r in results:
+        for m in (r, r.summary, *r.events):
+            assert m.__pydantic_fields_set__ == set(type(m).model_fields) and m.__pydantic_extra__ == {} and m.__pydantic_private__ is None
+            assert list(m.__dict__) == list(type(m).model_fields)
+        o = r.model_dump()
+        assert len(o.pop("analysis_id")) == 36 and o["metadata"].pop("processingTimeMs") >= 0
+        out.append(o)
+    return out
+
+
+@pytest.mark.parametrize("max_events", [0, 2, 50])
+@pytest.mark.parametrize("lazy", [False, True])
+def test_native_results_equal_those_built_in_python(lazy, max_events):
+    cp = compile_patterns(synthetic_library(60, seed=2))
+    docs = LogFactory(60, seed=3, pool_lines=256).batch(6, 9000)[0]
+    docs += [b"", b"\n", docs[0].rstrip(b"\n"), docs[1].replace(b"\n", b"\r\n"), docs[2][:2000] + b"\xff\xfe\n" + docs[2][2000:], docs[3] + docs[3]]
+    native, plain = (MatchEngine(cp, device="cpu", use_native_scorer=n, max_events=max_events) for n in (True, False))
+    for pods in (None, [(f"pod-{i}", "ns") for i in range(len(docs))]):
+        a, b = (e.analyze(docs, pods, lazy=lazy) for e in (native, plain))
+        assert _plain(a) == _plain(b)
+    assert any(r.events for r in a) == (max_events > 0) and len({r.analysis_id for r in a}) == len(docs)
+    assert _plain(native.analyze(tuple(docs))) == _plain(plain.analyze(docs))
+    assert native.analyze([]) == [] == plain.analyze([])
+
+
+def test_result_batch_refuses_what_does_not_fit():
+    P, eng = patterns(), MatchEngine(compile_patterns(synthetic_library(20, seed=2)), device="cpu")
+    eng.analyze([b"x\n"])
+    hits = np.asarray([[0, int(eng.cp.pattern_primary[0]), 0, 3]], dtype=np.int64)
+    ok = ([b"abc def\n"], hits, 50, 0.5, bytes(16))
+    for i, bad in ((0, ["text"]), (1, hits[:, :3]), (1, hits + [[1, 0, 0, 0]]), (4, bytes(15))):
+        with pytest.raises((TypeError, ValueError, IndexError)):
+            P.ResultBatch(eng._tables, *ok[:i], bad, *ok[i + 1:])
+    b = P.ResultBatch(eng._tables, *ok)
+    assert b.queries().tolist() == [[0, 3, 3]]
+    with pytest.raises(RuntimeError):
+        b.build(0, None, None, 0, 1.0)
+    for bad in (np.zeros((0, 4), np.int64), np.asarray([[0, 9, 0, 7]]), np.asarray([[3, 7, 0, 7]])):
+        with pytest.raises((ValueError, IndexError)):
+            b.windows(bad)
+    b.windows(np.asarray([[0, 7, 0, 7]]))
+    r = b.build(0, "p", "n", 1, 2.0)
+    assert r.events[0].context == ["abc def"] and r.events[0].matched_line == "abc def" and r.metadata["totalLines"] == 2
+    with pytest.raises(IndexError):
+        b.build(1, None, None, 0, 1.0)
+
+
+@pytest.mark.parametrize("rx,line", [(rb"^ab", b"xab"), (rb"^ab", b"ab"), (rb"a*$", b"bb"), (rb"abc\b", b"zabc abcd"), (rb"aab", b"aaab"), (rb"\Bb", b"ab"),
+                                     (rb"abab(c|$)", b"abaabab"), (rb"a.c", b"aac"), (rb"(^|x)y", b"ay xy"), (rb"abcd", b"abc"), (rb"b", b"")])
+def test_search_passes_over_bytes_no_match_starts_at(rx, line):
+    import re
+
+    from operator_amd.patterns.nfa import compile_nfa
+
+    prog = compile_nfa(rx, 0)
+    assert prog is not None
+    assert patterns().RegexSet([prog]).search(0, line) == (re.search(rx, line) is not None)
