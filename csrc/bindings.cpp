@@ -416,7 +416,7 @@ void gemm_pp(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::T
 }
 
 void gemm_skinny(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& y_opt,
-                 const c10::optional<at::Tensor>& p, int64_t splits, int64_t silu_gu) {
+                 const c10::optional<at::Tensor>& p, int64_t splits, int64_t silu_gu, int64_t blocks) {
   CHECK_DEV(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_CONTIG(x); CHECK_CONTIG(w);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && w.size(1) == x.size(1), "x [M,K], w [N,K]");
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
@@ -430,10 +430,11 @@ void gemm_skinny(const at::Tensor& x, const at::Tensor& w, const c10::optional<a
     TORCH_CHECK(y_opt->dim() == 2 && y_opt->size(0) == M && y_opt->size(1) == (silu_gu ? N / 2 : N), "gemm shapes");
     yp = ptr<bf16_t>(*y_opt);
   } else {
-    TORCH_CHECK(splits > 1 && !silu_gu, "y may be omitted only for split-K slabs summed by the consumer");
+    TORCH_CHECK((splits > 1 || (blocks > 0 && p.has_value())) && !silu_gu, "y may be omitted only for split-K slabs summed by the consumer");
   }
   float* pp = nullptr;
-  if (splits > 1) {
+  TORCH_CHECK(blocks >= 0 && (blocks == 0 || M <= 8), "gemm_skinny: workgroups of up to 8 rows");
+  if (splits > 1 || yp == nullptr) {
     TORCH_CHECK(p.has_value(), "split-K needs a partial buffer");
     CHECK_DT(*p, at::kFloat); CHECK_CONTIG(*p);
     TORCH_CHECK(p->numel() >= splits * M * N, "partial buffer too small");
@@ -443,7 +444,7 @@ void gemm_skinny(const at::Tensor& x, const at::Tensor& w, const c10::optional<a
   TORCH_CHECK(N * K < (1LL << 40) && M * K < (1LL << 31), "gemm too large");
   const c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
   RC(oamd::gemm_skinny(ptr<bf16_t>(x), ptr<bf16_t>(w), yp, pp, (int)M, (int)N, (int)K, (int)splits, (int)silu_gu,
-                       cur_stream()));
+                       (int)blocks, cur_stream()));
 }
 
 void quantize_fp8(const at::Tensor& x, at::Tensor& q, at::Tensor& sx) {
@@ -757,7 +758,7 @@ PYBIND11_MODULE(_C, m) {
         pybind11::arg("sk_ws") = pybind11::none(), pybind11::arg("sk_flags") = pybind11::none());
   m.def("gemm_pp_sk_grid", &oamd::gemm_pp_sk_grid, pybind11::arg("tiles"), pybind11::arg("steps"));
   m.def("gemm_skinny", &gemm_skinny, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("y"),
-        pybind11::arg("p") = pybind11::none(), pybind11::arg("splits") = 1, pybind11::arg("silu_gu") = 0);
+        pybind11::arg("p") = pybind11::none(), pybind11::arg("splits") = 1, pybind11::arg("silu_gu") = 0, pybind11::arg("blocks") = 0);
   m.def("attn_prefill", &attn_prefill, pybind11::arg("q"), pybind11::arg("k"), pybind11::arg("v"),
         pybind11::arg("o"), pybind11::arg("cu_seqlens"), pybind11::arg("work_seq"), pybind11::arg("work_q0"),
         pybind11::arg("scale"), pybind11::arg("block_q") = 64, pybind11::arg("pk") = pybind11::none(),

@@ -1,0 +1,198 @@
+// GEMM for the fewest rows (one to eight): Y[M, N] = X[M, K] . W[N, K]^T, bf16 in, fp32 sums.
+//
+// Nothing but the weights' stream bounds it. On the matrix units a wave's load takes 64 B of each of 16 rows, half a line a request,
+// and reaches 4.5 to 5.8 TB/s; here a wave reads 1 KB of one row per request, past the caches (nothing is read twice): 6.9 TB/s, where a bare
+// read loop reaches 7.2. The products are v_dot2 on the vector units, which eight rows still leave behind the stream; X stays in
+// registers, so a workgroup reads it once for all its rows of W. Four waves share K; a row's sums go over 16 lanes by DPP and over the
+// rest through LDS at the workgroup's end, with no barrier inside the stream. Two register sets of RF rows each are in flight by turns.
+// Measured against gemm_skinny, us: 128256 x 4096 of 1, 4 and 8 rows 151, 155, 164 (183, 199, 217); one row of 28672 x 4096 gated 36 (48),
+// 4096 x 14336 19.4 (24.4), 37888 x 3584 gated 42 (58), 128256 x 8192 301 (380).
+#include <type_traits>
+
+#include "common.h"
+#include "kernels.h"
+
+namespace oamd {
+
+namespace {
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+enum { kRowsStore = 0, kRowsPartial = 1, kRowsGlu = 2 };
+
+template <int CTRL>
+__device__ __forceinline__ float from(float v) {   // of the lane that CTRL names, 0 where it is none
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+constexpr int kNext = 0xb1, kNext2 = 0x4e;   // quad_perm: lane ^ 1, lane ^ 2
+constexpr int row_shr(int n) { return 0x110 + n; }   // lane - n of the same 16
+constexpr int row_shl(int n) { return 0x100 + n; }   // lane + n
+
+// MT values of every lane -> in the last MT lanes of each 16, lane l: the 16 lanes' sum of value l % MT
+template <int MT>
+__device__ __forceinline__ float sums16(const float (&v)[MT], int lane) {
+  float r;
+  if constexpr (MT == 1) {
+    r = v[0] + from<kNext>(v[0]);
+    r += from<kNext2>(r);
+  } else {
+    float h[MT / 2];
+    const bool hi = lane & 1;
+#pragma unroll
+    for (int i = 0; i < MT / 2; ++i) h[i] = (hi ? v[2 * i + 1] : v[2 * i]) + from<kNext>(hi ? v[2 * i] : v[2 * i + 1]);
+    const bool hi2 = lane & 2;
+    if constexpr (MT == 2) {
+      r = h[0] + from<kNext2>(h[0]);
+    } else {
+      r = (hi2 ? h[1] : h[0]) + from<kNext2>(hi2 ? h[0] : h[1]);
+      if constexpr (MT == 8) {   // the last four lanes of eight keep values 4 to 7, and of the values 0 to 3 the lanes before those get theirs
+        const float q = (hi2 ? h[3] : h[2]) + from<kNext2>(hi2 ? h[2] : h[3]);
+        const float hi4 = q + from<row_shr(4)>(q), lo4 = r + from<row_shl(4)>(r);   // every lane takes part in both
+        r = lane & 4 ? hi4 : lo4;
+        return r + from<row_shr(8)>(r);
+      }
+    }
+  }
+  r += from<row_shr(4)>(r);
+  return r + from<row_shr(8)>(r);
+}
+
+}  // namespace
+
+// A workgroup takes rows of W from f0 to f1 (GLU: of gate and up), its four waves a quarter each of the K slice; lane l of wave w holds the
+// X values of its 8 columns in every 512 of the quarter. MT: rows of X, J: 512-column pieces of the quarter, RF: rows of W requested at a time.
+template <int MT, int J, int RF, int EPI>
+__global__ void __launch_bounds__(256) gemm_rows_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, bf16_t* __restrict__ Y,
+                                                        float* __restrict__ P, int M, int N, int K, int S, GluAct act) {
+  constexpr int HALVES = EPI == kRowsGlu ? 2 : 1;
+  extern __shared__ float red[];   // [slot][MT][wave, its 16 lanes]
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int units = N / HALVES;
+  const int f0 = (int)((int64_t)units * blockIdx.x / gridDim.x), nf = (int)((int64_t)units * (blockIdx.x + 1) / gridDim.x) - f0;
+  const int n = nf * HALVES, kz = blockIdx.y, Kw = K / S / 4, k0 = kz * (K / S) + w * Kw;
+  const bool tail = ((J - 1) * 64 + lane) * 8 < Kw;   // this lane has columns in the last piece
+  auto col = [&](int j) { return k0 + (j < J - 1 || tail ? (j * 64 + lane) * 8 : 0); };
+  struct Rows { u32x4 v[RF][J]; } even, odd;
+  auto load = [&](Rows& r, int s0) {
+#pragma unroll
+    for (int i = 0; i < RF; ++i) {
+      const int s = min(s0 + i, n - 1), f = f0 + s / HALVES;
+      const int row = EPI == kRowsGlu ? (f >> 6) * 128 + (f & 63) + (s & 1) * 64 : f;
+      const bf16_t* p = W + (int64_t)row * K;
+#pragma unroll
+      for (int j = 0; j < J; ++j) r.v[i][j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p + col(j)));
+    }
+  };
+  u32x4 x[MT][J];   // requested in front of the first rows: their loop waits for none of its own loads
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int j = 0; j < J; ++j) x[m][j] = *reinterpret_cast<const u32x4*>(X + (int64_t)min(m, M - 1) * K + col(j));
+  load(even, 0);
+  load(odd, RF);
+  __builtin_amdgcn_sched_barrier(0);
+  auto clear = [&](u32x4& v) {   // where the last piece has no columns both operands are 0
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = tail ? v[e] : 0;
+  };
+#pragma unroll
+  for (int m = 0; m < MT; ++m) clear(x[m][J - 1]);
+  auto mul = [&](Rows& r, int s0) {
+    float t[RF];
+#pragma unroll
+    for (int i = 0; i < RF; ++i) {
+      clear(r.v[i][J - 1]);
+      float a[MT] = {};
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            a[m] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, (uint32_t)r.v[i][j][e]), __builtin_bit_cast(bf16x2, (uint32_t)x[m][j][e]), a[m], false);
+      t[i] = sums16<MT>(a, lane);
+    }
+    load(r, s0 + 2 * RF);
+    if ((lane & 15) >= 16 - MT)
+#pragma unroll
+      for (int i = 0; i < RF; ++i) red[((s0 + i) * MT + (lane & (MT - 1))) * 16 + 4 * w + (lane >> 4)] = t[i];
+  };
+  int s = 0;
+  for (; s + RF < n; s += 2 * RF) {
+    mul(even, s);
+    mul(odd, s + RF);
+  }
+  if (s < n) mul(even, s);
+  __syncthreads();
+  auto sum = [&](int slot, int m) {
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(red + (slot * MT + m) * 16 + 4 * i);
+      t += (v[0] + v[1]) + (v[2] + v[3]);
+    }
+    return t;
+  };
+  for (int e = threadIdx.x; e < nf * M; e += 256) {
+    const int m = e / nf, f = e % nf;
+    if constexpr (EPI == kRowsGlu) {
+      const float g = bf2f(f2bf(sum(2 * f, m))), u = bf2f(f2bf(sum(2 * f + 1, m)));
+      Y[(int64_t)m * units + f0 + f] = f2bf(bf2f(f2bf(glu_gate(g, act))) * u);
+    } else if constexpr (EPI == kRowsPartial) {
+      P[((int64_t)kz * M + m) * N + f0 + f] = sum(f, m);
+    } else {
+      Y[(int64_t)m * N + f0 + f] = f2bf(sum(f, m));
+    }
+  }
+}
+
+template <int MT, int J>
+static int launch_rows(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, int N, int K, int S, int glu, int blocks, hipStream_t stream) {
+  if constexpr (MT * J > 32) {
+    return -1;
+  } else {
+    constexpr int RF = J == 1 ? 8 : J == 2 ? 4 : J <= 4 ? 2 : 1;
+    constexpr int GF = RF < 2 ? 2 : RF;
+    const int units = glu ? N / 2 : N, most = (units + blocks - 1) / blocks * (glu ? 2 : 1) + GF;   // slots, and what the last rows run over
+    const size_t lds = (size_t)most * MT * 64;
+    if (lds > (48 << 10)) return -4;
+    const dim3 grid(blocks, S);
+    if (glu) gemm_rows_kernel<MT, J, GF, kRowsGlu><<<grid, 256, lds, stream>>>(X, W, Y, P, M, N, K, 1, glu_act(glu));
+    else if (S > 1 || Y == nullptr) gemm_rows_kernel<MT, J, RF, kRowsPartial><<<grid, 256, lds, stream>>>(X, W, Y, P, M, N, K, S, GluAct{});
+    else gemm_rows_kernel<MT, J, RF, kRowsStore><<<grid, 256, lds, stream>>>(X, W, Y, P, M, N, K, 1, GluAct{});
+    return 0;
+  }
+}
+
+template <int MT>
+static int rows_of(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, int N, int K, int S, int glu, int blocks, hipStream_t stream) {
+  switch ((K / S / 4 + 511) / 512) {
+    case 1: return launch_rows<MT, 1>(X, W, Y, P, M, N, K, S, glu, blocks, stream);
+    case 2: return launch_rows<MT, 2>(X, W, Y, P, M, N, K, S, glu, blocks, stream);
+    case 3: return launch_rows<MT, 3>(X, W, Y, P, M, N, K, S, glu, blocks, stream);
+    case 4: return launch_rows<MT, 4>(X, W, Y, P, M, N, K, S, glu, blocks, stream);
+    case 5: return launch_rows<MT, 5>(X, W, Y, P, M, N, K, S, glu, blocks, stream);
+    case 6: return launch_rows<MT, 6>(X, W, Y, P, M, N, K, S, glu, blocks, stream);
+    case 7: return launch_rows<MT, 7>(X, W, Y, P, M, N, K, S, glu, blocks, stream);
+    case 8: return launch_rows<MT, 8>(X, W, Y, P, M, N, K, S, glu, blocks, stream);
+    default: return -1;
+  }
+}
+
+int gemm_rows(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, int N, int K, int S, int glu, int blocks, hipStream_t stream) {
+  if (M < 1 || M > 8 || S < 1 || S > 8 || K % (32 * S) || N < 1 || blocks < 1) return -1;
+  if (glu && (S != 1 || N % 128)) return -2;
+  if ((S > 1 || Y == nullptr) && P == nullptr) return -3;
+  blocks = blocks < (glu ? N / 2 : N) ? blocks : (glu ? N / 2 : N);
+  int rc;
+  if (M == 1) rc = rows_of<1>(X, W, Y, P, M, N, K, S, glu, blocks, stream);
+  else if (M == 2) rc = rows_of<2>(X, W, Y, P, M, N, K, S, glu, blocks, stream);
+  else if (M <= 4) rc = rows_of<4>(X, W, Y, P, M, N, K, S, glu, blocks, stream);
+  else rc = rows_of<8>(X, W, Y, P, M, N, K, S, glu, blocks, stream);
+  if (rc) return rc;
+  OAMD_LAUNCH_CHECK();
+  return 0;
+}
+
+}  // namespace oamd

@@ -1,5 +1,5 @@
 // Skinny-M GEMM for small decode buckets: Y[M, N] = X[M, K] . W[N, K]^T with
-// M <= 32.
+// M <= 32 (most products of up to 8 rows go to gemm_rows.hip, whose rule is the caller's).
 //
 // At M = 1..32 the step is a pure weight stream (16 GB of bf16 weights per 8B
 // decode step): the kernel's only job is to keep enough W bytes in flight to
@@ -186,13 +186,21 @@ static int skinny_tiles(int M, int N, int Kb, int S, int glu) {
   return best;
 }
 
-int gemm_skinny(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, int N, int K, int S, int glu,
+int gemm_skinny(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, int N, int K, int S, int glu, int blocks,
                 hipStream_t stream) {
   if (M < 1 || M > 32) return -1;
   if (S < 1 || S > 8 || K % (S * sk::kWaves * 32) != 0) return -2;
   if (glu && (S != 1 || N % 128 != 0)) return -3;
   if (N % 16 != 0) return -4;
   if (S > 1 && P == nullptr) return -5;
+  if (blocks > 0) {
+    if (const int rc = gemm_rows(X, W, Y, P, M, N, K, S, glu, blocks, stream)) return rc;
+    if (S > 1 && Y != nullptr) {
+      if ((int64_t)M * N % 4 != 0) return -6;
+      return splitk_reduce(P, Y, (int64_t)M * N, S, stream);
+    }
+    return 0;
+  }
   const int nt = skinny_tiles(M, N, K / S, S, glu), steps = K / S / (sk::kWaves * 32), rounds = (N / (16 * nt) * S + kCus - 1) / kCus;
   // k-steps in flight: long streams of many rounds take more (128256 x 4096, one row: 16 steps 191 us, 8 196; 8 rows on two tiles: 8 steps
   // 222, 4 226), but not where it leaves a remainder, whose steps wait one by one

@@ -72,9 +72,11 @@ int splitk_reduce(const float* P, bf16_t* Y, int64_t MN, int S, hipStream_t stre
 int splitk_silu(const float* P, bf16_t* Y, int M, int N, int S, int glu, hipStream_t stream);
 // Skinny-M decode GEMM (M <= 32, gemm_skinny.hip): N % 16 == 0, K % (128 S) == 0; S-way split-K slabs P
 // reduced into Y (Y == nullptr: left for the consumer); glu: fused SwiGLU over the 64-row
-// interleaved gate|up weight, Y [M, N/2].
-int gemm_skinny(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, int N, int K, int S, int glu,
+// interleaved gate|up weight, Y [M, N/2]. blocks > 0 (M <= 8): gemm_rows on so many workgroups per slice, S == 1 with Y == nullptr too.
+int gemm_skinny(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, int N, int K, int S, int glu, int blocks,
                 hipStream_t stream);
+int gemm_rows(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, int N, int K, int S, int glu, int blocks,
+              hipStream_t stream);
 
 // FP8 e4m3fn W8A8: Y = (X8 . W8^T) * sx[m] * sw[n]; any M (BM-row tiles), S | 8 split-K.
 int gemm_fp8(const uint8_t* X, const uint8_t* W, const float* sx, const float* sw, bf16_t* Y, float* P, int M,

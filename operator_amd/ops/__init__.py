@@ -151,7 +151,11 @@ def gate_up_silu(x: torch.Tensor, wgu: torch.Tensor, block: int | None, act: int
             and K % 128 == 0 and x.is_contiguous() and wgu.is_contiguous()
             and skinny_plan(M, N, K) is not None and _gemm_table_get().get(("silu", M, N, K)) != "blas"):
         y = torch.empty(M, N // 2, dtype=x.dtype, device=x.device)
-        kernels().gemm_skinny(x, wgu, y, None, 1, act)
+        plan = rows_plan(M, N, K, True)
+        if plan is None:
+            kernels().gemm_skinny(x, wgu, y, None, 1, act)
+        else:
+            kernels().gemm_skinny(x, wgu, y, None, 1, act, plan[1])
         return y
     if (x.is_cuda and block == 64 and x.dtype == torch.bfloat16 and M % 64 == 0 and M <= 256 and N % 128 == 0
             and K % 64 == 0 and x.is_contiguous() and wgu.is_contiguous()):
@@ -465,6 +469,38 @@ def skinny_plan(M: int, N: int, K: int) -> int | None:
     return S
 
 
+ROWS_MAX_M = 8
+
+
+@functools.lru_cache(maxsize=4096)
+def rows_plan(M: int, N: int, K: int, glu: bool = False) -> tuple[int, int] | None:
+    """(K slices, workgroups) of one to eight rows on the row-streaming kernel (gemm_rows.hip), or None for gemm_skinny: shorter rows, which
+    leave lanes idle, and products of a few us, where the sums over lanes weigh (M > 4: 2048 x 2048 5.1 us against 4.8, 4096 x 4096 9.0 and 9.7;
+    else 1072 x 2048 3.8 and 3.6, 2048 x 1536 3.7 and 4.3).
+
+    One slice where the rows of X fit in registers. One workgroup per CU for most products (4096 x 14336 19.4 us, 20.6 on two per CU, 22.1 on
+    four), three or four, whichever comes out more even, for those that take 30 us (28672 x 4096 gated 37.1 on one, 36.2 on four); rows of
+    up to 2048 columns in one pass of eight rows a workgroup (32000 x 2048 22.3 on one per CU, 20.4 so), but not on one and a half per CU (3072 x
+    2048: 384 workgroups 4.6, 192 of sixteen rows 4.4)."""
+    if M > ROWS_MAX_M or K % 128 or K < 1536 or N % (128 if glu else 16) or N * K < (2.5e6 if M <= 4 else 8.5e6):
+        return None
+    mt = 1 << (M - 1).bit_length()
+    pieces = lambda s: -(-K // (2048 * s))  # noqa: E731 -- 512 columns a wave and piece
+    S = next((s for s in ((1,) if glu else (1, 2, 4, 8)) if K % (128 * s) == 0 and pieces(s) <= 8 and mt * pieces(s) <= 32), None)
+    if S is None:
+        return None
+    units = N // 2 if glu else N
+    if pieces(S) == 1:
+        B = N // 8 if N // 8 <= CUS or N // 8 >= 2 * CUS else N // 16
+    elif N * K < 9e7 or units < 48 * CUS:
+        B = CUS
+    else:
+        B = -min((-(-units // b) * b, -b) for b in (3 * CUS, 4 * CUS))[1]
+    while (-(-units // B) * (2 if glu else 1) + 8) * mt * 64 > 48 << 10:   # the workgroup's sums in LDS
+        B *= 2
+    return S, B
+
+
 def _mid_beats_skinny(M: int, N: int, K: int, defer: bool) -> bool:
     """gemm_skinny streams the weights once per call but pays for every row (a 128256 x 4096 vocabulary: 191 us at
     1 row, 222 at 8, 300 at 32; 4096 x 14336 26, 27 and 38: 2 % of the one-row time per row, 4 where its tiles do not come in
@@ -498,7 +534,7 @@ def _mid_few_rows(M: int, N: int, K: int, defer: bool) -> bool:
 
 # Every GPU GEMM of the model runs on the hand-written gfx950 kernels: prompts on gemm_mid or gemm_tile (csrc/kernels/gemm_tile.hip),
 # whichever has the tile rows that fit (tile_rows), in K slices (mid_plan) on gemm_mid, decode buckets on
-# gemm_pp / gemm_tn / gemm_mid / gemm_skinny, the lm_head on whichever of them its rows call for (_mid_beats_skinny,
+# gemm_pp / gemm_tn / gemm_mid / gemm_skinny / gemm_rows, the lm_head on whichever of them its rows call for (_mid_beats_skinny,
 # _vocab_plan, mid_plan), fp8 on gemm_fp8 and, past 64 rows, gemm_fp8_tile, fp32 on gemm_f32 in one of its two forms (f32_split_slices). hipBLASLt is reached
 # only by shapes none of them takes (K % 64 != 0, N % 16 != 0, non-bf16), counted in BLAS_CALLS.
 # OAMD_PREFILL_BLAS=1 routes the plain prefill projections (QKV, O, down) to hipBLASLt instead, for
@@ -727,7 +763,7 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, glu: int = 0, prompt: bool = Fa
 def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, splits: int | None = None,
            partial: torch.Tensor | None = None, bn: int | None = None, bm: int | None = None,
            defer_reduce: bool = False, stages: int | None = None, bias: torch.Tensor | None = None, prompt: bool = False):
-    """y = x @ w^T (+ bias) in bf16 on the gfx950 kernels: up to 32 rows on the weight-streaming gemm_skinny, or on
+    """y = x @ w^T (+ bias) in bf16 on the gfx950 kernels: up to 8 rows on gemm_rows (rows_plan), up to 32 on gemm_skinny, or on
     gemm_mid where the rows cost more than its tile (_mid_beats_skinny); 64, 128, 192 and 256 rows on the LDS-staged
     split-K gemm_decode (the measured table, else _decode_tiles; vocabularies _vocab_plan) or where it is estimated
     faster gemm_mid; everything else (prompts, the lm_head of many of them, biased projections) on gemm_mid's tiles of 96 to 160 rows,
@@ -752,6 +788,14 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, sp
     if (x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous() and M <= SKINNY_MAX_M
             and bm is None and bn is None):
         S = splits or skinny_plan(M, N, K)
+        rows = rows_plan(M, N, K) if splits is None and S is not None and (out is None or out.is_contiguous()) else None
+        if rows is not None:
+            deferred = defer_reduce and out is None and max(S, rows[0]) > 1
+            S = rows[0]
+            p = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if deferred or S > 1 else None
+            y = None if deferred else out if out is not None else torch.empty(M, N, dtype=x.dtype, device=x.device)
+            kernels().gemm_skinny(x, w, y, p, S, 0, rows[1])
+            return SplitK(p, S, M, N) if deferred else y
         if (S is not None and splits is None and out is None and _mid_beats_skinny(M, N, K, defer_reduce) and tile_ok(x, w)
                 and (x.data_ptr() | w.data_ptr()) % 16 == 0):
             return linear_tile(x, w, defer_reduce=defer_reduce)
