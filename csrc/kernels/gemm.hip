@@ -19,7 +19,12 @@
 //     [S][M][N] summed by gemm_splitk_reduce (or by a consumer kernel). With
 //     S | 8 the blocks of one K-slice share an XCD (block id % 8), so each
 //     XCD's L2 holds only its slice of X; other S (<= 16) cut K into slices
-//     that differ by at most one 64-column step.
+//     that differ by at most one 64-column step;
+//   * column tile n starts its slice at K step n % steps and goes round. Tiles in step would all read the same 128 columns of rows that lie a
+//     power of two apart, which HBM serves from some of its channels: 64 rows of 128256 x 4096 213 -> 175 us (4.9 -> 6.0 TB/s), 28672 x 4096
+//     gated 46 -> 38, 57344 x 8192 gated 175 -> 148, 32000 x 4096 59 -> 42, 8192 x 8192 32 -> 28; 128 rows of 32000 x 4096 59 -> 53. Where rows
+//     are no such distance apart (3584 columns) it changes nothing. Experts' tiles start 5 steps further an expert: 96 tokens on 8 experts of
+//     4096 x 4096 172 -> 134 us, on 64 of 2048 x 1024 178 -> 150.
 // MFMA v_mfma_f32_16x16x32_bf16; fragment maps as in attn_decode.hip.
 #include "common.h"
 #include "kernels.h"
@@ -36,6 +41,9 @@ constexpr int kStages = 3;  // default LDS ring depth (2: two blocks per CU for 
 // 8 waves (2 per SIMD: one wave's LDS-read latency hides under the other's
 // MFMAs) laid out 4 (M) x 2 (N).
 constexpr int kWaves = 8;
+// Most elements of X whose K steps go round. Tiles in step share a piece of X while it is in their XCD's L2, tiles that are not need all of
+// X there (4 MiB): 128 rows of 8192 x 28672 88 us in step, 96 round, of 3584 x 18944 30 and 41. 256-row tiles are not bound by HBM (32768 x 2048 40 and 43).
+constexpr int64_t kTurnX = 1 << 20;
 
 // BN = 128 halves the LDS fragment traffic per MFMA (64 x 64 wave tiles at
 // M = 256: 0.5 KB of ds_read per MFMA vs 0.75 KB at BN = 64, where the LDS
@@ -83,9 +91,12 @@ __global__ void __launch_bounds__(kWaves * 64, NS == 2 ? 2 : 1) gemm_tn_kernel(c
   const int kz = blockIdx.x % S, nt = blockIdx.x / S;
   const int n0 = nt * BN;
   const int m0 = blockIdx.y * BM;  // row tile (M may be split into BM-row tiles)
+  int turn = nt;
   if constexpr (GRP) {
     if ((int)blockIdx.y >= gtab[0]) return;
-    W += (int64_t)gtab[1 + blockIdx.y] * N * K;
+    const int e = gtab[1 + blockIdx.y];
+    W += (int64_t)e * N * K;
+    turn += 5 * e;
   }
   if (!GRP || src == nullptr) X += (int64_t)m0 * K;
   // K-slice kz = K-steps [kz * TK / S, (kz + 1) * TK / S): slices differ by at most one step
@@ -107,8 +118,9 @@ __global__ void __launch_bounds__(kWaves * 64, NS == 2 ? 2 : 1) gemm_tn_kernel(c
       if (src != nullptr && xrow[i] < BM) xrow[i] = max(src[m0 + xrow[i]], 0);
     }
   }
+  const int off = w_tiled & 4 ? turn % T : 0;
   auto issue_one = [&](int t, int buf, int i) {
-    const int k0 = kbase + t * kBK;
+    const int k0 = kbase + (t + off < T ? t + off : t + off - T) * kBK;
     char* sbase = lds + buf * C::STAGE_BYTES;
     {
       const int q = w + kWaves * i;
@@ -222,10 +234,13 @@ __global__ void __launch_bounds__(kWaves * 64, NS == 2 ? 2 : 1) gemm_tn_kernel(c
       u16x8 o;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const float g = bf2f(f2bf(GRP ? c * cr[f0 + e] : cr[f0 + e]));
-        const float u = bf2f(f2bf(GRP ? c * cr[64 + f0 + e] : cr[64 + f0 + e]));
-        const float sg = bf2f(f2bf(glu_gate(g, act)));
-        o[e] = f2bf(sg * u);
+        if constexpr (GRP) {   // as the list kernel of moe.hip: one rounding
+          const float g = c * cr[f0 + e], u = c * cr[64 + f0 + e];
+          o[e] = f2bf(g / (1.f + __expf(-g)) * u);
+        } else {
+          const float g = bf2f(f2bf(cr[f0 + e])), u = bf2f(f2bf(cr[64 + f0 + e]));
+          o[e] = f2bf(bf2f(f2bf(glu_gate(g, act))) * u);
+        }
       }
       *reinterpret_cast<u16x8*>(Y + (int64_t)(m0 + row) * NO + nt * 64 + f0) = o;
     }
@@ -273,22 +288,22 @@ int moe_gemm_rows(const bf16_t* X, const bf16_t* W, bf16_t* Y, int max_rows, int
   if (silu_gu && rscale == nullptr) return -2;
   const dim3 grid(N / 128, max_rows / bm);
   if (bm == 64 && silu_gu)
-    gemm_tn_kernel<64, 128, kEpiSiluGU, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2, gtab, src, rscale);
+    gemm_tn_kernel<64, 128, kEpiSiluGU, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2 | 4, gtab, src, rscale);
   else if (bm == 64)
-    gemm_tn_kernel<64, 128, kEpiStore, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2, gtab, src, rscale);
+    gemm_tn_kernel<64, 128, kEpiStore, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2 | 4, gtab, src, rscale);
   else if (silu_gu)
-    gemm_tn_kernel<128, 128, kEpiSiluGU, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2, gtab, src, rscale);
+    gemm_tn_kernel<128, 128, kEpiSiluGU, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2 | 4, gtab, src, rscale);
   else
-    gemm_tn_kernel<128, 128, kEpiStore, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2, gtab, src, rscale);
+    gemm_tn_kernel<128, 128, kEpiStore, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2 | 4, gtab, src, rscale);
   OAMD_LAUNCH_CHECK();
   return 0;
 }
 
 int gemm_decode(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, int N, int K, int S, int BN,
                 int BM, int glu, bool w_tiled_b, int stages, hipStream_t stream) {
-  // bit 0: tiled W layout; bit 1: W streams with the non-temporal policy (OAMD_BF16_WNT)
+  // bit 0: tiled W layout; bit 1: W streams with the non-temporal policy (OAMD_BF16_WNT); bit 2: K steps go round
   static const int wnt = [] { const char* e = getenv("OAMD_BF16_WNT"); return e && e[0] == '0' ? 0 : 2; }();
-  const int w_tiled = (w_tiled_b ? 1 : 0) | wnt;
+  const int w_tiled = (w_tiled_b ? 1 : 0) | wnt | (M <= 128 && (int64_t)M * K <= kTurnX ? 4 : 0);
   if (w_tiled_b && (N % 64 != 0 || K % 64 != 0)) return -6;
   if ((BM != 64 && BM != 128 && BM != 256) || M % BM != 0) return -1;
   if (glu) {  // fused SwiGLU: one K slice, 128-column tiles of 64 gate + 64 up rows

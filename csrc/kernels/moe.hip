@@ -307,18 +307,18 @@ int moe_gather(const void* h, const int* src, const int* gtab, int bm, int max_r
 
 // Expert GEMM for few rows per expert: the structure of gemm_skinny.hip (W straight to VGPRs as
 // the MFMA A fragment, 4 waves split K, partial tiles summed through LDS) with the expert in
-// blockIdx.y. A workgroup lists the slots routed to its expert, then walks them 16 * MT at a
-// time; an expert nobody chose costs one read of the id list. NT = 2: the SwiGLU pair (16 gate
+// blockIdx.y. A workgroup lists the slots routed to its expert, then walks them 16 at a
+// time (the sorted tiles of gemm.hip are faster from three rows an expert); an expert nobody chose costs one read of the id list. NT = 2: the SwiGLU pair (16 gate
 // rows and the 16 matching up rows of the 64-row interleave).
 constexpr int kMaxSlots = 4096;
 
-template <int NT, int MT>
+template <int NT>
 __global__ void __launch_bounds__(256) moe_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                          bf16_t* __restrict__ Y, const int* __restrict__ ids,
                                                          const float* __restrict__ weights, int slots, int div, int N,
                                                          int K) {
   constexpr int U = 8;
-  __shared__ float red[4][NT * MT][256];
+  __shared__ float red[4][NT][256];
   __shared__ unsigned short list[kMaxSlots];
   __shared__ int count;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -348,66 +348,44 @@ __global__ void __launch_bounds__(256) moe_skinny_kernel(const bf16_t* __restric
     wp[t] = reinterpret_cast<const u16x8*>(W + ((int64_t)ex * N + rows[t] + r) * K + kq * 8);
   const u16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
 
-  for (int c0 = 0; c0 < n; c0 += 16 * MT) {
-    const u16x8* xp[MT];
-    bool xv[MT];
+  for (int c0 = 0; c0 < n; c0 += 16) {
+    const bool xv = c0 + r < n;
+    const u16x8* xp = reinterpret_cast<const u16x8*>(X + (int64_t)(list[xv ? c0 + r : 0] / div) * K + kq * 8);
+    f32x4 acc[NT];
 #pragma unroll
-    for (int j = 0; j < MT; ++j) {
-      const int m = c0 + j * 16 + r;
-      xv[j] = m < n;
-      xp[j] = reinterpret_cast<const u16x8*>(X + (int64_t)(list[xv[j] ? m : 0] / div) * K + kq * 8);
-    }
-    f32x4 acc[NT][MT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int j = 0; j < MT; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     int s = s0;
     for (; s + U <= s1; s += U) {
-      u16x8 a[U][NT], b[U][MT];
+      u16x8 a[U][NT], b[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) a[u][t] = wp[t][(s + u) * 4];
-#pragma unroll
-        for (int j = 0; j < MT; ++j) b[u][j] = xv[j] ? xp[j][(s + u) * 4] : zero;
+        b[u] = xv ? xp[(s + u) * 4] : zero;
       }
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-          for (int j = 0; j < MT; ++j) acc[t][j] = mfma16(a[u][t], b[u][j], acc[t][j]);
+        for (int t = 0; t < NT; ++t) acc[t] = mfma16(a[u][t], b[u], acc[t]);
     }
     for (; s < s1; ++s) {
-      u16x8 a[NT], b[MT];
+      const u16x8 b = xv ? xp[s * 4] : zero;
 #pragma unroll
-      for (int t = 0; t < NT; ++t) a[t] = wp[t][s * 4];
-#pragma unroll
-      for (int j = 0; j < MT; ++j) b[j] = xv[j] ? xp[j][s * 4] : zero;
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int j = 0; j < MT; ++j) acc[t][j] = mfma16(a[t], b[j], acc[t][j]);
+      for (int t = 0; t < NT; ++t) acc[t] = mfma16(wp[t][s * 4], b, acc[t]);
     }
     __syncthreads();   // the previous round's sums are consumed
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int j = 0; j < MT; ++j)
-        *reinterpret_cast<f32x4*>(&red[w][t * MT + j][lane * 4]) = acc[t][j];
+    for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(&red[w][t][lane * 4]) = acc[t];
     __syncthreads();
     // lane l, register i of a tile: W row 4 (l >> 4) + i, X row l & 15; 4 rows per thread
-    for (int x = tid; x < MT * 64; x += 256) {
-      const int j = x >> 6, l = x & 63;
-      const int m = c0 + j * 16 + (l & 15);
-      if (m >= n) continue;
+    const int l = tid, m = c0 + (l & 15);
+    if (l < 64 && m < n) {
       f32x4 v[NT];
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        v[t] = *reinterpret_cast<const f32x4*>(&red[0][t * MT + j][l * 4]);
+        v[t] = *reinterpret_cast<const f32x4*>(&red[0][t][l * 4]);
 #pragma unroll
-        for (int ww = 1; ww < 4; ++ww) v[t] += *reinterpret_cast<const f32x4*>(&red[ww][t * MT + j][l * 4]);
+        for (int ww = 1; ww < 4; ++ww) v[t] += *reinterpret_cast<const f32x4*>(&red[ww][t][l * 4]);
       }
       const int slot = list[m];
       f32x4 o = v[0];
@@ -434,16 +412,8 @@ int moe_gemm_skinny(const bf16_t* X, const bf16_t* W, bf16_t* Y, const int* ids,
   if (slots > kMaxSlots || K % 32 || div < 1) return -1;
   if (silu_gu ? N % 128 : N % 16) return -2;
   const dim3 grid(silu_gu ? N / 32 : N / 16, E);
-  const int mt = slots <= 8 * (int64_t)E ? 1 : slots <= 20 * (int64_t)E ? 2 : 4;   // by the rows an expert gets on average
-  if (silu_gu) {
-    if (mt == 1) moe_skinny_kernel<2, 1><<<grid, 256, 0, stream>>>(X, W, Y, ids, weights, slots, div, N, K);
-    else if (mt == 2) moe_skinny_kernel<2, 2><<<grid, 256, 0, stream>>>(X, W, Y, ids, weights, slots, div, N, K);
-    else moe_skinny_kernel<2, 4><<<grid, 256, 0, stream>>>(X, W, Y, ids, weights, slots, div, N, K);
-  } else {
-    if (mt == 1) moe_skinny_kernel<1, 1><<<grid, 256, 0, stream>>>(X, W, Y, ids, weights, slots, div, N, K);
-    else if (mt == 2) moe_skinny_kernel<1, 2><<<grid, 256, 0, stream>>>(X, W, Y, ids, weights, slots, div, N, K);
-    else moe_skinny_kernel<1, 4><<<grid, 256, 0, stream>>>(X, W, Y, ids, weights, slots, div, N, K);
-  }
+  if (silu_gu) moe_skinny_kernel<2><<<grid, 256, 0, stream>>>(X, W, Y, ids, weights, slots, div, N, K);
+  else moe_skinny_kernel<1><<<grid, 256, 0, stream>>>(X, W, Y, ids, weights, slots, div, N, K);
   OAMD_LAUNCH_CHECK();
   return 0;
 }

@@ -176,8 +176,8 @@ def gate_up_silu(x: torch.Tensor, wgu: torch.Tensor, block: int | None, act: int
             kernels().splitk_silu(slabs, y, S, act)
             return y
         if t != "blas":
-            # one workgroup of 64-row tiles per CU: a fourth stage (64 rows of 28672 x 4096: 52 us on three, 49), two keep theirs in LDS on three
-            ns = t[1] if t and len(t) > 1 else 4 if bm == 64 and M // 64 * (N // 128) <= CUS else 3
+            # one workgroup per CU: a fourth stage (28672 x 4096: 64 rows 41 us on three, 38, 128 rows 53.5 and 51); two keep theirs in LDS on three
+            ns = t[1] if t and len(t) > 1 else 4 if bm <= 128 and M // bm * (N // 128) <= CUS else 3
             y = torch.empty(M, N // 2, dtype=x.dtype, device=x.device)
             kernels().gemm_decode(x, wgu, y, None, 1, 128, bm, act, False, ns)
             return y
@@ -440,11 +440,11 @@ def _decode_plan(M: int, N: int, K: int, defer: bool):
 def _vocab_plan(M: int, N: int, K: int):
     """Decode-bucket vocabulary projection: one row tile of all rows against 128-column tiles, so that the weights
     are read once (256 rows of 32768 x 4096: 73 us, 102 on 64 columns; 128 rows 59 and 62). A 128256-row
-    vocabulary at 256 rows is the tile kernel's (253 us against 289), one of 8192 columns too (64 rows 373 against
-    389, 256 rows 449 against 617); rows that are not one tile would read the weights again. Both lines lie between sizes
-    that were timed: 32000 to 152064 rows of 2048 to 8192 columns, 64 to 256 rows, none of them slower than on 64 columns
+    vocabulary at 256 rows is the tile kernel's (253 us against 289), one of 8192 columns too past 64 rows (128 rows 418 against
+    447, 256 rows 449 against 617; 64 rows 374 against 334); rows that are not one tile would read the weights again. Both lines lie between
+    sizes that were timed: 32000 to 152064 rows of 2048 to 8192 columns, 64 to 256 rows, none of them slower than on 64 columns
     (152064 x 3584: 64 rows 192 us against 223, 256 rows 306 against 430; profiles/plans_before_after.txt)."""
-    if row_tile(M) != M or K >= 8192 or (M == 256 and N >= 2 * LM_HEAD_MIN_N) or N % 128:
+    if row_tile(M) != M or (K >= 8192 and M > 64) or (M == 256 and N >= 2 * LM_HEAD_MIN_N) or N % 128:
         return None
     return (M, 128, 1, 3)
 

@@ -20,8 +20,14 @@ from ._native import kernels
 # general attention work items: 128 query rows whatever the head layout (attn_gd_prefill.hip)
 GD_VARIANT = 5
 GD_BLOCK_Q = 128
-# expert GEMMs (expert_plan): most rows per expert, on average, of each form
-MOE_LIST_ROWS, MOE_64_ROWS, MOE_128_ROWS = 7, 44, 220
+# expert GEMMs (expert_plan): most rows per expert, on average, of each form, timed on 8 to 64 experts of 1024 to 14336 features
+# (us of both products and what sorts the rows). 32 experts of 2048 x 1024: 2 rows 60 on lists, 64 on tiles of 64; 5 rows 85, 74; 80 rows 121 on tiles
+# of 64, 138 on 128. 8 of 4096 x 4096: 2 rows 102, 105; 3 rows 128, 122; 5 rows 165, 135; 80 rows 221, 257, 112 rows 276, 251;
+# 160 rows 301 on 128, 317 on 256, 224 rows 393, 307.
+MOE_LIST_ROWS, MOE_64_ROWS, MOE_128_ROWS = 2.8, 88, 170
+# Larger experts leave the caches between the tiles that share them (8 of 4096 x 14336: 40 rows 580 on 64, 593 on 128; 56 rows 673, 594;
+# 112 rows 861 on 128, 745 on 256)
+MOE_LARGE, MOE_LARGE_64_ROWS, MOE_LARGE_128_ROWS = 1 << 25, 44, 100
 MOE_LIST_MAX_SLOTS = 4096   # moe.hip kMaxSlots
 
 
@@ -430,14 +436,15 @@ def expert_rows_bound(slots: int, experts: int, bm: int) -> int:
     return pad_to(slots + min(experts, slots) * (bm - 1), bm)
 
 
-def expert_plan(slots: int, E: int) -> int:
+def expert_plan(slots: int, E: int, weights: int = 0) -> int:
     """How bf16 expert GEMMs run, by the rows an expert gets on average: 0 = weights streamed
     against the rows of each expert's own list, no sorting (few rows), 64 / 128 = sorted rows in
-    tiles of that many on the decode GEMM, 256 = the prefill tile kernel."""
+    tiles of that many on the decode GEMM, 256 = the prefill tile kernel. ``weights``: of an expert's down projection."""
     rows = slots / E
     if rows <= MOE_LIST_ROWS and slots <= MOE_LIST_MAX_SLOTS:
         return 0
-    return 64 if rows <= MOE_64_ROWS else 128 if rows <= MOE_128_ROWS else 256
+    r64, r128 = (MOE_LARGE_64_ROWS, MOE_LARGE_128_ROWS) if weights > MOE_LARGE else (MOE_64_ROWS, MOE_128_ROWS)
+    return 64 if rows <= r64 else 128 if rows <= r128 else 256
 
 
 def experts(h: torch.Tensor, ids: torch.Tensor, wt: torch.Tensor, wgu: torch.Tensor, wd: torch.Tensor,
@@ -453,7 +460,7 @@ def experts(h: torch.Tensor, ids: torch.Tensor, wt: torch.Tensor, wgu: torch.Ten
         return reference.experts(h, ids, wt, wgu, wd), None
     C, dev = kernels(), h.device
     bf16 = h.dtype == torch.bfloat16
-    bm = (expert_plan(slots, E) if plan is None else plan) if bf16 else 64
+    bm = (expert_plan(slots, E, ld * ff) if plan is None else plan) if bf16 else 64
     if bm in (64, 128) and bf16 and ld % 128:
         bm = 256   # the decode GEMM's column tiles
     if bm == 0:

@@ -1,0 +1,46 @@
+"""gemm_decode and the experts' tiles start their K steps by column tile and expert: fewer steps than tiles, one step, uneven slices, tiled
+weights, X on either side of the size that turns, against float64."""
+import pytest
+import torch
+
+from operator_amd import ops
+from operator_amd.ops import decoder, reference
+
+pytestmark = pytest.mark.gpu
+
+
+# fp32 sums of K products of bf16 numbers (exact each), then one rounding to bf16
+def _check(y, x, w, K):
+    want, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    assert ((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + (K + 16) * 2.0 ** -24 * mag).all()
+
+
+@pytest.mark.parametrize("M,N,K,S,bn,bm,stages", [
+    (64, 1152, 64, 1, 128, 64, 3), (64, 1152, 192, 3, 64, 64, 3), (64, 640, 704, 1, 128, 64, 4), (64, 2048, 1344, 5, 64, 64, 6),
+    (128, 1152, 448, 2, 128, 64, 3), (128, 384, 8192, 1, 128, 128, 4), (128, 128, 8256, 1, 128, 128, 3), (256, 512, 320, 1, 64, 256, 3)])
+def test_steps_go_round(M, N, K, S, bn, bm, stages):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x, w = (torch.randn(n, K, generator=g, device="cuda").bfloat16() for n in (M, N))
+    y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    p = torch.full((S, M, N), float("nan"), device="cuda") if S > 1 else None
+    C = ops.kernels()
+    C.gemm_decode(x, w, y, p, S, bn, bm, False, False, stages)
+    _check(y, x, w, K)
+    wt = w.view(N // 64, 64, K // 64, 64).transpose(1, 2).contiguous().view(N, K)
+    C.gemm_decode(x, wt, y.fill_(float("nan")), p, S, bn, bm, False, True, stages)
+    _check(y, x, w, K)
+
+
+@pytest.mark.parametrize("T,E,ld,ff,top,plan", [(9, 7, 128, 128, 2, 64), (70, 3, 256, 192, 1, 64), (40, 16, 384, 64, 4, 128), (17, 8, 2048, 1024, 2, None)])
+def test_experts(T, E, ld, ff, top, plan):
+    g = torch.Generator(device="cuda").manual_seed(T + E)
+    h = torch.randn(T, ld, generator=g, device="cuda").bfloat16()
+    ids = torch.rand(T, E, generator=g, device="cuda").topk(top).indices.int()
+    wt = torch.rand(T, top, generator=g, device="cuda")
+    wgu = (torch.randn(E, 2 * ff, ld, generator=g, device="cuda") * ld ** -0.5).bfloat16()
+    wd = (torch.randn(E, ld, ff, generator=g, device="cuda") * ff ** -0.5).bfloat16()
+    y, pos = decoder.experts(h, ids, wt, wgu, wd, plan)
+    got = y[pos.long()] if pos is not None else y.view(T, top, ld)
+    want = reference.experts(h.cpu().float(), ids.cpu(), wt.cpu(), wgu.cpu().float(), wd.cpu().float()).view(T, top, ld).to("cuda")
+    # gate, up, act(gate) and their product are rounded to bf16 (2^-9 each), the result once more: against the size of a row
+    assert ((got.float() - want).abs() <= 6 * 2.0 ** -9 * want.norm(dim=-1, keepdim=True) + 2.0 ** -8 * want.abs()).all()
