@@ -447,6 +447,42 @@ void gemm_skinny(const at::Tensor& x, const at::Tensor& w, const c10::optional<a
                        (int)blocks, cur_stream()));
 }
 
+void gemm_rows_norm(const at::Tensor& x, int64_t slabs, const c10::optional<at::Tensor>& residual, const c10::optional<at::Tensor>& sum,
+                    const at::Tensor& nw, double eps, const at::Tensor& w, const c10::optional<at::Tensor>& y, const c10::optional<at::Tensor>& p,
+                    int64_t silu_gu, int64_t blocks) {
+  CHECK_DEV(x); CHECK_CONTIG(x); CHECK_BF16(w); CHECK_CONTIG(w); CHECK_BF16(nw); CHECK_CONTIG(nw);
+  TORCH_CHECK(w.dim() == 2 && nw.numel() == w.size(1), "norm weight [K], w [N, K]");
+  const int64_t N = w.size(0), K = w.size(1);
+  const bool f32 = slabs > 0;
+  if (f32) { CHECK_DT(x, at::kFloat); } else { CHECK_BF16(x); }
+  TORCH_CHECK(y.has_value() != p.has_value(), "y or p");
+  const at::Tensor& like = y.has_value() ? *y : *p;
+  TORCH_CHECK(like.dim() == 2, "y or p [M, N]");
+  const int64_t M = like.size(0);
+  TORCH_CHECK(M >= 1 && M <= 4 && K % 128 == 0 && K <= 16384 && N < (1LL << 31) && N * K < (1LL << 40), "gemm_rows_norm: up to 4 rows of K % 128");
+  TORCH_CHECK(like.size(1) == (silu_gu ? N / 2 : N) && (!silu_gu || (y.has_value() && N % 128 == 0)), "gemm shapes");
+  TORCH_CHECK(f32 ? slabs <= 8 && x.numel() >= slabs * M * K : x.numel() == M * K, "rows [M, K]");
+  TORCH_CHECK(residual.has_value() == sum.has_value(), "residual and sum together");
+  oamd::RowsNorm nm{f32 ? x.data_ptr<float>() : nullptr, (int)slabs, nullptr, nullptr, ptr<bf16_t>(nw), (float)eps};
+  if (residual.has_value()) {
+    CHECK_BF16(*residual); CHECK_CONTIG(*residual); CHECK_BF16(*sum); CHECK_CONTIG(*sum);
+    TORCH_CHECK(residual->numel() == M * K && sum->numel() == M * K && residual->data_ptr() != sum->data_ptr(), "residual and sum [M, K], two tensors");
+    nm.res = ptr<bf16_t>(*residual);
+    nm.out = ptr<bf16_t>(*sum);
+  }
+  bf16_t* yp = nullptr;
+  float* pp = nullptr;
+  if (y.has_value()) {
+    CHECK_BF16(*y); CHECK_CONTIG(*y);
+    yp = ptr<bf16_t>(*y);
+  } else {
+    CHECK_DT(*p, at::kFloat); CHECK_CONTIG(*p);
+    pp = p->data_ptr<float>();
+  }
+  const c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+  RC(oamd::gemm_rows(f32 ? nullptr : ptr<bf16_t>(x), ptr<bf16_t>(w), yp, pp, (int)M, (int)N, (int)K, 1, (int)silu_gu, (int)blocks, &nm, cur_stream()));
+}
+
 void quantize_fp8(const at::Tensor& x, at::Tensor& q, at::Tensor& sx) {
   CHECK_DEV(x); CHECK_BF16(x); CHECK_CONTIG(q); CHECK_CONTIG(sx); CHECK_DT(sx, at::kFloat);
   TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1, "x must be [M, K] row-major");
@@ -759,6 +795,9 @@ PYBIND11_MODULE(_C, m) {
   m.def("gemm_pp_sk_grid", &oamd::gemm_pp_sk_grid, pybind11::arg("tiles"), pybind11::arg("steps"));
   m.def("gemm_skinny", &gemm_skinny, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("y"),
         pybind11::arg("p") = pybind11::none(), pybind11::arg("splits") = 1, pybind11::arg("silu_gu") = 0, pybind11::arg("blocks") = 0);
+  m.def("gemm_rows_norm", &gemm_rows_norm, pybind11::arg("x"), pybind11::arg("slabs"), pybind11::arg("residual"), pybind11::arg("sum"),
+        pybind11::arg("nw"), pybind11::arg("eps"), pybind11::arg("w"), pybind11::arg("y"), pybind11::arg("p") = pybind11::none(),
+        pybind11::arg("silu_gu") = 0, pybind11::arg("blocks") = 256);
   m.def("attn_prefill", &attn_prefill, pybind11::arg("q"), pybind11::arg("k"), pybind11::arg("v"),
         pybind11::arg("o"), pybind11::arg("cu_seqlens"), pybind11::arg("work_seq"), pybind11::arg("work_q0"),
         pybind11::arg("scale"), pybind11::arg("block_q") = 64, pybind11::arg("pk") = pybind11::none(),

@@ -194,7 +194,7 @@ int gemm_skinny(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, in
   if (N % 16 != 0) return -4;
   if (S > 1 && P == nullptr) return -5;
   if (blocks > 0) {
-    if (const int rc = gemm_rows(X, W, Y, P, M, N, K, S, glu, blocks, stream)) return rc;
+    if (const int rc = gemm_rows(X, W, Y, P, M, N, K, S, glu, blocks, nullptr, stream)) return rc;
     if (S > 1 && Y != nullptr) {
       if ((int64_t)M * N % 4 != 0) return -6;
       return splitk_reduce(P, Y, (int64_t)M * N, S, stream);

@@ -75,7 +75,16 @@ int splitk_silu(const float* P, bf16_t* Y, int M, int N, int S, int glu, hipStre
 // interleaved gate|up weight, Y [M, N/2]. blocks > 0 (M <= 8): gemm_rows on so many workgroups per slice, S == 1 with Y == nullptr too.
 int gemm_skinny(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, int N, int K, int S, int glu, int blocks,
                 hipStream_t stream);
-int gemm_rows(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, int N, int K, int S, int glu, int blocks,
+// RMSNorm in front of gemm_rows: row = X or the sum of S slabs p, rounded, + res (if any; the sum, rounded, goes to out, which is not res)
+struct RowsNorm {
+  const float* p;
+  int S;
+  const bf16_t* res;
+  bf16_t* out;
+  const bf16_t* w;
+  float eps;
+};
+int gemm_rows(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, int N, int K, int S, int glu, int blocks, const RowsNorm* norm,
               hipStream_t stream);
 
 // FP8 e4m3fn W8A8: Y = (X8 . W8^T) * sx[m] * sw[n]; any M (BM-row tiles), S | 8 split-K.

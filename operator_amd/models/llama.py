@@ -137,6 +137,13 @@ class LlamaModel(DecoderModel):
             return ops.linear_fp8(x, w, sc, defer_reduce=defer)
         return ops.linear(x, w, defer_reduce=defer and self.tp.world == 1, prompt=prompt)
 
+    def _norm(self, fb: ForwardBatch, t, w: torch.Tensor, h: torch.Tensor, quant: bool, into: torch.Tensor | None, glu: bool = False):
+        """(rmsnorm(t + h) for the projection ``into``, t + h): of a few decode rows the projection normalises them itself."""
+        if self.tp.world == 1 and not (fb.is_prefill or quant or into is None) and (
+                x := ops.norm_into(t, w, self.cfg.rms_eps, h, into, glu)) is not None:
+            return x, x.sum
+        return self.tp.all_reduce_rmsnorm(t, w, self.cfg.rms_eps, residual=h, quant=quant), h   # fused under TP
+
     def _shard_layer(self, wq, wk, wv, wo, wg, wu, wd, an, mn, bias=None) -> LayerWeights:
         """One layer's weights, sharded for this TP rank; ``bias`` = (bq, bk, bv) or None."""
         r, D = self.tp.rank, self.cfg.head_dim
@@ -224,7 +231,9 @@ class LlamaModel(DecoderModel):
         h = ops.embedding(fb.input_ids, self.embed)          # residual stream [T, H]
         T = h.shape[0]
         q8 = self.fp8 and h.is_cuda   # block epilogues emit e4m3fn rows for the next fp8 GEMM
-        x = (ops.rmsnorm_fp8 if q8 else ops.rmsnorm)(h, self.layers[0].attn_norm, c.rms_eps)
+        x = None if fb.is_prefill or q8 else ops.norm_into(h, self.layers[0].attn_norm, c.rms_eps, None, self.layers[0].wqkv)
+        if x is None:
+            x = (ops.rmsnorm_fp8 if q8 else ops.rmsnorm)(h, self.layers[0].attn_norm, c.rms_eps)
         lin = functools.partial(self._lin, prompt=True) if fb.is_prefill else self._lin
         ws = None
         if not fb.is_prefill and h.is_cuda:  # split-KV partials, shared by every layer
@@ -254,7 +263,7 @@ class LlamaModel(DecoderModel):
                                          fb.block_tables, fb.context_lens, self.scale, fb.num_splits, workspace=ws,
                                          bias=bias, k_scale=kv.k_scale, v_scale=kv.v_scale, quant=q8)
             a = lin(o if isinstance(o, tuple) else o.view(T, self.hq * c.head_dim), lw.wo, lw.so, defer=True)
-            x = self.tp.all_reduce_rmsnorm(a, lw.mlp_norm, c.rms_eps, residual=h, quant=q8)   # fused under TP
+            x, h = self._norm(fb, a, lw.mlp_norm, h, q8, lw.wgu if self.gu_block == 64 else None, True)
             if lw.sgu is None:
                 m = ops.gate_up_silu(x, lw.wgu, self.gu_block, prompt=fb.is_prefill)
             elif q8:   # SwiGLU (+ the split-K sum) fused into the down GEMM's input quantization
@@ -264,7 +273,8 @@ class LlamaModel(DecoderModel):
             d = lin(m, lw.wd, lw.sd, defer=True)
             last = i + 1 == len(self.layers)
             nw = self.final_norm if last else self.layers[i + 1].attn_norm
-            x = self.tp.all_reduce_rmsnorm(d, nw, c.rms_eps, residual=h, quant=q8 and not last)
+            nxt = self.layers[i + 1].wqkv if not last else self.lm_head if fb.logits_index is None else None
+            x, h = self._norm(fb, d, nw, h, q8 and not last, nxt)
         if fb.logits_index is not None:
             x = x.index_select(0, fb.logits_index)
         return ops.linear(x, self.lm_head)

@@ -51,6 +51,32 @@ class SplitK:
         return self.p[: self.S * M * N].view(self.S, M, N).sum(0).to(torch.bfloat16)
 
 
+class Normed:
+    """rmsnorm(t (+ residual)) that the projection it is for computes itself (``norm_into``); ``sum`` takes t + residual."""
+
+    __slots__ = ("t", "w", "eps", "residual", "blocks", "sum", "shape", "is_cuda")
+
+    def __init__(self, t, w: torch.Tensor, eps: float, residual: torch.Tensor | None, blocks: int):
+        self.t, self.w, self.eps, self.residual, self.blocks = t, w, eps, residual, blocks
+        self.sum = None if residual is None else torch.empty_like(residual)
+        self.shape, self.is_cuda = t.shape, True
+
+    def into(self, wt: torch.Tensor, y: torch.Tensor | None, p: torch.Tensor | None, act: int = 0) -> None:
+        x, S = (self.t.p, self.t.S) if isinstance(self.t, SplitK) else (self.t, 0)
+        kernels().gemm_rows_norm(x, S, self.residual, self.sum, self.w, self.eps, wt, y, p, act, self.blocks)
+
+
+def norm_into(t, w: torch.Tensor, eps: float, residual: torch.Tensor | None, wt: torch.Tensor, glu: bool = False) -> Normed | None:
+    """rmsnorm(t (+ residual)) of a few decode rows for the projection ``wt`` (``glu``: gate_up_silu of 64-row blocks) as a part of that
+    projection's kernel, or None where it is a kernel of its own. The residual stream goes on in the result's ``sum``."""
+    if not (t.is_cuda and t.dtype == torch.bfloat16 and wt.dtype == torch.bfloat16 and wt.is_contiguous() and len(t.shape) == 2
+            and (t.S <= 8 if isinstance(t, SplitK) else t.is_contiguous()) and (residual is None or residual.is_contiguous())):
+        return None
+    (M, K), N = t.shape, wt.shape[0]
+    blocks = _norm_blocks(M, N, K, glu)
+    return None if blocks is None else Normed(t, w, eps, residual, blocks)
+
+
 def rmsnorm(x, w: torch.Tensor, eps: float, residual: torch.Tensor | None = None,
             out: torch.Tensor | None = None) -> torch.Tensor:
     """RMSNorm; if ``residual`` is given it is updated in place to x + residual first.
@@ -145,13 +171,17 @@ def gate_up_silu(x: torch.Tensor, wgu: torch.Tensor, block: int | None, act: int
     other shapes run the GEMM then the silu_mul kernel. ``prompt``: as for ``linear``."""
     M, K = x.shape
     N = wgu.shape[0]
+    if isinstance(x, Normed):
+        y = torch.empty(M, N // 2, dtype=wgu.dtype, device=wgu.device)
+        x.into(wgu, y, None, act)
+        return y
     if x.is_cuda and block == 64 and f32_ok(x, wgu):
         return linear_f32(x, wgu, glu=act, prompt=prompt)
     if (x.is_cuda and block == 64 and x.dtype == torch.bfloat16 and M <= SKINNY_MAX_M and N % 128 == 0
             and K % 128 == 0 and x.is_contiguous() and wgu.is_contiguous()
             and skinny_plan(M, N, K) is not None and _gemm_table_get().get(("silu", M, N, K)) != "blas"):
         y = torch.empty(M, N // 2, dtype=x.dtype, device=x.device)
-        plan = rows_plan(M, N, K, True)
+        plan = _rows_plan(M, N, K, True)
         if plan is None:
             kernels().gemm_skinny(x, wgu, y, None, 1, act)
         else:
@@ -501,6 +531,26 @@ def rows_plan(M: int, N: int, K: int, glu: bool = False) -> tuple[int, int] | No
     return S, B
 
 
+def _rows_plan(M: int, N: int, K: int, glu: bool) -> tuple[int, int] | None:
+    """rows_plan where no measured entry or switch has another kernel."""
+    if M > ROWS_MAX_M or skinny_plan(M, N, K) is None or (_gemm_table_get().get(("silu", M, N, K)) == "blas" if glu else _measured_blas(M, N, K)):
+        return None
+    return rows_plan(M, N, K, glu)
+
+
+def _norm_blocks(M: int, N: int, K: int, glu: bool) -> int | None:
+    """Workgroups of a product of gemm_rows that normalises its rows itself, or None where rmsnorm in front of it is faster. Every workgroup does it
+    again, so many small ones are for a row or two only (us with rmsnorm and without: 28672 x 4096 gated of one row on 1024 41.0 and 38.2, of four 40.5
+    and 40.7), none at all for short rows (16384 x 2048 gated, one row: 2048 workgroups 15.0 and 16.4, 256 14.3; 151936 x 1536 on 1024 71.8 and
+    73.0), one per CU for up to four rows (6144 x 4096: 13.4 and 10.7, four rows 14.1 and 13.1). Eight pieces of rows (a power of
+    two) and 512 columns are what a wave's registers hold."""
+    plan = _rows_plan(M, N, K, glu)
+    if plan is None or plan[0] != 1 or M > 4 or (1 << (M - 1).bit_length()) * -(-K // 2048) > 8:
+        return None
+    B = plan[1] if plan[1] <= 4 * CUS else CUS
+    return None if (B < plan[1] and N * K >= 5e7) or (M > 2 and plan[1] > CUS) or (-(-(N // 2 if glu else N) // B) * (2 if glu else 1) + 8) * (1 << (M - 1).bit_length()) * 64 > 48 << 10 else B
+
+
 def _mid_beats_skinny(M: int, N: int, K: int, defer: bool) -> bool:
     """gemm_skinny streams the weights once per call but pays for every row (a 128256 x 4096 vocabulary: 191 us at
     1 row, 222 at 8, 300 at 32; 4096 x 14336 26, 27 and 38: 2 % of the one-row time per row, 4 where its tiles do not come in
@@ -775,6 +825,11 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, sp
     M, K = x.shape
     N = w.shape[0]
     plan = None
+    if isinstance(x, Normed):
+        deferred = defer_reduce and skinny_plan(M, N, K) > 1
+        y = torch.empty(M, N, dtype=torch.float32 if deferred else w.dtype, device=w.device)
+        x.into(w, *((None, y) if deferred else (y, None)))
+        return SplitK(y, 1, M, N) if deferred else y
     if x.is_cuda and bias is None and out is None and f32_ok(x, w):
         return linear_f32(x, w, prompt=prompt)
     if bias is not None:
