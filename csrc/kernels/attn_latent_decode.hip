@@ -6,7 +6,9 @@
 // to LDS, from which both products read. A tile's rows are loaded by eight threads each, with one page lookup and one address per row:
 // chunks dealt out over the whole tile cost a division, a lookup and an address each, and registers that some sizes spilled.
 // 48 sequences of 3600 rows, combine included: 16 heads on 320 columns 48 -> 39 us, on 384 117 -> 49, 32 heads on 576 75 -> 72
-// (2.8 TB/s: a tile's phases, one after the other behind four barriers, are what bounds it).
+// (2.8 TB/s: a tile's phases, one after the other behind four barriers, are what bounds it; with the value blocks unbranched 69, 16 heads on 320
+// columns 37, on 384 46). Two tiles in LDS, two barriers a tile, gain nothing: a launch of 240 workgroups of twelve tiles starts and ends
+// in 12 us, and a tile takes 3 us with every CU busy (6.2 TB/s).
 //
 //   S = K Q^T     v_mfma_f32_16x16x32_bf16, A = rows (tokens x dims), B = q (one head per column);
 //                 wave w of a head group takes tokens 16 w .. 16 w + 15
@@ -75,8 +77,7 @@ __global__ void __launch_bounds__(256 * HG, HG == 1 && NK < 12 ? 2 : 1) attn_lat
   u16x8 qf[NK];
 #pragma unroll
   for (int st = 0; st < NK; ++st)
-    qf[st] = h < a.G ? *reinterpret_cast<const u16x8*>(a.q + ((int64_t)b * a.G + h) * CK + 32 * st + 8 * lg)
-                     : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    qf[st] = *reinterpret_cast<const u16x8*>(a.q + ((int64_t)b * a.G + min(h, a.G - 1)) * CK + 32 * st + 8 * lg);   // past the heads: never stored
   __syncthreads();
 
   // a thread's rows of a tile are row0 and, of 16 heads, row0 + 32, its 16-B chunks of a row ch0 + 8 j: one page lookup and one
@@ -158,14 +159,13 @@ __global__ void __launch_bounds__(256 * HG, HG == 1 && NK < 12 ? 2 : 1) attn_lat
     for (int st = 0; st < 2; ++st) {   // 32 tokens: two 16-token blocks, 4 tokens of each per lane
       const s16x8 pb = __builtin_shufflevector(ps[hg][2 * st][lane], ps[hg][2 * st + 1][lane], 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
-      for (int m = 0; m < NB; ++m)
-        if (4 * m + w < nb) {
-          const char* v = vrow + RK * 32 * st + 128 * m;
-          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(v));
-          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(v + RK * 16));
-          const s16x8 va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-          acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, va), __builtin_bit_cast(bf16x8, pb), acc[m], 0, 0, 0);
-        }
+      for (int m = 0; m < NB; ++m) {   // the columns past rp too (never stored): behind a branch every block would wait for its own reads
+        const char* v = vrow + RK * 32 * st + 128 * m;
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(v));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(v + RK * 16));
+        const s16x8 va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, va), __builtin_bit_cast(bf16x8, pb), acc[m], 0, 0, 0);
+      }
     }
   };
   load(even, 0);
