@@ -28,6 +28,8 @@ MOE_LIST_ROWS, MOE_64_ROWS, MOE_128_ROWS = 2.8, 88, 170
 # Larger experts leave the caches between the tiles that share them (8 of 4096 x 14336: 40 rows 580 on 64, 593 on 128; 56 rows 673, 594;
 # 112 rows 861 on 128, 745 on 256)
 MOE_LARGE, MOE_LARGE_64_ROWS, MOE_LARGE_128_ROWS = 1 << 25, 44, 100
+# Widths that are no multiple of 128 have lists and the prefill tiles only (32 of 2880 x 2880: 3.5 rows 265 and 391)
+MOE_LIST_ROWS_ODD = 7
 MOE_LIST_MAX_SLOTS = 4096   # moe.hip kMaxSlots
 
 
@@ -436,15 +438,16 @@ def expert_rows_bound(slots: int, experts: int, bm: int) -> int:
     return pad_to(slots + min(experts, slots) * (bm - 1), bm)
 
 
-def expert_plan(slots: int, E: int, weights: int = 0) -> int:
+def expert_plan(slots: int, E: int, weights: int = 0, tiles: bool = True) -> int:
     """How bf16 expert GEMMs run, by the rows an expert gets on average: 0 = weights streamed
     against the rows of each expert's own list, no sorting (few rows), 64 / 128 = sorted rows in
-    tiles of that many on the decode GEMM, 256 = the prefill tile kernel. ``weights``: of an expert's down projection."""
+    tiles of that many on the decode GEMM, 256 = the prefill tile kernel. ``weights``: of an expert's down projection;
+    ``tiles``: its width takes the decode GEMM's column tiles."""
     rows = slots / E
-    if rows <= MOE_LIST_ROWS and slots <= MOE_LIST_MAX_SLOTS:
+    if rows <= (MOE_LIST_ROWS if tiles else MOE_LIST_ROWS_ODD) and slots <= MOE_LIST_MAX_SLOTS:
         return 0
     r64, r128 = (MOE_LARGE_64_ROWS, MOE_LARGE_128_ROWS) if weights > MOE_LARGE else (MOE_64_ROWS, MOE_128_ROWS)
-    return 64 if rows <= r64 else 128 if rows <= r128 else 256
+    return 256 if not tiles else 64 if rows <= r64 else 128 if rows <= r128 else 256
 
 
 def experts(h: torch.Tensor, ids: torch.Tensor, wt: torch.Tensor, wgu: torch.Tensor, wd: torch.Tensor,
@@ -460,7 +463,7 @@ def experts(h: torch.Tensor, ids: torch.Tensor, wt: torch.Tensor, wgu: torch.Ten
         return reference.experts(h, ids, wt, wgu, wd), None
     C, dev = kernels(), h.device
     bf16 = h.dtype == torch.bfloat16
-    bm = (expert_plan(slots, E, ld * ff) if plan is None else plan) if bf16 else 64
+    bm = (expert_plan(slots, E, ld * ff, ld % 128 == 0) if plan is None else plan) if bf16 else 64
     if bm in (64, 128) and bf16 and ld % 128:
         bm = 256   # the decode GEMM's column tiles
     if bm == 0:
