@@ -23,8 +23,8 @@
 //   * column tile n starts its slice at K step n % steps and goes round. Tiles in step would all read the same 128 columns of rows that lie a
 //     power of two apart, which HBM serves from some of its channels: 64 rows of 128256 x 4096 213 -> 175 us (4.9 -> 6.0 TB/s), 28672 x 4096
 //     gated 46 -> 38, 57344 x 8192 gated 175 -> 148, 32000 x 4096 59 -> 42, 8192 x 8192 32 -> 28; 128 rows of 32000 x 4096 59 -> 53. Where rows
-//     are no such distance apart (3584 columns) it changes nothing. Experts' tiles start 5 steps further an expert: 96 tokens on 8 experts of
-//     4096 x 4096 172 -> 134 us, on 64 of 2048 x 1024 178 -> 150.
+//     are no such distance apart (3584 columns) it changes nothing. Experts' tiles of 64 rows start 5 steps further an expert: 96 tokens on
+//     8 experts of 4096 x 4096 172 -> 134 us, on 64 of 2048 x 1024 178 -> 150; of 128 rows, whose X weighs more, they keep step (112 rows each 242, 258 round).
 // MFMA v_mfma_f32_16x16x32_bf16; fragment maps as in attn_decode.hip.
 #include "common.h"
 #include "kernels.h"
@@ -44,6 +44,9 @@ constexpr int kWaves = 8;
 // Most elements of X whose K steps go round. Tiles in step share a piece of X while it is in their XCD's L2, tiles that are not need all of
 // X there (4 MiB): 128 rows of 8192 x 28672 88 us in step, 96 round, of 3584 x 18944 30 and 41. 256-row tiles are not bound by HBM (32768 x 2048 40 and 43).
 constexpr int64_t kTurnX = 1 << 20;
+// Fewest weights whose K steps go round: the addresses cost a little (64 rows of 4096 x 4096 8.9 us in step, 9.8 round; 14336 x 2048 16.0 and 17.2; 4096 x 11008
+// 19.5 and 18.1, 12288 x 4096 24.7 and 20.6), as they do in 128 x 64 tiles (28672 x 4096 65 and 70).
+constexpr int64_t kTurnW = 1 << 25;
 
 // BN = 128 halves the LDS fragment traffic per MFMA (64 x 64 wave tiles at
 // M = 256: 0.5 KB of ds_read per MFMA vs 0.75 KB at BN = 64, where the LDS
@@ -77,7 +80,8 @@ enum { kEpiStore = 0, kEpiPartial = 1, kEpiSiluGU = 2 };
 // GRP: routed experts. Row tile y holds rows of one expert (moe_sort with bm = BM): gtab[0] = row
 // tiles, gtab[1 + y] = its expert, W [experts][N][K]; src != nullptr: row r reads X row src[r]
 // (< 0: padding, any row), and rscale[r] multiplies both SwiGLU operands.
-template <int BM, int BN, int EPI, int NS = kStages, bool GRP = false>
+// TURN: K steps go round by column tile (and expert)
+template <int BM, int BN, int EPI, int NS = kStages, bool GRP = false, bool TURN = false>
 __global__ void __launch_bounds__(kWaves * 64, NS == 2 ? 2 : 1) gemm_tn_kernel(const bf16_t* __restrict__ X,
                                                                  const bf16_t* __restrict__ W, bf16_t* __restrict__ Y,
                                                                  float* __restrict__ P, int M, int N, int K, int S,
@@ -118,9 +122,9 @@ __global__ void __launch_bounds__(kWaves * 64, NS == 2 ? 2 : 1) gemm_tn_kernel(c
       if (src != nullptr && xrow[i] < BM) xrow[i] = max(src[m0 + xrow[i]], 0);
     }
   }
-  const int off = w_tiled & 4 ? turn % T : 0;
+  const int off = TURN ? turn % T : 0;
   auto issue_one = [&](int t, int buf, int i) {
-    const int k0 = kbase + (t + off < T ? t + off : t + off - T) * kBK;
+    const int k0 = kbase + (!TURN ? t : t + off < T ? t + off : t + off - T) * kBK;
     char* sbase = lds + buf * C::STAGE_BYTES;
     {
       const int q = w + kWaves * i;
@@ -288,39 +292,45 @@ int moe_gemm_rows(const bf16_t* X, const bf16_t* W, bf16_t* Y, int max_rows, int
   if (silu_gu && rscale == nullptr) return -2;
   const dim3 grid(N / 128, max_rows / bm);
   if (bm == 64 && silu_gu)
-    gemm_tn_kernel<64, 128, kEpiSiluGU, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2 | 4, gtab, src, rscale);
+    gemm_tn_kernel<64, 128, kEpiSiluGU, 3, true, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2, gtab, src, rscale);
   else if (bm == 64)
-    gemm_tn_kernel<64, 128, kEpiStore, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2 | 4, gtab, src, rscale);
+    gemm_tn_kernel<64, 128, kEpiStore, 3, true, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2, gtab, src, rscale);
   else if (silu_gu)
-    gemm_tn_kernel<128, 128, kEpiSiluGU, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2 | 4, gtab, src, rscale);
+    gemm_tn_kernel<128, 128, kEpiSiluGU, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2, gtab, src, rscale);
   else
-    gemm_tn_kernel<128, 128, kEpiStore, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2 | 4, gtab, src, rscale);
+    gemm_tn_kernel<128, 128, kEpiStore, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2, gtab, src, rscale);
   OAMD_LAUNCH_CHECK();
   return 0;
 }
 
 int gemm_decode(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, int N, int K, int S, int BN,
                 int BM, int glu, bool w_tiled_b, int stages, hipStream_t stream) {
-  // bit 0: tiled W layout; bit 1: W streams with the non-temporal policy (OAMD_BF16_WNT); bit 2: K steps go round
+  // bit 0: tiled W layout; bit 1: W streams with the non-temporal policy (OAMD_BF16_WNT)
   static const int wnt = [] { const char* e = getenv("OAMD_BF16_WNT"); return e && e[0] == '0' ? 0 : 2; }();
-  const int w_tiled = (w_tiled_b ? 1 : 0) | wnt | (M <= 128 && (int64_t)M * K <= kTurnX ? 4 : 0);
+  const int w_tiled = (w_tiled_b ? 1 : 0) | wnt;
+  const bool turn = M <= 128 && (int64_t)M * K <= kTurnX && (int64_t)N * K >= kTurnW;
   if (w_tiled_b && (N % 64 != 0 || K % 64 != 0)) return -6;
   if ((BM != 64 && BM != 128 && BM != 256) || M % BM != 0) return -1;
   if (glu) {  // fused SwiGLU: one K slice, 128-column tiles of 64 gate + 64 up rows
     if (BN != 128 || S != 1 || N % 128 != 0 || K % kBK != 0) return -5;
     const dim3 grid(N / 128, M / BM);
-    switch (BM) {
-      case 64:
-        if (stages == 2) gemm_tn_kernel<64, 128, kEpiSiluGU, 2><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, 1, w_tiled, nullptr, nullptr, nullptr, glu_act(glu));
-        else if (stages == 4) gemm_tn_kernel<64, 128, kEpiSiluGU, 4><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, 1, w_tiled, nullptr, nullptr, nullptr, glu_act(glu));
-        else gemm_tn_kernel<64, 128, kEpiSiluGU><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, 1, w_tiled, nullptr, nullptr, nullptr, glu_act(glu));
-        break;
-      case 128:
-        if (stages == 4) gemm_tn_kernel<128, 128, kEpiSiluGU, 4><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, 1, w_tiled, nullptr, nullptr, nullptr, glu_act(glu));
-        else gemm_tn_kernel<128, 128, kEpiSiluGU><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, 1, w_tiled, nullptr, nullptr, nullptr, glu_act(glu));
-        break;
-      default: gemm_tn_kernel<256, 128, kEpiSiluGU><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, 1, w_tiled, nullptr, nullptr, nullptr, glu_act(glu)); break;
+#define OAMD_GLU(BM, NSS, TURN) \
+  gemm_tn_kernel<BM, 128, kEpiSiluGU, NSS, false, TURN><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, 1, w_tiled, nullptr, nullptr, nullptr, glu_act(glu))
+    if (BM == 64) {
+      if (stages == 2) OAMD_GLU(64, 2, false);
+      else if (stages == 4 && turn) OAMD_GLU(64, 4, true);
+      else if (stages == 4) OAMD_GLU(64, 4, false);
+      else if (turn) OAMD_GLU(64, 3, true);
+      else OAMD_GLU(64, 3, false);
+    } else if (BM == 128) {
+      if (stages == 4 && turn) OAMD_GLU(128, 4, true);
+      else if (stages == 4) OAMD_GLU(128, 4, false);
+      else if (turn) OAMD_GLU(128, 3, true);
+      else OAMD_GLU(128, 3, false);
+    } else {
+      OAMD_GLU(256, 3, false);
     }
+#undef OAMD_GLU
     OAMD_LAUNCH_CHECK();
     return 0;
   }
@@ -328,10 +338,15 @@ int gemm_decode(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, in
   if (S < 1 || S > 16 || K % kBK != 0 || K / kBK < S) return -3;
   if (S > 1 && P == nullptr) return -4;
   const dim3 grid((N / BN) * S, M / BM);
-#define OAMD_GEMM3(BM, BNN, NSS)                                                                               \
-  if (S > 1) gemm_tn_kernel<BM, BNN, kEpiPartial, NSS><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, S,   \
-                                                                                       w_tiled);              \
-  else gemm_tn_kernel<BM, BNN, kEpiStore, NSS><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, S, w_tiled)
+#define OAMD_GEMM4(BM, BNN, NSS, TURN)                                                                                                        \
+  if (S > 1) gemm_tn_kernel<BM, BNN, kEpiPartial, NSS, false, TURN><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, S, w_tiled);         \
+  else gemm_tn_kernel<BM, BNN, kEpiStore, NSS, false, TURN><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, S, w_tiled)
+#define OAMD_GEMM3(BM, BNN, NSS)                                                    \
+  if constexpr (BM == 64 || (BM == 128 && BNN == 128)) {                            \
+    if (turn) { OAMD_GEMM4(BM, BNN, NSS, true); } else { OAMD_GEMM4(BM, BNN, NSS, false); } \
+  } else {                                                                          \
+    OAMD_GEMM4(BM, BNN, NSS, false);                                                \
+  }
 #define OAMD_GEMM2(BM, BNN)                                   \
   if (stages == 2 && BM <= 128) {                              \
     OAMD_GEMM3(BM, BNN, 2);                                    \
@@ -354,6 +369,7 @@ int gemm_decode(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, in
 #undef OAMD_GEMM
 #undef OAMD_GEMM2
 #undef OAMD_GEMM3
+#undef OAMD_GEMM4
   OAMD_LAUNCH_CHECK();
   if (S > 1 && Y != nullptr) {  // Y == nullptr: the consumer sums the slabs (rmsnorm)
     const int64_t MN = (int64_t)M * N;

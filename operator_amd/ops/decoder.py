@@ -20,14 +20,13 @@ from ._native import kernels
 # general attention work items: 128 query rows whatever the head layout (attn_gd_prefill.hip)
 GD_VARIANT = 5
 GD_BLOCK_Q = 128
-# expert GEMMs (expert_plan): most rows per expert, on average, of each form, timed on 8 to 64 experts of 1024 to 14336 features
-# (us of both products and what sorts the rows). 32 experts of 2048 x 1024: 2 rows 60 on lists, 64 on tiles of 64; 5 rows 85, 74; 80 rows 121 on tiles
-# of 64, 138 on 128. 8 of 4096 x 4096: 2 rows 102, 105; 3 rows 128, 122; 5 rows 165, 135; 80 rows 221, 257, 112 rows 276, 251;
-# 160 rows 301 on 128, 317 on 256, 224 rows 393, 307.
-MOE_LIST_ROWS, MOE_64_ROWS, MOE_128_ROWS = 2.8, 88, 170
-# Larger experts leave the caches between the tiles that share them (8 of 4096 x 14336: 40 rows 580 on 64, 593 on 128; 56 rows 673, 594;
-# 112 rows 861 on 128, 745 on 256)
-MOE_LARGE, MOE_LARGE_64_ROWS, MOE_LARGE_128_ROWS = 1 << 25, 44, 100
+# expert GEMMs (expert_plan): most rows per expert, on average, of each form, timed on 8 to 64 experts of 1024 to 14336 features, evenly routed and
+# not (us of both products and what sorts the rows). 32 experts of 2048 x 1024: 2 rows 69 on lists and on tiles of 64; 5 rows 82, 77; 56 rows 102 on
+# tiles of 64, 107 on 128, 65 rows 114, 109. 8 of 4096 x 4096: 2 rows 102, 105; 3 rows 128, 122; 5 rows 151, 135; 56 rows 184, 191, 70 rows 208, 190. Of uneven
+# routes tiles of 64 stay faster up to 90 rows (70 rows 220, 253), which the rows alone do not tell
+MOE_LIST_ROWS, MOE_64_ROWS, MOE_128_ROWS = 2.8, 56, 220
+# Larger experts leave the caches between the tiles that share them (8 of 4096 x 14336: 40 rows 580 on 64, 593 on 128; 56 rows 673, 594)
+MOE_LARGE, MOE_LARGE_64_ROWS = 1 << 25, 44
 # Widths that are no multiple of 128 have lists and the prefill tiles only (32 of 2880 x 2880: 3.5 rows 265 and 391)
 MOE_LIST_ROWS_ODD = 7
 MOE_LIST_MAX_SLOTS = 4096   # moe.hip kMaxSlots
@@ -446,8 +445,9 @@ def expert_plan(slots: int, E: int, weights: int = 0, tiles: bool = True) -> int
     rows = slots / E
     if rows <= (MOE_LIST_ROWS if tiles else MOE_LIST_ROWS_ODD) and slots <= MOE_LIST_MAX_SLOTS:
         return 0
-    r64, r128 = (MOE_LARGE_64_ROWS, MOE_LARGE_128_ROWS) if weights > MOE_LARGE else (MOE_64_ROWS, MOE_128_ROWS)
-    return 256 if not tiles else 64 if rows <= r64 else 128 if rows <= r128 else 256
+    if not tiles or rows > MOE_128_ROWS:
+        return 256
+    return 64 if rows <= (MOE_LARGE_64_ROWS if weights > MOE_LARGE else MOE_64_ROWS) else 128
 
 
 def experts(h: torch.Tensor, ids: torch.Tensor, wt: torch.Tensor, wgu: torch.Tensor, wd: torch.Tensor,

@@ -1,5 +1,5 @@
 """gemm_decode and the experts' tiles start their K steps by column tile and expert: fewer steps than tiles, one step, uneven slices, tiled
-weights, X on either side of the size that turns, against float64."""
+weights, against float64."""
 import pytest
 import torch
 
@@ -15,9 +15,11 @@ def _check(y, x, w, K):
     assert ((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + (K + 16) * 2.0 ** -24 * mag).all()
 
 
+# on either side of the weights (2^25 elements) and the X (2^20) that turn, 128-row tiles over 64 columns, which never do
 @pytest.mark.parametrize("M,N,K,S,bn,bm,stages", [
-    (64, 1152, 64, 1, 128, 64, 3), (64, 1152, 192, 3, 64, 64, 3), (64, 640, 704, 1, 128, 64, 4), (64, 2048, 1344, 5, 64, 64, 6),
-    (128, 1152, 448, 2, 128, 64, 3), (128, 384, 8192, 1, 128, 128, 4), (128, 128, 8256, 1, 128, 128, 3), (256, 512, 320, 1, 64, 256, 3)])
+    (64, 1152, 192, 3, 64, 64, 3), (64, 524288, 64, 1, 128, 64, 3), (64, 175360, 192, 3, 64, 64, 3), (64, 32768, 1024, 1, 128, 64, 4),
+    (64, 25024, 1344, 5, 64, 64, 6), (128, 75008, 448, 2, 128, 64, 2), (128, 4096, 8192, 1, 128, 128, 4), (128, 4096, 8256, 3, 128, 128, 3),
+    (128, 32768, 1024, 1, 64, 128, 4), (256, 32768, 1024, 1, 128, 256, 3)])
 def test_steps_go_round(M, N, K, S, bn, bm, stages):
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     x, w = (torch.randn(n, K, generator=g, device="cuda").bfloat16() for n in (M, N))
@@ -42,5 +44,20 @@ def test_experts(T, E, ld, ff, top, plan):
     y, pos = decoder.experts(h, ids, wt, wgu, wd, plan)
     got = y[pos.long()] if pos is not None else y.view(T, top, ld)
     want = reference.experts(h.cpu().float(), ids.cpu(), wt.cpu(), wgu.cpu().float(), wd.cpu().float()).view(T, top, ld).to("cuda")
-    # gate, up, act(gate) and their product are rounded to bf16 (2^-9 each), the result once more: against the size of a row
+    # the gated product is rounded to bf16 (2^-8 of each, a random sum over ff: against the size of a row), the result once more
     assert ((got.float() - want).abs() <= 6 * 2.0 ** -9 * want.norm(dim=-1, keepdim=True) + 2.0 ** -8 * want.abs()).all()
+
+
+@pytest.mark.parametrize("M,N,K,ns", [(64, 32768, 1024, 4), (64, 33024, 1088, 3), (128, 32768, 1088, 4), (128, 32768, 1088, 3), (128, 1024, 1088, 4)])
+def test_gated(M, N, K, ns):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).bfloat16()
+    y = torch.full((M, N // 2), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ops.kernels().gemm_decode(x, w, y, None, 1, 128, M, 1, False, ns)
+    r = (x.double() @ w.double().t()).view(M, N // 128, 2, 64)
+    gate, up = r[:, :, 0].reshape(M, -1), r[:, :, 1].reshape(M, -1)
+    sg = torch.nn.functional.silu(gate)
+    # gate, silu(gate), up and the product are rounded to bf16: 2^-8 of each (silu's slope is at most 1.1); second order and the fp32 sums
+    tol = 1.02 * 2.0 ** -8 * up.abs() * (1.1 * gate.abs() + 3 * sg.abs()) + 1e-4 * (1 + up.abs() + gate.abs())
+    assert ((y.double() - sg * up).abs() <= tol).all()
