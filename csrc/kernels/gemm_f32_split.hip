@@ -19,6 +19,7 @@
 #include <utility>
 
 #include "common.h"
+#include "f32_piece.h"
 #include "gemm_f32.h"
 #include "kernels.h"
 
@@ -77,11 +78,11 @@ __global__ void __launch_bounds__(128 * WM, 2) gemm_f32_split_kernel(const GemmF
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
     const int row = lr + kPass * i;
-    src[i] = (row < kX ? a.X + min(m0 + row, a.M - 1) * a.ldx : a.W + (int64_t)min(n0 + row - kX, a.N - 1) * K) + 8 * lc;
+    src[i] = row < kX ? a.X + min(m0 + row, a.M - 1) * a.ldx : a.W + (int64_t)min(n0 + row - kX, a.N - 1) * K;
   }
   struct Piece { f32x4 v[2 * NR]; } even, odds;
-  auto load = [&](Piece& p, int i, int k) {   // past the row's end its first columns, which are cleared or never used
-    const float* from = src[i] + (k + 8 * lc < K ? k : 0);
+  auto load = [&](Piece& p, int i, int k) {
+    const float* from = src[i] + split_column(k, lc, K);
     p.v[2 * i] = *reinterpret_cast<const f32x4*>(from);
     p.v[2 * i + 1] = *reinterpret_cast<const f32x4*>(from + 4);
   };

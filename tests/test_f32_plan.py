@@ -1,4 +1,7 @@
 """Which fp32 kernel and slices a product takes (ops.f32_split_slices), without a GPU."""
+import os
+import subprocess
+
 import pytest
 
 from operator_amd import ops
@@ -20,3 +23,28 @@ def test_lines():
     assert ops.f32_split_rows(962, 16384, 2048, 1, ops.GELU_TANH) == 256
     assert ops.f32_split_slices(512, 2048, 288, 0) is None       # 9 us against 14
     assert ops.f32_split_slices(512, 2048, 8192, 0) is not None  # 161 against 99
+
+
+def test_the_split_kernels_loads_stay_in_their_rows(tmp_path):
+    """Every piece that the kernel requests, two behind the last of a row and of a slice among them, for all K up to 200 and slices up to 8."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    src, exe = tmp_path / "columns.cpp", tmp_path / "columns"
+    src.write_text("""
+#include <cstdio>
+#include "kernels/f32_piece.h"
+int main() {
+  for (int K = 16; K <= 200; K += 16)
+    for (int S = 1; S <= 8; ++S)
+      for (int z = 0; z < S; ++z) {
+        const int T = (K + 31) / 32, from = z * T / S * 32, to = (z + 1) * T / S * 32;
+        for (int k = from; k <= to + 128; k += 32)
+          for (int lc = 0; lc < 4; ++lc) {
+            const int at = oamd::split_column(k, lc, K);
+            if (at < 0 || at + 8 > K || (k + 8 * lc < K && at != k + 8 * lc)) return std::printf("K %d k %d lc %d: %d\\n", K, k, lc, at), 1;
+          }
+      }
+}
+""")
+    subprocess.run(["g++", "-std=c++17", "-I", os.path.join(root, "csrc"), str(src), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
