@@ -170,18 +170,20 @@ __global__ void __launch_bounds__(128 * WM, 2) gemm_f32_split_kernel(const GemmF
   if (k < kend) step(odds, 0, k);
 
   // A sum that is no ordinary number is done again in 32-bit products: infinities and NaN among the operands (or a value that
-  // rounds to infinity), and sums so small that the parts of their operands may have fallen below bf16's range.
-  bool odd = false;
+  // rounds to infinity), and sums so small that the parts of their operands may have fallen below bf16's range. That sum alone: the wave does its
+  // block again, but the other sums stay as they are, whoever shares the block.
+  auto odd = [](float sum) {
+    const float v = fabsf(sum);
+    return !(v <= 3.4028234e38f) || (v < 0x1p-64f && v != 0.f);
+  };
+  bool any = false;
 #pragma unroll
   for (int b = 0; b < 2; ++b)
 #pragma unroll
     for (int i = 0; i < TB; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float v = fabsf(acc[b][i][r]);
-        odd |= !(v <= 3.4028234e38f) || (v < 0x1p-64f && v != 0.f);
-      }
-  if (__any(odd)) {
+      for (int r = 0; r < 16; ++r) any |= odd(acc[b][i][r]);
+  if (__any(any)) {
 #pragma unroll
     for (int i = 0; i < TB; ++i) {
       const float* x = a.X + min(m0 + (wm * TB + i) * 32 + l31, a.M - 1) * a.ldx + 4 * half;
@@ -195,8 +197,11 @@ __global__ void __launch_bounds__(128 * WM, 2) gemm_f32_split_kernel(const GemmF
           u = __builtin_amdgcn_mfma_f32_32x32x2f32(uv[e], xv[e], u, 0, 0, 0);
         }
       }
-      acc[0][i] = g;
-      acc[1][i] = u;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        acc[0][i][r] = odd(acc[0][i][r]) ? g[r] : acc[0][i][r];
+        acc[1][i][r] = odd(acc[1][i][r]) ? u[r] : acc[1][i][r];
+      }
     }
   }
 

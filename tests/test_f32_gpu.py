@@ -239,3 +239,33 @@ def test_gemm_f32_split_keeps_odd_values_and_small_ones(rows, S):
     assert torch.equal(y[r.isinf()], r32[r.isinf()])
     fin = r.isfinite() & r32.isfinite()
     assert ((y[fin].double() - r[fin]).abs() <= (K + 8) * 2.0 ** -24 * mag[fin] + 1e-44).all()
+
+
+def _split(x, w, rows, S=1, glu=0):
+    M, N = x.shape[0], w.shape[0]
+    y = torch.full((M, N // 2 if glu else N), float("nan"), device=DEV)
+    part = torch.full((S * M * N,), float("nan"), device=DEV) if S > 1 else None
+    ops.kernels().gemm_f32(x, w, y, glu, partial=part, splits=S, rows=rows)
+    return y
+
+
+@pytest.mark.parametrize("S", [1, 3])
+@pytest.mark.parametrize("glu", [0, ops.SILU])
+def test_gemm_f32_split_odd_values_leave_other_rows_as_they_are(S, glu):
+    """What is done again in 32-bit products is the odd sum alone: other rows and columns keep their bits, and so do all between tile rows."""
+    torch.manual_seed(S)
+    M, N, K = 300, 256, 112
+    x, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV)
+    before = [_split(x, w, rows, S, glu) for rows in (64, 128, 256)]
+    x[3, 5], x[77, 0], w[131, 7] = float("inf"), float("nan"), float("-inf")
+    x[150] *= 1e-36
+    w[40] *= 1e-30
+    after = [_split(x, w, rows, S, glu) for rows in (64, 128, 256)]
+    r, c = torch.ones(M, dtype=torch.bool, device=DEV), torch.ones(N, dtype=torch.bool, device=DEV)
+    r[[3, 77, 150]] = False
+    c[[131, 40]] = False
+    if glu:   # a feature's gate and up
+        c = c.view(-1, 2, 64).all(1).flatten()
+    for y, z in zip(before, after):
+        assert torch.equal(y[r][:, c], z[r][:, c])
+        assert ((z == after[0]) | (z.isnan() & after[0].isnan())).all()
