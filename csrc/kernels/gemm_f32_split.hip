@@ -60,6 +60,7 @@ template <int WM, int TB, bool GLU, bool PART>
 __global__ void __launch_bounds__(128 * WM, 2) gemm_f32_split_kernel(const GemmF32 a) {
   constexpr int kX = 32 * WM * TB, kPass = 32 * WM, kRows = kX + 128, kPlane = kRows * 64, kBuf = 3 * kPlane, NR = kRows / kPass;
   __shared__ __attribute__((aligned(1024))) char lds[2 * kBuf];
+  __shared__ uint32_t kind[kRows / 4];   // a byte per row of X and W: 1 it holds an operand of 2^32 or more, 2 one other than 0
   const int K = a.K;
   const int lid = xcd_remap(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
   const int m0 = lid % gridDim.x * kX, n0 = lid / gridDim.x * 128;
@@ -80,7 +81,7 @@ __global__ void __launch_bounds__(128 * WM, 2) gemm_f32_split_kernel(const GemmF
     const int row = lr + kPass * i;
     src[i] = row < kX ? a.X + min(m0 + row, a.M - 1) * a.ldx : a.W + (int64_t)min(n0 + row - kX, a.N - 1) * K;
   }
-  struct Piece { f32x4 v[2 * NR]; } even, odds;
+  struct Piece { f32x4 v[2 * NR]; } even, uneven;
   auto load = [&](Piece& p, int i, int k) {
     const float* from = src[i] + split_column(k, lc, K);
     p.v[2 * i] = *reinterpret_cast<const f32x4*>(from);
@@ -94,8 +95,8 @@ __global__ void __launch_bounds__(128 * WM, 2) gemm_f32_split_kernel(const GemmF
   f32x16 acc[2][TB] = {};   // [W rows 32 wn and 64 + 32 wn][token block]
   constexpr int NF = 3 * (TB + 2);   // fragments of a 16-column half
   bf16x8 xf[2][3][TB], wf[2][3][2];
-  // partial product p: part kw[p] of W by part kx[p] of X, the small ones first; fragments in the order in which they are used
-  constexpr int kw[6] = {0, 2, 1, 0, 1, 0}, kx[6] = {2, 0, 1, 1, 0, 0}, order[3] = {0, 2, 1};
+  // partial product p: part pw[p] of W by part px[p] of X, the small ones first; fragments in the order in which they are used
+  constexpr int pw[6] = {0, 2, 1, 0, 1, 0}, px[6] = {2, 0, 1, 1, 0, 0}, order[3] = {0, 2, 1};
   auto rd = [&](int buf, int h, int i) {
     const int at = buf * kBuf + (((2 * h + half) ^ sw) << 4), s = i / (TB + 2), j = i % (TB + 2);
     if (j < 2) wf[h][order[s]][j] = *reinterpret_cast<const bf16x8*>(wr + order[s] * kPlane + j * 4096 + at);
@@ -104,16 +105,18 @@ __global__ void __launch_bounds__(128 * WM, 2) gemm_f32_split_kernel(const GemmF
   constexpr int kH = 12 * TB;   // MFMAs of a half
   auto mul = [&](int h, int v) {
     const int p = v / (2 * TB), b = v / TB % 2, i = v % TB;
-    acc[b][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[h][kw[p]][b], xf[h][kx[p]][i], acc[b][i], 0, 0, 0);
+    acc[b][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[h][pw[p]][b], xf[h][px[p]][i], acc[b][i], 0, 0, 0);
   };
   // level l of the work that makes a piece's parts: part l % 3 of pair l / 3 % 4 of 16-B row chunk l / 12; behind a chunk's last level
   // its parts are written and its registers are requested again, two pieces on
   constexpr int NL = 12 * NR;
   uint32_t q[3][4];
+  float most[NR] = {};   // of the magnitudes of this thread's part of its rows
   auto level = [&](Piece& p, int buf, int l, int k) {
     const int i = l / 12, j = l / 3 % 4, s = l % 3;
     f32x4 v = p.v[2 * i + (j >> 1)];
     float a = v[2 * (j & 1)], b = v[2 * (j & 1) + 1];
+    if (s == 0) asm volatile("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most[i]) : "v"(a), "v"(b));   // here, or the operands are kept for later
     q[s][j] = s < 2 ? part(a, b) : cvt2(a, b);
     v[2 * (j & 1)] = a;
     v[2 * (j & 1) + 1] = b;
@@ -155,7 +158,7 @@ __global__ void __launch_bounds__(128 * WM, 2) gemm_f32_split_kernel(const GemmF
 #pragma unroll
   for (int i = 0; i < NR; ++i) load(even, i, kbase);
 #pragma unroll
-  for (int i = 0; i < NR; ++i) load(odds, i, kbase + 32);
+  for (int i = 0; i < NR; ++i) load(uneven, i, kbase + 32);
   clear_tail(even, kbase);
 #pragma unroll
   for (int l = 0; l < NL; ++l) level(even, 0, l, kbase + 64);
@@ -164,25 +167,56 @@ __global__ void __launch_bounds__(128 * WM, 2) gemm_f32_split_kernel(const GemmF
   for (int i = 0; i < NF; ++i) rd(0, 0, i);
   int k = kbase;
   for (; k + 32 < kend; k += 64) {
-    step(odds, 0, k);
+    step(uneven, 0, k);
     step(even, 1, k + 32);
   }
-  if (k < kend) step(odds, 0, k);
+  if (k < kend) step(uneven, 0, k);
 
-  // A sum that is no ordinary number is done again in 32-bit products: infinities and NaN among the operands (or a value that
-  // rounds to infinity), and sums so small that the parts of their operands may have fallen below bf16's range. That sum alone: the wave does its
-  // block again, but the other sums stay as they are, whoever shares the block.
-  auto odd = [](float sum) {
-    const float v = fabsf(sum);
-    return !(v <= 3.4028234e38f) || (v < 0x1p-64f && v != 0.f);
+  // What is done again in 32-bit products: a sum that is infinite or NaN (so are operands, or one rounds to infinity in bf16), and one whose
+  // operands may have lost parts that count. Parts lose what lies below 2^-126, so a product of operands below 2^32 is off by 2^-92 at most, and
+  // a sum of up to 2^20 of them by no more than an fp32 rounding of 2^-48: a sum below that (0 too, but for rows of zeros) or of a row with an
+  // operand of 2^32 or more is done again. Largest and not smallest operands are looked for, as zeros are common and half an instruction
+  // finds the largest (2018 rows of 16384 x 2048 gated 655 us with and without on 256-row tiles, 832 and 797 on 64-row ones). That sum alone is replaced: the wave does its block again, but the others stay as they are, whoever shares the block.
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const uint64_t large = __ballot(most[i] >= 0x1p32f), some = __ballot(most[i] != 0.f);
+    if (lc == 0) reinterpret_cast<char*>(kind)[lr + kPass * i] = (large >> lane & 15 ? 1 : 0) | (some >> lane & 15 ? 2 : 0);
+  }
+  __syncthreads();
+  int kx[TB];
+  uint32_t kw[2][4];   // of rows 8 q + 4 half .. + 3
+#pragma unroll
+  for (int i = 0; i < TB; ++i) kx[i] = reinterpret_cast<const char*>(kind)[(wm * TB + i) * 32 + l31];
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int z = 0; z < 4; ++z) kw[b][z] = kind[(kX + 64 * b + wn * 32 + 8 * z) / 4 + half];
+  auto odd = [&](int b, int i, int r) {
+    const float v = fabsf(acc[b][i][r]);
+    const int w = kw[b][r >> 2] >> 8 * (r & 3);
+    return !(v <= 3.4028234e38f) || ((kx[i] | w) & 1) || (v < 0x1p-48f && (kx[i] & w & 2));
   };
+  float odds = 0.f, least = 0x1p32f;   // NaN where a sum is no number; the smallest: most blocks are passed by these
+  uint32_t kinds = 0;
   bool any = false;
 #pragma unroll
   for (int b = 0; b < 2; ++b)
 #pragma unroll
     for (int i = 0; i < TB; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) any |= odd(acc[b][i][r]);
+      for (int r = 0; r < 16; ++r) {
+        odds = __builtin_fmaf(acc[b][i][r], 0.f, odds);
+        least = fminf(least, fabsf(acc[b][i][r]));
+        kinds |= kx[i] | kw[b][r >> 2];
+      }
+  if (odds != 0.f || least < 0x1p-48f || (kinds & 0x01010101)) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int i = 0; i < TB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) any |= odd(b, i, r);
+  }
   if (__any(any)) {
 #pragma unroll
     for (int i = 0; i < TB; ++i) {
@@ -199,8 +233,8 @@ __global__ void __launch_bounds__(128 * WM, 2) gemm_f32_split_kernel(const GemmF
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        acc[0][i][r] = odd(acc[0][i][r]) ? g[r] : acc[0][i][r];
-        acc[1][i][r] = odd(acc[1][i][r]) ? u[r] : acc[1][i][r];
+        acc[0][i][r] = odd(0, i, r) ? g[r] : acc[0][i][r];
+        acc[1][i][r] = odd(1, i, r) ? u[r] : acc[1][i][r];
       }
     }
   }

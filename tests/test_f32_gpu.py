@@ -269,3 +269,28 @@ def test_gemm_f32_split_odd_values_leave_other_rows_as_they_are(S, glu):
     for y, z in zip(before, after):
         assert torch.equal(y[r][:, c], z[r][:, c])
         assert ((z == after[0]) | (z.isnan() & after[0].isnan())).all()
+
+
+@pytest.mark.parametrize("rows,S", [(64, 1), (128, 3), (256, 1)])
+@pytest.mark.parametrize("small,large", [(1e-36, 1e20), (1e-38, 1e22), (1e-41, 1e30), (1e-41, 1e9), (1e-30, 2e9), (1e-15, 1.0)])
+def test_gemm_f32_split_small_operands_beside_large_ones(small, large, rows, S):
+    """Operands whose parts leave bf16's range count where their partners are large: sums of them are what 32-bit products give, whether a row is
+    small all along or in one place, also where every part of it rounds to zero."""
+    torch.manual_seed(rows)
+    M, N, K = 150, 260, 272
+    x, w = torch.randn(M, K, dtype=torch.float64), torch.randn(N, K, dtype=torch.float64)
+    x[:40] *= small
+    w[:192] *= large   # whole blocks of sums without a small one
+    x[60:70] = 0.0
+    x[60:65, 100] = small
+    w[192:230] *= small
+    x[100:120, 3::4] *= large
+    x, w = x.float().to(DEV), w.float().to(DEV)
+    y, r = _split(x, w, rows, S), x.double() @ w.double().t()
+    mag = x.double().abs() @ w.double().abs().t()
+    fin = mag < 1e38
+    assert ((y.double() - r).abs() <= (K + 8) * 2.0 ** -24 * mag + K * 2.0 ** -149)[fin].all()
+    plain = _split(x, w, 0)   # the fp32 instruction: as close, but for the order of the sums
+    for a, b in ((slice(0, 40), slice(0, 192)), (slice(100, 120), slice(192, 230))):
+        err, ref = ((t.double() - r)[a, b].norm() for t in (y, plain))
+        assert err <= 1.25 * ref
