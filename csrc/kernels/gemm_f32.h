@@ -31,6 +31,6 @@ __device__ __forceinline__ void put4(float* y, const f32x4& v, int n, bool vec) 
   }
 }
 
-int gemm_f32_split(const GemmF32& a, bool glu, int rows, hipStream_t stream);   // rows of a tile: 64 or 128
+int gemm_f32_split(const GemmF32& a, bool glu, int rows, hipStream_t stream);   // rows of a tile: 64, 128 or 256
 
 }  // namespace oamd

@@ -1,12 +1,12 @@
 // fp32 products on the bf16 matrix instruction: each operand as the sum of three bf16 numbers (8 significand bits each: all 24 are kept),
 // six of the nine partial products, 32-bit sums. What is left out, the second part of one operand by the third of the other and the third
-// by the third, is below 2^-26 of a product, a quarter of an fp32 rounding; this is the splitting of Henry, Tang and Heinecke, "Leveraging
-// the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations" (2019). A sum is rounded 6 times per 16 columns
-// where the fp32 instruction rounds it for each: 962 rows of 2048 x 2048 are 7.0e-7 from the 64-bit result (the fp32 instruction's
-// 8.1e-7), of 2048 x 8192 in one slice 1.4e-6 (1.6e-6), in four 7.3e-7.
+// by the third, is at most 2^-24 of a product (just above a power of two: 1.0038986 squared), an fp32 rounding, and 2^-26.5
+// of evenly spread ones (root mean square); this is the splitting of Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For
+// Higher-Precision Computations" (2019). A sum is rounded 6 times per 16 columns where the fp32 instruction rounds it for each: 962 rows of
+// 2048 x 2048 are 7.0e-7 from the 64-bit result (the fp32 instruction's 8.1e-7), of 2048 x 8192 in one slice 1.4e-6 (1.6e-6), in four 7.3e-7.
 //
 // What bounds it: the bf16 matrix instruction's power. Six partial products are 192 clocks of MFMAs per 32 x 32 x 16 products where the fp32
-// instruction takes 512. An operand element costs 5.5 VALU instructions, done once per workgroup on the way into LDS and spread between
+// instruction takes 512. An operand element costs 6 VALU instructions, done once per workgroup on the way into LDS and spread between
 // the MFMAs of the step before; at the clock that is left 213 TFLOP/s (1.3 PFLOP/s of bf16 products, what a large bf16 product reaches), against
 // 122 of the fp32 instruction's kernel:
 //   962 rows   16384 x 2048 gated 560 -> 315 us, 2048 x 8192 298 -> 168, 2048 x 2048 80 -> 54
@@ -15,7 +15,8 @@
 // Why this shape: 256 rows x 128 features are 8 waves of 64 x 64, two per SIMD, so one wave's conversions, reads and waits run under the
 // other's MFMAs (four waves of 64 x 64 took 728 us where these take 634), and both operands' parts fit in LDS twice (147 KB): one barrier per
 // 32 columns. Pieces are requested two steps before they are split, in registers. With fewer rows 128-row tiles of eight waves
-// and 64-row ones of four, two to a CU, fill more CUs (ops.f32_split_rows); all sum K in the same order, so the bits are the same.
+// and 64-row ones of four, two to a CU, fill more CUs (ops.f32_split_rows); all sum K in the same order, and what
+// is done again is so by itself, so the bits are the same.
 #include <utility>
 
 #include "common.h"

@@ -294,3 +294,11 @@ def test_gemm_f32_split_small_operands_beside_large_ones(small, large, rows, S):
     for a, b in ((slice(0, 40), slice(0, 192)), (slice(100, 120), slice(192, 230))):
         err, ref = ((t.double() - r)[a, b].norm() for t in (y, plain))
         assert err <= 1.25 * ref
+
+
+@pytest.mark.parametrize("rows", [64, 256])
+def test_gemm_f32_split_drops_no_more_than_a_rounding(rows):
+    """Operands of which the products left out add up to the most: 2^-24 of each product, all to one side."""
+    x, w = (torch.full((n, 16), 1.0038986, device=DEV) for n in (70, 130))
+    r = x.double() @ w.double().t()
+    assert ((_split(x, w, rows).double() - r).abs() <= (1 + 6) * 2.0 ** -24 * r).all()   # and six roundings of the sum
