@@ -87,8 +87,14 @@ class Scorer {
   // hits [n, 3] = (doc, matcher, line) -> per doc its events (pattern, line, score), best first
   py::list score(py::array_t<int64_t, py::array::c_style | py::array::forcecast> hits, int64_t num_docs) const {
     if (hits.ndim() != 2 || hits.shape(1) != 3) throw std::invalid_argument("hits [n, 3]");
+    const int64_t *h = hits.data(), n = hits.shape(0);
+    std::vector<std::vector<Ev>> all;
+    {
+      py::gil_scoped_release others;
+      all = events(h, n, 3, num_docs);
+    }
     py::list result;
-    for (const auto& evs : events(hits.data(), hits.shape(0), 3, num_docs)) {
+    for (const auto& evs : all) {
       py::list dl(evs.size());
       for (size_t i = 0; i < evs.size(); ++i) dl[i] = py::make_tuple(evs[i].pat, evs[i].line, evs[i].score);
       result.append(std::move(dl));

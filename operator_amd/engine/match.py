@@ -166,8 +166,8 @@ class MatchEngine:
     """Compile a PatternSet once, then analyze batches of logs on one device."""
 
     SCAN_LANES = 256 * 1024   # ac_scan v2 streams on MI355X (256 CUs x 1024 threads)
-    # hits that are scored natively, and whose results are built so: 3077 events of 1024 logs 10.9 ms, 18.4 by way of the GPU's sorts and Python's
-    # results; 12828 of 64 logs 7.7 and 18.3
+    # hits that are scored natively, and whose results are built so: whole batches of 64 KiB logs with 2.6, 10, 41 and 82 thousand hits 3.4, 17, 89
+    # and 189 ms, 6.9, 34, 162 and 339 by way of the GPU's sorts and Python's results; other threads wait no longer (results.cpp)
     HOST_SCORE_HITS = 1 << 16
     # context windows of a few logs' events are located on the host (3 events: 1 us against 30 for the round trip to the GPU);
     # larger batches leave the host to the next batch's packing

@@ -161,3 +161,43 @@ def test_search_passes_over_bytes_no_match_starts_at(rx, line):
     prog = compile_nfa(rx, 0)
     assert prog is not None
     assert patterns().RegexSet([prog]).search(0, line) == (re.search(rx, line) is not None)
+
+
+def test_large_results_leave_the_lock_to_other_threads():
+    """Scoring, context lines and result objects of a large batch take a tenth of a second and more: another thread runs in between, not behind."""
+    import gc
+    import threading
+    import time
+
+    eng = MatchEngine(compile_patterns(synthetic_library(200, seed=2)), device="cpu", max_events=1000)
+    eng.analyze([b"x\n"])
+    rng = np.random.default_rng(0)
+    lines, per, n = 5000, 1000, 64
+    doc = b"".join(b"line %05d " % i + b"x" * 50 + b"\n" for i in range(lines))
+    rows = np.concatenate([np.stack([np.full(per, d), rng.choice(eng.cp.pattern_primary, per), rng.choice(lines, per, replace=False), np.zeros(per)], 1)
+                           for d in range(n)]).astype(np.int64)
+    rows[:, 3] = rows[:, 2] * (len(doc) // lines)
+    stop, ticks = threading.Event(), []
+
+    def tick():
+        while not stop.is_set():
+            ticks.append(time.perf_counter())
+
+    other = threading.Thread(target=tick)
+    was = gc.isenabled()
+    gc.disable()   # as in analyze: a collection holds the lock too
+    other.start()
+    try:
+        batch = patterns().ResultBatch(eng._tables, [doc] * n, rows, eng.max_events, 0.5, bytes(16 * n))
+        t0 = time.perf_counter()
+        batch.windows()
+        t1 = time.perf_counter()
+        assert len(batch.build_all(None, None, t0)) == n
+        t2 = time.perf_counter()
+    finally:
+        stop.set()
+        other.join()
+        if was:
+            gc.enable()
+    for a, b in ((t0, t1), (t1, t2)):
+        assert b - a < 0.02 or any(a + 0.3 * (b - a) < t < b - 0.3 * (b - a) for t in ticks)
