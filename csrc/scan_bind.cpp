@@ -166,37 +166,20 @@ std::pair<int64_t, int64_t> scan_batch(const at::Tensor& text, int64_t total, in
   return {r[num_docs], r[num_docs + 1]};
 }
 
-void context_spans(const at::Tensor& text, const at::Tensor& doc_base, const at::Tensor& doc_len,
-                   const at::Tensor& q, at::Tensor& out) {
-  CHECK_T(text, at::kByte);
-  CHECK_T(doc_base, at::kLong);
-  CHECK_T(doc_len, at::kLong);
-  CHECK_T(q, at::kLong);
-  CHECK_T(out, at::kLong);
-  TORCH_CHECK(q.dim() == 2 && q.size(1) == 3 && out.dim() == 2 && out.size(1) == 4 && out.size(0) >= q.size(0),
-              "context_spans: q [n, 3], out [n, 4]");
-  TORCH_CHECK(doc_base.numel() == doc_len.numel(), "context_spans: doc_base / doc_len");
-  const c10::hip::HIPGuardMasqueradingAsCUDA g(text.device());
-  const int rc = oamd::context_spans(text.data_ptr<uint8_t>(), doc_base.data_ptr<int64_t>(),
-                                     doc_len.data_ptr<int64_t>(), q.data_ptr<int64_t>(), (int)q.size(0),
-                                     out.data_ptr<int64_t>(), c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream());
-  TORCH_CHECK(rc == 0, "context_spans launch failed rc=", rc);
-}
-
-// The same for n queries in pinned memory, waited for: one launch instead of two copies, a launch and two allocations (192 queries
-// 86 -> 31 us). The kernel reads a query once, with one wave, and writes its answer once, so the host's memory costs it no more.
-void context_spans_pinned(const at::Tensor& text, const at::Tensor& doc_base, const at::Tensor& doc_len, const at::Tensor& q, at::Tensor& out,
-                          int64_t n) {
+// The line windows of n queries q [n, 3] = (doc, byte offset, lines) into out [n, 4], both the front of buffers in pinned memory, waited for: one
+// launch, where tensors on the GPU take two copies and two allocations more (192 queries 31 us against 86). The kernel reads a query once, with one wave, and writes its answer once, so the host's memory costs it no more.
+void context_spans(const at::Tensor& text, const at::Tensor& doc_base, const at::Tensor& doc_len, const at::Tensor& q, at::Tensor& out,
+                   int64_t n) {
   CHECK_T(text, at::kByte);
   CHECK_T(doc_base, at::kLong);
   CHECK_T(doc_len, at::kLong);
   for (const auto* t : {&q, static_cast<const at::Tensor*>(&out)})
-    TORCH_CHECK(t->is_pinned() && t->is_contiguous() && t->scalar_type() == at::kLong, "context_spans_pinned: pinned int64");
-  TORCH_CHECK(n >= 0 && n < (int64_t(1) << 31) && q.numel() >= 3 * n && out.numel() >= 4 * n, "context_spans_pinned: q [n, 3], out [n, 4]");
-  TORCH_CHECK(doc_base.numel() == doc_len.numel(), "context_spans_pinned: doc_base / doc_len");
+    TORCH_CHECK(t->is_pinned() && t->is_contiguous() && t->scalar_type() == at::kLong, "context_spans: pinned int64");
+  TORCH_CHECK(n >= 0 && n < (int64_t(1) << 31) && q.numel() >= 3 * n && out.numel() >= 4 * n, "context_spans: q [n, 3], out [n, 4]");
+  TORCH_CHECK(doc_base.numel() == doc_len.numel(), "context_spans: doc_base / doc_len");
   const int64_t* docs = q.data_ptr<int64_t>();
   for (int64_t i = 0; i < n; ++i)
-    TORCH_CHECK(docs[3 * i] >= 0 && docs[3 * i] < doc_base.numel(), "context_spans_pinned: doc");
+    TORCH_CHECK(docs[3 * i] >= 0 && docs[3 * i] < doc_base.numel(), "context_spans: doc");
   const c10::hip::HIPGuardMasqueradingAsCUDA g(text.device());
   const hipStream_t st = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
   const int rc = oamd::context_spans(text.data_ptr<uint8_t>(), doc_base.data_ptr<int64_t>(), doc_len.data_ptr<int64_t>(),
@@ -248,7 +231,6 @@ PYBIND11_MODULE(_S, m) {
   m.def("line_prefix", &line_prefix);
   m.def("doc_lines", &doc_lines);
   m.def("context_spans", &context_spans);
-  m.def("context_spans_pinned", &context_spans_pinned);
   m.def("line_prefix_state_words", [](int64_t n) { return (oamd::line_prefix_state_words(n) + 1) & ~1ll; });
   m.def("ac_scan", &ac_scan);
   m.def("scan_work_bytes", &scan_work_bytes);

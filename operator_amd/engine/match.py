@@ -437,7 +437,7 @@ class MatchEngine:
         # the kernel runs on the scan stream, behind the scan, and reads and writes pinned memory: no copy on a stream that the
         # LLM's decode graphs keep busy for tens of ms
         with (torch.cuda.stream(stream) if stream is not None else self._on_stream()):
-            kernels().context_spans_pinned(text, base, lens, q, out, n)
+            kernels().context_spans(text, base, lens, q, out, n)
         return out.numpy()[:4 * n].reshape(n, 4)
 
     def scan_cpu(self, docs: list[bytes]) -> np.ndarray:

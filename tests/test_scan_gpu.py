@@ -203,14 +203,23 @@ def test_context_spans_equal_host_contexts():
             q_doc.append(di)
             q_off.append(o)
             q_k.append(rng.randrange(0, 6))
-    q = torch.tensor(list(zip(q_doc, q_off, q_k)), dtype=torch.int64).cuda()
-    out = torch.empty(len(q_doc), 4, dtype=torch.int64, device="cuda")
+    n = len(q_doc)
+    q, out = (torch.full(((n + 5) * c,), -(1 << 40), dtype=torch.int64).pin_memory() for c in (3, 4))   # buffers of larger batches
+    q[:3 * n] = torch.tensor(list(zip(q_doc, q_off, q_k)), dtype=torch.int64).flatten()
     base = torch.tensor(first[:-1], dtype=torch.int64).cuda() * seg
     lens = torch.tensor([len(d) for d in docs], dtype=torch.int64).cuda()
-    kernels().context_spans(text, base, lens, q, out)
-    got = P.contexts_from_spans(docs, q_doc, out.cpu().numpy())
     want = P.contexts(docs, q_doc, q_off, q_k)
-    assert got == want
+    for m in (n, 3, 0):   # what lies behind the queries is neither read nor written
+        out.fill_(-7)
+        kernels().context_spans(text, base, lens, q, out, m)
+        assert P.contexts_from_spans(docs, q_doc[:m], out.numpy()[:4 * m].reshape(m, 4)) == want[:m] and (out[4 * m:] == -7).all()
+    for bad in (-1, len(docs)):   # refused on the host, before the launch
+        q[3] = bad
+        with pytest.raises(RuntimeError):
+            kernels().context_spans(text, base, lens, q, out, 2)
+    for args in ((q.cuda(), out, 1), (q, out.cuda(), 1), (q, out, n + 6), (q, out, -1), (q.int(), out, 1), (q.clone(), out, 1)):
+        with pytest.raises(RuntimeError):
+            kernels().context_spans(text, base, lens, *args)
     # through the engine: eager analyze locates its windows on the GPU, same results as the host
     ps = synthetic_library(200, seed=3)
     fac = LogFactory(n_patterns=200, seed=9)
