@@ -532,7 +532,8 @@ def rows_plan(M: int, N: int, K: int, glu: bool = False) -> tuple[int, int] | No
 
 
 def _rows_plan(M: int, N: int, K: int, glu: bool) -> tuple[int, int] | None:
-    """rows_plan where no measured entry or switch has another kernel."""
+    """rows_plan, but for products that a measured "blas" or OAMD_SKINNY=0 sends to hipBLASLt. Measured slice counts are gemm_skinny's: of a product
+    that goes to gemm_rows they only decide, as ever, whether it stays in fp32 for its consumer (more than one slice) or is rounded to bf16."""
     if M > ROWS_MAX_M or skinny_plan(M, N, K) is None or (_gemm_table_get().get(("silu", M, N, K)) == "blas" if glu else _measured_blas(M, N, K)):
         return None
     return rows_plan(M, N, K, glu)

@@ -77,6 +77,7 @@ def test_linear_takes_them_there(M, N, K):
     S, _ = ops.rows_plan(M, N, K)
     _close(ops.linear(x, w), x, w, False)
     d = ops.linear(x, w, defer_reduce=True)
+    assert isinstance(d, ops.SplitK) == (max(S, ops.skinny_plan(M, N, K)) > 1)
     if isinstance(d, ops.SplitK):
         assert d.S == S
         _close(d.p[:S * M * N].view(S, M, N).sum(0), x, w, True)
@@ -86,14 +87,10 @@ def test_linear_takes_them_there(M, N, K):
     assert ops.linear(x, w, out=out) is out
     _close(out, x, w, False)
     wide = torch.full((M, N + 16), float("nan"), dtype=torch.bfloat16, device=DEV)   # rows apart
-    if M > 1:
-        try:
+    if M > 1:   # refused, as by gemm_skinny, which takes whole rows
+        with pytest.raises(RuntimeError):
             ops.linear(x, w, out=wide[:, :N])
-        except RuntimeError:   # as gemm_skinny, which takes whole rows
-            pass
-        else:
-            _close(wide[:, :N], x, w, False)
-        assert wide[:, N:].isnan().all()
+        assert wide.isnan().all()
 
 
 @pytest.mark.gpu
