@@ -29,17 +29,22 @@ void put(const py::object& dict, const py::object& key, const py::object& value)
 
 // Lets go of the interpreter's lock every 8 ms: 51200 events of 1024 logs take 130 ms and more here, which kept every other thread waiting
 // to the end. A thread that waits asks for the lock after 5 ms (the interpreter's default), and a lock that was asked for is not taken back before
-// the other had it; let go more often it would be, before that thread is awake, and its 5 ms would start again.
+// the other had it; let go more often it would be, before that thread is awake, and its 5 ms would start again. The clock is read every 64 times,
+// about 0.3 ms: read for every event it was 4 % of a batch of 64 logs.
 class Turns {
  public:
   void operator()() {
-    if (std::chrono::steady_clock::now() - last_ < std::chrono::milliseconds(8)) return;
+    if (++count_ % 64) return;
+    const auto now = std::chrono::steady_clock::now();
+    if (count_ == 64) last_ = now;
+    if (now - last_ < std::chrono::milliseconds(8)) return;
     { py::gil_scoped_release others; }
     last_ = std::chrono::steady_clock::now();
   }
 
  private:
-  std::chrono::steady_clock::time_point last_ = std::chrono::steady_clock::now();
+  uint32_t count_ = 0;
+  std::chrono::steady_clock::time_point last_;
 };
 
 py::object number(int64_t v) { return steal(PyLong_FromLongLong(v)); }
