@@ -20,11 +20,13 @@
 //     S | 8 the blocks of one K-slice share an XCD (block id % 8), so each
 //     XCD's L2 holds only its slice of X; other S (<= 16) cut K into slices
 //     that differ by at most one 64-column step;
-//   * column tile n starts its slice at K step n % steps and goes round. Tiles in step would all read the same 128 columns of rows that lie a
-//     power of two apart, which HBM serves from some of its channels: 64 rows of 128256 x 4096 213 -> 175 us (4.9 -> 6.0 TB/s), 28672 x 4096
-//     gated 46 -> 38, 57344 x 8192 gated 175 -> 148, 32000 x 4096 59 -> 42, 8192 x 8192 32 -> 28; 128 rows of 32000 x 4096 59 -> 53. Where rows
-//     are no such distance apart (3584 columns) it changes nothing. Experts' tiles of 64 rows start 5 steps further an expert: 96 tokens on
-//     8 experts of 4096 x 4096 172 -> 134 us, on 64 of 2048 x 1024 178 -> 150; of 128 rows, whose X weighs more, they keep step (112 rows each 242, 258 round).
+//   * where rows lie a multiple of 4 KB apart (K % 2048 == 0), column tile n starts its slice at K step n % steps and goes round: tiles in step would
+//     all read the same 128 columns of such rows, which HBM serves from some of its channels (times of weights that no cache holds): 64 rows of
+//     128256 x 4096 217 -> 181 us (4.8 -> 5.8 TB/s), 57344 x 8192 gated 194 -> 158, 28672 x 6144 80 -> 63. At other distances it costs 1 to 10 %,
+//     most beside a multiple (64 rows of 4032 or 4160 columns 10 %, 3584 2 %; 128-row tiles 5 %), and gains in none but 11008 columns (5 %).
+//     Experts' tiles of 64 rows start 5 steps further an expert: 8 rows for each of 8 experts of 4096 x 4096 183 -> 140 us, of 64 of 2048 x 1024
+//     179 -> 155 (by the product over 2048 columns; 16 of 3456 x 2368 151 in step, 159 round); of 128 rows, whose X weighs more, they keep
+//     step (112 rows each 242, 258 round).
 // MFMA v_mfma_f32_16x16x32_bf16; fragment maps as in attn_decode.hip.
 #include "common.h"
 #include "kernels.h"
@@ -44,9 +46,11 @@ constexpr int kWaves = 8;
 // Most elements of X whose K steps go round. Tiles in step share a piece of X while it is in their XCD's L2, tiles that are not need all of
 // X there (4 MiB): 128 rows of 8192 x 28672 88 us in step, 96 round, of 3584 x 18944 30 and 41. 256-row tiles are not bound by HBM (32768 x 2048 40 and 43).
 constexpr int64_t kTurnX = 1 << 20;
-// Fewest weights whose K steps go round: the addresses cost a little (64 rows of 4096 x 4096 8.9 us in step, 9.8 round; 14336 x 2048 16.0 and 17.2; 4096 x 11008
-// 19.5 and 18.1, 12288 x 4096 24.7 and 20.6), as they do in 128 x 64 tiles (28672 x 4096 65 and 70).
-constexpr int64_t kTurnW = 1 << 25;
+// Fewest columns of Y whose K steps go round, by the rows of X and of a tile, in 64: fewer tiles leave channels idle either way, and the addresses
+// cost a little. 64 rows of K = 4096 and 8192: 14336 columns 37.0 us in step, 37.0 round and 70.1, 68.4, 20480 41.0, 39.6 and 80.8, 73.4, 8192
+// 32.1, 33.4 and 61.4, 65.1; 128 rows in 64-row tiles: 20480 69.0, 70.8 and 132.7, 133.4, 28672 86.2, 79.6 and 168, 152; in 128-row tiles: 28672 53.1, 55.1
+// and 97.0, 99.0, 34176 97.9, 92.8 and 186, 179.
+constexpr int kTurnN = 8192;
 
 // BN = 128 halves the LDS fragment traffic per MFMA (64 x 64 wave tiles at
 // M = 256: 0.5 KB of ds_read per MFMA vs 0.75 KB at BN = 64, where the LDS
@@ -285,20 +289,23 @@ int splitk_reduce(const float* P, bf16_t* Y, int64_t MN, int S, hipStream_t stre
   return 0;
 }
 
+static bool turns(int K) { return K % 2048 == 0; }
+
 int moe_gemm_rows(const bf16_t* X, const bf16_t* W, bf16_t* Y, int max_rows, int N, int K, int bm, bool silu_gu,
                   const int* gtab, const int* src, const float* rscale, hipStream_t stream) {
   if (max_rows == 0) return 0;
   if ((bm != 64 && bm != 128) || max_rows % bm != 0 || N % 128 != 0 || K % kBK != 0 || gtab == nullptr) return -1;
   if (silu_gu && rscale == nullptr) return -2;
   const dim3 grid(N / 128, max_rows / bm);
-  if (bm == 64 && silu_gu)
-    gemm_tn_kernel<64, 128, kEpiSiluGU, 3, true, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2, gtab, src, rscale);
-  else if (bm == 64)
-    gemm_tn_kernel<64, 128, kEpiStore, 3, true, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2, gtab, src, rscale);
-  else if (silu_gu)
-    gemm_tn_kernel<128, 128, kEpiSiluGU, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2, gtab, src, rscale);
-  else
-    gemm_tn_kernel<128, 128, kEpiStore, 3, true><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2, gtab, src, rscale);
+#define OAMD_ROWS(BM, EPI, TURN) \
+  gemm_tn_kernel<BM, 128, EPI, 3, true, TURN><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, nullptr, max_rows, N, K, 1, 2, gtab, src, rscale)
+  if (bm == 128 && silu_gu) OAMD_ROWS(128, kEpiSiluGU, false);
+  else if (bm == 128) OAMD_ROWS(128, kEpiStore, false);
+  else if (turns(K) && silu_gu) OAMD_ROWS(64, kEpiSiluGU, true);
+  else if (turns(K)) OAMD_ROWS(64, kEpiStore, true);
+  else if (silu_gu) OAMD_ROWS(64, kEpiSiluGU, false);
+  else OAMD_ROWS(64, kEpiStore, false);
+#undef OAMD_ROWS
   OAMD_LAUNCH_CHECK();
   return 0;
 }
@@ -308,7 +315,7 @@ int gemm_decode(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, in
   // bit 0: tiled W layout; bit 1: W streams with the non-temporal policy (OAMD_BF16_WNT)
   static const int wnt = [] { const char* e = getenv("OAMD_BF16_WNT"); return e && e[0] == '0' ? 0 : 2; }();
   const int w_tiled = (w_tiled_b ? 1 : 0) | wnt;
-  const bool turn = M <= 128 && (int64_t)M * K <= kTurnX && (int64_t)N * K >= kTurnW;
+  const bool turn = turns(K) && M <= 128 && (int64_t)M * K <= kTurnX && (int64_t)N * S >= kTurnN * ((M + BM) / 64);
   if (w_tiled_b && (N % 64 != 0 || K % 64 != 0)) return -6;
   if ((BM != 64 && BM != 128 && BM != 256) || M % BM != 0) return -1;
   if (glu) {  // fused SwiGLU: one K slice, 128-column tiles of 64 gate + 64 up rows

@@ -471,10 +471,10 @@ def _vocab_plan(M: int, N: int, K: int):
     """Decode-bucket vocabulary projection: one row tile of all rows against 128-column tiles, so that the weights
     are read once (256 rows of 32768 x 4096: 73 us, 102 on 64 columns; 128 rows 59 and 62). A 128256-row
     vocabulary at 256 rows is the tile kernel's (253 us against 289), one of 8192 columns too past 64 rows (128 rows 418 against
-    447, 256 rows 449 against 617; 64 rows 374 against 334); rows that are not one tile would read the weights again. Both lines lie between
+    447, 256 rows 449 against 617; 64 rows 374 against 334, on tiles whose K steps go round: more columns that are no multiple of 2048 stay); rows that are not one tile would read the weights again. Both lines lie between
     sizes that were timed: 32000 to 152064 rows of 2048 to 8192 columns, 64 to 256 rows, none of them slower than on 64 columns
     (152064 x 3584: 64 rows 192 us against 223, 256 rows 306 against 430; profiles/plans_before_after.txt)."""
-    if row_tile(M) != M or (K >= 8192 and M > 64) or (M == 256 and N >= 2 * LM_HEAD_MIN_N) or N % 128:
+    if row_tile(M) != M or (K >= 8192 and (M > 64 or K % 2048)) or (M == 256 and N >= 2 * LM_HEAD_MIN_N) or N % 128:
         return None
     return (M, 128, 1, 3)
 

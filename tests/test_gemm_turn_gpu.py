@@ -15,7 +15,7 @@ def _check(y, x, w, K):
     assert ((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + (K + 16) * 2.0 ** -24 * mag).all()
 
 
-# on either side of the weights (2^25 elements) and the X (2^20) that turn, 128-row tiles over 64 columns, which never do
+# on either side of the columns and the X (2^20) that turn and of 2048 columns apart, 128-row tiles over 64 columns, which never do
 @pytest.mark.parametrize("M,N,K,S,bn,bm,stages", [
     (64, 1152, 192, 3, 64, 64, 3), (64, 524288, 64, 1, 128, 64, 3), (64, 175360, 192, 3, 64, 64, 3), (64, 32768, 1024, 1, 128, 64, 4),
     (64, 25024, 1344, 5, 64, 64, 6), (128, 75008, 448, 2, 128, 64, 2), (128, 4096, 8192, 1, 128, 128, 4), (128, 4096, 8256, 3, 128, 128, 3),
@@ -61,3 +61,18 @@ def test_gated(M, N, K, ns):
     # gate, silu(gate), up and the product are rounded to bf16: 2^-8 of each (silu's slope is at most 1.1); second order and the fp32 sums
     tol = 1.02 * 2.0 ** -8 * up.abs() * (1.1 * gate.abs() + 3 * sg.abs()) + 1e-4 * (1 + up.abs() + gate.abs())
     assert ((y.double() - sg * up).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("M,N,K,bn,bm,turn", [
+    (64, 16384, 2048, 128, 64, True), (64, 16256, 2048, 128, 64, False), (64, 16384, 4096, 64, 64, True), (64, 28672, 3584, 128, 64, False),
+    (64, 34176, 4160, 128, 64, False), (128, 24576, 2048, 64, 64, True), (128, 24512, 2048, 64, 64, False), (128, 32768, 4096, 128, 128, True),
+    (128, 28672, 4096, 128, 128, False), (128, 34176, 4032, 128, 128, False)])
+def test_only_rows_a_multiple_of_2048_columns_apart_turn(M, N, K, bn, bm, turn):
+    """Where steps go round a column's sum depends on its tile, elsewhere it does not."""
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    x, w = (torch.randn(n, K, generator=g, device="cuda").bfloat16() for n in (M, N))
+    C, at = ops.kernels(), bn * 37
+    y, z = (torch.empty(M, n, device="cuda").bfloat16() for n in (N, bn))
+    C.gemm_decode(x, w, y, None, 1, bn, bm, False, False, 3)
+    C.gemm_decode(x, w[at:at + bn].contiguous(), z, None, 1, bn, bm, False, False, 3)   # one tile: in step
+    assert torch.equal(y[:, at:at + bn], z) != turn
