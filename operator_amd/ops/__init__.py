@@ -780,11 +780,14 @@ def _f32_plain_us(M: int, N: int, K: int, glu: int) -> float:
 def f32_split_slices(M: int, N: int, K: int, glu: int) -> int | None:
     """K slices in which ``M`` rows (f32_plan_rows) run on the split kernel (gemm_f32_split.hip), or None: on the fp32 matrix instruction
     (f32.hip), up to 32 rows and where the split kernel, whose steps wait for more before the first, is not estimated 10 % faster (512
-    rows of 2048 x 288 9 us against 14, of 2048 x 768 24 and 24, of 2048 x 2048 50 and 37; 2000 rows of 2048 x 288 27 and 20)."""
+    rows of 2048 x 288 9 us against 14, of 2048 x 768 24 and 24, of 2048 x 2048 50 and 37; 2000 rows of 2048 x 288 27 and 20). No fewer slices than
+    the fp32 instruction would have: sums that are as long are closer to the 64-bit result (0.86 of its distance), but one slice in the place of four is
+    further off (3200 x 1376 gated 1.8 times)."""
     if M <= SKINNY_MAX_M:
         return None
-    cost, S = min((_f32_split_us(r, s, M, N, K, glu), s) for r in _F32_SPLIT for s in range(1, 9)
-                  if s == 1 or (N % 4 == 0 and K // 32 // s >= 4))
+    plans = [(min(_f32_split_us(r, s, M, N, K, glu) for r in _F32_SPLIT), s) for s in range(kernels().gemm_f32_splits(M, N, K, glu), 9)
+             if s == 1 or (N % 4 == 0 and K // 32 // s >= 4)]
+    cost, S = min(plans, default=(float("inf"), 1))
     return S if cost < 0.9 * _f32_plain_us(M, N, K, glu) else None
 
 

@@ -25,6 +25,14 @@ def test_lines():
     assert ops.f32_split_slices(512, 2048, 8192, 0) is not None  # 161 against 99
 
 
+@pytest.mark.parametrize("N,K,glu", [(16384, 2048, ops.GELU_TANH), (2048, 8192, 0), (3200, 1376, ops.SILU), (8064, 960, ops.SILU), (384, 6048, ops.SILU),
+                                     (2912, 560, 0), (2050, 2048, 0), (704, 688, 0), (1024, 96, ops.SILU)])
+def test_sums_are_no_longer_than_on_the_fp32_instruction(N, K, glu):
+    for M in (33, 40, 64, 100, 200, 512, 1024, 1536, 2048, 4096):
+        S = ops.f32_split_slices(M, N, K, glu)
+        assert S is None or S >= ops.kernels().gemm_f32_splits(M, N, K, glu)
+
+
 def test_the_split_kernels_loads_stay_in_their_rows(tmp_path):
     """Every piece that the kernel requests, two behind the last of a row and of a slice among them, for all K up to 200 and slices up to 8."""
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
