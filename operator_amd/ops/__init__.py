@@ -769,8 +769,7 @@ def _f32_split_us(rows: int, S: int, M: int, N: int, K: int, glu: int) -> float:
     return max(t, 6 + 4e-6 * N * K / 4.5) + _f32_slabs(M, N, S, glu)
 
 
-def _f32_plain_us(M: int, N: int, K: int, glu: int) -> float:
-    S = kernels().gemm_f32_splits(M, N, K, glu)
+def _f32_plain_us(M: int, N: int, K: int, glu: int, S: int) -> float:
     full, last = divmod(-(-(-(-M // 64) * -(-(N // 2 if glu else N) // 64) * S) // CUS), 3)
     t = 3.2 + -(-K // (32 * S)) * (2 if glu else 1) * (full * _F32_PLAIN[2] + (_F32_PLAIN[last - 1] if last else 0))
     return max(t, 3.2 + 4e-6 * N * K / 4) + _f32_slabs(M, N, S, glu)
@@ -782,13 +781,19 @@ def f32_split_slices(M: int, N: int, K: int, glu: int) -> int | None:
     (f32.hip), up to 32 rows and where the split kernel, whose steps wait for more before the first, is not estimated 10 % faster (512
     rows of 2048 x 288 9 us against 14, of 2048 x 768 24 and 24, of 2048 x 2048 50 and 37; 2000 rows of 2048 x 288 27 and 20). No fewer slices than
     the fp32 instruction would have: sums that are as long are closer to the 64-bit result (0.86 of its distance), but one slice in the place of four is
-    further off (3200 x 1376 gated 1.8 times)."""
+    further off (3200 x 1376 gated 1.8 times).
+
+    A prompt's rows are padded to a multiple of 512 for its plan, but run as they are: slices count that are no slower at the fewest rows of that
+    plan either (33 rows of 6144 x 2048 in one slice 56 us against 46, in two 33; of 2912 x 560 19 and 11 whatever the slices)."""
     if M <= SKINNY_MAX_M:
         return None
-    plans = [(min(_f32_split_us(r, s, M, N, K, glu) for r in _F32_SPLIT), s) for s in range(kernels().gemm_f32_splits(M, N, K, glu), 9)
-             if s == 1 or (N % 4 == 0 and K // 32 // s >= 4)]
-    cost, S = min(plans, default=(float("inf"), 1))
-    return S if cost < 0.9 * _f32_plain_us(M, N, K, glu) else None
+    former = kernels().gemm_f32_splits(M, N, K, glu)
+    few = M if M % 512 else max(M - 511, SKINNY_MAX_M + 1)
+    us = lambda m, s: min(_f32_split_us(r, s, m, N, K, glu) for r in _F32_SPLIT)  # noqa: E731
+    limit = _f32_plain_us(few, N, K, glu, former)
+    cost, S = min(((us(M, s), s) for s in range(former, 9) if (s == 1 or (N % 4 == 0 and K // 32 // s >= 4)) and us(few, s) <= limit),
+                  default=(float("inf"), 1))
+    return S if cost < 0.9 * _f32_plain_us(M, N, K, glu, former) else None
 
 
 @functools.lru_cache(maxsize=4096)

@@ -33,6 +33,14 @@ def test_sums_are_no_longer_than_on_the_fp32_instruction(N, K, glu):
         assert S is None or S >= ops.kernels().gemm_f32_splits(M, N, K, glu)
 
 
+def test_the_fewest_rows_of_a_plan_are_no_slower():
+    """Prompts of 33 rows have the plan of 512: where the split kernel is slower for them in every number of slices, it is not taken."""
+    assert ops.f32_split_slices(512, 2912, 560, 0) is None and ops.f32_split_slices(512, 620, 3024, 0) is None   # 33 rows: 11 us against 18, 15 and 21
+    assert ops.f32_split_slices(512, 6144, 2048, 0) >= 2      # in one slice 46 us against 56, in two 33
+    assert ops.f32_split_slices(512, 2050, 2048, 0) is None   # has no slices: 47 and 56
+    assert ops.f32_split_slices(300, 2050, 2048, 0) is None and ops.f32_split_slices(500, 2050, 2048, 0) == 1   # no prompts: rows as they are
+
+
 def test_the_split_kernels_loads_stay_in_their_rows(tmp_path):
     """Every piece that the kernel requests, two behind the last of a row and of a slice among them, for all K up to 200 and slices up to 8."""
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
