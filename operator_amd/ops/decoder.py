@@ -29,6 +29,11 @@ MOE_LIST_ROWS, MOE_64_ROWS, MOE_128_ROWS = 2.8, 56, 220
 MOE_LARGE, MOE_LARGE_64_ROWS = 1 << 25, 44
 # Widths that are no multiple of 128 have lists and the prefill tiles only (32 of 2880 x 2880: 3.5 rows 265 and 391)
 MOE_LIST_ROWS_ODD = 7
+# and so do experts that are small, or whose tiles are too few for the chip: the sort and what surrounds it is 12 us, tiles of 64 rows have a workgroup
+# per 128 columns and expert (weights that no cache holds: 8 of 2048 x 2048 3 to 7 rows 43 to 47 on lists, 51 on tiles, 4 of 4096 x 2048 42 and 63, 64 of 512 x 704
+# 39 to 44 and 43; 4 of 4096 x 4096 76 to 83 and 86; 32 of 2048 x 704 60 to 71 and 58 to 61, 64 of 1024 x 704 65 to 75 and 64, 8 of 3072 x 2048
+# 64 to 69 and 63). In all weights (of the down projections) and in 128-column tiles of the smaller product
+MOE_SMALL, MOE_FEW_TILES = 45_000_000, 180
 MOE_LIST_MAX_SLOTS = 4096   # moe.hip kMaxSlots
 
 
@@ -437,13 +442,14 @@ def expert_rows_bound(slots: int, experts: int, bm: int) -> int:
     return pad_to(slots + min(experts, slots) * (bm - 1), bm)
 
 
-def expert_plan(slots: int, E: int, weights: int = 0, tiles: bool = True) -> int:
+def expert_plan(slots: int, E: int, weights: int = 0, tiles: bool = True, columns: int | None = None) -> int:
     """How bf16 expert GEMMs run, by the rows an expert gets on average: 0 = weights streamed
     against the rows of each expert's own list, no sorting (few rows), 64 / 128 = sorted rows in
     tiles of that many on the decode GEMM, 256 = the prefill tile kernel. ``weights``: of an expert's down projection;
-    ``tiles``: its width takes the decode GEMM's column tiles."""
+    ``tiles``: its width takes the decode GEMM's column tiles; ``columns``: of the smaller of an expert's two products."""
     rows = slots / E
-    if rows <= (MOE_LIST_ROWS if tiles else MOE_LIST_ROWS_ODD) and slots <= MOE_LIST_MAX_SLOTS:
+    lists = columns is not None and (E * weights < MOE_SMALL or E * columns < 128 * MOE_FEW_TILES)
+    if rows <= (MOE_LIST_ROWS if tiles and not lists else MOE_LIST_ROWS_ODD) and slots <= MOE_LIST_MAX_SLOTS:
         return 0
     if not tiles or rows > MOE_128_ROWS:
         return 256
@@ -463,7 +469,7 @@ def experts(h: torch.Tensor, ids: torch.Tensor, wt: torch.Tensor, wgu: torch.Ten
         return reference.experts(h, ids, wt, wgu, wd), None
     C, dev = kernels(), h.device
     bf16 = h.dtype == torch.bfloat16
-    bm = (expert_plan(slots, E, ld * ff, ld % 128 == 0) if plan is None else plan) if bf16 else 64
+    bm = (expert_plan(slots, E, ld * ff, ld % 128 == 0, min(ld, 2 * ff)) if plan is None else plan) if bf16 else 64
     if bm in (64, 128) and bf16 and ld % 128:
         bm = 256   # the decode GEMM's column tiles
     if bm == 0:
