@@ -511,8 +511,18 @@ def rows_plan(M: int, N: int, K: int, glu: bool = False) -> tuple[int, int] | No
     One slice where the rows of X fit in registers. One workgroup per CU for most products (4096 x 14336 19.4 us, 20.6 on two per CU, 22.1 on
     four), three or four, whichever comes out more even, for those that take 30 us (28672 x 4096 gated 37.1 on one, 36.2 on four); rows of
     up to 2048 columns in one pass of eight rows a workgroup (32000 x 2048 22.3 on one per CU, 20.4 so), but not on one and a half per CU (3072 x
-    2048: 384 workgroups 4.6, 192 of sixteen rows 4.4)."""
+    2048: 384 workgroups 4.6, 192 of sixteen rows 4.4).
+
+    Five rows and more keep the vector units busy a whole piece of 2048 columns (512 a wave) at a time, so that short rows that leave one part empty are no
+    longer bound by the stream (weights that no cache holds, 8 rows): vocabularies of 128256 x 1536 96 us and 72 on gemm_mid, x 2304 129 and 101,
+    61440 x 2560 63 and 57, but 34432 x 2560 40 and 44, 128256 x 2048 102 and 112, x 3072 137 and 135; and where gemm_skinny's tiles come in whole
+    rounds, 16384 x 1536 15.5 and 14.1, x 2304 21.5 and 19.4, x 1792 15.9 and 16.5, x 2560 22.0 and 23.6, 20480 x 2304 25.5 and 25.6 (gated 5 rows of
+    98304 x 1536 73.7 and 67.8)."""
     if M > ROWS_MAX_M or K % 128 or K < 1536 or N % (128 if glu else 16) or N * K < (2.5e6 if M <= 4 else 8.5e6):
+        return None
+    if M > 4 and not glu and K < 2816 and K % 2048 and (K <= 2304 or N >= 48 << 10) and _mid_beats_skinny(M, N, K, False):
+        return None
+    if M > 4 and (K <= 1664 or 2048 < K < 2560) and (N % 8192 == 0 or (glu and K <= 1664 and N > LM_HEAD_MIN_N)):
         return None
     mt = 1 << (M - 1).bit_length()
     pieces = lambda s: -(-K // (2048 * s))  # noqa: E731 -- 512 columns a wave and piece

@@ -121,3 +121,13 @@ def test_rule():
                 assert (-(-(N // 2 if glu else N) // B) * (2 if glu else 1) + 8) * mt * 64 <= 48 << 10
     assert ops.rows_plan(9, 4096, 4096) is None and ops.rows_plan(1, 2048, 1024) is None and ops.rows_plan(1, 1072, 2048) is None
     assert ops.rows_plan(5, 2048, 2048) is None and ops.rows_plan(4, 2048, 2048) == (1, 256)
+
+
+def test_short_rows_of_five_and_more_stay_where_they_are_faster():
+    """Both sides' times stand at the rule."""
+    for M in (5, 8):
+        for N, K in ((128256, 1536), (51072, 1536), (152064, 1792), (61440, 2304), (61440, 2560), (16384, 1536), (8192, 2304)):
+            assert ops.rows_plan(M, N, K) is None and ops.rows_plan(4, N, K) is not None
+        for N, K in ((34432, 2560), (128256, 2048), (128256, 3072), (6144, 1536), (16384, 1792), (20480, 2304), (16384, 2560)):
+            assert ops.rows_plan(M, N, K) is not None
+        assert ops.rows_plan(M, 98304, 1536, True) is None and ops.rows_plan(M, 20480, 1536, True) is not None
