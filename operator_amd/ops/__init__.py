@@ -181,7 +181,7 @@ def gate_up_silu(x: torch.Tensor, wgu: torch.Tensor, block: int | None, act: int
             and K % 128 == 0 and x.is_contiguous() and wgu.is_contiguous()
             and skinny_plan(M, N, K) is not None and _gemm_table_get().get(("silu", M, N, K)) != "blas"):
         y = torch.empty(M, N // 2, dtype=x.dtype, device=x.device)
-        plan = _rows_plan(M, N, K, True)
+        plan = rows_plan(M, N, K, True)
         if plan is None:
             kernels().gemm_skinny(x, wgu, y, None, 1, act)
         else:
@@ -541,23 +541,17 @@ def rows_plan(M: int, N: int, K: int, glu: bool = False) -> tuple[int, int] | No
     return S, B
 
 
-def _rows_plan(M: int, N: int, K: int, glu: bool) -> tuple[int, int] | None:
-    """rows_plan, but for products that a measured "blas" or OAMD_SKINNY=0 sends to hipBLASLt. Measured slice counts are gemm_skinny's: of a product
-    that goes to gemm_rows they only decide, as ever, whether it stays in fp32 for its consumer (more than one slice) or is rounded to bf16."""
-    if M > ROWS_MAX_M or skinny_plan(M, N, K) is None or (_gemm_table_get().get(("silu", M, N, K)) == "blas" if glu else _measured_blas(M, N, K)):
-        return None
-    return rows_plan(M, N, K, glu)
-
-
 def _norm_blocks(M: int, N: int, K: int, glu: bool) -> int | None:
     """Workgroups of a product of gemm_rows that normalises its rows itself, or None where rmsnorm in front of it is faster. Every workgroup does it
     again, so many small ones are for a row or two only (us with rmsnorm and without: 28672 x 4096 gated of one row on 1024 41.0 and 38.2, of four 40.5
     and 40.7), none at all for short rows (16384 x 2048 gated, one row: 2048 workgroups 15.0 and 16.4, 256 14.3; 151936 x 1536 on 1024 71.8 and
     73.0), one per CU for up to four rows (6144 x 4096: 13.4 and 10.7, four rows 14.1 and 13.1). Eight pieces of rows (a power of
     two) and 512 columns are what a wave's registers hold."""
-    plan = _rows_plan(M, N, K, glu)
-    if plan is None or plan[0] != 1 or M > 4 or (1 << (M - 1).bit_length()) * -(-K // 2048) > 8:
+    plan = rows_plan(M, N, K, glu) if M <= 4 else None
+    if plan is None or plan[0] != 1 or (1 << (M - 1).bit_length()) * -(-K // 2048) > 8:
         return None
+    if skinny_plan(M, N, K) is None or (_gemm_table_get().get(("silu", M, N, K)) == "blas" if glu else _measured_blas(M, N, K)):
+        return None   # hipBLASLt's, by OAMD_SKINNY=0 or a measured entry
     B = plan[1] if plan[1] <= 4 * CUS else CUS
     return None if (B < plan[1] and N * K >= 5e7) or (M > 2 and plan[1] > CUS) or (-(-(N // 2 if glu else N) // B) * (2 if glu else 1) + 8) * (1 << (M - 1).bit_length()) * 64 > 48 << 10 else B
 
