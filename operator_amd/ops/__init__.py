@@ -839,10 +839,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, sp
     N = w.shape[0]
     plan = None
     if isinstance(x, Normed):
-        deferred = defer_reduce and skinny_plan(M, N, K) > 1
-        y = torch.empty(M, N, dtype=torch.float32 if deferred else w.dtype, device=w.device)
-        x.into(w, *((None, y) if deferred else (y, None)))
-        return SplitK(y, 1, M, N) if deferred else y
+        y = torch.empty(M, N, dtype=torch.float32 if defer_reduce else w.dtype, device=w.device)
+        x.into(w, *((None, y) if defer_reduce else (y, None)))
+        return SplitK(y, 1, M, N) if defer_reduce else y
     if x.is_cuda and bias is None and out is None and f32_ok(x, w):
         return linear_f32(x, w, prompt=prompt)
     if bias is not None:
@@ -858,7 +857,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, sp
         S = splits or skinny_plan(M, N, K)
         rows = rows_plan(M, N, K) if splits is None and S is not None and (out is None or out.is_contiguous()) else None
         if rows is not None:
-            deferred = defer_reduce and out is None and max(S, rows[0]) > 1
+            deferred = defer_reduce and out is None   # in fp32, of one slice too
             S = rows[0]
             p = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if deferred or S > 1 else None
             y = None if deferred else out if out is not None else torch.empty(M, N, dtype=x.dtype, device=x.device)
