@@ -483,8 +483,8 @@ SKINNY_MAX_M = 32
 
 
 def skinny_plan(M: int, N: int, K: int) -> int | None:
-    """Split-K count for the gfx950 gemm_skinny kernel (M <= 32 decode buckets), or None
-    for hipBLASLt: tuned table entry ``skinny,M,N,K`` if present, else split K until
+    """Split-K count for the gfx950 gemm_skinny kernel (M <= 32 decode buckets; products that rows_plan takes have its slices), or
+    None for hipBLASLt: tuned table entry ``skinny,M,N,K`` if present, else split K until
     the 16-row tiles give >= 512 blocks (K permitting)."""
     if M > SKINNY_MAX_M or N % 16 or K % 128 or os.environ.get("OAMD_SKINNY", "1") == "0":
         return None

@@ -127,3 +127,9 @@ def test_short_rows_of_five_and_more_stay_where_they_are_faster():
         for N, K in ((34432, 2560), (128256, 2048), (128256, 3072), (6144, 1536), (16384, 1792), (20480, 2304), (16384, 2560)):
             assert ops.rows_plan(M, N, K) is not None
         assert ops.rows_plan(M, 98304, 1536, True) is None and ops.rows_plan(M, 20480, 1536, True) is not None
+
+
+def test_measured_slices_are_of_products_that_other_kernels_run():
+    for k in ops._gemm_table_get():
+        if k[0] in ("skinny", "silu"):
+            assert ops.rows_plan(*k[1:], k[0] == "silu") is None, k
