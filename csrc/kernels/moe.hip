@@ -308,7 +308,7 @@ int moe_gather(const void* h, const int* src, const int* gtab, int bm, int max_r
 // Expert GEMM for few rows per expert: the structure of gemm_skinny.hip (W straight to VGPRs as
 // the MFMA A fragment, 4 waves split K, partial tiles summed through LDS) with the expert in
 // blockIdx.y. A workgroup lists the slots routed to its expert, then walks them 16 at a
-// time (the sorted tiles of gemm.hip are faster from three rows an expert); an expert nobody chose costs one read of the id list. NT = 2: the SwiGLU pair (16 gate
+// time (sorted tiles take over from three rows an expert, seven where they are small or few); an expert nobody chose costs one read of the id list. NT = 2: the SwiGLU pair (16 gate
 // rows and the 16 matching up rows of the 64-row interleave).
 constexpr int kMaxSlots = 4096;
 
