@@ -502,6 +502,22 @@ def skinny_plan(M: int, N: int, K: int) -> int | None:
 ROWS_MAX_M = 8
 
 
+def _skinny_rounds_full(N: int, K: int, glu: bool) -> bool:
+    """Where gemm_skinny is faster than gemm_rows for five to eight short rows: in one slice, and its last round of 8192 rows of W is full or nearly
+    (8 rows on gemm_rows and on gemm_skinny, us: 16384 x 1536 15.5 and 14.1, 14464 x 1536 14.5 and 13.4, 14336 12.9 and 13.2, 24448 21.2 and 19.9; 7168 x
+    1536 gated 8.3 and 8.1, in two slices of gemm_skinny 8.1 and 10.1; 16256 x 2304 21.1 and 19.4, 14464 19.5 and 18.9, 20480 25.5 and 25.6; 16256 x 2176
+    gated 22.0 and 18.9; 8192 x 2048 9.5 and 9.2, 16256 15.6 and 15.9; 16384 x 1792 15.9 and 16.5, x 2560 22.0 and 23.6. At 1664 columns it is one of 5 and 6 gated
+    rows, 16256 5 %; at 2432 one of 8064 and 16256 rows of W, 6 %, not of 14464 and 24448. Gated 5 rows of 98304 x 1536 73.7 and 67.8)."""
+    lacks = -N % 8192
+    if not (glu or N >= 8192 or K % 256):   # gemm_skinny in slices
+        return False
+    if K <= 1536 or 2048 < K < 2432 or (K == 2048 and N <= 8192) or (K == 1664 and glu and N > 8192):
+        full = lacks < 2048
+    else:
+        full = (K == 1664 or 2048 < K < 2560) and lacks < (256 if K > 2048 and N <= 16384 else 1)
+    return full or (glu and K <= 1664 and N > LM_HEAD_MIN_N)
+
+
 @functools.lru_cache(maxsize=4096)
 def rows_plan(M: int, N: int, K: int, glu: bool = False) -> tuple[int, int] | None:
     """(K slices, workgroups) of one to eight rows on the row-streaming kernel (gemm_rows.hip), or None for gemm_skinny: shorter rows, which
@@ -515,14 +531,13 @@ def rows_plan(M: int, N: int, K: int, glu: bool = False) -> tuple[int, int] | No
 
     Five rows and more keep the vector units busy a whole piece of 2048 columns (512 a wave) at a time, so that short rows that leave one part empty are no
     longer bound by the stream (weights that no cache holds, 8 rows): vocabularies of 128256 x 1536 96 us and 72 on gemm_mid, x 2304 129 and 101,
-    61440 x 2560 63 and 57, but 34432 x 2560 40 and 44, 128256 x 2048 102 and 112, x 3072 137 and 135; and where gemm_skinny's tiles come in whole
-    rounds, 16384 x 1536 15.5 and 14.1, x 2304 21.5 and 19.4, x 1792 15.9 and 16.5, x 2560 22.0 and 23.6, 20480 x 2304 25.5 and 25.6 (gated 5 rows of
-    98304 x 1536 73.7 and 67.8)."""
+    61440 x 2560 63 and 57, but 34432 x 2560 40 and 44, 128256 x 2048 102 and 112, x 3072 137 and 135; and where gemm_skinny's tiles come in full
+    rounds (_skinny_rounds_full)."""
     if M > ROWS_MAX_M or K % 128 or K < 1536 or N % (128 if glu else 16) or N * K < (2.5e6 if M <= 4 else 8.5e6):
         return None
     if M > 4 and not glu and K < 2816 and K % 2048 and (K <= 2304 or N >= 48 << 10) and _mid_beats_skinny(M, N, K, False):
         return None
-    if M > 4 and (K <= 1664 or 2048 < K < 2560) and (N % 8192 == 0 or (glu and K <= 1664 and N > LM_HEAD_MIN_N)):
+    if M > 4 and _skinny_rounds_full(N, K, glu):
         return None
     mt = 1 << (M - 1).bit_length()
     pieces = lambda s: -(-K // (2048 * s))  # noqa: E731 -- 512 columns a wave and piece

@@ -127,6 +127,10 @@ def test_short_rows_of_five_and_more_stay_where_they_are_faster():
         for N, K in ((34432, 2560), (128256, 2048), (128256, 3072), (6144, 1536), (16384, 1792), (20480, 2304), (16384, 2560)):
             assert ops.rows_plan(M, N, K) is not None
         assert ops.rows_plan(M, 98304, 1536, True) is None and ops.rows_plan(M, 20480, 1536, True) is not None
+        for N, K in ((14464, 1536), (16256, 1536), (24448, 1536), (16256, 2304), (14464, 2176), (8064, 2176), (8192, 2048), (16256, 2432)):
+            assert ops.rows_plan(M, N, K) is None and ops.rows_plan(M, N, K, True) is None and ops.rows_plan(4, N, K) is not None
+        for N, K in ((7168, 1536), (14336, 1536), (8064, 2304), (16256, 2048), (14464, 2432), (24448, 2432), (16256, 1664)):   # two slices, a last round less full
+            assert ops.rows_plan(M, N, K) is not None
 
 
 def test_measured_slices_are_of_products_that_other_kernels_run():
