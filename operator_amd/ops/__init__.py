@@ -518,6 +518,15 @@ def _skinny_rounds_full(N: int, K: int, glu: bool) -> bool:
     return full or (glu and K <= 1664 and N > LM_HEAD_MIN_N)
 
 
+def _rows_in_step(N: int, K: int, B: int, glu: bool) -> bool:
+    """Whether gemm_rows' workgroups start at rows of W that are served from the same memory channels: 512 KiB or 1 MiB apart but for a 128th (of gate | up
+    a 64th). One row on 256 workgroups and on 768, us: 16256 x 4096 (63.5 rows, 508 KiB) 31.0 and 23.4, 16512 31.9 and 23.5, 16384 21.9 and 23.2, 16224 24.8 and 23.1; 8128 x
+    8192 (508) 31.5 and 23.0, 11008 x 6144 (516) 31.5 and 22.4, 18864 x 3584 (516) 31.6 and 23.0; 9440 x 14336 (1032) 54.8 and 43.6; gated 16128 x 8192 (1008) 63.3
+    and 42.4, 16640 x 4096 (520) 26.4 and 23.5."""
+    apart = 2 * K * N / (B << 19)
+    return any(abs(abs(apart / m - 1) - (2 if glu else 1) / 128) < 0.35 / 128 for m in (1, 2))
+
+
 @functools.lru_cache(maxsize=4096)
 def rows_plan(M: int, N: int, K: int, glu: bool = False) -> tuple[int, int] | None:
     """(K slices, workgroups) of one to eight rows on the row-streaming kernel (gemm_rows.hip), or None for gemm_skinny: shorter rows, which
@@ -547,10 +556,9 @@ def rows_plan(M: int, N: int, K: int, glu: bool = False) -> tuple[int, int] | No
     units = N // 2 if glu else N
     if pieces(S) == 1:
         B = N // 8 if N // 8 <= CUS or N // 8 >= 2 * CUS else N // 16
-    elif N * K < 9e7 or units < 48 * CUS:
-        B = CUS
     else:
-        B = -min((-(-units // b) * b, -b) for b in (3 * CUS, 4 * CUS))[1]
+        counts = (CUS, 3 * CUS) if N * K < 9e7 or units < 48 * CUS else sorted((3 * CUS, 4 * CUS), key=lambda b: (-(-units // b) * b, -b))
+        B = next((b for b in counts if not _rows_in_step(N, K, b, glu)), counts[0])
     while (-(-units // B) * (2 if glu else 1) + 8) * mt * 64 > 48 << 10:   # the workgroup's sums in LDS
         B *= 2
     return S, B

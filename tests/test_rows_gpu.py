@@ -133,6 +133,15 @@ def test_short_rows_of_five_and_more_stay_where_they_are_faster():
             assert ops.rows_plan(M, N, K) is not None
 
 
+def test_workgroups_do_not_start_in_step():
+    """Rows of W 508, 516, 1016 or 1032 KiB apart (gate | up 504, 520, 1008, 1040) have more and smaller workgroups."""
+    for N, K, glu in ((16256, 4096, False), (16512, 4096, False), (8128, 8192, False), (11008, 6144, False), (18864, 3584, False), (9440, 14336, False),
+                      (16128, 4096, True), (16640, 4096, True), (16128, 8192, True)):
+        assert ops.rows_plan(1, N, K, glu) == (1, 768)
+    for N, K, glu in ((16384, 4096, False), (16128, 4096, False), (4096, 4096, False), (4096, 14336, False), (16384, 4096, True), (16256, 4096, True)):
+        assert ops.rows_plan(1, N, K, glu) == (1, 256)
+
+
 def test_measured_slices_are_of_products_that_other_kernels_run():
     for k in ops._gemm_table_get():
         if k[0] in ("skinny", "silu"):
