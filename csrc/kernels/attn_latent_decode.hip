@@ -7,7 +7,8 @@
 // chunks dealt out over the whole tile cost a division, a lookup and an address each, and registers that some sizes spilled.
 // 48 sequences of 3600 rows, combine included: 16 heads on 320 columns 48 -> 39 us, on 384 117 -> 49, 32 heads on 576 75 -> 72
 // (2.8 TB/s: a tile's phases, one after the other behind four barriers, are what bounds it; with the value blocks unbranched 69, 16 heads on 320
-// columns 37, on 384 46). Two tiles in LDS, two barriers a tile, gain nothing: a launch of 240 workgroups of twelve tiles starts and ends
+// columns 37, on 384 46; 360 sizes take 0.98 of their time, but rows that are mostly rotated part 2 to 8 % more, as their blocks are multiplied too: 16 heads on
+// 32 + 224 columns 23.9 -> 25.3). Two tiles in LDS, two barriers a tile, gain nothing: a launch of 240 workgroups of twelve tiles starts and ends
 // in 12 us, and a tile takes 3 us with every CU busy (6.2 TB/s).
 //
 //   S = K Q^T     v_mfma_f32_16x16x32_bf16, A = rows (tokens x dims), B = q (one head per column);
