@@ -335,14 +335,17 @@ void gemm_tile(const at::Tensor& x, const at::Tensor& w, const c10::optional<at:
 
 void gemm_mid(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& y_opt,
               const c10::optional<at::Tensor>& bias, const c10::optional<at::Tensor>& partial, int64_t splits, int64_t silu_gu,
-              int64_t rows) {
+              int64_t rows, int64_t cols) {
   CHECK_DEV(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_CONTIG(x); CHECK_CONTIG(w);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && w.size(1) == x.size(1), "gemm_mid: x [M, K], w [N, K]");
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
   TORCH_CHECK(M >= 1 && N >= 16 && N % 16 == 0 && K % 64 == 0, "gemm_mid: N % 16 == 0, K % 64 == 0");
   TORCH_CHECK(M < (1LL << 24) && N < (1LL << 30) && K < (1LL << 22), "gemm too large");
   TORCH_CHECK(splits >= 1 && splits <= 16 && K / 64 >= splits, "gemm_mid: bad split count");
-  TORCH_CHECK(rows == 96 || rows == 128 || rows == 160, "gemm_mid: tiles of 96, 128 or 160 rows");
+  TORCH_CHECK(((rows == 96 || rows == 160) && (cols == 128 || cols == 256)) ||
+                  ((rows == 64 || rows == 128) && (cols == 64 || cols == 128 || cols == 256)),
+              "gemm_mid: tiles of 64, 96, 128 or 160 rows and 128 or 256 columns, of 64 or 128 rows and 64 columns");
+  TORCH_CHECK(cols > 64 || splits > 1 || !silu_gu, "gemm_mid: a gated epilogue needs 128 columns of a tile");
   TORCH_CHECK(!silu_gu || (N % 128 == 0 && !bias.has_value()), "gemm_mid: a gated epilogue needs N % 128, no bias");
   bf16_t* yp = nullptr;
   int64_t ldy = silu_gu ? N / 2 : N;
@@ -371,7 +374,7 @@ void gemm_mid(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::
   }
   const c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
   RC(oamd::gemm_mid(ptr<bf16_t>(x), ptr<bf16_t>(w), yp, optr<bf16_t>(bias), pp, (int)M, (int)N, (int)K, (int)ldy, (int)silu_gu,
-                    (int)splits, (int)rows, cur_stream()));
+                    (int)splits, (int)rows, (int)cols, cur_stream()));
 }
 
 void gemm_pp(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& y_opt,
@@ -784,7 +787,7 @@ PYBIND11_MODULE(_C, m) {
         pybind11::arg("stages") = 3);
   m.def("gemm_mid", &gemm_mid, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("y"), pybind11::arg("bias") = pybind11::none(),
         pybind11::arg("partial") = pybind11::none(), pybind11::arg("splits") = 1, pybind11::arg("silu_gu") = 0,
-        pybind11::arg("rows") = 128);
+        pybind11::arg("rows") = 128, pybind11::arg("cols") = 256);
   m.def("gemm_tile", &gemm_tile, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("y"),
         pybind11::arg("bias") = pybind11::none(), pybind11::arg("silu_gu") = 0, pybind11::arg("variant") = 0,
         pybind11::arg("splits") = 1, pybind11::arg("partial") = pybind11::none(), pybind11::arg("rows") = 256);

@@ -2,13 +2,16 @@
 // projections of one or a few prompts, and vocabularies of up to 128 rows.
 //
 // What bounds it: not the matrix cores but the CUs a launch keeps busy. The 256 x 256 tiles of gemm_tile make 64
-// workgroups of an 885 x 4096 product, each walking the whole K at 1.2 us per 64 columns. Here a tile is 96, 128 or 160 rows
-// (ops.tile_rows) by 256 columns and its K may be cut into S slices (fp32 slabs, summed by the consumer or by a reduce pass),
+// workgroups of an 885 x 4096 product, each walking the whole K at 1.2 us per 64 columns. Here a tile is 64 to 160 rows by
+// 64, 128 or 256 columns (ops.tile_rows, ops.prompt_tile) and its K may be cut into S slices (fp32 slabs, summed by the consumer or by a reduce pass),
 // so that the workgroups come close to one per CU or to whole rounds of them:
 //   885 rows (weights from HBM)   6144 x 4096, 96-row tiles: 49 us (128-row tiles 55); 4096 x 4096 in 2 slices 35; 4096 x 14336 in 2
 //                                 101 (297 on the 256-row tiles)
 //   300 rows                      28672 x 4096, 160-row tiles: 68 us (128 rows 110, 256 rows 95)
 //   1500 rows                     6144 x 4096, 160-row tiles: 62 us (128 rows 93, 256 rows 90)
+//   100 rows                      6144 x 4096 in 2 slices, 192 tiles of 128 x 64: 18 us (48 of 128 x 256 31); 4096 x 14336 in 4, 256 of
+//                                 128 x 64: 29 (55); 28672 x 4096 gated, 224 of 128 x 128: 56 (65)
+//   200 rows                      4096 x 14336 in 4 slices, 160 x 128 tiles: 37 us (96 x 256 48)
 //   vocabulary 128256 x 8192, 64 rows: 373 us (5.6 TB/s of weights; the 256-row tiles 422)
 // The first slice carries a bias (4608 x 3584, 300 rows: 54 us in one slice, 22 in 3).
 // A 128 x 256 step takes 0.63 us alone, 0.79 with every CU busy (clock). Its MFMAs are 0.47, its LDS-DMA pieces by themselves 0.45 (a CU's
@@ -16,8 +19,9 @@
 // the pieces are spread over the whole step: within the 24 MFMAs behind the barrier, as before, 885 rows of 6144 x 4096 took 60 us
 // and not 55, of 4096 x 4096 38 and not 35. A 64-row tile's step is no shorter than a 96-row one's (0.61, 0.65: the weight pieces).
 //
-// Why this shape: four waves, one per SIMD, 16 MI x 128 outputs each in AGPRs, so a step's fragment reads stay below its
-// MFMA time; three stages (44, 48 or 52 KiB) leave one to two steps in flight behind one barrier per step. 128-B rows with the
+// Why this shape: four waves, one per SIMD, 16 MI x 16 NW outputs each in AGPRs, so a step's fragment reads of the wide tiles stay below its
+// MFMA time; three stages of those (44, 48 or 52 KiB) leave one to two steps in flight behind one barrier per step, up to six of the narrow ones as
+// many bytes of the weights, which bound them. 128-B rows with the
 // chunk swizzle slot ^ (bit1(row) << 1 | bit3(row) << 2) read without bank conflicts; W fragments take interleaved feature
 // rows, so a lane ends with 8 neighbouring features: 16-B stores. A workgroup walks its units (tile, slice) in one
 // continuous LDS-DMA stream: the next unit's first stages load while this one's outputs are stored.
@@ -28,7 +32,6 @@ namespace oamd {
 
 namespace {
 
-constexpr int kBN = 256;     // tile columns
 constexpr int kBK = 64;      // K per step: one 128-B line per row
 
 enum { kEpiStore = 0, kEpiBias = 1, kEpiGlu = 2, kEpiPartial = 3 };   // partial: fp32 slab [M][N] of a K slice
@@ -66,15 +69,17 @@ __device__ __forceinline__ void store8(bf16_t* y, const f32x4& v0, const f32x4& 
 
 }  // namespace
 
-// MI: 32-row blocks of a tile
-template <int MI, int EPI>
+// MI: 32-row blocks of a tile, NW: its 32-column blocks
+template <int MI, int NW, int EPI>
 __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                        bf16_t* __restrict__ Y, const bf16_t* __restrict__ bias,
                                                        float* __restrict__ P, int M, int N, int K, int ldy, int S, GluAct act) {
   constexpr int AUX = 16;
   constexpr int kBM = 32 * MI;                   // a wave has MI X fragments and as many X pieces per step
-  constexpr int NP = MI + 8;                     // LDS-DMA pieces of a wave per step
-  constexpr int NS = 3;                          // stages: 132, 144 or 156 KiB
+  constexpr int kBN = 32 * NW;                   // ... and NW W fragments and pieces
+  constexpr int NP = MI + NW;                    // LDS-DMA pieces of a wave per step
+  constexpr int NS = 40 / NP < 6 ? 40 / NP : 6;  // stages of 4 NP KiB within 160
+  constexpr int kAhead = (NS - 2) * NP;          // pieces in flight behind a step's own
   constexpr int kGroupM = 32 / MI;               // row tiles that share a W panel before the next one
   constexpr int kX = kBM * 128, kStage = kX + kBN * 128;
   __shared__ __attribute__((aligned(1024))) char lds[NS * kStage];
@@ -88,9 +93,10 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
 
   auto swz = [](int row) { return (((row >> 1) & 1) << 1) | (((row >> 3) & 1) << 2); };
   const int lrow = lane >> 3, lslot = lane & 7;
-  uint32_t vo[8];
+  constexpr int NV = MI > NW ? MI : NW;
+  uint32_t vo[NV];
 #pragma unroll
-  for (int q = 0; q < 8; ++q) {
+  for (int q = 0; q < NV; ++q) {
     const int row = 8 * (w + 4 * q) + lrow;
     vo[q] = ((uint32_t)row * (uint32_t)K + (uint32_t)((lslot ^ swz(row)) * 8)) * 2u;
   }
@@ -140,21 +146,21 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
   const int xo[2] = {xb0 + ((lq ^ xs) << 4), xb0 + (((4 + lq) ^ xs) << 4)};
   const int wo[2] = {wb0 + ((lq ^ ws) << 4), wb0 + (((4 + lq) ^ ws) << 4)};
   // read f of a k-half: the X fragments, then the W ones (j = f-block * 4 + gate|up half * 2 + jj)
-  auto rd = [&](int off, int h, u16x8 (&xf)[MI], u16x8 (&wf)[8], int f) {
+  auto rd = [&](int off, int h, u16x8 (&xf)[MI], u16x8 (&wf)[NW], int f) {
     if (f < MI) {
       xf[f] = *reinterpret_cast<const u16x8*>(lds + off + xo[h] + f * 2048);
-    } else if (f < MI + 8) {
+    } else {
       const int j = f - MI, r = (j >> 2) * 128 + ((j >> 1) & 1) * 64 + (j & 1) * 4;
       wf[j] = *reinterpret_cast<const u16x8*>(lds + off + wo[h] + r * 128);
     }
   };
 
-  f32x4 acc[MI][8];
+  f32x4 acc[MI][NW];
   auto clear = [&]() {
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
+      for (int j = 0; j < NW; ++j) {
         acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         asm volatile("" : "+a"(acc[i][j]));
       }
@@ -165,7 +171,7 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
   // A barrier inside every step (after kBar of k-half 1's kH MFMAs) says that the step's stage has been read and the
   // next one has landed. The NP pieces of the step NS ahead go into that stage, spread over the 2 kH MFMAs up to
   // the next barrier: piece p with MFMA number p * 2 kH / NP behind it.
-  constexpr int kH = 8 * MI, kBar = 2 * MI, kTail = kH - kBar;
+  constexpr int kH = NW * MI, kBar = kH / 4, kTail = kH - kBar;
   auto piece = [&](int z, int o) {
     const int p = (z * NP + 2 * kH - 1) / (2 * kH);
     if (p < NP && p * 2 * kH / NP == z) {
@@ -182,15 +188,16 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
   }
 #pragma unroll
   for (int z = 0; z < kTail; ++z) piece(z, (NS - 1) * kStage);   // of the last stage, what k-half 1 of a step before would issue
-  vm_wait<NP>();
+  vm_wait<kAhead>();
   __builtin_amdgcn_s_barrier();
-  u16x8 xa[MI], wa[8], xb[MI], wb[8];
+  u16x8 xa[MI], wa[NW], xb[MI], wb[NW];
 #pragma unroll
   for (int f = 0; f < NP; ++f) rd(0, 0, xa, wa, f);
 
   int off = 0, prev = (NS - 1) * kStage;   // this step's stage, the one before
-  bool relax = false;   // the next wait may leave a whole tile's stores in flight behind the pieces
-  constexpr int kStores = MI * (EPI == kEpiGlu ? 2 : EPI == kEpiPartial ? 8 : 4);
+  int relax = 0;   // so many waits may leave a whole tile's stores in flight behind the pieces
+  constexpr int kStores = MI * NW / (EPI == kEpiGlu ? 4 : EPI == kEpiPartial ? 1 : 2);
+  static_assert(kAhead + kStores < 64 && NP <= kH, "a wait's count, a read per MFMA");
   for (int u = slot; u < units; u += G) {
     int m0, n0, kz, t0, T;
     unit(u, m0, n0, kz, t0, T);
@@ -210,11 +217,11 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
       for (int v = 0; v < kH; ++v) {
         if (v == kBar) {
           asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-          if (relax) {
-            vm_wait<NP + kStores>();
-            relax = false;
+          if (relax > 0) {
+            vm_wait<kAhead + kStores>();
+            --relax;
           } else {
-            vm_wait<NP>();
+            vm_wait<kAhead>();
           }
           __builtin_amdgcn_sched_barrier(0);
           __builtin_amdgcn_s_barrier();
@@ -225,8 +232,10 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
         if (v < kBar) {
           piece(kTail + kH + v, prev);
         } else {
-          const int z = v - kBar, f = (z * NP + kTail - 1) / kTail;
-          if (f < NP && f * kTail / NP == z) rd(nxt, 0, xa, wa, f);
+          const int z = v - kBar;
+#pragma unroll
+          for (int f = 0; f < NP; ++f)
+            if (f * kTail / NP == z) rd(nxt, 0, xa, wa, f);
           piece(z, off);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -241,7 +250,7 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
     for (int i = 0; i < MI; ++i) {
       const int tok = m0 + wm * (kBM / 2) + i * 16 + l15;
 #pragma unroll
-      for (int f = 0; f < 2; ++f) {
+      for (int f = 0; f < (NW + 3) / 4; ++f) {
         if constexpr (EPI == kEpiGlu) {
           f32x4 o[2];
 #pragma unroll
@@ -250,7 +259,7 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
           if (tok < M && 2 * col < N) store8(Y + (int64_t)tok * ldy + col, o[0], o[1]);
         } else {
 #pragma unroll
-          for (int ty = 0; ty < 2; ++ty) {
+          for (int ty = 0; ty < (NW == 2 ? 1 : 2); ++ty) {
             f32x4 v0 = acc[i][f * 4 + ty * 2], v1 = acc[i][f * 4 + ty * 2 + 1];
             const int col = n0 + f * 128 + ty * 64 + wn * 32 + 8 * lq;
             if (tok >= M || col >= N) continue;
@@ -268,35 +277,46 @@ __global__ void __launch_bounds__(256) gemm_mid_kernel(const bf16_t* __restrict_
       }
     }
     // a whole tile issued kStores stores: the next waits count past them
-    relax = m0 + kBM <= M && n0 + kBN <= N;
+    relax = m0 + kBM <= M && n0 + kBN <= N ? NS - 2 : 0;
     clear();
   }
   vm_wait<0>();   // the trailing re-loads land before the workgroup's LDS is released
 }
 
-template <int MI>
+template <int MI, int NW>
 static void launch_mid(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, float* P, int M, int N, int K, int ldy,
                        int glu, int S, int grid, hipStream_t stream) {
-  if (S > 1) gemm_mid_kernel<MI, kEpiPartial><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, GluAct{});
-  else if (glu) gemm_mid_kernel<MI, kEpiGlu><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, glu_act(glu));
-  else if (bias) gemm_mid_kernel<MI, kEpiBias><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, GluAct{});
-  else gemm_mid_kernel<MI, kEpiStore><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, GluAct{});
+  if (S > 1) gemm_mid_kernel<MI, NW, kEpiPartial><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, GluAct{});
+  else if (bias) gemm_mid_kernel<MI, NW, kEpiBias><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, GluAct{});
+  else if (!glu) gemm_mid_kernel<MI, NW, kEpiStore><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, GluAct{});
+  else if constexpr (NW >= 4) gemm_mid_kernel<MI, NW, kEpiGlu><<<grid, 256, 0, stream>>>(X, W, Y, bias, P, M, N, K, ldy, S, glu_act(glu));
 }
 
 int gemm_mid(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, float* P, int M, int N, int K, int ldy, int glu,
-             int S, int rows, hipStream_t stream) {
+             int S, int rows, int cols, hipStream_t stream) {
   if (M < 1 || N < 16 || N % 16 || K % kBK || S < 1 || S > 16 || K / kBK < S) return -1;
   if (glu && (N % 128 || bias)) return -2;
   if (S > 1 && P == nullptr) return -3;
   if (Y == nullptr ? (S == 1 || glu) : (ldy % 8 || reinterpret_cast<uintptr_t>(Y) % 16)) return -4;
   if (S > 1 && Y != nullptr && ldy != (glu ? N / 2 : N)) return -5;
-  if (rows != 96 && rows != 128 && rows != 160) return -7;
-  const int64_t units = (int64_t)((M + rows - 1) / rows) * ((N + kBN - 1) / kBN) * S;
+  const int64_t units = (int64_t)((M + rows - 1) / rows) * ((N + cols - 1) / cols) * S;
   if (units > (1LL << 30)) return -6;
+  if (cols == 64 && glu && S == 1) return -7;
   const int grid = (int)min((int64_t)device_cus(), units);
-  if (rows == 96) launch_mid<3>(X, W, Y, bias, P, M, N, K, ldy, glu, S, grid, stream);
-  else if (rows == 128) launch_mid<4>(X, W, Y, bias, P, M, N, K, ldy, glu, S, grid, stream);
-  else launch_mid<5>(X, W, Y, bias, P, M, N, K, ldy, glu, S, grid, stream);
+#define OAMD_MID(R, C) \
+  if (rows == R && cols == C) launch_mid<R / 32, C / 32>(X, W, Y, bias, P, M, N, K, ldy, glu, S, grid, stream)
+  OAMD_MID(96, 256);
+  else OAMD_MID(128, 256);
+  else OAMD_MID(160, 256);
+  else OAMD_MID(64, 256);
+  else OAMD_MID(64, 128);
+  else OAMD_MID(96, 128);
+  else OAMD_MID(128, 128);
+  else OAMD_MID(160, 128);
+  else OAMD_MID(64, 64);
+  else OAMD_MID(128, 64);
+  else return -8;
+#undef OAMD_MID
   OAMD_LAUNCH_CHECK();
   if (S == 1 || Y == nullptr) return 0;
   return glu ? splitk_silu(P, Y, M, N, S, glu, stream) : splitk_reduce(P, Y, (int64_t)M * N, S, stream);

@@ -47,10 +47,10 @@ int gemm_decode(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, in
 int gemm_tile(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, int M, int N, int K, int ldy,
               int glu, int variant, int S, float* P, int rows, hipStream_t stream);   // rows: 256, or 192 / 224 (one slice, 16-B aligned Y, ldy % 8 == 0)
 int device_cus();   // compute units of the current device (persistent grids)
-// The same product for few rows on tiles of `rows` (96, 128 or 160) x 256 (gemm_mid.hip), Y 16-B aligned, ldy % 8 == 0, K cut into S <= 16
+// The same product for few rows on tiles of `rows` (64, 96, 128 or 160) x `cols` (256, 128, of 64 or 128 rows also 64) (gemm_mid.hip), Y 16-B aligned, ldy % 8 == 0, K cut into S <= 16
 // slices: fp32 slabs P[S][M][N], then one reduce pass (ldy = the row's length) unless Y == nullptr. A bias is in the first slab.
 int gemm_mid(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, float* P, int M, int N, int K, int ldy, int glu,
-             int S, int rows, hipStream_t stream);
+             int S, int rows, int cols, hipStream_t stream);
 // Decode-bucket GEMM on the ping-pong schedule (gemm_pp.hip): Y[M,N] = X[M,K] W[N,K]^T, bm-row tiles
 // (128 / 256), 128-column tiles (N % 128 == 0), S-way split-K slabs P (S > 1; reduced into Y unless Y is
 // nullptr); glu: fused SwiGLU (S == 1), Y [M, N/2]; nt: non-temporal weight loads.

@@ -611,7 +611,7 @@ def _mid_few_rows(M: int, N: int, K: int, defer: bool) -> bool:
 
 
 # Every GPU GEMM of the model runs on the hand-written gfx950 kernels: prompts on gemm_mid or gemm_tile (csrc/kernels/gemm_tile.hip),
-# whichever has the tile rows that fit (tile_rows), in K slices (mid_plan) on gemm_mid, decode buckets on
+# whichever has the tiles that fit (tile_rows, prompt_tile), in K slices (mid_plan) on gemm_mid, decode buckets on
 # gemm_pp / gemm_tn / gemm_mid / gemm_skinny / gemm_rows, the lm_head on whichever of them its rows call for (_mid_beats_skinny,
 # _vocab_plan, mid_plan), fp8 on gemm_fp8 and, past 64 rows, gemm_fp8_tile, fp32 on gemm_f32 in one of its two forms (f32_split_slices). hipBLASLt is reached
 # only by shapes none of them takes (K % 64 != 0, N % 16 != 0, non-bf16), counted in BLAS_CALLS.
@@ -726,6 +726,40 @@ def tile_rows(M: int, N: int, K: int, S: int = 1) -> int:
     return min((_rows_us(r, M, N, K, S), r) for r in ((96, 128, 160) if S > 1 else _ROW_STEP))[1]
 
 
+# us of a prompt's tiles by (rows, columns): to start and to store, a 64-column piece of K on a CU, what it takes more with every CU busy, between
+# rounds. Fitted to 504 products of 25 shapes, 33 to 2000 rows, in their plans' slices, weights from HBM
+_MID_US = {(64, 64): (4.13, 0.186, 0.078, 0.4), (128, 64): (4.55, 0.221, 0.158, 1.2), (64, 128): (4.8, 0.376, 0.049, 0.4),
+           (96, 128): (5.64, 0.404, 0.048, 1.3), (128, 128): (5.64, 0.404, 0.175, 2.4), (160, 128): (7.22, 0.439, 0.111, 3.1),
+           (64, 256): (4.75, 0.684, 0.060, 1.4), (96, 256): (6.46, 0.679, 0.106, 2.0), (128, 256): (7.07, 0.697, 0.210, 2.3),
+           (160, 256): (9.97, 0.683, 0.211, 6.2), (192, 256): (10.32, 0.696, 0.317, 10.5), (224, 256): (11.09, 0.789, 0.363, 12.0),
+           (256, 256): (11.87, 0.899, 0.394, 12.0)}
+NARROW_MAX_M = 2048
+
+
+def _mid_us(rows: int, cols: int, M: int, N: int, K: int, S: int) -> float:
+    start, one, busy, between = _MID_US[rows, cols]
+    units = -(-M // rows) * -(-N // cols) * S
+    full, last = divmod(units, CUS)
+    rounds = full * (one + busy) + (one + busy * last / CUS if last else 0)
+    return start + -(-(K // 64) // S) * rounds + between * ((units - 1) // CUS)
+
+
+@functools.lru_cache(maxsize=4096)
+def prompt_tile(M: int, N: int, K: int, S: int = 1, glu: int = 0) -> tuple[int, int]:
+    """(rows, columns) of the tiles of a prompt's product in S slices of K: tile_rows' by 256 columns, or gemm_mid's of 64 or 128 columns
+    where those are estimated 7 % faster. Few rows in few slices leave most CUs without a tile of 256 columns (100 rows, us: 6144 x 4096 in two
+    slices 48 workgroups 31, 192 of 128 x 64 18; 4096 x 14336 in four 64 workgroups 55, 256 29; 28672 x 4096 gated 112 workgroups 65, 224 of 128 x 128
+    56; 40 rows of 16384 x 2048 gated 27 and, in 64 x 128 tiles, 20); 200 rows of 4096 x 14336 48 on 96 x 256, 37 on 160 x 128. The sums, and so the bits, are
+    the same for all. 333 of those 504 products take narrow tiles, 0.68 of the time of the others on average; none was slower. A gated product's
+    narrowest tile is the 128 rows of W that hold 64 gates and what they multiply."""
+    first = tile_rows(M, N, K, S), 256
+    if M > NARROW_MAX_M:
+        return first
+    us, tile = min((_mid_us(*t, M, N, K, S), t) for t in _MID_US
+                   if (t[1] < 256 or t[0] == 64) and (t[1] > 64 or not glu or S > 1))
+    return tile if us < 0.93 * _mid_us(*first, M, N, K, S) else first
+
+
 def loose_tiles(M: int, N: int, K: int) -> bool:
     """One row tile of a vocabulary whose rows are a power of two apart: gemm_tile's schedule of a workgroup per tile (h4), whose workgroups
     drift apart. In the persistent one all CUs walk their weight rows in step, and rows 8 or 16 KiB apart share memory channels:
@@ -738,19 +772,24 @@ def loose_tiles(M: int, N: int, K: int) -> bool:
 def linear_tile(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None,
                 bias: torch.Tensor | None = None, glu: int = 0, defer_reduce: bool = False, prompt: bool = False):
     """Prefill / lm_head GEMM on the compute-bound gfx950 tile kernels (fused bias or gated (``glu``: SILU /
-    GELU_TANH) epilogue): tiles of 96 to 256 rows (``tile_rows``), for few rows with K slices (``mid_plan``).
+    GELU_TANH) epilogue): tiles of 96 to 256 rows (``tile_rows``), of few rows of prompts also narrower ones (``prompt_tile``), for few rows with K
+    slices (``mid_plan``).
     ``defer_reduce``: K slices come back as fp32 slabs (:class:`SplitK`); ``prompt``: rows a prefill graph may pad."""
     M, K = x.shape
     N = w.shape[0]
     defer = defer_reduce and out is None and not glu
-    S, rows = None, 256
+    S, rows, cols = None, 256, 256
     if (out is None or (out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0)) and (
             bias is None or (bias.is_contiguous() and bias.data_ptr() % 16 == 0)):   # gemm_mid's 16-B accesses
         S = mid_plan(M, N, K, defer, out is None or out.stride(0) == out.shape[1], prompt)   # the reduce pass has no row stride
         if 128 <= K < 1 << 22 and M < 1 << 24 and N < 1 << 30:   # gemm_mid's
             rows = 256 if not glu and loose_tiles(M, N, K) else tile_rows(M, N, K, S or 1)
+            if prompt and (glu or N < LM_HEAD_MIN_N):
+                rows, cols = prompt_tile(M, N, K, S or 1, glu)
     part = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if S is not None and S > 1 else None
     opt = {} if rows == 128 else {"rows": rows}
+    if cols != 256:
+        opt["cols"] = cols
     if part is not None and defer:
         kernels().gemm_mid(x, w, None, bias, part, S, **opt)
         return SplitK(part, S, M, N)
