@@ -209,8 +209,11 @@ class _BucketState:
             else:
                 temp[:n] = np.fromiter((r.temperature for r in reqs), dtype=np.float32, count=n)
                 seeds[:n] = np.fromiter((r.seed for r in reqs), dtype=np.int64, count=n)
-            for i, r in enumerate(reqs):
-                bt[i, :len(r.pages)] = r.pages
+            if self._buf.is_cuda:
+                ops.kernels().page_rows(host, self._nbytes - bt.nbytes, bt.shape[1], [r.pages for r in reqs])
+            else:
+                for i, r in enumerate(reqs):
+                    bt[i, :len(r.pages)] = r.pages
         nb = self._buf.is_cuda
         self._buf.copy_(host.pin_memory() if nb else host, non_blocking=nb)   # step = 0
         self.step_host = 0
@@ -999,10 +1002,13 @@ class LLMEngine:
         stream (the call does not wait for them)."""
         self._after_given()
         out = torch.empty(len(reqs), self.model.cfg.vocab_size, dtype=torch.float32, device=self.device)
+        P = self.kv.page_size
         for r, t in zip(reqs, tokens):
             r.output.append(int(t))
-            self._reserve(r)
-        order = sorted(range(len(reqs)), key=lambda i: -reqs[i].length)
+            if not r.length <= min(len(r.pages) * P, self.max_context):
+                self._reserve(r)
+        lens = [r.length for r in reqs]
+        order = sorted(range(len(reqs)), key=lens.__getitem__, reverse=True)
         for a in range(0, len(order), self.max_batch):
             part = order[a:a + self.max_batch]
             rows = [reqs[i] for i in part]
