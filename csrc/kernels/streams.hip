@@ -25,11 +25,19 @@ __device__ __forceinline__ f32x4 ld4(const void* p, int64_t i, bool f32) {
   return f32x4{bf2f(v[0]), bf2f(v[1]), bf2f(v[2]), bf2f(v[3])};
 }
 
+__device__ __forceinline__ f32x4 f4(const u16x4& v) { return f32x4{bf2f(v[0]), bf2f(v[1]), bf2f(v[2]), bf2f(v[3])}; }
+
+constexpr int kTopRegs = 4;   // expert rows of a token that are requested together
+
 }  // namespace
 
 // One workgroup per row; thread t owns 4-feature vectors t, t + NT, ... (MAXV of them).
 // S: compile-time bound of the stream count a.S. POST: y is normalised first (post_w).
-template <int S, int NT, int MAXV, bool POST>
+// ASK: the output comes as bf16 rows (y, e), whose conversion waits for each load in turn; here up to four vectors' rows and streams are requested before any
+// of them is used, and the streams pass by the caches, which keep the experts' rows (7950 rows of 4 x 4096, two experts each, streams not written
+// back: 153 us -> 114, 4.7 -> 6.3 TB/s; written back 243 -> 229; one stream with post_w, 15000 rows of 4096 150 -> 133). Slabs and fp32
+// rows convert nothing and lose by the registers (900 fp32 rows of 4 x 2048 16 -> 19 us).
+template <int S, int NT, int MAXV, bool POST, bool ASK>
 __global__ void __launch_bounds__(NT) stream_step_kernel(const StreamStep a) {
   __shared__ float scratch[NT / 64];
   __shared__ float coef[S * S + 2 * S];   // mix[from][to], out, in
@@ -58,9 +66,40 @@ __global__ void __launch_bounds__(NT) stream_step_kernel(const StreamStep a) {
 
   const int nv = a.ld >> 2;
   float* xr = a.x + row * (int64_t)a.S * a.ld;
-  auto output = [&](int v) {   // 4 features of the sublayer's output
+  constexpr int U = !ASK ? 1 : S > 4 ? 2 : MAXV < 4 ? MAXV : 4;   // vectors of a group
+  static_assert(MAXV % U == 0, "whole groups");
+  u16x4 yq[U], eq[U][kTopRegs];
+  f32x4 xq[U][S];
+  [[maybe_unused]] int64_t er[kTopRegs];
+  if constexpr (ASK) {
+#pragma unroll
+    for (int k = 0; k < kTopRegs; ++k)
+      if (k < a.top) er[k] = (a.epos ? (int64_t)a.epos[row * a.top + k] : row * a.top + k) * a.ld;
+  }
+  // requests vectors i0 .. i0 + U - 1: the output's rows (out), the streams (streams)
+  auto ask = [&](int i0, bool out, bool streams) {
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const int v = tid + (i0 + j) * NT;
+      if (v >= nv) continue;
+      if (out) {
+        if (a.y) yq[j] = *reinterpret_cast<const u16x4*>(static_cast<const bf16_t*>(a.y) + row * a.ld + 4 * v);
+#pragma unroll
+        for (int k = 0; k < kTopRegs; ++k)
+          if (k < a.top) eq[j][k] = *reinterpret_cast<const u16x4*>(static_cast<const bf16_t*>(a.e) + er[k] + 4 * v);
+      }
+      if (streams) {
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+          xq[j][s] = s < a.S ? __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(xr + (int64_t)s * a.ld + 4 * v)) : f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  };
+  auto output = [&](int v, int j) {   // 4 features of the sublayer's output; j: the vector's place in its group
     f32x4 y = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (a.yp) {
+    if constexpr (ASK) {
+      if (a.y) y = f4(yq[j]);
+    } else if (a.yp) {
       const float* p = a.yp + row * a.ld + 4 * v;
       int s0 = 0;
       if constexpr (MAXV == 1) {   // up to 8 slabs requested before the first add: one round trip
@@ -78,6 +117,12 @@ __global__ void __launch_bounds__(NT) stream_step_kernel(const StreamStep a) {
       y = ld4(a.y, row * a.ld + 4 * v, a.f32);
     }
     if (a.gate) y *= gate;
+    if constexpr (ASK) {
+#pragma unroll
+      for (int k = 0; k < kTopRegs; ++k)
+        if (k < a.top) y += f4(eq[j][k]);
+      return y;
+    }
     for (int k = 0; k < a.top; ++k) {
       const int64_t sl = row * a.top + k;
       const int64_t er = a.epos ? (int64_t)a.epos[sl] : sl;
@@ -91,7 +136,8 @@ __global__ void __launch_bounds__(NT) stream_step_kernel(const StreamStep a) {
 #pragma unroll
     for (int i = 0; i < MAXV; ++i) {
       const int v = tid + i * NT;
-      yn[i] = v < nv ? output(v) : f32x4{0.f, 0.f, 0.f, 0.f};
+      if (ASK && i % U == 0) ask(i, true, false);
+      yn[i] = v < nv ? output(v, i % U) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < 4; ++j) ys += yn[i][j] * yn[i][j];
     }
@@ -108,6 +154,7 @@ __global__ void __launch_bounds__(NT) stream_step_kernel(const StreamStep a) {
   for (int i = 0; i < MAXV; ++i) {
     const int v = tid + i * NT;
     u[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (ASK && i % U == 0) ask(i, !POST, true);
     if (v < nv) {
       f32x4 nx[S];
       if (a.ids) {
@@ -120,10 +167,11 @@ __global__ void __launch_bounds__(NT) stream_step_kernel(const StreamStep a) {
         f32x4 xo[S];
 #pragma unroll
         for (int s = 0; s < S; ++s)
-          xo[s] = s < a.S ? *reinterpret_cast<const f32x4*>(xr + (int64_t)s * a.ld + 4 * v) : f32x4{0.f, 0.f, 0.f, 0.f};
+          if constexpr (ASK) xo[s] = xq[i % U][s];
+          else xo[s] = s < a.S ? *reinterpret_cast<const f32x4*>(xr + (int64_t)s * a.ld + 4 * v) : f32x4{0.f, 0.f, 0.f, 0.f};
         f32x4 y;
         if constexpr (POST) y = yn[i];
-        else y = output(v);
+        else y = output(v, i % U);
 #pragma unroll
         for (int t = 0; t < S; ++t) {
           f32x4 n = y * coef[S * S + t];
@@ -164,18 +212,23 @@ static void launch_streams(const StreamStep& a, int n, hipStream_t stream) {
   if constexpr (S <= 4) {
     // few rows (decode): a vector per thread, so a row's loads all leave in one round trip
     if (n <= 512 && nv > 256) {
-      if (nv <= 512) stream_step_kernel<S, 512, 1, POST><<<n, 512, 0, stream>>>(a);
-      else if (nv <= 1024) stream_step_kernel<S, 1024, 1, POST><<<n, 1024, 0, stream>>>(a);
-      else if (nv <= 2048) stream_step_kernel<S, 1024, 2, POST><<<n, 1024, 0, stream>>>(a);
-      else stream_step_kernel<S, 1024, 4, POST><<<n, 1024, 0, stream>>>(a);
+      if (nv <= 512) stream_step_kernel<S, 512, 1, POST, false><<<n, 512, 0, stream>>>(a);
+      else if (nv <= 1024) stream_step_kernel<S, 1024, 1, POST, false><<<n, 1024, 0, stream>>>(a);
+      else if (nv <= 2048) stream_step_kernel<S, 1024, 2, POST, false><<<n, 1024, 0, stream>>>(a);
+      else stream_step_kernel<S, 1024, 4, POST, false><<<n, 1024, 0, stream>>>(a);
       return;
     }
   }
-  if (nv <= 64) stream_step_kernel<S, 64, 1, POST><<<n, 64, 0, stream>>>(a);
-  else if (nv <= 256) stream_step_kernel<S, 256, 1, POST><<<n, 256, 0, stream>>>(a);
-  else if (nv <= 1024) stream_step_kernel<S, 256, 4, POST><<<n, 256, 0, stream>>>(a);
-  else if (nv <= 2048) stream_step_kernel<S, 256, 8, POST><<<n, 256, 0, stream>>>(a);
-  else stream_step_kernel<S, 256, 16, POST><<<n, 256, 0, stream>>>(a);
+  // ASK: bf16 rows beside streams that no cache holds for long. From 128 MiB of them on it was faster whether they came from memory or from the
+  // step before (5000 rows of 4 x 2048, four experts: 92 us -> 69, 71 -> 67); of 59 MiB (900 rows of 4 x 4096, two experts) 30.5 -> 28.2, but 23.8 -> 25.2
+  const bool ask = !a.f32 && !a.yp && !a.ids && a.top <= kTopRegs && (int64_t)n * a.S * a.ld * 4 >= (128 << 20);
+  if (ask && nv > 256 && nv <= 1024) stream_step_kernel<S, 256, 4, POST, true><<<n, 256, 0, stream>>>(a);
+  else if (ask && S == 1 && nv > 1024 && nv <= 2048) stream_step_kernel<S, 256, S == 1 ? 8 : 4, POST, true><<<n, 256, 0, stream>>>(a);
+  else if (nv <= 64) stream_step_kernel<S, 64, 1, POST, false><<<n, 64, 0, stream>>>(a);
+  else if (nv <= 256) stream_step_kernel<S, 256, 1, POST, false><<<n, 256, 0, stream>>>(a);
+  else if (nv <= 1024) stream_step_kernel<S, 256, 4, POST, false><<<n, 256, 0, stream>>>(a);
+  else if (nv <= 2048) stream_step_kernel<S, 256, 8, POST, false><<<n, 256, 0, stream>>>(a);
+  else stream_step_kernel<S, 256, 16, POST, false><<<n, 256, 0, stream>>>(a);
 }
 
 int stream_step(const StreamStep& a, int n_rows, hipStream_t stream) {
