@@ -167,18 +167,60 @@ void decode_slots(const at::Tensor& bt, const at::Tensor& pos, const at::Tensor&
                         (int)B, (int)bt.size(1), (int)page_size, cur_stream()));
 }
 
-void decode_advance(const at::Tensor& tok, at::Tensor& ids, at::Tensor& hist, at::Tensor& pos, at::Tensor& ctx,
-                    at::Tensor& step) {
-  CHECK_DEV(tok); CHECK_DT(tok, at::kLong); CHECK_CONTIG(tok); CHECK_DT(ids, at::kLong); CHECK_CONTIG(ids);
+void decode_advance(const c10::optional<at::Tensor>& tok, at::Tensor& ids, at::Tensor& hist, at::Tensor& pos, at::Tensor& ctx,
+                    at::Tensor& step, const c10::optional<at::Tensor>& bt, const c10::optional<at::Tensor>& slots,
+                    const c10::optional<at::Tensor>& spos, int64_t page_size, const c10::optional<at::Tensor>& part,
+                    const c10::optional<at::Tensor>& temperature, const c10::optional<at::Tensor>& given) {
+  CHECK_DEV(ids); CHECK_DT(ids, at::kLong); CHECK_CONTIG(ids);
   CHECK_DT(hist, at::kLong); CHECK_CONTIG(hist); CHECK_DT(pos, at::kLong); CHECK_CONTIG(pos);
   CHECK_DT(ctx, at::kInt); CHECK_CONTIG(ctx); CHECK_DT(step, at::kLong);
   const int64_t B = ids.numel();
-  TORCH_CHECK(tok.numel() == B && pos.numel() == B && ctx.numel() == B && hist.dim() == 2 && hist.size(0) == B &&
+  TORCH_CHECK(pos.numel() == B && ctx.numel() == B && hist.dim() == 2 && hist.size(0) == B && hist.size(1) > 0 &&
                   step.numel() == 1 && B <= 1024,
-              "decode_advance: tok/ids/pos/ctx [B], hist [B, ms], step [1], B <= 1024");
+              "decode_advance: ids/pos/ctx [B], hist [B, ms], step [1], B <= 1024");
+  TORCH_CHECK(tok.has_value() != part.has_value(), "decode_advance: tokens or candidates");
+  oamd::DecodeAdvance a{};
+  if (tok.has_value()) {
+    CHECK_DEV(*tok); CHECK_DT(*tok, at::kLong); CHECK_CONTIG(*tok);
+    TORCH_CHECK(tok->numel() == B, "decode_advance: tok [B]");
+    a.tok = ptr<int64_t>(*tok);
+  } else {
+    TORCH_CHECK(temperature.has_value(), "decode_advance: candidates need the rows' temperatures");
+    CHECK_DEV(*part); CHECK_DT(*part, at::kFloat); CHECK_CONTIG(*part);
+    CHECK_DEV(*temperature); CHECK_DT(*temperature, at::kFloat); CHECK_CONTIG(*temperature);
+    TORCH_CHECK(B > 0 && part->dim() == 3 && part->size(0) == B && part->size(1) >= 1 && part->size(1) <= 1024 && part->size(2) == 2 &&
+                    temperature->numel() == B,
+                "decode_advance: candidates [B, parts, 2], temperature [B]");
+    a.part = reinterpret_cast<const float2*>(part->data_ptr<float>());
+    a.parts = (int)part->size(1);
+    a.temperature = temperature->data_ptr<float>();
+  }
+  if (bt.has_value()) {
+    TORCH_CHECK(slots.has_value() && spos.has_value() && page_size > 0, "decode_advance: bt with slots, spos and the page's size");
+    CHECK_DEV(*bt); CHECK_DT(*bt, at::kInt); CHECK_CONTIG(*bt); CHECK_DEV(*slots); CHECK_DT(*slots, at::kLong); CHECK_CONTIG(*slots);
+    CHECK_DEV(*spos); CHECK_DT(*spos, at::kLong); CHECK_CONTIG(*spos);
+    TORCH_CHECK(bt->dim() == 2 && bt->size(0) == B && bt->size(1) > 0 && slots->numel() == B && spos->numel() == B,
+                "decode_advance: bt [B, max_pages], slots/spos [B]");
+    a.bt = ptr<int>(*bt);
+    a.slots = ptr<int64_t>(*slots);
+    a.spos = ptr<int64_t>(*spos);
+    a.max_pages = (int)bt->size(1);
+    a.page_size = (int)page_size;
+  }
+  if (given.has_value()) {
+    CHECK_DEV(*given); CHECK_DT(*given, at::kLong); CHECK_CONTIG(*given);
+    TORCH_CHECK(given->numel() == 2, "decode_advance: given [2]");
+    a.out = ptr<int64_t>(*given);
+  }
+  a.ids = ptr<int64_t>(ids);
+  a.hist = ptr<int64_t>(hist);
+  a.pos = ptr<int64_t>(pos);
+  a.ctx = ptr<int>(ctx);
+  a.step = ptr<int64_t>(step);
+  a.B = (int)B;
+  a.ms = (int)hist.size(1);
   const c10::hip::HIPGuardMasqueradingAsCUDA g(ids.device());
-  RC(oamd::decode_advance(ptr<int64_t>(tok), ptr<int64_t>(ids), ptr<int64_t>(hist), ptr<int64_t>(pos),
-                          ptr<int>(ctx), ptr<int64_t>(step), (int)B, (int)hist.size(1), cur_stream()));
+  RC(oamd::decode_advance(a, cur_stream()));
 }
 
 void scatter_rows_f32(const at::Tensor& x, const at::Tensor& dst, at::Tensor& out) {
@@ -704,7 +746,8 @@ void attn_prefill(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
 
 void sample(const at::Tensor& logits, const at::Tensor& temperature, const at::Tensor& seeds,
             const at::Tensor& positions, at::Tensor& out, int64_t col_offset,
-            const c10::optional<at::Tensor>& out_val, const c10::optional<at::Tensor>& part) {
+            const c10::optional<at::Tensor>& out_val, const c10::optional<at::Tensor>& part, bool merge,
+            const c10::optional<at::Tensor>& given, const c10::optional<at::Tensor>& dst) {
   CHECK_DEV(logits);
   TORCH_CHECK(logits.dim() == 2 && logits.stride(1) == 1, "logits must be [rows, vocab] row-major");
   TORCH_CHECK(logits.scalar_type() == at::kFloat || logits.scalar_type() == at::kBFloat16, "logits dtype");
@@ -720,10 +763,17 @@ void sample(const at::Tensor& logits, const at::Tensor& temperature, const at::T
     CHECK_DEV(*part); CHECK_DT(*part, at::kFloat); CHECK_CONTIG(*part);
     TORCH_CHECK(part->numel() >= 2 * rows * oamd::sample_parts((int)rows, (int)logits.size(1)), "sampler workspace too small");
   }
+  oamd::GivenRows gr{};
+  if (given.has_value()) {
+    TORCH_CHECK(dst.has_value() && col_offset == 0, "sampler: given rows go to rows dst of whole vocabularies");
+    CHECK_DEV(*given); CHECK_DT(*given, at::kLong); CHECK_CONTIG(*given); CHECK_DEV(*dst); CHECK_DT(*dst, at::kInt); CHECK_CONTIG(*dst);
+    TORCH_CHECK(given->numel() == 2 && dst->numel() == rows, "sampler: given [2], dst [rows]");
+    gr = {ptr<int64_t>(*given), ptr<int>(*dst)};
+  }
   const c10::hip::HIPGuardMasqueradingAsCUDA g(logits.device());
   RC(oamd::sample_tokens(logits.data_ptr(), logits.scalar_type() == at::kBFloat16, logits.stride(0), (int)rows,
                          (int)logits.size(1), ptr<float>(temperature), ptr<int64_t>(seeds), ptr<int64_t>(positions),
-                         ptr<int64_t>(out), col_offset, optr<float>(out_val), optr<float>(part), cur_stream()));
+                         ptr<int64_t>(out), col_offset, optr<float>(out_val), optr<float>(part), merge, gr, cur_stream()));
 }
 
 }  // namespace
@@ -732,13 +782,20 @@ void sample(const at::Tensor& logits, const at::Tensor& temperature, const at::T
 // GIL released (decode windows: one call per window instead of one Python
 // replay per step, so host threads contending for the GIL cannot stall the feed).
 // The page lists of a decode batch into the rows of its table (on the host, `at` bytes into `buf`, int32 rows of `cols` pages; what a row
-// holds past its list stays). Page by page through numpy's list conversion, 51 lists of 240 pages took 420 us of the host's time, here 40.
-void page_rows(const at::Tensor& buf, int64_t at, int64_t cols, const pybind11::list& lists) {
+// holds past its list stays), and with `page_size` each row's cache slot, `slots` bytes into `buf`, of the position that stands `pos` bytes into it. Page by page through numpy's list conversion, 51 lists of 240 pages took 420 us of the host's time, here 40.
+void page_rows(const at::Tensor& buf, int64_t at, int64_t cols, const pybind11::list& lists, int64_t page_size, int64_t pos, int64_t slots) {
   TORCH_CHECK(buf.device().is_cpu() && buf.is_contiguous() && buf.scalar_type() == at::kByte && at >= 0 && cols > 0 && cols < (1 << 30) &&
                   at <= buf.numel() && (int64_t)lists.size() <= (buf.numel() - at) / (cols * 4) &&
                   (reinterpret_cast<uintptr_t>(buf.data_ptr()) + at) % 4 == 0,
               "page_rows: bytes of at least a row of cols int32 per list");
-  int32_t* row = reinterpret_cast<int32_t*>(static_cast<char*>(buf.data_ptr()) + at);
+  char* const base = static_cast<char*>(buf.data_ptr());
+  int32_t* row = reinterpret_cast<int32_t*>(base + at);
+  const int64_t words = page_size > 0 ? (int64_t)lists.size() * 8 : 0;
+  TORCH_CHECK(page_size >= 0 && (page_size == 0 || (pos >= 0 && slots >= 0 && pos <= buf.numel() - words && slots <= buf.numel() - words &&
+                                                    (reinterpret_cast<uintptr_t>(base) | pos | slots) % 8 == 0)),
+              "page_rows: int64 positions and slots inside the buffer");
+  const int64_t* p = reinterpret_cast<const int64_t*>(base + pos);
+  int64_t* s = reinterpret_cast<int64_t*>(base + slots);
   for (const auto& h : lists) {
     TORCH_CHECK(PyList_Check(h.ptr()), "page_rows: lists of pages");
     const Py_ssize_t n = PyList_GET_SIZE(h.ptr());
@@ -748,6 +805,11 @@ void page_rows(const at::Tensor& buf, int64_t at, int64_t cols, const pybind11::
       if (v == -1 && PyErr_Occurred()) throw pybind11::error_already_set();
       TORCH_CHECK(v >= INT32_MIN && v <= INT32_MAX, "page_rows: a page that int32 does not hold");
       row[i] = (int32_t)v;
+    }
+    if (page_size > 0) {
+      TORCH_CHECK(*p >= 0, "page_rows: a position below 0");
+      *s++ = (int64_t)row[std::min(*p / page_size, cols - 1)] * page_size + *p % page_size;
+      ++p;
     }
     row += cols;
   }
@@ -791,7 +853,10 @@ PYBIND11_MODULE(_C, m) {
         pybind11::arg("sin") = pybind11::none(), pybind11::arg("slots") = pybind11::none(),
         pybind11::arg("bias") = pybind11::none());
   m.def("decode_slots", &decode_slots);
-  m.def("decode_advance", &decode_advance);
+  m.def("decode_advance", &decode_advance, pybind11::arg("tok"), pybind11::arg("ids"), pybind11::arg("hist"), pybind11::arg("pos"),
+        pybind11::arg("ctx"), pybind11::arg("step"), pybind11::arg("bt") = pybind11::none(), pybind11::arg("slots") = pybind11::none(),
+        pybind11::arg("spos") = pybind11::none(), pybind11::arg("page_size") = 0, pybind11::arg("part") = pybind11::none(),
+        pybind11::arg("temperature") = pybind11::none(), pybind11::arg("given") = pybind11::none());
   m.def("scatter_rows_f32", &scatter_rows_f32, pybind11::arg("x"), pybind11::arg("dst"), pybind11::arg("out"));
   m.def("quantize_fp8", &quantize_fp8);
   m.def("silu_quantize_fp8", &silu_quantize_fp8, pybind11::arg("gu"), pybind11::arg("q"), pybind11::arg("sx"),
@@ -830,10 +895,12 @@ PYBIND11_MODULE(_C, m) {
   m.def("attn_prefill_block_q", &oamd::attn_prefill_block_q);
   m.def("sample", &sample, pybind11::arg("logits"), pybind11::arg("temperature"), pybind11::arg("seeds"),
         pybind11::arg("positions"), pybind11::arg("out"), pybind11::arg("col_offset") = 0,
-        pybind11::arg("out_val") = pybind11::none(), pybind11::arg("part") = pybind11::none());
+        pybind11::arg("out_val") = pybind11::none(), pybind11::arg("part") = pybind11::none(), pybind11::arg("merge") = true,
+        pybind11::arg("given") = pybind11::none(), pybind11::arg("dst") = pybind11::none());
   m.attr("NO_SAMPLE_BITS") = oamd::kNoSampleBits;
   m.def("sample_parts", &oamd::sample_parts, pybind11::arg("rows"), pybind11::arg("vocab"));
-  m.def("page_rows", &page_rows, pybind11::arg("buf"), pybind11::arg("at"), pybind11::arg("cols"), pybind11::arg("lists"));
+  m.def("page_rows", &page_rows, pybind11::arg("buf"), pybind11::arg("at"), pybind11::arg("cols"), pybind11::arg("lists"),
+        pybind11::arg("page_size") = 0, pybind11::arg("pos") = 0, pybind11::arg("slots") = 0);
   m.def("graph_launch", &graph_launch, pybind11::arg("graph_exec"), pybind11::arg("count"), pybind11::arg("stream"));
   register_decoder_bindings(m);
   m.attr("ARCH") = "gfx950";

@@ -18,15 +18,28 @@ int rmsnorm_fp8(const bf16_t* x, bf16_t* residual, const bf16_t* w, uint8_t* q, 
                 int64_t r_stride, float eps, const float* xp, int S, hipStream_t stream);
 int silu_mul(const bf16_t* gu, bf16_t* out, int64_t rows, int inter, int block, int64_t in_stride,
              int64_t out_stride, int glu, hipStream_t stream);   // glu: Glu of common.h
-// Decode-step bookkeeping (norm_act.hip): cache slots + sampler positions of the step's tokens,
-// then the state advance after sampling (B <= 1024 rows, one workgroup each).
+// Decode-step bookkeeping (norm_act.hip): cache slots + sampler positions of a step's tokens from its state, and the state
+// advance after sampling, which has the next step's too (B <= 1024 rows, one workgroup each).
 int decode_slots(const int* bt, const int64_t* pos, const int* ctx, int64_t* slots, int64_t* spos, int B,
                  int max_pages, int page_size, hipStream_t stream);
 // out[dst[r]] [cols] = fp32 of row r of x (bf16 or fp32, row stride ld); rows whose dst is outside [0, n_out) are dropped
 int scatter_rows_f32(const void* x, bool bf16, int64_t ld, const int* dst, float* out, int rows, int n_out, int cols,
                      hipStream_t stream);
-int decode_advance(const int64_t* tok, int64_t* ids, int64_t* hist, int64_t* pos, int* ctx, int64_t* step, int B,
-                   int ms, hipStream_t stream);
+struct DecodeAdvance {
+  const int64_t* tok;         // [B], or
+  const float2* part;         // [B][parts] candidates of sample_tokens (parts > 0) and the rows' temperatures
+  int parts;
+  const float* temperature;
+  int64_t *ids, *hist, *pos;  // [B], [B][ms], [B]
+  int* ctx;
+  int64_t* step;
+  int B, ms;
+  const int* bt;              // [B][max_pages], or nullptr: slots and spos stay
+  int64_t *slots, *spos;
+  int max_pages, page_size;
+  int64_t* out;               // GivenRows::out, whose address is taken back once a step has used it, or nullptr
+};
+int decode_advance(const DecodeAdvance& a, hipStream_t stream);
 int embedding(const int64_t* ids, const bf16_t* table, bf16_t* out, int tokens, int hidden,
               int64_t vocab, hipStream_t stream);
 int rope_kv(const bf16_t* qkv, int64_t qkv_stride, const int64_t* pos, const float* cos_t,
@@ -146,10 +159,15 @@ int attn_prefill(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16_t* o, c
                  float scale, int variant, hipStream_t stream,
                  const bf16_t* pk = nullptr, const bf16_t* pv = nullptr, const int* seq_pfx = nullptr);
 constexpr uint32_t kNoSampleBits = 0x7fc5a5a5u;   // temperature of a row that is not sampled: a quiet NaN that nothing computes
+struct GivenRows {            // rows that are not sampled go to an output whose address the step's state holds
+  const int64_t* out;         // device: [address of fp32 rows [n][vocab] or 0, n], or nullptr
+  const int* dst;             // [rows]: the output's row, < 0: none
+};
 int sample_tokens(const void* logits, bool logits_bf16, int64_t stride, int rows, int vocab,
                   const float* temperature, const int64_t* seeds, const int64_t* positions,
-                  int64_t* out_tokens, int64_t col_offset, float* out_val, float* part, hipStream_t stream);
-int sample_parts(int rows, int vocab);   // part: 2 x rows x sample_parts floats, or nullptr (one workgroup per row)
+                  int64_t* out_tokens, int64_t col_offset, float* out_val, float* part, bool merge, const GivenRows& given, hipStream_t stream);
+int sample_parts(int rows, int vocab);   // part: 2 x rows x sample_parts floats, or nullptr (one workgroup per row). merge false: where there are several,
+                                         // they are left for decode_advance and out_tokens is not written
 
 // One-shot all-reduce over peer-mapped fine-grained buffers (allreduce.hip).
 size_t car_buffer_bytes(size_t cap_bytes, int world);

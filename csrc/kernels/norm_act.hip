@@ -4,6 +4,7 @@
 // model. All bf16 traffic is 16 B per lane.
 #include "common.h"
 #include "kernels.h"
+#include "sample.h"
 
 namespace oamd {
 
@@ -265,36 +266,60 @@ int embedding(const int64_t* ids, const bf16_t* table, bf16_t* out, int tokens,
 //   decode_slots:   slot = page(bt[row], pos / P) * P + pos % P for live rows (ctx > 0), else -1;
 //                   spos = pos + 1 (the sampler's stream position)
 //   decode_advance: ids = tok; hist[row, step % ms] = tok; live rows pos += 1, ctx += 1; then
-//                   (one thread) step += 1
+//                   (one thread) step += 1. With parts, tok is the best of a row's sampling candidates (sample.hip); with bt, slots
+//                   and spos become the next step's, as decode_slots has them.
+// The engine writes the first step's slots itself, so a step has one launch behind its sampler instead of two and one in front of it (one row, 4 layers
+// of 4096: 538 us a step and 537; 2 rows of 4 layers of 2048 273 and 270).
+__device__ __forceinline__ int64_t decode_slot(const int* bt, int r, int64_t p, int ctx, int max_pages, int page_size) {
+  int64_t pg = p / page_size;
+  pg = pg < max_pages - 1 ? pg : max_pages - 1;
+  return ctx > 0 ? (int64_t)bt[(int64_t)r * max_pages + pg] * page_size + p % page_size : -1;
+}
+
 __global__ void decode_slots_kernel(const int* __restrict__ bt, const int64_t* __restrict__ pos,
                                     const int* __restrict__ ctx, int64_t* __restrict__ slots,
                                     int64_t* __restrict__ spos, int B, int max_pages, int page_size) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= B) return;
   const int64_t p = pos[r];
-  int64_t pg = p / page_size;
-  pg = pg < max_pages - 1 ? pg : max_pages - 1;
-  slots[r] = ctx[r] > 0 ? (int64_t)bt[(int64_t)r * max_pages + pg] * page_size + p % page_size : -1;
+  slots[r] = decode_slot(bt, r, p, ctx[r], max_pages, page_size);
   spos[r] = p + 1;
 }
 
-__global__ void decode_advance_kernel(const int64_t* __restrict__ tok, int64_t* __restrict__ ids,
-                                      int64_t* __restrict__ hist, int64_t* __restrict__ pos, int* __restrict__ ctx,
-                                      int64_t* __restrict__ step, int B, int ms) {
+__global__ void __launch_bounds__(1024) decode_advance_kernel(const DecodeAdvance a) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < B) {
-    const int64_t t = tok[r];
-    ids[r] = t;
-    hist[(int64_t)r * ms + (int)(step[0] % ms)] = t;
-    if (ctx[r] > 0) {
-      pos[r] += 1;
-      ctx[r] += 1;
+  int64_t* const step = a.step;
+  if (r < a.B) {
+    int c = a.ctx[r];
+    int64_t p = a.pos[r], t;
+    if (a.parts > 0) {
+      float v = -INFINITY;
+      int id = 0x7fffffff;
+      if (!no_sample(a.temperature[r])) {   // its candidates were not written
+        const float2* q = a.part + (int64_t)r * a.parts;
+#pragma unroll 8
+        for (int i = 0; i < a.parts; ++i) argmax_merge(v, id, q[i].x, __float_as_int(q[i].y));
+      }
+      t = id == 0x7fffffff ? 0 : id;
+    } else {
+      t = a.tok[r];
+    }
+    a.ids[r] = t;
+    a.hist[(int64_t)r * a.ms + (int)(step[0] % a.ms)] = t;
+    if (c > 0) {
+      a.pos[r] = ++p;
+      a.ctx[r] = ++c;
+    }
+    if (a.bt != nullptr) {
+      a.slots[r] = decode_slot(a.bt, r, p, c, a.max_pages, a.page_size);
+      a.spos[r] = p + 1;
     }
   }
   __syncthreads();
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     // every block read step[0] before block 0's thread 0 bumps it: one block covers all rows
     step[0] += 1;
+    if (a.out != nullptr) a.out[0] = 0;
   }
 }
 
@@ -307,11 +332,10 @@ int decode_slots(const int* bt, const int64_t* pos, const int* ctx, int64_t* slo
   return 0;
 }
 
-int decode_advance(const int64_t* tok, int64_t* ids, int64_t* hist, int64_t* pos, int* ctx, int64_t* step, int B,
-                   int ms, hipStream_t stream) {
-  if (B <= 0) return 0;
-  if (B > 1024) return -1;   // one block: every row reads step before it is bumped
-  decode_advance_kernel<<<1, 1024, 0, stream>>>(tok, ids, hist, pos, ctx, step, B, ms);
+int decode_advance(const DecodeAdvance& a, hipStream_t stream) {
+  if (a.B <= 0) return 0;
+  if (a.B > 1024) return -1;   // one block: every row reads step before it is bumped
+  decode_advance_kernel<<<1, 1024, 0, stream>>>(a);
   OAMD_LAUNCH_CHECK();
   return 0;
 }

@@ -9,6 +9,7 @@
 // same tokens and the kernel needs no RNG state on the device.
 #include "common.h"
 #include "kernels.h"
+#include "sample.h"
 
 namespace oamd {
 
@@ -19,13 +20,44 @@ __device__ __forceinline__ float load_logit<float>(const float* p, int64_t i) { 
 template <>
 __device__ __forceinline__ float load_logit<bf16_t>(const bf16_t* p, int64_t i) { return bf2f(p[i]); }
 
-__device__ __forceinline__ void argmax_merge(float& bv, int& bi, float v, int i) {
-  if (v > bv || (v == bv && i < bi)) { bv = v; bi = i; }
+// Columns [a, b) vectors of 16 bytes and [sa, sb) of a row to fp32, by the whole workgroup. A step's given rows leave through the sampler, which
+// is in their step anyway, and not through a launch of their own behind it, which with its gap cost a step 12 us (one row, 4 layers of 4096: 537 us a
+// step and 532).
+template <typename T, int NT>
+__device__ __forceinline__ void copy_f32(const T* lr, float* yr, int a, int b, int sa, int sb, bool vec) {
+  constexpr int VEC = 16 / static_cast<int>(sizeof(T)), UNR = 4;
+  const uint4* lv = reinterpret_cast<const uint4*>(lr);
+  auto put = [&](const uint4& raw, int v) {
+    const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+    f32x4 o[VEC / 4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if constexpr (sizeof(T) == 2) {
+        o[k / 2][2 * (k & 1)] = __uint_as_float(w[k] << 16);
+        o[k / 2][2 * (k & 1) + 1] = __uint_as_float(w[k] & 0xffff0000u);
+      } else {
+        o[0][k] = __uint_as_float(w[k]);
+      }
+    }
+    if (vec) {
+#pragma unroll
+      for (int k = 0; k < VEC / 4; ++k) *reinterpret_cast<f32x4*>(yr + VEC * v + 4 * k) = o[k];
+    } else {
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) yr[VEC * v + k] = o[k / 4][k & 3];
+    }
+  };
+  int v = a + threadIdx.x;
+  for (; v + (UNR - 1) * NT < b; v += UNR * NT) {
+    uint4 raw[UNR];
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) raw[u] = lv[v + u * NT];
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) put(raw[u], v + u * NT);
+  }
+  for (; v < b; v += NT) put(lv[v], v);
+  for (int i = sa + threadIdx.x; i < sb; i += NT) yr[i] = load_logit<T>(lr, i);
 }
-
-// Rows whose token nobody reads (given tokens, the padding rows of a bucket) carry this NaN as their temperature: they get
-// token 0 and their logits are not read (256 rows of 128256: 36 us, 5 when all are skipped). Any other NaN is greedy, as ever.
-__device__ __forceinline__ bool no_sample(float temperature) { return __float_as_uint(temperature) == kNoSampleBits; }
 
 // PARTS: workgroup blockIdx.y of gridDim.y, its best (value in base-2 units, column) to part
 template <typename T, int NT, bool PARTS>
@@ -34,13 +66,26 @@ __global__ void __launch_bounds__(NT) sample_kernel(const T* __restrict__ logits
                                                       const int64_t* __restrict__ seeds,
                                                       const int64_t* __restrict__ positions,
                                                       int64_t* __restrict__ out_tokens, int64_t col_offset,
-                                                      float* __restrict__ out_val, float2* __restrict__ part) {
+                                                      float* __restrict__ out_val, float2* __restrict__ part, GivenRows given) {
   __shared__ float sv[NT / 64];
   __shared__ int si[NT / 64];
   const int row = blockIdx.x;
   const T* lr = logits + row * stride;
   const float temp = temperature[row];
+  // 16-B loads over the aligned body of the row (8 bf16 / 4 fp32 per lane), scalar tail: this workgroup's vectors [va, nv) and its
+  // share [sa, sb) of the tail, which is the whole row when that is misaligned
+  constexpr int VEC = 16 / static_cast<int>(sizeof(T));
+  const int all = (reinterpret_cast<uintptr_t>(lr) & 15) == 0 ? vocab / VEC : 0;
+  const int py = PARTS ? blockIdx.y : 0, np = PARTS ? gridDim.y : 1;
+  const int va = (int)((int64_t)all * py / np), nv = (int)((int64_t)all * (py + 1) / np);
+  const int ta = all * VEC, tail = vocab - ta, sa = ta + (int)((int64_t)tail * py / np), sb = ta + (int)((int64_t)tail * (py + 1) / np);
   if (no_sample(temp)) {
+    if (given.out != nullptr) {
+      float* const to = reinterpret_cast<float*>(given.out[0]);
+      const int64_t d = given.dst[row];
+      if (to != nullptr && d >= 0 && d < given.out[1])
+        copy_f32<T, NT>(lr, to + d * vocab, va, nv, sa, sb, vocab % 4 == 0 && reinterpret_cast<uintptr_t>(to) % 16 == 0);
+    }
     if (!PARTS && threadIdx.x == 0) {
       out_tokens[row] = col_offset;
       if (out_val) out_val[row] = 0.f;
@@ -67,15 +112,8 @@ __global__ void __launch_bounds__(NT) sample_kernel(const T* __restrict__ logits
     }
     argmax_merge(bv, bi, x, i);
   };
-  // 16-B loads over the aligned body of the row (8 bf16 / 4 fp32 per lane), scalar tail.
   // argmax_merge is a total order (value, then smaller index), so the visiting order
   // does not change the result.
-  constexpr int VEC = 16 / static_cast<int>(sizeof(T));
-  // this workgroup's vectors [va, nv) and its share [sa, sb) of the scalar tail, which is the whole row when that is misaligned
-  const int all = (reinterpret_cast<uintptr_t>(lr) & 15) == 0 ? vocab / VEC : 0;
-  const int py = PARTS ? blockIdx.y : 0, np = PARTS ? gridDim.y : 1;
-  const int va = (int)((int64_t)all * py / np), nv = (int)((int64_t)all * (py + 1) / np);
-  const int ta = all * VEC, tail = vocab - ta, sa = ta + (int)((int64_t)tail * py / np), sb = ta + (int)((int64_t)tail * (py + 1) / np);
   auto visit16 = [&](const uint4& raw, int v) {
     const uint32_t wv[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
@@ -163,17 +201,17 @@ int sample_parts(int rows, int vocab) {
 
 int sample_tokens(const void* logits, bool logits_bf16, int64_t stride, int rows, int vocab,
                   const float* temperature, const int64_t* seeds, const int64_t* positions,
-                  int64_t* out_tokens, int64_t col_offset, float* out_val, float* part, hipStream_t stream) {
+                  int64_t* out_tokens, int64_t col_offset, float* out_val, float* part, bool merge, const GivenRows& given, hipStream_t stream) {
   if (rows == 0) return 0;
   const int parts = part ? sample_parts(rows, vocab) : 1;
   float2* pp = reinterpret_cast<float2*>(part);
 #define OAMD_SAMPLE(T)                                                                                                              \
   if (parts > 1)                                                                                                                    \
     sample_kernel<T, 256, true><<<dim3(rows, parts), 256, 0, stream>>>(static_cast<const T*>(logits), stride, vocab, temperature,   \
-                                                                       seeds, positions, out_tokens, col_offset, out_val, pp);      \
+                                                                       seeds, positions, out_tokens, col_offset, out_val, pp, given);      \
   else                                                                                                                              \
     sample_kernel<T, 1024, false><<<rows, 1024, 0, stream>>>(static_cast<const T*>(logits), stride, vocab, temperature, seeds,      \
-                                                             positions, out_tokens, col_offset, out_val, nullptr)
+                                                             positions, out_tokens, col_offset, out_val, nullptr, given)
   if (logits_bf16) {
     OAMD_SAMPLE(bf16_t);
   } else {
@@ -181,7 +219,7 @@ int sample_tokens(const void* logits, bool logits_bf16, int64_t stride, int rows
   }
 #undef OAMD_SAMPLE
   OAMD_LAUNCH_CHECK();
-  if (parts > 1) {
+  if (parts > 1 && merge) {
     sample_merge_kernel<<<(rows + 3) / 4, 256, 0, stream>>>(pp, rows, parts, temperature, out_tokens, col_offset, out_val);
     OAMD_LAUNCH_CHECK();
   }

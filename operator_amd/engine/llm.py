@@ -25,6 +25,7 @@ from __future__ import annotations
 import contextlib
 import gc
 import itertools
+import math
 import threading
 import time
 from collections import deque
@@ -153,21 +154,28 @@ class _BucketState:
     """Device-resident decode state of one batch bucket (shared by its graphs).
 
     One step = forward + sample + state advance (ids <- sampled token,
-    pos/ctx += 1 on active rows, token appended to ``hist[:, step]``), so the
-    host can replay several steps back-to-back and read ``hist`` once.
+    pos/ctx += 1 on active rows, token appended to ``hist[:, step]``, the next step's
+    ``slots`` and ``spos``), so the host can replay several steps back-to-back and read ``hist`` once.
     Rows with ctx == 0 are padding: slot -1 (no KV write), zero attention.
     """
 
     def __init__(self, eng: "LLMEngine", bp: int):
         dev = eng.device
         self.bp = bp
+        self.page_size = eng.kv.page_size
         # the per-row state ``load`` rewrites lives in one byte buffer (one H2D copy per
         # batch-composition change instead of six)
         mp = eng.max_pages
-        self._spec = (("step", (1,), torch.long), ("ids", (bp,), torch.long), ("pos", (bp,), torch.long),
-                      ("seeds", (bp,), torch.long), ("ctx", (bp,), torch.int32), ("dst", (bp,), torch.int32), ("temp", (bp,), torch.float32),
+        self._spec = (("step", (1,), torch.long), ("out", (2,), torch.long),   # (address, rows) of a given step's logits, see given_next
+                      ("ids", (bp,), torch.long), ("pos", (bp,), torch.long),
+                      ("seeds", (bp,), torch.long),
+                      ("slots", (bp,), torch.long), ("spos", (bp,), torch.long),   # the step's: cache slot of each row's token, sampler stream position
+                      ("ctx", (bp,), torch.int32), ("dst", (bp,), torch.int32), ("temp", (bp,), torch.float32),
                       ("bt", (bp, mp), torch.int32))
-        self._nbytes = sum(int(np.prod(s)) * torch.empty((), dtype=dt).element_size() for _, s, dt in self._spec)
+        self._at, self._nbytes = {}, 0   # bytes from the buffer's start: 8-byte fields first, then 4-byte, so every view is aligned
+        for name, shape, dt in self._spec:
+            self._at[name] = self._nbytes
+            self._nbytes += math.prod(shape) * dt.itemsize
         self._buf = torch.zeros(self._nbytes, dtype=torch.uint8, device=dev)
         for n, t in self._views(self._buf).items():
             setattr(self, n, t)
@@ -177,20 +185,14 @@ class _BucketState:
         # no kernel to reset it (the one-element fill it replaced sat ~1 ms behind the previous
         # window's token copy on the GPU at every window boundary)
         self.step_host = 0
-        self.slots = torch.zeros(bp, dtype=torch.long, device=dev)   # per step: cache slot of each row's token
-        self.spos = torch.zeros(bp, dtype=torch.long, device=dev)    # per step: sampler stream position
+        self.slots.fill_(-1)
 
     def _views(self, buf: torch.Tensor) -> dict:
-        out, off = {}, 0
-        for n, shape, dt in self._spec:   # 8-byte fields first, then 4-byte: every view aligned
-            nb = int(np.prod(shape)) * torch.empty((), dtype=dt).element_size()
-            out[n] = buf[off:off + nb].view(dt).view(shape)
-            off += nb
-        return out
+        return {n: buf[self._at[n]:self._at[n] + math.prod(shape) * dt.itemsize].view(dt).view(shape) for n, shape, dt in self._spec}
 
-    def load(self, reqs: list[GenRequest], max_pages: int, dst: list[int] | None = None) -> None:
-        """Write the per-row state of ``reqs`` (rows beyond are padding; ``dst``: the row of the caller's logits each
-        takes, see given_next; their tokens are not sampled). Built in numpy
+    def load(self, reqs: list[GenRequest], max_pages: int, dst: list[int] | None = None, out: torch.Tensor | None = None) -> None:
+        """Write the per-row state of ``reqs`` (rows beyond are padding; ``dst``: the row of the caller's logits ``out`` each
+        takes in the next step, and in no later one, see given_next; their tokens are not sampled). Built in numpy
         (one pass over the rows, no per-element tensor indexing: ~0.3 ms instead of
         ~10 ms for 256 rows at every batch-composition change) and copied in once."""
         n = len(reqs)
@@ -199,6 +201,11 @@ class _BucketState:
         ids, pos, ctx, bt, temp, seeds = v["ids"], v["pos"], v["ctx"], v["bt"], v["temp"], v["seeds"]
         assert bt.shape[1] == max_pages
         temp.view(np.uint32)[:] = ops.NO_SAMPLE_BITS   # padding rows, and given tokens
+        v["slots"][:] = -1
+        v["spos"][:] = 1
+        v["dst"][:] = -1
+        if out is not None:
+            v["out"][:] = out.data_ptr(), out.shape[0]
         if n:
             lens = np.fromiter((r.length for r in reqs), dtype=np.int64, count=n)
             ids[:n] = np.fromiter((r.output[-1] for r in reqs), dtype=np.int64, count=n)
@@ -210,10 +217,12 @@ class _BucketState:
                 temp[:n] = np.fromiter((r.temperature for r in reqs), dtype=np.float32, count=n)
                 seeds[:n] = np.fromiter((r.seed for r in reqs), dtype=np.int64, count=n)
             if self._buf.is_cuda:
-                ops.kernels().page_rows(host, self._nbytes - bt.nbytes, bt.shape[1], [r.pages for r in reqs])
+                at = self._at
+                ops.kernels().page_rows(host, at["bt"], max_pages, [r.pages for r in reqs], self.page_size, at["pos"], at["slots"])
             else:
                 for i, r in enumerate(reqs):
                     bt[i, :len(r.pages)] = r.pages
+            v["spos"][:n] = lens
         nb = self._buf.is_cuda
         self._buf.copy_(host.pin_memory() if nb else host, non_blocking=nb)   # step = 0
         self.step_host = 0
@@ -250,8 +259,7 @@ class _DecodeGraph:
         e, st = self.eng, self.st
         P = e.kv.page_size
         gpu = st.ids.is_cuda
-        if gpu:   # one bookkeeping kernel before and one after the forward (norm_act.hip)
-            ops.kernels().decode_slots(st.bt, st.pos, st.ctx, st.slots, st.spos, P)
+        if gpu:   # set by ``load`` or the step before: one bookkeeping kernel, behind the sampler (norm_act.hip)
             slots, spos = st.slots, st.spos
         else:
             act = st.ctx > 0
@@ -261,10 +269,15 @@ class _DecodeGraph:
         fb = ForwardBatch(st.ids, st.pos, slots, False, None, block_tables=st.bt, context_lens=st.ctx,
                           num_splits=self.splits)
         self.logits = e.model.forward(fb, e.kv)   # [bp, vocab]: a replay overwrites them in place
-        tok = e.model.sample(self.logits, st.temp, st.seeds, spos)
         if gpu:
-            ops.kernels().decode_advance(tok, st.ids, st.hist, st.pos, st.ctx, st.step)
+            if e.model.tp.world == 1:
+                tok = ops.sample_candidates(self.logits, st.temp, st.seeds, spos, st.out, st.dst)
+            else:
+                tok = {"tok": e.model.sample(self.logits, st.temp, st.seeds, spos)}
+            ops.kernels().decode_advance(ids=st.ids, hist=st.hist, pos=st.pos, ctx=st.ctx, step=st.step, bt=st.bt, slots=slots, spos=spos,
+                                         page_size=P, given=st.out, **tok)
         else:
+            tok = e.model.sample(self.logits, st.temp, st.seeds, spos)
             st.ids.copy_(tok)
             st.hist.index_copy_(1, st.step % e.multi_step, tok.unsqueeze(1))   # wrap: a stray replay can never index past hist
             st.pos.add_(act.to(torch.long))
@@ -275,22 +288,23 @@ class _DecodeGraph:
         # warm up on a side stream (allocator + hipBLASLt heuristics), then capture; the
         # state is snapshotted and restored so capture never perturbs live rows
         st = self.st
-        snap = [t.clone() for t in (st.ids, st.pos, st.ctx, st.step)]
+        state = (st.ids, st.pos, st.ctx, st.step, st.slots, st.spos, st.out)
+        snap = [t.clone() for t in state]
+        st.ctx.zero_()  # all rows padding while warming up: no KV writes
+        st.out.zero_()  # ... and no logits to anyone
+        ops.kernels().decode_slots(st.bt, st.pos, st.ctx, st.slots, st.spos, self.eng.kv.page_size)
         s = torch.cuda.Stream(device=self.eng.device)
         s.wait_stream(torch.cuda.current_stream())
-        saved_ctx = st.ctx.clone()
-        st.ctx.zero_()  # all rows padding while warming up: no KV writes
         with torch.cuda.stream(s):
             for _ in range(2):
                 st.step.zero_()
                 self._run()
         torch.cuda.current_stream().wait_stream(s)
-        st.ctx.copy_(torch.zeros_like(saved_ctx))
         g = torch.cuda.CUDAGraph()
         with _no_gc(), torch.cuda.graph(g, pool=pool):
             self._run()
         self.graph = g
-        for t, v in zip((st.ids, st.pos, st.ctx, st.step), snap):
+        for t, v in zip(state, snap):
             t.copy_(v)
 
     def run(self, use_graph: bool) -> None:
@@ -1014,12 +1028,13 @@ class LLMEngine:
             rows = [reqs[i] for i in part]
             bp = self._bucket(len(rows))
             g = self._graph(bp, self._splits(rows[0].length, bp))
-            g.st.load(rows, self.max_pages, part)
+            own = out.is_cuda and self.model.tp.world == 1   # the step's sampler writes them: the address and order travel with the rows' state
+            g.st.load(rows, self.max_pages, part, out if own else None)
             g.run(self.use_graphs)
             n = len(rows)
-            if out.is_cuda:   # the order travelled with the rows' state: nothing here waits for the GPU
+            if out.is_cuda and not own:
                 ops.kernels().scatter_rows_f32(g.logits[:n], g.st.dst[:n], out)
-            else:
+            elif not own:
                 out[part] = g.logits[:n].float()
             self.stats.decode_tokens += len(rows)
         self._given_queued()

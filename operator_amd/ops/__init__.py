@@ -1228,4 +1228,20 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, seeds: torch.Tensor,
     return o
 
 
+def sample_candidates(logits: torch.Tensor, temperature: torch.Tensor, seeds: torch.Tensor, positions: torch.Tensor,
+                      given: torch.Tensor | None = None, dst: torch.Tensor | None = None) -> dict:
+    """``sample`` as far as the next kernel takes it: decode_advance's ``tok``, or ``part`` [rows, parts, 2] where several workgroups share a
+    row, whose best that kernel takes itself. ``given`` [2] (on the device: the address of fp32 rows, 0: none, and their number): rows that are
+    not sampled (NO_SAMPLE_BITS) go to its rows ``dst``."""
+    rows = logits.shape[0]
+    parts = kernels().sample_parts(rows, logits.shape[1])
+    tok = torch.empty(rows, dtype=torch.long, device=logits.device)
+    if parts <= 1:
+        kernels().sample(logits, temperature, seeds, positions, tok, 0, None, None, True, given, dst)
+        return {"tok": tok}
+    part = torch.empty(rows, parts, 2, dtype=torch.float32, device=logits.device)
+    kernels().sample(logits, temperature, seeds, positions, tok, 0, None, part, False, given, dst)
+    return {"tok": None, "part": part, "temperature": temperature}
+
+
 from . import decoder  # noqa: E402 - uses SplitK and prefill_work_list above

@@ -31,3 +31,20 @@ def test_page_rows_refuses():
     for at, cols in ((4, 16), (-4, 4), (2, 4), (68, 4), (0, 0)):
         with pytest.raises(RuntimeError):
             C.page_rows(t, at, cols, [[1]])
+
+
+def test_slots_of_the_positions():
+    rows, cols, P = 5, 6, 16
+    buf = torch.zeros(8 + 2 * rows * 8 + rows * cols * 4, dtype=torch.uint8)
+    n = buf.numpy()
+    pos, slots = n[8:8 + 8 * rows].view(np.int64), n[8 + 8 * rows:8 + 16 * rows].view(np.int64)
+    pos[:] = [0, 15, 16, 95, 200]   # the last one past the table: its last page
+    lists = [[3], [4], [5, 6], list(range(10, 16)), list(range(20, 26))]
+    ops.kernels().page_rows(buf, 8 + 16 * rows, cols, lists, P, 8, 8 + 8 * rows)
+    assert slots.tolist() == [48, 79, 96, 15 * 16 + 15, 25 * 16 + 8]
+    for page_size, at, to in ((-1, 8, 48), (16, -8, 48), (16, 4, 48), (16, 8, 180), (16, 8, 49)):
+        with pytest.raises(RuntimeError):
+            ops.kernels().page_rows(buf, 8 + 16 * rows, cols, lists, page_size, at, to)
+    pos[1] = -1
+    with pytest.raises(RuntimeError):
+        ops.kernels().page_rows(buf, 8 + 16 * rows, cols, lists, P, 8, 48)
