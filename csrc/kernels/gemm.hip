@@ -28,6 +28,8 @@
 //     179 -> 155 (by the product over 2048 columns; 16 of 3456 x 2368 151 in step, 159 round); of 128 rows, whose X weighs more, they keep
 //     step (112 rows each 242, 258 round).
 // MFMA v_mfma_f32_16x16x32_bf16; fragment maps as in attn_decode.hip.
+#include <type_traits>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -64,9 +66,10 @@ struct GemmCfg {
   static constexpr int FN = BN / WN / 16;                // 16-col fragments per wave
   static constexpr int ROWS = BM + BN;                   // rows of one stage (A then B)
   static constexpr int STAGE_BYTES = ROWS * kBK * 2;     // bf16
-  static constexpr int GL = ROWS / 8 / kWaves;           // LDS-DMA instructions per wave per stage
+  static constexpr int GL = (ROWS / 8 + kWaves - 1) / kWaves;   // LDS-DMA instructions per wave per stage, one fewer ...
+  static constexpr int FULL = ROWS / 8 % kWaves;                // ... from wave FULL on (0: as many)
   static constexpr int LDS_BYTES = NS * STAGE_BYTES;
-  static_assert(ROWS % (8 * kWaves) == 0, "stage rows must split evenly over the waves");
+  static_assert(ROWS % 8 == 0, "whole LDS-DMA instructions");
 };
 
 __device__ __forceinline__ int swz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
@@ -78,7 +81,9 @@ __device__ __forceinline__ void wait_vmcnt() {
 
 // Epilogues: plain bf16 store, fp32 split-K slab, or the fused SwiGLU of the
 // gate|up projection (weights interleaved in 64-row blocks: tile columns
-// [0,64) = gate, [64,128) = up of the same 64 features; output [M, N/2]).
+// [0,64) = gate, [64,128) = up of the same 64 features; output [M, N/2]). Gated tiles of 64 and 160 columns take the gate and up rows of 32 and 80 features
+// from wherever they are: a workgroup takes in 45 bytes per ns whatever its tile, so the width is chosen for one full round of the
+// CUs (ops.gate_up_tile: 64 rows of 37888 x 3584 62 us in 296 workgroups of 128 columns, 44 in 237 of 160; 256 rows 112 -> 75).
 enum { kEpiStore = 0, kEpiPartial = 1, kEpiSiluGU = 2 };
 
 // GRP: routed experts. Row tile y holds rows of one expert (moe_sort with bm = BM): gtab[0] = row
@@ -99,7 +104,9 @@ __global__ void __launch_bounds__(kWaves * 64, NS == 2 ? 2 : 1) gemm_tn_kernel(c
   const int kz = blockIdx.x % S, nt = blockIdx.x / S;
   const int n0 = nt * BN;
   const int m0 = blockIdx.y * BM;  // row tile (M may be split into BM-row tiles)
-  int turn = nt;
+  // gated tiles that are not an interleaved block of 64: BN / 2 features' gate rows, then their up rows, wherever those are
+  constexpr bool kSplitGU = EPI == kEpiSiluGU && BN != 128;
+  int turn = kSplitGU ? nt * (BN / 2) >> 6 : nt;   // a block's tiles start alike, so a column's sum does not depend on the tile
   if constexpr (GRP) {
     if ((int)blockIdx.y >= gtab[0]) return;
     const int e = gtab[1 + blockIdx.y];
@@ -134,7 +141,11 @@ __global__ void __launch_bounds__(kWaves * 64, NS == 2 ? 2 : 1) gemm_tn_kernel(c
       const int q = w + kWaves * i;
       const int row = 8 * q + lrow;
       const int chunk = swz(row, lslot);
-      const int wn_ = n0 + row - BM;
+      int wn_ = n0 + row - BM;
+      if constexpr (kSplitGU) {
+        const int up = row - BM >= BN / 2, f = min(nt * (BN / 2) + row - BM - up * (BN / 2), N / 2 - 1);   // past the last feature: any row
+        wn_ = (f >> 6) * 128 + up * 64 + (f & 63);
+      }
       // tiled W ([N/64][K/64][64][64]): each 8-row x 128-B piece of a stage is one
       // contiguous 1 KB of HBM instead of 8 separate 128-B row segments
       const bf16_t* wsrc = (w_tiled & 1) ? W + ((int64_t)(wn_ >> 6) * (K >> 6) + (k0 >> 6)) * 4096 + (wn_ & 63) * 64 + chunk * 8
@@ -146,9 +157,11 @@ __global__ void __launch_bounds__(kWaves * 64, NS == 2 ? 2 : 1) gemm_tn_kernel(c
         __builtin_amdgcn_global_load_lds(from, (__attribute__((address_space(3))) void*)(sbase + q * 1024), 16, 0, 0);
     }
   };
+  const bool full = C::FULL == 0 || w < C::FULL;   // this wave has a last instruction
   auto issue = [&](int t, int buf) {
 #pragma unroll
-    for (int i = 0; i < C::GL; ++i) issue_one(t, buf, i);
+    for (int i = 0; i < C::GL; ++i)
+      if (i < C::GL - 1 || full) issue_one(t, buf, i);
   };
 
   const int wm = w / C::WN, wn = w % C::WN;
@@ -189,7 +202,7 @@ __global__ void __launch_bounds__(kWaves * 64, NS == 2 ? 2 : 1) gemm_tn_kernel(c
           const int idx = (s * C::FM + i) * C::FN + j + 1;
 #pragma unroll
           for (int g = 0; g < C::GL; ++g)
-            if (idx == ((g + 1) * TOT) / (C::GL + 1) && do_issue) issue_one(tn, tn % NS, g);
+            if (idx == ((g + 1) * TOT) / (C::GL + 1) && do_issue && (g < C::GL - 1 || full)) issue_one(tn, tn % NS, g);
         }
     }
   };
@@ -203,11 +216,16 @@ __global__ void __launch_bounds__(kWaves * 64, NS == 2 ? 2 : 1) gemm_tn_kernel(c
   for (int t = 0; t < T; ++t) {
     // stages issued so far: min(T, t + NS - 1); leave all but stage t in flight
     const int rem = min(T - 1 - t, NS - 2);   // stages younger than t in flight
-    if (NS >= 6 && rem >= 4) wait_vmcnt<4 * C::GL>();
-    else if (NS >= 5 && rem >= 3) wait_vmcnt<3 * C::GL>();
-    else if (NS >= 4 && rem >= 2) wait_vmcnt<2 * C::GL>();
-    else if (NS >= 3 && rem >= 1) wait_vmcnt<C::GL>();
-    else wait_vmcnt<0>();
+    auto wait = [&](auto gl) {
+      constexpr int GL = decltype(gl)::value;
+      if (NS >= 6 && rem >= 4) wait_vmcnt<4 * GL>();
+      else if (NS >= 5 && rem >= 3) wait_vmcnt<3 * GL>();
+      else if (NS >= 4 && rem >= 2) wait_vmcnt<2 * GL>();
+      else if (NS >= 3 && rem >= 1) wait_vmcnt<GL>();
+      else wait_vmcnt<0>();
+    };
+    if (full) wait(std::integral_constant<int, C::GL>{});
+    else wait(std::integral_constant<int, C::GL - 1>{});
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -218,39 +236,45 @@ __global__ void __launch_bounds__(kWaves * 64, NS == 2 ? 2 : 1) gemm_tn_kernel(c
     // Stage the tile through LDS (the ring is idle now) so each thread sees a
     // feature's gate and up values: HF numerics, act(bf16(g)) rounded to bf16,
     // times bf16(u), rounded.
-    static_assert(BN == 128, "fused SwiGLU needs gate and up halves in one tile");
     constexpr int LD = BN + 4;  // fp32 row stride (+4: spreads the column writes over banks)
-    static_assert(BM * LD * 4 <= C::LDS_BYTES, "C tile must fit the LDS ring");
+    constexpr int HR = BM * LD * 4 <= C::LDS_BYTES ? BM : BM / 2;   // rows at a time: the whole C tile, or half of it
+    static_assert(HR * LD * 4 <= C::LDS_BYTES && HR % (BM / C::WM) == 0, "C tile must fit the LDS ring, halves are whole waves'");
     float* ct = reinterpret_cast<float*>(lds);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < C::FM; ++i)
-#pragma unroll
-      for (int j = 0; j < C::FN; ++j) {
-        const int col = wn * (BN / C::WN) + 16 * j + l15;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) ct[(wm * (BM / C::WM) + 16 * i + 4 * lg + r) * LD + col] = acc[i][j][r];
-      }
-    __syncthreads();
     const int NO = N / 2;  // output features
-    for (int v = tid; v < BM * 8; v += kWaves * 64) {
-      const int row = v >> 3, f0 = (v & 7) * 8;
-      const float* cr = ct + row * LD;
+#pragma unroll
+    for (int h0 = 0; h0 < BM; h0 += HR) {
+    __syncthreads();
+    if (HR == BM || (wm * (BM / C::WM) >= h0 && wm * (BM / C::WM) < h0 + HR)) {
+#pragma unroll
+      for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+        for (int j = 0; j < C::FN; ++j) {
+          const int col = wn * (BN / C::WN) + 16 * j + l15;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) ct[(wm * (BM / C::WM) - h0 + 16 * i + 4 * lg + r) * LD + col] = acc[i][j][r];
+        }
+    }
+    __syncthreads();
+    for (int v = tid; v < HR * (BN / 16); v += kWaves * 64) {
+      const int row = h0 + v / (BN / 16), f0 = v % (BN / 16) * 8;
+      if (kSplitGU && nt * (BN / 2) + f0 >= NO) continue;
+      const float* cr = ct + (row - h0) * LD;
       float c = 1.f;
       if constexpr (GRP) c = rscale[m0 + row];
       u16x8 o;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         if constexpr (GRP) {   // as the list kernel of moe.hip: one rounding
-          const float g = c * cr[f0 + e], u = c * cr[64 + f0 + e];
+          const float g = c * cr[f0 + e], u = c * cr[BN / 2 + f0 + e];
           o[e] = f2bf(g / (1.f + __expf(-g)) * u);
         } else {
-          const float g = bf2f(f2bf(cr[f0 + e])), u = bf2f(f2bf(cr[64 + f0 + e]));
+          const float g = bf2f(f2bf(cr[f0 + e])), u = bf2f(f2bf(cr[BN / 2 + f0 + e]));
           o[e] = f2bf(bf2f(f2bf(glu_gate(g, act))) * u);
         }
       }
-      *reinterpret_cast<u16x8*>(Y + (int64_t)(m0 + row) * NO + nt * 64 + f0) = o;
+      *reinterpret_cast<u16x8*>(Y + (int64_t)(m0 + row) * NO + nt * (BN / 2) + f0) = o;
+    }
     }
   } else {
     // ---- C lane l -> row 4*lg + r, col l15 of each fragment ----
@@ -318,8 +342,28 @@ int gemm_decode(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, in
   const bool turn = turns(K) && M <= 128 && (int64_t)M * K <= kTurnX && (int64_t)N * S >= kTurnN * ((M + BM) / 64);
   if (w_tiled_b && (N % 64 != 0 || K % 64 != 0)) return -6;
   if ((BM != 64 && BM != 128 && BM != 256) || M % BM != 0) return -1;
-  if (glu) {  // fused SwiGLU: one K slice, 128-column tiles of 64 gate + 64 up rows
-    if (BN != 128 || S != 1 || N % 128 != 0 || K % kBK != 0) return -5;
+  if (glu) {  // fused SwiGLU: one K slice, tiles of BN / 2 gate and as many up rows
+    if ((BN != 64 && BN != 128 && BN != 160) || S != 1 || N % 128 != 0 || K % kBK != 0) return -5;
+    if (BN != 128) {
+      if (w_tiled_b) return -6;
+      const dim3 grid((N + BN - 1) / BN, M / BM);
+#define OAMD_GLU(BM, BNN, NSS)                                                                                                                 \
+  if (turn) gemm_tn_kernel<BM, BNN, kEpiSiluGU, NSS, false, BM <= 128><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, 1, w_tiled, nullptr, nullptr, nullptr, glu_act(glu)); \
+  else gemm_tn_kernel<BM, BNN, kEpiSiluGU, NSS, false, false><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, 1, w_tiled, nullptr, nullptr, nullptr, glu_act(glu))
+      if (BM == 64 && BN == 64 && stages == 6) { OAMD_GLU(64, 64, 6); }
+      else if (BM == 64 && BN == 64) { OAMD_GLU(64, 64, 4); }
+      else if (BM == 64 && stages == 5) { OAMD_GLU(64, 160, 5); }
+      else if (BM == 64) { OAMD_GLU(64, 160, 4); }
+      else if (BM == 128 && BN == 64) { OAMD_GLU(128, 64, 4); }
+      else if (BM == 128 && stages == 4) { OAMD_GLU(128, 160, 4); }
+      else if (BM == 128) { OAMD_GLU(128, 160, 3); }
+      else if (BN == 64 && stages == 4) { OAMD_GLU(256, 64, 4); }
+      else if (BN == 64) { OAMD_GLU(256, 64, 3); }
+      else { OAMD_GLU(256, 160, 3); }
+#undef OAMD_GLU
+      OAMD_LAUNCH_CHECK();
+      return 0;
+    }
     const dim3 grid(N / 128, M / BM);
 #define OAMD_GLU(BM, NSS, TURN) \
   gemm_tn_kernel<BM, 128, kEpiSiluGU, NSS, false, TURN><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, 1, w_tiled, nullptr, nullptr, nullptr, glu_act(glu))

@@ -165,6 +165,29 @@ def gate_up_plan(M: int, N: int):
     return 64 if M // 64 * tiles <= CUS else None
 
 
+# stages of gemm_decode's gated tiles of other widths, by (rows, columns)
+_GU_TILES = {(64, 64): 4, (128, 64): 4, (256, 64): 4, (64, 160): 4, (128, 160): 3, (256, 160): 3}
+
+
+@functools.lru_cache(maxsize=4096)
+def gate_up_tile(M: int, N: int, K: int) -> tuple[int, int, int] | None:
+    """(rows, columns, stages) of a gated decode tile of 64 or 160 columns, or None for gate_up_plan's of 128. What a workgroup takes
+    in sets its time, so the best width is the one whose workgroups are one round of the CUs, none of them idle (us): 64 rows of 16384 x 2048 in 128 tiles of 128
+    columns 20.5, in 256 of 64 16.7; of 37888 x 3584 in 296 of 128 62, 237 of 160 44; 128 rows of it (gemm_mid) 67 and 50, 256 rows (gemm_pp) 112 and
+    75; 256 rows of 8192 x 4096 43 and, in 128 x 64, 32. Taken where rounds times rows and columns are a tenth less; the smallest differences
+    that were timed gained 8 %. Fewer than 96 tiles are cut along K (_gu_splits), which for longer rows is as fast (64 rows of 8192 x
+    4096 25.1 and 25.3); 192 rows, no bucket's, have their 64-row tiles."""
+    cost = lambda bm, bn: -(-(M // bm * -(-N // bn)) // CUS) * (bm + bn)  # noqa: E731
+    now = gate_up_plan(M, N)
+    if (M == 192 and now is None) or (isinstance(now, int) and _gu_splits(M, N, K, now) > 1 and K > 2048):
+        return None
+    tiles = [t for t in _GU_TILES if M % t[0] == 0 and 96 <= M // t[0] * -(-N // t[1]) <= CUS]
+    best = min(tiles, key=lambda t: (cost(*t), t), default=None)
+    if best is None or cost(*best) >= 0.9 * (cost(now, 128) if isinstance(now, int) else cost(256, 128) if now else cost(128, 256)):
+        return None
+    return *best, _GU_TILES[best]
+
+
 def gate_up_silu(x: torch.Tensor, wgu: torch.Tensor, block: int | None, act: int = SILU, prompt: bool = False) -> torch.Tensor:
     """act(x Wg^T) * (x Wu^T) from the interleaved gate|up weight (``act``: SILU or GELU_TANH). Decode
     buckets run one fused gfx950 kernel (GEMM + gated epilogue, no [M, 2I] intermediate);
@@ -190,6 +213,10 @@ def gate_up_silu(x: torch.Tensor, wgu: torch.Tensor, block: int | None, act: int
     if (x.is_cuda and block == 64 and x.dtype == torch.bfloat16 and M % 64 == 0 and M <= 256 and N % 128 == 0
             and K % 64 == 0 and x.is_contiguous() and wgu.is_contiguous()):
         t = _gemm_table_get().get(("silu", M, N, K))
+        if t is None and (tile := gate_up_tile(M, N, K)) is not None:
+            y = torch.empty(M, N // 2, dtype=x.dtype, device=x.device)
+            kernels().gemm_decode(x, wgu, y, None, 1, tile[1], tile[0], act, False, tile[2])
+            return y
         bm = gate_up_plan(M, N) if t is None else t if isinstance(t, str) else t[0]
         if t is None and bm is None:
             return linear_tile(x, wgu, glu=act, prompt=prompt)
