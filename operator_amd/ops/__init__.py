@@ -760,7 +760,7 @@ _MID_US = {(64, 64): (4.13, 0.186, 0.078, 0.4), (128, 64): (4.55, 0.221, 0.158, 
            (64, 256): (4.75, 0.684, 0.060, 1.4), (96, 256): (6.46, 0.679, 0.106, 2.0), (128, 256): (7.07, 0.697, 0.210, 2.3),
            (160, 256): (9.97, 0.683, 0.211, 6.2), (192, 256): (10.32, 0.696, 0.317, 10.5), (224, 256): (11.09, 0.789, 0.363, 12.0),
            (256, 256): (11.87, 0.899, 0.394, 12.0)}
-NARROW_MAX_M = 2048
+NARROW_MAX_M = 4096
 
 
 def _mid_us(rows: int, cols: int, M: int, N: int, K: int, S: int) -> float:
@@ -777,7 +777,8 @@ def prompt_tile(M: int, N: int, K: int, S: int = 1, glu: int = 0) -> tuple[int, 
     where those are estimated 7 % faster. Few rows in few slices leave most CUs without a tile of 256 columns (100 rows, us: 6144 x 4096 in two
     slices 48 workgroups 31, 192 of 128 x 64 18; 4096 x 14336 in four 64 workgroups 55, 256 29; 28672 x 4096 gated 112 workgroups 65, 224 of 128 x 128
     56; 40 rows of 16384 x 2048 gated 27 and, in 64 x 128 tiles, 20); 200 rows of 4096 x 14336 48 on 96 x 256, 37 on 160 x 128. The sums, and so the bits, are
-    the same for all. 333 of those 504 products take narrow tiles, 0.68 of the time of the others on average; none was slower. A gated product's
+    the same for all. 333 of those 504 products take narrow tiles, 0.68 of the time of the others on average, and 16 of 84 more of 1600 to 3800 rows (2300 of
+    2048 x 8192 89 us on 96 x 256, 70 on 160 x 128); none was slower. A gated product's
     narrowest tile is the 128 rows of W that hold 64 gates and what they multiply."""
     first = tile_rows(M, N, K, S), 256
     if M > NARROW_MAX_M:

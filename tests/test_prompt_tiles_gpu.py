@@ -52,7 +52,7 @@ def test_other_tiles_are_refused(opt):
 
 def test_tiles_that_the_kernels_have():
     for N, K in ((16, 128), (272, 192), (4096, 4096), (28672, 4096), (3584, 18944), (37888, 3584)):
-        for M in (1, 24, 33, 64, 65, 128, 129, 300, 885, 2048, 2049, 30000):
+        for M in (1, 24, 33, 64, 65, 128, 129, 300, 885, 2048, 2049, 4096, 4097, 30000):
             for S in (1, 2, 8):
                 for glu in (0, ops.SILU):
                     t = ops.prompt_tile(M, N, K, S, glu)
