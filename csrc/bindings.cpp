@@ -313,7 +313,8 @@ void gemm_decode(const at::Tensor& x, const at::Tensor& w, const c10::optional<a
   TORCH_CHECK(w.size(1) == K, "gemm shapes (a tiled w keeps its logical [N, K] shape)");
   TORCH_CHECK(!silu_gu || splits == 1, "fused SwiGLU: one K slice");
   if (bm == 0) bm = std::min<int64_t>(M, 256);
-  TORCH_CHECK((bm == 64 || bm == 128 || bm == 256) && M % bm == 0, "gemm_decode: M % bm, bm in {64,128,256}");
+  TORCH_CHECK((bm == 64 || bm == 128 || bm == 256) && (M % bm == 0 || (M < bm && !silu_gu && splits == 1)),
+              "gemm_decode: M % bm or, plain in one slice, M < bm, bm in {64,128,256}");
   TORCH_CHECK(silu_gu ? N % 128 == 0 && (bn == 128 || (!w_tiled && (bn == 64 || bn == 160))) : (bn == 64 || bn == 128) && N % bn == 0,
               "gemm_decode: N % bn, bn in {64, 128}; gated N % 128, also bn = 160");
   TORCH_CHECK(splits >= 1 && splits <= 16 && K % 64 == 0 && K / 64 >= splits, "gemm_decode: bad split count");

@@ -131,6 +131,8 @@ __global__ void __launch_bounds__(kWaves * 64, NS == 2 ? 2 : 1) gemm_tn_kernel(c
     xrow[i] = 8 * (w + kWaves * i) + lrow;
     if constexpr (GRP) {
       if (src != nullptr && xrow[i] < BM) xrow[i] = max(src[m0 + xrow[i]], 0);
+    } else if constexpr (EPI == kEpiStore) {   // rows past M repeat the last one
+      if (xrow[i] < BM) xrow[i] = min(xrow[i], M - 1 - m0);
     }
   }
   const int off = TURN ? turn % T : 0;
@@ -287,7 +289,7 @@ __global__ void __launch_bounds__(kWaves * 64, NS == 2 ? 2 : 1) gemm_tn_kernel(c
         for (int r = 0; r < 4; ++r) {
           const int row = wm * (BM / C::WM) + 16 * i + 4 * lg + r;
           if constexpr (EPI == kEpiPartial) P[((int64_t)kz * M + m0 + row) * N + col] = acc[i][j][r];
-          else Y[(int64_t)(m0 + row) * N + col] = f2bf(acc[i][j][r]);
+          else if (GRP || m0 + row < M) Y[(int64_t)(m0 + row) * N + col] = f2bf(acc[i][j][r]);
         }
       }
   }
@@ -339,14 +341,16 @@ int gemm_decode(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, in
   // bit 0: tiled W layout; bit 1: W streams with the non-temporal policy (OAMD_BF16_WNT)
   static const int wnt = [] { const char* e = getenv("OAMD_BF16_WNT"); return e && e[0] == '0' ? 0 : 2; }();
   const int w_tiled = (w_tiled_b ? 1 : 0) | wnt;
-  const bool turn = turns(K) && M <= 128 && (int64_t)M * K <= kTurnX && (int64_t)N * S >= kTurnN * ((M + BM) / 64);
+  if (BM != 64 && BM != 128 && BM != 256) return -1;
+  const int mt = (M + BM - 1) / BM, Mt = mt * BM;   // tiles' rows: a part of one tile has the sums of a whole one
+  if (M < 1 || (M != Mt && (M > BM || glu || S != 1))) return -1;
+  const bool turn = turns(K) && Mt <= 128 && (int64_t)Mt * K <= kTurnX && (int64_t)N * S >= kTurnN * ((Mt + BM) / 64);
   if (w_tiled_b && (N % 64 != 0 || K % 64 != 0)) return -6;
-  if ((BM != 64 && BM != 128 && BM != 256) || M % BM != 0) return -1;
   if (glu) {  // fused SwiGLU: one K slice, tiles of BN / 2 gate and as many up rows
     if ((BN != 64 && BN != 128 && BN != 160) || S != 1 || N % 128 != 0 || K % kBK != 0) return -5;
     if (BN != 128) {
       if (w_tiled_b) return -6;
-      const dim3 grid((N + BN - 1) / BN, M / BM);
+      const dim3 grid((N + BN - 1) / BN, mt);
 #define OAMD_GLU(BM, BNN, NSS)                                                                                                                 \
   if (turn) gemm_tn_kernel<BM, BNN, kEpiSiluGU, NSS, false, BM <= 128><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, 1, w_tiled, nullptr, nullptr, nullptr, glu_act(glu)); \
   else gemm_tn_kernel<BM, BNN, kEpiSiluGU, NSS, false, false><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, 1, w_tiled, nullptr, nullptr, nullptr, glu_act(glu))
@@ -364,7 +368,7 @@ int gemm_decode(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, in
       OAMD_LAUNCH_CHECK();
       return 0;
     }
-    const dim3 grid(N / 128, M / BM);
+    const dim3 grid(N / 128, mt);
 #define OAMD_GLU(BM, NSS, TURN) \
   gemm_tn_kernel<BM, 128, kEpiSiluGU, NSS, false, TURN><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, 1, w_tiled, nullptr, nullptr, nullptr, glu_act(glu))
     if (BM == 64) {
@@ -388,7 +392,7 @@ int gemm_decode(const bf16_t* X, const bf16_t* W, bf16_t* Y, float* P, int M, in
   if ((BN != 64 && BN != 128) || N % BN != 0) return -2;
   if (S < 1 || S > 16 || K % kBK != 0 || K / kBK < S) return -3;
   if (S > 1 && P == nullptr) return -4;
-  const dim3 grid((N / BN) * S, M / BM);
+  const dim3 grid((N / BN) * S, mt);
 #define OAMD_GEMM4(BM, BNN, NSS, TURN)                                                                                                        \
   if (S > 1) gemm_tn_kernel<BM, BNN, kEpiPartial, NSS, false, TURN><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, S, w_tiled);         \
   else gemm_tn_kernel<BM, BNN, kEpiStore, NSS, false, TURN><<<grid, kWaves * 64, 0, stream>>>(X, W, Y, P, M, N, K, S, w_tiled)

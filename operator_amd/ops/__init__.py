@@ -506,6 +506,19 @@ def _vocab_plan(M: int, N: int, K: int):
     return (M, 128, 1, 3)
 
 
+@functools.lru_cache(maxsize=4096)
+def vocab_rows_plan(M: int, N: int, K: int):
+    """gemm_decode's plan for the vocabulary of 9 to 127 rows (as many prompts' first tokens), or None: a part of the one row tile that a decode bucket
+    has, whose K steps start apart. It streams the weights at 5.2 to 6.4 TB/s, gemm_mid's and gemm_skinny's tiles at 4.1 to 5.3 (9 to 63 rows, us): 128256 x 4096
+    222 to 232 and 175, x 2048 118 to 123 and 101, x 8192 370 and 333, 152064 x 3584 207 to 216 and 198, 32768 x 4096 71 to 75 and 43, 32000 x 2048 30 to 37 and
+    25. Fewer columns leave CUs without a tile (16128 x 4096 31 and 39). Of 65 to 127 rows a vocabulary of one or two rounds gains (32768 x
+    4096 76 to 83 and 56, 32000 x 2048 38 and 32), a larger one does not (128256 x 2048 123 to 131 and 127, 152064 x 3584 216 to 233 and 245)."""
+    if not ROWS_MAX_M < M < 128 or M == 64 or 10 * (N // 128) < 9 * CUS or N % 128 or K % 64 or (M > 64 and N >= 2 * LM_HEAD_MIN_N):
+        return None
+    plan = gemm_plan(64 if M < 64 else 128, N, K, False)
+    return plan if plan is not None and plan[0] >= M and plan[2] == 1 else None
+
+
 SKINNY_MAX_M = 32
 
 
@@ -918,7 +931,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, sp
            defer_reduce: bool = False, stages: int | None = None, bias: torch.Tensor | None = None, prompt: bool = False):
     """y = x @ w^T (+ bias) in bf16 on the gfx950 kernels: up to 8 rows on gemm_rows (rows_plan), up to 32 on gemm_skinny, or on
     gemm_mid where the rows cost more than its tile (_mid_beats_skinny); 64, 128, 192 and 256 rows on the LDS-staged
-    split-K gemm_decode (the measured table, else _decode_tiles; vocabularies _vocab_plan) or where it is estimated
+    split-K gemm_decode (the measured table, else _decode_tiles; vocabularies _vocab_plan, of 9 to 127 rows vocab_rows_plan) or where it is estimated
     faster gemm_mid; everything else (prompts, the lm_head of many of them, biased projections) on gemm_mid's tiles of 96 to 160 rows,
     with K slices where mid_plan has them, or gemm_tile's of 192 to 256 (tile_rows). ``defer_reduce``: K
     slices come back as fp32 slabs (:class:`SplitK`). fp32 operands: linear_f32. hipBLASLt only
@@ -942,6 +955,11 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, sp
         return _blas(x, w, out, None)
     if PREFILL_BLAS and x.is_cuda and M > 256 and N < LM_HEAD_MIN_N and splits is None and x.dtype == torch.bfloat16:
         return _blas(x, w, out, None, planned=True)
+    if (not prompt and out is None and bm is None and bn is None and splits is None and x.is_cuda and x.dtype == w.dtype == torch.bfloat16
+            and x.is_contiguous() and w.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0 and (part := vocab_rows_plan(M, N, K)) is not None):
+        y = torch.empty(M, N, dtype=x.dtype, device=x.device)
+        kernels().gemm_decode(x, w, y, None, 1, part[1], part[0], False, False, part[3] if len(part) > 3 else 3)
+        return y
     if (x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous() and M <= SKINNY_MAX_M
             and bm is None and bn is None):
         S = splits or skinny_plan(M, N, K)
