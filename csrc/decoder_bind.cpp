@@ -250,7 +250,10 @@ void attn_gd_prefill(const at::Tensor& q, const at::Tensor& k, const at::Tensor&
     return;
   }
   oamd::AttnPrefill a{};
-  a.q = p<bf16_t>(q); a.k = p<bf16_t>(k); a.v = p<bf16_t>(v); a.o = p<bf16_t>(o);
+  const at::Tensor k16 = on16(k), v16 = on16(v);
+  OptT pk16, pv16;
+  if (pk.has_value()) pk16 = on16(*pk), pv16 = on16(*pv);
+  a.q = p<bf16_t>(q); a.k = p<bf16_t>(k16); a.v = p<bf16_t>(v16); a.o = p<bf16_t>(o);
   a.o_ld = (int)o.size(1);
   TORCH_CHECK(a.o_ld % 4 == 0, "attn_gd_prefill: o rows");
   a.cu_seqlens = p<int>(cu); a.work_seq = p<int>(*work_seq); a.work_q0 = p<int>(*work_q0);
@@ -259,7 +262,7 @@ void attn_gd_prefill(const at::Tensor& q, const at::Tensor& k, const at::Tensor&
   a.gc = a.G % 4 == 0 ? 4 : a.G % 3 == 0 ? 3 : a.G % 2 == 0 ? 2 : 1;
   a.dkp = (int)dkp; a.dvp = (int)dvp;
   a.scale_log2 = (float)(scale * 1.4426950408889634);
-  a.pk = op<bf16_t>(pk); a.pv = op<bf16_t>(pv); a.seq_pfx = op<int>(seq_pfx);
+  a.pk = op<bf16_t>(pk16); a.pv = op<bf16_t>(pv16); a.seq_pfx = op<int>(seq_pfx);
   a.window = win; a.gate = op<float>(gate);
   RC(oamd::attn_gd_prefill(a, (int)work_seq->numel(), cur_stream()));
 }

@@ -13,6 +13,12 @@
 // raises it by more than 8 in log2 units).
 // seq_pfx: keys of a shared prompt prefix (rows of pk / pv) come before a sequence's own.
 // window: tiles that no row of the workgroup sees are never loaded.
+// Two LDS buffers of a K and a V tile, filled by LDS-DMA while the tile before is used, one barrier a tile. What bounds it is a wave's
+// chain through a tile (products, softmax, products), and of short prompts the longest row's tiles; one buffer filled from registers behind two
+// barriers put loads, LDS writes and waits into that chain. us, before and now, of 8 sequences of 900 tokens: 32 heads of 192 / 128 208 -> 137 (480
+// TFLOP/s), 32 / 8 of 128 115 -> 97, of 96 96 -> 80, of 64 / 256 260 -> 128, 16 of 64 37 -> 34; one of 300: 32 of 192 / 128 21 -> 13, 32 / 8 of 128 16 -> 13.
+// Both buffers fit twice into a CU's 160 KB (192 / 128 exactly), as two workgroups did before, up to 320 columns of K and V together; larger ones have
+// a CU alone (16 / 4 heads of 256: 233 -> 168).
 #include "attn_gd.h"
 
 namespace oamd {
@@ -30,13 +36,13 @@ __device__ __forceinline__ s16x4 tr16(const char* p) {
 // DK, DV: instantiated sizes >= the stored sizes dkp, dvp (the rest is zero in LDS)
 template <int DK, int DV>
 __global__ void __launch_bounds__(256, (DK + DV <= 320) ? 2 : 1) attn_gd_prefill_kernel(const AttnPrefill a) {
-  constexpr int BK = 64, RK = 2 * DK + 16;       // K rows padded by 16 B: conflict-free row reads
-  constexpr int RV = DV <= 128 ? 256 : 512;      // V rows: the 16-chunk swizzle below needs 256-B rows
-  constexpr int CK = DK / 8, CV = DV / 8;
-  constexpr int NCK = BK * CK / 256, NCV = BK * CV / 256;
+  constexpr int BK = 64, RK = 2 * DK;            // LDS row bytes of the tiles
+  constexpr int RV = DV <= 32 ? 64 : DV <= 64 ? 128 : DV <= 128 ? 256 : 512;   // a power of two: the swizzle below
+  constexpr int CK = RK / 16, CV = RV / 16;      // 16-B chunks of a row = KiB of a tile
+  constexpr int NPK = CK / 4, NPV = CV / 4;      // KiB pieces a wave stages per tile
+  constexpr int kKTile = BK * RK, kTile = kKTile + BK * RV;
   constexpr int KS = DK / 16, DB = DV / 32;
-  __shared__ __attribute__((aligned(16))) char Ks[BK * RK];
-  __shared__ __attribute__((aligned(16))) char Vs[BK * RV];
+  __shared__ __attribute__((aligned(1024))) char lds[2 * kTile];
 
   int wi = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
   if (gridDim.y % 8 == 0) {   // a head's workgroups on one XCD, an item's sub-blocks next to each other
@@ -94,137 +100,136 @@ __global__ void __launch_bounds__(256, (DK + DV <= 320) ? 2 : 1) attn_gd_prefill
 
   const int gi = lane & 15, g = lane >> 4;
   const int trq = gi >> 2, trp = gi & 3;
-  auto v_img = [](int r, int ch) { return RV * r + 16 * ((ch & 16) | ((ch & 15) ^ (((r & 3) << 2) | ((r >> 2) & 3)))); };
+  // Images: chunk ch of row r in a slot that depends on the row, as the LDS-DMA's source order. K: 16 rows' reads of one chunk hit 16
+  // slots of the banks; a row of CK chunks shifts those by CK % 16, its swizzle covers the rest.
+  constexpr int kP = CK % 16 == 0 ? 16 : CK % 8 == 0 ? 8 : 4;   // chunks that trade places
+  auto k_swz = [](int r) { return (r / (16 / kP)) & (kP - 1); };
+  // V: the transposed reads take 4 chunks of 4 neighbouring rows at a time.
+  auto v_swz = [](int r) { return CV >= 16 ? ((r & 3) << 2) | ((r >> 2) & 3) : CV == 8 ? (r & 2) << 1 : 0; };
+  auto v_img = [&](int r, int ch) { return RV * r + 16 * (ch ^ v_swz(r)); };
 
-  u16x8 kr[NCK], vr[NCV];
-  // rows of key tile kt: prefix rows (kt < npt) or own rows of tile kt - npt
-  auto row_of = [&](int kt, int key, bool& ok) -> int64_t {
+  // staging: slot 64 p + lane of piece p; chunks past the stored sizes and rows past the end read as zeros
+  const int rbk = a.Hkv * a.dkp * 2, rbv = a.Hkv * a.dvp * 2;   // bytes from row to row
+  uint32_t vk[NPK], vv[NPV];
+#pragma unroll
+  for (int i = 0; i < NPK; ++i) {
+    const int at = 64 * (w + 4 * i) + lane, row = at / CK, ch = (at % CK) ^ k_swz(row);
+    vk[i] = 8 * ch < a.dkp ? (uint32_t)(row * rbk + 16 * ch) : 0x7ffffff0u;
+  }
+#pragma unroll
+  for (int i = 0; i < NPV; ++i) {
+    const int at = 64 * (w + 4 * i) + lane, row = at / CV, ch = (at % CV) ^ v_swz(row);
+    vv[i] = 8 * ch < a.dvp ? (uint32_t)(row * rbv + 16 * ch) : 0x7ffffff0u;
+  }
+  auto stage = [&](int kt, int buf) {   // key tile kt: a prefix tile (kt < npt) or own tile kt - npt
+    const bf16_t *kp, *vp;
+    int rows;
     if (kt < npt) {
-      ok = kt * BK + key < pl;
-      return kt * BK + key;
+      const int64_t r = (int64_t)kt * BK * a.Hkv + kvh;
+      kp = a.pk + r * a.dkp; vp = a.pv + r * a.dvp; rows = pl - kt * BK;
+    } else {
+      const int64_t r = (int64_t)(s0 + (kt - npt) * BK) * a.Hkv + kvh;
+      kp = a.k + r * a.dkp; vp = a.v + r * a.dvp; rows = slen - (kt - npt) * BK;
     }
-    ok = (kt - npt) * BK + key < slen;
-    return (int64_t)s0 + (kt - npt) * BK + key;
-  };
-  auto load_tile = [&](int kt) {
-    const bf16_t* kp = kt < npt ? a.pk : a.k;
-    const bf16_t* vp = kt < npt ? a.pv : a.v;
+    const int last = min(rows, BK) - 1, nk = last * rbk + 2 * a.dkp, nv = last * rbv + 2 * a.dvp;
+    char* dst = lds + buf * kTile + w * 1024;
 #pragma unroll
-    for (int r = 0; r < NCK; ++r) {
-      const int c = tid + r * 256, key = c / CK, ch = c % CK;
-      bool ok;
-      const int64_t row = row_of(kt, key, ok);
-      kr[r] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-      if (ok && 8 * ch < a.dkp) kr[r] = *reinterpret_cast<const u16x8*>(kp + (row * a.Hkv + kvh) * a.dkp + 8 * ch);
-    }
+    for (int i = 0; i < NPK; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)kp, (short)0, nk, 0x00020000),
+                                               (__attribute__((address_space(3))) void*)(dst + 4096 * i), 16, (int)vk[i], 0, 0, 0);
 #pragma unroll
-    for (int r = 0; r < NCV; ++r) {
-      const int c = tid + r * 256, key = c / CV, ch = c % CV;
-      bool ok;
-      const int64_t row = row_of(kt, key, ok);
-      vr[r] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-      if (ok && 8 * ch < a.dvp) vr[r] = *reinterpret_cast<const u16x8*>(vp + (row * a.Hkv + kvh) * a.dvp + 8 * ch);
-    }
-  };
-  auto store_tile = [&]() {
-#pragma unroll
-    for (int r = 0; r < NCK; ++r) {
-      const int c = tid + r * 256, key = c / CK, ch = c % CK;
-      *reinterpret_cast<u16x8*>(Ks + RK * key + 16 * ch) = kr[r];
-    }
-#pragma unroll
-    for (int r = 0; r < NCV; ++r) {
-      const int c = tid + r * 256, key = c / CV, ch = c % CV;
-      *reinterpret_cast<u16x8*>(Vs + v_img(key, ch)) = vr[r];
-    }
+    for (int i = 0; i < NPV; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)vp, (short)0, nv, 0x00020000),
+                                               (__attribute__((address_space(3))) void*)(dst + kKTile + 4096 * i), 16, (int)vv[i], 0, 0, 0);
   };
 
-  load_tile(kt0);
-  for (int kt = kt0; kt < ntiles; ++kt) {
+  const int ks = h ^ k_swz(r32);
+  stage(kt0, 0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  for (int kt = kt0, buf = 0; kt < ntiles; ++kt, buf ^= 1) {
+    if (kt + 1 < ntiles) stage(kt + 1, buf ^ 1);
     const int kb = (kt - npt) * BK;   // own-key coordinates (negative: a prefix tile)
-    __syncthreads();
-    store_tile();
-    __syncthreads();
-    if (!active || kb >= wend) {      // wave-uniform: no visible key for this wave
-      if (kt + 1 < ntiles) load_tile(kt + 1);
-      continue;
-    }
-    f32x16 sacc[2];
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) sacc[b][i] = 0.f;
-      const char* krow = Ks + RK * (32 * b + r32) + 16 * h;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const u16x8 ka = *reinterpret_cast<const u16x8*>(krow + 32 * s);
-        sacc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf8(ka), bf8(qb[s]), sacc[b], 0, 0, 0);
-      }
-    }
-    if (kt + 1 < ntiles) load_tile(kt + 1);   // in flight during softmax + P.V
-    // register i of block b is key kb + 32b + (i&3) + 8(i>>2) + 4h
-    const bool ptile = kb < 0;
-    const int pend = pl - kt * BK;
-    const int wlo = qrow - a.window - (ptile ? kt * BK - pl : kb);   // tile keys up to here are out of the row's window
-    const bool mask = (ptile ? (pend < BK) : ((kb + BK > rbase + 1) || (kb + BK > slen))) ||
-                      rbase + 31 - a.window >= (ptile ? kt * BK - pl : kb);
-    if (mask) {   // the tile's first key past those the row sees, the last one before them
-      const int end = (ptile ? pend : min(qrow + 1, slen) - kb) - 4 * h, out = wlo - 4 * h;
+    const char *Ks = lds + buf * kTile, *Vs = Ks + kKTile;
+    if (active && kb < wend) {   // wave-uniform: a key this wave sees
+      f32x16 sacc[2];
 #pragma unroll
       for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int j = 32 * b + (i & 3) + 8 * (i >> 2);
-          if (j >= end || j <= out) sacc[b][i] = -INFINITY;
+        for (int i = 0; i < 16; ++i) sacc[b][i] = 0.f;
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          const u16x8 ka = *reinterpret_cast<const u16x8*>(Ks + RK * (32 * b + r32) + 16 * ((2 * s) ^ ks));
+          sacc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf8(ka), bf8(qb[s]), sacc[b], 0, 0, 0);
+        }
+      // register i of block b is key kb + 32b + (i&3) + 8(i>>2) + 4h
+      const bool ptile = kb < 0;
+      const int pend = pl - kt * BK;
+      const int wlo = qrow - a.window - (ptile ? kt * BK - pl : kb);   // tile keys up to here are out of the row's window
+      const bool mask = (ptile ? (pend < BK) : ((kb + BK > rbase + 1) || (kb + BK > slen))) ||
+                        rbase + 31 - a.window >= (ptile ? kt * BK - pl : kb);
+      if (mask) {   // the tile's first key past those the row sees, the last one before them
+        const int end = (ptile ? pend : min(qrow + 1, slen) - kb) - 4 * h, out = wlo - 4 * h;
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int j = 32 * b + (i & 3) + 8 * (i >> 2);
+            if (j >= end || j <= out) sacc[b][i] = -INFINITY;
+          }
+      }
+      float mx = sacc[0][0];
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[b][i]);
+      mx = fmaxf(mx, __shfl_xor(mx, 32, kWave)) * scale;
+      float mnew = fmaxf(mrow, mx);
+      const bool rescale = mrow == -INFINITY || mnew > mrow + 8.f;
+      if (!rescale) mnew = mrow;
+      const float msafe = (mnew == -INFINITY) ? 0.f : mnew;
+      const float alpha = rescale ? exp2_weight(mrow - msafe) : 1.f;
+      mrow = mnew;
+      float rs = 0.f;
+      u16x8 pb[2][2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          f32x8 p;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            p[j] = exp2_weight(weight_arg(sacc[b][8 * s + j], scale, msafe));
+            rs += p[j];
+          }
+          pb[b][s] = __builtin_bit_cast(u16x8, __builtin_convertvector(p, bf16x8));
+        }
+      lpart = lpart * alpha + rs;
+      if (__any(rescale)) {
+#pragma unroll
+        for (int dd = 0; dd < DB; ++dd)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) oacc[dd][i] *= alpha;
+      }
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const int r0 = 32 * b + 16 * s + 4 * h + trq;
+#pragma unroll
+          for (int dd = 0; dd < DB; ++dd) {
+            const int d = 32 * dd + 16 * (g & 1) + 4 * trp;
+            const s16x4 lo = tr16(Vs + v_img(r0, d >> 3) + 8 * ((d >> 2) & 1));
+            const s16x4 hi = tr16(Vs + v_img(r0 + 8, d >> 3) + 8 * ((d >> 2) & 1));
+            const s16x8 va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+            oacc[dd] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va), bf8(pb[b][s]), oacc[dd], 0, 0, 0);
+          }
         }
     }
-    float mx = sacc[0][0];
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[b][i]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave)) * scale;
-    float mnew = fmaxf(mrow, mx);
-    const bool rescale = mrow == -INFINITY || mnew > mrow + 8.f;
-    if (!rescale) mnew = mrow;
-    const float msafe = (mnew == -INFINITY) ? 0.f : mnew;
-    const float alpha = rescale ? exp2_weight(mrow - msafe) : 1.f;
-    mrow = mnew;
-    float rs = 0.f;
-    u16x8 pb[2][2];
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        f32x8 p;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          p[j] = exp2_weight(weight_arg(sacc[b][8 * s + j], scale, msafe));
-          rs += p[j];
-        }
-        pb[b][s] = __builtin_bit_cast(u16x8, __builtin_convertvector(p, bf16x8));
-      }
-    lpart = lpart * alpha + rs;
-    if (__any(rescale)) {
-#pragma unroll
-      for (int dd = 0; dd < DB; ++dd)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) oacc[dd][i] *= alpha;
-    }
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int r0 = 32 * b + 16 * s + 4 * h + trq;
-#pragma unroll
-        for (int dd = 0; dd < DB; ++dd) {
-          const int d = 32 * dd + 16 * (g & 1) + 4 * trp;
-          const s16x4 lo = tr16(Vs + v_img(r0, d >> 3) + 8 * ((d >> 2) & 1));
-          const s16x4 hi = tr16(Vs + v_img(r0 + 8, d >> 3) + 8 * ((d >> 2) & 1));
-          const s16x8 va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-          oacc[dd] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va), bf8(pb[b][s]), oacc[dd], 0, 0, 0);
-        }
-      }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
   }
   if (!active) return;
   const float lsum = lpart + __shfl_xor(lpart, 32, kWave);
