@@ -386,9 +386,10 @@ void gemm_mid(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::
   TORCH_CHECK(M >= 1 && N >= 16 && N % 16 == 0 && K % 64 == 0, "gemm_mid: N % 16 == 0, K % 64 == 0");
   TORCH_CHECK(M < (1LL << 24) && N < (1LL << 30) && K < (1LL << 22), "gemm too large");
   TORCH_CHECK(splits >= 1 && splits <= 16 && K / 64 >= splits, "gemm_mid: bad split count");
-  TORCH_CHECK(((rows == 96 || rows == 160) && (cols == 128 || cols == 256)) ||
-                  ((rows == 64 || rows == 128) && (cols == 64 || cols == 128 || cols == 256)),
-              "gemm_mid: tiles of 64, 96, 128 or 160 rows and 128 or 256 columns, of 64 or 128 rows and 64 columns");
+  TORCH_CHECK(((rows == 64 || rows == 96 || rows == 128 || rows == 160) && (cols == 128 || cols == 256)) ||
+                  ((rows == 192 || rows == 224 || rows == 256) && cols == 128) ||
+                  ((rows == 64 || rows == 128) && cols == 64),
+              "gemm_mid: tiles of 64, 96, 128 or 160 rows and 256 columns, these and 192, 224 or 256 rows and 128, 64 or 128 rows and 64");
   TORCH_CHECK(cols > 64 || splits > 1 || !silu_gu, "gemm_mid: a gated epilogue needs 128 columns of a tile");
   TORCH_CHECK(!silu_gu || (N % 128 == 0 && !bias.has_value()), "gemm_mid: a gated epilogue needs N % 128, no bias");
   bf16_t* yp = nullptr;

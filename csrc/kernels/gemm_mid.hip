@@ -3,15 +3,15 @@
 //
 // What bounds it: not the matrix cores but the CUs a launch keeps busy. The 256 x 256 tiles of gemm_tile make 64
 // workgroups of an 885 x 4096 product, each walking the whole K at 1.2 us per 64 columns. Here a tile is 64 to 160 rows by
-// 64, 128 or 256 columns (ops.tile_rows, ops.prompt_tile) and its K may be cut into S slices (fp32 slabs, summed by the consumer or by a reduce pass),
+// 64, 128 or 256 columns, or 192 to 256 by 128 (ops.tile_rows, ops.prompt_tile), and its K may be cut into S slices (fp32 slabs, summed by the consumer or by a reduce pass),
 // so that the workgroups come close to one per CU or to whole rounds of them:
-//   885 rows (weights from HBM)   6144 x 4096, 96-row tiles: 49 us (128-row tiles 55); 4096 x 4096 in 2 slices 35; 4096 x 14336 in 2
-//                                 101 (297 on the 256-row tiles)
+//   885 rows (weights from HBM)   6144 x 4096, 192 x 128 tiles: 45 us (96 x 256 49, 128 x 256 55); 4096 x 4096 in 2 slices, 224 x 128: 33
+//                                 (128 x 256 36); 4096 x 14336 in 2, 224 x 128: 96 (101; 297 on the 256-row tiles)
 //   300 rows                      28672 x 4096, 160-row tiles: 68 us (128 rows 110, 256 rows 95)
 //   1500 rows                     6144 x 4096, 160-row tiles: 62 us (128 rows 93, 256 rows 90)
 //   100 rows                      6144 x 4096 in 2 slices, 192 tiles of 128 x 64: 18 us (48 of 128 x 256 31); 4096 x 14336 in 4, 256 of
 //                                 128 x 64: 29 (55); 28672 x 4096 gated, 224 of 128 x 128: 56 (65)
-//   200 rows                      4096 x 14336 in 4 slices, 160 x 128 tiles: 37 us (96 x 256 48)
+//   200 rows                      4096 x 14336 in 4 slices, 160 x 128 tiles: 37 us (96 x 256 48); 28672 x 4096 gated, 224 x 128: 60 (128 x 256 64)
 //   vocabulary 128256 x 8192, 64 rows: 373 us (5.6 TB/s of weights; the 256-row tiles 422)
 // The first slice carries a bias (4608 x 3584, 300 rows: 54 us in one slice, 22 in 3).
 // A 128 x 256 step takes 0.63 us alone, 0.79 with every CU busy (clock). Its MFMAs are 0.47, its LDS-DMA pieces by themselves 0.45 (a CU's
@@ -313,6 +313,9 @@ int gemm_mid(const bf16_t* X, const bf16_t* W, bf16_t* Y, const bf16_t* bias, fl
   else OAMD_MID(96, 128);
   else OAMD_MID(128, 128);
   else OAMD_MID(160, 128);
+  else OAMD_MID(192, 128);
+  else OAMD_MID(224, 128);
+  else OAMD_MID(256, 128);
   else OAMD_MID(64, 64);
   else OAMD_MID(128, 64);
   else return -8;

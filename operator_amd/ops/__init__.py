@@ -767,9 +767,11 @@ def tile_rows(M: int, N: int, K: int, S: int = 1) -> int:
 
 
 # us of a prompt's tiles by (rows, columns): to start and to store, a 64-column piece of K on a CU, what it takes more with every CU busy, between
-# rounds. Fitted to 504 products of 25 shapes, 33 to 2000 rows, in their plans' slices, weights from HBM
+# rounds. Fitted to 504 products of 25 shapes, 33 to 2000 rows, in their plans' slices, weights from HBM; 192 to 256 rows by 128 columns to 266 of 14, 140 to
+# 3000 rows, and 1 us to start added, without which two products of some 20 us were 2 and 5 % slower
 _MID_US = {(64, 64): (4.13, 0.186, 0.078, 0.4), (128, 64): (4.55, 0.221, 0.158, 1.2), (64, 128): (4.8, 0.376, 0.049, 0.4),
            (96, 128): (5.64, 0.404, 0.048, 1.3), (128, 128): (5.64, 0.404, 0.175, 2.4), (160, 128): (7.22, 0.439, 0.111, 3.1),
+           (192, 128): (7.51, 0.463, 0.210, 3.0), (224, 128): (7.82, 0.469, 0.291, 2.0), (256, 128): (8.41, 0.482, 0.353, 2.4),
            (64, 256): (4.75, 0.684, 0.060, 1.4), (96, 256): (6.46, 0.679, 0.106, 2.0), (128, 256): (7.07, 0.697, 0.210, 2.3),
            (160, 256): (9.97, 0.683, 0.211, 6.2), (192, 256): (10.32, 0.696, 0.317, 10.5), (224, 256): (11.09, 0.789, 0.363, 12.0),
            (256, 256): (11.87, 0.899, 0.394, 12.0)}
@@ -791,7 +793,9 @@ def prompt_tile(M: int, N: int, K: int, S: int = 1, glu: int = 0) -> tuple[int, 
     slices 48 workgroups 31, 192 of 128 x 64 18; 4096 x 14336 in four 64 workgroups 55, 256 29; 28672 x 4096 gated 112 workgroups 65, 224 of 128 x 128
     56; 40 rows of 16384 x 2048 gated 27 and, in 64 x 128 tiles, 20); 200 rows of 4096 x 14336 48 on 96 x 256, 37 on 160 x 128. The sums, and so the bits, are
     the same for all. 333 of those 504 products take narrow tiles, 0.68 of the time of the others on average, and 16 of 84 more of 1600 to 3800 rows (2300 of
-    2048 x 8192 89 us on 96 x 256, 70 on 160 x 128); none was slower. A gated product's
+    2048 x 8192 89 us on 96 x 256, 70 on 160 x 128); none was slower. Tiles of 192 to 256 rows by 128 columns take in the fewest bytes for what they compute where the wide
+    ones' rounds do not come out: 43 of 266 more have them, 2 to 16 % faster (885 rows of 4096 x 14336 101 us on 128 x 256, 96 on 224 x 128; 1200 of 4608 x 3584 47
+    and, on 192 x 128, 40), none slower by more than the 1.5 % that two runs differ by. A gated product's
     narrowest tile is the 128 rows of W that hold 64 gates and what they multiply."""
     first = tile_rows(M, N, K, S), 256
     if M > NARROW_MAX_M:
@@ -835,7 +839,7 @@ def linear_tile(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = Non
         kernels().gemm_mid(x, w, None, bias, part, S, **opt)
         return SplitK(part, S, M, N)
     y = out if out is not None else torch.empty(M, N // 2 if glu else N, dtype=x.dtype, device=x.device)
-    if rows < 192:
+    if rows < 192 or cols < 256:
         kernels().gemm_mid(x, w, y, bias, part, S or 1, glu, **opt)
     else:
         kernels().gemm_tile(x, w, y, bias, glu, 1 if not glu and loose_tiles(M, N, K) else 0, rows=rows)
