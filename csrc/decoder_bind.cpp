@@ -574,7 +574,7 @@ void head_gemm(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, int64_t 
 }
 
 void gemm_f32(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, int64_t silu_gu, const OptT& gtab, const OptT& rscale,
-              const OptT& partial, int64_t splits, int64_t rows) {
+              const OptT& partial, int64_t splits, int64_t rows, int64_t blocks) {
   TORCH_CHECK(x.dim() == 2 && y.dim() == 2, "gemm_f32: x [M, K], y [M, N]");
   const int64_t M = x.size(0), K = x.size(1), N = w.size(-2);
   need(x, at::kFloat, M * K, "x");
@@ -593,6 +593,12 @@ void gemm_f32(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, int64_t s
   if (splits > 1) {
     TORCH_CHECK(partial.has_value() && !gtab.has_value() && !rscale.has_value() && N % 4 == 0, "gemm_f32: K slices");
     need(*partial, at::kFloat, splits * M * N, "partial");
+  }
+  if (blocks) {
+    TORCH_CHECK(blocks > 0 && blocks < (1 << 20) && M >= 1 && M <= 8 && w.dim() == 2 && !rscale.has_value() && splits == 1 && rows == 0 && N < (1 << 30) && K < (1 << 24),
+                "gemm_f32: one to eight plain rows stream W");
+    RC(oamd::gemm_f32_rows(p<float>(x), p<float>(w), p<float>(y), (int)M, (int)N, (int)K, (int)y.size(1), (int)silu_gu, (int)blocks, cur_stream()));
+    return;
   }
   const bool tiles = rows || oamd::f32_tiles((int)M, (int)K, gtab.has_value());
   const at::Tensor xa = tiles ? on16(x) : x, wa = tiles ? on16(w) : w;
@@ -748,7 +754,8 @@ void register_decoder_bindings(pybind11::module_& m) {
   m.def("head_gemm", &head_gemm, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("x0") = 0, py::arg("nx") = 0);
   m.def("gemm_f32_splits", &oamd::gemm_f32_splits, py::arg("M"), py::arg("N"), py::arg("K"), py::arg("glu"));
   m.def("gemm_f32", &gemm_f32, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("silu_gu") = 0,
-        py::arg("gtab") = no, py::arg("rscale") = no, py::arg("partial") = no, py::arg("splits") = 1, py::arg("rows") = 0);
+        py::arg("gtab") = no, py::arg("rscale") = no, py::arg("partial") = no, py::arg("splits") = 1, py::arg("rows") = 0, py::arg("blocks") = 0);
+  m.def("f32_rows_waves", &oamd::f32_rows_waves);
   m.def("moe_route", &moe_route, py::arg("h"), py::arg("wr"), py::arg("E"), py::arg("ids"), py::arg("weights"),
         py::arg("gate") = no, py::arg("logits") = no);
   m.def("moe_topk", &moe_topk, py::arg("logits"), py::arg("E"), py::arg("ids"), py::arg("weights"), py::arg("gate") = no);

@@ -210,7 +210,8 @@ __global__ void __launch_bounds__(256) slabs_f32_kernel(const GemmF32 a) {
   put4(a.Y + m * a.ldy + f, v, 4, a.vec);
 }
 
-// The same product for at most 16 MT rows: small decode batches and the last rows of a prefill.
+// The same product for at most 16 MT rows: small decode batches and the last rows of a prefill; up to eight of 768 columns and more run in
+// gemm_f32_rows.hip (ops.f32_rows_blocks).
 // What bounds it: streaming W once from HBM (1 row: 16384 x 2048 gated 37 us, 3.6 TB/s; 32000 x 2048 53 us, 5 TB/s; the
 // 64-row FMA tiles before took 450 and 180). A workgroup takes 16 features (GLU: 16 gate and 16 up rows); its waves
 // take 32-column pieces of K in turn, whole 128-B lines of 16 rows straight into MFMA fragments (two to four pieces

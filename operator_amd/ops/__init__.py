@@ -914,12 +914,34 @@ def f32_split_rows(M: int, N: int, K: int, S: int, glu: int) -> int:
     return min((_f32_split_us(r, S, M, N, K, glu), r) for r in _F32_SPLIT)[1]
 
 
+@functools.lru_cache(maxsize=4096)
+def f32_rows_blocks(M: int, N: int, K: int, glu: int) -> int | None:
+    """Workgroups in which one to eight fp32 rows run on the row-streaming kernel (gemm_f32_rows.hip), or None for gemm_f32: rows too long for
+    its registers, and those under 768 columns, which leave it idle lanes and little to stream (one and eight rows, us, here and on gemm_f32: 2048 x 768
+    4.9, 5.1 and 5.2, 5.6; 4096 x 512 5.1, 5.8 and 4.6, 4.7).
+
+    One workgroup per CU up to 3e7 weights (2048 x 8192 13.3 us, 15.0 on three, 6144 x 4096 18.6 and 19.4), three past that (28672 x 4096
+    gated 76 and 72, 32000 x 2048 of eight rows 46 on two, 45 on three), and where one per CU starts at rows of the same memory channels (_rows_in_step: 8128
+    x 4096 32.3 and 22.6, 16256 x 2048 32.2 and 24.0)."""
+    if not 1 <= M <= ROWS_MAX_M or K % 16 or K < 768 or N * K < 5e5 or (glu and N % 128) or not kernels().f32_rows_waves(M, K):
+        return None
+    counts = (CUS, 3 * CUS) if N * K < 3e7 else (3 * CUS, 4 * CUS)
+    B = next((b for b in counts if not _rows_in_step(N, 2 * K, b, bool(glu))), counts[0])
+    lds = 16 * kernels().f32_rows_waves(M, K) << (M - 1).bit_length()   # bytes of a row's sums
+    while (-(-(N // 2 if glu else N) // B) * (2 if glu else 1) + 8) * lds > 48 << 10:
+        B *= 2
+    return B
+
+
 def linear_f32(x: torch.Tensor, w: torch.Tensor, glu: int = 0, prompt: bool = False) -> torch.Tensor:
     """x @ w^T with 32-bit operands and sums, optionally with the gated epilogue (SILU / GELU_TANH) over a 64-row
     interleaved gate|up weight. ``prompt``: as for ``linear``."""
     M, K = x.shape
     N = w.shape[0]
     y = torch.empty(M, N // 2 if glu else N, dtype=x.dtype, device=x.device)
+    if (blocks := f32_rows_blocks(M, N, K, glu)) is not None:
+        kernels().gemm_f32(x, w, y, glu, blocks=blocks)
+        return y
     plan = f32_plan_rows(M, prompt)
     S = f32_split_slices(plan, N, K, glu) if M else None
     rows = 0 if S is None else f32_split_rows(M, N, K, S, glu)
