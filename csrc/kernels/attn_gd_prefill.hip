@@ -18,7 +18,8 @@
 // barriers put loads, LDS writes and waits into that chain. us, before and now, of 8 sequences of 900 tokens: 32 heads of 192 / 128 208 -> 137 (480
 // TFLOP/s), 32 / 8 of 128 115 -> 97, of 96 96 -> 80, of 64 / 256 260 -> 128, 16 of 64 37 -> 34; one of 300: 32 of 192 / 128 21 -> 13, 32 / 8 of 128 16 -> 13.
 // Both buffers fit twice into a CU's 160 KB (192 / 128 exactly), as two workgroups did before, up to 320 columns of K and V together; larger ones have
-// a CU alone (16 / 4 heads of 256: 233 -> 168).
+// a CU alone (16 / 4 heads of 256: 233 -> 168). K's fragments requested four steps ahead, a weight's argument in one FMA and the halves' maximum without LDS:
+// 16 / 4 heads of 256 168 -> 145, 8 / 2 of 160 79 -> 72, 32 / 8 of 128 97 -> 93, 16 of 64 34 -> 31; 192 / 128 as before.
 #include "attn_gd.h"
 
 namespace oamd {
@@ -157,13 +158,23 @@ __global__ void __launch_bounds__(256, (DK + DV <= 320) ? 2 : 1) attn_gd_prefill
       for (int b = 0; b < 2; ++b)
 #pragma unroll
         for (int i = 0; i < 16; ++i) sacc[b][i] = 0.f;
+      constexpr int KA = KS < 4 ? KS : 4;
+      u16x8 ka[KA][2];   // fragments of four 16-dim steps, requested that far ahead
+      auto rdk = [&](int s) {
 #pragma unroll
-      for (int s = 0; s < KS; ++s)
+        for (int b = 0; b < 2; ++b) ka[s % KA][b] = *reinterpret_cast<const u16x8*>(Ks + RK * (32 * b + r32) + 16 * ((2 * s) ^ ks));
+      };
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-          const u16x8 ka = *reinterpret_cast<const u16x8*>(Ks + RK * (32 * b + r32) + 16 * ((2 * s) ^ ks));
-          sacc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf8(ka), bf8(qb[s]), sacc[b], 0, 0, 0);
-        }
+      for (int s = 0; s < KA; ++s) rdk(s);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) sacc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf8(ka[s % KA][b]), bf8(qb[s]), sacc[b], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (s + KA < KS) rdk(s + KA);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       // register i of block b is key kb + 32b + (i&3) + 8(i>>2) + 4h
       const bool ptile = kb < 0;
       const int pend = pl - kt * BK;
@@ -185,7 +196,7 @@ __global__ void __launch_bounds__(256, (DK + DV <= 320) ? 2 : 1) attn_gd_prefill
       for (int b = 0; b < 2; ++b)
 #pragma unroll
         for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[b][i]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32, kWave)) * scale;
+      mx = max_halves(mx) * scale;
       float mnew = fmaxf(mrow, mx);
       const bool rescale = mrow == -INFINITY || mnew > mrow + 8.f;
       if (!rescale) mnew = mrow;
@@ -201,7 +212,7 @@ __global__ void __launch_bounds__(256, (DK + DV <= 320) ? 2 : 1) attn_gd_prefill
           f32x8 p;
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
-            p[j] = exp2_weight(weight_arg(sacc[b][8 * s + j], scale, msafe));
+            p[j] = exp2_weight(__builtin_fmaf(sacc[b][8 * s + j], scale, -msafe));
             rs += p[j];
           }
           pb[b][s] = __builtin_bit_cast(u16x8, __builtin_convertvector(p, bf16x8));

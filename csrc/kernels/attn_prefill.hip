@@ -413,8 +413,11 @@ __device__ __forceinline__ s16x4 ds_read_tr16(const char* p) {
 // the library's exp2f (range checks around v_exp_f32), a scale, a select and a subtraction per score and K/V staged through registers
 // behind two barriers a tile took 2.9 us alone on a CU. The bare v_exp_f32 (arguments are at most 8, and what underflows
 // is zero), the maximum over unscaled scores, masks in tiles that need them only: 2.0; LDS-DMA: 1.6. 885 tokens, 32 / 8 heads:
-// 44.6 -> 25.8 us, 32 prompts of about 885: 430 -> 335 (600 TFLOP/s), 4 x 2048: 267 -> 175. Neither more tiles in flight nor fragments
-// read ahead gained, nor keys split over two groups of waves (23 us, but 440 for the 32 prompts).
+// 44.6 -> 25.8 us, 32 prompts of about 885: 430 -> 335 (600 TFLOP/s), 4 x 2048: 267 -> 175. More tiles in flight did not gain, nor keys split over
+// two groups of waves (23 us, but 440 for the 32 prompts), nor tiles of 32 keys on three waves a SIMD (322 for those, but 34 for the one), nor a DMA
+// that no compiler's wait in front of the transposed reads stands behind. K's fragments requested four steps ahead (behind scheduling
+// barriers: by itself the compiler asks for two and waits for them), a weight's argument in one FMA and the halves' maximum without LDS:
+// 885 tokens 25.5 -> 24.0, 2048 70 -> 65, 32 x 885 340 -> 329, 4 x 2048 190 -> 182, 3 x 700 on 16 / 4 heads 22.7 -> 21.2.
 // NW: waves per workgroup. 8 (one work item = 8 waves of (head, 32-row block)) holds a CU
 // alone at over 200 VGPRs (2 waves per SIMD), so every barrier of its K/V tile loop idles the
 // CU; NW = 4 (G <= 4) halves the work item and puts two workgroups on each CU.
@@ -528,13 +531,22 @@ __global__ void __launch_bounds__(NW * 64, 2) attn_prefill_mfma32_kernel(
       for (int b = 0; b < 2; ++b)
 #pragma unroll
         for (int i = 0; i < 16; ++i) sacc[b][i] = 0.f;
+      u16x8 ka[4][2];   // fragments of four 16-dim steps, requested that far ahead
+      auto rdk = [&](int s) {
 #pragma unroll
-      for (int s = 0; s < 8; ++s)
+        for (int b = 0; b < 2; ++b) ka[s & 3][b] = *reinterpret_cast<const u16x8*>(Kc + k_img(32 * b + r32, 2 * s + h));
+      };
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-          const u16x8 ka = *reinterpret_cast<const u16x8*>(Kc + k_img(32 * b + r32, 2 * s + h));
-          sacc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(ka), as_bf8(qb[s]), sacc[b], 0, 0, 0);
-        }
+      for (int s = 0; s < 4; ++s) rdk(s);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) sacc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(ka[s & 3][b]), as_bf8(qb[s]), sacc[b], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (s < 4) rdk(s + 4);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       // ---- online softmax: register i of block b is key kb + 32b + (i&3) + 8(i>>2) + 4h ----
       const bool ptile = kb < 0;
       const int pend = pl - kt * BK;   // prefix tile: its keys below pend are prefix keys
@@ -553,7 +565,7 @@ __global__ void __launch_bounds__(NW * 64, 2) attn_prefill_mfma32_kernel(
       for (int b = 0; b < 2; ++b)
 #pragma unroll
         for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[b][i]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32, kWave)) * scale_log2;
+      mx = max_halves(mx) * scale_log2;
       float mnew = fmaxf(mrow, mx);
       const bool rescale = mrow == -INFINITY || mnew > mrow + 8.f;   // deferred rescale
       if (!rescale) mnew = mrow;
@@ -569,7 +581,7 @@ __global__ void __launch_bounds__(NW * 64, 2) attn_prefill_mfma32_kernel(
           f32x8 p;
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
-            p[j] = exp2_weight(weight_arg(sacc[b][8 * s + j], scale_log2, msafe));
+            p[j] = exp2_weight(__builtin_fmaf(sacc[b][8 * s + j], scale_log2, -msafe));
             rs += p[j];
           }
           pb[b][s] = __builtin_bit_cast(u16x8, __builtin_convertvector(p, bf16x8_t));

@@ -64,12 +64,11 @@ __device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) {
 // results below 2^-126, which are zero weights here.
 __device__ __forceinline__ float exp2_weight(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// A weight's argument from the raw score: scaled and rounded, then the row's maximum (a scaled score itself) subtracted. Not
-// contracted, so the largest score's own argument is exactly 0.
-__device__ __forceinline__ float weight_arg(float score, float scale, float top) {
-#pragma clang fp contract(off)
-  const float x = score * scale;
-  return x - top;
+// The larger of v and of lane ^ 32's: the halves trade places in registers, where a shuffle is a round trip to LDS.
+__device__ __forceinline__ float max_halves(float v) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
 __device__ __forceinline__ float wave_sum(float v) {
