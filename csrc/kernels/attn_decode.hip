@@ -468,15 +468,10 @@ __global__ void __launch_bounds__(256, (NT == 1 && G <= 4) ? 3 : 2)
 
   // ---- merge the 4 token groups of each wave, then the 4 waves ----
   {
-    float M = m_run;   // lane (head l15, group lg)
-    M = fmaxf(M, __shfl_xor(M, 16, kWave));
-    M = fmaxf(M, __shfl_xor(M, 32, kWave));
+    const float M = max_rows(m_run);   // lane (head l15, group lg)
     const float f = exp2_weight(m_run - M);
-    float L = l_run * f;
-    L += __shfl_xor(L, 16, kWave);
-    L += __shfl_xor(L, 32, kWave);
     m_run = M;
-    l_run = L;
+    l_run = sum_rows(l_run * f);
     if (l15 < G) pwv[TW * GP + lg * GP + l15] = f;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -488,26 +483,27 @@ __global__ void __launch_bounds__(256, (NT == 1 && G <= 4) ? 3 : 2)
       for (int j = 0; j < 8; ++j) acc[h][j] *= fg;
     }
   }
+  // group lg keeps every fourth sum (of heads, or of a head's dims): 24 exchanges in registers for four heads, where 64 shuffles through LDS took
+  // about 1 us of a workgroup
+  if constexpr (G % 4 == 0) {
 #pragma unroll
-  for (int h = 0; h < G; ++h)
+    for (int h = 0; h < G; h += 4) {
+      float t[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float a = acc[h][j];
-      a += __shfl_xor(a, 16, kWave);
-      a += __shfl_xor(a, 32, kWave);
-      acc[h][j] = a;
+      for (int j = 0; j < 8; ++j) t[j] = sums_rows(acc[h][j], acc[h + 1][j], acc[h + 2][j], acc[h + 3][j]);
+      float* rr = &red[w][h + lg][8 * l15];
+      *reinterpret_cast<f32x4*>(rr) = f32x4{t[0], t[1], t[2], t[3]};
+      *reinterpret_cast<f32x4*>(rr + 4) = f32x4{t[4], t[5], t[6], t[7]};
     }
-  if (lg == 0) {
+  } else {
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      float* rr = &red[w][h][8 * l15];
-      *reinterpret_cast<f32x4*>(rr) = f32x4{acc[h][0], acc[h][1], acc[h][2], acc[h][3]};
-      *reinterpret_cast<f32x4*>(rr + 4) = f32x4{acc[h][4], acc[h][5], acc[h][6], acc[h][7]};
-    }
-    if (l15 < G) {
-      mls[w][l15][0] = m_run;
-      mls[w][l15][1] = l_run;
-    }
+    for (int h = 0; h < G; ++h)
+#pragma unroll
+      for (int j = 0; j < 8; j += 4) red[w][h][8 * l15 + j + lg] = sums_rows(acc[h][j], acc[h][j + 1], acc[h][j + 2], acc[h][j + 3]);
+  }
+  if (lg == 0 && l15 < G) {
+    mls[w][l15][0] = m_run;
+    mls[w][l15][1] = l_run;
   }
   __syncthreads();
   for (int e = tid; e < G * D; e += 256) {

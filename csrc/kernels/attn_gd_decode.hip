@@ -127,8 +127,7 @@ __global__ void __launch_bounds__(256, (NK + NV <= 8) ? 2 : 1) attn_gd_decode_ke
         mx = fmaxf(mx, sc[i][j]);
       }
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+    mx = max_rows(mx);
     if (__any(mx > m_run)) {
       const float alpha = exp2_weight(m_run - mx);
       l_run *= alpha;
@@ -173,8 +172,7 @@ __global__ void __launch_bounds__(256, (NK + NV <= 8) ? 2 : 1) attn_gd_decode_ke
       }
     }
   }
-  l_run += __shfl_xor(l_run, 16, kWave);
-  l_run += __shfl_xor(l_run, 32, kWave);
+  l_run = sum_rows(l_run);
   if (l15 < nh) {
 #pragma unroll
     for (int m = 0; m < 2 * NV; ++m) *reinterpret_cast<f32x4*>(&red[w][l15][16 * m + 4 * lg]) = acc[m];

@@ -133,8 +133,7 @@ __global__ void __launch_bounds__(256 * HG, HG == 1 && NK < 12 ? 2 : 1) attn_lat
       sc[i] = i < left ? (d0[i] + d1[i]) * a.scale_log2 : -INFINITY;
       mx = fmaxf(mx, sc[i]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+    mx = max_rows(mx);
     if (lg == 0) stat[hg][w][l15] = mx;
     __syncthreads();
     mx = m_run;
@@ -175,8 +174,7 @@ __global__ void __launch_bounds__(256 * HG, HG == 1 && NK < 12 ? 2 : 1) attn_lat
     work(even, ti);
     if (kAhead == 2 && ti + 1 < ntile) work(odd, ti + 1);
   }
-  l_run += __shfl_xor(l_run, 16, kWave);
-  l_run += __shfl_xor(l_run, 32, kWave);
+  l_run = sum_rows(l_run);
   __syncthreads();
   if (lg == 0) stat[hg][w][l15] = l_run;   // the sum over this wave's tokens
   __syncthreads();

@@ -64,11 +64,49 @@ __device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) {
 // results below 2^-126, which are zero weights here.
 __device__ __forceinline__ float exp2_weight(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// The larger of v and of lane ^ 32's: the halves trade places in registers, where a shuffle is a round trip to LDS.
-__device__ __forceinline__ float max_halves(float v) {
+// Exchanges between rows of 16 lanes in registers, where a shuffle is a round trip to LDS. swap16: a's odd rows and b's even rows trade places;
+// swap32: a's upper half and b's lower half.
+__device__ __forceinline__ void swap16(float& a, float& b) {
   typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-  const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false));
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false));
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap32(float& a, float& b) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false));
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+
+// The larger of v and of lane ^ 32's
+__device__ __forceinline__ float max_halves(float v) {
+  float u = v;
+  swap32(u, v);
+  return fmaxf(u, v);
+}
+// The largest v, the sum of v over the four lanes l % 16
+__device__ __forceinline__ float max_rows(float v) {
+  float u = v;
+  swap16(u, v);
+  return max_halves(fmaxf(u, v));
+}
+__device__ __forceinline__ float sum_rows(float v) {
+  float u = v;
+  swap16(u, v);
+  v += u;
+  u = v;
+  swap32(u, v);
+  return u + v;
+}
+// Row lg of 16 lanes gets the four rows' sum of v[lg], in sum_rows' order.
+__device__ __forceinline__ float sums_rows(float v0, float v1, float v2, float v3) {
+  swap16(v0, v1);
+  swap16(v2, v3);
+  v0 += v1;
+  v2 += v3;
+  swap32(v0, v2);
+  return v0 + v2;
 }
 
 __device__ __forceinline__ float wave_sum(float v) {

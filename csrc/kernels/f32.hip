@@ -358,8 +358,7 @@ __device__ __forceinline__ float soften(f32x4 (&st)[NB], int j0, int g, int lo, 
       st[kb][r] = j >= lo && j < n ? st[kb][r] * scale : -INFINITY;
       top = fmaxf(top, st[kb][r]);
     }
-  top = fmaxf(top, __shfl_xor(top, 16, kWave));
-  top = fmaxf(top, __shfl_xor(top, 32, kWave));
+  top = max_rows(top);
   const float mn = fmaxf(q.m, top), alpha = expf(q.m - mn);
   float sum = 0.f;
 #pragma unroll
@@ -372,11 +371,6 @@ __device__ __forceinline__ float soften(f32x4 (&st)[NB], int j0, int g, int lo, 
   q.m = mn;
   q.l = q.l * alpha + sum;   // this lane's keys; the query's four lanes meet at the end
   return alpha;
-}
-
-__device__ __forceinline__ float lanes_sum(float v) {
-  v += __shfl_xor(v, 16, kWave);
-  return v + __shfl_xor(v, 32, kWave);
 }
 
 }  // namespace
@@ -563,7 +557,7 @@ __global__ void __launch_bounds__(256 * NG, NG == 1 && D == 64 ? 4 : 1) attn_f32
         acc[b][r] = f;
       }
   }
-  const float l = lanes_sum(st.l);
+  const float l = sum_rows(st.l);
   if (n <= 0) return;
   const float c = (a.gate ? a.gate[(int64_t)(s0 + qrow) * Hq + hq] : 1.f);
 #pragma unroll
@@ -707,7 +701,7 @@ __global__ void __launch_bounds__(512) attn_f32_decode_kernel(const AttnF32 a, i
       }
     }
   }
-  const float l = lanes_sum(st.l);
+  const float l = sum_rows(st.l);
   if (g == 0) {
     mls[w][0][l15] = st.m;
     mls[w][1][l15] = l;
