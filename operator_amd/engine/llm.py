@@ -947,11 +947,12 @@ class LLMEngine:
             st = self._states[bp] = _BucketState(self, bp)
         return st
 
-    def _splits(self, context: int, bp: int) -> int:
-        return ops.decode_splits(context, bp, self.hkv, self.model.split_tokens)
+    def _splits(self, context: int, bp: int, rows: int | None = None) -> int:
+        return ops.decode_splits(context, bp, self.hkv, self.model.split_tokens, rows)
 
     def split_options(self, bp: int) -> list[int]:
-        top = self._splits(self.max_context, bp)
+        fewest = max((b for b in self.buckets if b < bp), default=0) + 1   # rows that this bucket is taken for
+        top = self._splits(self.max_context, bp, fewest)
         return [1 << i for i in range(top.bit_length())]
 
     def _graph(self, bp: int, splits: int) -> _DecodeGraph:
@@ -1027,7 +1028,7 @@ class LLMEngine:
             part = order[a:a + self.max_batch]
             rows = [reqs[i] for i in part]
             bp = self._bucket(len(rows))
-            g = self._graph(bp, self._splits(rows[0].length, bp))
+            g = self._graph(bp, self._splits(rows[0].length, bp, len(rows)))
             own = out.is_cuda and self.model.tp.world == 1   # the step's sampler writes them: the address and order travel with the rows' state
             g.st.load(rows, self.max_pages, part, out if own else None)
             g.run(self.use_graphs)
@@ -1053,7 +1054,7 @@ class LLMEngine:
         bp = self._bucket(B)
         k = max(1, min(self.multi_step, min(r.max_tokens - len(r.output) - ahead for r in reqs)))
         # decode-attention split count for the longest context reached in this window
-        splits = self._splits(max(r.length for r in reqs) + ahead + k - 1, bp)
+        splits = self._splits(max(r.length for r in reqs) + ahead + k - 1, bp, B)
         g = self._graph(bp, splits)
         st = g.st
         if self._active is not st:

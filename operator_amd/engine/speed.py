@@ -135,7 +135,7 @@ def run(names: list[str], layers: int = 4, prefill=PREFILL, decode=DECODE, emit=
                 eng._reserve(r)
                 r.pages = r.pages + kv.allocator.alloc(1)   # the steps below pass the page's end
             bp = eng._bucket(b)
-            g = eng._graph(bp, eng._splits(c, bp))
+            g = eng._graph(bp, eng._splits(c, bp, b))
 
             def steps():
                 g.st.load(reqs, eng.max_pages)

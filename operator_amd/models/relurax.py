@@ -212,8 +212,9 @@ class ReluraxModel(PaddedModel):
         if fb.is_prefill:
             o = self._prefill(i, q, k, v, gate, fb, L, a.window)
         else:
-            # the step's split count is chosen for whole contexts; a window needs no more than its own
-            splits = min(fb.num_splits, ops.decode_splits(a.window or self.cfg.max_position, h.shape[0], L.kv_heads, self.split_tokens))
+            # the step's split count is chosen for whole contexts; a window needs no more than its own, for as many rows as that count stands for
+            rows = max(1, min(h.shape[0], ops.DECODE_TARGET_BLOCKS // (fb.num_splits * self.hkv)))
+            splits = min(fb.num_splits, ops.decode_splits(a.window or self.cfg.max_position, h.shape[0], L.kv_heads, self.split_tokens, rows))
             o = dec.attn_gd_decode(q, cache, fb.block_tables, fb.context_lens, L, a.scale, splits, ws, a.window, gate)
         return ops.linear(o, lw.wo, defer_reduce=True, prompt=fb.is_prefill)
 

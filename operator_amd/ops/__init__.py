@@ -1180,13 +1180,17 @@ def linear_fp8(x: torch.Tensor | tuple[torch.Tensor, torch.Tensor], w8: torch.Te
     return y
 
 
-def decode_splits(max_context: int, batch: int = 1, kv_heads: int = 8, min_tokens: int | None = None) -> int:
+def decode_splits(max_context: int, batch: int = 1, kv_heads: int = 8, min_tokens: int | None = None, rows: int | None = None) -> int:
     """Workgroups per (sequence, kv-head) for decode attention: split only while
     ``batch * kv_heads`` workgroups cannot fill the GPU, never into pieces shorter
     than ``min_tokens`` (256; measured on MI355X, B=16 ctx=1024: 1 split 25.9 us, 4 splits
     23.7 us, 16 splits 47.8 us). Powers of two, so a graph captured per value
-    covers every context length with few captures."""
-    want = -(-DECODE_TARGET_BLOCKS // max(1, batch * kv_heads))
+    covers every context length with few captures.
+
+    ``rows``: how many of the batch's are sequences, where the others are padding, whose workgroups end at once: a bucket of 64 that holds 9 to 32 is cut
+    as far as its sequences still come to one workgroup per CU (two layers, whole steps, us: 16 x 3000 tokens of 28 / 4 heads 593 in one split, 539 in four; 24 x 3000 601 and, in two,
+    567; 12 x 3000 of 32 / 8 545 and, in two, 518; 9 to 31 x 1000 0 to 4 % less). Not further: 24 x 3000 of 32 / 8 535 and, in two, 571."""
+    want = max(-(-DECODE_TARGET_BLOCKS // max(1, batch * kv_heads)), DECODE_TARGET_BLOCKS // max(1, (rows or batch) * kv_heads))
     cap = -(-max(1, int(max_context)) // (min_tokens or DECODE_MIN_SPLIT_TOKENS))
     ns = max(1, min(want, cap, 256))
     # the power of two at or BELOW: splits of 256-512 tokens, not 128-256 (B = 64, one kv-head,
