@@ -595,9 +595,9 @@ void gemm_f32(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, int64_t s
     need(*partial, at::kFloat, splits * M * N, "partial");
   }
   if (blocks) {
-    TORCH_CHECK(blocks > 0 && blocks < (1 << 20) && M >= 1 && M <= 8 && w.dim() == 2 && !rscale.has_value() && splits == 1 && rows == 0 && N < (1 << 30) && K < (1 << 24),
-                "gemm_f32: one to eight plain rows stream W");
-    RC(oamd::gemm_f32_rows(p<float>(x), p<float>(w), p<float>(y), (int)M, (int)N, (int)K, (int)y.size(1), (int)silu_gu, (int)blocks, cur_stream()));
+    TORCH_CHECK(blocks > 0 && blocks < (1 << 20) && M >= 1 && M <= 16 && w.dim() == 2 && !rscale.has_value() && rows == 0 && N < (1 << 30) && K < (1 << 24),
+                "gemm_f32: one to sixteen plain rows stream W");
+    RC(oamd::gemm_f32_rows(p<float>(x), p<float>(w), p<float>(y), op<float>(partial), (int)splits, (int)M, (int)N, (int)K, (int)y.size(1), (int)silu_gu, (int)blocks, cur_stream()));
     return;
   }
   const bool tiles = rows || oamd::f32_tiles((int)M, (int)K, gtab.has_value());

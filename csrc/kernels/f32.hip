@@ -210,8 +210,8 @@ __global__ void __launch_bounds__(256) slabs_f32_kernel(const GemmF32 a) {
   put4(a.Y + m * a.ldy + f, v, 4, a.vec);
 }
 
-// The same product for at most 16 MT rows: small decode batches and the last rows of a prefill; up to eight of 768 columns and more run in
-// gemm_f32_rows.hip (ops.f32_rows_blocks).
+// The same product for at most 16 MT rows: small decode batches and the last rows of a prefill; up to sixteen of 768 columns and more run in
+// gemm_f32_rows.hip (ops.f32_rows_plan).
 // What bounds it: streaming W once from HBM (1 row: 16384 x 2048 gated 37 us, 3.6 TB/s; 32000 x 2048 53 us, 5 TB/s; the
 // 64-row FMA tiles before took 450 and 180). A workgroup takes 16 features (GLU: 16 gate and 16 up rows); its waves
 // take 32-column pieces of K in turn, whole 128-B lines of 16 rows straight into MFMA fragments (two to four pieces
@@ -292,6 +292,13 @@ template <bool GLU, int NW>
 static void launch_skinny(const GemmF32& a, dim3 grid, hipStream_t stream) {
   if (a.M <= 16) gemm_f32_skinny_kernel<GLU, 1, NW><<<grid, 64 * NW, 0, stream>>>(a);
   else gemm_f32_skinny_kernel<GLU, 2, NW><<<grid, 64 * NW, 0, stream>>>(a);
+}
+
+int sum_f32_slabs(const float* P, float* Y, int S, int M, int N, int ldy, hipStream_t stream) {
+  GemmF32 a{nullptr, nullptr, Y, const_cast<float*>(P), M, N, 0, S, 0, ldy, 0, 0, nullptr, nullptr, GluAct{}, ldy % 4 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0};
+  slabs_f32_kernel<false><<<(int)(((int64_t)M * N / 4 + 255) / 256), 256, 0, stream>>>(a);
+  OAMD_LAUNCH_CHECK();
+  return 0;
 }
 
 static int run_f32(GemmF32 a, bool glu, int H, int rows, hipStream_t stream) {

@@ -33,4 +33,6 @@ __device__ __forceinline__ void put4(float* y, const f32x4& v, int n, bool vec) 
 
 int gemm_f32_split(const GemmF32& a, bool glu, int rows, hipStream_t stream);   // rows of a tile: 64, 128 or 256
 
+int sum_f32_slabs(const float* P, float* Y, int S, int M, int N, int ldy, hipStream_t stream);   // f32.hip
+
 }  // namespace oamd

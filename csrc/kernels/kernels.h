@@ -360,8 +360,8 @@ int head_gemm(const HeadGemm& a, hipStream_t stream);
 int gemm_f32(const float* X, const float* W, float* Y, float* P, int S, int M, int N, int K, int ldy, int glu, const int* gtab,
              const float* rscale, int rows, hipStream_t stream);
 int gemm_f32_splits(int M, int N, int K, int glu);
-// One to eight rows, streaming W (gemm_f32_rows.hip) in so many workgroups; f32_rows_waves: 0 where K is too long for it.
-int gemm_f32_rows(const float* X, const float* W, float* Y, int M, int N, int K, int ldy, int glu, int blocks, hipStream_t stream);
+// One to sixteen rows, streaming W (gemm_f32_rows.hip) in so many workgroups for each of S slices of K; f32_rows_waves: 0 where a slice is too long for it.
+int gemm_f32_rows(const float* X, const float* W, float* Y, float* P, int S, int M, int N, int K, int ldy, int glu, int blocks, hipStream_t stream);
 int f32_rows_waves(int M, int K);
 bool f32_tiles(int M, int K, bool grouped);   // these run on the tile kernel, whose operands are 16-B aligned
 // One product per head: as HeadGemm, without the extra columns.

@@ -520,6 +520,7 @@ def vocab_rows_plan(M: int, N: int, K: int):
 
 
 SKINNY_MAX_M = 32
+F32_ROWS_MAX_M = 16
 
 
 def skinny_plan(M: int, N: int, K: int) -> int | None:
@@ -854,7 +855,7 @@ def f32_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def f32_plan_rows(M: int, prompt: bool) -> int:
     """Rows whose K slices an fp32 product takes: a prompt's are those of its padded prefill graph (see mid_plan), so its
-    numbers are the same padded or not; up to 32 rows run on the few-row kernel."""
+    numbers are the same padded or not; up to 32 rows have plans of their own."""
     return -(-M // 512) * 512 if prompt and M > SKINNY_MAX_M else M
 
 
@@ -889,14 +890,14 @@ def _f32_plain_us(M: int, N: int, K: int, glu: int, S: int) -> float:
 @functools.lru_cache(maxsize=4096)
 def f32_split_slices(M: int, N: int, K: int, glu: int) -> int | None:
     """K slices in which ``M`` rows (f32_plan_rows) run on the split kernel (gemm_f32_split.hip), or None: on the fp32 matrix instruction
-    (f32.hip), up to 32 rows and where the split kernel, whose steps wait for more before the first, is not estimated 10 % faster (512
-    rows of 2048 x 288 9 us against 14, of 2048 x 768 24 and 24, of 2048 x 2048 50 and 37; 2000 rows of 2048 x 288 27 and 20). No fewer slices than
+    (f32.hip), on its few-row kernel (up to 16 rows, 32 of less than 2048 columns) and where the split kernel, whose steps wait for more before the first, is not
+    estimated 10 % faster (32 rows of 28672 x 4096 gated 161 us, 127 split, of 32000 x 2048 92 and 69, of 4096 x 14336 78 and 67; 512 rows of 2048 x 288 9 us against 14, of 2048 x 768 24 and 24, of 2048 x 2048 50 and 37; 2000 rows of 2048 x 288 27 and 20). No fewer slices than
     the fp32 instruction would have: sums that are as long are closer to the 64-bit result (0.86 of its distance), but one slice in the place of four is
     further off (3200 x 1376 gated 1.8 times).
 
     A prompt's rows are padded to a multiple of 512 for its plan, but run as they are: slices count that are no slower at the fewest rows of that
     plan either (33 rows of 6144 x 2048 in one slice 56 us against 46, in two 33; of 2912 x 560 19 and 11 whatever the slices)."""
-    if M <= SKINNY_MAX_M:
+    if M <= F32_ROWS_MAX_M or (M <= SKINNY_MAX_M and K < 2048):   # gemm_f32's few-row kernel
         return None
     former = kernels().gemm_f32_splits(M, N, K, glu)
     few = M if M % 512 else max(M - 511, SKINNY_MAX_M + 1)
@@ -915,22 +916,34 @@ def f32_split_rows(M: int, N: int, K: int, S: int, glu: int) -> int:
 
 
 @functools.lru_cache(maxsize=4096)
-def f32_rows_blocks(M: int, N: int, K: int, glu: int) -> int | None:
-    """Workgroups in which one to eight fp32 rows run on the row-streaming kernel (gemm_f32_rows.hip), or None for gemm_f32: rows too long for
-    its registers, and those under 768 columns, which leave it idle lanes and little to stream (one and eight rows, us, here and on gemm_f32: 2048 x 768
-    4.9, 5.1 and 5.2, 5.6; 4096 x 512 5.1, 5.8 and 4.6, 4.7).
+def f32_rows_plan(M: int, N: int, K: int, glu: int) -> tuple[int, int] | None:
+    """(K slices, workgroups of a slice) in which one to sixteen fp32 rows run on the row-streaming kernel (gemm_f32_rows.hip), or None for gemm_f32: rows too
+    long for its registers, and those under 768 columns (1024 of nine rows and more), which leave it idle lanes and little to stream (one and eight rows, us, here
+    and on gemm_f32: 2048 x 768 4.9, 5.1 and 5.2, 5.6; 4096 x 512 5.1, 5.8 and 4.6, 4.7; sixteen: 2048 x 768 6.2 and 6.0).
 
-    One workgroup per CU up to 3e7 weights (2048 x 8192 13.3 us, 15.0 on three, 6144 x 4096 18.6 and 19.4), three past that (28672 x 4096
+    Up to eight rows one workgroup per CU up to 3e7 weights (2048 x 8192 13.3 us, 15.0 on three, 6144 x 4096 18.6 and 19.4), three past that (28672 x 4096
     gated 76 and 72, 32000 x 2048 of eight rows 46 on two, 45 on three), and where one per CU starts at rows of the same memory channels (_rows_in_step: 8128
-    x 4096 32.3 and 22.6, 16256 x 2048 32.2 and 24.0)."""
-    if not 1 <= M <= ROWS_MAX_M or K % 16 or K < 768 or N * K < 5e5 or (glu and N % 128) or not kernels().f32_rows_waves(M, K):
+    x 4096 32.3 and 22.6, 16256 x 2048 32.2 and 24.0). Nine to sixteen keep the vector units busy: slices of up to 2048 columns, whose X four waves hold, on one
+    workgroup per CU or, past 2e7 weights and in slices, two, which is what a CU has room for (sixteen, us: 16384 x 2048 gated 33, 40 on three and 41 on gemm_f32;
+    2048 x 8192 in four slices 23 and 37; 2048 x 2048 8.3 and 10.8; 3072 x 2048 10.2, 12.5 on two and 12.4; 32000 x 2048 63 and 77; 28672 x 4096
+    gated, of eight waves, 156 and 133)."""
+    if not 1 <= M <= F32_ROWS_MAX_M or K % 16 or K < (768 if M <= ROWS_MAX_M else 1024) or N * K < 5e5 or (glu and N % 128):
         return None
-    counts = (CUS, 3 * CUS) if N * K < 3e7 else (3 * CUS, 4 * CUS)
-    B = next((b for b in counts if not _rows_in_step(N, 2 * K, b, bool(glu))), counts[0])
-    lds = 16 * kernels().f32_rows_waves(M, K) << (M - 1).bit_length()   # bytes of a row's sums
+    S = 1 if M <= ROWS_MAX_M else -(-K // 2048)
+    if K % (16 * S) or S > 8 or (S > 1 and (glu or N % 4)):
+        return None
+    waves = kernels().f32_rows_waves(M, K // S)
+    if not waves or (M > ROWS_MAX_M and waves > 4):
+        return None
+    if M > ROWS_MAX_M:
+        B = CUS if S == 1 and N * K < 2e7 else 2 * CUS // S
+    else:
+        counts = (CUS, 3 * CUS) if N * K < 3e7 else (3 * CUS, 4 * CUS)
+        B = next((b for b in counts if not _rows_in_step(N, 2 * K, b, bool(glu))), counts[0])
+    lds = 16 * waves << (M - 1).bit_length()   # bytes of a row's sums
     while (-(-(N // 2 if glu else N) // B) * (2 if glu else 1) + 8) * lds > 48 << 10:
         B *= 2
-    return B
+    return S, B
 
 
 def linear_f32(x: torch.Tensor, w: torch.Tensor, glu: int = 0, prompt: bool = False) -> torch.Tensor:
@@ -939,8 +952,10 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, glu: int = 0, prompt: bool = Fa
     M, K = x.shape
     N = w.shape[0]
     y = torch.empty(M, N // 2 if glu else N, dtype=x.dtype, device=x.device)
-    if (blocks := f32_rows_blocks(M, N, K, glu)) is not None:
-        kernels().gemm_f32(x, w, y, glu, blocks=blocks)
+    if (rows := f32_rows_plan(M, N, K, glu)) is not None:
+        S, blocks = rows
+        part = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if S > 1 else None
+        kernels().gemm_f32(x, w, y, glu, partial=part, splits=S, blocks=blocks)
         return y
     plan = f32_plan_rows(M, prompt)
     S = f32_split_slices(plan, N, K, glu) if M else None
