@@ -18,8 +18,8 @@
 // barriers put loads, LDS writes and waits into that chain. us, before and now, of 8 sequences of 900 tokens: 32 heads of 192 / 128 208 -> 137 (480
 // TFLOP/s), 32 / 8 of 128 115 -> 97, of 96 96 -> 80, of 64 / 256 260 -> 128, 16 of 64 37 -> 34; one of 300: 32 of 192 / 128 21 -> 13, 32 / 8 of 128 16 -> 13.
 // Both buffers fit twice into a CU's 160 KB (192 / 128 exactly), as two workgroups did before, up to 320 columns of K and V together; larger ones have
-// a CU alone (16 / 4 heads of 256: 233 -> 168). K's fragments requested four steps ahead, a weight's argument in one FMA and the halves' maximum without LDS:
-// 16 / 4 heads of 256 168 -> 145, 8 / 2 of 160 79 -> 72, 32 / 8 of 128 97 -> 93, 16 of 64 34 -> 31; 192 / 128 as before.
+// a CU alone (16 / 4 heads of 256: 233 -> 168). K's fragments requested four steps ahead and the halves' maximum without LDS:
+// 16 / 4 heads of 256 168 -> 146, 8 / 2 of 160 79 -> 72, 32 / 8 of 128 97 -> 94, 16 of 64 34 -> 32; 192 / 128 as before.
 #include "attn_gd.h"
 
 namespace oamd {
@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(256, (DK + DV <= 320) ? 2 : 1) attn_gd_prefill
           f32x8 p;
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
-            p[j] = exp2_weight(__builtin_fmaf(sacc[b][8 * s + j], scale, -msafe));
+            p[j] = exp2_weight(weight_arg(sacc[b][8 * s + j], scale, msafe));
             rs += p[j];
           }
           pb[b][s] = __builtin_bit_cast(u16x8, __builtin_convertvector(p, bf16x8));

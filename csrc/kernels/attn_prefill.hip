@@ -416,8 +416,8 @@ __device__ __forceinline__ s16x4 ds_read_tr16(const char* p) {
 // 44.6 -> 25.8 us, 32 prompts of about 885: 430 -> 335 (600 TFLOP/s), 4 x 2048: 267 -> 175. More tiles in flight did not gain, nor keys split over
 // two groups of waves (23 us, but 440 for the 32 prompts), nor tiles of 32 keys on three waves a SIMD (322 for those, but 34 for the one), nor a DMA
 // that no compiler's wait in front of the transposed reads stands behind. K's fragments requested four steps ahead (behind scheduling
-// barriers: by itself the compiler asks for two and waits for them), a weight's argument in one FMA and the halves' maximum without LDS:
-// 885 tokens 25.5 -> 24.0, 2048 70 -> 65, 32 x 885 340 -> 329, 4 x 2048 190 -> 182, 3 x 700 on 16 / 4 heads 22.7 -> 21.2.
+// barriers: by itself the compiler asks for two and waits for them) and the halves' maximum without LDS: 885 tokens
+// 25.2 -> 23.9, 2048 69.5 -> 65.8, 3 x 700 on 16 / 4 heads 22.7 -> 21.4, 16 x 500 on 16 / 8 40.4 -> 39.2, 32 x 885 335 -> 332.
 // NW: waves per workgroup. 8 (one work item = 8 waves of (head, 32-row block)) holds a CU
 // alone at over 200 VGPRs (2 waves per SIMD), so every barrier of its K/V tile loop idles the
 // CU; NW = 4 (G <= 4) halves the work item and puts two workgroups on each CU.
@@ -581,7 +581,7 @@ __global__ void __launch_bounds__(NW * 64, 2) attn_prefill_mfma32_kernel(
           f32x8 p;
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
-            p[j] = exp2_weight(__builtin_fmaf(sacc[b][8 * s + j], scale_log2, -msafe));
+            p[j] = exp2_weight(weight_arg(sacc[b][8 * s + j], scale_log2, msafe));
             rs += p[j];
           }
           pb[b][s] = __builtin_bit_cast(u16x8, __builtin_convertvector(p, bf16x8_t));

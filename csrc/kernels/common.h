@@ -64,6 +64,14 @@ __device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) {
 // results below 2^-126, which are zero weights here.
 __device__ __forceinline__ float exp2_weight(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// A weight's argument from the raw score: scaled and rounded, then the row's maximum (a scaled score itself) subtracted. Not
+// contracted, so the largest score's own argument is exactly 0.
+__device__ __forceinline__ float weight_arg(float score, float scale, float top) {
+#pragma clang fp contract(off)
+  const float x = score * scale;
+  return x - top;
+}
+
 // Exchanges between rows of 16 lanes in registers, where a shuffle is a round trip to LDS. swap16: a's odd rows and b's even rows trade places;
 // swap32: a's upper half and b's lower half.
 __device__ __forceinline__ void swap16(float& a, float& b) {
