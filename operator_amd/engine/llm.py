@@ -495,8 +495,8 @@ class LLMEngine:
         self._graphs: dict[tuple[int, int], _DecodeGraph] = {}
         self._states: dict[int, _BucketState] = {}
         self._pool = None
-        # in fp32 the products of 64 rows are bound by the matrix units: relurax-1b, a step of 16 sequences of 600 tokens 816 us on 64 rows, 648 on 16,
-        # of 32 828 and 767
+        # in fp32 the products of 64 rows are bound by the matrix units: relurax-1b, a step of 16 sequences of 600 tokens 834 us on 64 rows, 562 on 16,
+        # of 32 845 and 783
         self.buckets = _buckets(max_batch, () if model.dtype == torch.float32 else SKIP_BUCKETS)
         self.eos = set(model.cfg.eos_ids)
         # called with the requests a step finished, before their waiters wake (ExplainEngine
